@@ -1,25 +1,23 @@
 """Projection GEMMs for decode: y = x @ W^T.
 
-At decode batch 1-4 the projection is a pure stream of the weight matrix; for the shapes where it
-measured faster the HIP weight-streaming kernel (``kernels/skinny_gemm.hip``) runs it instead
-of a library GEMM.  Larger batches (and CPU tensors) go to ``torch.matmul`` (hipBLASLt with the
-tuned table)."""
+Up to 64 rows the projection is a stream of the weight matrix: the HIP kernels
+``seqmix/thin_gemm.hip`` (1 - 64 rows) and ``kernels/skinny_gemm.hip`` (1 row) run it where they
+measured faster than a library GEMM.  Larger batches (and CPU tensors) go to ``torch.matmul``
+(hipBLASLt with the tuned table)."""
 from __future__ import annotations
 
 import os
 from typing import Optional
 
 import torch
+import torch.nn.functional as F
 
 from ._native import native, use_native
 
-# Measured per shape against hipBLASLt with the tuned table (lumen/bench/skinny_bench.py
-# --m1-forms, profiles/r02_serve/m1_forms.jsonl): the rows-per-lane weight-streaming kernel
-# reaches 4.3-6.5 TB/s at M = 1 and beats hipBLASLt at every Llama-2-7B projection (qkv 17.0 vs
-# 22.9 us, o 7.8 vs 22.7, gate_up 27.8 vs 37.3, down 16.5 vs 27.5, lm_head 38.4 vs 60.6); at
-# M = 2 it still wins or ties everywhere (o 10.4 vs 22.6, down 20.7 vs 27.6, lm_head 51.4 vs
-# 59.0); at M = 3-4 only the N = 4096 projections (o, down) stay ahead, and from M = 5 on
-# hipBLASLt wins, so those are library GEMMs.
+# One row: the rows-per-lane weight-streaming kernel reaches 4.3-6.5 TB/s and beats hipBLASLt at
+# every Llama-2-7B projection (qkv 17.0 vs 22.9 us, o 7.8 vs 22.7, gate_up 27.8 vs 37.3, down 16.5 vs
+# 27.5, lm_head 38.4 vs 60.6); 2 - 4 rows that the thin kernel does not take (K not a multiple of 64)
+# go to it as well, where it wins or ties (2 rows everywhere, 3 - 4 rows up to N = 4096).
 SKINNY_MAX_M = int(os.environ.get("LUMEN_SKINNY_MAX_M", "4"))
 SKINNY_MAX_N = int(os.environ.get("LUMEN_SKINNY_MAX_N", str(1 << 30)))
 SKINNY_WIDE_MAX_M = 2  # above this M only N <= 4096 projections take the GEMV
@@ -33,6 +31,57 @@ def skinny_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
             and x.stride(1) == 1 and w.is_contiguous() and x.shape[1] == w.shape[1]
             and (w.shape[0] % 4 == 0 and w.shape[1] % 8 == 0 and x.stride(0) % 8 == 0
                  if x.shape[0] <= 4 else w.shape[0] % 16 == 0 and w.shape[1] % 128 == 0))
+
+
+# Thin GEMM (seqmix/thin_gemm.hip, whose header holds the measurements).  One row: matrices under 128 MB
+# with K <= 3072 (2048 x 2048: 3.8 vs 4.4 us with the GEMV; 2048 x 5632: 7.3 vs 6.6, 22528 x 4096: 30.7 vs
+# 28.5, and a batch-1 Llama step of 4 layers of width 4096: 432 vs 407 us -- those stay with it).  33 - 64 rows: up to 24 M weights (11264 x 2048: 15.3 vs 17.6 us in the
+# library; 22528 x 4096: 52.0 vs 45.1).  Anything between: always.
+THIN_MAX_M = 64
+THIN_ROW_MAX_K, THIN_ROW_MAX_W = 3072, 1 << 26
+THIN_BATCH_MAX_W = 24 << 20
+
+
+def thin_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Can and should the thin GEMM run x [M, K] @ w [N, K]^T?"""
+    if not (x.is_cuda and x.dim() == 2 and w.dim() == 2 and 0 < x.shape[0] <= THIN_MAX_M
+            and x.dtype == w.dtype and x.dtype in (torch.bfloat16, torch.float16)
+            and x.shape[1] == w.shape[1] and w.is_contiguous() and x.stride(1) == 1
+            and x.stride(0) % 8 == 0 and x.stride(0) >= x.shape[1]):
+        return False
+    (M, K), N = x.shape, w.shape[0]
+    if K == 0 or K % 64 or N % 4 or (x.data_ptr() | w.data_ptr()) % 16 or K >= 1 << 24:
+        return False
+    if M == 1:
+        return K <= THIN_ROW_MAX_K and N * K < THIN_ROW_MAX_W
+    return M <= 32 or N * K <= THIN_BATCH_MAX_W
+
+
+def thin_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
+    """x [M, K] @ w [N, K]^T (+ ``bias`` [N]) on the thin GEMM kernel, fp32 accumulation; the result
+    in x's dtype or (``out_dtype``) fp32.  Callers ask ``thin_ok`` first."""
+    from ._seqmix import DT, call, use_seqmix
+
+    use_seqmix(x)
+    (M, K), N = x.shape, w.shape[0]
+    assert bias is None or (bias.dtype == x.dtype and bias.shape == (N,) and bias.stride(0) == 1)
+    y = torch.empty(M, N, device=x.device, dtype=out_dtype or x.dtype)
+    call("sm_thin_gemm", DT[x.dtype], x, x.stride(0), w, bias, y, N, M, N, K,
+         int(y.dtype == torch.float32))
+    return y
+
+
+def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``F.linear`` of a served stack: few rows on the weight-streaming kernels (thin GEMM; GEMV for
+    one row of a large matrix), the library otherwise."""
+    if thin_ok(x, w) and (bias is None or bias.dtype == x.dtype):
+        return thin_linear(x, w, bias)
+    if bias is None and x.dim() == 2 and x.shape[0] == 1 and skinny_ok(x, w):
+        y = torch.empty(1, w.shape[0], device=x.device, dtype=x.dtype)
+        native().skinny_gemm(x, w, y)
+        return y
+    return F.linear(x, w, bias)
 
 
 # Decode batches 5..256: the decode-batch MFMA GEMM (kernels/decode_gemm.hip) where the measured
@@ -211,6 +260,8 @@ def mm_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 def linear_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x [M, K] @ w[N, K]^T -> [M, N]."""
+    if use_native(x) and thin_ok(x, w):
+        return thin_linear(x, w)
     if skinny_ok(x, w):
         y = torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=x.dtype)
         native().skinny_gemm(x, w, y)

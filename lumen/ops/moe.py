@@ -49,14 +49,21 @@ def route_topk(z: torch.Tensor, top: int) -> torch.Tensor:
     return out
 
 
-def router_logits(h: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """fp32 router logits h [T, W] @ w [E, W]^T for h and w in the model dtype.  16-bit values
-    multiply exactly in fp32, so on the GPU the product runs on the matrix cores with fp32
-    accumulation and an fp32 result -- the arithmetic of an fp32 GEMM on the widened operands
+def router_logits(h: torch.Tensor, w: torch.Tensor,
+                  bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """fp32 router logits h [T, W] @ w [E, W]^T (+ ``bias`` [E]) for operands in the model dtype.
+    16-bit values multiply exactly in fp32, so on the GPU the product runs on the matrix cores with
+    fp32 accumulation and an fp32 result -- the arithmetic of an fp32 GEMM on the widened operands
     without the pass that widens them."""
+    from .gemm import thin_linear, thin_ok
+
+    if thin_ok(h, w) and (bias is None or bias.dtype == h.dtype):
+        return thin_linear(h, w, bias, torch.float32)
     if h.is_cuda and h.dtype == w.dtype and h.dtype in (torch.bfloat16, torch.float16):
-        return torch.mm(h, w.t(), out_dtype=torch.float32)
-    return h.float() @ w.float().t()
+        z = torch.mm(h, w.t(), out_dtype=torch.float32)
+    else:
+        z = h.float() @ w.float().t()
+    return z if bias is None else z.add_(bias)
 
 
 def route_groups_ref(z, correction, top, n_groups, keep, scale, sum_eps=1e-20, rank_top=2,
@@ -211,7 +218,9 @@ def _act(z, wts, E, ff, ffs, act, gated, weigh):
 
 def moe_dense(h, wts, gu_w, down_w, E: int, ff: int, ffs: int, act="silu", gated: bool = True,
               weigh: str = "output") -> torch.Tensor:
-    return F.linear(_act(F.linear(h, gu_w), wts, E, ff, ffs, act, gated, weigh), down_w)
+    from .gemm import project
+
+    return project(_act(project(h, gu_w), wts, E, ff, ffs, act, gated, weigh), down_w)
 
 
 def moe_grouped(h, wts, gu_w, down_w, E: int, ff: int, ffs: int, act="silu", gated: bool = True,

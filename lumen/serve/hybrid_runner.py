@@ -48,6 +48,7 @@ from ..ops.attention import (chunk_sink_attention, diff_head_combine, head_norm_
                              write_key_cache)
 from ..ops.conv import dyt_canon, short_conv
 from ..ops.embedding import embed_positions, embed_scaled, gated_token_slice, soft_cap
+from ..ops.gemm import project
 from ..ops.moe import (ClampedGate, gated_act, moe, route_groups, route_topk, router_logits,
                        scaled_act)
 from ..ops.norm import (SPLIT, depth_mix_norm, dyt, dyt_residual, embed_rms, gated_rms_norm,
@@ -127,8 +128,8 @@ class HybridWeights:
                             gu += [t(y + "shared.gate"), t(y + "shared.up")]
                             dn.append(t(y + "shared.down"))
                         L.ff = dict(E=E, top=top, ff=ffe, ffs=ffs, gu=torch.cat(gu, 0).contiguous(),
-                                    down=torch.cat(dn, 1).contiguous(), router=f32(y + "router"),
-                                    router_b=f32(y + "router.b"))
+                                    down=torch.cat(dn, 1).contiguous(), router=t(y + "router").detach(),
+                                    router_b=t(y + "router.b").detach())
                 self.layers.append(L)
 
 
@@ -140,7 +141,7 @@ class HybridWeights:
         return run_layers(self, st, tokens, seg, observe)
 
     def head(self, x: torch.Tensor) -> torch.Tensor:
-        return F.linear(dyt(x, self.final, self.dtype), self.lm_head)
+        return project(dyt(x, self.final, self.dtype), self.lm_head)
 
 
 class HybridState:
@@ -258,7 +259,7 @@ def run_layers(w: HybridWeights, st: HybridState, tokens: torch.Tensor, seg: Seg
         h = dyt_canon(x, L.norms["norm1"], L.canon, st.tail[i], seg, dt)
         if L.kind == "attention":
             H, G, D = m["heads"], m["kv_heads"], m["dim"]
-            qk = F.linear(h, L.w["qk"])
+            qk = project(h, L.w["qk"])
             write_key_cache(qk[:, H * D:], st.keys[i], seg.cache_slots)
             o = chunk_sink_attention(qk[:, :H * D], st.keys[i], seg, H, G, D, float(m["scale"]),
                                      int(m["mask"]["size"]), eps, sink=True)
@@ -266,18 +267,18 @@ def run_layers(w: HybridWeights, st: HybridState, tokens: torch.Tensor, seg: Seg
             H, D = m["heads"], m["dim"]
             mix = token_shift(h, L.w["mu"], st.prev[i], seg)
             rkvg = torch.bmm(mix[:4], L.w["rkvg"])
-            wl = F.linear(torch.tanh(F.linear(mix[4], L.w["w1"])), L.w["w2"])
+            wl = project(torch.tanh(project(mix[4], L.w["w1"])), L.w["w2"])
             o = wkv_scan(rkvg[0], rkvg[1], rkvg[2], wl, rkvg[3], L.w["w0"], L.w["u"], L.w["norm"],
                          st.S[i], seg, H, D, eps)
         else:
             H, D = m["heads"], m["dim"]
             HD = H * D
-            z = F.linear(h, L.w["in"])
-            wl = F.linear(torch.tanh(z[:, 5 * HD:]), L.w["w2"])
+            z = project(h, L.w["in"])
+            wl = project(torch.tanh(z[:, 5 * HD:]), L.w["w2"])
             o = delta_scan(z[:, :HD], z[:, HD:2 * HD], z[:, 2 * HD:3 * HD], wl,
                            z[:, 4 * HD:5 * HD], z[:, 3 * HD:4 * HD], L.w["w0"], L.w["a_b"],
                            L.w["norm"], st.S[i], seg, H, D, eps, DELTA_DECAY, DELTA_KEY_EPS)
-        y = F.linear(o, L.w["o"])
+        y = project(o, L.w["o"])
         f = L.ff
         if f is None:
             x, _ = dyt_residual(x, y, L.norms["norm1b"], None, dt)
@@ -285,11 +286,11 @@ def run_layers(w: HybridWeights, st: HybridState, tokens: torch.Tensor, seg: Seg
             x, h2 = dyt_residual(x, y, L.norms["norm1b"], L.norms["norm2"], dt)
             if f["E"]:
                 # the router in fp32, on the (possibly 16-bit rounded) normed row
-                z = torch.addmm(f["router_b"], h2.float(), f["router"].t())
+                z = router_logits(h2, f["router"], f["router_b"])
                 y2 = moe(h2, route_topk(z, f["top"]), f["gu"], f["down"], f["E"], f["top"],
                          f["ff"], f["ffs"])
             else:
-                y2 = F.linear(gated_act(F.linear(h2, f["gu"]), None, 0, 0, f["ffs"]), f["down"])
+                y2 = project(gated_act(project(h2, f["gu"]), None, 0, 0, f["ffs"]), f["down"])
             x, _ = dyt_residual(x, y2, L.norms["norm2b"], None, dt)
         if observe is not None:
             observe(i, x)
@@ -392,7 +393,7 @@ class DalavikWeights:
 
     def head(self, x: torch.Tensor) -> torch.Tensor:
         h = group_rms_norm(x, self.final, self.cfg.norm_groups, self.cfg.rms_norm_eps, self.dtype)
-        return F.linear(h, self.lm_head)
+        return project(h, self.lm_head)
 
 
 class DalavikState:
@@ -441,12 +442,12 @@ def run_dalavik_layers(w: DalavikWeights, st: DalavikState, tokens: torch.Tensor
         if L.kind == "latent_attention":
             H, D, Dr, Dv, R, Q = (m["heads"], m["dim"], m["rot_dim"], m["vdim"], m["kv_rank"],
                                   m["q_rank"])
-            z = F.linear(xb, L.w["down"])
+            z = project(xb, L.w["down"])
             if L.kv_layer == i:
                 latent_write(z[:, Q:], L.w["dkv_norm"], L.w["inv_freq"], seg.positions,
                              seg.cache_slots, st.lat[i], R, m["rot"]["dims"], eps, st.latT[i])
             cache = st.lat[L.kv_layer]
-            q = F.linear(group_rms_norm(z[:, :Q], L.w["dq_norm"], 1, eps, dt), L.w["uq"])
+            q = project(group_rms_norm(z[:, :Q], L.w["dq_norm"], 1, eps, dt), L.w["uq"])
             rotate_interleaved_(q, seg.positions, H, D + Dr, D, m["rot"]["dims"], L.w["inv_freq"])
             q3 = q.view(T, H, D + Dr)
             qa = torch.bmm(q3[:, :, :D].transpose(0, 1), L.w["uk"])              # [H, T, R]
@@ -457,7 +458,7 @@ def run_dalavik_layers(w: DalavikWeights, st: DalavikState, tokens: torch.Tensor
             torch.bmm(ol, L.w["uvT"], out=o.transpose(0, 1))
         else:
             H, G, D, Dv = m["heads"], m["kv_heads"], m["dim"], m["vdim"]
-            qkv = F.linear(xb, L.w["qkv"], L.w["qkv_b"])
+            qkv = project(xb, L.w["qkv"], L.w["qkv_b"])
             head_norm_write(qkv, L.w["q.norm"], L.w["k.norm"], seg.cache_slots, st.k[i], st.v[i],
                             H, G, D, Dv, eps)
             qt = m.get("q_temp")
@@ -466,18 +467,18 @@ def run_dalavik_layers(w: DalavikWeights, st: DalavikState, tokens: torch.Tensor
                           float(m["scale"]), float(m.get("softcap") or 0.0),
                           (float(qt["coef"]), int(qt["every"])) if qt else None,
                           L.w["r1"], L.w["r2"], L.w["talk"], L.w["sink"])
-        y = F.linear(o.view(T, H * Dv), L.w["o"])
+        y = project(o.view(T, H * Dv), L.w["o"])
         x, xc = group_rms_residual(x, y, L.norm1, groups, eps, cast)
         xb = xc if cast is not None else x
         f = L.ff
         if f is not None:
-            y = F.linear(gated_act(F.linear(xb, f["gu"]), None, 0, 0, f["ff"], "relu"), f["down"])
+            y = project(gated_act(project(xb, f["gu"]), None, 0, 0, f["ff"], "relu"), f["down"])
             x, xc = group_rms_residual(x, y, f["norm"], groups, eps, cast)
             xb = xc if cast is not None else x
         sd = L.side
         if sd is not None:
-            g = gated_token_slice(F.linear(xb, sd["gate"]), w.side_embed, tokens, sd["col0"])
-            x, xc = group_rms_residual(x, F.linear(g, sd["proj"]), sd["norm"], 1, eps, cast)
+            g = gated_token_slice(project(xb, sd["gate"]), w.side_embed, tokens, sd["col0"])
+            x, xc = group_rms_residual(x, project(g, sd["proj"]), sd["norm"], 1, eps, cast)
             xb = xc if cast is not None else x
         if observe is not None:
             observe(i, x)
@@ -573,7 +574,7 @@ class FanopelWeights:
         return run_fanopel_layers(self, st, tokens, seg, observe)
 
     def head(self, x: torch.Tensor) -> torch.Tensor:
-        return F.linear(weight_layer_norm(x, self.final, self.cfg.rms_norm_eps, self.dtype),
+        return project(weight_layer_norm(x, self.final, self.cfg.rms_norm_eps, self.dtype),
                         self.lm_head)
 
 
@@ -605,7 +606,7 @@ def run_fanopel_layers(w: FanopelWeights, st: FanopelState, tokens: torch.Tensor
     for i, L in enumerate(w.layers):
         m = L.m
         H, G, D = m["heads"], m["kv_heads"], m["dim"]
-        z = F.linear(h, L.w["qkg"])
+        z = project(h, L.w["qkg"])
         row_norm_write(z, L.w["q.norm"], L.w["k.norm"], seg.cache_slots, st.k[i], st.v[i],
                        H * D, G * D, eps)
         o = torch.empty(T, H, D, dtype=dt, device=x.device)
@@ -614,7 +615,7 @@ def run_fanopel_layers(w: FanopelWeights, st: FanopelState, tokens: torch.Tensor
                       float(m["scale"]), float(m.get("softcap") or 0.0), slopes=L.w["slopes"],
                       window=int(mask["size"]), keep_first=int(mask.get("keep_first", 0)),
                       gate=z[:, (H + G) * D:(H + G) * D + H])
-        y = F.linear(o.view(T, H * D), L.w["o"])
+        y = project(o.view(T, H * D), L.w["o"])
         nxt = w.layers[i + 1].norm1 if i + 1 < n_layers else None
         f = L.ff
         if f is None:
@@ -841,7 +842,7 @@ def run_foderax_layers(w: FoderaxWeights, st: FoderaxState, tokens: torch.Tensor
         if L.kind == "parallel":
             a = m["left"]
             H, G, D, Dv, Wd = a["heads"], a["kv_heads"], a["dim"], a["vdim"], m["right"]["width"]
-            z = F.linear(h, L.w["in"])
+            z = project(h, L.w["in"])
             rotary_write(z, seg.positions, seg.cache_slots, st.k[i], st.v[i], H, G, D,
                          int(a["rot"]["dims"]), L.w["inv_freq"], True)
             o = torch.empty(T, H, Dv, dtype=dt, device=dev)
@@ -850,13 +851,13 @@ def run_foderax_layers(w: FoderaxWeights, st: FoderaxState, tokens: torch.Tensor
             c0 = (H + G) * D + G * Dv
             r = min_gru_scan(z[:, c0:c0 + 3 * Wd], L.w["b_z"], L.w["b_x"], st.S[i], seg, Wd,
                              w.shift)
-            ys = [F.linear(o.view(T, H * Dv), L.w["o_l"]), F.linear(r, L.w["o_r"])]
+            ys = [project(o.view(T, H * Dv), L.w["o_l"]), project(r, L.w["o_r"])]
         elif L.kind == "latent_attention":
             H, D, Dv, R, Q = m["heads"], m["dim"], m["vdim"], m["kv_rank"], m["q_rank"]
-            z = F.linear(h, L.w["in"])
+            z = project(h, L.w["in"])
             latent_write(z[:, Q:Q + R], L.w["dkv_norm"], None, seg.positions, seg.cache_slots,
                          st.lat[i], R, 0, eps, st.latT[i])
-            q = F.linear(group_rms_norm(z[:, :Q], L.w["dq_norm"], 1, eps, dt), L.w["uq"])
+            q = project(group_rms_norm(z[:, :Q], L.w["dq_norm"], 1, eps, dt), L.w["uq"])
             qa = torch.bmm(q.view(T, H, D).transpose(0, 1), L.w["uk"])          # [H, T, R]
             ol = torch.empty(H, T, R, dtype=dt, device=dev)
             row_attention(qa.transpose(0, 1), None, st.lat[i], st.lat[i], R, ol.transpose(0, 1),
@@ -864,11 +865,11 @@ def run_foderax_layers(w: FoderaxWeights, st: FoderaxState, tokens: torch.Tensor
                           gate=z[:, Q + R:Q + R + H])
             o = torch.empty(T, H, Dv, dtype=dt, device=dev)
             torch.bmm(ol, L.w["uvT"], out=o.transpose(0, 1))
-            ys = [F.linear(o.view(T, H * Dv), L.w["o"])]
+            ys = [project(o.view(T, H * Dv), L.w["o"])]
         else:
             H, G, D, Dv = m["heads"], m["kv_heads"], m["dim"], m["vdim"]
             own = L.kv_layer == i
-            z = F.linear(h, L.w["in"], L.w["in_b"])
+            z = project(h, L.w["in"], L.w["in_b"])
             rotary_write(z, seg.positions, seg.cache_slots, st.k[i], st.v[i], 2 * H,
                          2 * G if own else 0, D, int(m["rot"]["dims"]), L.w["inv_freq"], False)
             av = torch.empty(T, 2 * H, Dv, dtype=dt, device=dev)
@@ -877,7 +878,7 @@ def run_foderax_layers(w: FoderaxWeights, st: FoderaxState, tokens: torch.Tensor
             g0 = 2 * H * D + ((2 * G * D + G * Dv) if own else 0)
             o = diff_head_combine(av.view(T, 2 * H * Dv), L.c["lam"], 1.0 - float(m["diff"]), eps,
                                   z[:, g0:g0 + H * Dv], G, H // G, Dv)
-            ys = [F.linear(o, L.w["o"])]
+            ys = [project(o, L.w["o"])]
         scales = list(L.w["scales"])
         f = L.ff
         if f is not None:
@@ -1064,7 +1065,7 @@ def _silonex_mixer(L: SilonexLayerW, w: SilonexWeights, st: SilonexState, n: int
 
     m, dt, eps = L.m, w.dtype, w.cfg.rms_norm_eps
     T = h.shape[0]
-    z = F.linear(h, L.w["in"])
+    z = project(h, L.w["in"])
     H, Dk, Dv, C, _ = _silonex_state_sizes(L.kind, m)
     if L.kind == "parallel":
         a, r = m["left"], m["right"]
@@ -1082,20 +1083,20 @@ def _silonex_mixer(L: SilonexLayerW, w: SilonexWeights, st: SilonexState, n: int
                       (z[:, a0:a0 + H], L.w["A_log"], L.w["dt_bias"]), beta=z[:, b0:b0 + H],
                       rep=H // r["kv_heads"], key_eps=w.unit_eps, q_scale=float(Dk) ** -0.5)
         y = gated_rms_norm(y, z[:, g0:g0 + H * Dv], L.w["norm"], H, eps, "silu", False)
-        return [F.linear(o.view(T, Ha * Da), L.w["o_l"]), F.linear(y, L.w["o_r"])]
+        return [project(o.view(T, Ha * Da), L.w["o_l"]), project(y, L.w["o_r"])]
     if L.kind == "lightning":
         q0, k0, v0, g0 = L.cols
         y = head_scan(z[:, q0:q0 + H * Dk], z[:, k0:k0 + H * Dk], z[:, v0:v0 + H * Dv], st.S[n],
                       seg, H, Dk, Dv, L.w["log_decay"], silu_in=True)
         y = gated_rms_norm(y, z[:, g0:g0 + H * Dv], L.w["norm"], 1, eps, "sigmoid", False)
-        return [F.linear(y, L.w["o"])]
+        return [project(y, L.w["o"])]
     inner, GN = H * Dv, m["groups"] * Dk
     c = short_conv(z[:, inner:inner + C], L.w["conv"], L.w["conv.b"], st.tail[n], seg)
     y = head_scan(c[:, inner + GN:], c[:, inner:inner + GN], c[:, :inner], st.S[n], seg, H, Dk, Dv,
                   (z[:, inner + C:inner + C + H], L.w["A_log"], L.w["dt_bias"]), skip=L.w["D"],
                   rep=H // m["groups"])
     y = gated_rms_norm(y, z[:, :inner], L.w["norm"], int(m["norm_groups"]), eps, "silu", True)
-    return [F.linear(y, L.w["o"])]
+    return [project(y, L.w["o"])]
 
 
 def run_silonex_layers(w: SilonexWeights, st: SilonexState, tokens: torch.Tensor, seg: SegBatch,
@@ -1117,7 +1118,7 @@ def run_silonex_layers(w: SilonexWeights, st: SilonexState, tokens: torch.Tensor
                 pair = (L.w["out_l"], L.w["out_r"], eps)
         else:
             f = L.ff
-            ys = [F.linear(gated_act(F.linear(h, f["gu"]), None, 0, 0, f["ff"]), f["down"])]
+            ys = [project(gated_act(project(h, f["gu"]), None, 0, 0, f["ff"]), f["down"])]
         _, out, mix = L.hc[q]
         last = k + 1 == len(subs)
         if last:
@@ -1280,25 +1281,25 @@ def _tazulix_mixer(L: TazulixLayerW, w: TazulixWeights, st: TazulixState, n: int
     H, D, Dv = m["heads"], m["dim"], m["vdim"]
     if L.kind == "attention":
         G = m["kv_heads"]
-        z = F.linear(h, L.w["in"], L.w["in_b"])
+        z = project(h, L.w["in"], L.w["in_b"])
         row_norm_rotary_write(z, L.w["q.norm"], L.w["k.norm"], seg.positions, seg.cache_slots,
                               st.k[n], st.v[n], H, G, D, Dv, L.rot_dims, L.w["inv_freq"], L.amp,
                               eps)
         o = torch.empty(T, H, Dv, dtype=dt, device=h.device)
         row_attention(z[:, :H * D].view(T, H, D), None, st.k[n], st.v[n], Dv, o, seg, H, G,
                       float(m["scale"]))
-        return F.linear(o.view(T, H * Dv), L.w["o"])
-    z = F.linear(h, L.w["in"])
+        return project(o.view(T, H * Dv), L.w["o"])
+    z = project(h, L.w["in"])
     q0, k0, v0, g0 = L.cols
     y = head_scan(z[:, q0:q0 + H * D], z[:, k0:k0 + H * D], z[:, v0:v0 + H * Dv], st.S[n], seg, H,
                   D, Dv, L.w["log_decay"], silu_in=True)
     y = gated_rms_norm(y, z[:, g0:g0 + H * Dv], L.w["norm"], 1, eps, "sigmoid", False)
-    return F.linear(y, L.w["o"])
+    return project(y, L.w["o"])
 
 
 def _tazulix_ff(f: dict, h) -> torch.Tensor:
     if not f["E"]:
-        return F.linear(scaled_act(F.linear(h, f["up"]), None, 0, 0, f["ff"], "relu2"), f["down"])
+        return project(scaled_act(project(h, f["up"]), None, 0, 0, f["ff"], "relu2"), f["down"])
     # the router in fp32, on the (possibly 16-bit rounded) normed row
     r = route_groups(router_logits(h, f["router"]), None, f["top"], 1, 1, normalize=False)
     return moe(h, r, f["gu"], f["down"], f["E"], f["top"], f["ff"], f["ffs"], f["act"],

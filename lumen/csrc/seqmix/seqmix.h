@@ -34,6 +34,37 @@ template <> __device__ __forceinline__ void store4<float>(float* __restrict__ p,
   *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
 }
 
+// the gate's activation: 0 SiLU, 1 ReLU, 2 tanh-GELU, 3 squared ReLU
+__device__ __forceinline__ float gate_act(float g, int act) {
+  if (act == 3) {
+    const float r = fmaxf(g, 0.f);
+    return r * r;
+  }
+  return act == 0 ? silu_f(g) : act == 1 ? fmaxf(g, 0.f) : gelu_tanh_f(g);
+}
+
+struct GateForm {
+  int act;                                  // as above; 4: clamped, with the constants below
+  int weigh_in;                             // the weight multiplies gate and up, not the result
+  float limit, limit_s, slope, shift;       // limit: experts; limit_s: the unweighted block
+};
+
+// the gated activation of one (gate, up) pair with routing weight w
+__device__ __forceinline__ float gated_f(float g, float u, float w, bool shared,
+                                         const GateForm& f) {
+  if (f.weigh_in) { g *= w; u *= w; }
+  float y;
+  if (f.act == 4) {
+    const float lim = shared ? f.limit_s : f.limit;
+    g = fminf(g, lim);
+    u = fminf(fmaxf(u, -lim), lim);
+    y = g * sigmoid_f(f.slope * g) * (u + f.shift);
+  } else {
+    y = gate_act(g, f.act) * u;
+  }
+  return f.weigh_in ? y : y * w;
+}
+
 }  // namespace lumen
 
 // run `CALL(T)` with T = float / fp16 / bf16 for dtype code `dt`

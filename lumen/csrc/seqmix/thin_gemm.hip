@@ -25,6 +25,16 @@
 //   M = 64: 6.5 / 9.0, 15.3 / 17.6, 17.4 / 18.4, 29.4 / 27.9, 13.3 / 14.3, 52.0 / 45.1, 33.9 / 34.9
 //   M = 1:  3.8 / 8.3 (GEMV 4.4), 9.8 / 16.1 (10.5), 7.3 / 11.7 (6.6), 22.4 / 32.0 (22.9), 7.5 / 12.1
 //           (8.1), 30.7 / 51.6 (28.5), 17.2 / 20.6 (17.2)
+// The activation form (thin_act): a workgroup's tile is 16 activation columns -- their gate rows and
+// their up rows -- so act(gate) * up, times the row's routing weight, is formed from the fp32 sums and
+// the [M, 2 ff] intermediate and its kernel are gone.  Routed experts: W holds every expert, and a
+// step of a few rows uses few of them.  `sparse` reads the routing weights first and streams the
+// weights of experts some row chose only -- in the first projection by tile, in the second (K runs
+// over [experts x ff]) by k stage; what an unchosen expert would add is zero.
+// Measured like the above, a whole feed-forward against two library GEMMs and the activation kernel:
+//   dense 2048 -> 5632 (gated): 1 row 18.3 / 28.8 us, 8 rows 22.8 / 31.8, 32 rows 27.9 / 35.8
+//   16 experts of 1408, top 3, and a shared one: 1 row 17.5 / 113.9, 8 rows 49.3 / 122.3, 32 rows 88.2 /
+//   144.6; width 4096, experts of 2816: 8 rows 189.4 / 269.6, 32 rows 248.4 / 406.8
 // From 33 rows on every tile re-reads more x than W, so the widest matrices stay with the library
 // there; at M = 1 the GEMV stays ahead on long rows (ops/gemm.py has the rule).
 #include "seqmix.h"
@@ -77,42 +87,115 @@ struct ThinArgs {
   void* y;
   int M, N, K;
   long long ldx, ldy;
-  int tiles;       // ceil(N / (16 RT))
+  int tiles;       // plain: ceil(N / (16 RT))
   int out32;       // fp32 result
+  // routed experts: weights [M, E] fp32, blocks of ff columns and a last one of ffs (E = 0: just it)
+  const float* wts;
+  int E, ff, ffs;
+  int sparse;      // skip experts that no row chose
+  GateForm form;
 };
 
-// XP: pieces of 8 x rows (1, 2, 4, 8: M <= 8, 16, 32, 64)
-template <typename T, int RT, int XP, int NW, int D>
+constexpr int kMaxWts = 2048;     // routing weights held in LDS (M * E)
+
+// the i-th set bit of a mask
+__device__ __forceinline__ int nth_bit(unsigned long long m, int i) {
+  for (; i > 0; --i) m &= m - 1;
+  return __builtin_ctzll(m);
+}
+
+// XP: pieces of 8 x rows (1, 2, 4, 8: M <= 8, 16, 32, 64).  ACT: 0 plain, 1 activation of RT = 1 row
+// tile (no gate), 2 gated (RT = 2: the tile's gate rows, its up rows).
+template <typename T, int RT, int XP, int NW, int D, int ACT>
 __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
   constexpr int MT = XP < 2 ? 1 : XP / 2;
   constexpr int WB = RT * 16 * ROWB, SB = WB + XP * 8 * ROWB;
   constexpr int G = 2 * RT + XP;                   // DMA instructions of a stage
   constexpr int PB = RT * MT * 1024;               // a wave's partial tile
+  constexpr int WTS = XP <= 4 ? kMaxWts * 4 : 0;
   static_assert(G * (D - 1) < 64, "stages in flight");
-  static_assert(NW * D * SB + 2 * NW * PB <= 163840, "LDS");
-  __shared__ __attribute__((aligned(16))) char lds[NW * D * SB + 2 * NW * PB];
+  static_assert(ACT == 0 || RT == ACT, "an activation tile is one row tile per operand");
+  static_assert(NW * D * SB + 2 * NW * PB + WTS <= 163840, "LDS");
+  __shared__ __attribute__((aligned(16))) char lds[NW * D * SB + 2 * NW * PB + WTS];
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   char* ring = lds + wid * D * SB;
   char* part = lds + NW * D * SB;                  // [2][NW][PB]: this tile's and the last one's
+  float* wts = reinterpret_cast<float*>(part + 2 * NW * PB);
   const T* x = (const T*)p.x;
   const T* W = (const T*)p.W;
-  const int kt = p.K / BK;
+
+  // experts some row chose (every one of them unless `sparse`)
+  unsigned long long chosen = 0;
+  int n_chosen = 0;
+  if (WTS > 0 && p.E > 0) {
+    if (p.wts != nullptr) {
+      for (int i = threadIdx.x; i < p.M * p.E; i += 64 * NW) wts[i] = p.wts[i];
+      __syncthreads();
+    }
+    if (p.sparse) {
+      bool on = false;
+      if (lane < p.E)
+        for (int m = 0; m < p.M; ++m) on |= !(wts[m * p.E + lane] == 0.f);
+      chosen = __ballot(on);
+      n_chosen = __popcll(chosen);
+    }
+  }
+  int tiles = p.tiles, kt = p.K / BK;
+  const int per = p.ff >> 4, ks = p.ff >> 6;       // tiles / k stages of an expert
+  if (p.sparse) {
+    if (ACT) tiles = n_chosen * per + (p.ffs >> 4);
+    else kt = n_chosen * ks + (p.ffs >> 6);
+  }
   const int k0 = kt * wid / NW, nk = kt * (wid + 1) / NW - k0;
-  const int mine = (p.tiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int mine = max(0, (tiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x);
   const int total = mine * nk;                     // stages this wave streams
   const int rr = lane >> 3, c = lane & 7;          // row within a piece, LDS chunk
+  // expert (E: the last block) and column of activation tile t
+  const auto block_of = [&](int t, int& e, int& col) {
+    const int i = per > 0 ? t / per : 0;
+    const int n = p.sparse ? n_chosen : p.E;
+    if (p.E > 0 && i < n) {
+      e = p.sparse ? nth_bit(chosen, i) : i;
+      col = (t - i * per) * 16;
+    } else {
+      e = p.E;
+      col = (t - n * per) * 16;
+    }
+  };
   int at_t = blockIdx.x, at_k = 0, issued = 0, put = 0;
+  int left = 0, seg = 0, kk = 0;                   // sparse second projection: place in the k walk
+  const auto seek = [&]() {                        // to this wave's first stage
+    if (ACT || !p.sparse) { kk = k0 * BK; return; }
+    seg = ks > 0 ? min(k0 / ks, n_chosen) : 0;
+    const int in = k0 - seg * ks;
+    left = seg < n_chosen ? ks - in : 0x7fffffff;
+    kk = (seg < n_chosen ? nth_bit(chosen, seg) : p.E) * p.ff + in * BK;
+  };
+  const T *Wa = W, *Wb = W;                        // first row of the tile's (gate | up) rows
+  int last = 0;
+  const auto seat = [&]() {
+    if constexpr (ACT == 0) {
+      Wa = W + (long long)at_t * (RT * 16) * p.K;
+      last = min(RT * 16, p.N - at_t * RT * 16) - 1;
+    } else {
+      int e, col;
+      block_of(at_t, e, col);
+      Wa = W + ((long long)e * RT * p.ff + col) * p.K;
+      Wb = Wa + (long long)(e < p.E ? p.ff : p.ffs) * p.K;
+      last = RT * 16 - 1;
+    }
+  };
+  seek();
+  if (total > 0) seat();
   const auto issue = [&]() {
     char* img = ring + put * SB;
-    const int kk = (k0 + at_k) * BK;
-    const T* Wt = W + (long long)at_t * (RT * 16) * p.K;
-    const int last = min(RT * 16, p.N - at_t * RT * 16) - 1;
 #pragma unroll
     for (int q = 0; q < 2 * RT; ++q) {
       const int r = 8 * q + rr;
-      dma16(Wt, ((unsigned)min(r, last) * (unsigned)p.K + kk + 8 * (c ^ swz(r))) * 2u,
-            img + 8 * q * ROWB);
+      const T* base = ACT == 2 && q >= 2 ? Wb : Wa;
+      const int row = ACT == 2 && q >= 2 ? r - 16 : min(r, last);
+      dma16(base, ((unsigned)row * (unsigned)p.K + kk + 8 * (c ^ swz(r))) * 2u, img + 8 * q * ROWB);
     }
 #pragma unroll
     for (int q = 0; q < XP; ++q) {
@@ -122,14 +205,26 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
     }
     put = put + 1 == D ? 0 : put + 1;
     ++issued;
-    if (++at_k == nk) { at_k = 0; at_t += gridDim.x; }
+    if (++at_k == nk) {
+      at_k = 0;
+      at_t += gridDim.x;
+      seek();
+      if (issued < total) seat();
+    } else {
+      kk += BK;
+      if (ACT == 0 && p.sparse && --left == 0) {
+        ++seg;
+        left = seg < n_chosen ? ks : 0x7fffffff;
+        kk = (seg < n_chosen ? nth_bit(chosen, seg) : p.E) * p.ff;
+      }
+    }
   };
 #pragma unroll
   for (int d = 0; d < D - 1; ++d)
     if (issued < total) issue();
   const int lr = lane & 15, lg = lane >> 4;
   int get = 0, done = 0, buf = 0;
-  for (int t = blockIdx.x; t < p.tiles; t += gridDim.x) {
+  for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
     f32x4 acc[RT][MT];
 #pragma unroll
     for (int i = 0; i < RT; ++i)
@@ -175,34 +270,57 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    for (int q = wid; q < RT * MT; q += NW) {
-      const int i = q / MT, j = q - i * MT;
+    const auto sum = [&](int q) {
       f32x4 v = *reinterpret_cast<const f32x4*>(pb + q * 1024 + lane * 16);
 #pragma unroll
       for (int w = 1; w < NW; ++w)
         v += *reinterpret_cast<const f32x4*>(pb + w * PB + q * 1024 + lane * 16);
-      const int m = 16 * j + lr, n = t * RT * 16 + 16 * i + 4 * lg;
-      if (m >= p.M || n >= p.N) continue;
-      if (p.bias != nullptr) {
-        const T* b = (const T*)p.bias + n;
+      return v;
+    };
+    if constexpr (ACT == 0) {
+      for (int q = wid; q < RT * MT; q += NW) {
+        const int i = q / MT, j = q - i * MT;
+        f32x4 v = sum(q);
+        const int m = 16 * j + lr, n = t * RT * 16 + 16 * i + 4 * lg;
+        if (m >= p.M || n >= p.N) continue;
+        if (p.bias != nullptr) {
+          const T* b = (const T*)p.bias + n;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] += to_f32(b[e]);
+          for (int e = 0; e < 4; ++e) v[e] += to_f32(b[e]);
+        }
+        if (p.out32)
+          *reinterpret_cast<f32x4*>((float*)p.y + (long long)m * p.ldy + n) = v;
+        else
+          *reinterpret_cast<uint2*>((T*)p.y + (long long)m * p.ldy + n) =
+              make_uint2(pk2<T>(v[0], v[1]), pk2<T>(v[2], v[3]));
       }
-      if (p.out32)
-        *reinterpret_cast<f32x4*>((float*)p.y + (long long)m * p.ldy + n) = v;
-      else
-        *reinterpret_cast<uint2*>((T*)p.y + (long long)m * p.ldy + n) =
-            make_uint2(pk2<T>(v[0], v[1]), pk2<T>(v[2], v[3]));
+    } else {
+      int e, col;
+      block_of(t, e, col);
+      for (int j = wid; j < MT; j += NW) {
+        const int m = 16 * j + lr;
+        f32x4 g = sum(j), u = ACT == 2 ? sum(MT + j) : f32x4{1.f, 1.f, 1.f, 1.f};
+        if (m >= p.M) continue;
+        const float w = e < p.E ? wts[m * p.E + e] : 1.f;
+        float o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          o[i] = w == 0.f ? 0.f
+                 : ACT == 2 ? gated_f(g[i], u[i], w, e == p.E, p.form)
+                            : gate_act(g[i], p.form.act) * w;
+        *reinterpret_cast<uint2*>((T*)p.y + (long long)m * p.ldy + e * p.ff + col + 4 * lg) =
+            make_uint2(pk2<T>(o[0], o[1]), pk2<T>(o[2], o[3]));
+      }
     }
     buf ^= 1;
   }
 }
 
-template <typename T, int RT, int XP, int NW, int D>
+template <typename T, int RT, int XP, int NW, int D, int ACT = 0>
 hipError_t run(ThinArgs p, int per_cu, hipStream_t st) {
-  p.tiles = (p.N + 16 * RT - 1) / (16 * RT);
+  p.tiles = ACT ? (p.E * p.ff + p.ffs) / 16 : (p.N + 16 * RT - 1) / (16 * RT);
   const int grid = p.tiles < 256 * per_cu ? p.tiles : 256 * per_cu;
-  thin_kernel<T, RT, XP, NW, D><<<grid, 64 * NW, 0, st>>>(p);
+  thin_kernel<T, RT, XP, NW, D, ACT><<<grid, 64 * NW, 0, st>>>(p);
   return hipGetLastError();
 }
 
@@ -233,25 +351,76 @@ hipError_t pick(const ThinArgs& p, hipStream_t st) {
   return run<T, 1, 8, 4, 3>(p, 1, st);
 }
 
+template <typename T>
+hipError_t pick_act(const ThinArgs& p, int gated, hipStream_t st) {
+  if (gated) {
+    if (p.M <= 8) return run<T, 2, 1, 4, 4, 2>(p, 1, st);
+    if (p.M <= 16) return run<T, 2, 2, 4, 4, 2>(p, 1, st);
+    return run<T, 2, 4, 4, 3, 2>(p, 1, st);
+  }
+  if (p.M <= 8) return run<T, 1, 1, 4, 4, 1>(p, 2, st);
+  if (p.M <= 16) return run<T, 1, 2, 4, 4, 1>(p, 2, st);
+  return run<T, 1, 4, 4, 3, 1>(p, 1, st);
+}
+
+bool aligned(const void* x, const void* W, const void* y) {
+  return ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(W) |
+           reinterpret_cast<uintptr_t>(y)) & 15) == 0;
+}
+
 }  // namespace
 
 extern "C" {
 
 // M <= 64, K % 64 == 0, N % 4 == 0; W contiguous, x rows at stride ldx (% 8), y rows at stride ldy
-// (% 4); x, W and y aligned to 16 bytes.  bias [N] in the operands' dtype, or null.
+// (% 4); x, W and y aligned to 16 bytes.  bias [N] in the operands' dtype, or null.  wts (or null):
+// K is E blocks of ff and one of ffs (both % 64), and blocks whose column of wts [M, E] is zero add
+// nothing and are not read (M <= 32, M * E <= 2048, E <= 64).
 hipError_t sm_thin_gemm(int dt, const void* x, long long ldx, const void* W, const void* bias,
-                        void* y, long long ldy, int M, int N, int K, int out32, hipStream_t st) {
+                        void* y, long long ldy, int M, int N, int K, int out32, const float* wts,
+                        int E, int ff, int ffs, hipStream_t st) {
   if (M == 0 || N == 0) return hipSuccess;
   if (M < 0 || M > 64 || N < 4 || N % 4 || K < BK || K % BK || ldx < K || ldx % 8 || ldy < N ||
-      ldy % 4 ||
-      ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(W) |
-        reinterpret_cast<uintptr_t>(y)) & 15) != 0)
+      ldy % 4 || !aligned(x, W, y))
     return hipErrorInvalidValue;
   // lane offsets are 32-bit byte offsets from a tile's first row and from x
   if (64LL * K * 2 >= (1LL << 32) || 64LL * ldx * 2 >= (1LL << 32)) return hipErrorInvalidValue;
-  const ThinArgs p{x, W, bias, y, M, N, K, ldx, ldy, 0, out32};
+  if (wts != nullptr && (M > 32 || E < 1 || E > 64 || M * E > kMaxWts || ff < 64 || ff % 64 ||
+                         ffs < 0 || ffs % 64 || (long long)E * ff + ffs != K))
+    return hipErrorInvalidValue;
+  ThinArgs p{};
+  p.x = x; p.W = W; p.bias = bias; p.y = y;
+  p.M = M; p.N = N; p.K = K; p.ldx = ldx; p.ldy = ldy; p.out32 = out32;
+  if (wts != nullptr) { p.wts = wts; p.E = E; p.ff = ff; p.ffs = ffs; p.sparse = 1; }
   if (dt == kBF16) return pick<bf16>(p, st);
   if (dt == kF16) return pick<fp16>(p, st);
+  return hipErrorInvalidValue;
+}
+
+// y [M, E ff + ffs] = the activation of x @ W^T: W [E (1 + gated) ff + (1 + gated) ffs, K] holds per block
+// the gate rows then the up rows (or up rows alone), expert e's block weighed by wts [M, E] (see
+// GateForm), the last one not.  ff, ffs % 16; M <= 32, M * E <= 2048, E <= 64; the rest as above.
+// sparse: blocks of experts that no row chose are not written (ff, ffs % 64).
+hipError_t sm_thin_act(int dt, const void* x, long long ldx, const void* W, const float* wts, void* y,
+                       int M, int K, int E, int ff, int ffs, int gated, int sparse, int act,
+                       int weigh_in, float limit, float limit_s, float slope, float shift,
+                       hipStream_t st) {
+  if (M == 0) return hipSuccess;
+  const long long out = (long long)E * ff + ffs;
+  if (M < 0 || M > 32 || K < BK || K % BK || ldx < K || ldx % 8 || E < 0 || E > 64 || ff < 0 ||
+      ff % 16 || ffs < 0 || ffs % 16 || out < 16 || out >= (1LL << 27) || M * E > kMaxWts ||
+      (E > 0 && (wts == nullptr || ff < 16)) || (E == 0 && ff != 0) || act < 0 ||
+      act > (gated ? 4 : 3) || (weigh_in && !gated) || !aligned(x, W, y))
+    return hipErrorInvalidValue;
+  if (sparse && (E < 1 || ff % 64 || ffs % 64)) return hipErrorInvalidValue;
+  if (64LL * K * 2 >= (1LL << 32) || 64LL * ldx * 2 >= (1LL << 32)) return hipErrorInvalidValue;
+  ThinArgs p{};
+  p.x = x; p.W = W; p.y = y;
+  p.M = M; p.N = (int)out; p.K = K; p.ldx = ldx; p.ldy = out;
+  p.wts = wts; p.E = E; p.ff = ff; p.ffs = ffs; p.sparse = sparse;
+  p.form = GateForm{act, weigh_in, limit, limit_s, slope, shift};
+  if (dt == kBF16) return pick_act<bf16>(p, gated, st);
+  if (dt == kF16) return pick_act<fp16>(p, gated, st);
   return hipErrorInvalidValue;
 }
 

@@ -58,9 +58,12 @@ def thin_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def thin_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
-                out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
+                out_dtype: Optional[torch.dtype] = None, blocks: Optional[tuple] = None
+                ) -> torch.Tensor:
     """x [M, K] @ w [N, K]^T (+ ``bias`` [N]) on the thin GEMM kernel, fp32 accumulation; the result
-    in x's dtype or (``out_dtype``) fp32.  Callers ask ``thin_ok`` first."""
+    in x's dtype or (``out_dtype``) fp32.  ``blocks`` = (wts [M, E], E, ff, ffs): K is E blocks of ff
+    and one of ffs, and the blocks whose column of wts is all zero are taken as zero without being
+    read.  Callers ask ``thin_ok`` first."""
     from ._seqmix import DT, call, use_seqmix
 
     use_seqmix(x)
@@ -68,7 +71,7 @@ def thin_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] =
     assert bias is None or (bias.dtype == x.dtype and bias.shape == (N,) and bias.stride(0) == 1)
     y = torch.empty(M, N, device=x.device, dtype=out_dtype or x.dtype)
     call("sm_thin_gemm", DT[x.dtype], x, x.stride(0), w, bias, y, N, M, N, K,
-         int(y.dtype == torch.float32))
+         int(y.dtype == torch.float32), *(blocks or (None, 0, 0, 0)))
     return y
 
 

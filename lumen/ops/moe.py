@@ -216,11 +216,69 @@ def _act(z, wts, E, ff, ffs, act, gated, weigh):
     return scaled_act(z, wts, E, ff, ffs, act)
 
 
-def moe_dense(h, wts, gu_w, down_w, E: int, ff: int, ffs: int, act="silu", gated: bool = True,
-              weigh: str = "output") -> torch.Tensor:
-    from .gemm import project
+# Few-row steps: the first projection forms the activation in its epilogue (seqmix/thin_gemm.hip), one
+# launch and the [T, 2 ff] intermediate less.  ``top`` known and T * top <= SPARSE_ROWS * E: a row's experts
+# are few enough that reading the chosen ones only pays (uniform choices leave exp(-T top / E) of them out:
+# 5 % at 3, about the cost of reading the routing weights first).
+THIN_ACT_MAX_M, THIN_ACT_MAX_WTS, THIN_ACT_MAX_E = 32, 2048, 64
+SPARSE_ROWS = 3
 
+
+def thin_act_ok(h, wts, gu_w, E: int, ff: int, ffs: int, act="silu", gated: bool = True,
+                weigh: str = "output") -> bool:
+    """Can and should ``thin_act`` run the first projection and the activation in one kernel?"""
+    from .gemm import thin_ok
+
+    if not (h.is_cuda and h.dim() == 2 and 0 < h.shape[0] <= THIN_ACT_MAX_M and ff % 16 == 0
+            and ffs % 16 == 0 and E * ff + ffs > 0 and E <= THIN_ACT_MAX_E
+            and h.shape[0] * E <= THIN_ACT_MAX_WTS and (gated or isinstance(act, str))
+            and (E == 0 or (wts is not None and wts.dtype == torch.float32
+                            and wts.is_contiguous()))):
+        return False
+    k = 2 if gated else 1
+    if gu_w.shape[0] != k * (E * ff + ffs) or (weigh == "input" and not gated):
+        return False
+    # one row: thin_ok also says whether the thin kernel beats the GEMV; experts are mostly skipped
+    return thin_ok(h, gu_w[:16] if E and h.shape[0] == 1 else gu_w)
+
+
+def thin_act(h, gu_w, wts, E: int, ff: int, ffs: int, act="silu", gated: bool = True,
+             weigh: str = "output", sparse: bool = False) -> torch.Tensor:
+    """``gated_act`` (or ``scaled_act``) of h @ gu_w^T, [T, E * ff + ffs], from the fp32 sums.
+    ``sparse``: the blocks of experts that no row chose are left unwritten."""
+    from ._seqmix import DT, call, use_seqmix
+
+    use_seqmix(h)
+    if weigh not in ("output", "input"):
+        raise ValueError(f"unknown place of the routing weight {weigh!r}")
+    out = torch.empty(h.shape[0], E * ff + ffs, dtype=h.dtype, device=h.device)
+    code, c = (GATE_ACTS[act], (0.0,) * 4) if isinstance(act, str) else (
+        4, (act.limit, act.limit_shared, act.slope, act.shift))
+    call("sm_thin_act", DT[h.dtype], h, h.stride(0), gu_w, wts, out, h.shape[0], h.shape[1], E, ff,
+         ffs, int(gated), int(sparse), code, int(weigh == "input"), *c)
+    return out
+
+
+def moe_dense(h, wts, gu_w, down_w, E: int, ff: int, ffs: int, act="silu", gated: bool = True,
+              weigh: str = "output", top: Optional[int] = None) -> torch.Tensor:
+    """``top`` (optional): every row has at most that many non-zero weights."""
+    from .gemm import project, thin_linear
+
+    if thin_act_ok(h, wts, gu_w, E, ff, ffs, act, gated, weigh):
+        sparse = (top is not None and 0 < E and h.shape[0] * top <= SPARSE_ROWS * E
+                  and ff % 64 == 0 and ffs % 64 == 0 and down_w.is_contiguous()
+                  and down_w.shape[0] % 4 == 0 and down_w.data_ptr() % 16 == 0)
+        a = thin_act(h, gu_w, wts, E, ff, ffs, act, gated, weigh, sparse)
+        if sparse:
+            return thin_linear(a, down_w, blocks=(wts, E, ff, ffs))
+        return project(a, down_w)
     return project(_act(project(h, gu_w), wts, E, ff, ffs, act, gated, weigh), down_w)
+
+
+def feed_forward(h, gu_w, down_w, ff: int, act="silu", gated: bool = True) -> torch.Tensor:
+    """Dense feed-forward W_down (act(W_gate h) * W_up h) ([gate | up] rows stacked in ``gu_w``), or
+    without a gate W_down act(W_up h)."""
+    return moe_dense(h, None, gu_w, down_w, 0, 0, ff, act, gated)
 
 
 def moe_grouped(h, wts, gu_w, down_w, E: int, ff: int, ffs: int, act="silu", gated: bool = True,
@@ -311,5 +369,6 @@ def moe(h, wts, gu_w, down_w, E: int, top: int, ff: int, ffs: int, act="silu",
                and not (h.is_cuda and torch.cuda.is_current_stream_capturing()))
     if grouped and grouped_mm_ok(h, ff):
         return moe_grouped_mm(h, wts, gu_w, down_w, E, top, ff, ffs, act, gated, weigh)
-    return (moe_grouped if grouped else moe_dense)(h, wts, gu_w, down_w, E, ff, ffs, act, gated,
-                                                   weigh)
+    if grouped:
+        return moe_grouped(h, wts, gu_w, down_w, E, ff, ffs, act, gated, weigh)
+    return moe_dense(h, wts, gu_w, down_w, E, ff, ffs, act, gated, weigh, top)

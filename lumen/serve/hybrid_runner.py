@@ -49,8 +49,7 @@ from ..ops.attention import (chunk_sink_attention, diff_head_combine, head_norm_
 from ..ops.conv import dyt_canon, short_conv
 from ..ops.embedding import embed_positions, embed_scaled, gated_token_slice, soft_cap
 from ..ops.gemm import project
-from ..ops.moe import (ClampedGate, gated_act, moe, route_groups, route_topk, router_logits,
-                       scaled_act)
+from ..ops.moe import ClampedGate, feed_forward, moe, route_groups, route_topk, router_logits
 from ..ops.norm import (SPLIT, depth_mix_norm, dyt, dyt_residual, embed_rms, gated_rms_norm,
                         group_rms_norm, group_rms_residual, hyper_mix, hyper_start, parts_rms,
                         residual_rms, scaled_residual_layer_norm, weight_layer_norm)
@@ -290,7 +289,7 @@ def run_layers(w: HybridWeights, st: HybridState, tokens: torch.Tensor, seg: Seg
                 y2 = moe(h2, route_topk(z, f["top"]), f["gu"], f["down"], f["E"], f["top"],
                          f["ff"], f["ffs"])
             else:
-                y2 = project(gated_act(project(h2, f["gu"]), None, 0, 0, f["ffs"]), f["down"])
+                y2 = feed_forward(h2, f["gu"], f["down"], f["ffs"])
             x, _ = dyt_residual(x, y2, L.norms["norm2b"], None, dt)
         if observe is not None:
             observe(i, x)
@@ -472,7 +471,7 @@ def run_dalavik_layers(w: DalavikWeights, st: DalavikState, tokens: torch.Tensor
         xb = xc if cast is not None else x
         f = L.ff
         if f is not None:
-            y = project(gated_act(project(xb, f["gu"]), None, 0, 0, f["ff"], "relu"), f["down"])
+            y = feed_forward(xb, f["gu"], f["down"], f["ff"], "relu")
             x, xc = group_rms_residual(x, y, f["norm"], groups, eps, cast)
             xb = xc if cast is not None else x
         sd = L.side
@@ -1118,7 +1117,7 @@ def run_silonex_layers(w: SilonexWeights, st: SilonexState, tokens: torch.Tensor
                 pair = (L.w["out_l"], L.w["out_r"], eps)
         else:
             f = L.ff
-            ys = [project(gated_act(project(h, f["gu"]), None, 0, 0, f["ff"]), f["down"])]
+            ys = [feed_forward(h, f["gu"], f["down"], f["ff"])]
         _, out, mix = L.hc[q]
         last = k + 1 == len(subs)
         if last:
@@ -1299,7 +1298,7 @@ def _tazulix_mixer(L: TazulixLayerW, w: TazulixWeights, st: TazulixState, n: int
 
 def _tazulix_ff(f: dict, h) -> torch.Tensor:
     if not f["E"]:
-        return project(scaled_act(project(h, f["up"]), None, 0, 0, f["ff"], "relu2"), f["down"])
+        return feed_forward(h, f["up"], f["down"], f["ff"], "relu2", gated=False)
     # the router in fp32, on the (possibly 16-bit rounded) normed row
     r = route_groups(router_logits(h, f["router"]), None, f["top"], 1, 1, normalize=False)
     return moe(h, r, f["gu"], f["down"], f["E"], f["top"], f["ff"], f["ffs"], f["act"],

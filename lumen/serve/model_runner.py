@@ -35,6 +35,7 @@ from ..ops.embedding import embedding
 from ..ops.attention import (flash_attention_fresh, flash_attention_paged, paged_decode,
                              rope_write_kv)
 from ..ops.gemm import linear_nt, swiglu_linear_nt
+from ..ops.moe import thin_act, thin_act_ok
 from ..ops.norm import rms_norm
 from ..ops.rope import rope_tables
 
@@ -223,10 +224,15 @@ class ModelRunner:
             if ml is not None:
                 ml.apply(i, "o", o, a, masks, self._allreduce)
             y2, res = rms_norm(a, L.ln2, cfg.rms_norm_eps, res)
+            if ml is None and use_native(y2) and thin_act_ok(y2, None, L.gate_up, 0, 0, self.w.F):
+                # few decode rows: the activation in the gate|up projection's epilogue
+                act = thin_act(y2, L.gate_up, None, 0, 0, self.w.F)
+                h = self._allreduce(linear_nt(act, L.down))
+                continue
             gu = linear_nt(y2, L.gate_up)
             if ml is not None:
                 ml.apply(i, "gate_up", y2, gu, masks)
-            if ml is None:  # SwiGLU kernel + down projection (GEMV at batch <= 4)
+            if ml is None:  # SwiGLU kernel + down projection (GEMV at batch 1)
                 h = self._allreduce(swiglu_linear_nt(gu, L.down))
             else:
                 act = swiglu(gu)

@@ -5,6 +5,8 @@ import pytest
 import torch
 
 from lumen.ops.gemm import project, thin_linear, thin_ok
+from lumen.ops.moe import (ClampedGate, gated_act_ref, moe_dense, scaled_act_ref, thin_act,
+                           thin_act_ok)
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +71,55 @@ def test_captured_call_replays_on_new_rows():
         x.copy_(torch.randn(3, 512, device="cuda"))
         graph.replay()
         assert torch.equal(y, thin_linear(x, w))
+
+
+def routed(M, E, top, g):
+    """[M, E] weights with ``top`` non-zero ones a row."""
+    idx = torch.rand(M, E, device="cuda", generator=g).topk(top, 1).indices
+    return torch.zeros(M, E, device="cuda").scatter_(
+        1, idx, 0.2 + torch.rand(M, top, device="cuda", generator=g))
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 2.0 ** -8), (torch.float16, 2.0 ** -11)])
+@pytest.mark.parametrize("act,gated,weigh", [("silu", True, "output"), ("relu", True, "output"),
+                                             (ClampedGate(1.0, 0.7, 1.702, 1.0), True, "input"),
+                                             ("relu2", False, "output")])
+@pytest.mark.parametrize("M,E,top,ff,ffs", [(1, 17, 3, 64, 128), (3, 8, 2, 128, 0), (8, 16, 4, 192, 64),
+                                            (17, 5, 1, 48, 32), (32, 64, 2, 64, 64), (9, 0, 0, 0, 208)])
+def test_act_and_skipped_experts(M, E, top, ff, ffs, act, gated, weigh, dtype, tol):
+    g = torch.Generator(device="cuda").manual_seed(M * 7 + E)
+    K, k, W = 320, 2 if gated else 1, 96
+    h = torch.randn(M, K, device="cuda", generator=g).to(dtype)
+    gu = (torch.randn(k * (E * ff + ffs), K, device="cuda", generator=g) / K ** 0.5).to(dtype)
+    down = torch.randn(W, E * ff + ffs, device="cuda", generator=g).to(dtype)
+    wts = routed(M, E, top, g) if E else None
+    fn = gated_act_ref if gated else scaled_act_ref
+    args = (act, weigh) if gated else (act,)
+    want = fn(h.double() @ gu.double().t(), wts, E, ff, ffs, *args).double()   # (fp32 formulas)
+    assert thin_act_ok(h, wts, gu, E, ff, ffs, act, gated, weigh)
+    a = thin_act(h, gu, wts, E, ff, ffs, act, gated, weigh)
+    # one rounding to 16 bits; the fp32 sums and the activation add 1e-5 of the sums' size (~1)
+    assert ((a.double() - want).abs() <= want.abs() * tol + 4e-5).all()
+    ref = a.double() @ down.double().t()
+    y = moe_dense(h, wts, gu, down, E, ff, ffs, act, gated, weigh, top or None)
+    slack = (a.double().abs() @ down.double().abs().t()) * 1e-5
+    assert ((y.double() - ref).abs() <= slack + ref.abs() * tol).all()
+    # blocks nobody chose may hold anything: they are neither read nor multiplied
+    if E and ff % 64 == 0 and ffs % 64 == 0:
+        dead = (wts == 0).all(0).nonzero().flatten().tolist()
+        for e in dead:
+            gu[e * k * ff:(e + 1) * k * ff] = float("nan")
+            down[:, e * ff:(e + 1) * ff] = float("nan")
+        if M * top <= 3 * E:
+            assert torch.equal(moe_dense(h, wts, gu, down, E, ff, ffs, act, gated, weigh, top), y)
+
+
+def test_no_chosen_expert_gives_the_shared_one_alone():
+    h = torch.randn(2, 128, device="cuda").bfloat16()
+    gu = torch.randn(2 * (4 * 64 + 64), 128, device="cuda").bfloat16()
+    down = torch.randn(32, 4 * 64 + 64, device="cuda").bfloat16()
+    wts = torch.zeros(2, 4, device="cuda")
+    y = moe_dense(h, wts, gu, down, 4, 64, 64, top=1)
+    ref = moe_dense(h, None, gu[512:], down[:, 256:].contiguous(), 0, 0, 64)
+    assert torch.equal(y, ref)
+    assert not moe_dense(h, wts, gu[:512], down[:, :256].contiguous(), 4, 64, 0, top=1).any()

@@ -13,10 +13,9 @@
 // while staging) and read back as 16-byte broadcasts; each lane group's slice is padded by four
 // floats so the KS slices of a wave fall into different banks.  The read-outs of the batch are
 // then normalised per head (RMS over the value channels), scaled by the channel weight and the
-// output gate, and stored in the compute dtype.  Sequential in time by construction: parallelism
-// is segments x heads workgroups, which fills the chip for decode batches and mixed steps; a
-// single long prompt runs on `heads` workgroups (the chunk-parallel matrix form is the known
-// faster shape for that case).
+// output gate, and stored in the compute dtype.  Sequential in time by construction: this kernel
+// runs decoded rows and fp32 models; prompt portions of 16-bit models take the chunked matrix form
+// (recurrent_chunk.hip).
 // State in HBM: [slot, head, i, j] fp32; a segment starting at position 0 starts from zero.
 #include "seqmix.h"
 

@@ -1,0 +1,364 @@
+// The `wkv` and generalised-delta recurrences of recurrent.hip over a step's prompt portions, sixteen
+// tokens at a time.  With w_t the decays of token t (one per key channel), P_t = w_1 ... w_t within the
+// chunk, S_0 the state before it, and for the delta rule b_t = a_t un_t:
+//   delta  c_t = un_t^T S_(t-1),   S_t = diag(w_t) S_(t-1) - b_t c_t^T + k_t v_t^T,   o_t = S_t^T r_t
+//   wkv    o_t = S_(t-1)^T r_t + (sum_i r u k) v_t,   S_t = diag(w_t) S_(t-1) + k_t v_t^T
+// and the scaled rows  K_t = k_t / P_t,  B_t = b_t / P_t,  U_t = un_t P_(t-1),  R_t = r_t P_t (wkv:
+// r_t P_(t-1)), all of it is matrix products:
+//   C = (I + strict(U B^T))^-1 (U S_0 + strict(U K^T) V)
+//   O = R S_0 + lower(R K^T) V - lower(R B^T) C      (wkv: strict, its diagonal the bonus; no C)
+//   S' = P_16 (S_0 + K^T V - B^T C)
+// Rows past a chunk's end (or a portion's) enter with w = 1 and zeros, so they change nothing.
+//
+// What bounded the token-by-token kernel: every lane re-read its slice of five vectors from LDS for
+// every token (40 16-byte reads per wave and token at head size 128, ~2 us a token whatever else it did)
+// on segments x heads workgroups.  Here a workgroup owns 64 value columns of a (segment, head), a wave
+// 16 of them with its [D x 16] slice of the state in accumulator registers for the whole portion: the
+// 16x16x4 product's accumulator register e of lane group g holds row 4 g + e, which IS the right operand
+// of a product over the inner rows {4 g + e}, so S, V, C and U S_0 never pass through LDS; the left
+// operands are staged there once for the four waves and read 16 bytes at a time.  All products are
+// fp32 matrix instructions; decays, their products and reciprocals are fp32, as before.
+// The read-outs leave in fp32; the per-head norm and gate follow in gated_rms (rms_group.hip).
+// Measured (8 portions of 512 tokens, width 2048, bf16; the norm kernel's 19 us included): delta, 16 heads
+// of 128: 1000 -> 318 us; wkv, 32 heads of 64: 460 -> 200 us.  A chunk is now a chain of three barriers
+// -- decays and sums, scaled rows, products -- with one wave per SIMD at this size.
+// Against float64 (512 tokens) the read-outs are as far off as the serial walk's (1.66e-3, the bf16 result's
+// rounding); the state 1.4e-7 (serial: 0.9e-7), the order of fp32 sums.
+//
+// Range: 1 / P_t must stay finite.  A chunk ends before the token that would take some channel's P below
+// 2^-80 (a single decay is bounded there: what it keeps of the old state is 1e-24 of it, far below fp32's
+// last place); the delta rule's decays, at least e^-decay_scale per token, never come near.  A chunk
+// that holds an infinity or a NaN runs one token at a time, so earlier tokens stay as they are.
+#include "seqmix.h"
+
+using namespace lumen;
+
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f32x4 mma(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+constexpr int kC = 16;                 // tokens per chunk
+constexpr int LP = 20;                 // row stride of the chunk matrices in LDS
+constexpr float kMinP = 0x1p-80f;      // smallest product of a chunk's decays, and a group's share of it
+template <int NG> constexpr float kGroupP() {
+  return NG == 1 ? 0x1p-80f : NG == 2 ? 0x1p-40f : NG == 4 ? 0x1p-20f : 0x1p-10f;
+}
+
+__device__ __forceinline__ bool finite_f(float x) { return fabsf(x) < INFINITY; }
+
+template <typename T> struct ScanArgs {
+  const T *r, *k, *v, *wl, *al;        // rows of H * D; al: removal rates (delta)
+  long long ldr, ldk, ldv, ldw, lda;
+  const float *w0, *ub;                // decay offsets; u (wkv) / removal-rate bias (delta) [H * D]
+  float* state;                        // [slots][H][D][D]
+  float* out;                          // [T][H * D]
+  const int *cu, *slot, *start;
+  int H, D;
+  float decay_scale, key_eps;
+};
+
+template <int CTRL> __device__ __forceinline__ float dpp(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL,
+                                                               0xF, 0xF, false));
+}
+__device__ __forceinline__ float sum16(float v) {        // over the 16 lanes of a row
+  v += dpp<0xB1>(v);
+  v += dpp<0x4E>(v);
+  v += dpp<0x141>(v);
+  return v + dpp<0x140>(v);
+}
+
+// KB: key channels in blocks of 16
+template <typename T, int KB, bool DELTA>
+__global__ void __launch_bounds__(256)
+scan_chunk_kernel(const ScanArgs<T> a) {
+  constexpr int DKP = 16 * KB, LK = DKP + 4;
+  constexpr int NG = 256 / DKP, TG = kC / NG;            // staging: token groups, tokens of each
+  constexpr int NM = DELTA ? 4 : 1;
+  __shared__ __attribute__((aligned(16))) float s_r[kC * LK], s_k[kC * LK];
+  __shared__ __attribute__((aligned(16))) float s_u[DELTA ? kC * LK : 4], s_b[DELTA ? kC * LK : 4];
+  __shared__ __attribute__((aligned(16))) float s_m[NM][kC * LP];
+  __shared__ __attribute__((aligned(16))) float s_P[DKP], s_gp[NG][DKP], s_red[kC][KB];
+  __shared__ float s_tok[kC];
+  __shared__ int s_n[2], s_low[2];
+  const int sg = blockIdx.x, hd = blockIdx.y;
+  const int r0 = a.cu[sg], len = a.cu[sg + 1] - r0;
+  if (len <= 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lr = lane & 15, lg = lane >> 4;
+  const int D = a.D, col0 = hd * D;
+  const int j = (blockIdx.z * 4 + w) * 16 + lr;                  // this lane's value column
+  const bool on = j < D;
+  const int ch = tid % DKP, tg = tid / DKP;                      // staging: channel, token group
+  const bool chan = ch < D;
+  const float w0 = chan ? a.w0[col0 + ch] : 0.f, ub = chan ? a.ub[col0 + ch] : 0.f;
+
+  f32x4 S[KB];
+  float* st = a.state + ((long long)a.slot[sg] * a.H + hd) * D * D + j;
+  const bool fresh = a.start[sg] == 0;
+#pragma unroll
+  for (int b = 0; b < KB; ++b)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int i = 16 * b + 4 * lg + e;
+      S[b][e] = (!fresh && on && i < D) ? st[(long long)i * D] : 0.f;
+    }
+
+  // the chunk at t0, as loaded: this thread's channel of its tokens, this lane's values (4 lg + e)
+  T pr[TG], pk[TG], pw[TG], pa[TG], pv[4];
+  const auto fetch = [&](int t0) {
+#pragma unroll
+    for (int q = 0; q < TG; ++q) {
+      const int t = t0 + tg * TG + q;
+      const bool live = t < len && chan;
+      const long long row = r0 + t;
+      const T zero = from_f32<T>(0.f);
+      pr[q] = live ? a.r[row * a.ldr + col0 + ch] : zero;
+      pk[q] = live ? a.k[row * a.ldk + col0 + ch] : zero;
+      pw[q] = live ? a.wl[row * a.ldw + col0 + ch] : zero;
+      if (DELTA) pa[q] = live ? a.al[row * a.lda + col0 + ch] : zero;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int t = t0 + 4 * lg + e;
+      pv[e] = (on && t < len) ? a.v[(r0 + t) * a.ldv + col0 + j] : from_f32<T>(0.f);
+    }
+  };
+  if (tid < 2) { s_n[tid] = kC; s_low[tid] = 0; }
+  fetch(0);
+  __syncthreads();
+  for (int t0 = 0, par = 0; t0 < len; par ^= 1) {
+    // ---- decays, removal rates, the channel sums of every token ----
+    float rv[TG], kv[TG], wv[TG], av[TG];
+    {
+      bool ok = true;
+      float gp = 1.f;
+#pragma unroll
+      for (int q = 0; q < TG; ++q) {
+        const bool live = t0 + tg * TG + q < len && chan;
+        rv[q] = to_f32(pr[q]);
+        kv[q] = to_f32(pk[q]);
+        const float zl = to_f32(pw[q]), z = zl + w0;
+        const float d = DELTA ? expf(-a.decay_scale * sigmoid_f(z)) : expf(-expf(z));
+        wv[q] = !live ? 1.f : d < kMinP ? kMinP : d;
+        gp *= wv[q];
+        ok = ok && finite_f(rv[q]) && finite_f(kv[q]) && finite_f(zl);
+        if (DELTA) {
+          const float al = to_f32(pa[q]);
+          ok = ok && finite_f(al);
+          av[q] = live ? sigmoid_f(al + ub) : 0.f;
+        }
+        const float s = sum16(DELTA ? kv[q] * kv[q] : rv[q] * ub * kv[q]);
+        if (lr == 0) s_red[tg * TG + q][ch >> 4] = s;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ok = ok && finite_f(to_f32(pv[e]));
+      s_gp[tg][ch] = gp;
+      if (!ok) atomicMin(&s_n[par], 1);
+      // no group's product below its share of the range: no chunk product leaves it
+      if (!DELTA && !(gp >= kGroupP<NG>())) s_low[par] = 1;
+    }
+    __syncthreads();
+    float P = 1.f, tok[TG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const float q = s_gp[g][ch];
+      P *= g < tg ? q : 1.f;
+    }
+#pragma unroll
+    for (int q = 0; q < TG; ++q) {
+      float s = 0.f;
+#pragma unroll
+      for (int b = 0; b < KB; ++b) s += s_red[tg * TG + q][b];
+      tok[q] = DELTA ? 1.f / sqrtf(s + a.key_eps) : s;
+    }
+    if (!DELTA && s_low[par]) {          // where does a channel's product leave the range?
+      float p = P;
+#pragma unroll
+      for (int q = 0; q < TG; ++q) {
+        p *= wv[q];
+        if (p < kMinP && tg * TG + q > 0) atomicMin(&s_n[par], tg * TG + q);
+      }
+      __syncthreads();
+    }
+    const int n = min(s_n[par], len - t0);
+    if (tid == 0) { s_n[par ^ 1] = kC; s_low[par ^ 1] = 0; }
+    // ---- the scaled rows ----
+#pragma unroll
+    for (int q = 0; q < TG; ++q) {
+      const int t = tg * TG + q, at = t * LK + ch;
+      const bool live = t < n;
+      const float Pn = live ? P * wv[q] : P, inv = 1.f / Pn;
+      s_r[at] = live ? rv[q] * (DELTA ? Pn : P) : 0.f;
+      s_k[at] = live ? kv[q] * inv : 0.f;
+      if (DELTA) {
+        const float u = kv[q] * tok[q];
+        s_u[at] = live ? u * P : 0.f;
+        s_b[at] = live ? u * av[q] * inv : 0.f;
+      } else if (ch == 0) {
+        s_tok[t] = tok[q];
+      }
+      P = Pn;
+    }
+    if (tg == (n - 1) / TG) s_P[ch] = P;   // the groups before it are whole
+    f32x4 V;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) V[e] = 4 * lg + e < n ? to_f32(pv[e]) : 0.f;
+    const int next = t0 + n;
+    if (next < len) fetch(next);         // in flight during the products
+    __syncthreads();
+    // ---- chunk matrices, one per wave: U K^T, U B^T (then inverted), R K^T, R B^T ----
+    if (w < NM) {
+      const float* x = (DELTA && w < 2 ? s_u : s_r) + lr * LK + 4 * lg;
+      const float* y = (DELTA && (w & 1) ? s_b : s_k) + lr * LK + 4 * lg;
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int b = 0; b < KB; ++b) {
+        const float4 xa = *reinterpret_cast<const float4*>(x + 16 * b);
+        const float4 ya = *reinterpret_cast<const float4*>(y + 16 * b);
+        acc = mma(xa.x, ya.x, acc);
+        acc = mma(xa.y, ya.y, acc);
+        acc = mma(xa.z, ya.z, acc);
+        acc = mma(xa.w, ya.w, acc);
+      }
+      float* m = s_m[w];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 4 * lg + e;        // row: token t; column lr: token s
+        float z = i < n && (DELTA && w >= 2 ? lr <= i : lr < i) ? acc[e] : 0.f;
+        if (!DELTA && lr == i && i < n) z = s_tok[i];
+        m[i * LP + lr] = z;
+      }
+      if (DELTA && w == 1) {             // (I + M)^-1, a lane per column
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        float t[kC];
+#pragma unroll
+        for (int i = 0; i < kC; ++i) {
+          float s = 0.f;
+#pragma unroll
+          for (int q = 0; q < kC; q += 4)
+            if (q < i) {
+              const float4 xr = *reinterpret_cast<const float4*>(&m[i * LP + q]);
+              s += xr.x * t[q];
+              if (q + 1 < i) s += xr.y * t[q + 1];
+              if (q + 2 < i) s += xr.z * t[q + 2];
+              if (q + 3 < i) s += xr.w * t[q + 3];
+            }
+          t[i] = i == lr ? 1.f : i > lr ? -s : 0.f;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (lane < 16) {
+#pragma unroll
+          for (int i = 0; i < kC; ++i) m[i * LP + lr] = t[i];
+        }
+      }
+    }
+    // ---- what the old state gives ----
+    f32x4 O = {0.f, 0.f, 0.f, 0.f}, C = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int b = 0; b < KB; ++b) {
+      const float4 x = *reinterpret_cast<const float4*>(&s_r[lr * LK + 16 * b + 4 * lg]);
+      O = mma(x.x, S[b][0], O);
+      O = mma(x.y, S[b][1], O);
+      O = mma(x.z, S[b][2], O);
+      O = mma(x.w, S[b][3], O);
+      if (DELTA) {
+        const float4 u = *reinterpret_cast<const float4*>(&s_u[lr * LK + 16 * b + 4 * lg]);
+        C = mma(u.x, S[b][0], C);
+        C = mma(u.y, S[b][1], C);
+        C = mma(u.z, S[b][2], C);
+        C = mma(u.w, S[b][3], C);
+      }
+    }
+    __syncthreads();                     // chunk matrices complete
+    const auto small = [&](int m, const f32x4& x, f32x4 acc) {
+      const float4 y = *reinterpret_cast<const float4*>(&s_m[m][lr * LP + 4 * lg]);
+      acc = mma(y.x, x[0], acc);
+      acc = mma(y.y, x[1], acc);
+      acc = mma(y.z, x[2], acc);
+      return mma(y.w, x[3], acc);
+    };
+    if (DELTA) {
+      C = small(0, V, C);
+      C = small(1, C, f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+      for (int e = 0; e < 4; ++e) C[e] = 4 * lg + e < n ? -C[e] : 0.f;
+      O = small(3, C, small(2, V, O));
+    } else {
+      O = small(0, V, O);
+    }
+    if (on) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (4 * lg + e < n)
+          a.out[(long long)(r0 + t0 + 4 * lg + e) * a.H * D + col0 + j] = O[e];
+    }
+    // ---- the state moves on ----
+#pragma unroll
+    for (int b = 0; b < KB; ++b) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        S[b] = mma(s_k[(4 * lg + e) * LK + 16 * b + lr], V[e], S[b]);
+        if (DELTA) S[b] = mma(s_b[(4 * lg + e) * LK + 16 * b + lr], C[e], S[b]);
+      }
+      const float4 P = *reinterpret_cast<const float4*>(&s_P[16 * b + 4 * lg]);
+      S[b][0] *= P.x; S[b][1] *= P.y; S[b][2] *= P.z; S[b][3] *= P.w;
+    }
+    t0 = next;
+  }
+  if (on) {
+#pragma unroll
+    for (int b = 0; b < KB; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 16 * b + 4 * lg + e;
+        if (i < D) st[(long long)i * D] = S[b][e];
+      }
+  }
+}
+
+template <typename T, bool DELTA>
+hipError_t launch(const ScanArgs<T>& a, int n_seg, hipStream_t st) {
+  const dim3 grid(n_seg, a.H, (a.D + 63) / 64);
+  if (a.D <= 32) scan_chunk_kernel<T, 2, DELTA><<<grid, 256, 0, st>>>(a);
+  else if (a.D <= 64) scan_chunk_kernel<T, 4, DELTA><<<grid, 256, 0, st>>>(a);
+  else if (a.D <= 128) scan_chunk_kernel<T, 8, DELTA><<<grid, 256, 0, st>>>(a);
+  else scan_chunk_kernel<T, 16, DELTA><<<grid, 256, 0, st>>>(a);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+extern "C" {
+
+// 16-bit rows; delta: al, the removal rates, and decay_scale <= 3 (16 tokens keep P above 2^-80).
+// Segments [0, n_seg) of cu / slot / start; out [T][H * D] fp32, un-normalised read-outs.
+hipError_t sm_scan_chunk(int dt, int delta, const void* r, long long ldr, const void* k, long long ldk,
+                         const void* v, long long ldv, const void* wl, long long ldw, const void* al,
+                         long long lda, const float* w0, const float* ub, float* state, float* out,
+                         const int* cu, const int* slot, const int* start, int n_seg, int H, int D,
+                         float decay_scale, float key_eps, hipStream_t st) {
+  if (n_seg == 0) return hipSuccess;
+  if (n_seg < 0 || H < 1 || D < 1 || D > 256 || (delta && (al == nullptr || decay_scale > 3.f)))
+    return hipErrorInvalidValue;
+#define GO(T)                                                                                   \
+  {                                                                                             \
+    const ScanArgs<T> a{(const T*)r, (const T*)k, (const T*)v, (const T*)wl, (const T*)al, ldr, ldk, \
+                        ldv, ldw, lda, w0, ub, state, out, cu, slot, start, H, D,               \
+                        decay_scale, key_eps};                                                  \
+    return delta ? launch<T, true>(a, n_seg, st) : launch<T, false>(a, n_seg, st);              \
+  }
+  if (dt == kBF16) GO(bf16)
+  if (dt == kF16) GO(fp16)
+  return hipErrorInvalidValue;
+#undef GO
+}
+
+}  // extern "C"

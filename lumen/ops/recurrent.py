@@ -1,5 +1,5 @@
-"""Linear-recurrence token mixers with a per-sequence matrix state (HIP:
-``csrc/seqmix/recurrent.hip``).
+"""Linear-recurrence token mixers with a per-sequence matrix state (HIP: ``csrc/seqmix/recurrent.hip``;
+prompt portions of 16-bit models ``csrc/seqmix/recurrent_chunk.hip``).
 
 Both scans carry one fp32 state S [heads, D, D] (key channel x value channel) per sequence in
 ``state`` [slots, heads, D, D]; a segment whose ``start`` is 0 begins from zero whatever its
@@ -118,6 +118,31 @@ def _check_state(state, H, D):
         raise ValueError(f"recurrent head size {D} > 256 is not supported")
 
 
+# The chunked kernel takes the prompt portions of 16-bit steps: sixteen tokens per matrix step against ~2 us
+# per token of the serial walk (8 portions of 512 tokens, delta rule, 16 heads of 128: 1000 -> 318 us).  Decoded
+# rows are one token each, and fp32 models keep the serial order of the sums.
+DELTA_CHUNK_MAX_DECAY = 3.0      # e^(-16 decay_scale), a chunk's smallest decay product, in fp32's range
+
+
+def _chunk_portions(r, k, v, wl, al, gl, w0, ub, norm_w, state, out, seg: SegBatch, H, D, eps, gate,
+                    decay_scale=0.0, key_eps=0.0) -> int:
+    """Run the step's prompt portions on the chunked kernel, if it takes them; the number of segments
+    done (they come first)."""
+    from ._seqmix import DT, call
+
+    P, rows = seg.portions()
+    if P == 0 or r.dtype not in (torch.bfloat16, torch.float16) or \
+            decay_scale > DELTA_CHUNK_MAX_DECAY:
+        return 0
+    o = torch.empty(rows, H * D, dtype=torch.float32, device=r.device)
+    call("sm_scan_chunk", DT[r.dtype], int(al is not None), r, _ld(r), k, _ld(k), v, _ld(v), wl,
+         _ld(wl), al, _ld(al) if al is not None else 0, w0, ub, state, o, seg.cu, seg.slot,
+         seg.start, P, H, D, decay_scale, key_eps)
+    call("sm_gated_rms", DT[r.dtype], o, gl, _ld(gl), norm_w, out, rows, H * D, H, 0, 0,
+         int(gate == "sigmoid"), eps)
+    return P
+
+
 def wkv_scan(r, k, v, wl, g, w0, u, norm_w, state, seg: SegBatch, H: int, D: int, eps: float):
     from ._seqmix import DT, call, use_seqmix
 
@@ -126,8 +151,9 @@ def wkv_scan(r, k, v, wl, g, w0, u, norm_w, state, seg: SegBatch, H: int, D: int
     _check_state(state, H, D)
     T = r.shape[0]
     out = torch.empty(T, H * D, dtype=r.dtype, device=r.device)
+    P = _chunk_portions(r, k, v, wl, None, g, w0, u, norm_w, state, out, seg, H, D, eps, "silu")
     call("sm_wkv", DT[r.dtype], r, _ld(r), k, _ld(k), v, _ld(v), wl, _ld(wl), g, _ld(g), w0, u,
-         norm_w, state, out, H * D, seg.cu, seg.slot, seg.start, seg.S, H, D, eps)
+         norm_w, state, out, H * D, seg.cu[P:], seg.slot[P:], seg.start[P:], seg.S - P, H, D, eps)
     return out
 
 
@@ -141,9 +167,11 @@ def delta_scan(r, k, v, wl, al, gl, w0, a_b, norm_w, state, seg: SegBatch, H: in
     _check_state(state, H, D)
     T = r.shape[0]
     out = torch.empty(T, H * D, dtype=r.dtype, device=r.device)
+    P = _chunk_portions(r, k, v, wl, al, gl, w0, a_b, norm_w, state, out, seg, H, D, eps, "sigmoid",
+                        float(decay_scale), float(key_eps))
     call("sm_gdelta", DT[r.dtype], r, _ld(r), k, _ld(k), v, _ld(v), wl, _ld(wl), al, _ld(al), gl,
-         _ld(gl), w0, a_b, norm_w, state, out, H * D, seg.cu, seg.slot, seg.start, seg.S, H, D,
-         eps, decay_scale, key_eps)
+         _ld(gl), w0, a_b, norm_w, state, out, H * D, seg.cu[P:], seg.slot[P:], seg.start[P:],
+         seg.S - P, H, D, eps, decay_scale, key_eps)
     return out
 
 

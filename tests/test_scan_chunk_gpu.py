@@ -1,0 +1,127 @@
+"""The chunked prompt scans (seqmix/recurrent_chunk.hip) against float64 token loops: portions around the
+chunk length, state carried over, head sizes on and off the blocks, decays from none to total, and rows
+that are not finite."""
+import math
+
+import pytest
+import torch
+
+from _ref_gedatar import ref_unit_rms
+from lumen.ops.recurrent import delta_scan, wkv_scan
+from lumen.ops.segments import SegBatch, tile_list
+
+pytestmark = pytest.mark.gpu
+KEY_EPS, SCALE, EPS = 1e-6, math.exp(-0.5), 1e-6
+
+
+def batch(pieces, decoded, starts):
+    """Portions of ``pieces`` rows, then ``decoded`` one-row segments; slots in reverse."""
+    cu = [0]
+    for n in list(pieces) + [1] * decoded:
+        cu.append(cu[-1] + n)
+    S, i32 = len(cu) - 1, dict(dtype=torch.int32, device="cuda")
+    t = torch.tensor
+    rows = sum(pieces)
+    row_seg = torch.cat([torch.full((b - a,), i) for i, (a, b) in enumerate(zip(cu, cu[1:]))])
+    pos = torch.cat([torch.arange(b - a) + s for (a, b), s in zip(zip(cu, cu[1:]), starts)])
+    return cu, SegBatch(t(cu, **i32), t(list(range(S))[::-1], **i32), t(starts, **i32),
+                        row_seg.int().cuda(), pos.int().cuda(), None, None,
+                        t(tile_list(cu, len(pieces)), **i32).view(-1, 2), rows, 128)
+
+
+def rows(T, H, D, dtype, g, pad):
+    return [torch.randn(T, H * D + pad, generator=g).to(dtype).cuda()[:, pad:] for _ in range(6)]
+
+
+def exact(kind, x, w0, ub, nw, S0, H, D):
+    """One segment from the state S0 in float64: (normed, gated rows; last state)."""
+    f = lambda t: t.detach().cpu().double()  # noqa: E731
+    r, k, v, wl, al, g = (f(t).reshape(-1, H, D) for t in x)
+    z = wl + f(w0).view(H, D)
+    S = S0.clone()
+    out = []
+    for t in range(r.shape[0]):
+        kv = k[t][:, :, None] * v[t][:, None, :]
+        if kind == "wkv":
+            w = torch.exp(-torch.exp(z[t]))
+            out.append(torch.einsum("hkv,hk->hv", S + f(ub).view(H, D)[:, :, None] * kv, r[t]))
+            S = w[:, :, None] * S + kv
+        else:
+            w = torch.exp(-SCALE * torch.sigmoid(z[t]))
+            un = k[t] / torch.sqrt(k[t].square().sum(-1, keepdim=True) + KEY_EPS)
+            b = torch.sigmoid(al[t] + f(ub).view(H, D)) * un
+            S = w[:, :, None] * S - b[:, :, None] * torch.einsum("hk,hkv->hv", un, S)[:, None] + kv
+            out.append(torch.einsum("hkv,hk->hv", S, r[t]))
+    gate = torch.sigmoid(g) * (g if kind == "wkv" else 1.0)
+    y = ref_unit_rms(torch.stack(out), EPS) * f(nw).view(H, D) * gate
+    return y.reshape(-1, H * D), S
+
+
+def run(kind, x, w0, ub, nw, state, seg, H, D):
+    r, k, v, wl, al, g = x
+    if kind == "wkv":
+        return wkv_scan(r, k, v, wl, g, w0, ub, nw, state, seg, H, D, EPS)
+    return delta_scan(r, k, v, wl, al, g, w0, ub, nw, state, seg, H, D, EPS, SCALE, KEY_EPS)
+
+
+@pytest.mark.parametrize("kind", ["wkv", "delta"])
+@pytest.mark.parametrize("dtype,ulp", [(torch.bfloat16, 2.0 ** -8), (torch.float16, 2.0 ** -11)])
+@pytest.mark.parametrize("H,D,pad", [(2, 128, 0), (3, 64, 8), (2, 32, 3), (1, 20, 0), (1, 256, 0),
+                                     (2, 100, 4), (1, 136, 8)])
+def test_portions_and_decoded_rows(kind, dtype, ulp, H, D, pad):
+    g = torch.Generator().manual_seed(D + H)
+    pieces, decoded = [1, 15, 16, 17, 33, 50], 2
+    starts = [0, 3, 0, 40, 7, 0, 9, 0]
+    cu, seg = batch(pieces, decoded, starts)
+    x = rows(cu[-1], H, D, dtype, g, pad)
+    w0 = torch.linspace(-3, 1, H * D).cuda()
+    ub, nw = torch.randn(H * D, generator=g).cuda(), (1 + 0.1 * torch.randn(H * D, generator=g)).cuda()
+    state = torch.randn(len(starts), H, D, D, generator=g).cuda()
+    before = state.clone()
+    y = run(kind, x, w0, ub, nw, state, seg, H, D)
+    for s, (a, b) in enumerate(zip(cu, cu[1:])):
+        slot = len(starts) - 1 - s
+        S0 = before[slot].cpu().double() * (starts[s] > 0)
+        want, S = exact(kind, [t[a:b] for t in x], w0, ub, nw, S0, H, D)
+        # one rounding of the result; fp32 sums over <= 50 tokens and 256 channels: 2e-5 of a row's size
+        err = (y[a:b].cpu().double() - want).abs()
+        assert (err <= want.abs() * ulp + 2e-5 * want.abs().max()).all(), (s, err.max())
+        assert (state[slot].cpu().double() - S).norm() <= 2e-6 * S.norm()
+
+
+@pytest.mark.parametrize("H,D", [(2, 64), (1, 128)])
+def test_wkv_decays_from_none_to_total(H, D):
+    """exp(-exp(z)) for z from -20 (keeps everything) to 8 (keeps nothing), channel by channel and token
+    by token: products over a chunk leave fp32's range many times over."""
+    g = torch.Generator().manual_seed(5)
+    cu, seg = batch([70], 0, [4])
+    x = rows(70, H, D, torch.bfloat16, g, 0)
+    x[3] = (torch.rand(70, H * D, generator=g) * 28 - 20).bfloat16().cuda()
+    x[3][:, ::3] = 3.0                         # e^-20 a token: four of them pass 2^-80
+    w0, ub, nw = torch.zeros(H * D).cuda(), torch.randn(H * D, generator=g).cuda(), torch.ones(H * D).cuda()
+    state = torch.randn(1, H, D, D, generator=g).cuda()
+    S0 = state[0].cpu().double()
+    y = run("wkv", x, w0, ub, nw, state, seg, H, D)
+    want, S = exact("wkv", x, w0, ub, nw, S0, H, D)
+    err = (y.cpu().double() - want).abs()
+    assert (err <= want.abs() * 2.0 ** -8 + 2e-5 * want.abs().max()).all()
+    assert (state[0].cpu().double() - S).norm() <= 2e-6 * S.norm()
+
+
+@pytest.mark.parametrize("kind", ["wkv", "delta"])
+def test_a_row_that_is_not_finite_spoils_no_earlier_row(kind):
+    H, D = 2, 64
+    g = torch.Generator().manual_seed(9)
+    cu, seg = batch([40, 21], 0, [0, 0])
+    x = rows(61, H, D, torch.bfloat16, g, 0)
+    w0, ub, nw = torch.zeros(H * D).cuda(), torch.zeros(H * D).cuda(), torch.ones(H * D).cuda()
+    clean = run(kind, x, w0, ub, nw, torch.zeros(2, H, D, D).cuda(), seg, H, D)
+    x[2][21, 5] = float("nan")                 # a value of head 0
+    x[1][50, 70] = float("inf")                # a key of head 1
+    y = run(kind, x, w0, ub, nw, torch.zeros(2, H, D, D).cuda(), seg, H, D)
+    tol = dict(rtol=2.0 ** -7, atol=1e-4)
+    torch.testing.assert_close(y[:21], clean[:21], **tol)
+    torch.testing.assert_close(y[40:50], clean[40:50], **tol)
+    torch.testing.assert_close(y[21:40, D:], clean[21:40, D:], **tol)
+    torch.testing.assert_close(y[50:, :D], clean[50:, :D], **tol)
+    assert torch.isnan(y[21, :D]).any() and not torch.isfinite(y[51, D:]).all()

@@ -62,6 +62,7 @@ SIGNATURES = {
     "sm_head_scan_step": "ii" "plplplplpl" "pppp" "pp" "ppp" "iiiiiiff",
     "sm_short_conv": "iplpppp" "pppp" "iii",
     "sm_conv_tail": "iiplpppp" "ppp" "iii",
+    "sm_latent_tiles": "i" "plli" "plli" "pl" "pi" "pll" "pi" "pii" "pp" "ii" "fffi" "ppp" "pl",
     "sm_scan_chunk": "ii" "plplplplpl" "pppp" "ppp" "iii" "ff",
     "sm_thin_gemm": "iplpppliiii" "piii",
     "sm_thin_act": "iplppp" "iiiiiiiii" "ffff",
@@ -91,6 +92,8 @@ def _load():
         lib.sm_row_attn_lds.restype = ctypes.c_int
         lib.sm_latent_attn_ok.argtypes = [ctypes.c_int] * 5
         lib.sm_latent_attn_ok.restype = ctypes.c_int
+        lib.sm_latent_tiles_ok.argtypes = [ctypes.c_int] * 6
+        lib.sm_latent_tiles_ok.restype = ctypes.c_int
         lib.sm_min_gru_sub.argtypes = []
         lib.sm_min_gru_sub.restype = ctypes.c_int
         _lib = lib
@@ -136,6 +139,11 @@ def row_attn_lds(HB: int, Dk: int) -> int:
 def latent_attn_ok(dt: int, Dv: int, Dk: int, D1: int, bs: int) -> bool:
     """Does the matrix-core latent attention have a kernel for these sizes?"""
     return bool(_load().sm_latent_attn_ok(dt, Dv, Dk, D1, bs))
+
+
+def latent_tiles_ok(dt: int, Dv: int, Dk: int, D1: int, bs: int, max_blocks: int) -> bool:
+    """Does the latent attention have a kernel that shares key tiles among rows for these sizes?"""
+    return bool(_load().sm_latent_tiles_ok(dt, Dv, Dk, D1, bs, max_blocks))
 
 
 def min_gru_sub() -> int:

@@ -901,6 +901,9 @@ def _heads_per_block(H: int, Dk: int, need_all: bool) -> int:
     return hb
 
 
+LATENT_TILE_ROWS = 2048      # rows x 16-head blocks from which prompt portions take the tiled latent kernel
+
+
 def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Tensor,
                   vcache: torch.Tensor, Dv: int, out: torch.Tensor, seg, H: int, G: int,
                   scale: float, softcap: float = 0.0, q_temp=None, r1=None, r2=None, talk=None,
@@ -935,9 +938,10 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
     matrix-core kernel of ``csrc/seqmix/window_attention.hip`` when the keys and values have caches
     of their own, one query part, head sizes it is built for (values as wide as the keys or twice
     as wide), a 16-bit dtype and none of temperature, logarithmic bias, head mixing or sink; the latent layout with ``vt`` goes to the
-    latent kernel; every other row (decoded rows, fp32, other shapes) to the row kernel.  A row's
+    latent kernels (``latent_tile.hip`` for large prompt portions); every other row (decoded rows, fp32, other shapes) to the row kernel.  A row's
     result does not depend on which of them computed it beyond rounding."""
-    from ._seqmix import DT, call, latent_attn_ok, use_seqmix, win_tiles_ok
+    from ._seqmix import (DT, call, latent_attn_ok, latent_tiles_ok, use_seqmix,
+                          win_tiles_ok)
 
     T, _, D1 = q1.shape
     D2 = q2.shape[2] if q2 is not None else 0
@@ -975,6 +979,29 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
             and krow % 8 == 0 and al8(q1) and (q2 is None or al8(q2)) and out.data_ptr() % 8 == 0
             and out.stride(0) % 4 == 0 and out.stride(1) % 4 == 0):
         assert tuple(vt.shape) == (kcache.shape[0], Dv, bs) and vt.is_contiguous()
+        row_seg, positions = seg.row_seg, seg.positions
+        # a step's prompt portions: eight rows share a tile's operands (4010 rows, 16 heads: 234 -> 159
+        # us).  Below 256 such workgroups the row kernel, which deals a row's keys out, fills the chip
+        # better (512 rows: 53 vs 94 us)
+        if (seg.q_tiles is not None and seg.tile_rows * ((H + 15) // 16) >= LATENT_TILE_ROWS
+                and krow <= 16384
+                and latent_tiles_ok(DT[q1.dtype], Dv, Dk, D1, bs, seg.tables.shape[1])):
+            Tp = seg.tile_rows
+            call("sm_latent_tiles", DT[q1.dtype], q1, q1.stride(0), q1.stride(1), D1,
+                 q2, q2.stride(0) if q2 is not None else 0, q2.stride(1) if q2 is not None else 0,
+                 D2, kcache, krow, vt, Dv, out, out.stride(0), out.stride(1), seg.tables,
+                 seg.tables.shape[1], seg.q_tiles, seg.q_tiles.shape[0], seg.tile_size, seg.cu,
+                 seg.start, H, bs, scale, float(softcap or 0.0), coef, every, r1, r2, sink, gate,
+                 gate.stride(0) if gate is not None else 0)
+            if Tp >= T:
+                return out
+            full, T = out, T - Tp
+            q1, out = q1[Tp:], out[Tp:]
+            q2 = q2[Tp:] if q2 is not None else None
+            gate = gate[Tp:] if gate is not None else None
+            row_seg, positions = row_seg[Tp:], positions[Tp:]
+        else:
+            full = out
         blocks = T * ((H + 15) // 16)
         tiles = (seg.tables.shape[1] * bs + 127) // 128
         nsplit = max(1, min(tiles, 32, 512 // max(blocks, 1)))
@@ -985,10 +1012,10 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
         call("sm_latent_attn", DT[q1.dtype], q1, q1.stride(0), q1.stride(1), D1,
              q2, q2.stride(0) if q2 is not None else 0, q2.stride(1) if q2 is not None else 0, D2,
              kcache, krow, vt, Dv, out, out.stride(0), out.stride(1),
-             seg.tables, seg.tables.shape[1], seg.row_seg, seg.positions, T, H, bs,
+             seg.tables, seg.tables.shape[1], row_seg, positions, T, H, bs,
              scale, float(softcap or 0.0), coef, every, r1, r2, sink,
              gate, gate.stride(0) if gate is not None else 0, nsplit, ws_ml, ws_o)
-        return out
+        return full
     # a step's prompt portions: tiles of consecutive rows of one segment on the matrix cores, when
     # nothing needs all heads of a (row, key) pair at once and the kernel has the head size; the
     # decoded rows after them (and every other case) take the row kernel below

@@ -5,7 +5,7 @@
 // `sink` adds a key of score 0 that carries no value, i.e. the running softmax starts from
 // (max 0, denominator 1) instead of (-inf, 0).
 //
-// Four waves per (row, query head), for prefill chunks and decode rows alike (a row is a row: its
+// Eight waves per (row, query head), for prefill chunks and decode rows alike (a row is a row: its
 // position and its segment's block table say which keys it sees, so the result cannot depend on
 // how the step was cut).  The waves take the 64-key tiles in turn; within a tile lane l scores key j0 + l -- the dot
 // product and the key's sum of squares come from the same 16-byte loads -- then the wave takes
@@ -21,7 +21,9 @@ namespace {
 
 constexpr int kMaxD = 256;
 
-constexpr int kRowWaves = 4;   // waves per (row, head): each takes every fourth 64-key tile
+// waves per (row, head), each takes every kRowWaves-th 64-key tile: eight walk a context of 512 keys in one
+// step each (8 rows x 16 heads: 20.2 us with four and un-unrolled loads, 17.7 with eight)
+constexpr int kRowWaves = 8;
 
 template <typename T>
 __global__ void __launch_bounds__(64 * kRowWaves)
@@ -68,6 +70,7 @@ chunk_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ 
       const T* kp = cache + rowoff;
       float dot = 0.f, k2 = 0.f;
       if (vec) {
+#pragma unroll 8
         for (int d = 0; d < D; d += 8) {
           float kv[8];
           load8<T>(kp + d, kv);
@@ -100,6 +103,7 @@ chunk_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ 
 #pragma unroll
       for (int e = 0; e < 8; ++e) acc8[e] *= corr;
       if (grp < kpi) {
+#pragma unroll 4
         for (int jj = grp; jj < nk; jj += kpi) {
           const float pj = s_p[w][jj];
           float kv[8];
@@ -143,7 +147,7 @@ chunk_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ 
   }
   if (lane == 0) { s_m[w] = m; s_l[w] = l; }
   __syncthreads();
-  if (w == 0) {
+  if ((int)threadIdx.x < D) {          // (D <= 256 < the workgroup's threads)
     float mt = -INFINITY;
 #pragma unroll
     for (int x = 0; x < kRowWaves; ++x) mt = fmaxf(mt, s_m[x]);
@@ -154,12 +158,11 @@ chunk_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ 
       lt += s_l[x] * f[x];
     }
     const float inv = 1.f / lt;
-    for (int d = lane; d < D; d += 64) {
-      float o = 0.f;
+    const int d = threadIdx.x;
+    float o = 0.f;
 #pragma unroll
-      for (int x = 0; x < kRowWaves; ++x) o += s_acc[x][d] * f[x];
-      out[((long long)t * H + hd) * D + d] = from_f32<T>(o * inv);
-    }
+    for (int x = 0; x < kRowWaves; ++x) o += s_acc[x][d] * f[x];
+    out[((long long)t * H + hd) * D + d] = from_f32<T>(o * inv);
   }
 }
 

@@ -59,6 +59,10 @@ def dyt_canon(x: torch.Tensor, norm, conv_w: torch.Tensor, tail: torch.Tensor, s
     assert x.dtype == torch.float32 and x.is_contiguous() and conv_w.dtype == torch.float32
     assert tail.dtype == torch.float32 and tail.shape[1:] == (max(taps - 1, 0), W) or taps == 1
     out = torch.empty(T, W, dtype=out_dtype, device=x.device)
+    if seg.portions() == (0, 0) and W % 4 == 0 and taps <= 8 and 0 < seg.S <= 65535:
+        call("sm_dyt_canon_rows", DT[out_dtype], x, norm[0], norm[1], norm[2], conv_w, tail, out,
+             seg.cu, seg.slot, seg.start, seg.S, W, taps)
+        return out
     call("sm_dyt_canon", DT[out_dtype], x, norm[0], norm[1], norm[2], conv_w, tail, out, seg.cu,
          seg.slot, seg.start, seg.row_seg, T, W, taps)
     if taps > 1:

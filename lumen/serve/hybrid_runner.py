@@ -56,7 +56,7 @@ from ..ops.norm import (SPLIT, depth_mix_norm, dyt, dyt_residual, embed_rms, gat
 from ..ops.recurrent import delta_scan, head_scan, min_gru_scan, token_shift, wkv_scan
 from ..ops.rope import rotary_write, rotate_interleaved_
 from ..ops.segments import SegBatch, whole_sequences
-from .model_runner import ModelRunner, StepInput
+from .model_runner import ModelRunner, StepInput, fill_step
 
 
 @dataclass
@@ -433,9 +433,9 @@ def run_dalavik_layers(w: DalavikWeights, st: DalavikState, tokens: torch.Tensor
     dt = w.dtype
     eps, groups = cfg.rms_norm_eps, cfg.norm_groups
     T = tokens.shape[0]
-    x = F.embedding(tokens, w.embed).float()
+    xb = F.embedding(tokens, w.embed).to(dt)      # (the rows as stored are their own copy in `dt`)
+    x = xb.float()
     cast = dt if dt != torch.float32 else None
-    xb = x.to(dt) if cast is not None else x
     for i, L in enumerate(w.layers):
         m = L.m
         if L.kind == "latent_attention":
@@ -1397,18 +1397,11 @@ class HybridRunner(ModelRunner):
                                 torch.full((bucket,), -1, dtype=torch.long, device=dev))}
 
     def _fill_static(self, st: dict, inp: StepInput, N: int, bucket: int) -> None:
+        # padding rows: position 0 of the spare state slot, no key written
         sg, src = st["seg"], inp.seg
-        st["tokens"][:N].copy_(inp.tokens)
-        sg.slot[:N].copy_(src.slot)
-        sg.start[:N].copy_(src.start)
-        sg.positions[:N].copy_(src.positions)
-        sg.tables[:N, :src.tables.shape[1]].copy_(src.tables)
-        sg.cache_slots[:N].copy_(src.cache_slots)
-        if N < bucket:  # padding rows: position 0 of the spare state slot, no key written
-            sg.slot[N:].fill_(self.state.spare)
-            sg.start[N:].zero_()
-            sg.positions[N:].zero_()
-            sg.cache_slots[N:].fill_(-1)
+        fill_step([(src.slot, sg.slot, self.state.spare), (src.start, sg.start, 0),
+                   (src.positions, sg.positions, 0)], inp.tokens, st["tokens"], src.cache_slots,
+                  sg.cache_slots, src.tables, sg.tables, N, bucket)
 
     def _decode_static(self, st: dict) -> torch.Tensor:
         return self._logits_rows(self.w.run_layers(self.state, st["tokens"], st["seg"]), None)

@@ -48,6 +48,42 @@ FRESH_PREFILL = os.environ.get("LUMEN_FRESH_PREFILL", "1") != "0"
 DECODE_SPLIT_MIN = int(os.environ.get("LUMEN_DECODE_SPLIT", "0"))
 
 
+KEEP = -(1 << 31)     # sm_fill_step: the padding rows of this buffer are not written
+
+
+def fill_step(rows, tokens, tok_dst, slots, slot_dst, tables, table_dst, N: int,
+              bucket: int) -> None:
+    """A decode step's inputs into the static buffers of its captured graph: ``rows`` = int32 (source [N],
+    buffer, padding value or None: the buffer keeps what it has there), token ids, cache slots (padding
+    rows: -1) and the block tables.  One launch on the GPU (HIP ``csrc/seqmix/step_input.hip``) for the
+    layouts the engine builds, a copy per buffer otherwise."""
+    from ..ops._seqmix import call, use_seqmix
+
+    src = [s for s, _, _ in rows] + [tokens, slots, tables]
+    dst = [d for _, d, _ in rows] + [tok_dst, slot_dst, table_dst]
+    if (tokens.is_cuda and len(rows) <= 3 and N > 0 and use_seqmix(tokens)
+            and all(t.is_contiguous() and t.device == tokens.device for t in src + dst)
+            and all(t.dtype == torch.int32 for t in src[:len(rows)] + dst[:len(rows)]
+                    + [tables, table_dst])
+            and all(t.dtype == torch.int64 for t in (tokens, tok_dst, slots, slot_dst))
+            and all(t.numel() == N for t in src[:-1]) and tables.shape[0] == N
+            and N * tables.shape[1] < 1 << 30 and tables.shape[1] <= table_dst.shape[1]):
+        a = []
+        for s, d, p in rows + [(None, None, None)] * (3 - len(rows)):
+            a += [s, d, KEEP if p is None else p]
+        call("sm_fill_step", *a, tokens, tok_dst, slots, slot_dst, -1, tables, table_dst,
+             tables.shape[1], table_dst.shape[1], N, bucket)
+        return
+    for s, d in zip(src[:-1], dst[:-1]):
+        d[:N].copy_(s)
+    table_dst[:N, :tables.shape[1]].copy_(tables)
+    if N < bucket:
+        slot_dst[N:].fill_(-1)
+        for _, d, p in rows:
+            if p is not None:
+                d[N:].fill_(p)
+
+
 @dataclass
 class LayerW:
     ln1: torch.Tensor
@@ -424,17 +460,12 @@ class ModelRunner:
         return st
 
     def _fill_static(self, st: dict, inp: StepInput, N: int, bucket: int) -> None:
-        st["tokens"][:N].copy_(inp.tokens)
-        st["positions"][:N].copy_(inp.positions)
-        st["slots"][:N].copy_(inp.slots)
-        nb = inp.block_tables.shape[1]
-        st["block_tables"][:N, :nb].copy_(inp.block_tables)
-        st["context_lens"][:N].copy_(inp.context_lens)
+        # padding rows: no cache write, one-token context on block 0
+        rows = [(inp.positions, st["positions"], None), (inp.context_lens, st["context_lens"], 1)]
         if self.lora is not None:
-            st["lora_ids"][:N].copy_(inp.lora_ids)
-        if N < bucket:  # padding rows: no cache write, one-token context on block 0
-            st["slots"][N:].fill_(-1)
-            st["context_lens"][N:].fill_(1)
+            rows.append((inp.lora_ids, st["lora_ids"], None))
+        fill_step(rows, inp.tokens, st["tokens"], inp.slots, st["slots"], inp.block_tables,
+                  st["block_tables"], N, bucket)
 
     def _decode_static(self, st: dict) -> torch.Tensor:
         return self._decode_eager(st["tokens"], st["positions"], st["slots"], st["block_tables"],

@@ -1,13 +1,41 @@
-"""The decoded rows' DyT convolution in one launch: exactly what the separate kernels leave behind."""
+"""A decode step's inputs into static graph buffers, and the decoded rows' DyT convolution, each in one
+launch: exactly what the separate copies, fills and kernels leave behind."""
 import pytest
 import torch
 
 from lumen.ops import _seqmix
 from lumen.ops import conv as conv_mod
 from lumen.ops.segments import SegBatch
+from lumen.serve.model_runner import fill_step
 
 pytestmark = pytest.mark.gpu
 dev = "cuda"
+
+
+@pytest.mark.parametrize("n,bucket,width,ld", [(1, 1, 1, 1), (1, 8, 3, 7), (64, 64, 40, 64), (257, 512, 9, 9),
+                                               (5, 8, 0, 4)])
+@pytest.mark.parametrize("strided", [False, True])
+def test_fill_step(n, bucket, width, ld, strided):
+    g = torch.Generator().manual_seed(n)
+    i32 = lambda *s: torch.randint(0, 1 << 30, s, generator=g, dtype=torch.int32).to(dev)  # noqa: E731
+    i64 = lambda *s: torch.randint(0, 1 << 40, s, generator=g).to(dev)  # noqa: E731
+    cut = (lambda t: t.repeat_interleave(2, -1)[..., ::2]) if strided else (lambda t: t)
+    src = [cut(i32(n)) for _ in range(3)]
+    tok, slot, tab = cut(i64(n)), cut(i64(n)), cut(i32(n, width))
+    pads = [None, 7, -1]
+    dst = [i32(bucket) for _ in range(3)]
+    td, sd, bd = i64(bucket), i64(bucket), i32(bucket, ld)
+    want = [d.clone() for d in dst + [td, sd, bd]]
+    for w, s, p in zip(want, src, pads):
+        w[:n] = s
+        if p is not None:
+            w[n:] = p
+    want[3][:n], want[4][:n] = tok, slot
+    want[4][n:] = -1
+    want[5][:n, :width] = tab
+    fill_step(list(zip(src, dst, pads)), tok, td, slot, sd, tab, bd, n, bucket)
+    for w, d in zip(want, dst + [td, sd, bd]):
+        assert torch.equal(w, d)
 
 
 @pytest.mark.parametrize("taps", [1, 2, 4, 8])

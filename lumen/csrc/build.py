@@ -34,6 +34,20 @@ def ext_path() -> str:
     return os.path.join(PKG, "_C" + suffix)
 
 
+# Files whose matrix instructions are kept on architectural registers.  By default the compiler puts their
+# accumulators in the accumulation registers as soon as a kernel may use more than 256 and then moves
+# values to and fro (moves in the assembly, default -> with the option: lora_v3 5080 -> 590,
+# head_scan_chunk16 7675 -> 1938).  Where it measured faster: the LoRA gradients of 8 x 512 tokens, width
+# 4096, dy3 40.7 -> 33.8 us and dxa3 46.6 -> 35.8; the 16-token scans of one 512-token prompt 59.0 -> 54.8 us.
+# The others are equal or slower (row_attention.hip's latent_attn_kernel 24.6 -> 32.1 us).
+MFMA_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
+MFMA_FORM_FILES = ("lora_v3.hip", "head_scan_chunk16.hip")
+
+
+def _mfma_form(src: str) -> list:
+    return MFMA_FORM if os.path.basename(src) in MFMA_FORM_FILES else []
+
+
 def _torch_flags():
     import torch
     from torch.utils import cpp_extension as ce
@@ -148,7 +162,7 @@ def _build_locked(jobs, force, verbose, build_dir, out) -> str:
         if force or _newer([src] + headers, obj):
             # no packed-fp32 instructions (v_pk_*_f32): scalar fp32 code only
             cmd = [HIPCC, f"--offload-arch={ARCH}", "-munsafe-fp-atomics", "-Xclang",
-                   "-target-feature", "-Xclang", "-packed-fp32-ops", *common, "-c", src,
+                   "-target-feature", "-Xclang", "-packed-fp32-ops", *_mfma_form(src), *common, "-c", src,
                    "-o", obj]
             jobs_list.append(cmd)
     cpu_src = os.path.join(HERE, "cpu", "cpu_adam.cpp")
@@ -214,7 +228,7 @@ def seqmix_sources() -> list:
 def seqmix_digest() -> str:
     import hashlib
 
-    h = hashlib.sha256()
+    h = hashlib.sha256(" ".join(SEQMIX_FLAGS + list(MFMA_FORM_FILES)).encode())
     for f in seqmix_sources():
         with open(f, "rb") as fh:
             h.update(os.path.relpath(f, PKG).encode() + b":" + fh.read())
@@ -252,7 +266,7 @@ def build_seqmix(jobs: int = 8, force: bool = False, verbose: bool = True) -> st
                 return out
             hips = [f for f in seqmix_sources() if f.endswith(".hip")]
             objs = [os.path.join(build_dir, os.path.basename(f) + ".o") for f in hips]
-            cmds = [[HIPCC, f"--offload-arch={ARCH}", *SEQMIX_FLAGS, "-c", f, "-o", o]
+            cmds = [[HIPCC, f"--offload-arch={ARCH}", *SEQMIX_FLAGS, *_mfma_form(f), "-c", f, "-o", o]
                     for f, o in zip(hips, objs)]
             with ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
                 for cmd, (dt, _) in zip(cmds, ex.map(_run, cmds)):

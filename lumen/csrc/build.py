@@ -41,7 +41,7 @@ def ext_path() -> str:
 # 4096, dy3 40.7 -> 33.8 us and dxa3 46.6 -> 35.8; the 16-token scans of one 512-token prompt 59.0 -> 54.8 us.
 # The others are equal or slower (row_attention.hip's latent_attn_kernel 24.6 -> 32.1 us).
 MFMA_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
-MFMA_FORM_FILES = ("lora_v3.hip", "head_scan_chunk16.hip")
+MFMA_FORM_FILES = ("lora_v3.hip", "head_scan_chunk16.hip", "split_gemm.hip")
 
 
 def _mfma_form(src: str) -> list:

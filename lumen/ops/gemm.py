@@ -2,8 +2,9 @@
 
 Up to 64 rows the projection is a stream of the weight matrix: the HIP kernels
 ``seqmix/thin_gemm.hip`` (1 - 64 rows) and ``kernels/skinny_gemm.hip`` (1 row) run it where they
-measured faster than a library GEMM.  Larger batches (and CPU tensors) go to ``torch.matmul``
-(hipBLASLt with the tuned table)."""
+measured faster than a library GEMM; long contractions over some more rows are cut along K
+(``seqmix/split_gemm.hip``).  The rest (and CPU tensors) goes to ``torch.matmul`` (hipBLASLt with the
+tuned table)."""
 from __future__ import annotations
 
 import os
@@ -75,6 +76,58 @@ def thin_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] =
     return y
 
 
+# Split-K GEMM (seqmix/split_gemm.hip): long contractions over a few hundred rows, whose output has too few
+# tiles to fill the chip.  us, library -> split: K = 11008, N = 4096, rows 72 / 256 / 512 / 1000: 41 -> 32, 51 ->
+# 35, 72 -> 50, 113 -> 87; K = 22016 at 512: 139 (tuned) -> 91; K = 32000 at 512: 290 -> 123; K = 11264, N = 2048 at
+# 320 / 1000: 48 -> 32, 72 -> 51.  Below K = 8192 the slabs cost what the split gains (K = 4096 at 512 rows: 28.2
+# and 28.4; K = 5632, N = 2048 at 200: 19.2 and 21.5).  Over 128 tiles a slice would be less than half of K
+# on more workgroups than CUs; under 128 workgroups most CUs idle.
+SPLIT_MIN_M, SPLIT_MIN_K, SPLIT_MAX_S = 65, 8192, 8
+
+
+def split_slices(x: torch.Tensor, w: torch.Tensor) -> int:
+    """Slices of K in which the split-K GEMM should run x [M, K] @ w [N, K]^T (0: leave it to the library)."""
+    if not (x.is_cuda and x.dim() == 2 and w.dim() == 2 and x.dtype == w.dtype
+            and x.dtype in (torch.bfloat16, torch.float16) and x.device == w.device
+            and x.shape[0] >= SPLIT_MIN_M and x.shape[1] == w.shape[1] >= SPLIT_MIN_K):
+        return 0
+    # a plain call: nothing to differentiate, trace or batch
+    if (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)
+            or torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
+            or any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in (x, w))
+            or not use_native(x)):
+        return 0
+    (M, K), N = x.shape, w.shape[0]
+    tiles = -(-M // 256) * -(-N // 128)
+    if not 0 < tiles <= 128:
+        return 0
+    S = min(SPLIT_MAX_S, 256 // tiles)
+    if (tiles * S < 128 or K % 64 or N % 4 or K >= 1 << 22 or (x.data_ptr() | w.data_ptr()) % 16
+            or any(t.stride(1) != 1 or t.stride(0) % 8 or not K <= t.stride(0) <= 1 << 22
+                   for t in (x, w))):
+        return 0
+    return S
+
+
+def split_linear(x: torch.Tensor, w: torch.Tensor, S: int) -> torch.Tensor:
+    """x [M, K] @ w [N, K]^T in S slices of K, their fp32 sums added in order and rounded once.  Callers
+    take S from ``split_slices``."""
+    from ._seqmix import DT, call, use_seqmix
+
+    use_seqmix(x)
+    (M, K), N = x.shape, w.shape[0]
+    y = torch.empty(M, N, device=x.device, dtype=x.dtype)
+    ws = torch.empty(S * -(-M // 256) * -(-N // 128) * 32768, dtype=torch.float32, device=x.device)
+    call("sm_split_gemm", DT[x.dtype], x, x.stride(0), w, w.stride(0), y, N, ws, M, N, K, S)
+    return y
+
+
+def matmul_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x @ w[N, K]^T: the split-K GEMM where it is the faster one, else ``torch.matmul``."""
+    S = split_slices(x, w)
+    return split_linear(x, w, S) if S else torch.matmul(x, w.t())
+
+
 def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``F.linear`` of a served stack: few rows on the weight-streaming kernels (thin GEMM; GEMV for
     one row of a large matrix), the library otherwise."""
@@ -84,7 +137,8 @@ def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = Non
         y = torch.empty(1, w.shape[0], device=x.device, dtype=x.dtype)
         native().skinny_gemm(x, w, y)
         return y
-    return F.linear(x, w, bias)
+    S = split_slices(x, w) if bias is None else 0
+    return split_linear(x, w, S) if S else F.linear(x, w, bias)
 
 
 # Decode batches 5..256: the decode-batch MFMA GEMM (kernels/decode_gemm.hip) where the measured
@@ -254,7 +308,7 @@ def mm_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     on the GPU (see ``split_cols``)."""
     n1 = _split_plan(x, w)
     if not n1:
-        return torch.matmul(x, w.t())
+        return matmul_nt(x, w)
     y = torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=torch.result_type(x, w))
     torch.mm(x, w[:n1].t(), out=y[:, :n1])
     torch.mm(x, w[n1:].t(), out=y[:, n1:])

@@ -14,6 +14,7 @@ from typing import Callable
 import torch
 import torch.nn.functional as F
 
+from .gemm import matmul_nt
 from ._native import native, use_native
 
 IGNORE_INDEX = -100
@@ -47,7 +48,7 @@ class _LMHeadCE(torch.autograd.Function):
         # TN against the frozen head's cached W^T when it keeps one (K-contiguous operands:
         # 778 vs 874 us at Llama-2-7B's 8 x 512 tokens, gpurun r5_55), else NN against W
         wt = ctx.wt_fn() if ctx.wt_fn is not None else None
-        dh = torch.matmul(dlogits, wt.t()) if wt is not None else torch.matmul(dlogits, ctx.weight_fn())
+        dh = matmul_nt(dlogits, wt) if wt is not None else torch.matmul(dlogits, ctx.weight_fn())
         # upstream grad (a 0-dim f32 tensor): multiplied in f32 math, never cast to 16 bits
         # first (2^16, the initial fp16 loss scale, is not representable in fp16); dlogits that
         # already carry the hinted scale are divided by it (ratio 1 on the engine's path)

@@ -1,0 +1,56 @@
+"""Split-K GEMM against float64, over the edges of its tiles and slices, and the rule that picks it."""
+import pytest
+import torch
+
+from lumen.ops import gemm
+from lumen.ops._seqmix import DT, call
+
+pytestmark = pytest.mark.gpu
+dev = "cuda"
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K,S", [(65, 128, 64, 1), (256, 128, 128, 2), (257, 132, 192, 3), (300, 388, 576, 1),
+                                     (513, 260, 1088, 8), (1, 4, 320, 1), (512, 4096, 8192, 4)])
+def test_split_gemm(M, N, K, S, dt):
+    g = torch.Generator().manual_seed(M + K)
+    x = torch.randn(M, K + 8, generator=g).to(dt).to(dev)[:, :K]          # rows of a wider buffer
+    w = torch.randn(N, K, generator=g).to(dt).to(dev)
+    y = torch.full((M, N), float("nan"), dtype=dt, device=dev)
+    ws = torch.full((S * -(-M // 256) * -(-N // 128) * 32768,), float("nan"), device=dev)
+    call("sm_split_gemm", DT[dt], x, x.stride(0), w, w.stride(0), y, N, ws, M, N, K, S)
+    xd, wd = x.double().cpu(), w.double().cpu()
+    want, mag = xd @ wd.t(), xd.abs() @ wd.abs().t()
+    # one rounding to dt, and K fp32 additions of products that are exact in fp32
+    tol = want.abs() * torch.finfo(dt).eps / 2 + mag * K * 2.0 ** -24 + torch.finfo(dt).tiny
+    assert ((y.double().cpu() - want).abs() <= tol).all()
+
+
+def test_non_finite_stays_in_its_row():
+    x = torch.randn(300, 8192, device=dev).bfloat16()
+    w = torch.randn(2048, 8192, device=dev).bfloat16()
+    x[17, 5000] = float("nan")
+    S = gemm.split_slices(x, w)
+    assert S > 1
+    bad = ~torch.isfinite(gemm.split_linear(x, w, S)).all(1)
+    assert bad.nonzero().flatten().tolist() == [17]
+
+
+def test_rule():
+    x, w = torch.randn(512, 8192, device=dev).bfloat16(), torch.randn(4096, 8192, device=dev).bfloat16()
+    assert gemm.split_slices(x, w) == 4
+    for a, b in ((x[:64], w), (x[:, :8128], w[:, :8128]), (x.float(), w.float()), (x.cpu(), w.cpu()),
+                 (x, w.t().contiguous().t()), (x, w[:256]), (x, w.repeat(2, 1)[:, :]), (x.half(), w)):
+        s = gemm.split_slices(a, b)
+        assert s == (2 if b.shape[0] == 8192 else 0)
+    xr = x.clone().requires_grad_()
+    y = gemm.mm_nt(xr, w)
+    assert gemm.split_slices(xr, w) == 0 and y.requires_grad          # differentiable: the library's
+    with torch.no_grad():
+        assert gemm.split_slices(xr, w) == 4
+        got = gemm.mm_nt(xr, w)
+    # both round one fp32-accumulated product: at most one unit apart plus the sums' own error
+    ref = x.double() @ w.double().t()
+    tol = ref.abs() * 2.0 ** -9 + (x.double().abs() @ w.double().abs().t()) * 8192 * 2.0 ** -24
+    assert ((got.double() - ref).abs() <= tol).all()
+    assert torch.equal(torch.func.vmap(lambda v: gemm.matmul_nt(v, w))(x[None]), torch.matmul(x[None], w.t()))

@@ -85,17 +85,21 @@ def thin_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] =
 SPLIT_MIN_M, SPLIT_MIN_K, SPLIT_MAX_S = 65, 8192, 8
 
 
+def _plain(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """A call with nothing to differentiate, trace or batch."""
+    return not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)
+                or torch.compiler.is_compiling()
+                or torch._C._functorch.peek_interpreter_stack() is not None
+                or any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in (x, w)))
+
+
 def split_slices(x: torch.Tensor, w: torch.Tensor) -> int:
     """Slices of K in which the split-K GEMM should run x [M, K] @ w [N, K]^T (0: leave it to the library)."""
     if not (x.is_cuda and x.dim() == 2 and w.dim() == 2 and x.dtype == w.dtype
             and x.dtype in (torch.bfloat16, torch.float16) and x.device == w.device
             and x.shape[0] >= SPLIT_MIN_M and x.shape[1] == w.shape[1] >= SPLIT_MIN_K):
         return 0
-    # a plain call: nothing to differentiate, trace or batch
-    if (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)
-            or torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
-            or any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in (x, w))
-            or not use_native(x)):
+    if not _plain(x, w) or not use_native(x):
         return 0
     (M, K), N = x.shape, w.shape[0]
     tiles = -(-M // 256) * -(-N // 128)
@@ -137,8 +141,7 @@ def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = Non
         y = torch.empty(1, w.shape[0], device=x.device, dtype=x.dtype)
         native().skinny_gemm(x, w, y)
         return y
-    S = split_slices(x, w) if bias is None else 0
-    return split_linear(x, w, S) if S else F.linear(x, w, bias)
+    return mm_nt(x, w) if bias is None else F.linear(x, w, bias)
 
 
 # Decode batches 5..256: the decode-batch MFMA GEMM (kernels/decode_gemm.hip) where the measured
@@ -261,6 +264,25 @@ def split_cols(M: int, N: int) -> int:
     return n1 if 0 < n1 < N else 0
 
 
+# A shape that the tuned table does not hold takes the library's own choice, a 256 x 256 stream-K kernel that
+# pays for an unfilled last wave with more than the wave (0.9 - 1.25 PFLOP/s against 1.45 on whole waves).  Cut
+# at the last whole wave, from two waves on, us: 4010 x 22016 x 4096 662 -> 509, x 11008 408 -> 261, 4010 x 11264 x
+# 2048 166 -> 141, 1900 x 22016 x 4096 395 -> 258, 8000 x 11008 x 4096 619 -> 488; of 29 shapes with 1900 - 8000
+# rows two lost more than noise (3300 x 12288 248 -> 256).  With one whole wave it is even (2305 x 12288 168 ->
+# 176, 2048 x 11008 159 -> 143): left whole.
+WAVE_MIN, WAVE_MIN_K = 2, 2048
+
+
+def wave_cols(M: int, N: int, K: int) -> int:
+    """Column count of the whole waves of 256 x 256 tiles of an [M, N] output with any M (0: no cut)."""
+    tm, tn = -(-M // SPLIT_TILE), -(-N // SPLIT_TILE)
+    if not 0 < tm <= SPLIT_CUS or N % 8 or K < WAVE_MIN_K:
+        return 0
+    waves, tail = divmod(tm * tn, SPLIT_CUS)
+    n1 = waves * (SPLIT_CUS // tm) * SPLIT_TILE
+    return n1 if waves >= WAVE_MIN and tail and 0 < n1 < N else 0
+
+
 _tuned: dict = {"n": -1, "sigs": frozenset()}
 
 
@@ -284,28 +306,33 @@ def _split_plan(x: torch.Tensor, w: torch.Tensor) -> int:
             and w.stride(1) == 1):
         return 0
     (M, K), N = x.shape, w.shape[0]
-    n1 = split_cols(M, N)
-    if not n1:
+    n1, n2 = split_cols(M, N), wave_cols(M, N, K)
+    if not (n1 or n2):
         return 0
-    # only where both parts have tuned solutions (untuned shapes would fall to the heuristic);
-    # decided once per problem (the table is loaded before the first training GEMM)
+    # the first where both parts have tuned solutions, the second where neither the whole nor the parts
+    # have; decided once per problem (the table is loaded before the first training GEMM)
     key = (M, N, K, w.stride(0), x.stride(0))
     hit = _plans.get(key)
     if hit is None:
         sigs = _tuned_sigs()
         lds = f"ld_{w.stride(0)}_{x.stride(0)}_{N}"
-        hit = n1 if (f"tn_{n1}_{M}_{K}_{lds}" in sigs
-                     and f"tn_{N - n1}_{M}_{K}_{lds}" in sigs) else 0
+        if n1 and f"tn_{n1}_{M}_{K}_{lds}" in sigs and f"tn_{N - n1}_{M}_{K}_{lds}" in sigs:
+            hit = n1
+        else:
+            hit = 0 if f"tn_{N}_{M}_{K}_{lds}" in sigs else n2
+        if len(_plans) >= MAX_PLANS:
+            _plans.clear()
         _plans[key] = hit
-    return hit
+    return hit if hit and _plain(x, w) and x.dtype == w.dtype and x.dtype != torch.float32 else 0
 
 
 _plans: dict = {}
+MAX_PLANS = 4096          # (M, N, K, strides) -> columns; ragged prompts bring a new M each
 
 
 def mm_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x [M, K] @ w[N, K]^T -> [M, N] (w row-contiguous), split at the last whole wave of tiles
-    on the GPU (see ``split_cols``)."""
+    on the GPU (see ``split_cols`` and ``wave_cols``)."""
     n1 = _split_plan(x, w)
     if not n1:
         return matmul_nt(x, w)

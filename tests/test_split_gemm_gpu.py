@@ -54,3 +54,18 @@ def test_rule():
     tol = ref.abs() * 2.0 ** -9 + (x.double().abs() @ w.double().abs().t()) * 8192 * 2.0 ** -24
     assert ((got.double() - ref).abs() <= tol).all()
     assert torch.equal(torch.func.vmap(lambda v: gemm.matmul_nt(v, w))(x[None]), torch.matmul(x[None], w.t()))
+
+
+@pytest.mark.parametrize("M,N,K", [(4010, 11264, 2048), (1900, 22016, 2048), (2305, 16384, 4096)])
+def test_whole_wave_columns(M, N, K):
+    x = torch.randn(M, K, device=dev).bfloat16()
+    w = torch.randn(N, K, device=dev).bfloat16()
+    n1 = gemm.wave_cols(M, N, K)
+    assert n1 and gemm._split_plan(x, w) == n1
+    y = gemm.mm_nt(x, w)
+    for c in (0, n1 - 8, N - 8):                                # both sides of the cut, and the last columns
+        xd, wd = x.double(), w[c:c + 16].double()
+        want, mag = xd @ wd.t(), xd.abs() @ wd.abs().t()
+        tol = want.abs() * 2.0 ** -8 + mag * K * 2.0 ** -24     # one rounding, K fp32 additions
+        assert ((y[:, c:c + 16].double() - want).abs() <= tol).all()
+    assert gemm._split_plan(x.requires_grad_(), w) == 0         # differentiable: in one piece

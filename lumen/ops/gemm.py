@@ -34,17 +34,20 @@ def skinny_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
                  if x.shape[0] <= 4 else w.shape[0] % 16 == 0 and w.shape[1] % 128 == 0))
 
 
-# Thin GEMM (seqmix/thin_gemm.hip, whose header holds the measurements).  One row: matrices under 128 MB
-# with K <= 3072 (2048 x 2048: 3.8 vs 4.4 us with the GEMV; 2048 x 5632: 7.3 vs 6.6, 22528 x 4096: 30.7 vs
-# 28.5, and a batch-1 Llama step of 4 layers of width 4096: 432 vs 407 us -- those stay with it).  33 - 64 rows: up to 24 M weights (11264 x 2048: 15.3 vs 17.6 us in the
-# library; 22528 x 4096: 52.0 vs 45.1).  Anything between: always.
+# Thin GEMM (seqmix/thin_gemm.hip, whose header holds the measurements).  One row where the GEMV could take it:
+# matrices under 128 MB with K <= 3072 (2048 x 2048: 3.8 vs 4.4 us with the GEMV; 2048 x 5632: 7.3 vs 6.6,
+# 22528 x 4096: 30.7 vs 28.5, and a batch-1 Llama step of 4 layers of width 4096: 432 vs 407 us -- those stay
+# with it).  33 - 64 rows: up to 24 M weights (11264 x 2048: 15.3 vs 17.6 us in the library; 22528 x 4096: 52.0 vs
+# 45.1).  Anything between, and one row with an fp32 result (32000 x 4096: 44.0 vs 55.3 in the library): up
+# to 208 M weights (50256 x 4096, 32 rows: 90.0 vs 96.8; 32000 x 8192, fp32 result: 108 vs 97).
 THIN_MAX_M = 64
 THIN_ROW_MAX_K, THIN_ROW_MAX_W = 3072, 1 << 26
 THIN_BATCH_MAX_W = 24 << 20
+THIN_MAX_W = 208 << 20
 
 
-def thin_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Can and should the thin GEMM run x [M, K] @ w [N, K]^T?"""
+def thin_ok(x: torch.Tensor, w: torch.Tensor, gemv: bool = True) -> bool:
+    """Can and should the thin GEMM run x [M, K] @ w [N, K]^T?  ``gemv``: one row could go to the GEMV."""
     if not (x.is_cuda and x.dim() == 2 and w.dim() == 2 and 0 < x.shape[0] <= THIN_MAX_M
             and x.dtype == w.dtype and x.dtype in (torch.bfloat16, torch.float16)
             and x.shape[1] == w.shape[1] and w.is_contiguous() and x.stride(1) == 1
@@ -53,9 +56,9 @@ def thin_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     (M, K), N = x.shape, w.shape[0]
     if K == 0 or K % 64 or N % 4 or (x.data_ptr() | w.data_ptr()) % 16 or K >= 1 << 24:
         return False
-    if M == 1:
+    if M == 1 and gemv:
         return K <= THIN_ROW_MAX_K and N * K < THIN_ROW_MAX_W
-    return M <= 32 or N * K <= THIN_BATCH_MAX_W
+    return N * K <= (THIN_MAX_W if M <= 32 else THIN_BATCH_MAX_W)
 
 
 def thin_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,

@@ -57,7 +57,7 @@ def router_logits(h: torch.Tensor, w: torch.Tensor,
     without the pass that widens them."""
     from .gemm import thin_linear, thin_ok
 
-    if thin_ok(h, w) and (bias is None or bias.dtype == h.dtype):
+    if thin_ok(h, w, gemv=False) and (bias is None or bias.dtype == h.dtype):
         return thin_linear(h, w, bias, torch.float32)
     if h.is_cuda and h.dtype == w.dtype and h.dtype in (torch.bfloat16, torch.float16):
         z = torch.mm(h, w.t(), out_dtype=torch.float32)

@@ -300,7 +300,7 @@ class ModelRunner:
         if rows.numel() == 0:  # a chunk that completes no prompt samples nothing
             return torch.empty(0, self.cfg.vocab_size, device=h.device, dtype=h.dtype)
         y, _ = rms_norm(h[rows], self.w.norm, self.cfg.rms_norm_eps, res[rows])
-        return self._vocab_gather(torch.matmul(y, self.w.lm_head.t()))
+        return self._vocab_gather(linear_nt(y, self.w.lm_head))
 
     # ---- mixed step: prefill chunks (whole prompts or pieces of long ones) + decode rows -----
     @torch.no_grad()

@@ -260,8 +260,10 @@ class ModelRunner:
             if ml is not None:
                 ml.apply(i, "o", o, a, masks, self._allreduce)
             y2, res = rms_norm(a, L.ln2, cfg.rms_norm_eps, res)
-            if ml is None and use_native(y2) and thin_act_ok(y2, None, L.gate_up, 0, 0, self.w.F):
-                # few decode rows: the activation in the gate|up projection's epilogue
+            if (ml is None and DECODE_SPLIT_MIN == 0 and use_native(y2)
+                    and thin_act_ok(y2, None, L.gate_up, 0, 0, self.w.F)):
+                # few decode rows: the activation in the gate|up projection's epilogue (not for the halves
+                # of a split batch, which round the projection like the whole batch does)
                 act = thin_act(y2, L.gate_up, None, 0, 0, self.w.F)
                 h = self._allreduce(linear_nt(act, L.down))
                 continue

@@ -72,6 +72,8 @@ hipError_t lumen_skinny_gemm(int, const void*, const void*, void*, int, int, int
                              long long, hipStream_t);
 hipError_t lumen_decode_gemm(int, const void*, const void*, void*, float*, int*, int, int, int,
                              long long, long long, int, int, int, int, int, hipStream_t);
+hipError_t lumen_split_gemm(int, const void*, long long, const void*, long long, void*, long long,
+                            float*, int, int, int, int, hipStream_t);
 hipError_t lumen_mlp_gemm(int, int, const void*, long long, const void*, long long, void*, long long,
                           void*, long long, const void*, long long, int, int, int, int, int, float*,
                           int*, int, hipStream_t);
@@ -246,6 +248,24 @@ void skinny_gemm(const at::Tensor& x, const at::Tensor& w, at::Tensor& y) {
                           static_cast<int>(x.size(0)), static_cast<int>(w.size(0)),
                           static_cast<int>(w.size(1)), x.stride(0), y.stride(0), cur_stream()),
         "skinny_gemm");
+}
+
+// x @ w^T in s slices of K (kernels/split_gemm.hip); the slabs are the call's own
+at::Tensor split_gemm(const at::Tensor& x, const at::Tensor& w, int64_t s) {
+  if (!x.is_cuda() || !w.is_cuda() || x.device() != w.device())
+    throw std::invalid_argument("lumen: split_gemm needs tensors of one GPU");
+  if (x.dim() != 2 || w.dim() != 2 || x.stride(1) != 1 || w.stride(1) != 1 ||
+      x.size(1) != w.size(1) || x.scalar_type() != w.scalar_type() || s < 1)
+    throw std::invalid_argument("lumen: split_gemm shape/layout mismatch");
+  const int64_t M = x.size(0), N = w.size(0), tiles = (M + 255) / 256 * ((N + 127) / 128);
+  at::Tensor y = at::empty({M, N}, x.options());
+  at::Tensor ws = at::empty({s > 1 ? s * tiles * 32768 : 0}, x.options().dtype(at::kFloat));
+  check(lumen_split_gemm(dcode(w), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(),
+                         N, s > 1 ? ws.data_ptr<float>() : nullptr, static_cast<int>(M),
+                         static_cast<int>(N), static_cast<int>(x.size(1)), static_cast<int>(s),
+                         cur_stream()),
+        "split_gemm");
+  return y;
 }
 
 // decode-batch MFMA GEMM (kernels/decode_gemm.hip): y = x @ w^T with block tile (bm, bn) and
@@ -1064,6 +1084,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("transpose2d", &transpose2d);
   m.def("skinny_gemm", &skinny_gemm);
   m.def("skinny_swiglu_gemm", &skinny_swiglu_gemm);
+  m.def("split_gemm", &split_gemm);
   m.def("decode_gemm", &decode_gemm);
   m.def("mlp_gemm", &mlp_gemm, py::arg("epi"), py::arg("x"), py::arg("w"), py::arg("c"),
         py::arg("act") = py::none(), py::arg("gu") = py::none(), py::arg("group_m") = 4,

@@ -15,11 +15,10 @@
 // Measured (bf16, us, library -> here): 512 x 4096 x 22016 139 -> 91, x 32000 290 -> 123, x 11008 72 -> 50; 256 x
 // 4096 x 11008 51 -> 35; 1000 x 2048 x 11264 72 -> 51.  Bound now by LDS bandwidth and latency: one wave per
 // SIMD runs its matrix core at 59 %.
-#include "seqmix.h"
+#include "common.h"
 
-using namespace lumen;
-
-namespace {
+namespace lumen {
+namespace sg {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -54,6 +53,11 @@ struct SplitArgs {
 // 16-byte chunk c of stage row r lies at chunk c ^ swz(r): a fragment read (16 rows at one chunk) and an
 // LDS-DMA piece (8 whole rows) are both conflict free
 __device__ __forceinline__ int swz(int r) { return (r >> 1) & 7; }
+
+template <typename T>
+__device__ __forceinline__ void store4(T* p, const float (&f)[4]) {
+  *reinterpret_cast<uint2*>(p) = make_uint2(pk2<T>(f[0], f[1]), pk2<T>(f[2], f[3]));
+}
 
 template <int N>
 __device__ __forceinline__ void wait_vm() {
@@ -180,7 +184,7 @@ __global__ void __launch_bounds__(256, 1) split_gemm_kernel(const SplitArgs a) {
         float f[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) f[e] = acc[i][j][e];
-        if (m < a.M && n < a.N) store4<T>(y + (long long)m * a.ldy + n, f);
+        if (m < a.M && n < a.N) store4(y + (long long)m * a.ldy + n, f);
       }
     }
   }
@@ -202,17 +206,20 @@ __global__ void __launch_bounds__(256) split_sum_kernel(const SplitArgs a) {
   float o[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) o[e] = s[e];
-  store4<T>((T*)a.y + (long long)m * a.ldy + n, o);
+  store4((T*)a.y + (long long)m * a.ldy + n, o);
 }
 
-}  // namespace
+}  // namespace sg
+}  // namespace lumen
 
 extern "C" {
 
 // y [M, N] = x [M, K] w [N, K]^T (16-bit, rows at ldx, ldw, ldy), K in S slices; ws: S * tiles * 32768 fp32
 // for S > 1.  K % 64 == 0, N % 4 == 0, rows of x and w at 16-byte addresses, of y at 8-byte ones.
-hipError_t sm_split_gemm(int dt, const void* x, long long ldx, const void* w, long long ldw, void* y,
+hipError_t lumen_split_gemm(int dt, const void* x, long long ldx, const void* w, long long ldw, void* y,
                          long long ldy, float* ws, int M, int N, int K, int S, hipStream_t st) {
+  using namespace lumen;
+  using namespace lumen::sg;
   if ((long long)M * N == 0) return hipSuccess;
   if (K <= 0 || K % BK || N % 4 || S < 1 || S > K / BK || ldx % 8 || ldw % 8 || ldy % 4 || ldx < K ||
       ldw < K || ldy < N || ldx > (1 << 22) || ldw > (1 << 22) || (S > 1 && !ws) || (dt != kF16 && dt != kBF16) ||

@@ -62,7 +62,6 @@ SIGNATURES = {
     "sm_head_scan_step": "ii" "plplplplpl" "pppp" "pp" "ppp" "iiiiiiff",
     "sm_short_conv": "iplpppp" "pppp" "iii",
     "sm_conv_tail": "iiplpppp" "ppp" "iii",
-    "sm_split_gemm": "iplplplp" "iiii",
     "sm_fill_step": "ppippippi" "pp" "ppl" "ppii" "ii",
     "sm_dyt_canon_rows": "ipppppppppp" "iii",
     "sm_latent_tiles": "i" "plli" "plli" "pl" "pi" "pll" "pi" "pii" "pp" "ii" "fffi" "ppp" "pl",

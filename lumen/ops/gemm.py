@@ -3,7 +3,7 @@
 Up to 64 rows the projection is a stream of the weight matrix: the HIP kernels
 ``seqmix/thin_gemm.hip`` (1 - 64 rows) and ``kernels/skinny_gemm.hip`` (1 row) run it where they
 measured faster than a library GEMM; long contractions over some more rows are cut along K
-(``seqmix/split_gemm.hip``).  The rest (and CPU tensors) goes to ``torch.matmul`` (hipBLASLt with the
+(``kernels/split_gemm.hip``).  The rest (and CPU tensors) goes to ``torch.matmul`` (hipBLASLt with the
 tuned table)."""
 from __future__ import annotations
 
@@ -79,7 +79,7 @@ def thin_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] =
     return y
 
 
-# Split-K GEMM (seqmix/split_gemm.hip): long contractions over a few hundred rows, whose output has too few
+# Split-K GEMM (kernels/split_gemm.hip): long contractions over a few hundred rows, whose output has too few
 # tiles to fill the chip.  us, library -> split: K = 11008, N = 4096, rows 72 / 256 / 512 / 1000: 41 -> 32, 51 ->
 # 35, 72 -> 50, 113 -> 87; K = 22016 at 512: 139 (tuned) -> 91; K = 32000 at 512: 290 -> 123; K = 11264, N = 2048 at
 # 320 / 1000: 48 -> 32, 72 -> 51.  Below K = 8192 the slabs cost what the split gains (K = 4096 at 512 rows: 28.2
@@ -98,20 +98,21 @@ def _plain(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 def split_slices(x: torch.Tensor, w: torch.Tensor) -> int:
     """Slices of K in which the split-K GEMM should run x [M, K] @ w [N, K]^T (0: leave it to the library)."""
-    if not (x.is_cuda and x.dim() == 2 and w.dim() == 2 and x.dtype == w.dtype
-            and x.dtype in (torch.bfloat16, torch.float16) and x.device == w.device
-            and x.shape[0] >= SPLIT_MIN_M and x.shape[1] == w.shape[1] >= SPLIT_MIN_K):
-        return 0
-    if not _plain(x, w) or not use_native(x):
-        return 0
-    (M, K), N = x.shape, w.shape[0]
+    if x.shape[-1] < SPLIT_MIN_K or x.dim() != 2 or w.dim() != 2 or not x.is_cuda:
+        return 0                                   # (nearly every call: as little host time as can be)
+    (M, K), (N, Kw) = x.shape, w.shape
     tiles = -(-M // 256) * -(-N // 128)
-    if not 0 < tiles <= 128:
+    if not (M >= SPLIT_MIN_M and K == Kw and 0 < tiles <= 128):
         return 0
     S = min(SPLIT_MAX_S, 256 // tiles)
-    if (tiles * S < 128 or K % 64 or N % 4 or K >= 1 << 22 or (x.data_ptr() | w.data_ptr()) % 16
-            or any(t.stride(1) != 1 or t.stride(0) % 8 or not K <= t.stride(0) <= 1 << 22
-                   for t in (x, w))):
+    dt = x.dtype
+    if (tiles * S < 128 or K % 64 or N % 4 or K >= 1 << 22 or dt != w.dtype
+            or dt not in (torch.bfloat16, torch.float16) or x.device != w.device
+            or not _plain(x, w) or not use_native(x)):
+        return 0
+    (lx, ex), (lw, ew) = x.stride(), w.stride()
+    if (ex != 1 or ew != 1 or lx % 8 or lw % 8 or not K <= lx <= 1 << 22 or not K <= lw <= 1 << 22
+            or (x.data_ptr() | w.data_ptr()) % 16):
         return 0
     return S
 
@@ -119,14 +120,7 @@ def split_slices(x: torch.Tensor, w: torch.Tensor) -> int:
 def split_linear(x: torch.Tensor, w: torch.Tensor, S: int) -> torch.Tensor:
     """x [M, K] @ w [N, K]^T in S slices of K, their fp32 sums added in order and rounded once.  Callers
     take S from ``split_slices``."""
-    from ._seqmix import DT, call, use_seqmix
-
-    use_seqmix(x)
-    (M, K), N = x.shape, w.shape[0]
-    y = torch.empty(M, N, device=x.device, dtype=x.dtype)
-    ws = torch.empty(S * -(-M // 256) * -(-N // 128) * 32768, dtype=torch.float32, device=x.device)
-    call("sm_split_gemm", DT[x.dtype], x, x.stride(0), w, w.stride(0), y, N, ws, M, N, K, S)
-    return y
+    return native().split_gemm(x, w, S)
 
 
 def matmul_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -274,6 +268,7 @@ def split_cols(M: int, N: int) -> int:
 # rows two lost more than noise (3300 x 12288 248 -> 256).  With one whole wave it is even (2305 x 12288 168 ->
 # 176, 2048 x 11008 159 -> 143): left whole.
 WAVE_MIN, WAVE_MIN_K = 2, 2048
+MIN_CUT = 1 << 23
 
 
 def wave_cols(M: int, N: int, K: int) -> int:
@@ -309,6 +304,8 @@ def _split_plan(x: torch.Tensor, w: torch.Tensor) -> int:
             and w.stride(1) == 1):
         return 0
     (M, K), N = x.shape, w.shape[0]
+    if M * N < MIN_CUT:                            # less than one whole wave of tiles
+        return 0
     n1, n2 = split_cols(M, N), wave_cols(M, N, K)
     if not (n1 or n2):
         return 0

@@ -238,8 +238,9 @@ def thin_act_ok(h, wts, gu_w, E: int, ff: int, ffs: int, act="silu", gated: bool
     k = 2 if gated else 1
     if gu_w.shape[0] != k * (E * ff + ffs) or (weigh == "input" and not gated):
         return False
-    # one row: thin_ok also says whether the thin kernel beats the GEMV; experts are mostly skipped
-    return thin_ok(h, gu_w[:16] if E and h.shape[0] == 1 else gu_w)
+    # thin_ok also says whether the thin kernel beats the GEMV (one row) or the library (huge matrices):
+    # of a stack of experts most are skipped
+    return thin_ok(h, gu_w[:16] if E else gu_w)
 
 
 def thin_act(h, gu_w, wts, E: int, ff: int, ffs: int, act="silu", gated: bool = True,

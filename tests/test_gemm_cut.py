@@ -10,6 +10,8 @@ def test_wave_cols():
             n1 = gemm.wave_cols(M, N, 4096)
             tm, tn = -(-M // 256), -(-N // 256)
             assert n1 % 256 == 0 and 0 <= n1 < N
+            if n1 or gemm.split_cols(M, N):
+                assert M * N >= gemm.MIN_CUT
             if n1:
                 assert N % 8 == 0 and tm * tn % 256 and n1 // 256 * tm >= 2 * (256 // tm) * tm
             assert gemm.wave_cols(M, N, 1024) == 0

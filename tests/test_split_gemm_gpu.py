@@ -3,7 +3,7 @@ import pytest
 import torch
 
 from lumen.ops import gemm
-from lumen.ops._seqmix import DT, call
+from lumen.ops._native import native
 
 pytestmark = pytest.mark.gpu
 dev = "cuda"
@@ -16,9 +16,7 @@ def test_split_gemm(M, N, K, S, dt):
     g = torch.Generator().manual_seed(M + K)
     x = torch.randn(M, K + 8, generator=g).to(dt).to(dev)[:, :K]          # rows of a wider buffer
     w = torch.randn(N, K, generator=g).to(dt).to(dev)
-    y = torch.full((M, N), float("nan"), dtype=dt, device=dev)
-    ws = torch.full((S * -(-M // 256) * -(-N // 128) * 32768,), float("nan"), device=dev)
-    call("sm_split_gemm", DT[dt], x, x.stride(0), w, w.stride(0), y, N, ws, M, N, K, S)
+    y = native().split_gemm(x, w, S)
     xd, wd = x.double().cpu(), w.double().cpu()
     want, mag = xd @ wd.t(), xd.abs() @ wd.abs().t()
     # one rounding to dt, and K fp32 additions of products that are exact in fp32

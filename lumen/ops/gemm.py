@@ -132,13 +132,16 @@ def matmul_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``F.linear`` of a served stack: few rows on the weight-streaming kernels (thin GEMM; GEMV for
     one row of a large matrix), the library otherwise."""
+    if x.dim() == 2 and x.shape[0] > THIN_MAX_M:       # (first: short prompts are bound by the host)
+        big = x.shape[1] >= SPLIT_MIN_K or x.shape[0] * w.shape[0] >= MIN_CUT
+        return mm_nt(x, w) if big and bias is None and x.is_cuda else F.linear(x, w, bias)
     if thin_ok(x, w) and (bias is None or bias.dtype == x.dtype):
         return thin_linear(x, w, bias)
     if bias is None and x.dim() == 2 and x.shape[0] == 1 and skinny_ok(x, w):
         y = torch.empty(1, w.shape[0], device=x.device, dtype=x.dtype)
         native().skinny_gemm(x, w, y)
         return y
-    return mm_nt(x, w) if bias is None else F.linear(x, w, bias)
+    return F.linear(x, w, bias)
 
 
 # Decode batches 5..256: the decode-batch MFMA GEMM (kernels/decode_gemm.hip) where the measured

@@ -49,7 +49,7 @@ THIN_MAX_W = 208 << 20
 def thin_ok(x: torch.Tensor, w: torch.Tensor, gemv: bool = True) -> bool:
     """Can and should the thin GEMM run x [M, K] @ w [N, K]^T?  ``gemv``: one row could go to the GEMV."""
     if not (x.is_cuda and x.dim() == 2 and w.dim() == 2 and 0 < x.shape[0] <= THIN_MAX_M
-            and x.dtype == w.dtype and x.dtype in (torch.bfloat16, torch.float16)
+            and x.device == w.device and x.dtype == w.dtype and x.dtype in (torch.bfloat16, torch.float16)
             and x.shape[1] == w.shape[1] and w.is_contiguous() and x.stride(1) == 1
             and x.stride(0) % 8 == 0 and x.stride(0) >= x.shape[1]):
         return False
@@ -61,18 +61,40 @@ def thin_ok(x: torch.Tensor, w: torch.Tensor, gemv: bool = True) -> bool:
     return N * K <= (THIN_MAX_W if M <= 32 else THIN_BATCH_MAX_W)
 
 
+def row_bias_ok(bias: Optional[torch.Tensor], x: torch.Tensor, N: int) -> bool:
+    """Is ``bias`` (or None) one the kernels add: N consecutive values of x's type, on its device?"""
+    return bias is None or (bias.dtype == x.dtype and bias.dim() == 1 and bias.shape[0] == N
+                            and bias.is_contiguous() and bias.device == x.device)
+
+
+def weights_ok(wts: Optional[torch.Tensor], h: torch.Tensor, E: int) -> bool:
+    """Are ``wts`` routing weights the kernels read for the rows of ``h``: [rows, E] fp32, its device?"""
+    return (wts is not None and wts.dtype == torch.float32 and wts.is_contiguous()
+            and wts.dim() == 2 and wts.shape[0] == h.shape[0] and wts.shape[1] == E
+            and wts.device == h.device)
+
+
 def thin_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
                 out_dtype: Optional[torch.dtype] = None, blocks: Optional[tuple] = None
                 ) -> torch.Tensor:
     """x [M, K] @ w [N, K]^T (+ ``bias`` [N]) on the thin GEMM kernel, fp32 accumulation; the result
     in x's dtype or (``out_dtype``) fp32.  ``blocks`` = (wts [M, E], E, ff, ffs): K is E blocks of ff
     and one of ffs, and the blocks whose column of wts is all zero are taken as zero without being
-    read.  Callers ask ``thin_ok`` first."""
+    read.  Callers ask ``thin_ok`` (and ``row_bias_ok``) first; the kernel is handed bare addresses, so what
+    does not fit them is an error here."""
     from ._seqmix import DT, call, use_seqmix
 
     use_seqmix(x)
+    if x.dim() != 2 or x.stride(1) != 1 or w.dim() != 2 or not w.is_contiguous() \
+            or x.shape[1] != w.shape[1] or x.dtype != w.dtype or x.device != w.device:
+        raise ValueError("few-row GEMM: rows x [M, K] and contiguous w [N, K] of one type and device")
     (M, K), N = x.shape, w.shape[0]
-    assert bias is None or (bias.dtype == x.dtype and bias.shape == (N,) and bias.stride(0) == 1)
+    if not row_bias_ok(bias, x, N):
+        raise ValueError(f"few-row GEMM: the bias is not [{N}] contiguous values like x's")
+    if blocks is not None:
+        wts, E, ff, ffs = blocks
+        if not weights_ok(wts, x, E) or E * ff + ffs != K:
+            raise ValueError("few-row GEMM: routing weights [M, E] in fp32, K = E blocks of ff and one of ffs")
     y = torch.empty(M, N, device=x.device, dtype=out_dtype or x.dtype)
     call("sm_thin_gemm", DT[x.dtype], x, x.stride(0), w, bias, y, N, M, N, K,
          int(y.dtype == torch.float32), *(blocks or (None, 0, 0, 0)))
@@ -135,7 +157,7 @@ def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = Non
     if x.dim() == 2 and x.shape[0] > THIN_MAX_M:       # (first: short prompts are bound by the host)
         big = x.shape[1] >= SPLIT_MIN_K or x.shape[0] * w.shape[0] >= MIN_CUT
         return mm_nt(x, w) if big and bias is None and x.is_cuda else F.linear(x, w, bias)
-    if thin_ok(x, w) and (bias is None or bias.dtype == x.dtype):
+    if thin_ok(x, w) and row_bias_ok(bias, x, w.shape[0]):
         return thin_linear(x, w, bias)
     if bias is None and x.dim() == 2 and x.shape[0] == 1 and skinny_ok(x, w):
         y = torch.empty(1, w.shape[0], device=x.device, dtype=x.dtype)

@@ -55,9 +55,9 @@ def router_logits(h: torch.Tensor, w: torch.Tensor,
     16-bit values multiply exactly in fp32, so on the GPU the product runs on the matrix cores with
     fp32 accumulation and an fp32 result -- the arithmetic of an fp32 GEMM on the widened operands
     without the pass that widens them."""
-    from .gemm import thin_linear, thin_ok
+    from .gemm import row_bias_ok, thin_linear, thin_ok
 
-    if thin_ok(h, w, gemv=False) and (bias is None or bias.dtype == h.dtype):
+    if thin_ok(h, w, gemv=False) and row_bias_ok(bias, h, w.shape[0]):
         return thin_linear(h, w, bias, torch.float32)
     if h.is_cuda and h.dtype == w.dtype and h.dtype in (torch.bfloat16, torch.float16):
         z = torch.mm(h, w.t(), out_dtype=torch.float32)
@@ -227,13 +227,12 @@ SPARSE_ROWS = 3
 def thin_act_ok(h, wts, gu_w, E: int, ff: int, ffs: int, act="silu", gated: bool = True,
                 weigh: str = "output") -> bool:
     """Can and should ``thin_act`` run the first projection and the activation in one kernel?"""
-    from .gemm import thin_ok
+    from .gemm import thin_ok, weights_ok
 
     if not (h.is_cuda and h.dim() == 2 and 0 < h.shape[0] <= THIN_ACT_MAX_M and ff % 16 == 0
             and ffs % 16 == 0 and E * ff + ffs > 0 and E <= THIN_ACT_MAX_E
             and h.shape[0] * E <= THIN_ACT_MAX_WTS and (gated or isinstance(act, str))
-            and (E == 0 or (wts is not None and wts.dtype == torch.float32
-                            and wts.is_contiguous()))):
+            and (E == 0 or weights_ok(wts, h, E))):
         return False
     k = 2 if gated else 1
     if gu_w.shape[0] != k * (E * ff + ffs) or (weigh == "input" and not gated):
@@ -248,10 +247,15 @@ def thin_act(h, gu_w, wts, E: int, ff: int, ffs: int, act="silu", gated: bool = 
     """``gated_act`` (or ``scaled_act``) of h @ gu_w^T, [T, E * ff + ffs], from the fp32 sums.
     ``sparse``: the blocks of experts that no row chose are left unwritten."""
     from ._seqmix import DT, call, use_seqmix
+    from .gemm import weights_ok
 
     use_seqmix(h)
     if weigh not in ("output", "input"):
         raise ValueError(f"unknown place of the routing weight {weigh!r}")
+    if h.dim() != 2 or h.stride(1) != 1 or not gu_w.is_contiguous() or gu_w.dtype != h.dtype \
+            or gu_w.device != h.device or (E and not weights_ok(wts, h, E)) \
+            or tuple(gu_w.shape) != ((2 if gated else 1) * (E * ff + ffs), h.shape[1]):
+        raise ValueError("few-row experts: rows h, stacked weights and routing weights do not fit")
     out = torch.empty(h.shape[0], E * ff + ffs, dtype=h.dtype, device=h.device)
     code, c = (GATE_ACTS[act], (0.0,) * 4) if isinstance(act, str) else (
         4, (act.limit, act.limit_shared, act.slope, act.shift))
@@ -268,6 +272,8 @@ def moe_dense(h, wts, gu_w, down_w, E: int, ff: int, ffs: int, act="silu", gated
     if thin_act_ok(h, wts, gu_w, E, ff, ffs, act, gated, weigh):
         sparse = (top is not None and 0 < E and h.shape[0] * top <= SPARSE_ROWS * E
                   and ff % 64 == 0 and ffs % 64 == 0 and down_w.is_contiguous()
+                  and down_w.dim() == 2 and down_w.shape[1] == E * ff + ffs
+                  and down_w.dtype == h.dtype and down_w.device == h.device
                   and down_w.shape[0] % 4 == 0 and down_w.data_ptr() % 16 == 0)
         a = thin_act(h, gu_w, wts, E, ff, ffs, act, gated, weigh, sparse)
         if sparse:

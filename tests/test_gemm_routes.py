@@ -1,0 +1,79 @@
+"""Which calls the projection kernels take, and what happens to the ones they cannot."""
+import pytest
+import torch
+
+from lumen.ops import _seqmix, gemm
+from lumen.ops import moe as M
+
+
+@pytest.fixture
+def launched(monkeypatch):
+    """The few-row kernels' launches, recorded instead of run (CPU tensors)."""
+    calls = []
+    monkeypatch.setattr(_seqmix, "use_seqmix", lambda t: True)
+    monkeypatch.setattr(_seqmix, "call", lambda name, *a: calls.append((name, a)))
+    return calls
+
+
+BF = dict(dtype=torch.bfloat16)
+
+
+def test_few_row_kernel_refuses_operands_it_would_misread(launched):
+    x, w = torch.zeros(3, 128, **BF), torch.zeros(8, 128, **BF)
+    wts = torch.zeros(3, 1)
+    bad = [dict(w=torch.zeros(8, 64, **BF)), dict(w=torch.zeros(8, 256, **BF)[:, ::2]),
+           dict(w=torch.zeros(8, 128, device="meta", **BF)), dict(w=w.half()), dict(x=torch.zeros(128, 3, **BF).t()),
+           dict(bias=torch.zeros(4, **BF)), dict(bias=torch.zeros(16, **BF)[::2]),
+           dict(bias=torch.zeros(8, device="meta", **BF)), dict(bias=torch.zeros(8)),
+           dict(blocks=(wts[:2], 1, 64, 64)), dict(blocks=(wts.half(), 1, 64, 64)),
+           dict(blocks=(wts.to("meta"), 1, 64, 64)), dict(blocks=(torch.zeros(3, 2), 1, 64, 64))]
+    for kw in bad:
+        with pytest.raises(ValueError):
+            gemm.thin_linear(kw.pop("x", x), kw.pop("w", w), **kw)
+    assert not launched
+    gemm.thin_linear(x, w, torch.zeros(8, **BF), blocks=(wts, 1, 64, 64))
+    assert [n for n, _ in launched] == ["sm_thin_gemm"]
+
+
+def test_activation_form_refuses_operands_it_would_misread(launched):
+    h, gu, wts = torch.zeros(3, 128, **BF), torch.zeros(2 * (2 * 64 + 64), 128, **BF), torch.zeros(3, 2)
+    args = (2, 64, 64)
+    for a in ((h, gu[:-1], wts), (h, gu[:, :64].contiguous(), wts), (h, gu.half(), wts), (h, gu, None),
+              (h, gu, wts[:2]), (h, gu, torch.zeros(3, 4)[:, :2]), (h, gu, wts.half()),
+              (h, gu.to("meta"), wts), (h, gu, wts.to("meta"))):
+        with pytest.raises(ValueError):
+            M.thin_act(*a, *args)
+    assert not launched
+    M.thin_act(h, gu, wts, *args)
+    assert [n for n, _ in launched] == ["sm_thin_act"]
+
+
+@pytest.mark.parametrize("down", [(96, 128), (96, 256), (94, 192)])
+def test_second_projection_of_another_shape_is_not_read(launched, monkeypatch, down):
+    """A [W, K] that does not fit the activation goes to the library, whose error it always was; one
+    of a width the kernel does not have (94) is multiplied there."""
+    monkeypatch.setattr(M, "thin_act_ok", lambda *a, **k: True)
+    monkeypatch.setattr(M, "thin_act", lambda h, gu, wts, E, ff, ffs, *a: torch.zeros(
+        h.shape[0], E * ff + ffs, **BF))
+    h, gu, wts = torch.zeros(3, 128, **BF), torch.zeros(384, 128, **BF), torch.zeros(3, 2)
+    run = lambda: M.moe_dense(h, wts, gu, torch.zeros(*down, **BF), 2, 64, 64, top=1)  # noqa: E731
+    if down[1] == 192:
+        assert run().shape == (3, 94)
+    else:
+        with pytest.raises(RuntimeError):
+            run()
+    assert not launched
+
+
+@pytest.mark.gpu
+def test_operands_of_two_devices_stay_with_the_library():
+    x, w = torch.zeros(3, 128, device="cuda", **BF), torch.zeros(8, 128, **BF)
+    assert not gemm.thin_ok(x, w) and gemm.thin_ok(x, w.cuda())
+    with pytest.raises(RuntimeError):
+        gemm.project(x, w)
+    with pytest.raises(RuntimeError):
+        gemm.project(x, w.cuda(), torch.zeros(8, **BF))
+    gu, wts = torch.zeros(384, 128, device="cuda", **BF), torch.zeros(3, 2, device="cuda")
+    assert M.thin_act_ok(x, wts, gu, 2, 64, 64)
+    for t in (wts.cpu(), wts[:2], torch.zeros(3, 3, device="cuda")):
+        assert not M.thin_act_ok(x, t, gu, 2, 64, 64)

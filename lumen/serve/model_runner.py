@@ -67,6 +67,7 @@ def fill_step(rows, tokens, tok_dst, slots, slot_dst, tables, table_dst, N: int,
                     + [tables, table_dst])
             and all(t.dtype == torch.int64 for t in (tokens, tok_dst, slots, slot_dst))
             and all(t.numel() == N for t in src[:-1]) and tables.shape[0] == N
+            and N <= bucket <= table_dst.shape[0] and all(t.numel() == bucket for t in dst[:-1])
             and N * tables.shape[1] < 1 << 30 and tables.shape[1] <= table_dst.shape[1]):
         a = []
         for s, d, p in rows + [(None, None, None)] * (3 - len(rows)):

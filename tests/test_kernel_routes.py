@@ -1,4 +1,4 @@
-"""Which calls the projection kernels take, and what happens to the ones they cannot."""
+"""Which calls the kernels of few rows and of decode steps take, and what happens to the ones they cannot."""
 import pytest
 import torch
 
@@ -63,6 +63,32 @@ def test_second_projection_of_another_shape_is_not_read(launched, monkeypatch, d
         with pytest.raises(RuntimeError):
             run()
     assert not launched
+
+
+class OnGpu(torch.Tensor):
+    """A CPU tensor that a dispatch takes for the GPU's."""
+    is_cuda = True
+
+
+@pytest.mark.parametrize("n,bucket,have,table_rows", [(3, 8, 8, 8), (3, 8, 5, 8), (3, 8, 16, 8), (3, 8, 8, 4),
+                                                      (8, 4, 8, 8)])
+def test_step_inputs_never_pass_the_buffers_end(launched, n, bucket, have, table_rows):
+    """The one-launch form writes ``bucket`` entries: buffers of another length are filled by copies."""
+    from lumen.serve.model_runner import fill_step
+
+    i32 = dict(dtype=torch.int32)
+    tok, slots = torch.arange(n).as_subclass(OnGpu), torch.arange(n)
+    pos, tables = torch.arange(n, **i32), torch.ones(n, 2, **i32)
+    td, sd, pd = torch.full((have,), 9), torch.full((have,), 9), torch.full((have,), 9, **i32)
+    tab = torch.zeros(table_rows, 4, **i32)
+    fill_step([(pos, pd, 0)], tok, td, slots, sd, tables, tab, n, bucket)
+    if (n, bucket, have, table_rows) == (3, 8, 8, 8):
+        assert [c for c, _ in launched] == ["sm_fill_step"]
+        return
+    assert not launched
+    assert pd[:n].tolist() == list(range(n)) and tab[:n, :2].eq(1).all()
+    if n < bucket:
+        assert pd[n:].eq(0).all() and sd[n:].eq(-1).all() and td[n:].eq(9).all()
 
 
 @pytest.mark.gpu

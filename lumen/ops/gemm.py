@@ -12,6 +12,7 @@ from typing import Optional
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from ._native import native, use_native
 
@@ -110,12 +111,22 @@ def thin_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] =
 SPLIT_MIN_M, SPLIT_MIN_K, SPLIT_MAX_S = 65, 8192, 8
 
 
-def _plain(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """A call with nothing to differentiate, trace or batch."""
-    return not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)
-                or torch.compiler.is_compiling()
-                or torch._C._functorch.peek_interpreter_stack() is not None
-                or any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in (x, w)))
+def _plain(*tensors: torch.Tensor) -> bool:
+    """A call with nothing to differentiate (backward or forward), batch, trace or cast: the kernels that
+    are launched from here compute on the values alone."""
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if (grad and t.requires_grad or type(t) not in (torch.Tensor, torch.nn.Parameter)
+                or t.layout is not torch.strided or t.is_neg()):
+            return False
+    if (torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch._C._get_tracing_state() is not None or torch._C._len_torch_dispatch_stack()):
+        return False
+    if forward_ad._current_level >= 0 and any(
+            forward_ad.unpack_dual(t).tangent is not None for t in tensors):
+        return False
+    return not (torch.is_autocast_enabled("cuda")
+                and torch.get_autocast_dtype("cuda") != tensors[0].dtype)
 
 
 def split_slices(x: torch.Tensor, w: torch.Tensor) -> int:

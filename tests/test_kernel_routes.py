@@ -103,3 +103,50 @@ def test_operands_of_two_devices_stay_with_the_library():
     assert M.thin_act_ok(x, wts, gu, 2, 64, 64)
     for t in (wts.cpu(), wts[:2], torch.zeros(3, 3, device="cuda")):
         assert not M.thin_act_ok(x, t, gu, 2, 64, 64)
+
+
+def test_a_plain_call_has_nothing_to_differentiate_batch_or_trace():
+    """Of each kind of tensor, and inside each transform, the rule that sends products past autograd."""
+    import torch.autograd.forward_ad as fwd
+    from torch.utils.flop_counter import FlopCounterMode
+
+    x, w, seen = torch.randn(3, 8), torch.randn(4, 8), []
+
+    def probe(v):
+        seen.append(gemm._plain(v, w))
+        return v @ w.t()
+
+    assert gemm._plain(x, w) and gemm._plain(torch.nn.Parameter(w, requires_grad=False), x)
+    xr = x.clone().requires_grad_()
+    assert not gemm._plain(xr, w) and not gemm._plain(w, x, xr)
+    with torch.no_grad():
+        assert gemm._plain(xr, w)
+    assert not gemm._plain(x.as_subclass(OnGpu), w) and not gemm._plain(x.to_sparse(), w)
+    with fwd.dual_level():
+        assert gemm._plain(x, w)
+        dual = fwd.make_dual(x, torch.ones_like(x))
+        assert not gemm._plain(dual, w) and not gemm._plain(w, dual)
+    torch.func.vmap(probe)(x[None])
+    torch.func.jvp(probe, (x,), (x,))
+    torch.func.grad(lambda v: probe(v).sum())(x)
+    torch.jit.trace(probe, x, check_trace=False)
+    with FlopCounterMode(display=False):
+        probe(x)
+    assert seen and not any(seen)
+
+
+@pytest.mark.gpu
+def test_long_contractions_and_cut_products_keep_tangents_and_transforms():
+    import torch.autograd.forward_ad as fwd
+
+    g = torch.Generator(device="cuda").manual_seed(1)
+    for M_, N, K in ((512, 4096, 8192), (1900, 22016, 2048)):
+        x, t = (torch.randn(M_, K, device="cuda", generator=g).bfloat16() for _ in range(2))
+        w = torch.randn(N, K, device="cuda", generator=g).bfloat16()
+        assert gemm.split_slices(x, w) or gemm._split_plan(x, w)
+        with fwd.dual_level():
+            y = fwd.unpack_dual(gemm.mm_nt(fwd.make_dual(x, t), w))
+        want = torch.matmul(t, w.t())
+        assert y.tangent is not None and ((y.tangent - want).norm() <= 2.0 ** -7 * want.norm())
+        with torch.autocast("cuda", torch.float16):
+            assert gemm.mm_nt(x, w).dtype == torch.float16

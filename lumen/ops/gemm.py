@@ -35,6 +35,24 @@ def skinny_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
                  if x.shape[0] <= 4 else w.shape[0] % 16 == 0 and w.shape[1] % 128 == 0))
 
 
+def _plain(*tensors: torch.Tensor) -> bool:
+    """A call with nothing to differentiate (backward or forward), batch, trace or cast: the kernels that
+    are launched from here compute on the values alone."""
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if (grad and t.requires_grad or type(t) not in (torch.Tensor, torch.nn.Parameter)
+                or t.layout is not torch.strided or t.is_neg()):
+            return False
+    if (torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch._C._get_tracing_state() is not None or torch._C._len_torch_dispatch_stack()):
+        return False
+    if forward_ad._current_level >= 0 and any(
+            forward_ad.unpack_dual(t).tangent is not None for t in tensors):
+        return False
+    return not (torch.is_autocast_enabled("cuda")
+                and torch.get_autocast_dtype("cuda") != tensors[0].dtype)
+
+
 # Thin GEMM (seqmix/thin_gemm.hip, whose header holds the measurements).  One row where the GEMV could take it:
 # matrices under 128 MB with K <= 3072 (2048 x 2048: 3.8 vs 4.4 us with the GEMV; 2048 x 5632: 7.3 vs 6.6,
 # 22528 x 4096: 30.7 vs 28.5, and a batch-1 Llama step of 4 layers of width 4096: 432 vs 407 us -- those stay
@@ -51,7 +69,7 @@ def thin_ok(x: torch.Tensor, w: torch.Tensor, gemv: bool = True) -> bool:
     """Can and should the thin GEMM run x [M, K] @ w [N, K]^T?  ``gemv``: one row could go to the GEMV."""
     if not (x.is_cuda and x.dim() == 2 and w.dim() == 2 and 0 < x.shape[0] <= THIN_MAX_M
             and x.device == w.device and x.dtype == w.dtype and x.dtype in (torch.bfloat16, torch.float16)
-            and x.shape[1] == w.shape[1] and w.is_contiguous() and x.stride(1) == 1
+            and x.shape[1] == w.shape[1] and _plain(x, w) and w.is_contiguous() and x.stride(1) == 1
             and x.stride(0) % 8 == 0 and x.stride(0) >= x.shape[1]):
         return False
     (M, K), N = x.shape, w.shape[0]
@@ -111,24 +129,6 @@ def thin_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] =
 SPLIT_MIN_M, SPLIT_MIN_K, SPLIT_MAX_S = 65, 8192, 8
 
 
-def _plain(*tensors: torch.Tensor) -> bool:
-    """A call with nothing to differentiate (backward or forward), batch, trace or cast: the kernels that
-    are launched from here compute on the values alone."""
-    grad = torch.is_grad_enabled()
-    for t in tensors:
-        if (grad and t.requires_grad or type(t) not in (torch.Tensor, torch.nn.Parameter)
-                or t.layout is not torch.strided or t.is_neg()):
-            return False
-    if (torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch._C._get_tracing_state() is not None or torch._C._len_torch_dispatch_stack()):
-        return False
-    if forward_ad._current_level >= 0 and any(
-            forward_ad.unpack_dual(t).tangent is not None for t in tensors):
-        return False
-    return not (torch.is_autocast_enabled("cuda")
-                and torch.get_autocast_dtype("cuda") != tensors[0].dtype)
-
-
 def split_slices(x: torch.Tensor, w: torch.Tensor) -> int:
     """Slices of K in which the split-K GEMM should run x [M, K] @ w [N, K]^T (0: leave it to the library)."""
     if x.shape[-1] < SPLIT_MIN_K or x.dim() != 2 or w.dim() != 2 or not x.is_cuda:
@@ -168,9 +168,9 @@ def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = Non
     if x.dim() == 2 and x.shape[0] > THIN_MAX_M:       # (first: short prompts are bound by the host)
         big = x.shape[1] >= SPLIT_MIN_K or x.shape[0] * w.shape[0] >= MIN_CUT
         return mm_nt(x, w) if big and bias is None and x.is_cuda else F.linear(x, w, bias)
-    if thin_ok(x, w) and row_bias_ok(bias, x, w.shape[0]):
+    if thin_ok(x, w) and (bias is None or row_bias_ok(bias, x, w.shape[0]) and _plain(bias)):
         return thin_linear(x, w, bias)
-    if bias is None and x.dim() == 2 and x.shape[0] == 1 and skinny_ok(x, w):
+    if bias is None and x.dim() == 2 and x.shape[0] == 1 and _plain(x, w) and skinny_ok(x, w):
         y = torch.empty(1, w.shape[0], device=x.device, dtype=x.dtype)
         native().skinny_gemm(x, w, y)
         return y

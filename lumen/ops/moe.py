@@ -55,9 +55,10 @@ def router_logits(h: torch.Tensor, w: torch.Tensor,
     16-bit values multiply exactly in fp32, so on the GPU the product runs on the matrix cores with
     fp32 accumulation and an fp32 result -- the arithmetic of an fp32 GEMM on the widened operands
     without the pass that widens them."""
-    from .gemm import row_bias_ok, thin_linear, thin_ok
+    from .gemm import _plain, row_bias_ok, thin_linear, thin_ok
 
-    if thin_ok(h, w, gemv=False) and row_bias_ok(bias, h, w.shape[0]):
+    if thin_ok(h, w, gemv=False) and (bias is None or row_bias_ok(bias, h, w.shape[0])
+                                      and _plain(bias)):
         return thin_linear(h, w, bias, torch.float32)
     if h.is_cuda and h.dtype == w.dtype and h.dtype in (torch.bfloat16, torch.float16):
         z = torch.mm(h, w.t(), out_dtype=torch.float32)
@@ -227,12 +228,12 @@ SPARSE_ROWS = 3
 def thin_act_ok(h, wts, gu_w, E: int, ff: int, ffs: int, act="silu", gated: bool = True,
                 weigh: str = "output") -> bool:
     """Can and should ``thin_act`` run the first projection and the activation in one kernel?"""
-    from .gemm import thin_ok, weights_ok
+    from .gemm import _plain, thin_ok, weights_ok
 
     if not (h.is_cuda and h.dim() == 2 and 0 < h.shape[0] <= THIN_ACT_MAX_M and ff % 16 == 0
             and ffs % 16 == 0 and E * ff + ffs > 0 and E <= THIN_ACT_MAX_E
             and h.shape[0] * E <= THIN_ACT_MAX_WTS and (gated or isinstance(act, str))
-            and (E == 0 or weights_ok(wts, h, E))):
+            and (E == 0 or weights_ok(wts, h, E) and _plain(wts))):
         return False
     k = 2 if gated else 1
     if gu_w.shape[0] != k * (E * ff + ffs) or (weigh == "input" and not gated):

@@ -150,3 +150,44 @@ def test_long_contractions_and_cut_products_keep_tangents_and_transforms():
         assert y.tangent is not None and ((y.tangent - want).norm() <= 2.0 ** -7 * want.norm())
         with torch.autocast("cuda", torch.float16):
             assert gemm.mm_nt(x, w).dtype == torch.float16
+
+
+def test_few_row_rule_asks_for_a_plain_call(monkeypatch):
+    x, w = torch.zeros(3, 128, **BF), torch.zeros(8, 128, **BF)
+    wts, gu = torch.zeros(3, 2), torch.zeros(384, 128, **BF)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    assert gemm.thin_ok(x, w) and M.thin_act_ok(x, wts, gu, 2, 64, 64)
+    for a, b, c in ((x.clone().requires_grad_(), wts, gu), (x, wts, gu.clone().requires_grad_()),
+                    (x, wts.clone().requires_grad_(), gu)):
+        assert not M.thin_act_ok(a, b, c, 2, 64, 64)
+    assert not gemm.thin_ok(x.clone().requires_grad_(), w)
+    assert not gemm.thin_ok(x, w.clone().requires_grad_())
+    seen = []
+    torch.func.vmap(lambda v: (seen.append(gemm.thin_ok(v, w)), v)[1])(x[None])
+    assert seen == [False]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 8])
+def test_few_row_products_keep_gradients_tangents_and_batching(rows):
+    """What the library answered before the few-row kernels: history, tangents, vmap."""
+    import torch.autograd.forward_ad as fwd
+
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    r = lambda *s: torch.randn(*s, device="cuda", generator=g).bfloat16()  # noqa: E731
+    x, t, w, b = r(rows, 4096), r(rows, 4096), r(256, 4096), r(256)
+    near = lambda a, e: ((a - e).norm() <= 2.0 ** -7 * e.norm())  # noqa: E731
+    for f, ref in ((lambda v: gemm.project(v, w), lambda v: v @ w.t()),
+                   (lambda v: gemm.project(v, w, b), lambda v: v @ w.t() + b)) + (
+                       ((lambda v: gemm.linear_nt(v, w), lambda v: v @ w.t()),) if rows > 4 else ()):
+        xr = x.clone().requires_grad_()
+        y = f(xr)
+        assert y.requires_grad and near(y.detach(), ref(x))
+        y.sum().backward()
+        assert near(xr.grad, w.sum(0, keepdim=True).expand_as(x))
+        assert near(torch.func.vmap(f)(x[None])[0], ref(x))
+        with fwd.dual_level():
+            tan = fwd.unpack_dual(f(fwd.make_dual(x, t))).tangent
+        assert tan is not None and near(tan.float(), (t @ w.t()).float())
+    xr = x.clone().requires_grad_()
+    assert M.router_logits(xr, w).requires_grad == torch.mm(xr, w.t(), out_dtype=torch.float32).requires_grad

@@ -119,8 +119,9 @@ def _check_state(state, H, D):
 
 
 # The chunked kernel takes the prompt portions of 16-bit steps: sixteen tokens per matrix step against ~2 us
-# per token of the serial walk (8 portions of 512 tokens, delta rule, 16 heads of 128: 1000 -> 318 us).  Decoded
+# per token of the serial walk (8 portions of 512 tokens, delta rule, 16 heads of 128: 1000 -> 290 us).  Decoded
 # rows are one token each, and fp32 models keep the serial order of the sums.
+CHUNK_MAX_STRIDE = 1 << 26       # elements between rows (32-bit offsets within a chunk)
 DELTA_CHUNK_MAX_DECAY = 3.0      # e^(-16 decay_scale), a chunk's smallest decay product, in fp32's range
 
 
@@ -132,7 +133,8 @@ def _chunk_portions(r, k, v, wl, al, gl, w0, ub, norm_w, state, out, seg: SegBat
 
     P, rows = seg.portions()
     if P == 0 or r.dtype not in (torch.bfloat16, torch.float16) or \
-            decay_scale > DELTA_CHUNK_MAX_DECAY:
+            not 0.0 <= decay_scale <= DELTA_CHUNK_MAX_DECAY or \
+            max(t.stride(0) for t in (r, k, v, wl, al) if t is not None) >= CHUNK_MAX_STRIDE:
         return 0
     o = torch.empty(rows, H * D, dtype=torch.float32, device=r.device)
     call("sm_scan_chunk", DT[r.dtype], int(al is not None), r, _ld(r), k, _ld(k), v, _ld(v), wl,

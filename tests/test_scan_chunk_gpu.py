@@ -125,3 +125,45 @@ def test_a_row_that_is_not_finite_spoils_no_earlier_row(kind):
     torch.testing.assert_close(y[21:40, D:], clean[21:40, D:], **tol)
     torch.testing.assert_close(y[50:, :D], clean[50:, :D], **tol)
     assert torch.isnan(y[21, :D]).any() and not torch.isfinite(y[51, D:]).all()
+
+
+@pytest.mark.parametrize("kind", ["wkv", "delta"])
+@pytest.mark.parametrize("what,by", [(1, 58), (0, 50), (0, -50), (1, -100), (2, 50), (1, 30)])
+def test_large_and_small_values_of_a_range_without_end(kind, what, by):
+    """bf16 reaches 2^127 (and the norm of a read-out 2^63): rows of r, k or v far from 1, under decays whose products over a chunk leave
+    the range of the scaled rows, as the token-by-token walk takes them."""
+    H, D, T = 2, 64, 50
+    g = torch.Generator().manual_seed(7)
+    cu, seg = batch([T], 0, [4])
+    x = rows(T, H, D, torch.bfloat16, g, 0)
+    scale = torch.ones(T, 1)
+    scale[[3, 9, 10, 30]] = 2.0 ** by
+    x[what] = (x[what].float().cpu() * scale).bfloat16().cuda()
+    if what == 1 and by > 0:                    # products k v of ordinary size
+        x[2] = (x[2].float().cpu() / scale).bfloat16().cuda()
+    x[3][:, ::5] = 1.6                          # wkv: e^-5 a token
+    w0, ub = torch.zeros(H * D).cuda(), torch.randn(H * D, generator=g).cuda()
+    nw = torch.ones(H * D).cuda()
+    state = torch.randn(1, H, D, D, generator=g).cuda()
+    S0 = state[0].cpu().double()
+    y = run(kind, x, w0, ub, nw, state, seg, H, D)
+    want, S = exact(kind, x, w0, ub, nw, S0, H, D)
+    err = (y.cpu().double() - want).abs()
+    assert torch.isfinite(y).all() and torch.isfinite(state).all()
+    # of each row's own size: one rounding of the result; fp32 sums over <= 50 tokens and 64 channels
+    assert (err <= want.abs() * 2.0 ** -8 + 2e-5 * want.abs().amax(1, keepdim=True) + 1e-30).all()
+    assert (state[0].cpu().double() - S).norm() <= 2e-6 * S.norm()
+
+
+def test_a_total_decay_leaves_nothing():
+    H, D = 1, 64
+    g = torch.Generator().manual_seed(3)
+    cu, seg = batch([20], 0, [4])
+    x = rows(20, H, D, torch.bfloat16, g, 0)
+    x[3].fill_(-3.0)
+    x[3][5] = 5.0                               # exp(-e^5) = 0 in fp32
+    w0, ub, nw = torch.zeros(D).cuda(), torch.zeros(D).cuda(), torch.ones(D).cuda()
+    state = 2.0 ** 100 * torch.randn(1, H, D, D, generator=g).cuda()
+    run("wkv", x, w0, ub, nw, state, seg, H, D)
+    _, S = exact("wkv", x, w0, ub, nw, torch.zeros(H, D, D).double(), H, D)
+    assert (state[0].cpu().double() - S).norm() <= 2e-6 * S.norm()

@@ -17,13 +17,15 @@
 // 16x16x4 product's accumulator register e of lane group g holds row 4 g + e, which IS the right operand
 // of a product over the inner rows {4 g + e}, so S, V, C and U S_0 never pass through LDS; the left
 // operands are staged there once for the four waves and read 16 bytes at a time.  All products are
-// fp32 matrix instructions; decays, their products and reciprocals are fp32, as before.
+// fp32 matrix instructions; decays are fp32, their products fp64.
 // The read-outs leave in fp32; the per-head norm and gate follow in gated_rms (rms_group.hip).
-// Measured (8 portions of 512 tokens, width 2048, bf16; the norm kernel's 19 us included): delta, 16 heads
-// of 128: 1000 -> 290 us; wkv, 32 heads of 64: 460 -> 122 us.  A chunk is now a chain of three barriers
+// Measured (8 portions of 512 tokens, width 2048, bf16; the norm kernel's 17 us included): delta, 16 heads
+// of 128: 1000 -> 310 us; wkv, 32 heads of 64: 460 -> 119 us.  A chunk is now a chain of three barriers
 // -- decays and sums, scaled rows, products -- with one wave per SIMD at this size.
-// Against float64 (512 tokens) the read-outs are as far off as the serial walk's (1.66e-3, the bf16 result's
-// rounding); the state 1.4e-7 (serial: 0.9e-7), the order of fp32 sums.
+// Error against float64 (512 tokens, heads of 32 - 256): the read-outs are as far off as the serial walk's
+// (1.66e-3, the bf16 result's rounding), the state a little less (delta 0.86e-7, serial 0.88e-7; wkv 0.60e-7,
+// serial 0.62e-7).  That takes the decays' products in float64 (in fp32: + 0.1e-7) and care with the sums
+// (see the state's update; term by term 1.4e-7 and 0.9e-7), which cost 20 us of the delta scan.
 //
 // Range: P_t and 1 / P_16 must stay finite, and so must the masked entries' factors.  A wkv chunk ends
 // before the token that would take some channel's P below 2^-100, so a decay beyond that (0 too) is alone in
@@ -31,7 +33,7 @@
 // stay above 2^-70.  r and k that scaled rows could not hold as normal numbers (kLarge, kTiny*), infinities and
 // NaN run one token at a time, so that earlier tokens stay as they are; wkv values below kSmall make the
 // chunk end at 2^-40.  A chunk of one token costs what one of sixteen does: decays up to e^-50 a token (wkv,
-// 8 x 512 tokens, 32 heads of 64, log decays -e^N(1, 1) at the fast end) take 790 us, the
+// 8 x 512 tokens, 32 heads of 64, log decays -e^N(1, 1) at the fast end) take 770 us, the
 // serial walk 460.
 #include "seqmix.h"
 
@@ -98,7 +100,7 @@ scan_chunk_kernel(const ScanArgs<T> a) {
   __shared__ __attribute__((aligned(16))) float s_u[DELTA ? kC * LK : 4], s_b[DELTA ? kC * LK : 4];
   __shared__ __attribute__((aligned(16))) float s_m[NM][kC * LP];
   __shared__ __attribute__((aligned(16))) float s_P[DKP], s_iP[DKP], s_red[kC][KB];
-  __shared__ float s_gp[NG][DKP];
+  __shared__ double s_gp[NG][DKP];
   __shared__ float s_tok[kC];
   __shared__ int s_n[2], s_low[2], s_small[2];
   const int sg = blockIdx.x, hd = blockIdx.y;
@@ -128,7 +130,7 @@ scan_chunk_kernel(const ScanArgs<T> a) {
   T pr[TG], pk[TG], pw[TG], pa[TG], pv[4];
   const int chc = min(ch, D - 1), jc = min(j, D - 1);
   // the token of a lane's e-th value: an inner index of every product with V
-  const auto tok_of = [&](int e) { return 4 * lg + e; };
+  const auto tok_of = [&](int e) { return DELTA ? 4 * lg + e : 4 * e + lg; };
   // row t + i of `base`'s chunk at t0, column c (uniform base, 32-bit byte offset; i known when compiled)
   const auto get = [&](const T* base, long long ld, int t0, int t, int i, int c)
                        __attribute__((always_inline)) {
@@ -146,7 +148,7 @@ scan_chunk_kernel(const ScanArgs<T> a) {
       if (DELTA) pa[q] = get(a.al, a.lda, t0, tg * TG, q, chc);
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) pv[e] = get(a.v, a.ldv, t0, tok_of(0), e, jc);
+    for (int e = 0; e < 4; ++e) pv[e] = get(a.v, a.ldv, t0, tok_of(0), DELTA ? e : 4 * e, jc);
   };
   if (tid < 2) { s_n[tid] = kC; s_low[tid] = s_small[tid] = 0; }
   fetch(0);
@@ -156,7 +158,7 @@ scan_chunk_kernel(const ScanArgs<T> a) {
     float rv[TG], kv[TG], wv[TG], av[TG];
     {
       unsigned top = 0u, low = ~0u, lim = 0u;   // r and k: largest, smallest - 1; the others: largest
-      float gp = 1.f;
+      double gp = 1.;
 #pragma unroll
       for (int q = 0; q < TG; ++q) {
         const bool live = t0 + tg * TG + q < len && chan;
@@ -204,7 +206,7 @@ scan_chunk_kernel(const ScanArgs<T> a) {
     if (s_n[par] < kC || s_low[par] || s_small[par]) {   // a shorter chunk (one decision for the workgroup)
       if (!DELTA) {                      // where does a channel's product leave the range?
         const float least = s_small[par] ? kSmallP : kMinP;
-        float p = 1.f;
+        double p = 1.;
         for (int g = 0; g < tg; ++g) p *= s_gp[g][ch];
 #pragma unroll
         for (int q = 0; q < TG; ++q) {
@@ -213,7 +215,7 @@ scan_chunk_kernel(const ScanArgs<T> a) {
         }
       }
       __syncthreads();
-      float p = 1.f;                     // the rows that are left for the next chunk decay nothing
+      double p = 1.;                     // the rows that are left for the next chunk decay nothing
 #pragma unroll
       for (int q = 0; q < TG; ++q) {
         if (tg * TG + q >= s_n[par]) wv[q] = 1.f;
@@ -225,12 +227,12 @@ scan_chunk_kernel(const ScanArgs<T> a) {
     const int n = __builtin_amdgcn_readfirstlane(min(s_n[par], len - t0));
     if (tid == 0) { s_n[par ^ 1] = kC; s_low[par ^ 1] = s_small[par ^ 1] = 0; }
     // ---- the scaled rows ----
-    float P = 1., Q = 1.f;               // decay of the token groups before and after this one
+    double P = 1., Q = 1.;               // decay of the token groups before and after this one
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
-      const float q = s_gp[g][ch];
-      P *= g < tg ? q : 1.f;
-      Q *= g > tg ? q : 1.f;
+      const double q = s_gp[g][ch];
+      P *= g < tg ? q : 1.;
+      Q *= g > tg ? q : 1.;
     }
 #pragma unroll
     for (int q = TG - 1; q >= 0; --q) {  // decayed to the chunk's end
@@ -340,7 +342,12 @@ scan_chunk_kernel(const ScanArgs<T> a) {
     }
     __syncthreads();                     // chunk matrices complete
     const auto small = [&](int m, const f32x4& x, f32x4 acc) {
-      const float4 y = *reinterpret_cast<const float4*>(&s_m[m][lr * LP + 4 * lg]);
+      float4 y;
+      if (DELTA) y = *reinterpret_cast<const float4*>(&s_m[m][lr * LP + 4 * lg]);
+      else {
+        const float* r = &s_m[m][lr * LP + lg];
+        y = make_float4(r[0], r[4], r[8], r[12]);
+      }
       acc = mma(y.x, x[0], acc);
       acc = mma(y.y, x[1], acc);
       acc = mma(y.z, x[2], acc);
@@ -364,15 +371,31 @@ scan_chunk_kernel(const ScanArgs<T> a) {
       for (int e = 0; e < 4; ++e)
         if (4 * lg + e < n) o[(unsigned)(4 * lg) * HD + (unsigned)e * HD + (unsigned)j] = O[e];
     }
-    // ---- the state moves on ----
+    // ---- the state moves on.  wkv: decayed, then the tokens' terms in order, the last (and least decayed)
+    // ones last, so that a fast channel sees few roundings.  Delta: what the chunk adds is summed apart, in
+    // fours, and meets the state in one rounding; added term by term to it the error was 1.4 - 1.6 times
+    // the serial walk's ----
 #pragma unroll
     for (int b = 0; b < KB; ++b) {
       const float4 P = *reinterpret_cast<const float4*>(&s_P[16 * b + 4 * lg]);
-      S[b][0] *= P.x; S[b][1] *= P.y; S[b][2] *= P.z; S[b][3] *= P.w;
+      const float p[4] = {P.x, P.y, P.z, P.w};
+      if (DELTA) {
+        f32x4 d[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        S[b] = mma(s_k[(4 * lg + e) * LK + 16 * b + lr], V[e], S[b]);
-        if (DELTA) S[b] = mma(s_b[(4 * lg + e) * LK + 16 * b + lr], C[e], S[b]);
+        for (int e = 0; e < 4; ++e) {
+          const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+          d[e] = mma(s_k[(4 * lg + e) * LK + 16 * b + lr], V[e], zero) +
+                 mma(s_b[(4 * lg + e) * LK + 16 * b + lr], C[e], zero);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          S[b][e] = fmaf(p[e], S[b][e], (d[0][e] + d[1][e]) + (d[2][e] + d[3][e]));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[b][e] *= p[e];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          S[b] = mma(s_k[(4 * e + lg) * LK + 16 * b + lr], V[e], S[b]);
       }
     }
     t0 = next;

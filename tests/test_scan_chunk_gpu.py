@@ -167,3 +167,26 @@ def test_a_total_decay_leaves_nothing():
     run("wkv", x, w0, ub, nw, state, seg, H, D)
     _, S = exact("wkv", x, w0, ub, nw, torch.zeros(H, D, D).double(), H, D)
     assert (state[0].cpu().double() - S).norm() <= 2e-6 * S.norm()
+
+
+@pytest.mark.parametrize("kind,D", [("wkv", 64), ("delta", 64), ("delta", 128)])
+def test_state_is_no_further_from_float64_than_the_serial_walk(kind, D, monkeypatch):
+    import lumen.ops.recurrent as R
+
+    H, err = 2, []
+    g = torch.Generator().manual_seed(D)
+    cu, seg = batch([400, 300], 0, [0, 5])
+    x = rows(cu[-1], H, D, torch.bfloat16, g, 0)
+    w0 = torch.linspace(-3, 1, H * D).cuda()
+    ub, nw = 0.5 * torch.randn(H * D, generator=g).cuda(), torch.ones(H * D).cuda()
+    before = torch.randn(2, H, D, D, generator=g).cuda()
+    want = [exact(kind, [t[a:b] for t in x], w0, ub, nw, before[1 - i].cpu().double() * i, H, D)[1]
+            for i, (a, b) in enumerate(zip(cu, cu[1:]))]
+    for portions in (R._chunk_portions, lambda *a, **k: 0):          # the chunked kernel, the serial one
+        monkeypatch.setattr(R, "_chunk_portions", portions)
+        state = before.clone()
+        run(kind, x, w0, ub, nw, state, seg, H, D)
+        err.append(sum(((state[1 - i].cpu().double() - S).norm() / S.norm()).item()
+                       for i, S in enumerate(want)))
+    # measured over 36 portions: 0.94 - 1.0 of the serial walk's on average, +- 0.05 for one draw
+    assert err[0] <= 1.1 * err[1], err

@@ -299,22 +299,34 @@ def split_cols(M: int, N: int) -> int:
 
 # A shape that the tuned table does not hold takes the library's own choice, a 256 x 256 stream-K kernel that
 # pays for an unfilled last wave with more than the wave (0.9 - 1.25 PFLOP/s against 1.45 on whole waves).  Cut
-# at the last whole wave, from two waves on, us: 4010 x 22016 x 4096 662 -> 509, x 11008 408 -> 261, 4010 x 11264 x
-# 2048 166 -> 141, 1900 x 22016 x 4096 395 -> 258, 8000 x 11008 x 4096 619 -> 488; of 29 shapes with 1900 - 8000
-# rows two lost more than noise (3300 x 12288 248 -> 256).  With one whole wave it is even (2305 x 12288 168 ->
-# 176, 2048 x 11008 159 -> 143): left whole.
+# after ``waves`` times as many columns of tiles as fit one wave, from two waves on, us: 4010 x 22016 x 4096
+# 637 -> 490, x 11008 407 -> 266, 4010 x 11264 x 2048 162 -> 141, 1300 x 22016 x 4096 299 -> 207, 300 x 95744 x
+# 4096 325 -> 238, 8000 x 11008 x 4096 627 -> 477.  Taking the columns that fill the waves nearest instead
+# (39 of 43 at 3100 rows x 11008: 507 of 512 tiles) sends the main part back to stream-K: 354 -> 369, with 38
+# columns 218.  With one whole wave it is even (2305 x 12288 173 -> 172): left whole.
+# Where the row tiles do not divide 256, every wave of the main part leaves 256 mod tm tiles to the rest.  Up to 8
+# waves that costs less than stream-K does even when the rest passes one wave (4874 x 22016: 734 -> 647, 5100 x
+# 22016 x 2048 in fp16 369 -> 379); from 9 on it does not (5100 x 32000 897 -> 1032, 7300 x 25344 580 -> 644):
+# left whole.  So is everything over 32 row tiles, where both forms win by turns (16000 x 25344 1252 -> 1173,
+# 9500 x 12288 667 -> 732, 11000 x 12288 819 -> 1039).  Over 250 timings of cuts by this rule (300 - 8000 rows, K
+# 2048 - 4096, both types) the mean is 0.90 of the whole product's time; 19 are more than 2.5 % above it,
+# most of them at 1300 - 1536 rows and 2.3 - 2.9 waves (1500 x 28672 x 2048 139 -> 153, worst 116 -> 129).
 WAVE_MIN, WAVE_MIN_K = 2, 2048
+WAVE_MAX_TM, WAVE_SPILL_MAX = 32, 8
 MIN_CUT = 1 << 23
 
 
 def wave_cols(M: int, N: int, K: int) -> int:
     """Column count of the whole waves of 256 x 256 tiles of an [M, N] output with any M (0: no cut)."""
     tm, tn = -(-M // SPLIT_TILE), -(-N // SPLIT_TILE)
-    if not 0 < tm <= SPLIT_CUS or N % 8 or K < WAVE_MIN_K:
+    if not 0 < tm <= WAVE_MAX_TM or N % 8 or K < WAVE_MIN_K:
         return 0
     waves, tail = divmod(tm * tn, SPLIT_CUS)
     n1 = waves * (SPLIT_CUS // tm) * SPLIT_TILE
-    return n1 if waves >= WAVE_MIN and tail and 0 < n1 < N else 0
+    if waves < WAVE_MIN or not tail or not 0 < n1 < N:
+        return 0
+    rest = tail + waves * (SPLIT_CUS % tm)
+    return n1 if waves <= WAVE_SPILL_MAX or rest <= SPLIT_CUS else 0
 
 
 _tuned: dict = {"n": -1, "sigs": frozenset()}

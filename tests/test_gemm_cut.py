@@ -5,17 +5,33 @@ from lumen.ops import gemm
 
 
 def test_wave_cols():
-    for M in (1, 255, 256, 1900, 2048, 4010, 4096, 8000, 65536, 65537, 1 << 20):
-        for N in (8, 1000, 2048, 4096, 11008, 11264, 12288, 22016, 22020, 32000):
+    cuts = 0
+    for M in (1, 255, 256, 300, 1300, 1900, 2048, 3300, 4010, 4096, 4874, 5120, 6500, 7300, 8000, 8192, 8193,
+              9500, 65536, 65537, 1 << 20):
+        for N in (8, 1000, 2048, 4096, 11008, 11264, 12288, 22016, 22020, 25344, 32000, 95744):
             n1 = gemm.wave_cols(M, N, 4096)
             tm, tn = -(-M // 256), -(-N // 256)
             assert n1 % 256 == 0 and 0 <= n1 < N
             if n1 or gemm.split_cols(M, N):
                 assert M * N >= gemm.MIN_CUT
-            if n1:
-                assert N % 8 == 0 and tm * tn % 256 and n1 // 256 * tm >= 2 * (256 // tm) * tm
+            if not n1:
+                continue
+            cuts += 1
+            assert N % 8 == 0 and tm * tn % 256 and M <= 8192          # the measured range
+            # the main part: at least two whole waves of the columns of tiles that fit one
+            per_wave = 256 // tm
+            waves = n1 // 256 // per_wave
+            assert n1 // 256 % per_wave == 0 and 2 <= waves <= tm * tn // 256
+            # no wave more than in one piece, but up to 8 waves, where a rest of two was faster all the same
+            rest = tm * (tn - n1 // 256)
+            if waves > 8:
+                assert waves + -(-rest // 256) <= -(-tm * tn // 256)
             assert gemm.wave_cols(M, N, 1024) == 0
+    assert cuts > 60
     assert gemm.wave_cols(4010, 22016, 4096) == 20480
+    assert gemm.wave_cols(4874, 22016, 4096) == 72 * 256        # 20 row tiles: 12 columns a wave
+    assert gemm.wave_cols(5100, 32000, 4096) == 0               # 9 waves, 340 tiles left: one wave more
+    assert gemm.wave_cols(7300, 25344, 2048) == gemm.wave_cols(6500, 32000, 4096) == 0
     assert gemm.wave_cols(4096, 4096, 4096) == 0                # whole waves already
 
 

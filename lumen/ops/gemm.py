@@ -347,6 +347,14 @@ def _tuned_sigs() -> frozenset:
     return _tuned["sigs"]
 
 
+def _tuning() -> bool:
+    """Is TunableOp timing solutions?  Its rotating copies of C start at the column view's address and
+    would read past the buffer's end (utils/gemm_tuning.py): then no untuned product is cut."""
+    import torch.cuda.tunable as tn
+
+    return tn.is_enabled() and tn.tuning_is_enabled()
+
+
 def _split_plan(x: torch.Tensor, w: torch.Tensor) -> int:
     if not (GEMM_SPLIT and x.is_cuda and x.dim() == 2 and w.dim() == 2 and x.stride(1) == 1
             and w.stride(1) == 1):
@@ -371,7 +379,8 @@ def _split_plan(x: torch.Tensor, w: torch.Tensor) -> int:
         if len(_plans) >= MAX_PLANS:
             _plans.clear()
         _plans[key] = hit
-    return hit if hit and _plain(x, w) and x.dtype == w.dtype and x.dtype != torch.float32 else 0
+    return hit if (hit and _plain(x, w) and x.dtype == w.dtype and x.dtype != torch.float32
+                   and not _tuning()) else 0
 
 
 _plans: dict = {}

@@ -41,3 +41,30 @@ def test_cpu_and_tracked_calls_keep_one_product():
     y.sum().backward()
     assert torch.allclose(y, x @ w.t()) and x.grad is not None
     assert gemm.split_slices(x, w) == 0 and gemm._split_plan(x, w) == 0
+
+
+def on_gpu(monkeypatch, enabled=True, tuning=False, results=()):
+    """CPU (meta) tensors taken for the GPU's, and a tuned table that says so."""
+    import torch.cuda.tunable as tn
+
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    monkeypatch.setattr(tn, "is_enabled", lambda: enabled)
+    monkeypatch.setattr(tn, "tuning_is_enabled", lambda: tuning)
+    monkeypatch.setattr(tn, "get_results", lambda: list(results))
+    monkeypatch.setattr(gemm, "_plans", {})
+    monkeypatch.setattr(gemm, "_tuned", dict(gemm._tuned, n=-1))
+
+
+def operands(M, N, K, dt=torch.bfloat16):
+    return (torch.empty(M, K, dtype=dt, device="meta"), torch.empty(N, K, dtype=dt, device="meta"))
+
+
+def test_no_product_is_cut_while_solutions_are_timed(monkeypatch):
+    """TunableOp's rotating copies of a column view read past the end of the buffer it is a view of."""
+    x, w = operands(4010, 22016, 4096)
+    on_gpu(monkeypatch)
+    assert gemm._split_plan(x, w) == 20480
+    on_gpu(monkeypatch, tuning=True)
+    assert gemm._split_plan(x, w) == 0
+    on_gpu(monkeypatch, enabled=False, tuning=True)
+    assert gemm._split_plan(x, w) == 20480

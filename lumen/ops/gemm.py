@@ -329,11 +329,13 @@ def wave_cols(M: int, N: int, K: int) -> int:
     return n1 if waves <= WAVE_SPILL_MAX or rest <= SPLIT_CUS else 0
 
 
-_tuned: dict = {"n": -1, "sigs": frozenset()}
+_tuned: dict = {"n": -1, "sigs": {}}
+_OP = {torch.bfloat16: "GemmTunableOp_BFloat16_TN", torch.float16: "GemmTunableOp_Half_TN"}
 
 
-def _tuned_sigs() -> frozenset:
-    """Problem signatures of the loaded TunableOp table (refreshed when its size changes)."""
+def _tuned_sigs(dtype: torch.dtype) -> frozenset:
+    """Problem signatures that the loaded TunableOp table holds for x @ w^T in ``dtype`` (read again when
+    the table's size changes)."""
     try:
         import torch.cuda.tunable as tn
 
@@ -343,8 +345,9 @@ def _tuned_sigs() -> frozenset:
     except Exception:  # noqa: BLE001
         return frozenset()
     if len(res) != _tuned["n"]:
-        _tuned["n"], _tuned["sigs"] = len(res), frozenset(r[1] for r in res)
-    return _tuned["sigs"]
+        _tuned["n"] = len(res)
+        _tuned["sigs"] = {dt: frozenset(r[1] for r in res if r[0] == op) for dt, op in _OP.items()}
+    return _tuned["sigs"][dtype]
 
 
 def _tuning() -> bool:
@@ -356,8 +359,8 @@ def _tuning() -> bool:
 
 
 def _split_plan(x: torch.Tensor, w: torch.Tensor) -> int:
-    if not (GEMM_SPLIT and x.is_cuda and x.dim() == 2 and w.dim() == 2 and x.stride(1) == 1
-            and w.stride(1) == 1):
+    if not (GEMM_SPLIT and x.is_cuda and x.dim() == 2 and w.dim() == 2 and x.dtype in _OP
+            and x.dtype == w.dtype and x.stride(1) == 1 and w.stride(1) == 1):
         return 0
     (M, K), N = x.shape, w.shape[0]
     if M * N < MIN_CUT:                            # less than one whole wave of tiles
@@ -366,25 +369,32 @@ def _split_plan(x: torch.Tensor, w: torch.Tensor) -> int:
     if not (n1 or n2):
         return 0
     # the first where both parts have tuned solutions, the second where neither the whole nor the parts
-    # have; decided once per problem (the table is loaded before the first training GEMM)
-    key = (M, N, K, w.stride(0), x.stride(0))
+    # have; decided once per problem, type and table (utils/gemm_tuning.py forgets the plans when it loads one)
+    key = (M, N, K, w.stride(0), x.stride(0), x.dtype)
     hit = _plans.get(key)
     if hit is None:
-        sigs = _tuned_sigs()
+        sigs = _tuned_sigs(x.dtype)
         lds = f"ld_{w.stride(0)}_{x.stride(0)}_{N}"
         if n1 and f"tn_{n1}_{M}_{K}_{lds}" in sigs and f"tn_{N - n1}_{M}_{K}_{lds}" in sigs:
-            hit = n1
+            hit = (n1, True)
         else:
-            hit = 0 if f"tn_{N}_{M}_{K}_{lds}" in sigs else n2
-        if len(_plans) >= MAX_PLANS:
-            _plans.clear()
-        _plans[key] = hit
-    return hit if (hit and _plain(x, w) and x.dtype == w.dtype and x.dtype != torch.float32
-                   and not _tuning()) else 0
+            hit = (0 if f"tn_{N}_{M}_{K}_{lds}" in sigs else n2, False)
+        if sigs:                                   # (no table: it may still be loaded)
+            if len(_plans) >= MAX_PLANS:
+                _plans.clear()
+            _plans[key] = hit
+    cols, tuned = hit
+    return cols if cols and _plain(x, w) and (tuned or not _tuning()) else 0
 
 
 _plans: dict = {}
-MAX_PLANS = 4096          # (M, N, K, strides) -> columns; ragged prompts bring a new M each
+MAX_PLANS = 4096          # (M, N, K, strides, type) -> columns; ragged prompts bring a new M each
+
+
+def forget_plans() -> None:
+    """The tuned table has changed: products are planned again."""
+    _plans.clear()
+    _tuned["n"] = -1
 
 
 def mm_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -393,7 +403,7 @@ def mm_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     n1 = _split_plan(x, w)
     if not n1:
         return matmul_nt(x, w)
-    y = torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=torch.result_type(x, w))
+    y = torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=x.dtype)
     torch.mm(x, w[:n1].t(), out=y[:, :n1])
     torch.mm(x, w[n1:].t(), out=y[:, n1:])
     return y

@@ -28,6 +28,8 @@ def load_tuned_gemms(path: Optional[str] = None) -> bool:
         return False
     import torch.cuda.tunable as tn
 
+    from ..ops.gemm import forget_plans
+
     tn.enable(True)
     tn.tuning_enable(False)
     try:
@@ -35,6 +37,7 @@ def load_tuned_gemms(path: Optional[str] = None) -> bool:
     except Exception:  # noqa: BLE001 - older builds
         pass
     ok = bool(tn.read_file(path))
+    forget_plans()
     if not ok:
         tn.enable(False)
     return ok
@@ -47,6 +50,8 @@ def start_gemm_tuning(out_path: str, max_ms: int = 60, rotating_mb: Optional[int
     Infinity Cache (``rotating_mb``, env ``LUMEN_TUNE_ROTATING_MB``, default 1024), i.e. with
     weights streaming from HBM as they do inside a training step, not from a warm cache."""
     import torch.cuda.tunable as tn
+
+    from ..ops.gemm import forget_plans
 
     if rotating_mb is None:
         rotating_mb = int(os.environ.get("LUMEN_TUNE_ROTATING_MB", "1024"))
@@ -62,6 +67,7 @@ def start_gemm_tuning(out_path: str, max_ms: int = 60, rotating_mb: Optional[int
     tn.set_max_tuning_iterations(100)
     if os.path.isfile(out_path):
         tn.read_file(out_path)
+    forget_plans()
 
 
 def tuned_entries() -> int:

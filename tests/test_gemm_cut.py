@@ -68,3 +68,30 @@ def test_no_product_is_cut_while_solutions_are_timed(monkeypatch):
     assert gemm._split_plan(x, w) == 0
     on_gpu(monkeypatch, enabled=False, tuning=True)
     assert gemm._split_plan(x, w) == 20480
+
+
+def test_plans_are_of_one_type_and_one_table(monkeypatch):
+    """A bf16 solution says nothing of the fp16 product, and a plan made before the table was there
+    does not outlive its loading."""
+    sig = "tn_22016_2048_4096_ld_4096_4096_22016"
+    cut = gemm.wave_cols(2048, 22016, 4096)
+    bf, half = operands(2048, 22016, 4096), operands(2048, 22016, 4096, torch.float16)
+    assert cut
+    on_gpu(monkeypatch, results=[("GemmTunableOp_BFloat16_TN", sig, "x", 1.0)])
+    for _ in range(2):
+        assert gemm._split_plan(*bf) == 0 and gemm._split_plan(*half) == cut
+    on_gpu(monkeypatch)                                          # before a table is loaded
+    assert gemm._split_plan(*bf) == cut
+    import torch.cuda.tunable as tn
+    monkeypatch.setattr(tn, "get_results", lambda: [("GemmTunableOp_BFloat16_TN", sig, "x", 1.0)])
+    assert gemm._split_plan(*bf) == 0 and gemm._split_plan(*half) == cut
+    # the whole-wave parts of 4096 rows: tuned in bf16 only
+    parts = [("GemmTunableOp_BFloat16_TN", f"tn_{n}_4096_4096_ld_4096_4096_22016", "x", 1.0)
+             for n in (20480, 1536)]
+    bf, half = operands(4096, 22016, 4096), operands(4096, 22016, 4096, torch.float16)
+    on_gpu(monkeypatch, results=parts + [("GemmTunableOp_Half_TN", "tn_22016_4096_4096_ld_4096_4096_22016",
+                                          "x", 1.0)])
+    assert gemm._split_plan(*bf) == 20480 and gemm._split_plan(*half) == 0
+    monkeypatch.setattr(tn, "get_results", lambda: [])
+    gemm.forget_plans()                                          # another table has been read
+    assert gemm._split_plan(*half) == gemm.wave_cols(4096, 22016, 4096)

@@ -153,26 +153,24 @@ def min_gru_sub() -> int:
     return int(_load().sm_min_gru_sub())
 
 
-def _arg(kind, v):
-    if kind == "p":
-        if v is None:
-            return None
-        if torch.is_tensor(v):
-            return v.data_ptr()
-        return v
-    if kind == "f":
-        return float(v)
-    return int(v)
-
-
 def call(name: str, *args) -> None:
     """Launch ``name`` on the current stream; tensors are passed by their data pointers."""
     lib = _load()
     sig = SIGNATURES[name]
     if len(args) != len(sig):
         raise TypeError(f"{name}: {len(args)} arguments for signature {sig!r}")
-    dev_t = next(a for a in args if torch.is_tensor(a))
-    stream = torch.cuda.current_stream(dev_t.device).cuda_stream
-    rc = getattr(lib, name)(*[_arg(k, a) for k, a in zip(sig, args)], stream)
+    dev, vals = None, []
+    for kind, v in zip(sig, args):                 # (host time: short prompts are bound by it)
+        if kind == "p":
+            if isinstance(v, torch.Tensor):
+                if dev is None:
+                    dev = v.device.index
+                v = v.data_ptr()
+        elif kind == "f":
+            v = float(v)
+        elif type(v) is not int:
+            v = int(v)
+        vals.append(v)
+    rc = getattr(lib, name)(*vals, torch._C._cuda_getCurrentRawStream(dev))
     if rc != 0:
         raise RuntimeError(f"{name}: HIP error {rc}")

@@ -67,17 +67,22 @@ THIN_MAX_W = 208 << 20
 
 def thin_ok(x: torch.Tensor, w: torch.Tensor, gemv: bool = True) -> bool:
     """Can and should the thin GEMM run x [M, K] @ w [N, K]^T?  ``gemv``: one row could go to the GEMV."""
-    if not (x.is_cuda and x.dim() == 2 and w.dim() == 2 and 0 < x.shape[0] <= THIN_MAX_M
-            and x.device == w.device and x.dtype == w.dtype and x.dtype in (torch.bfloat16, torch.float16)
-            and x.shape[1] == w.shape[1] and _plain(x, w) and w.is_contiguous() and x.stride(1) == 1
-            and x.stride(0) % 8 == 0 and x.stride(0) >= x.shape[1]):
+    xs, ws = x.shape, w.shape                      # (in order of host time: short prompts wait for it)
+    if len(xs) != 2 or not 0 < xs[0] <= THIN_MAX_M or len(ws) != 2 or not x.is_cuda:
         return False
-    (M, K), N = x.shape, w.shape[0]
-    if K == 0 or K % 64 or N % 4 or (x.data_ptr() | w.data_ptr()) % 16 or K >= 1 << 24:
+    (M, K), (N, Kw), dt = xs, ws, x.dtype
+    if (K != Kw or K % 64 or not 0 < K < 1 << 24 or N % 4 or dt != w.dtype
+            or dt not in (torch.bfloat16, torch.float16) or x.device != w.device):
         return False
     if M == 1 and gemv:
-        return K <= THIN_ROW_MAX_K and N * K < THIN_ROW_MAX_W
-    return N * K <= (THIN_MAX_W if M <= 32 else THIN_BATCH_MAX_W)
+        if K > THIN_ROW_MAX_K or N * K >= THIN_ROW_MAX_W:
+            return False
+    elif N * K > (THIN_MAX_W if M <= 32 else THIN_BATCH_MAX_W):
+        return False
+    if not _plain(x, w) or not w.is_contiguous():
+        return False
+    ld, one = x.stride()
+    return one == 1 and ld % 8 == 0 and ld >= K and (x.data_ptr() | w.data_ptr()) % 16 == 0
 
 
 def row_bias_ok(bias: Optional[torch.Tensor], x: torch.Tensor, N: int) -> bool:
@@ -99,24 +104,29 @@ def thin_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] =
     """x [M, K] @ w [N, K]^T (+ ``bias`` [N]) on the thin GEMM kernel, fp32 accumulation; the result
     in x's dtype or (``out_dtype``) fp32.  ``blocks`` = (wts [M, E], E, ff, ffs): K is E blocks of ff
     and one of ffs, and the blocks whose column of wts is all zero are taken as zero without being
-    read.  Callers ask ``thin_ok`` (and ``row_bias_ok``) first; the kernel is handed bare addresses, so what
-    does not fit them is an error here."""
-    from ._seqmix import DT, call, use_seqmix
-
-    use_seqmix(x)
+    read.  The kernel is handed bare addresses: what does not fit them is an error here."""
     if x.dim() != 2 or x.stride(1) != 1 or w.dim() != 2 or not w.is_contiguous() \
             or x.shape[1] != w.shape[1] or x.dtype != w.dtype or x.device != w.device:
         raise ValueError("few-row GEMM: rows x [M, K] and contiguous w [N, K] of one type and device")
-    (M, K), N = x.shape, w.shape[0]
+    K, N = x.shape[1], w.shape[0]
     if not row_bias_ok(bias, x, N):
         raise ValueError(f"few-row GEMM: the bias is not [{N}] contiguous values like x's")
     if blocks is not None:
         wts, E, ff, ffs = blocks
         if not weights_ok(wts, x, E) or E * ff + ffs != K:
             raise ValueError("few-row GEMM: routing weights [M, E] in fp32, K = E blocks of ff and one of ffs")
-    y = torch.empty(M, N, device=x.device, dtype=out_dtype or x.dtype)
-    call("sm_thin_gemm", DT[x.dtype], x, x.stride(0), w, bias, y, N, M, N, K,
-         int(y.dtype == torch.float32), *(blocks or (None, 0, 0, 0)))
+    return _thin(x, w, bias, out_dtype, blocks)
+
+
+def _thin(x, w, bias=None, out_dtype=None, blocks=None) -> torch.Tensor:
+    """``thin_linear`` of operands that ``thin_ok``, ``row_bias_ok`` and ``weights_ok`` have let pass."""
+    from ._seqmix import DT, call, use_seqmix
+
+    use_seqmix(x)
+    (M, K), N, dt = x.shape, w.shape[0], x.dtype
+    y = torch.empty((M, N), device=x.device, dtype=out_dtype or dt)
+    call("sm_thin_gemm", DT[dt], x, x.stride(0), w, bias, y, N, M, N, K, int(out_dtype is torch.float32),
+         *(blocks or (None, 0, 0, 0)))
     return y
 
 
@@ -131,9 +141,10 @@ SPLIT_MIN_M, SPLIT_MIN_K, SPLIT_MAX_S = 65, 8192, 8
 
 def split_slices(x: torch.Tensor, w: torch.Tensor) -> int:
     """Slices of K in which the split-K GEMM should run x [M, K] @ w [N, K]^T (0: leave it to the library)."""
-    if x.shape[-1] < SPLIT_MIN_K or x.dim() != 2 or w.dim() != 2 or not x.is_cuda:
+    xs = x.shape
+    if len(xs) != 2 or xs[1] < SPLIT_MIN_K or w.dim() != 2 or not x.is_cuda:
         return 0                                   # (nearly every call: as little host time as can be)
-    (M, K), (N, Kw) = x.shape, w.shape
+    (M, K), (N, Kw) = xs, w.shape
     tiles = -(-M // 256) * -(-N // 128)
     if not (M >= SPLIT_MIN_M and K == Kw and 0 < tiles <= 128):
         return 0
@@ -165,12 +176,14 @@ def matmul_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``F.linear`` of a served stack: few rows on the weight-streaming kernels (thin GEMM; GEMV for
     one row of a large matrix), the library otherwise."""
-    if x.dim() == 2 and x.shape[0] > THIN_MAX_M:       # (first: short prompts are bound by the host)
-        big = x.shape[1] >= SPLIT_MIN_K or x.shape[0] * w.shape[0] >= MIN_CUT
-        return mm_nt(x, w) if big and bias is None and x.is_cuda else F.linear(x, w, bias)
+    xs = x.shape
+    if len(xs) == 2 and xs[0] > THIN_MAX_M:            # (first: short prompts are bound by the host)
+        if bias is None and (xs[1] >= SPLIT_MIN_K or xs[0] * w.shape[0] >= MIN_CUT) and x.is_cuda:
+            return mm_nt(x, w)
+        return F.linear(x, w, bias)
     if thin_ok(x, w) and (bias is None or row_bias_ok(bias, x, w.shape[0]) and _plain(bias)):
-        return thin_linear(x, w, bias)
-    if bias is None and x.dim() == 2 and x.shape[0] == 1 and _plain(x, w) and skinny_ok(x, w):
+        return _thin(x, w, bias)
+    if bias is None and len(xs) == 2 and xs[0] == 1 and _plain(x, w) and skinny_ok(x, w):
         y = torch.empty(1, w.shape[0], device=x.device, dtype=x.dtype)
         native().skinny_gemm(x, w, y)
         return y
@@ -262,14 +275,17 @@ def dg_plans() -> dict:
 
 
 def dg_plan(x: torch.Tensor, w: torch.Tensor) -> Optional[tuple]:
-    if not (DGEMM and use_native(x) and x.dim() == 2 and w.dim() == 2 and 4 < x.shape[0] <= 256
-            and x.dtype == w.dtype and x.dtype in (torch.bfloat16, torch.float16)
+    if x.dim() != 2 or w.dim() != 2 or not 4 < x.shape[0] <= DG_BMS[-1]:
+        return None
+    bm = dg_bucket(x.shape[0])
+    p = dg_plans().get((w.shape[0], w.shape[1], bm))   # (most shapes have none: asked first)
+    if p is None:
+        return None
+    if not (DGEMM and use_native(x) and x.dtype == w.dtype and x.dtype in (torch.bfloat16, torch.float16)
             and x.stride(1) == 1 and x.stride(0) % 8 == 0 and w.is_contiguous()
             and x.shape[1] == w.shape[1] and w.shape[1] % 64 == 0 and w.shape[0] % 4 == 0):
         return None
-    bm = dg_bucket(x.shape[0])
-    p = dg_plans().get((w.shape[0], w.shape[1], bm))
-    return (bm,) + tuple(p) if p is not None else None
+    return (bm,) + tuple(p)
 
 
 # Training-shape GEMMs run 256 x 256 macro tiles, one per CU at a time, so a GEMM with 5.375 or
@@ -313,7 +329,7 @@ def split_cols(M: int, N: int) -> int:
 # most of them at 1300 - 1536 rows and 2.3 - 2.9 waves (1500 x 28672 x 2048 139 -> 153, worst 116 -> 129).
 WAVE_MIN, WAVE_MIN_K = 2, 2048
 WAVE_MAX_TM, WAVE_SPILL_MAX = 32, 8
-MIN_CUT = 1 << 23
+MIN_CUT = 1 << 24         # fewer elements than any cut product has
 
 
 def wave_cols(M: int, N: int, K: int) -> int:
@@ -359,12 +375,13 @@ def _tuning() -> bool:
 
 
 def _split_plan(x: torch.Tensor, w: torch.Tensor) -> int:
-    if not (GEMM_SPLIT and x.is_cuda and x.dim() == 2 and w.dim() == 2 and x.dtype in _OP
-            and x.dtype == w.dtype and x.stride(1) == 1 and w.stride(1) == 1):
+    xs, ws = x.shape, w.shape
+    if len(xs) != 2 or len(ws) != 2 or xs[0] * ws[0] < MIN_CUT:
+        return 0                                   # (nearly every call: as little host time as can be)
+    if not (GEMM_SPLIT and x.is_cuda and x.dtype in _OP and x.dtype == w.dtype and x.stride(1) == 1
+            and w.stride(1) == 1):
         return 0
-    (M, K), N = x.shape, w.shape[0]
-    if M * N < MIN_CUT:                            # less than one whole wave of tiles
-        return 0
+    (M, K), N = xs, ws[0]
     n1, n2 = split_cols(M, N), wave_cols(M, N, K)
     if not (n1 or n2):
         return 0
@@ -411,13 +428,15 @@ def mm_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 def linear_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x [M, K] @ w[N, K]^T -> [M, N]."""
-    if use_native(x) and thin_ok(x, w):
-        return thin_linear(x, w)
-    if skinny_ok(x, w):
-        y = torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=x.dtype)
-        native().skinny_gemm(x, w, y)
-        return y
-    p = dg_plan(x, w)
+    M = x.shape[0]
+    if M <= THIN_MAX_M:
+        if thin_ok(x, w) and use_native(x):
+            return _thin(x, w)
+        if skinny_ok(x, w):
+            y = torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=x.dtype)
+            native().skinny_gemm(x, w, y)
+            return y
+    p = dg_plan(x, w) if M <= DG_BMS[-1] else None
     if p is not None:
         return decode_gemm(x, w, *p)
     # prefill / mixed steps (M = 2048-4096 tokens): the whole-wave column split where both

@@ -26,6 +26,8 @@ from typing import Optional, Union
 import torch
 import torch.nn.functional as F
 
+from .gemm import _plain, _thin, project, row_bias_ok, thin_ok, weights_ok
+
 
 def route_topk_ref(z: torch.Tensor, top: int) -> torch.Tensor:
     val, idx = torch.sort(z.float(), dim=-1, descending=True, stable=True)  # ties: lowest index
@@ -55,11 +57,9 @@ def router_logits(h: torch.Tensor, w: torch.Tensor,
     16-bit values multiply exactly in fp32, so on the GPU the product runs on the matrix cores with
     fp32 accumulation and an fp32 result -- the arithmetic of an fp32 GEMM on the widened operands
     without the pass that widens them."""
-    from .gemm import _plain, row_bias_ok, thin_linear, thin_ok
-
     if thin_ok(h, w, gemv=False) and (bias is None or row_bias_ok(bias, h, w.shape[0])
                                       and _plain(bias)):
-        return thin_linear(h, w, bias, torch.float32)
+        return _thin(h, w, bias, torch.float32)
     if h.is_cuda and h.dtype == w.dtype and h.dtype in (torch.bfloat16, torch.float16):
         z = torch.mm(h, w.t(), out_dtype=torch.float32)
     else:
@@ -228,9 +228,7 @@ SPARSE_ROWS = 3
 def thin_act_ok(h, wts, gu_w, E: int, ff: int, ffs: int, act="silu", gated: bool = True,
                 weigh: str = "output") -> bool:
     """Can and should ``thin_act`` run the first projection and the activation in one kernel?"""
-    from .gemm import _plain, thin_ok, weights_ok
-
-    if not (h.is_cuda and h.dim() == 2 and 0 < h.shape[0] <= THIN_ACT_MAX_M and ff % 16 == 0
+    if not (h.dim() == 2 and 0 < h.shape[0] <= THIN_ACT_MAX_M and h.is_cuda and ff % 16 == 0
             and ffs % 16 == 0 and E * ff + ffs > 0 and E <= THIN_ACT_MAX_E
             and h.shape[0] * E <= THIN_ACT_MAX_WTS and (gated or isinstance(act, str))
             and (E == 0 or weights_ok(wts, h, E) and _plain(wts))):
@@ -247,38 +245,41 @@ def thin_act(h, gu_w, wts, E: int, ff: int, ffs: int, act="silu", gated: bool = 
              weigh: str = "output", sparse: bool = False) -> torch.Tensor:
     """``gated_act`` (or ``scaled_act``) of h @ gu_w^T, [T, E * ff + ffs], from the fp32 sums.
     ``sparse``: the blocks of experts that no row chose are left unwritten."""
-    from ._seqmix import DT, call, use_seqmix
-    from .gemm import weights_ok
-
-    use_seqmix(h)
     if weigh not in ("output", "input"):
         raise ValueError(f"unknown place of the routing weight {weigh!r}")
     if h.dim() != 2 or h.stride(1) != 1 or not gu_w.is_contiguous() or gu_w.dtype != h.dtype \
             or gu_w.device != h.device or (E and not weights_ok(wts, h, E)) \
             or tuple(gu_w.shape) != ((2 if gated else 1) * (E * ff + ffs), h.shape[1]):
         raise ValueError("few-row experts: rows h, stacked weights and routing weights do not fit")
-    out = torch.empty(h.shape[0], E * ff + ffs, dtype=h.dtype, device=h.device)
+    return _thin_act(h, gu_w, wts, E, ff, ffs, act, gated, weigh, sparse)
+
+
+def _thin_act(h, gu_w, wts, E, ff, ffs, act="silu", gated=True, weigh="output", sparse=False):
+    """``thin_act`` of operands that ``thin_act_ok`` has let pass."""
+    from ._seqmix import DT, call, use_seqmix
+
+    use_seqmix(h)
+    M, K = h.shape
+    out = torch.empty((M, E * ff + ffs), dtype=h.dtype, device=h.device)
     code, c = (GATE_ACTS[act], (0.0,) * 4) if isinstance(act, str) else (
         4, (act.limit, act.limit_shared, act.slope, act.shift))
-    call("sm_thin_act", DT[h.dtype], h, h.stride(0), gu_w, wts, out, h.shape[0], h.shape[1], E, ff,
-         ffs, int(gated), int(sparse), code, int(weigh == "input"), *c)
+    call("sm_thin_act", DT[h.dtype], h, h.stride(0), gu_w, wts, out, M, K, E, ff, ffs, int(gated),
+         int(sparse), code, int(weigh == "input"), *c)
     return out
 
 
 def moe_dense(h, wts, gu_w, down_w, E: int, ff: int, ffs: int, act="silu", gated: bool = True,
               weigh: str = "output", top: Optional[int] = None) -> torch.Tensor:
     """``top`` (optional): every row has at most that many non-zero weights."""
-    from .gemm import project, thin_linear
-
-    if thin_act_ok(h, wts, gu_w, E, ff, ffs, act, gated, weigh):
+    if h.shape[0] <= THIN_ACT_MAX_M and thin_act_ok(h, wts, gu_w, E, ff, ffs, act, gated, weigh):
         sparse = (top is not None and 0 < E and h.shape[0] * top <= SPARSE_ROWS * E
                   and ff % 64 == 0 and ffs % 64 == 0 and down_w.is_contiguous()
                   and down_w.dim() == 2 and down_w.shape[1] == E * ff + ffs
                   and down_w.dtype == h.dtype and down_w.device == h.device
                   and down_w.shape[0] % 4 == 0 and down_w.data_ptr() % 16 == 0)
-        a = thin_act(h, gu_w, wts, E, ff, ffs, act, gated, weigh, sparse)
+        a = _thin_act(h, gu_w, wts, E, ff, ffs, act, gated, weigh, sparse)
         if sparse:
-            return thin_linear(a, down_w, blocks=(wts, E, ff, ffs))
+            return _thin(a, down_w, blocks=(wts, E, ff, ffs))
         return project(a, down_w)
     return project(_act(project(h, gu_w), wts, E, ff, ffs, act, gated, weigh), down_w)
 
@@ -286,7 +287,9 @@ def moe_dense(h, wts, gu_w, down_w, E: int, ff: int, ffs: int, act="silu", gated
 def feed_forward(h, gu_w, down_w, ff: int, act="silu", gated: bool = True) -> torch.Tensor:
     """Dense feed-forward W_down (act(W_gate h) * W_up h) ([gate | up] rows stacked in ``gu_w``), or
     without a gate W_down act(W_up h)."""
-    return moe_dense(h, None, gu_w, down_w, 0, 0, ff, act, gated)
+    if h.shape[0] <= THIN_ACT_MAX_M and thin_act_ok(h, None, gu_w, 0, 0, ff, act, gated):
+        return project(_thin_act(h, gu_w, None, 0, 0, ff, act, gated), down_w)
+    return project(_act(project(h, gu_w), None, 0, 0, ff, act, gated, "output"), down_w)
 
 
 def moe_grouped(h, wts, gu_w, down_w, E: int, ff: int, ffs: int, act="silu", gated: bool = True,

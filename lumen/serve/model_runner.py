@@ -35,7 +35,7 @@ from ..ops.embedding import embedding
 from ..ops.attention import (flash_attention_fresh, flash_attention_paged, paged_decode,
                              rope_write_kv)
 from ..ops.gemm import linear_nt, swiglu_linear_nt
-from ..ops.moe import thin_act, thin_act_ok
+from ..ops.moe import THIN_ACT_MAX_M, thin_act, thin_act_ok
 from ..ops.norm import rms_norm
 from ..ops.rope import rope_tables
 
@@ -261,7 +261,7 @@ class ModelRunner:
             if ml is not None:
                 ml.apply(i, "o", o, a, masks, self._allreduce)
             y2, res = rms_norm(a, L.ln2, cfg.rms_norm_eps, res)
-            if (ml is None and DECODE_SPLIT_MIN == 0 and use_native(y2)
+            if (T <= THIN_ACT_MAX_M and ml is None and DECODE_SPLIT_MIN == 0 and use_native(y2)
                     and thin_act_ok(y2, None, L.gate_up, 0, 0, self.w.F)):
                 # few decode rows: the activation in the gate|up projection's epilogue (not for the halves
                 # of a split batch, which round the projection like the whole batch does)

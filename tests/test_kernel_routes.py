@@ -53,7 +53,7 @@ def test_second_projection_of_another_shape_is_not_read(launched, monkeypatch, d
     """A [W, K] that does not fit the activation goes to the library, whose error it always was; one
     of a width the kernel does not have (94) is multiplied there."""
     monkeypatch.setattr(M, "thin_act_ok", lambda *a, **k: True)
-    monkeypatch.setattr(M, "thin_act", lambda h, gu, wts, E, ff, ffs, *a: torch.zeros(
+    monkeypatch.setattr(M, "_thin_act", lambda h, gu, wts, E, ff, ffs, *a: torch.zeros(
         h.shape[0], E * ff + ffs, **BF))
     h, gu, wts = torch.zeros(3, 128, **BF), torch.zeros(384, 128, **BF), torch.zeros(3, 2)
     run = lambda: M.moe_dense(h, wts, gu, torch.zeros(*down, **BF), 2, 64, 64, top=1)  # noqa: E731

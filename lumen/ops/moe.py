@@ -226,8 +226,9 @@ SPARSE_ROWS = 3
 
 
 def thin_act_ok(h, wts, gu_w, E: int, ff: int, ffs: int, act="silu", gated: bool = True,
-                weigh: str = "output") -> bool:
-    """Can and should ``thin_act`` run the first projection and the activation in one kernel?"""
+                weigh: str = "output", sparse: bool = False) -> bool:
+    """Can and should ``thin_act`` run the first projection and the activation in one kernel?  ``sparse``:
+    it would read the chosen experts only."""
     if not (h.dim() == 2 and 0 < h.shape[0] <= THIN_ACT_MAX_M and h.is_cuda and ff % 16 == 0
             and ffs % 16 == 0 and E * ff + ffs > 0 and E <= THIN_ACT_MAX_E
             and h.shape[0] * E <= THIN_ACT_MAX_WTS and (gated or isinstance(act, str))
@@ -236,9 +237,11 @@ def thin_act_ok(h, wts, gu_w, E: int, ff: int, ffs: int, act="silu", gated: bool
     k = 2 if gated else 1
     if gu_w.shape[0] != k * (E * ff + ffs) or (weigh == "input" and not gated):
         return False
-    # thin_ok also says whether the thin kernel beats the GEMV (one row) or the library (huge matrices):
-    # of a stack of experts most are skipped
-    return thin_ok(h, gu_w[:16] if E else gu_w)
+    # thin_ok also says whether the thin kernel beats the library on a huge matrix, which a stack of experts
+    # is not a case of (16 rows of it stand for the strides), and for one row the GEMV on a long K.  The GEMV
+    # reads every expert: skipping wins at any width (one row, both projections, us: width 4096, 16 experts
+    # of 2816, top 3, and a shared one 174 -> 57, of 1408 94 -> 36; 4 of 1024, top 2 28 -> 20; ungated 120 -> 49).
+    return thin_ok(h, gu_w[:16] if E else gu_w, gemv=not sparse)
 
 
 def thin_act(h, gu_w, wts, E: int, ff: int, ffs: int, act="silu", gated: bool = True,
@@ -271,12 +274,13 @@ def _thin_act(h, gu_w, wts, E, ff, ffs, act="silu", gated=True, weigh="output", 
 def moe_dense(h, wts, gu_w, down_w, E: int, ff: int, ffs: int, act="silu", gated: bool = True,
               weigh: str = "output", top: Optional[int] = None) -> torch.Tensor:
     """``top`` (optional): every row has at most that many non-zero weights."""
-    if h.shape[0] <= THIN_ACT_MAX_M and thin_act_ok(h, wts, gu_w, E, ff, ffs, act, gated, weigh):
-        sparse = (top is not None and 0 < E and h.shape[0] * top <= SPARSE_ROWS * E
-                  and ff % 64 == 0 and ffs % 64 == 0 and down_w.is_contiguous()
-                  and down_w.dim() == 2 and down_w.shape[1] == E * ff + ffs
-                  and down_w.dtype == h.dtype and down_w.device == h.device
-                  and down_w.shape[0] % 4 == 0 and down_w.data_ptr() % 16 == 0)
+    M = h.shape[0]
+    sparse = (M <= THIN_ACT_MAX_M and top is not None and 0 < E and M * top <= SPARSE_ROWS * E
+              and ff % 64 == 0 and ffs % 64 == 0 and down_w.is_contiguous()
+              and down_w.dim() == 2 and down_w.shape[1] == E * ff + ffs
+              and down_w.dtype == h.dtype and down_w.device == h.device
+              and down_w.shape[0] % 4 == 0 and down_w.data_ptr() % 16 == 0 and _plain(down_w))
+    if M <= THIN_ACT_MAX_M and thin_act_ok(h, wts, gu_w, E, ff, ffs, act, gated, weigh, sparse):
         a = _thin_act(h, gu_w, wts, E, ff, ffs, act, gated, weigh, sparse)
         if sparse:
             return _thin(a, down_w, blocks=(wts, E, ff, ffs))

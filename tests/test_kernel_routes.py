@@ -191,3 +191,17 @@ def test_few_row_products_keep_gradients_tangents_and_batching(rows):
         assert tan is not None and near(tan.float(), (t @ w.t()).float())
     xr = x.clone().requires_grad_()
     assert M.router_logits(xr, w).requires_grad == torch.mm(xr, w.t(), out_dtype=torch.float32).requires_grad
+
+
+@pytest.mark.parametrize("M_,K,top,ff,kernels", [(1, 4096, 3, 64, 2), (2, 4096, 3, 64, 2), (1, 2048, 3, 64, 2),
+                                                 (1, 4096, 3, 48, 0), (1, 4096, None, 64, 0)])
+def test_one_row_skips_experts_at_any_width(launched, monkeypatch, M_, K, top, ff, kernels):
+    """The GEMV's limit on K is one of a matrix that is read whole: it holds where no expert is skipped."""
+    E = 16
+    h, wts = torch.zeros(M_, K, **BF), torch.zeros(M_, E)
+    gu, down = torch.zeros(2 * (E + 1) * ff, K, **BF), torch.zeros(64, (E + 1) * ff, **BF)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    monkeypatch.setattr(M, "project", lambda x, w, bias=None: torch.zeros(x.shape[0], w.shape[0], **BF))
+    monkeypatch.setattr(M, "_act", lambda z, wts, E, ff, ffs, *a: torch.zeros(z.shape[0], E * ff + ffs, **BF))
+    M.moe_dense(h, wts, gu, down, E, ff, ff, top=top)
+    assert [n for n, _ in launched] == ["sm_thin_act", "sm_thin_gemm"][:kernels]

@@ -123,3 +123,22 @@ def test_no_chosen_expert_gives_the_shared_one_alone():
     ref = moe_dense(h, None, gu[512:], down[:, 256:].contiguous(), 0, 0, 64)
     assert torch.equal(y, ref)
     assert not moe_dense(h, wts, gu[:512], down[:, :256].contiguous(), 4, 64, 0, top=1).any()
+
+
+def test_one_row_of_a_wide_model_skips_experts():
+    """Width 4096, where one dense row goes to the GEMV: experts nobody chose may hold anything."""
+    g = torch.Generator(device="cuda").manual_seed(4)
+    K, E, top, ff, ffs, W = 4096, 16, 3, 64, 128, 64
+    h = torch.randn(1, K, device="cuda", generator=g).bfloat16()
+    gu = (torch.randn(2 * (E * ff + ffs), K, device="cuda", generator=g) / K ** 0.5).bfloat16()
+    down = torch.randn(W, E * ff + ffs, device="cuda", generator=g).bfloat16()
+    wts = routed(1, E, top, g)
+    a = gated_act_ref(h.double() @ gu.double().t(), wts, E, ff, ffs).bfloat16().double()
+    ref = a @ down.double().t()
+    for e in (wts == 0).all(0).nonzero().flatten().tolist():
+        gu[e * 2 * ff:(e + 1) * 2 * ff] = float("nan")
+        down[:, e * ff:(e + 1) * ff] = float("nan")
+    y = moe_dense(h, wts, gu, down, E, ff, ffs, top=top)
+    # each activation may round to the other side (2^-7 of it at most, two neighbours), then the result rounds
+    slack = (a.abs() @ down.double().nan_to_num().abs().t()) * 2.0 ** -7
+    assert ((y.double() - ref).abs() <= slack + ref.abs() * 2.0 ** -8).all()

@@ -4,7 +4,8 @@
   targets, no CUDA, no hipify) -- these translation units include only HIP headers, so they
   rebuild in seconds;
 * ``cpu/cpu_adam.cpp`` (host AdamW for ZeRO-Offload) by the host compiler with OpenMP;
-* ``binding.cpp`` (pybind11 + torch headers, the slow one) only when it changed;
+* ``binding.cpp`` (pybind11 + torch headers, the slow one) only when it changed (a file is compiled when
+  it, a header or its compile command is not the one its object was made of);
 * linked into one shared object next to ``lumen/__init__.py`` so it travels with the repo
   snapshot to the GPU box (no JIT cache under ~/.cache).
 
@@ -45,8 +46,18 @@ MFMA_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 MFMA_FORM_FILES = ("lora_v3.hip", "head_scan_chunk16.hip", "recurrent_chunk.hip", "split_gemm.hip")
 
 
+# no packed-fp32 instructions (v_pk_*_f32): scalar fp32 code only
+KERNEL_FLAGS = ["-munsafe-fp-atomics", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-O3",
+                "-fPIC", "-std=c++17"]
+
+
 def _mfma_form(src: str) -> list:
     return MFMA_FORM if os.path.basename(src) in MFMA_FORM_FILES else []
+
+
+def _options(flags: list) -> str:
+    """The compile options that the sources do not show: part of a library's digest."""
+    return " ".join([*flags, "|", *MFMA_FORM, "|", *MFMA_FORM_FILES])
 
 
 def _torch_flags():
@@ -76,14 +87,15 @@ def sources() -> list:
 
 
 def source_digest() -> dict:
-    """{relative path: sha256} of ``sources()`` and their combined digest."""
+    """{relative path: sha256} of ``sources()`` and their combined digest, kernel options included."""
     import hashlib
 
     files = {}
     for f in sources():
         with open(f, "rb") as fh:
             files[os.path.relpath(f, PKG)] = hashlib.sha256(fh.read()).hexdigest()
-    total = hashlib.sha256("".join(f"{k}:{v};" for k, v in sorted(files.items())).encode())
+    total = hashlib.sha256((_options(KERNEL_FLAGS) + ";" + "".join(
+        f"{k}:{v};" for k, v in sorted(files.items()))).encode())
     return {"sha256": total.hexdigest(), "files": files}
 
 
@@ -109,13 +121,31 @@ def _newer(src_list, obj):
     return any(os.path.getmtime(s) > t for s in src_list)
 
 
+def _said(cmd) -> str:
+    """A compile command without its target."""
+    i = cmd.index("-o")
+    return " ".join([*cmd[:i], *cmd[i + 2:]])
+
+
+def _same_command(cmd, obj) -> bool:
+    """Was ``obj`` compiled by this command (kept beside it by ``_run``)?"""
+    try:
+        with open(obj + ".cmd") as f:
+            return f.read() == _said(cmd)
+    except OSError:
+        return False
+
+
 def _run(cmd):
     """Run a compile / link; its ``-o`` target is written under a temporary name and renamed
     on success, so an interrupted build never leaves a truncated object that looks current."""
     t0 = time.time()
+    said = _said(cmd)
     cmd = list(cmd)
     i = cmd.index("-o") + 1
     final = cmd[i]
+    if os.path.exists(final + ".cmd"):
+        os.remove(final + ".cmd")
     cmd[i] = tmp = f"{final}.part{os.getpid()}"
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
@@ -124,6 +154,9 @@ def _run(cmd):
             os.remove(tmp)
         raise RuntimeError(f"compile failed: {final}")
     os.replace(tmp, final)
+    if "-c" in cmd:
+        with open(final + ".cmd", "w") as f:
+            f.write(said)
     return time.time() - t0, r.stderr
 
 
@@ -154,32 +187,28 @@ def build(jobs: int = 8, force: bool = False, verbose: bool = True,
 
 def _build_locked(jobs, force, verbose, build_dir, out) -> str:
     headers = glob.glob(os.path.join(HERE, "kernels", "*.h"))
-    common = ["-O3", "-fPIC", "-std=c++17"]
     jobs_list = []
     objs = []
     for src in sorted(glob.glob(os.path.join(HERE, "kernels", "*.hip"))):
         obj = os.path.join(build_dir, os.path.basename(src) + ".o")
         objs.append(obj)
-        if force or _newer([src] + headers, obj):
-            # no packed-fp32 instructions (v_pk_*_f32): scalar fp32 code only
-            cmd = [HIPCC, f"--offload-arch={ARCH}", "-munsafe-fp-atomics", "-Xclang",
-                   "-target-feature", "-Xclang", "-packed-fp32-ops", *_mfma_form(src), *common, "-c", src,
-                   "-o", obj]
+        cmd = [HIPCC, f"--offload-arch={ARCH}", *KERNEL_FLAGS, *_mfma_form(src), "-c", src, "-o", obj]
+        if force or _newer([src] + headers, obj) or not _same_command(cmd, obj):
             jobs_list.append(cmd)
     cpu_src = os.path.join(HERE, "cpu", "cpu_adam.cpp")
     cpu_obj = os.path.join(build_dir, "cpu_adam.o")
     objs.append(cpu_obj)
-    if force or _newer([cpu_src], cpu_obj):
-        jobs_list.append(["g++", "-O3", "-fPIC", "-std=c++17", "-fopenmp", "-c", cpu_src, "-o",
-                          cpu_obj])
+    cmd = ["g++", "-O3", "-fPIC", "-std=c++17", "-fopenmp", "-c", cpu_src, "-o", cpu_obj]
+    if force or _newer([cpu_src], cpu_obj) or not _same_command(cmd, cpu_obj):
+        jobs_list.append(cmd)
     bind_src = os.path.join(HERE, "binding.cpp")
     bind_obj = os.path.join(build_dir, "binding.o")
     objs.append(bind_obj)
     cflags, ldflags = _torch_flags()
-    if force or _newer([bind_src], bind_obj):
-        # host-only translation unit: plain g++ against the HIP host API headers
-        jobs_list.append(["g++", "-O2", "-fPIC", "-std=c++17", f"-I{ROCM}/include", *cflags, "-c",
-                          bind_src, "-o", bind_obj])
+    # host-only translation unit: plain g++ against the HIP host API headers
+    cmd = ["g++", "-O2", "-fPIC", "-std=c++17", f"-I{ROCM}/include", *cflags, "-c", bind_src, "-o", bind_obj]
+    if force or _newer([bind_src], bind_obj) or not _same_command(cmd, bind_obj):
+        jobs_list.append(cmd)
     if jobs_list:
         with ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
             for cmd, (dt, _) in zip(jobs_list, ex.map(_run, jobs_list)):
@@ -229,7 +258,7 @@ def seqmix_sources() -> list:
 def seqmix_digest() -> str:
     import hashlib
 
-    h = hashlib.sha256(" ".join(SEQMIX_FLAGS + list(MFMA_FORM_FILES)).encode())
+    h = hashlib.sha256(_options(SEQMIX_FLAGS).encode())
     for f in seqmix_sources():
         with open(f, "rb") as fh:
             h.update(os.path.relpath(f, PKG).encode() + b":" + fh.read())

@@ -283,8 +283,9 @@ def test_concurrent_native_builds(tmp_path):
     bdir = tmp_path / "build"
     bdir.mkdir()
     for name in ("binding.o", "flash_attn.hip.o", "paged_attention.hip.o", "lora_v3.hip.o"):
-        if os.path.exists(os.path.join(seed_dir, name)):
-            shutil.copy2(os.path.join(seed_dir, name), bdir / name)
+        for f in (name, name + ".cmd"):
+            if os.path.exists(os.path.join(seed_dir, f)):
+                shutil.copy2(os.path.join(seed_dir, f), bdir / f)
     out = tmp_path / "ext" / "_C.so"
     code = ("import sys; sys.path.insert(0, %r); from lumen.csrc.build import build; "
             "build(jobs=2, build_dir=%r, out=%r)" % (ROOT, str(bdir), str(out)))
@@ -562,3 +563,37 @@ def test_box_hwmon_sampler_reads_fake_sysfs(tmp_path):
     assert "power_w_mean" not in s
     # CPU: no device properties -> no hwmon path
     assert gpu_hwmon() is None
+
+
+def test_build_follows_its_compile_options(monkeypatch, tmp_path):
+    """An object made with other options is compiled again, and a library of other options does not pass
+    for the tree's: file times and source hashes alone say nothing of them."""
+    from lumen.csrc import build as B
+
+    ran = []
+
+    def run(cmd):
+        ran.append(cmd)
+        out = cmd[cmd.index("-o") + 1]
+        with open(out, "w") as f:
+            f.write("x")
+        if "-c" in cmd:
+            with open(out + ".cmd", "w") as f:
+                f.write(B._said(cmd))
+        return 0.0, ""
+
+    monkeypatch.setattr(B, "_run", run)
+    kw = dict(verbose=False, build_dir=str(tmp_path / "b"), out=str(tmp_path / "_C.so"))
+    B.build(**kw)
+    first, digest = len(ran), B.source_digest()["sha256"]
+    assert first > 20
+    ran.clear()
+    B.build(**kw)
+    assert not ran and B.source_digest()["sha256"] == digest          # nothing to do
+    monkeypatch.setattr(B, "MFMA_FORM_FILES", B.MFMA_FORM_FILES[1:])  # lora_v3.hip without its option
+    seq = B.seqmix_digest()
+    B.build(**kw)
+    assert [os.path.basename(c[c.index("-c") + 1]) for c in ran if "-c" in c] == ["lora_v3.hip"]
+    assert len(ran) == 2 and B.source_digest()["sha256"] != digest    # ... and linked
+    monkeypatch.setattr(B, "MFMA_FORM", ["-mllvm", "-other"])
+    assert B.seqmix_digest() != seq

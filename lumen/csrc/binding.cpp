@@ -255,13 +255,13 @@ at::Tensor split_gemm(const at::Tensor& x, const at::Tensor& w, int64_t s) {
   if (!x.is_cuda() || !w.is_cuda() || x.device() != w.device())
     throw std::invalid_argument("lumen: split_gemm needs tensors of one GPU");
   if (x.dim() != 2 || w.dim() != 2 || x.stride(1) != 1 || w.stride(1) != 1 ||
-      x.size(1) != w.size(1) || x.scalar_type() != w.scalar_type() || s < 1)
+      x.size(1) != w.size(1) || x.scalar_type() != w.scalar_type() || s < 2)
     throw std::invalid_argument("lumen: split_gemm shape/layout mismatch");
   const int64_t M = x.size(0), N = w.size(0), tiles = (M + 255) / 256 * ((N + 127) / 128);
   at::Tensor y = at::empty({M, N}, x.options());
-  at::Tensor ws = at::empty({s > 1 ? s * tiles * 32768 : 0}, x.options().dtype(at::kFloat));
+  at::Tensor ws = at::empty({s * tiles * 32768}, x.options().dtype(at::kFloat));
   check(lumen_split_gemm(dcode(w), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(),
-                         N, s > 1 ? ws.data_ptr<float>() : nullptr, static_cast<int>(M),
+                         N, ws.data_ptr<float>(), static_cast<int>(M),
                          static_cast<int>(N), static_cast<int>(x.size(1)), static_cast<int>(s),
                          cur_stream()),
         "split_gemm");

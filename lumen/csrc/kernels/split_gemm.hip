@@ -78,7 +78,7 @@ __device__ __forceinline__ void done_reading() {
   asm volatile("" ::: "memory");
 }
 
-template <typename T, bool SPLIT>
+template <typename T>
 __global__ void __launch_bounds__(256, 1) split_gemm_kernel(const SplitArgs a) {
   __shared__ __attribute__((aligned(16))) char lds[NSTAGE * STAGE];
   const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
@@ -166,28 +166,12 @@ __global__ void __launch_bounds__(256, 1) split_gemm_kernel(const SplitArgs a) {
     half(1, next, -1, 0);     // (the last step reads a slot that holds an earlier stage: unused)
     slot = next;
   }
-  // lane (lr, lg) holds row 16 j + lr, columns 16 i + 4 lg .. + 3 of its wave's block
-  if constexpr (SPLIT) {
-    f32x4* o = (f32x4*)a.ws + (((long long)slice * a.tiles + tile) * 4 + wid) * (NI * MJ * 64) + lane;
+  // (lane (lr, lg) holds row 16 j + lr, columns 16 i + 4 lg .. + 3 of its wave's block)
+  f32x4* o = (f32x4*)a.ws + (((long long)slice * a.tiles + tile) * 4 + wid) * (NI * MJ * 64) + lane;
 #pragma unroll
-    for (int j = 0; j < MJ; ++j)
+  for (int j = 0; j < MJ; ++j)
 #pragma unroll
-      for (int i = 0; i < NI; ++i) o[(j * NI + i) * 64] = acc[i][j];
-  } else {
-    T* y = (T*)a.y;
-#pragma unroll
-    for (int j = 0; j < MJ; ++j) {
-      const int m = m0 + 128 * wm + 16 * j + lr;
-#pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int n = n0 + 64 * wn + 16 * i + 4 * lg;
-        float f[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) f[e] = acc[i][j][e];
-        if (m < a.M && n < a.N) store4(y + (long long)m * a.ldy + n, f);
-      }
-    }
-  }
+    for (int i = 0; i < NI; ++i) o[(j * NI + i) * 64] = acc[i][j];
 }
 
 // y = the sum of the S slabs, which lie in the order of the lanes that wrote them
@@ -214,26 +198,23 @@ __global__ void __launch_bounds__(256) split_sum_kernel(const SplitArgs a) {
 
 extern "C" {
 
-// y [M, N] = x [M, K] w [N, K]^T (16-bit, rows at ldx, ldw, ldy), K in S slices; ws: S * tiles * 32768 fp32
-// for S > 1.  K % 64 == 0, N % 4 == 0, rows of x and w at 16-byte addresses, of y at 8-byte ones.
+// y [M, N] = x [M, K] w [N, K]^T (16-bit, rows at ldx, ldw, ldy), K in S >= 2 slices; ws: S * tiles * 32768
+// fp32.  K % 64 == 0, N % 4 == 0, rows of x and w at 16-byte addresses, of y at 8-byte ones.
 hipError_t lumen_split_gemm(int dt, const void* x, long long ldx, const void* w, long long ldw, void* y,
                          long long ldy, float* ws, int M, int N, int K, int S, hipStream_t st) {
   using namespace lumen;
   using namespace lumen::sg;
   if ((long long)M * N == 0) return hipSuccess;
-  if (K <= 0 || K % BK || N % 4 || S < 1 || S > K / BK || ldx % 8 || ldw % 8 || ldy % 4 || ldx < K ||
-      ldw < K || ldy < N || ldx > (1 << 22) || ldw > (1 << 22) || (S > 1 && !ws) || (dt != kF16 && dt != kBF16) ||
+  if (K <= 0 || K % BK || N % 4 || S < 2 || S > K / BK || ldx % 8 || ldw % 8 || ldy % 4 || ldx < K ||
+      ldw < K || ldy < N || ldx > (1 << 22) || ldw > (1 << 22) || !ws || (dt != kF16 && dt != kBF16) ||
       ((uintptr_t)x | (uintptr_t)w | (uintptr_t)ws) % 16 || (uintptr_t)y % 8)
     return hipErrorInvalidValue;
   const long long tm = (M + BM - 1) / BM, tiles = tm * ((N + BN - 1) / BN);
   if (tiles * S >= (1 << 20)) return hipErrorInvalidValue;
   const SplitArgs a{x, ldx, w, ldw, y, ldy, ws, M, N, K, (int)tm, (int)tiles, S};
 #define CALL(TT)                                                                     \
-  if (S == 1) split_gemm_kernel<TT, false><<<(int)tiles, 256, 0, st>>>(a);           \
-  else {                                                                             \
-    split_gemm_kernel<TT, true><<<(int)tiles * S, 256, 0, st>>>(a);                  \
-    split_sum_kernel<TT><<<(int)tiles * NI * MJ, 256, 0, st>>>(a);                   \
-  }
+  split_gemm_kernel<TT><<<(int)tiles * S, 256, 0, st>>>(a);                          \
+  split_sum_kernel<TT><<<(int)tiles * NI * MJ, 256, 0, st>>>(a);
   if (dt == kBF16) { CALL(bf16) } else { CALL(fp16) }
 #undef CALL
   return hipGetLastError();

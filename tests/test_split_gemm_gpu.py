@@ -10,8 +10,8 @@ dev = "cuda"
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("M,N,K,S", [(65, 128, 64, 1), (256, 128, 128, 2), (257, 132, 192, 3), (300, 388, 576, 1),
-                                     (513, 260, 1088, 8), (1, 4, 320, 1), (512, 4096, 8192, 4)])
+@pytest.mark.parametrize("M,N,K,S", [(65, 128, 128, 2), (256, 128, 128, 2), (257, 132, 192, 3), (300, 388, 576, 4),
+                                     (513, 260, 1088, 8), (1, 4, 320, 5), (512, 4096, 8192, 4), (700, 1000, 512, 2)])
 def test_split_gemm(M, N, K, S, dt):
     g = torch.Generator().manual_seed(M + K)
     x = torch.randn(M, K + 8, generator=g).to(dt).to(dev)[:, :K]          # rows of a wider buffer

@@ -73,11 +73,35 @@ def test_tiled_rows(H, Dr, bs, opts, dtype, ulp, monkeypatch):
     assert ((got - want).abs() <= want.abs() * ulp + 1e-4 * want.abs().max()).all()
 
 
-def test_rule_and_row_kernel_agree():
-    """Steps below the rule's size, and sizes the kernel does not have, take the row kernel."""
+@pytest.mark.parametrize("rows,kernel", [(2047, "sm_latent_attn"), (2048, "sm_latent_tiles")])
+def test_rule_and_row_kernel_agree(rows, kernel, monkeypatch):
+    """The rule's two sides at its edge (rows x 16-head blocks), and the same step on the row kernel."""
     import lumen.ops._seqmix as sm
 
-    assert sm.latent_tiles_ok(2, 512, 576, 512, 16, 256)
+    H, R, Dr, bs = 16, 512, 64, 16
+    g = torch.Generator().manual_seed(rows)
+    T, seg, lat, vt = step([1024, rows - 1024], [0, 0], bs, R, Dr, torch.bfloat16, g)
+    assert seg.tile_rows * ((H + 15) // 16) == rows
+    q = torch.randn(T, H, R + Dr, generator=g).bfloat16().cuda()
+    calls = []
+    orig = sm.call
+    monkeypatch.setattr(sm, "call", lambda n, *a: (calls.append(n), orig(n, *a))[1])
+    out = [torch.zeros(H, T, R, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    for o, at in zip(out, (A.LATENT_TILE_ROWS, 1 << 30)):
+        monkeypatch.setattr(A, "LATENT_TILE_ROWS", at)
+        A.row_attention(q[:, :, :R], q[:, :, R:], lat, lat, R, o.transpose(0, 1), seg, H, 1, 0.05, vt=vt)
+    assert calls == [kernel, "sm_latent_attn"]
+    a, b = (o.float() for o in out)
+    assert torch.isfinite(a).all()
+    # each rounds an fp32 result once: a unit apart at most, and sums over <= 1024 keys in another order
+    assert ((a - b).abs() <= b.abs() * 2.0 ** -7 + 1e-4 * b.abs().max()).all()
+
+
+def test_sizes_the_tiled_kernel_has():
+    """The sizes it has, and sizes of which each is one step outside."""
+    import lumen.ops._seqmix as sm
+
+    assert sm.latent_tiles_ok(2, 512, 576, 512, 16, 256) and sm.latent_tiles_ok(1, 512, 512, 512, 4096, 4096)
     for dt, Dv, Dk, D1, bs, mb in ((0, 512, 576, 512, 16, 4), (2, 256, 320, 256, 16, 4),
                                    (2, 512, 544, 512, 16, 4), (2, 512, 576, 512, 8, 4),
                                    (2, 512, 576, 512, 48, 4), (2, 512, 576, 512, 16, 4097)):

@@ -15,7 +15,7 @@ dev = "cuda"
 @pytest.mark.parametrize("n,bucket,width,ld", [(1, 1, 1, 1), (1, 8, 3, 7), (64, 64, 40, 64), (257, 512, 9, 9),
                                                (5, 8, 0, 4)])
 @pytest.mark.parametrize("strided", [False, True])
-def test_fill_step(n, bucket, width, ld, strided):
+def test_fill_step(n, bucket, width, ld, strided, monkeypatch):
     g = torch.Generator().manual_seed(n)
     i32 = lambda *s: torch.randint(0, 1 << 30, s, generator=g, dtype=torch.int32).to(dev)  # noqa: E731
     i64 = lambda *s: torch.randint(0, 1 << 40, s, generator=g).to(dev)  # noqa: E731
@@ -33,7 +33,13 @@ def test_fill_step(n, bucket, width, ld, strided):
     want[3][:n], want[4][:n] = tok, slot
     want[4][n:] = -1
     want[5][:n, :width] = tab
+    called = []
+    real = _seqmix.call
+    monkeypatch.setattr(_seqmix, "call", lambda name, *a: (called.append(name), real(name, *a)))
     fill_step(list(zip(src, dst, pads)), tok, td, slot, sd, tab, bd, n, bucket)
+    # one launch for contiguous rows (of one entry, any stride is), copies for the others
+    one = all(t.is_contiguous() for t in src + [tok, slot, tab])
+    assert called == ["sm_fill_step"] * one and (one or strided)
     for w, d in zip(want, dst + [td, sd, bd]):
         assert torch.equal(w, d)
 

@@ -131,10 +131,11 @@ scan_chunk_kernel(const ScanArgs<T> a) {
   const int chc = min(ch, D - 1), jc = min(j, D - 1);
   // the token of a lane's e-th value: an inner index of every product with V
   const auto tok_of = [&](int e) { return DELTA ? 4 * lg + e : 4 * e + lg; };
-  // row t + i of `base`'s chunk at t0, column c (uniform base, 32-bit byte offset; i known when compiled)
+  // row t + i of `base`'s chunk at t0, column c (uniform base, 32-bit byte offset from the chunk's first row,
+  // so the rows that are left count up to a chunk's; i known when compiled)
   const auto get = [&](const T* base, long long ld, int t0, int t, int i, int c)
                        __attribute__((always_inline)) {
-    const unsigned step = (unsigned)ld, last = (unsigned)(len - 1 - t0) * step;
+    const unsigned step = (unsigned)ld, last = (unsigned)min(len - 1 - t0, kC - 1) * step;
     const unsigned at = min((unsigned)t * step + (unsigned)i * step, last) + (unsigned)c;
     return *reinterpret_cast<const T*>(
         reinterpret_cast<const char*>(base + (long long)(r0 + t0) * ld + col0) + at * (unsigned)sizeof(T));

@@ -63,6 +63,7 @@ THIN_MAX_M = 64
 THIN_ROW_MAX_K, THIN_ROW_MAX_W = 3072, 1 << 26
 THIN_BATCH_MAX_W = 24 << 20
 THIN_MAX_W = 208 << 20
+THIN_MAX_K, THIN_MAX_LD = 1 << 24, 1 << 25    # 64 rows lie within 32-bit byte offsets
 
 
 def thin_ok(x: torch.Tensor, w: torch.Tensor, gemv: bool = True) -> bool:
@@ -71,7 +72,7 @@ def thin_ok(x: torch.Tensor, w: torch.Tensor, gemv: bool = True) -> bool:
     if len(xs) != 2 or not 0 < xs[0] <= THIN_MAX_M or len(ws) != 2 or not x.is_cuda:
         return False
     (M, K), (N, Kw), dt = xs, ws, x.dtype
-    if (K != Kw or K % 64 or not 0 < K < 1 << 24 or N % 4 or dt != w.dtype
+    if (K != Kw or K % 64 or not 0 < K < THIN_MAX_K or N % 4 or dt != w.dtype
             or dt not in (torch.bfloat16, torch.float16) or x.device != w.device):
         return False
     if M == 1 and gemv:
@@ -82,7 +83,7 @@ def thin_ok(x: torch.Tensor, w: torch.Tensor, gemv: bool = True) -> bool:
     if not _plain(x, w) or not w.is_contiguous():
         return False
     ld, one = x.stride()
-    return one == 1 and ld % 8 == 0 and ld >= K and (x.data_ptr() | w.data_ptr()) % 16 == 0
+    return one == 1 and ld % 8 == 0 and K <= ld < THIN_MAX_LD and (x.data_ptr() | w.data_ptr()) % 16 == 0
 
 
 def row_bias_ok(bias: Optional[torch.Tensor], x: torch.Tensor, N: int) -> bool:

@@ -26,7 +26,7 @@ from typing import Optional, Union
 import torch
 import torch.nn.functional as F
 
-from .gemm import _plain, _thin, project, row_bias_ok, thin_ok, weights_ok
+from .gemm import THIN_MAX_K, _plain, _thin, project, row_bias_ok, thin_ok, weights_ok
 
 
 def route_topk_ref(z: torch.Tensor, top: int) -> torch.Tensor:
@@ -230,7 +230,7 @@ def thin_act_ok(h, wts, gu_w, E: int, ff: int, ffs: int, act="silu", gated: bool
     """Can and should ``thin_act`` run the first projection and the activation in one kernel?  ``sparse``:
     it would read the chosen experts only."""
     if not (h.dim() == 2 and 0 < h.shape[0] <= THIN_ACT_MAX_M and h.is_cuda and ff % 16 == 0
-            and ffs % 16 == 0 and E * ff + ffs > 0 and E <= THIN_ACT_MAX_E
+            and ffs % 16 == 0 and 0 < E * ff + ffs < THIN_MAX_K and E <= THIN_ACT_MAX_E
             and h.shape[0] * E <= THIN_ACT_MAX_WTS and (gated or isinstance(act, str))
             and (E == 0 or weights_ok(wts, h, E) and _plain(wts))):
         return False

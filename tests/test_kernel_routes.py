@@ -205,3 +205,18 @@ def test_one_row_skips_experts_at_any_width(launched, monkeypatch, M_, K, top, f
     monkeypatch.setattr(M, "_act", lambda z, wts, E, ff, ffs, *a: torch.zeros(z.shape[0], E * ff + ffs, **BF))
     M.moe_dense(h, wts, gu, down, E, ff, ff, top=top)
     assert [n for n, _ in launched] == ["sm_thin_act", "sm_thin_gemm"][:kernels]
+
+
+@pytest.mark.parametrize("M_", [1, 3])
+def test_rows_too_far_apart_for_the_kernels_offsets_stay_with_the_library(launched, monkeypatch, M_):
+    """The last rows of long sequences (hidden[:, -1]): 64 rows at the stride have to lie within 2^32 bytes."""
+    w = torch.zeros(8, 128, **BF)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    for ld, ok in (((1 << 25) - 8, True), (1 << 25, False)):
+        x = torch.empty(2 * ld + 128 if M_ > 1 else 128, device="meta", **BF).as_strided((M_, 128), (ld, 1))
+        assert gemm.thin_ok(x, w.to("meta")) == ok
+    h, wts = torch.empty(M_, 128, device="meta", **BF), torch.empty(M_, 1, device="meta")
+    for ffs, ok in ((0, True), (64, False)):             # the second projection's K
+        ff = (1 << 24) - 64
+        gu = torch.empty(2 * (ff + ffs), 128, device="meta", **BF)
+        assert M.thin_act_ok(h, wts, gu, 1, ff, ffs, sparse=True) == ok

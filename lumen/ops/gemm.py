@@ -362,8 +362,8 @@ def _tuned_sigs(dtype: torch.dtype) -> frozenset:
     except Exception:  # noqa: BLE001
         return frozenset()
     if len(res) != _tuned["n"]:
-        _tuned["n"] = len(res)
         _tuned["sigs"] = {dt: frozenset(r[1] for r in res if r[0] == op) for dt, op in _OP.items()}
+        _tuned["n"] = len(res)                     # (last: another thread may ask in between)
     return _tuned["sigs"][dtype]
 
 

@@ -95,3 +95,17 @@ def test_plans_are_of_one_type_and_one_table(monkeypatch):
     monkeypatch.setattr(tn, "get_results", lambda: [])
     gemm.forget_plans()                                          # another table has been read
     assert gemm._split_plan(*half) == gemm.wave_cols(4096, 22016, 4096)
+
+
+def test_table_is_whole_when_its_size_says_it_is_read(monkeypatch):
+    """A second thread that plans a product while the first reads the table."""
+    class Watched(dict):
+        def __setitem__(self, k, v):
+            super().__setitem__(k, v)
+            if k == "n":
+                seen.append(gemm._tuned_sigs(torch.bfloat16))
+
+    seen, sig = [], "tn_22016_2048_4096_ld_4096_4096_22016"
+    on_gpu(monkeypatch, results=[("GemmTunableOp_BFloat16_TN", sig, "x", 1.0)])
+    monkeypatch.setattr(gemm, "_tuned", Watched(n=-1, sigs={}))
+    assert gemm._tuned_sigs(torch.bfloat16) == {sig} and seen == [{sig}]

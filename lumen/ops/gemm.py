@@ -53,6 +53,13 @@ def _plain(*tensors: torch.Tensor) -> bool:
                 and torch.get_autocast_dtype("cuda") != tensors[0].dtype)
 
 
+def _here(x: torch.Tensor) -> bool:
+    """Is ``x`` on the current device?  The library follows its operands to another one; the kernels
+    launched from here take their memory and stream where the program is."""
+    i = x.device.index
+    return i is None or i == torch._C._cuda_getDevice()
+
+
 # Thin GEMM (seqmix/thin_gemm.hip, whose header holds the measurements).  One row where the GEMV could take it:
 # matrices under 128 MB with K <= 3072 (2048 x 2048: 3.8 vs 4.4 us with the GEMV; 2048 x 5632: 7.3 vs 6.6,
 # 22528 x 4096: 30.7 vs 28.5, and a batch-1 Llama step of 4 layers of width 4096: 432 vs 407 us -- those stay
@@ -80,7 +87,7 @@ def thin_ok(x: torch.Tensor, w: torch.Tensor, gemv: bool = True) -> bool:
             return False
     elif N * K > (THIN_MAX_W if M <= 32 else THIN_BATCH_MAX_W):
         return False
-    if not _plain(x, w) or not w.is_contiguous():
+    if not _plain(x, w) or not w.is_contiguous() or not _here(x):
         return False
     ld, one = x.stride()
     return one == 1 and ld % 8 == 0 and K <= ld < THIN_MAX_LD and (x.data_ptr() | w.data_ptr()) % 16 == 0
@@ -153,7 +160,7 @@ def split_slices(x: torch.Tensor, w: torch.Tensor) -> int:
     dt = x.dtype
     if (tiles * S < 128 or K % 64 or N % 4 or K >= 1 << 22 or dt != w.dtype
             or dt not in (torch.bfloat16, torch.float16) or x.device != w.device
-            or not _plain(x, w) or not use_native(x)):
+            or not _plain(x, w) or not _here(x) or not use_native(x)):
         return 0
     (lx, ex), (lw, ew) = x.stride(), w.stride()
     if (ex != 1 or ew != 1 or lx % 8 or lw % 8 or not K <= lx <= 1 << 22 or not K <= lw <= 1 << 22
@@ -184,7 +191,7 @@ def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = Non
         return F.linear(x, w, bias)
     if thin_ok(x, w) and (bias is None or row_bias_ok(bias, x, w.shape[0]) and _plain(bias)):
         return _thin(x, w, bias)
-    if bias is None and len(xs) == 2 and xs[0] == 1 and _plain(x, w) and skinny_ok(x, w):
+    if bias is None and len(xs) == 2 and xs[0] == 1 and _plain(x, w) and _here(x) and skinny_ok(x, w):
         y = torch.empty(1, w.shape[0], device=x.device, dtype=x.dtype)
         native().skinny_gemm(x, w, y)
         return y

@@ -220,3 +220,23 @@ def test_rows_too_far_apart_for_the_kernels_offsets_stay_with_the_library(launch
         ff = (1 << 24) - 64
         gu = torch.empty(2 * (ff + ffs), 128, device="meta", **BF)
         assert M.thin_act_ok(h, wts, gu, 1, ff, ffs, sparse=True) == ok
+
+
+@pytest.mark.parametrize("current,taken", [(1, True), (0, False)])
+def test_products_of_another_device_follow_the_library(launched, monkeypatch, current, taken):
+    """The kernels launch on the current device; the library goes where its operands are."""
+    class Second(torch.Tensor):
+        device = torch.device("cuda", 1)
+
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: current, raising=False)
+    for name in ("_plain", "use_native"):
+        monkeypatch.setattr(gemm, name, lambda *a: True)
+    on = lambda *s: torch.empty(*s, device="meta", **BF).as_subclass(Second)  # noqa: E731
+    assert gemm.thin_ok(on(3, 128), on(8, 128)) == taken
+    assert bool(gemm.split_slices(on(512, 8192), on(4096, 8192))) == taken
+    asked = []
+    monkeypatch.setattr(gemm, "skinny_ok", lambda *a: asked.append(a))
+    monkeypatch.setattr(gemm.F, "linear", lambda *a: None)
+    gemm.project(on(1, 4096), on(64, 4096))
+    assert bool(asked) == taken

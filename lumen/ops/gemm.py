@@ -336,14 +336,14 @@ def split_cols(M: int, N: int) -> int:
 # 2048 - 4096, both types) the mean is 0.90 of the whole product's time; 19 are more than 2.5 % above it,
 # most of them at 1300 - 1536 rows and 2.3 - 2.9 waves (1500 x 28672 x 2048 139 -> 153, worst 116 -> 129).
 WAVE_MIN, WAVE_MIN_K = 2, 2048
-WAVE_MAX_TM, WAVE_SPILL_MAX = 32, 8
+WAVE_MIN_M, WAVE_MAX_TM, WAVE_SPILL_MAX = 300, 32, 8
 MIN_CUT = 1 << 24         # fewer elements than any cut product has
 
 
 def wave_cols(M: int, N: int, K: int) -> int:
     """Column count of the whole waves of 256 x 256 tiles of an [M, N] output with any M (0: no cut)."""
     tm, tn = -(-M // SPLIT_TILE), -(-N // SPLIT_TILE)
-    if not 0 < tm <= WAVE_MAX_TM or N % 8 or K < WAVE_MIN_K:
+    if M < WAVE_MIN_M or tm > WAVE_MAX_TM or N % 8 or K < WAVE_MIN_K:
         return 0
     waves, tail = divmod(tm * tn, SPLIT_CUS)
     n1 = waves * (SPLIT_CUS // tm) * SPLIT_TILE

@@ -33,6 +33,7 @@ def test_wave_cols():
     assert gemm.wave_cols(5100, 32000, 4096) == 0               # 9 waves, 340 tiles left: one wave more
     assert gemm.wave_cols(7300, 25344, 2048) == gemm.wave_cols(6500, 32000, 4096) == 0
     assert gemm.wave_cols(4096, 4096, 4096) == 0                # whole waves already
+    assert gemm.wave_cols(300, 152064, 4096) == 2 * 128 * 2 * 256 and gemm.wave_cols(200, 152064, 4096) == 0
 
 
 def test_cpu_and_tracked_calls_keep_one_product():

@@ -454,8 +454,8 @@ def linear_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 # batch <= 4 decode, opt-in (LUMEN_SWIGLU_GEMV=1): SwiGLU formed inside the rows-per-lane weight
 # stream, one launch fewer per layer.  Measured slower both ways: the row-group GEMV form 21.4 vs
-# 18.5 us per call, the rows-per-lane form 3.085 vs 2.99-3.01 ms per batch-1 decode step (gpurun
-# r5_35) -- every workgroup re-reads and re-activates the whole 2 x 11008 gate|up row
+# 18.5 us per call, the rows-per-lane form 3.085 vs 2.99-3.01 ms per batch-1 decode step
+# -- every workgroup re-reads and re-activates the whole 2 x 11008 gate|up row
 SWIGLU_GEMV = os.environ.get("LUMEN_SWIGLU_GEMV", "0") == "1"
 
 

@@ -46,7 +46,7 @@ class _LMHeadCE(torch.autograd.Function):
     def backward(ctx, g):
         dlogits, h = ctx.saved_tensors
         # TN against the frozen head's cached W^T when it keeps one (K-contiguous operands:
-        # 778 vs 874 us at Llama-2-7B's 8 x 512 tokens, gpurun r5_55), else NN against W
+        # 778 vs 874 us at Llama-2-7B's 8 x 512 tokens), else NN against W
         wt = ctx.wt_fn() if ctx.wt_fn is not None else None
         dh = matmul_nt(dlogits, wt) if wt is not None else torch.matmul(dlogits, ctx.weight_fn())
         # upstream grad (a 0-dim f32 tensor): multiplied in f32 math, never cast to 16 bits

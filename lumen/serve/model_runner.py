@@ -10,7 +10,7 @@ Per layer (token-major activations, no autograd):
 A "mixed" step packs [prefill chunk tokens | decode tokens] into one forward (every GEMM sees
 all of them); a pure decode step replays a hipGraph.
 
-Tensor parallelism (SURVEY P9/X9-X11): Megatron-style column split of q|k|v and gate|up by
+Tensor parallelism: Megatron-style column split of q|k|v and gate|up by
 heads / FFN columns, row split of o and down followed by an all-reduce over the TP group.
 Rank 0 owns the scheduler; every step it broadcasts one int64 metadata tensor (token ids,
 positions, slots, block tables, lengths) so worker ranks run the same kernels (no pickling).
@@ -127,7 +127,7 @@ class ServeWeights:
                                           qkv, o, gu, dn))
         self.embed = model.embed_tokens.weight
         self.norm = model.norm.weight
-        # vocab-parallel LM head (SURVEY X10): each rank scores V/TP rows, logits all-gathered
+        # vocab-parallel LM head: each rank scores V/TP rows, logits all-gathered
         V = cfg.vocab_size
         self.vocab_shard = V // tp_size if V % tp_size == 0 else V
         lm = model.lm_head.weight

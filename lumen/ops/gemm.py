@@ -283,13 +283,13 @@ def dg_plans() -> dict:
 
 
 def dg_plan(x: torch.Tensor, w: torch.Tensor) -> Optional[tuple]:
-    if x.dim() != 2 or w.dim() != 2 or not 4 < x.shape[0] <= DG_BMS[-1]:
+    if not DGEMM or x.dim() != 2 or w.dim() != 2 or not 4 < x.shape[0] <= DG_BMS[-1] or not x.is_cuda:
         return None
     bm = dg_bucket(x.shape[0])
     p = dg_plans().get((w.shape[0], w.shape[1], bm))   # (most shapes have none: asked first)
     if p is None:
         return None
-    if not (DGEMM and use_native(x) and x.dtype == w.dtype and x.dtype in (torch.bfloat16, torch.float16)
+    if not (use_native(x) and x.dtype == w.dtype and x.dtype in (torch.bfloat16, torch.float16)
             and x.stride(1) == 1 and x.stride(0) % 8 == 0 and w.is_contiguous()
             and x.shape[1] == w.shape[1] and w.shape[1] % 64 == 0 and w.shape[0] % 4 == 0):
         return None

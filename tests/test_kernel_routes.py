@@ -240,3 +240,16 @@ def test_products_of_another_device_follow_the_library(launched, monkeypatch, cu
     monkeypatch.setattr(gemm.F, "linear", lambda *a: None)
     gemm.project(on(1, 4096), on(64, 4096))
     assert bool(asked) == taken
+
+
+def test_decode_plans_are_read_for_calls_that_can_use_one(monkeypatch, tmp_path):
+    """Neither with the plans switched off nor for CPU tensors (a file that is no table)."""
+    bad = tmp_path / "plans.json"
+    bad.write_text("{")
+    monkeypatch.setenv("LUMEN_DGEMM_PLANS", str(bad))
+    monkeypatch.setattr(gemm, "_dg_plans", None)
+    x, w = torch.zeros(70, 64, **BF), torch.zeros(8, 64, **BF)
+    assert gemm.dg_plan(x, w) is None and gemm.linear_nt(x, w).shape == (70, 8)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    monkeypatch.setattr(gemm, "DGEMM", False)
+    assert gemm.dg_plan(x, w) is None

@@ -168,9 +168,13 @@ chunk_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ 
 
 // ---- prefill tiles on the matrix cores (16-bit dtypes, D a multiple of 32) ---------------------
 // A workgroup of NW waves takes 32 * NW consecutive rows of ONE segment and one query head; the
-// keys the tile can see (from the first row's chunk start to the last row's position) are
-// visited 32 at a time, staged in LDS twice (row-major for the scores, transposed for the value
-// pass) and shared by the waves.  Per wave (32 queries) and key tile, with v_mfma_f32_32x32x16:
+// keys the tile can see (from the first row's chunk start to the last row's position) are visited KT = 64
+// at a time (32 for heads over 128), staged in LDS twice (row-major for the scores, transposed for the value
+// pass) and shared by the waves.  Bound by the chain of tiles at two waves per SIMD; the loads of a tile leave
+// together one tile ahead and two buffers leave one barrier per tile, as in window_attention.hip.  us, tiles of
+// 32 keys, one buffer -> now (bf16, heads of 128): 8 x 512 rows x 16 heads 83 -> 39, 1 x 200 28 -> 20, 32 of 12 -
+// 100 25 -> 15, 1 x 4096 x 32 (chunk 1024) 284 -> 123; heads of 64 45 -> 28, 96 49 -> 34, 256 113 -> 109.
+// Per wave (32 queries) and 32 keys, with v_mfma_f32_32x32x16:
 //   S^T = K Q^T      keys on the accumulator rows, queries on the columns (lane & 31): a lane
 //                    owns ONE query, so its running max / sum / correction are plain scalars;
 //                    q and k enter un-normalised (exactly as projected) and the two RMS factors
@@ -183,6 +187,8 @@ chunk_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ 
 //                    (two products), which keeps ~16 mantissa bits of the fp32 weights.
 // Accumulator layout of the 32x32 products: lane l, register 4j + i = row 8j + 4(l >> 5) + i,
 // column l & 31; operand lanes hold k = 8(l >> 5) + 0..7.
+constexpr float kRise = 5.f;      // log of the largest weight a tile may form before its maximum moves the reference
+
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8v __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8v __attribute__((ext_vector_type(8)));
@@ -226,27 +232,27 @@ __device__ __forceinline__ float sumsq8(uint4 v) {
   return s;
 }
 
-// (register budget: three waves per SIMD up to head size 128 -- 168 VGPRs, no scratch -- two
-// above; left to itself the compiler takes > 300 registers and runs one wave per SIMD, which
-// measured slower than the staging it was meant to speed up)
-template <typename T, int D, int NW>
-__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 3 : 2)))
+// (register budget: left to itself the compiler takes > 300 registers and runs one wave per SIMD.  Two waves
+// for heads of 96 and 128, where three spill; of 256 two with spills are ahead of one without, 109 us against 135)
+template <typename T, int D, int NW, int KT>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 3 : 2)))
 tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ cache,
                  T* __restrict__ out, const int* __restrict__ tables, int maxb,
                  const int* __restrict__ tiles, const int* __restrict__ cu,
                  const int* __restrict__ start, int H, int G, int bs, float scale, float eps,
                  int chunk, int sink) {
-  constexpr int QT = 32 * NW, LK = D + 8, LT = 40, NV = D / 8;
-  __shared__ __align__(16) T s_k[32 * LK];    // key tile, row-major
-  __shared__ __align__(16) T s_t[D * LT];     // key tile, transposed [d][key]
-  __shared__ float s_kn[32];                  // 1 / rms of the tile's keys (power-of-two D / 8)
+  constexpr int QT = 32 * NW, LK = D + 8, LT = KT + 8, NV = D / 8, SB = KT / 32;
+  // two buffers: a tile is stored while the one before it is read, one barrier per tile
+  __shared__ __align__(16) T s_kb[2][KT * LK];    // key tile, row-major
+  __shared__ __align__(16) T s_tb[2][D * LT];     // key tile, transposed [d][key]
+  __shared__ float s_nb[2][KT];                   // 1 / rms of the tile's keys (power-of-two D / 8)
   constexpr int kTbl = 512;                   // block-table entries of the visible keys, in LDS
   __shared__ int s_tbl[kTbl];
   constexpr bool kStagedNorm = (NV & (NV - 1)) == 0 && NV <= 64;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 31, hi = lane >> 5;
-  const int hd = blockIdx.y, g = hd / (H / G);
-  // tiles are listed in row order, so later tiles see more keys: issue them first
-  const int tix = gridDim.x - 1 - blockIdx.x;
+  int tix, hd;
+  heavy_first(blockIdx.x, gridDim.x, H, tix, hd);
+  const int g = hd / (H / G);
   const int sg = tiles[2 * tix], row0 = tiles[2 * tix + 1];
   const int seg_r0 = cu[sg], p0 = start[sg];
   const int nrows = min(QT, cu[sg + 1] - row0);
@@ -273,14 +279,16 @@ tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ c
   const int wpos_min = pos_first + 32 * w, wpos_max = min(kend, wpos_min + 31);
   const int wlo_min = chunk > 0 ? (wpos_min / chunk) * chunk : 0;
 
-  // the block ids of the keys this tile can see, so that a key's address never waits for a
-  // table load (entries beyond kTbl, i.e. very long chunks, are read from global memory)
+  // the block ids of the keys this tile can see, so that a key's address never waits for a table load
+  // (a range of more than kTbl blocks, i.e. a very long chunk, is read from the table)
   const int b_first = kbeg / bs, b_count = kend / bs - b_first + 1;
-  for (int i = tid; i < min(b_count, kTbl); i += 64 * NW) s_tbl[i] = tbl[b_first + i];
+  const bool in_lds = b_count <= kTbl;
+  if (in_lds)
+    for (int i = tid; i < b_count; i += 64 * NW) s_tbl[i] = tbl[b_first + i];
   const int bshift = (bs & (bs - 1)) == 0 ? __ffs(bs) - 1 : -1;
   __syncthreads();
 
-  float m = sink ? 0.f : -INFINITY, l = sink ? 1.f : 0.f;
+  float m = sink ? 0.f : -INFINITY, l = sink && hi == 0 ? 1.f : 0.f;   // (l: the lane's half)
   f32x16 O[D / 32];
 #pragma unroll
   for (int db = 0; db < D / 32; ++db)
@@ -291,35 +299,51 @@ tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ c
   // image takes them as they are, the transposed image takes eight 8-byte stores of 4 keys each
   // (transposed in registers).  The next tile's loads are issued before this tile's products, so
   // their latency hides behind the matrix work.
-  constexpr int NT = 64 * NW, ITEMS = (D + NT - 1) / NT;
+  constexpr int NT = 64 * NW, NTOT = D * SB, ITEMS = (NTOT + NT - 1) / NT;
   uint4 pre[ITEMS][4];
-  auto prefetch = [&](int k0) {
+  auto prefetch = [&](int k0) __attribute__((always_inline)) {
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
       const int item = tid + it * NT;
-      if (item < D) {
-        const int kq = item / NV, part = item % NV;
+      if (NTOT % NT == 0 || item < NTOT) {
+        const int kq = item / NV, part = item % NV, j = k0 + 4 * kq;
+        // the four cache rows first and without a branch per key (past the last key: that one again;
+        // `commit` blanks it): then the four loads leave together
+        int jb[4], blk[4];
+        if (bshift >= 0) {
+#pragma unroll
+          for (int x = 0; x < 4; ++x) jb[x] = min(j + x, kend) >> bshift;
+        } else {
+#pragma unroll
+          for (int x = 0; x < 4; ++x) jb[x] = min(j + x, kend) / bs;
+        }
+        if (in_lds) {
+#pragma unroll
+          for (int x = 0; x < 4; ++x) blk[x] = s_tbl[jb[x] - b_first];
+        } else {
+#pragma unroll
+          for (int x = 0; x < 4; ++x) blk[x] = tbl[jb[x]];
+        }
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
-          const int j = k0 + 4 * kq + x;
-          pre[it][x] = make_uint4(0, 0, 0, 0);
-          if (j <= kend) {
-            const int jb = bshift >= 0 ? j >> bshift : j / bs, jo = j - jb * bs;
-            const int bi = jb - b_first;
-            const int blk = bi < kTbl ? s_tbl[bi] : tbl[jb];
-            const long long off = (((long long)blk * bs + jo) * G + g) * D;
-            pre[it][x] = *reinterpret_cast<const uint4*>(cache + off + 8 * part);
-          }
+          const long long row = (long long)blk[x] * bs + (min(j + x, kend) - jb[x] * bs);
+          pre[it][x] = *reinterpret_cast<const uint4*>(cache + (row * G + g) * D + 8 * part);
         }
       }
     }
   };
-  auto commit = [&]() {
+  auto commit = [&](int k0, T* s_k, T* s_t, float* s_kn) __attribute__((always_inline)) {
+    const bool tail = k0 + KT - 1 > kend;            // keys past the last one: zeros
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
       const int item = tid + it * NT;
-      if (item < D) {
+      if (NTOT % NT == 0 || item < NTOT) {
         const int kq = item / NV, part = item % NV;
+        if (tail) {
+#pragma unroll
+          for (int x = 0; x < 4; ++x)
+            if (k0 + 4 * kq + x > kend) pre[it][x] = make_uint4(0, 0, 0, 0);
+        }
 #pragma unroll
         for (int x = 0; x < 4; ++x)
           *reinterpret_cast<uint4*>(&s_k[(4 * kq + x) * LK + 8 * part]) = pre[it][x];
@@ -350,72 +374,87 @@ tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ c
     }
   };
 
-  prefetch(kbeg);
-  for (int k0 = kbeg; k0 <= kend; k0 += 32) {
-    __syncthreads();                       // the previous tile has been consumed
-    commit();
-    __syncthreads();
-    if (k0 + 32 <= kend) prefetch(k0 + 32);
-    if (!wave_on || k0 > wpos_max || k0 + 31 < wlo_min) continue;   // nothing this wave may see
+  const int t0 = c * LT + 4 * (hi ^ (c >> 3)), t1 = c * LT + 4 * ((2 + hi) ^ (c >> 3));
+  // the wave's share of tile k0
+  auto tile = [&](int k0, const T* s_k, const T* s_t, const float* s_kn) __attribute__((always_inline)) {
+    if (!wave_on || k0 > wpos_max || k0 + KT - 1 < wlo_min) return;   // nothing this wave may see
 
-    f32x16 acc;
+    f32x16 sc[SB];
+    float k2[SB], kn[SB];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    float k2 = 0.f;
+    for (int b = 0; b < SB; ++b) {
 #pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk) {
-      const uint4 a = *reinterpret_cast<const uint4*>(&s_k[c * LK + 16 * kk + 8 * hi]);
-      if (!kStagedNorm) k2 += sumsq8<T>(a);
-      acc = Mma32<T>::run(a, qreg[kk], acc);
+      for (int r = 0; r < 16; ++r) sc[b][r] = 0.f;
+      k2[b] = kn[b] = 0.f;
     }
-    float kn = 0.f;                                      // of key k0 + c (other head sizes)
-    if (!kStagedNorm) {
-      k2 += __shfl_xor(k2, 32, 64);
-      kn = 1.f / sqrtf(k2 / D + eps);
-    }
-    // a tile every query of the wave sees whole needs no mask
-    const bool whole = k0 >= (chunk > 0 ? (wpos_max / chunk) * chunk : 0) && k0 + 31 <= wpos_min &&
-                       32 * w + 31 < nrows;
-    float sc[16];
-    float mloc = -INFINITY;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int keyr = 8 * (r >> 2) + 4 * hi + (r & 3);
-      const float knr = kStagedNorm ? s_kn[keyr] : __shfl(kn, keyr, 64);
-      sc[r] = acc[r] * qn * knr;
-    }
-    if (!whole) {
+    for (int kk = 0; kk < D / 16; ++kk)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int j = k0 + 8 * (r >> 2) + 4 * hi + (r & 3);
-        sc[r] = (j >= lo && j <= pos) ? sc[r] : -INFINITY;
+      for (int b = 0; b < SB; ++b) {
+        const uint4 a = *reinterpret_cast<const uint4*>(&s_k[(32 * b + c) * LK + 16 * kk + 8 * hi]);
+        if (!kStagedNorm) k2[b] += sumsq8<T>(a);
+        sc[b] = Mma32<T>::run(a, qreg[kk], sc[b]);
+      }
+    if (!kStagedNorm) {                                  // of key k0 + 32 b + c (other head sizes)
+#pragma unroll
+      for (int b = 0; b < SB; ++b) {
+        k2[b] += __shfl_xor(k2[b], 32, 64);
+        kn[b] = 1.f / sqrtf(k2[b] / D + eps);
       }
     }
+    // register r of sc[b] is key k0 + key_of(b, r)
+    const auto key_of = [&](int b, int r) { return 32 * b + 8 * (r >> 2) + 4 * hi + (r & 3); };
+    // a tile every query of the wave sees whole needs no mask
+    const bool whole = k0 >= (chunk > 0 ? (wpos_max / chunk) * chunk : 0) && k0 + KT - 1 <= wpos_min &&
+                       32 * w + 31 < nrows;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, sc[r]);
+    for (int b = 0; b < SB; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float knr = kStagedNorm ? s_kn[key_of(b, r)] : __shfl(kn[b], key_of(0, r), 64);
+        sc[b][r] *= qn * knr;
+      }
+    if (!whole) {
+#pragma unroll
+      for (int b = 0; b < SB; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int j = k0 + key_of(b, r);
+          sc[b][r] = (j >= lo && j <= pos) ? sc[b][r] : -INFINITY;
+        }
+    }
+    float mloc = -INFINITY;
+#pragma unroll
+    for (int b = 0; b < SB; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, sc[b][r]);
     mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
-    const float mn = fmaxf(m, mloc);
-    const float ms = mn == -INFINITY ? 0.f : mn;
-    // (v_exp_f32: this kernel serves 16-bit dtypes only, the weights are rounded to ~16 bits)
-    const float corr = __expf(m - ms);
-    float psum = 0.f;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) { sc[r] = __expf(sc[r] - ms); psum += sc[r]; }
-    psum += __shfl_xor(psum, 32, 64);
-    l = l * corr + psum;
-    m = mn;
-    if (__any(corr != 1.f)) {              // the running max moved for some query of the wave
+    // the reference of the weights follows the running maximum only when that passes it by kRise: weights
+    // stay under e^kRise, and the accumulators are rescaled on a few tiles of a row, not on most
+    if (__any(mloc > m + kRise)) {
+      const float mn = mloc > m + kRise ? mloc : m;
+      const float corr = mn == m ? 1.f : __expf(m - mn);
+      l *= corr;
+      m = mn;
 #pragma unroll
       for (int db = 0; db < D / 32; ++db)
 #pragma unroll
         for (int r = 0; r < 16; ++r) O[db][r] *= corr;
     }
+    const float ms = m == -INFINITY ? 0.f : m;
+    // (v_exp_f32: this kernel serves 16-bit dtypes only, the weights are rounded to ~16 bits)
+    float psum = 0.f;
 #pragma unroll
-    for (int s2 = 0; s2 < 2; ++s2) {
+    for (int b = 0; b < SB; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) { sc[b][r] = __expf(sc[b][r] - ms); psum += sc[b][r]; }
+    l += psum;                                 // (the lane's half: the other lane's is added at the end)
+#pragma unroll
+    for (int s2 = 0; s2 < 2 * SB; ++s2) {
       unsigned ph[4], pl[4];
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
-        const float a0 = sc[8 * s2 + 2 * x], a1 = sc[8 * s2 + 2 * x + 1];
+        const float a0 = sc[s2 / 2][8 * (s2 & 1) + 2 * x], a1 = sc[s2 / 2][8 * (s2 & 1) + 2 * x + 1];
         ph[x] = pk2<T>(a0, a1);                      // one packed conversion
         float h0, h1;
         unpack2<T>(ph[x], h0, h1);
@@ -425,16 +464,30 @@ tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ c
       const uint4 bl = make_uint4(pl[0], pl[1], pl[2], pl[3]);
 #pragma unroll
       for (int db = 0; db < D / 32; ++db) {
-        const int row = 32 * db + c, sw = (row >> 3) & 7;     // undo the store's permutation
-        const T* tp = &s_t[row * LT];
-        const uint2 a0 = *reinterpret_cast<const uint2*>(tp + 4 * ((4 * s2 + hi) ^ sw));
-        const uint2 a1 = *reinterpret_cast<const uint2*>(tp + 4 * ((4 * s2 + 2 + hi) ^ sw));
+        // quads 4 s2 + hi and 4 s2 + 2 + hi of row 32 db + c, under the store's permutation: both low
+        // bits lie in t0 / t1, the others in the instruction's offset
+        const int at = 32 * db * LT + 32 * (s2 >> 1) + 16 * ((s2 & 1) ^ (db & 1));
+        const uint2 a0 = *reinterpret_cast<const uint2*>(s_t + t0 + at);
+        const uint2 a1 = *reinterpret_cast<const uint2*>(s_t + t1 + at);
         const uint4 a = make_uint4(a0.x, a0.y, a1.x, a1.y);
         O[db] = Mma32<T>::run(a, bh, O[db]);
         O[db] = Mma32<T>::run(a, bl, O[db]);
       }
     }
+  };
+
+  prefetch(kbeg);
+  commit(kbeg, s_kb[0], s_tb[0], s_nb[0]);
+  __builtin_amdgcn_s_waitcnt(0xF70);       // vmcnt(0): or the loop's first product would wait, every time, for
+  __syncthreads();                         // the queries, and with them for the tile just asked for
+  for (int k0 = kbeg, cur = 0; k0 <= kend; k0 += KT, cur ^= 1) {
+    const bool more = k0 + KT <= kend;
+    if (more) prefetch(k0 + KT);
+    tile(k0, s_kb[cur], s_tb[cur], s_nb[cur]);
+    if (more) commit(k0 + KT, s_kb[cur ^ 1], s_tb[cur ^ 1], s_nb[cur ^ 1]);
+    __syncthreads();
   }
+  l += __shfl_xor(l, 32, 64);
   if (qv) {
     const float inv = 1.f / l;
     T* op = out + ((long long)qrow * H + hd) * D;
@@ -455,16 +508,19 @@ hipError_t launch_tiles(const void* q, long long ldq, const void* cache, void* o
                         const int* tables, int maxb, const int* tiles, int ntiles, const int* cu,
                         const int* start, int H, int G, int D, int bs, float scale, float eps,
                         int chunk, int sink, int tile_rows, hipStream_t st) {
-  const dim3 grid(ntiles, H);
+  const dim3 grid((unsigned)((long long)ntiles * H));
 #define GO(DD)                                                                                   \
-  if (tile_rows == 128)                                                                          \
-    tile_attn_kernel<T, DD, 4><<<grid, 256, 0, st>>>((const T*)q, ldq, (const T*)cache, (T*)out, \
-                                                     tables, maxb, tiles, cu, start, H, G, bs,   \
-                                                     scale, eps, chunk, sink);                   \
-  else                                                                                           \
-    tile_attn_kernel<T, DD, 2><<<grid, 128, 0, st>>>((const T*)q, ldq, (const T*)cache, (T*)out, \
-                                                     tables, maxb, tiles, cu, start, H, G, bs,   \
-                                                     scale, eps, chunk, sink)
+  {                                                                                              \
+    constexpr int KT = DD <= 128 ? 64 : 32;                                                      \
+    if (tile_rows == 128)                                                                        \
+      tile_attn_kernel<T, DD, 4, KT><<<grid, 256, 0, st>>>((const T*)q, ldq, (const T*)cache, (T*)out, \
+                                                       tables, maxb, tiles, cu, start, H, G, bs, \
+                                                       scale, eps, chunk, sink);                 \
+    else                                                                                         \
+      tile_attn_kernel<T, DD, 2, KT><<<grid, 128, 0, st>>>((const T*)q, ldq, (const T*)cache, (T*)out, \
+                                                       tables, maxb, tiles, cu, start, H, G, bs, \
+                                                       scale, eps, chunk, sink);                 \
+  }
   switch (D) {
     case 32: GO(32); break;
     case 64: GO(64); break;

@@ -65,6 +65,17 @@ __device__ __forceinline__ float gated_f(float g, float u, float w, bool shared,
   return f.weigh_in ? y : y * w;
 }
 
+// Workgroup `b` of `n` = tiles x heads -> (tile, head).  Tiles are listed in row order, so the later ones of a
+// prompt see more keys: they go first.  Two workgroups share a CU, b and b + 256 as they are handed out:
+// every second round of 256 runs backwards, or equal prompts would put two of their last tiles on one CU
+// and two first ones on another (16 heads x 8 prompts of 512: 16 key steps against 4).
+__device__ __forceinline__ void heavy_first(unsigned b, unsigned n, int heads, int& tile, int& head) {
+  const unsigned r = b >> 8;
+  if (r & 1) b = (r << 8) + min(256u, n - (r << 8)) - 1 - (b & 255);
+  tile = (int)(n / heads) - 1 - (int)(b / heads);
+  head = (int)(b % heads);
+}
+
 }  // namespace lumen
 
 // run `CALL(T)` with T = float / fp16 / bf16 for dtype code `dt`

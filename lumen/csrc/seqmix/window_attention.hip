@@ -12,13 +12,21 @@
 // may share one value head (several score maps over the same values).
 //
 // A workgroup of NW waves takes 32 * NW consecutive rows of ONE segment and one query head.  The
-// keys the tile can see are visited 32 at a time: first the tiles of the kept keys that lie below
-// the window of the tile's first row, then the tiles from that window's start to the last row's
-// position; what lies between is never loaded, so a long prompt's portion costs rows x (window +
+// keys the tile can see are visited KT = 64 at a time (32 for values over 128 wide): first the tiles of the
+// kept keys that lie below the window of the tile's first row, then the tiles from that window's start to the
+// last row's position; what lies between is never loaded, so a long prompt's portion costs rows x (window +
 // keep) and not rows x position.  A key tile is staged in LDS from the key cache (row-major, the
-// score operand) and from the value cache (transposed, the value operand) and shared by the
-// waves; the next tile's loads are issued before this tile's products.  Per wave (32 queries)
-// and key tile, with v_mfma_f32_32x32x16:
+// score operand) and from the value cache (transposed, the value operand) and shared by the waves.
+//
+// What bounds it: the chain of one tile after the other at one or two waves per SIMD, ~9000 cycles per 64 keys
+// where the products take 1500.  So the loads of a tile leave together one tile ahead (block ids from LDS, no
+// branch between two loads: a table lookup that could also go to memory made each wait for the one
+// before), two LDS buffers leave one barrier per tile, 64 keys share its exchanges, and the accumulators follow
+// the maximum only when it rises by kRise.  Measured (us, tiles of 32 keys, one buffer -> now; bf16, heads of
+// 128, soft cap): 1 x 512 rows x 32 heads 55 -> 33, 8 x 512 x 16 91 -> 43, 14 of 63 - 509 x 16 110 -> 58, 1 x 4096 x 32
+// (window 1024) 380 -> 168; heads of 64 44 -> 23, of 256 191 -> 113, values of 256 169 -> 101.
+//
+// Per wave (32 queries) and 32 keys, with v_mfma_f32_32x32x16:
 //   S^T = K Q^T      keys on the accumulator rows, queries on the columns (lane & 31): a lane
 //                    owns ONE query, so its running max / sum / correction are plain scalars;
 //   O^T += V^T P^T   the accumulator registers 8s .. 8s+7 of S^T are keys {16s + 4hi + 0..3,
@@ -65,8 +73,12 @@ template <> __device__ __forceinline__ void unpack2<fp16>(unsigned v, float& a, 
   b = static_cast<float>(h[1]);
 }
 
+constexpr float kRise = 5.f;      // log of the largest weight a tile may form before its maximum moves the reference
+
 // tanh through one exponential: 1 - 2 / (1 + e^(2x)); exact limits at both ends
-__device__ __forceinline__ float tanh_exp(float x) { return 1.f - 2.f / (1.f + __expf(2.f * x)); }
+__device__ __forceinline__ float tanh_exp(float x) {
+  return 1.f - 2.f * __builtin_amdgcn_rcpf(1.f + __expf(2.f * x));
+}
 
 template <typename T>
 struct WinTileArgs {
@@ -83,21 +95,22 @@ struct WinTileArgs {
   const float* sigb; int vdiv;               // sigmoid weights' bias [H] (nullable); key heads per value head
 };
 
-template <typename T, int D, int DV, int NW>
+template <typename T, int D, int DV, int NW, int KT>
 __global__ void __launch_bounds__(64 * NW)
     __attribute__((amdgpu_waves_per_eu((D <= 128 && DV <= 128) ? 2 : 1)))
 win_tile_attn_kernel(const WinTileArgs<T> a) {
-  constexpr int QT = 32 * NW, LK = D + 8, LT = 40, NV = D / 8, NVV = DV / 8;
-  __shared__ __align__(16) T s_k[32 * LK];    // key tile, row-major
-  __shared__ __align__(16) T s_t[DV * LT];    // value tile, transposed [d][key]
+  constexpr int QT = 32 * NW, LK = D + 8, LT = KT + 8, NV = D / 8, NVV = DV / 8, SB = KT / 32;
+  // two buffers: a tile is stored while the one before it is read, one barrier per tile
+  __shared__ __align__(16) T s_kb[2][KT * LK];    // key tile, row-major
+  __shared__ __align__(16) T s_tb[2][DV * LT];    // value tile, transposed [d][key]
   constexpr int kTbl = 512;                   // block-table entries of the window's keys, in LDS
   __shared__ int s_tbl[kTbl];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 31, hi = lane >> 5;
-  const int hd = blockIdx.y, g = hd / (a.H / a.G);
+  int tix, hd;
+  heavy_first(blockIdx.x, gridDim.x, a.H, tix, hd);
+  const int g = hd / (a.H / a.G);
   const int Gv = a.G / a.vdiv, gv = g / a.vdiv;
   const float sbias = a.sigb != nullptr ? a.sigb[hd] : 0.f;
-  // tiles are listed in row order, so later tiles see more keys: issue them first
-  const int tix = gridDim.x - 1 - blockIdx.x;
   const int sg = a.tiles[2 * tix], row0 = a.tiles[2 * tix + 1];
   const int seg_r0 = a.cu[sg], p0 = a.start[sg];
   const int nrows = min(QT, a.cu[sg + 1] - row0);
@@ -115,23 +128,26 @@ win_tile_attn_kernel(const WinTileArgs<T> a) {
   const float slope = a.slopes != nullptr ? a.slopes[hd] : 0.f;
   const float cap = a.softcap, rcap = cap > 0.f ? 1.f / cap : 0.f;
 
-  // key tiles: [0, khead) in steps of 32 (kept keys below the window), then from kwin on
+  // key tiles: [0, khead) in steps of KT (kept keys below the window), then from kwin on
   const int pos_first = p0 + (row0 - seg_r0), kend = pos_first + nrows - 1;
   const int wlo = window > 0 ? max(0, pos_first - window + 1) : 0;
   const int kwin = wlo / 32 * 32;
-  const int khead = min((min(keep, wlo) + 31) / 32 * 32, kwin);
+  const int khead = min((min(keep, wlo) + KT - 1) / KT * KT, kwin);
   const int kfirst = khead > 0 ? 0 : kwin;
   auto next_tile = [&](int k0) {
-    const int n = k0 + 32;
+    const int n = k0 + KT;
     return (n >= khead && n < kwin) ? kwin : n;
   };
   const bool wave_on = 32 * w < nrows;
   const int wpos_min = pos_first + 32 * w, wpos_max = min(kend, wpos_min + 31);
 
-  // block ids of the window's keys, so that a key's address never waits for a table load (the
-  // few kept keys' entries, and entries beyond kTbl, are read from global memory)
-  const int b_first = kwin / bs, b_count = kend / bs - b_first + 1;
-  for (int i = tid; i < min(b_count, kTbl); i += 64 * NW) s_tbl[i] = tbl[b_first + i];
+  // block ids of the keys the tile visits (the kept keys' blocks, then the window's), so that a key's
+  // address never waits for a table load; a range of more than kTbl blocks is read from the table
+  const int b_first = kwin / bs, b_head = khead > 0 ? min((khead + bs - 1) / bs, b_first) : 0;
+  const int b_count = b_head + kend / bs - b_first + 1;
+  const bool in_lds = b_count <= kTbl;
+  if (in_lds)
+    for (int i = tid; i < b_count; i += 64 * NW) s_tbl[i] = tbl[i < b_head ? i : i - b_head + b_first];
   const int bshift = (bs & (bs - 1)) == 0 ? __ffs(bs) - 1 : -1;
   __syncthreads();
 
@@ -142,67 +158,73 @@ win_tile_attn_kernel(const WinTileArgs<T> a) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) O[db][r] = 0.f;
 
-  // staging: one item = 4 consecutive keys x 8 channels of the key cache AND of the value cache
-  // (four 16-byte loads each); the row-major image takes the keys as they are, the transposed
-  // image takes eight 8-byte stores of 4 values each (transposed in registers)
-  constexpr int NT = 64 * NW, ITEMS = (D + NT - 1) / NT, ITEMS_V = (DV + NT - 1) / NT;
-  uint4 pk[ITEMS][4], pv[ITEMS_V][4];
-  auto cache_row = [&](int j) -> long long {
-    const int jb = bshift >= 0 ? j >> bshift : j / bs, jo = j - jb * bs;
-    const int bi = jb - b_first;
-    const int blk = (bi >= 0 && bi < kTbl) ? s_tbl[bi] : tbl[jb];
-    return (long long)blk * bs + jo;
+  // staging: one item = 4 consecutive keys x 8 channels of the key cache or of the value cache (four
+  // 16-byte loads); the row-major image takes the keys as they are, the transposed image takes eight
+  // 8-byte stores of 4 values each (transposed in registers)
+  constexpr int NT = 64 * NW, NK = D * SB, NTOT = (D + DV) * SB, ITEMS = (NTOT + NT - 1) / NT;
+  uint4 pre[ITEMS][4];
+  // cache rows of the four keys from j on (past the last key: that one again; `commit` blanks it).  The
+  // rows come first and without a branch per key: then an item's four loads leave together
+  auto cache_rows = [&](int j, long long (&row)[4]) __attribute__((always_inline)) {
+    int jb[4], jo[4], blk[4];
+    if (bshift >= 0) {
+#pragma unroll
+      for (int x = 0; x < 4; ++x) jb[x] = min(j + x, kend) >> bshift;
+    } else {
+#pragma unroll
+      for (int x = 0; x < 4; ++x) jb[x] = min(j + x, kend) / bs;
+    }
+#pragma unroll
+    for (int x = 0; x < 4; ++x) jo[x] = min(j + x, kend) - jb[x] * bs;
+    if (in_lds) {
+#pragma unroll
+      for (int x = 0; x < 4; ++x) blk[x] = s_tbl[jb[x] >= b_first ? jb[x] - b_first + b_head : jb[x]];
+    } else {
+#pragma unroll
+      for (int x = 0; x < 4; ++x) blk[x] = tbl[jb[x]];
+    }
+#pragma unroll
+    for (int x = 0; x < 4; ++x) row[x] = (long long)blk[x] * bs + jo[x];
   };
-  auto prefetch = [&](int k0) {
+  auto prefetch = [&](int k0) __attribute__((always_inline)) {
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
       const int item = tid + it * NT;
-      if (item < D) {
-        const int kq = item / NV, part = item % NV;
+      const bool val = item >= NK;
+      const int i = val ? item - NK : item;
+      if (NTOT % NT != 0 && item >= NTOT) continue;
+      const int kq = val ? i / NVV : i / NV, part = val ? i % NVV : i % NV;
+      long long row[4];
+      cache_rows(k0 + 4 * kq, row);
+      const T* base = val ? a.vc + (long long)gv * DV + 8 * part : a.kc + (long long)g * D + 8 * part;
+      const long long ld = val ? (long long)Gv * DV : (long long)a.G * D;
 #pragma unroll
-        for (int x = 0; x < 4; ++x) {
-          const int j = k0 + 4 * kq + x;
-          pk[it][x] = make_uint4(0, 0, 0, 0);
-          if (j <= kend)
-            pk[it][x] = *reinterpret_cast<const uint4*>(a.kc + (cache_row(j) * a.G + g) * D + 8 * part);
-        }
-      }
-    }
-#pragma unroll
-    for (int it = 0; it < ITEMS_V; ++it) {
-      const int item = tid + it * NT;
-      if (item < DV) {
-        const int kq = item / NVV, part = item % NVV;
-#pragma unroll
-        for (int x = 0; x < 4; ++x) {
-          const int j = k0 + 4 * kq + x;
-          pv[it][x] = make_uint4(0, 0, 0, 0);
-          if (j <= kend)
-            pv[it][x] = *reinterpret_cast<const uint4*>(a.vc + (cache_row(j) * Gv + gv) * DV + 8 * part);
-        }
-      }
+      for (int x = 0; x < 4; ++x) pre[it][x] = *reinterpret_cast<const uint4*>(base + row[x] * ld);
     }
   };
-  auto commit = [&]() {
+  auto commit = [&](int k0, T* s_k, T* s_t) __attribute__((always_inline)) {
+    const bool tail = k0 + KT - 1 > kend;            // keys past the last one: zeros
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
       const int item = tid + it * NT;
-      if (item < D) {
-        const int kq = item / NV, part = item % NV;
+      const bool val = item >= NK;
+      const int i = val ? item - NK : item;
+      if (NTOT % NT != 0 && item >= NTOT) continue;
+      const int kq = val ? i / NVV : i / NV, part = val ? i % NVV : i % NV;
+      if (tail) {
 #pragma unroll
         for (int x = 0; x < 4; ++x)
-          *reinterpret_cast<uint4*>(&s_k[(4 * kq + x) * LK + 8 * part]) = pk[it][x];
+          if (k0 + 4 * kq + x > kend) pre[it][x] = make_uint4(0, 0, 0, 0);
       }
-    }
+      if (!val) {
 #pragma unroll
-    for (int it = 0; it < ITEMS_V; ++it) {
-      const int item = tid + it * NT;
-      if (item < DV) {
-        const int kq = item / NVV, part = item % NVV;
-        const unsigned w0[4] = {pv[it][0].x, pv[it][0].y, pv[it][0].z, pv[it][0].w};
-        const unsigned w1[4] = {pv[it][1].x, pv[it][1].y, pv[it][1].z, pv[it][1].w};
-        const unsigned w2[4] = {pv[it][2].x, pv[it][2].y, pv[it][2].z, pv[it][2].w};
-        const unsigned w3[4] = {pv[it][3].x, pv[it][3].y, pv[it][3].z, pv[it][3].w};
+        for (int x = 0; x < 4; ++x)
+          *reinterpret_cast<uint4*>(&s_k[(4 * kq + x) * LK + 8 * part]) = pre[it][x];
+      } else {
+        const unsigned w0[4] = {pre[it][0].x, pre[it][0].y, pre[it][0].z, pre[it][0].w};
+        const unsigned w1[4] = {pre[it][1].x, pre[it][1].y, pre[it][1].z, pre[it][1].w};
+        const unsigned w2[4] = {pre[it][2].x, pre[it][2].y, pre[it][2].z, pre[it][2].w};
+        const unsigned w3[4] = {pre[it][3].x, pre[it][3].y, pre[it][3].z, pre[it][3].w};
 #pragma unroll
         for (int mm = 0; mm < 4; ++mm) {     // word mm holds channels 2mm (low half), 2mm + 1
           // the key quads of a row are permuted by the row's group of 8 (all rows a lane
@@ -217,76 +239,95 @@ win_tile_attn_kernel(const WinTileArgs<T> a) {
     }
   };
 
-  prefetch(kfirst);
-  for (int k0 = kfirst; k0 <= kend; k0 = next_tile(k0)) {
-    __syncthreads();                       // the previous tile has been consumed
-    commit();
-    __syncthreads();
-    const int kn = next_tile(k0);
-    if (kn <= kend) prefetch(kn);
+  const int t0 = c * LT + 4 * (hi ^ (c >> 3)), t1 = c * LT + 4 * ((2 + hi) ^ (c >> 3));
+  // the wave's share of tile k0
+  auto tile = [&](int k0, const T* s_k, const T* s_t) __attribute__((always_inline)) {
     // nothing this wave may see: past its last row, or before its first row's window and not kept
-    if (!wave_on || k0 > wpos_max || (window > 0 && k0 + 31 < wpos_min - window + 1 && k0 >= keep))
-      continue;
+    if (!wave_on || k0 > wpos_max ||
+        (window > 0 && k0 + KT - 1 < wpos_min - window + 1 && k0 >= keep))
+      return;
 
-    f32x16 acc;
+    f32x16 sc[SB];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    for (int b = 0; b < SB; ++b)
 #pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk) {
-      const uint4 av = *reinterpret_cast<const uint4*>(&s_k[c * LK + 16 * kk + 8 * hi]);
-      acc = Mma32<T>::run(av, qreg[kk], acc);
-    }
+      for (int r = 0; r < 16; ++r) sc[b][r] = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < D / 16; ++kk)
+#pragma unroll
+      for (int b = 0; b < SB; ++b)
+        sc[b] = Mma32<T>::run(*reinterpret_cast<const uint4*>(&s_k[(32 * b + c) * LK + 16 * kk + 8 * hi]),
+                              qreg[kk], sc[b]);
+    // register r of sc[b] is key k0 + key_of(b, r)
+    const auto key_of = [&](int b, int r) { return 32 * b + 8 * (r >> 2) + 4 * hi + (r & 3); };
     // a tile every query of the wave sees whole needs no mask
-    const bool whole = k0 + 31 <= wpos_min && 32 * w + 31 < nrows &&
-                       (window <= 0 || k0 >= wpos_max - window + 1 || k0 + 31 < keep);
-    float sc[16];
-    float mloc = -INFINITY;
+    const bool whole = k0 + KT - 1 <= wpos_min && 32 * w + 31 < nrows &&
+                       (window <= 0 || k0 >= wpos_max - window + 1 || k0 + KT - 1 < keep);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int j = k0 + 8 * (r >> 2) + 4 * hi + (r & 3);
-      float sv = acc[r] * a.scale;
-      if (cap > 0.f) sv = cap * tanh_exp(sv * rcap);
-      sc[r] = sv - slope * (float)(pos - j);
+    for (int b = 0; b < SB; ++b) sc[b] *= a.scale;
+    if (cap > 0.f) {
+#pragma unroll
+      for (int b = 0; b < SB; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sc[b][r] = cap * tanh_exp(sc[b][r] * rcap);
+    }
+    if (a.slopes != nullptr) {
+      const float d0 = (float)(pos - k0);
+#pragma unroll
+      for (int b = 0; b < SB; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sc[b][r] -= slope * (d0 - (float)key_of(b, r));
     }
     if (!whole) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int j = k0 + 8 * (r >> 2) + 4 * hi + (r & 3);
-        const bool seen = j <= pos && (window <= 0 || pos - j < window || j < keep);
-        sc[r] = seen ? sc[r] : -INFINITY;
-      }
+      for (int b = 0; b < SB; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int j = k0 + key_of(b, r);
+          const bool seen = j <= pos && (window <= 0 || pos - j < window || j < keep);
+          sc[b][r] = seen ? sc[b][r] : -INFINITY;
+        }
     }
     if (a.sigb != nullptr) {
       // weights as they are: a hidden key's -inf gives 1 / (1 + e^inf) = 0
 #pragma unroll
-      for (int r = 0; r < 16; ++r) sc[r] = 1.f / (1.f + __expf(-(sc[r] + sbias)));
+      for (int b = 0; b < SB; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sc[b][r] = 1.f / (1.f + __expf(-(sc[b][r] + sbias)));
     } else {
+      float mloc = -INFINITY;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, sc[r]);
+      for (int b = 0; b < SB; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, sc[b][r]);
       mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
-      const float mn = fmaxf(m, mloc);
-      const float ms = mn == -INFINITY ? 0.f : mn;
-      // (v_exp_f32: this kernel serves 16-bit dtypes only, the weights are rounded to ~16 bits)
-      const float corr = __expf(m - ms);
-      float psum = 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) { sc[r] = __expf(sc[r] - ms); psum += sc[r]; }
-      psum += __shfl_xor(psum, 32, 64);
-      l = l * corr + psum;
-      m = mn;
-      if (__any(corr != 1.f)) {            // the running max moved for some query of the wave
+      // the reference of the weights follows the running maximum only when that passes it by kRise: weights
+      // stay under e^kRise, and the accumulators are rescaled on a few tiles of a row, not on most
+      if (__any(mloc > m + kRise)) {
+        const float mn = mloc > m + kRise ? mloc : m;
+        const float corr = mn == m ? 1.f : __expf(m - mn);
+        l *= corr;
+        m = mn;
 #pragma unroll
         for (int db = 0; db < DV / 32; ++db)
 #pragma unroll
           for (int r = 0; r < 16; ++r) O[db][r] *= corr;
       }
+      const float ms = m == -INFINITY ? 0.f : m;
+      // (v_exp_f32: this kernel serves 16-bit dtypes only, the weights are rounded to ~16 bits)
+      float psum = 0.f;
+#pragma unroll
+      for (int b = 0; b < SB; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) { sc[b][r] = __expf(sc[b][r] - ms); psum += sc[b][r]; }
+      l += psum;                               // (the lane's half: the other lane's is added at the end)
     }
 #pragma unroll
-    for (int s2 = 0; s2 < 2; ++s2) {
+    for (int s2 = 0; s2 < 2 * SB; ++s2) {
       unsigned ph[4], pl[4];
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
-        const float a0 = sc[8 * s2 + 2 * x], a1 = sc[8 * s2 + 2 * x + 1];
+        const float a0 = sc[s2 / 2][8 * (s2 & 1) + 2 * x], a1 = sc[s2 / 2][8 * (s2 & 1) + 2 * x + 1];
         ph[x] = pk2<T>(a0, a1);                      // one packed conversion
         float h0, h1;
         unpack2<T>(ph[x], h0, h1);
@@ -296,16 +337,33 @@ win_tile_attn_kernel(const WinTileArgs<T> a) {
       const uint4 bl = make_uint4(pl[0], pl[1], pl[2], pl[3]);
 #pragma unroll
       for (int db = 0; db < DV / 32; ++db) {
-        const int row = 32 * db + c, sw = (row >> 3) & 7;     // undo the store's permutation
-        const T* tp = &s_t[row * LT];
-        const uint2 a0 = *reinterpret_cast<const uint2*>(tp + 4 * ((4 * s2 + hi) ^ sw));
-        const uint2 a1 = *reinterpret_cast<const uint2*>(tp + 4 * ((4 * s2 + 2 + hi) ^ sw));
+        // quads 4 s2 + hi and 4 s2 + 2 + hi of row 32 db + c, under the store's permutation: both low
+        // bits lie in t0 / t1, the others in the instruction's offset
+        const int at = 32 * db * LT + 32 * (s2 >> 1) + 16 * ((s2 & 1) ^ (db & 1));
+        const uint2 a0 = *reinterpret_cast<const uint2*>(s_t + t0 + at);
+        const uint2 a1 = *reinterpret_cast<const uint2*>(s_t + t1 + at);
         const uint4 av = make_uint4(a0.x, a0.y, a1.x, a1.y);
         O[db] = Mma32<T>::run(av, bh, O[db]);
         O[db] = Mma32<T>::run(av, bl, O[db]);
       }
     }
+  };
+
+  // tile n is stored after tile n - 1 was read: the loads of a tile have the products of the one before
+  // it to arrive in
+  prefetch(kfirst);
+  commit(kfirst, s_kb[0], s_tb[0]);
+  __builtin_amdgcn_s_waitcnt(0xF70);       // vmcnt(0): or the loop's first product would wait, every time, for
+  __syncthreads();                         // the queries, and with them for the tile just asked for
+  for (int k0 = kfirst, cur = 0; k0 <= kend; cur ^= 1) {
+    const int kn = next_tile(k0);
+    if (kn <= kend) prefetch(kn);
+    tile(k0, s_kb[cur], s_tb[cur]);
+    if (kn <= kend) commit(kn, s_kb[cur ^ 1], s_tb[cur ^ 1]);
+    __syncthreads();
+    k0 = kn;
   }
+  l += __shfl_xor(l, 32, 64);
   if (qv) {
     float inv = a.sigb != nullptr ? 1.f : 1.f / l;   // l > 0: a row always sees its own key
     if (a.gate != nullptr) inv *= sigmoid_f(to_f32(a.gate[(long long)qrow * a.gater + hd]));
@@ -325,10 +383,13 @@ win_tile_attn_kernel(const WinTileArgs<T> a) {
 template <typename T>
 hipError_t launch_win_tiles(const WinTileArgs<T>& a, int ntiles, int D, int Dv, int tile_rows,
                             hipStream_t st) {
-  const dim3 grid(ntiles, a.H);
+  const dim3 grid((unsigned)((long long)ntiles * a.H));
 #define GO(DD, DVV)                                                                          \
-  if (tile_rows == 128) win_tile_attn_kernel<T, DD, DVV, 4><<<grid, 256, 0, st>>>(a);        \
-  else win_tile_attn_kernel<T, DD, DVV, 2><<<grid, 128, 0, st>>>(a)
+  {                                                                                          \
+    constexpr int KT = DVV <= 128 ? 64 : 32;                                                 \
+    if (tile_rows == 128) win_tile_attn_kernel<T, DD, DVV, 4, KT><<<grid, 256, 0, st>>>(a);  \
+    else win_tile_attn_kernel<T, DD, DVV, 2, KT><<<grid, 128, 0, st>>>(a);                   \
+  }
   switch (D * 1024 + Dv) {
     case 32 * 1024 + 32: GO(32, 32); break;
     case 64 * 1024 + 64: GO(64, 64); break;

@@ -102,14 +102,17 @@ __global__ void __launch_bounds__(256)
 latent_write_kernel(const T* __restrict__ z, long long ldz, const float* __restrict__ wn,
                     const float* __restrict__ inv_freq, const int* __restrict__ positions,
                     const long long* __restrict__ slots, T* __restrict__ cache,
-                    T* __restrict__ vt, int bs, int Tn, int R, int Dr, int dims, float eps) {
+                    T* __restrict__ vt, T* __restrict__ own, int bs, int Tn, int R, int Dr, int dims,
+                    float eps) {
   const int lane = threadIdx.x & 63;
   const int t = blockIdx.x * kWaves + (threadIdx.x >> 6);
   if (t >= Tn) return;
   const long long s = slots[t];
-  if (s < 0) return;
+  if (s < 0 && own == nullptr) return;
   const T* zr = z + (long long)t * ldz;
-  T* dst = cache + s * (R + Dr);
+  T* dst = s >= 0 ? cache + s * (R + Dr) : nullptr;
+  // own (optional): the cache rows once more, row after row of the step
+  T* od = own ? own + (long long)t * (R + Dr) : nullptr;
   float ss = 0.f;
   for (int c = lane; c < R; c += 64) {
     const float v = to_f32(zr[c]);
@@ -119,10 +122,14 @@ latent_write_kernel(const T* __restrict__ z, long long ldz, const float* __restr
   const float inv = 1.f / sqrtf(ss / (float)R + eps);
   // vt (optional): the normed latent once more, transposed per cache block [block][R][bs], for
   // the matrix-core value product that contracts over the keys
-  T* dt = vt ? vt + (s / bs) * (long long)R * bs + s % bs : nullptr;
+  T* dt = vt && s >= 0 ? vt + (s / bs) * (long long)R * bs + s % bs : nullptr;
+  const auto put = [&](int c, T v) {
+    if (dst) dst[c] = v;
+    if (od) od[c] = v;
+  };
   for (int c = lane; c < R; c += 64) {
     const T v = from_f32<T>(to_f32(zr[c]) * inv * wn[c]);
-    dst[c] = v;
+    put(c, v);
     if (dt) dt[(long long)c * bs] = v;
   }
   const float pos = (float)positions[t];
@@ -130,10 +137,10 @@ latent_write_kernel(const T* __restrict__ z, long long ldz, const float* __restr
     float sn, cs;
     sincosf(pos * inv_freq[pr], &sn, &cs);
     const float u = to_f32(zr[R + 2 * pr]), v = to_f32(zr[R + 2 * pr + 1]);
-    dst[R + 2 * pr] = from_f32<T>(u * cs - v * sn);
-    dst[R + 2 * pr + 1] = from_f32<T>(v * cs + u * sn);
+    put(R + 2 * pr, from_f32<T>(u * cs - v * sn));
+    put(R + 2 * pr + 1, from_f32<T>(v * cs + u * sn));
   }
-  for (int c = dims + lane; c < Dr; c += 64) dst[R + c] = zr[R + c];
+  for (int c = dims + lane; c < Dr; c += 64) put(R + c, zr[R + c]);
 }
 
 template <typename T, bool VEC>
@@ -919,11 +926,11 @@ hipError_t sm_rotate_heads(int dt, void* x, long long ldr, long long ldh, int he
 
 hipError_t sm_latent_write(int dt, const void* z, long long ldz, const float* wn,
                            const float* inv_freq, const int* positions, const long long* slots,
-                           void* cache, void* vt, int bs, int T, int R, int Dr, int dims,
+                           void* cache, void* vt, void* own, int bs, int T, int R, int Dr, int dims,
                            float eps, hipStream_t st) {
   if (T == 0) return hipSuccess;
   if (dims % 2 || dims > Dr) return hipErrorInvalidValue;
-#define CALL(TT) latent_write_kernel<TT><<<(T + kWaves - 1) / kWaves, 256, 0, st>>>((const TT*)z, ldz, wn, inv_freq, positions, slots, (TT*)cache, (TT*)vt, bs, T, R, Dr, dims, eps)
+#define CALL(TT) latent_write_kernel<TT><<<(T + kWaves - 1) / kWaves, 256, 0, st>>>((const TT*)z, ldz, wn, inv_freq, positions, slots, (TT*)cache, (TT*)vt, (TT*)own, bs, T, R, Dr, dims, eps)
   SM_DISPATCH(dt, CALL)
 #undef CALL
   return hipGetLastError();

@@ -84,6 +84,9 @@ template <typename T>
 struct WinTileArgs {
   const T* q; long long ldq;                 // rows [T][>= H * D]
   const T* kc; const T* vc;                  // [blocks][bs][G][D], [blocks][bs][G / vdiv][DV]
+  // FRESH: the step's own rows, head after head (row strides ldk, ldv), and the kDr last columns of a key,
+  // which the heads share
+  const T* kr; long long ldk, ldv, ldr;
   T* out;                                    // [T][H][DV]
   const T* gate; long long gater;            // gate logits [T][H], row stride (nullable)
   const int* tables; int maxb;
@@ -95,9 +98,17 @@ struct WinTileArgs {
   const float* sigb; int vdiv;               // sigmoid weights' bias [H] (nullable); key heads per value head
 };
 
-template <typename T, int D, int DV, int NW, int KT>
+constexpr int kDr = 64;
+
+// FRESH: prompts whose every key is a row of this step (positions from 0): keys and values are read where the
+// projection left them and the block tables are not used.  A key is the head's own D - kDr columns, then kDr
+// columns that all heads share.  Latent attention of fresh prompts (keys and values expanded from the latents): 192
+// + 128 columns a score and value instead of 576 + 512, so ~0.3 of the products of latent_tile.hip.  us, projections
+// around it included, absorbed -> expanded (bf16): 14 prompts of 63 - 509 tokens x 16 heads 197 -> 81 (this kernel
+// 58), 8 x 512 224 -> 65, 1 x 512 72 -> 42, 1 x 30 60 -> 29, 1 x 2048 x 32 714 -> 141: at every size.
+template <typename T, int D, int DV, int NW, int KT, bool FRESH = false>
 __global__ void __launch_bounds__(64 * NW)
-    __attribute__((amdgpu_waves_per_eu((D <= 128 && DV <= 128) ? 2 : 1)))
+    __attribute__((amdgpu_waves_per_eu((D <= 128 || FRESH) && DV <= 128 ? 2 : 1)))
 win_tile_attn_kernel(const WinTileArgs<T> a) {
   constexpr int QT = 32 * NW, LK = D + 8, LT = KT + 8, NV = D / 8, NVV = DV / 8, SB = KT / 32;
   // two buffers: a tile is stored while the one before it is read, one barrier per tile
@@ -143,10 +154,10 @@ win_tile_attn_kernel(const WinTileArgs<T> a) {
 
   // block ids of the keys the tile visits (the kept keys' blocks, then the window's), so that a key's
   // address never waits for a table load; a range of more than kTbl blocks is read from the table
-  const int b_first = kwin / bs, b_head = khead > 0 ? min((khead + bs - 1) / bs, b_first) : 0;
-  const int b_count = b_head + kend / bs - b_first + 1;
+  const int b_first = FRESH ? 0 : kwin / bs, b_head = khead > 0 ? min((khead + bs - 1) / bs, b_first) : 0;
+  const int b_count = FRESH ? 0 : b_head + kend / bs - b_first + 1;
   const bool in_lds = b_count <= kTbl;
-  if (in_lds)
+  if (!FRESH && in_lds)
     for (int i = tid; i < b_count; i += 64 * NW) s_tbl[i] = tbl[i < b_head ? i : i - b_head + b_first];
   const int bshift = (bs & (bs - 1)) == 0 ? __ffs(bs) - 1 : -1;
   __syncthreads();
@@ -195,6 +206,16 @@ win_tile_attn_kernel(const WinTileArgs<T> a) {
       if (NTOT % NT != 0 && item >= NTOT) continue;
       const int kq = val ? i / NVV : i / NV, part = val ? i % NVV : i % NV;
       long long row[4];
+      if constexpr (FRESH) {
+        constexpr int P1 = (D - kDr) / 8;
+        const T* base = val ? a.vc + gv * DV + 8 * part
+                            : part < P1 ? a.kc + g * (D - kDr) + 8 * part : a.kr + 8 * (part - P1);
+        const long long ld = val ? a.ldv : part < P1 ? a.ldk : a.ldr;
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+          pre[it][x] = *reinterpret_cast<const uint4*>(base + (seg_r0 + min(k0 + 4 * kq + x, kend)) * ld);
+        continue;
+      }
       cache_rows(k0 + 4 * kq, row);
       const T* base = val ? a.vc + (long long)gv * DV + 8 * part : a.kc + (long long)g * D + 8 * part;
       const long long ld = val ? (long long)Gv * DV : (long long)a.G * D;
@@ -409,9 +430,46 @@ hipError_t launch_win_tiles(const WinTileArgs<T>& a, int ntiles, int D, int Dv, 
   return hipGetLastError();
 }
 
+template <typename T>
+hipError_t launch_fresh_tiles(const WinTileArgs<T>& a, int ntiles, int tile_rows, hipStream_t st) {
+  const dim3 grid((unsigned)((long long)ntiles * a.H));
+  if (tile_rows == 128) win_tile_attn_kernel<T, 192, 128, 4, 32, true><<<grid, 256, 0, st>>>(a);
+  else win_tile_attn_kernel<T, 192, 128, 2, 32, true><<<grid, 128, 0, st>>>(a);
+  return hipGetLastError();
+}
+
 }  // namespace
 
 extern "C" {
+
+// Prompts from position 0 whose keys and values are rows of the step: q rows [T][>= H * (D1 + Dr)], k rows
+// [T][>= H * D1] and v rows [T][>= H * Dv] head after head, kr rows [T][>= Dr] the key part all heads share;
+// D1 = Dv = 128, Dr = 64; row strides % 8, 16-byte aligned bases; out [T][H][Dv] contiguous; tiles, cu and start
+// as below (every start is 0).
+int sm_fresh_tiles_ok(int dt, int D1, int Dr, int Dv) {
+  return (dt == kBF16 || dt == kF16) && D1 == 128 && Dr == kDr && Dv == 128;
+}
+
+hipError_t sm_fresh_tiles(int dt, const void* q, long long ldq, const void* k, long long ldk, const void* kr,
+                          long long ldr, const void* v, long long ldv, void* out, const int* tiles, int ntiles,
+                          int tile_rows, const int* cu, const int* start, int H, int D1, int Dr, int Dv,
+                          float scale, hipStream_t st) {
+  if (ntiles == 0) return hipSuccess;
+  if (!sm_fresh_tiles_ok(dt, D1, Dr, Dv) || ntiles < 0 || H < 1 || (tile_rows != 64 && tile_rows != 128) ||
+      ldq % 8 || ldk % 8 || ldr % 8 || ldv % 8 || ldq < (long long)H * (D1 + Dr) || ldk < (long long)H * D1 ||
+      ldr < Dr || ldv < (long long)H * Dv ||
+      ((uintptr_t)q | (uintptr_t)k | (uintptr_t)kr | (uintptr_t)v) % 16 || (uintptr_t)out % 8)
+    return hipErrorInvalidValue;
+#define CALL(TT)                                                                                          \
+  {                                                                                                       \
+    WinTileArgs<TT> a{(const TT*)q, ldq, (const TT*)k, (const TT*)v, (const TT*)kr, ldk, ldv, ldr, (TT*)out, \
+                      nullptr, 0, nullptr, 0, tiles, cu, start, H, H, 1, scale, 0.f, nullptr, 0, 0, nullptr, 1}; \
+    return launch_fresh_tiles<TT>(a, ntiles, tile_rows, st);                                              \
+  }
+  if (dt == kBF16) CALL(bf16)
+  CALL(fp16)
+#undef CALL
+}
 
 // 1 when sm_win_attn_tiles has a kernel for this dtype / key size / value size
 int sm_win_attn_tiles_ok(int dt, int D, int Dv) {
@@ -439,7 +497,7 @@ hipError_t sm_win_attn_tiles(int dt, const void* q, long long ldq, const void* k
   if (tile_rows != 64 && tile_rows != 128) return hipErrorInvalidValue;
 #define CALL(TT)                                                                               \
   {                                                                                            \
-    WinTileArgs<TT> a{(const TT*)q, ldq, (const TT*)kc, (const TT*)vc, (TT*)out,               \
+    WinTileArgs<TT> a{(const TT*)q, ldq, (const TT*)kc, (const TT*)vc, nullptr, 0, 0, 0, (TT*)out, \
                       (const TT*)gate, gater, tables, maxb, tiles, cu, start, H, G, bs, scale, \
                       softcap, slopes, window, keep, sigb, vdiv};                              \
     return launch_win_tiles<TT>(a, ntiles, D, Dv, tile_rows, st);                              \

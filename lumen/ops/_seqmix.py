@@ -36,12 +36,13 @@ SIGNATURES = {
     "sm_group_rms": "iiplpppliiif",
     "sm_gate_rows": "iplplpiipi",
     "sm_rotate_heads": "iplliiippi",
-    "sm_latent_write": "iplppppppiiiiif",
+    "sm_latent_write": "iplpppppppiiiiif",
     "sm_head_norm_write": "iplpppppiiiiif",
     "sm_latent_attn": "i" "plli" "plli" "pl" "pi" "pll" "pi" "pp" "iii" "fffi" "ppp" "pl" "ipp",
     "sm_row_attn": "i" "plli" "plli" "pl" "pli" "pll" "pi" "pp" "iiiii" "fffi" "pppp" "piipl"
                    "pi" "ipp",
     "sm_win_attn_tiles": "iplppppl" "pi" "pi" "pp" "iiii" "ff" "p" "iii" "ipi",
+    "sm_fresh_tiles": "i" "plplplpl" "p" "pii" "pp" "iiii" "f",
     "sm_row_norm_write": "iplpppppiiif",
     "sm_layer_norm": "iippfpppiif",
     "sm_embed_pos": "ipppppiiii",
@@ -90,6 +91,8 @@ def _load():
         lib.sm_chunk_attn_tiles_ok.restype = ctypes.c_int
         lib.sm_win_attn_tiles_ok.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int]
         lib.sm_win_attn_tiles_ok.restype = ctypes.c_int
+        lib.sm_fresh_tiles_ok.argtypes = [ctypes.c_int] * 4
+        lib.sm_fresh_tiles_ok.restype = ctypes.c_int
         lib.sm_row_attn_lds.argtypes = [ctypes.c_int, ctypes.c_int]
         lib.sm_row_attn_lds.restype = ctypes.c_int
         lib.sm_latent_attn_ok.argtypes = [ctypes.c_int] * 5
@@ -131,6 +134,12 @@ def win_tiles_ok(dt: int, D: int, Dv: int = 0) -> bool:
     """Does the matrix-core prefill attention over paged key and value caches have a kernel for
     this dtype code / key size / value size (0: the key size)?"""
     return bool(_load().sm_win_attn_tiles_ok(dt, D, Dv or D))
+
+
+def fresh_tiles_ok(dt: int, D1: int, Dr: int, Dv: int) -> bool:
+    """Does the prompt attention over a step's own rows have a kernel for this dtype code / key size / shared key
+    size / value size?"""
+    return bool(_load().sm_fresh_tiles_ok(dt, D1, Dr, Dv))
 
 
 def row_attn_lds(HB: int, Dk: int) -> int:

@@ -588,7 +588,7 @@ def chunk_sink_attention(q: torch.Tensor, cache: torch.Tensor, seg, H: int, G: i
 # dot product and the softmax is a parameter: a position-dependent query temperature, a tanh soft
 # cap, a logarithmic distance bias per head, a mixing of the heads' scores, a per-head sink in
 # the softmax denominator.  Scores and weights are fp32.
-def latent_write_ref(z, w_norm, inv_freq, positions, slots, cache, R, dims, eps, vt=None):
+def latent_write_ref(z, w_norm, inv_freq, positions, slots, cache, R, dims, eps, vt=None, own=None):
     zf = z.float()
     c = zf[:, :R]
     c = c / torch.sqrt((c * c).mean(-1, keepdim=True) + eps) * w_norm.float()
@@ -603,6 +603,8 @@ def latent_write_ref(z, w_norm, inv_freq, positions, slots, cache, R, dims, eps,
     if vt is not None:
         bs = vt.shape[2]
         vt[slots[ok] // bs, :, slots[ok] % bs] = c[ok].to(vt.dtype)
+    if own is not None:
+        own.copy_(torch.cat([c, kr], 1))
 
 
 def transposed_values_ok(dtype, R: int, Dr: int, block_size: int, device) -> bool:
@@ -617,12 +619,14 @@ def transposed_values_ok(dtype, R: int, Dr: int, block_size: int, device) -> boo
 
 def latent_write(z: torch.Tensor, w_norm: torch.Tensor, inv_freq: torch.Tensor,
                  positions: torch.Tensor, slots: torch.Tensor, cache: torch.Tensor, R: int,
-                 dims: int, eps: float, vt: Optional[torch.Tensor] = None) -> None:
+                 dims: int, eps: float, vt: Optional[torch.Tensor] = None,
+                 own: Optional[torch.Tensor] = None) -> None:
     """Rows of a latent-attention layer's down projection z [T, R + Dr] into the paged cache
     [blocks, block, R + Dr] at ``slots`` (int64; -1 skips): the first R columns RMS-normed with
     ``w_norm``, the rest (the key part all heads share) rotated on its first ``dims`` columns.
     ``vt`` [blocks, R, block] (optional) takes the normed latents once more, transposed within
-    each cache block: the layout the matrix-core value product reads (keys contiguous)."""
+    each cache block: the layout the matrix-core value product reads (keys contiguous).  ``own``
+    [T, R + Dr] (optional) takes the cache rows once more, in the step's order, skipped ones too."""
     from ._seqmix import DT, call, use_seqmix
 
     Dr = z.shape[1] - R
@@ -633,11 +637,61 @@ def latent_write(z: torch.Tensor, w_norm: torch.Tensor, inv_freq: torch.Tensor,
                            or vt.dtype != cache.dtype or not vt.is_contiguous()):
         raise ValueError(f"transposed copy {tuple(vt.shape)} does not match cache "
                          f"{tuple(cache.shape)} with latent size {R}")
+    if own is not None and (tuple(own.shape) != (z.shape[0], R + Dr) or own.dtype != cache.dtype
+                            or not own.is_contiguous()):
+        raise ValueError(f"rows {tuple(own.shape)} do not match a step of {z.shape[0]} rows of {R + Dr}")
     if not use_seqmix(z):
-        return latent_write_ref(z, w_norm, inv_freq, positions, slots, cache, R, dims, eps, vt)
+        return latent_write_ref(z, w_norm, inv_freq, positions, slots, cache, R, dims, eps, vt, own)
     assert z.stride(1) == 1 and cache.is_contiguous() and cache.dtype == z.dtype
     call("sm_latent_write", DT[z.dtype], z, z.stride(0), w_norm, inv_freq, positions, slots, cache,
-         vt, cache.shape[1], z.shape[0], R, Dr, dims, eps)
+         vt, own, cache.shape[1], z.shape[0], R, Dr, dims, eps)
+
+
+def fresh_latent_ok(dtype: torch.dtype, seg, D: int, Dr: int, Dv: int) -> bool:
+    """Can ``fresh_latent_attention`` run the step's prompt portions?"""
+    from ._seqmix import DT, fresh_tiles_ok
+
+    return (seg.fresh and seg.q_tiles is not None and seg.tile_rows > 0 and seg.cu.is_cuda
+            and dtype in (torch.bfloat16, torch.float16) and fresh_tiles_ok(DT[dtype], D, Dr, Dv))
+
+
+def fresh_latent_attention_ref(q, k, kr, v, out, seg, scale):
+    n, rows = seg.portions()
+    cu = seg.cu.tolist()
+    for a, b in zip(cu[:n], cu[1:n + 1]):
+        H = k.shape[1]
+        kk = torch.cat([k[a:b].float(), kr[a:b].float()[:, None].expand(-1, H, -1)], 2)
+        s = torch.einsum("thd,jhd->htj", q[a:b].float(), kk) * scale
+        s = s.masked_fill(torch.ones(b - a, b - a, dtype=torch.bool, device=s.device).triu(1), -math.inf)
+        out[a:b] = torch.einsum("htj,jhd->thd", torch.softmax(s, -1), v[a:b].float()).to(out.dtype)
+    return out
+
+
+def fresh_latent_attention(q: torch.Tensor, k: torch.Tensor, kr: torch.Tensor, v: torch.Tensor, out: torch.Tensor,
+                           seg, scale: float) -> torch.Tensor:
+    """Causal attention of a step's prompt portions that all start at position 0 (``seg.fresh``) over their own
+    rows: q [T, H, D + Dr] against the keys [k_h | kr], k [T, H, D] and kr [T, Dr], which the heads share; values
+    v [T, H, Dv].  ``out`` [T, H, Dv].  Heads and columns are contiguous, rows have any stride of whole 16-byte
+    chunks.  Latent attention of a fresh prompt: expanding a row's latent into its heads' keys and values takes
+    the products that projecting the queries into the latent space and the result out of it do, and the scores
+    and sums then run over D + Dr and Dv columns instead of R + Dr and R."""
+    from ._seqmix import DT, call, use_seqmix
+
+    T, H, D = k.shape
+    Dr, Dv = kr.shape[1], v.shape[2]
+    if not seg.fresh or seg.q_tiles is None:
+        raise ValueError("fresh latent attention: a step with prompt portions from position 0")
+    rows = seg.tile_rows
+    if (tuple(q.shape[1:]) != (H, D + Dr) or v.shape[1] != H or min(q.shape[0], T, kr.shape[0], v.shape[0],
+            out.shape[0]) < rows or tuple(out.shape[1:]) != (H, Dv) or not out.is_contiguous()
+            or any(x.dtype != q.dtype or x.device != q.device for x in (k, kr, v, out))
+            or any(x.stride(2) != 1 or x.stride(1) != x.shape[2] for x in (q, k, v)) or kr.stride(1) != 1):
+        raise ValueError("fresh latent attention: q [T, H, D + Dr], k [T, H, D], kr [T, Dr], v and out [T, H, Dv]")
+    if not use_seqmix(q):
+        return fresh_latent_attention_ref(q, k, kr, v, out, seg, scale)
+    call("sm_fresh_tiles", DT[q.dtype], q, q.stride(0), k, k.stride(0), kr, kr.stride(0), v, v.stride(0), out,
+         seg.q_tiles, seg.q_tiles.shape[0], seg.tile_size, seg.cu, seg.start, H, D, Dr, Dv, scale)
+    return out
 
 
 def head_norm_write_ref(qkv, wq, wk, slots, kcache, vcache, H, G, D, Dv, eps):

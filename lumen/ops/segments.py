@@ -6,7 +6,7 @@ the recurrent state already hold).  The kernels need, per segment, where its row
 state slot carries its sequence and which cache blocks hold its keys."""
 from __future__ import annotations
 
-from dataclasses import dataclass
+from dataclasses import dataclass, replace
 from typing import Optional
 
 import torch
@@ -27,6 +27,7 @@ class SegBatch:
     q_tiles: Optional[torch.Tensor] = None
     tile_rows: int = 0
     tile_size: int = 64       # rows per tile of q_tiles (TILE_ROWS when they were cut)
+    fresh: bool = False       # every portion starts at position 0: its keys are rows of this step
 
     @property
     def S(self) -> int:
@@ -44,6 +45,13 @@ class SegBatch:
             return self.S - (self.T - self.tile_rows), self.tile_rows
         return (0, 0) if self.S == self.T else (self.S, self.T)
 
+    def decoded(self) -> "SegBatch":
+        """The rows after the prompt portions, with the step's segments, offsets and tables: what a row's
+        attention reads (``row_seg``, ``positions``, ``tables``, ``cache_slots``)."""
+        n = self.tile_rows
+        return replace(self, row_seg=self.row_seg[n:], positions=self.positions[n:], q_tiles=None, tile_rows=0,
+                       fresh=False, cache_slots=None if self.cache_slots is None else self.cache_slots[n:])
+
 
 import os
 
@@ -57,6 +65,13 @@ def tile_list(cu, n_segments: int, rows: int = 0):
     (host ints) in tiles of ``rows`` (default TILE_ROWS) rows."""
     rows = rows or TILE_ROWS
     return [(s, r) for s in range(n_segments) for r in range(int(cu[s]), int(cu[s + 1]), rows)]
+
+
+def whole_prompts(cu, kv_lens, tile_rows: int) -> bool:
+    """Do the portions of row offsets ``cu`` (host ints) that make a step's first ``tile_rows`` rows all start at
+    position 0, i.e. has each as many rows as its sequence has keys (``kv_lens``, host)?"""
+    return (tile_rows > 0 and kv_lens is not None and cu is not None and len(cu) == len(kv_lens) + 1
+            and cu[-1] == tile_rows and all(b - a == n for a, b, n in zip(cu, cu[1:], kv_lens)))
 
 
 def whole_sequences(lengths, device, slots=None, block_size: int = 16) -> SegBatch:
@@ -80,4 +95,4 @@ def whole_sequences(lengths, device, slots=None, block_size: int = 16) -> SegBat
     return SegBatch(torch.tensor(cu, **i32),
                     torch.tensor(list(slots) if slots is not None else list(range(S)), **i32),
                     torch.zeros(S, **i32), row_seg, pos, tables, torch.cat(cache_slots),
-                    torch.tensor(tile_list(cu, S), **i32).view(-1, 2), cu[-1], TILE_ROWS)
+                    torch.tensor(tile_list(cu, S), **i32).view(-1, 2), cu[-1], TILE_ROWS, True)

@@ -34,7 +34,7 @@ being static buffers; padding rows use the spare state slot and write no keys.
 """
 from __future__ import annotations
 
-from dataclasses import dataclass, field
+from dataclasses import dataclass, field, replace
 from typing import Dict, List, Optional
 
 import torch
@@ -42,7 +42,8 @@ import torch.nn.functional as F
 
 from ..models.config import ModelConfig
 from ..models.gedatar import DELTA_DECAY, DELTA_KEY_EPS
-from ..ops.attention import (chunk_sink_attention, diff_head_combine, head_norm_rotary_write,
+from ..ops.attention import (chunk_sink_attention, diff_head_combine, fresh_latent_attention,
+                             fresh_latent_ok, head_norm_rotary_write,
                              head_norm_write, latent_write, row_attention,
                              row_norm_rotary_write, row_norm_write, transposed_values_ok,
                              write_key_cache)
@@ -55,7 +56,7 @@ from ..ops.norm import (SPLIT, depth_mix_norm, dyt, dyt_residual, embed_rms, gat
                         residual_rms, scaled_residual_layer_norm, weight_layer_norm)
 from ..ops.recurrent import delta_scan, head_scan, min_gru_scan, token_shift, wkv_scan
 from ..ops.rope import rotary_write, rotate_interleaved_
-from ..ops.segments import SegBatch, whole_sequences
+from ..ops.segments import SegBatch, whole_prompts, whole_sequences
 from .model_runner import ModelRunner, StepInput, fill_step
 
 
@@ -306,7 +307,9 @@ def run_layers(w: HybridWeights, st: HybridState, tokens: torch.Tensor, seg: Seg
 #       q  = W_uq (rms(z_q) * w), its rotated part turned in place               (rotate_interleaved_)
 #       qa = per-head W_uk^T q_plain         the query in the latent space (batched GEMM)
 #       ol = row_attention([qa | q_rot] against the cached row, value = its first R columns)
-#       y  = W_o (per-head W_uv ol)          (batched GEMM into the token-major layout, then GEMM)
+#       o  = per-head W_uv ol                (batched GEMM into the token-major layout);  y = W_o o
+#       prompts from position 0: [k | v] = [W_uk ; W_uv] latent of the step's rows instead (one GEMM), then
+#       o  = fresh_latent_attention(q, [k | rotated part], v)
 #   attention
 #       qkv = [W_q ; W_k ; W_v] xb + b       one GEMM
 #       q normed in place, normed k and v into their caches                      (head_norm_write)
@@ -366,7 +369,8 @@ class DalavikWeights:
                     if own:
                         L.w["dkv_norm"] = f32(x + "dkv.norm")
                     L.w["uq"] = t(x + "uq").detach()
-                    L.w["uk"] = t(x + "uk").detach().view(H, D, R)                   # q_h @ uk[h]
+                    L.w["ukv"] = torch.cat([t(x + "uk"), t(x + "uv")], 0).contiguous()
+                    L.w["uk"] = L.w["ukv"][:H * D].view(H, D, R)                     # q_h @ uk[h]
                     L.w["uvT"] = t(x + "uv").detach().view(H, Dv, R).transpose(1, 2).contiguous()
                     L.w["inv_freq"] = interleaved_inv_freq(m["rot"]["dims"], m["rot"]["base"], dev)
                 else:
@@ -436,25 +440,37 @@ def run_dalavik_layers(w: DalavikWeights, st: DalavikState, tokens: torch.Tensor
     xb = F.embedding(tokens, w.embed).to(dt)      # (the rows as stored are their own copy in `dt`)
     x = xb.float()
     cast = dt if dt != torch.float32 else None
+    own: Dict[int, Optional[torch.Tensor]] = {}
     for i, L in enumerate(w.layers):
         m = L.m
         if L.kind == "latent_attention":
             H, D, Dr, Dv, R, Q = (m["heads"], m["dim"], m["rot_dim"], m["vdim"], m["kv_rank"],
                                   m["q_rank"])
             z = project(xb, L.w["down"])
+            fresh = seg.tile_rows if fresh_latent_ok(dt, seg, D, Dr, Dv) else 0
             if L.kv_layer == i:
+                # the step's own cache rows, for this layer's fresh prompts and those of borrowing layers
+                own[i] = torch.empty(T, R + Dr, dtype=dt, device=x.device) if fresh else None
                 latent_write(z[:, Q:], L.w["dkv_norm"], L.w["inv_freq"], seg.positions,
-                             seg.cache_slots, st.lat[i], R, m["rot"]["dims"], eps, st.latT[i])
+                             seg.cache_slots, st.lat[i], R, m["rot"]["dims"], eps, st.latT[i], own[i])
             cache = st.lat[L.kv_layer]
             q = project(group_rms_norm(z[:, :Q], L.w["dq_norm"], 1, eps, dt), L.w["uq"])
             rotate_interleaved_(q, seg.positions, H, D + Dr, D, m["rot"]["dims"], L.w["inv_freq"])
             q3 = q.view(T, H, D + Dr)
-            qa = torch.bmm(q3[:, :, :D].transpose(0, 1), L.w["uk"])              # [H, T, R]
-            ol = torch.empty(H, T, R, dtype=dt, device=x.device)
-            row_attention(qa.transpose(0, 1), q3[:, :, D:], cache, cache, R, ol.transpose(0, 1),
-                          seg, H, 1, float(m["scale"]), vt=st.latT[L.kv_layer])
             o = torch.empty(T, H, Dv, dtype=dt, device=x.device)
-            torch.bmm(ol, L.w["uvT"], out=o.transpose(0, 1))
+            if fresh:
+                c = own[L.kv_layer][:fresh]
+                kv = project(c[:, :R], L.w["ukv"])
+                fresh_latent_attention(q3[:fresh], kv[:, :H * D].view(fresh, H, D), c[:, R:],
+                                       kv[:, H * D:].view(fresh, H, Dv), o[:fresh], seg, float(m["scale"]))
+            if fresh < T:
+                n, sg = T - fresh, seg.decoded() if fresh else seg
+                q3, od = q3[fresh:], o[fresh:]
+                qa = torch.bmm(q3[:, :, :D].transpose(0, 1), L.w["uk"])          # [H, T, R]
+                ol = torch.empty(H, n, R, dtype=dt, device=x.device)
+                row_attention(qa.transpose(0, 1), q3[:, :, D:], cache, cache, R, ol.transpose(0, 1),
+                              sg, H, 1, float(m["scale"]), vt=st.latT[L.kv_layer])
+                torch.bmm(ol, L.w["uvT"], out=od.transpose(0, 1))
         else:
             H, G, D, Dv = m["heads"], m["kv_heads"], m["dim"], m["vdim"]
             qkv = project(xb, L.w["qkv"], L.w["qkv_b"])
@@ -1373,7 +1389,10 @@ class HybridRunner(ModelRunner):
 
     @torch.no_grad()
     def execute(self, inp: StepInput) -> torch.Tensor:
-        x = self.w.run_layers(self.state, inp.tokens, inp.seg, self.observe)
+        seg = inp.seg
+        if not seg.fresh and whole_prompts(inp.cu_seqlens, inp.kv_lens, seg.tile_rows):
+            seg = replace(seg, fresh=True)
+        x = self.w.run_layers(self.state, inp.tokens, seg, self.observe)
         if inp.extra_rows is not None and inp.extra_rows.numel():
             self.extra_logits = self._logits_rows(x, inp.extra_rows)
         return self._logits_rows(x, inp.sample_rows)

@@ -95,3 +95,79 @@ def test_scores_that_creep(rise, dtype, ulp):
     row_attention(q, None, k, v, D, out, seg, H, G, 1.0)
     row_attention_ref(q.float(), None, k.float(), v.float(), D, ref, seg, H, G, 1.0)
     close(out, ref, ulp)
+
+
+@pytest.mark.parametrize("dtype,ulp", DTYPES)
+@pytest.mark.parametrize("lens,extra", [([31, 32, 33, 1, 65], 0), ([127, 128, 129, 260], 3)])
+@pytest.mark.parametrize("H,tile", [(1, 128), (5, 128), (2, 64)])
+def test_fresh_latent_rows(H, tile, lens, extra, dtype, ulp):
+    """Prompts over their own rows against the reference, rows of wider buffers, decoded rows behind them."""
+    from lumen.ops.attention import fresh_latent_attention, fresh_latent_attention_ref, fresh_latent_ok
+
+    D, Dr, Dv = 128, 64, 128
+    g = torch.Generator().manual_seed(H + len(lens))
+    n, seg, _ = portions(lens + [1] * extra, [0] * len(lens) + [9] * extra, 16, g)
+    n -= extra
+    seg.q_tiles = torch.tensor(tile_list(seg.cu.tolist(), len(lens), tile), dtype=torch.int32, device="cuda").view(-1, 2)
+    seg.tile_rows, seg.tile_size, seg.fresh = n, tile, True
+    assert fresh_latent_ok(dtype, seg, D, Dr, Dv) and not fresh_latent_ok(dtype, seg, 64, Dr, Dv)
+    f = lambda *s: torch.randn(*s, generator=g).to(dtype).cuda()  # noqa: E731
+    q, kv, c = f(n + extra, H * (D + Dr) + 8), f(n, H * (D + Dv)), f(n, 24 + Dr)
+    args = (q[:n, :H * (D + Dr)].view(n, H, D + Dr), kv[:, :H * D].view(n, H, D), c[:, 24:],
+            kv[:, H * D:].view(n, H, Dv))
+    out, ref = (torch.zeros(n, H, Dv, dtype=dt, device="cuda") for dt in (dtype, torch.float32))
+    fresh_latent_attention(*args, out, seg, 0.07)
+    fresh_latent_attention_ref(*args, ref, seg, 0.07)
+    close(out, ref, ulp)
+    seg.fresh = False
+    with pytest.raises(ValueError):
+        fresh_latent_attention(*args, out, seg, 0.07)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_fresh_and_cached_prompts_agree(dtype):
+    """One engine step of whole prompts (expanded keys) against the same prompts in two portions (the cached latent):
+    logits of the same rows, with a decoded sequence beside them."""
+    import lumen.serve.hybrid_runner as R
+    from lumen.bench.hybrid_bench import dalavik_config
+    from lumen.models import build_model
+    from lumen.ops.segments import whole_sequences
+    from lumen.serve.model_runner import StepInput
+
+    cfg = dalavik_config(1024)
+    cfg.vocab_size = 512
+    torch.manual_seed(3)
+    model = build_model(cfg, dtype=dtype, device=torch.device("cuda"), init="random")
+    lens = [70, 1, 133]
+    tok = torch.randint(3, 500, (sum(lens),), device="cuda")
+    routes = []
+    real, R.fresh_latent_attention = R.fresh_latent_attention, lambda *a: (routes.append(1), real(*a))[1]
+    try:
+        out = []
+        for cut in (False, True):
+            run = R.HybridRunner(R.WEIGHTS["dalavik"](model), 64, 16, torch.device("cuda"), 256, 4, use_graphs=False)
+            whole = whole_sequences(lens, "cuda")
+            pos, cu = whole.positions, [0, 70, 71, 204]
+            parts = [[(0, 0, 40), (1, 0, 1), (2, 0, 90)], [(0, 40, 70), (2, 90, 133)]] if cut else \
+                [[(i, 0, n) for i, n in enumerate(lens)]]
+            x = None
+            for part in parts:
+                rows = torch.cat([torch.arange(cu[i] + a, cu[i] + b) for i, a, b in part]).cuda()
+                c = [0]
+                for _, a, b in part:
+                    c.append(c[-1] + b - a)
+                ids = torch.tensor([i for i, _, _ in part])
+                i32 = dict(dtype=torch.int32, device="cuda")
+                seg = SegBatch(torch.tensor(c, **i32), ids.int().cuda(), torch.tensor([a for _, a, _ in part], **i32),
+                               torch.cat([torch.full((b - a,), k) for k, (_, a, b) in enumerate(part)]).int().cuda(),
+                               pos[rows], whole.tables[ids.cuda()], whole.cache_slots[rows],
+                               torch.tensor(tile_list(c, len(part)), **i32).view(-1, 2), c[-1], 128)
+                inp = StepInput("mixed", tok[rows], pos[rows], seg.cache_slots, c, kv_lens=[b for _, _, b in part],
+                                sample_rows=torch.tensor(c[1:], device="cuda") - 1, seg=seg)
+                x = run.execute(inp)
+            out.append(x[[0, -1]].float())
+    finally:
+        R.fresh_latent_attention = real
+    assert len(routes) == 6                              # the whole prompts and the first portions, 3 layers
+    err = (out[0] - out[1]).norm() / out[1].norm()
+    assert err < (0.02 if dtype == torch.bfloat16 else 0.003), err       # 4 layers of 16-bit roundings

@@ -43,6 +43,7 @@ SIGNATURES = {
                    "pi" "ipp",
     "sm_win_attn_tiles": "iplppppl" "pi" "pi" "pp" "iiii" "ff" "p" "iii" "ipi",
     "sm_fresh_tiles": "i" "plplplpl" "p" "pii" "pp" "iiii" "f",
+    "sm_talk_tiles": "i" "pll" "pp" "pll" "pi" "pii" "pp" "iiiii" "fffi" "pppp",
     "sm_row_norm_write": "iplpppppiiif",
     "sm_layer_norm": "iippfpppiif",
     "sm_embed_pos": "ipppppiiii",
@@ -93,6 +94,8 @@ def _load():
         lib.sm_win_attn_tiles_ok.restype = ctypes.c_int
         lib.sm_fresh_tiles_ok.argtypes = [ctypes.c_int] * 4
         lib.sm_fresh_tiles_ok.restype = ctypes.c_int
+        lib.sm_talk_tiles_ok.argtypes = [ctypes.c_int] * 5
+        lib.sm_talk_tiles_ok.restype = ctypes.c_int
         lib.sm_row_attn_lds.argtypes = [ctypes.c_int, ctypes.c_int]
         lib.sm_row_attn_lds.restype = ctypes.c_int
         lib.sm_latent_attn_ok.argtypes = [ctypes.c_int] * 5
@@ -140,6 +143,11 @@ def fresh_tiles_ok(dt: int, D1: int, Dr: int, Dv: int) -> bool:
     """Does the prompt attention over a step's own rows have a kernel for this dtype code / key size / shared key
     size / value size?"""
     return bool(_load().sm_fresh_tiles_ok(dt, D1, Dr, Dv))
+
+
+def talk_tiles_ok(dt: int, H: int, G: int, D: int, Dv: int) -> bool:
+    """Does the prompt attention with mixed heads have a kernel for this dtype code / heads / sizes?"""
+    return bool(_load().sm_talk_tiles_ok(dt, H, G, D, Dv))
 
 
 def row_attn_lds(HB: int, Dk: int) -> int:

@@ -988,13 +988,14 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
     values that are a prefix of the key rows and a 16-bit dtype, the whole kernel runs on the
     matrix cores.
 
-    Three kernels serve it.  The prompt portions of a step (``seg.q_tiles``) go to the tiled
+    Several kernels serve it.  The prompt portions of a step (``seg.q_tiles``) go to the tiled
     matrix-core kernel of ``csrc/seqmix/window_attention.hip`` when the keys and values have caches
     of their own, one query part, head sizes it is built for (values as wide as the keys or twice
-    as wide), a 16-bit dtype and none of temperature, logarithmic bias, head mixing or sink; the latent layout with ``vt`` goes to the
+    as wide), a 16-bit dtype and none of temperature, logarithmic bias, head mixing or sink; with head mixing (heads
+    of 128, no window, linear bias, gate or sigmoid weights) to ``talk_attention.hip``; the latent layout with ``vt`` goes to the
     latent kernels (``latent_tile.hip`` for large prompt portions); every other row (decoded rows, fp32, other shapes) to the row kernel.  A row's
     result does not depend on which of them computed it beyond rounding."""
-    from ._seqmix import (DT, call, latent_attn_ok, latent_tiles_ok, use_seqmix,
+    from ._seqmix import (DT, call, latent_attn_ok, latent_tiles_ok, talk_tiles_ok, use_seqmix,
                           win_tiles_ok)
 
     T, _, D1 = q1.shape
@@ -1089,6 +1090,19 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
             return out
         q1, out, T = q1[Tp:], out[Tp:], T - Tp
         gate = gate[Tp:] if gate is not None else None
+    # mixed heads: 16 rows and all heads of a tile on the matrix cores
+    elif (talk is not None and seg.q_tiles is not None and seg.tile_rows > 0 and q2 is None and slopes is None
+            and window == 0 and gate is None and sigmoid_bias is None and v_div == 1
+            and vcache is not kcache and krow == G * D1 and vrow == G * Dv
+            and q1.dtype in (torch.bfloat16, torch.float16) and talk_tiles_ok(DT[q1.dtype], H, G, D1, Dv)
+            and al8(q1) and out.data_ptr() % 8 == 0 and out.stride(0) % 4 == 0 and out.stride(1) % 4 == 0):
+        Tp = seg.tile_rows
+        call("sm_talk_tiles", DT[q1.dtype], q1, q1.stride(0), q1.stride(1), kcache, vcache, out, out.stride(0),
+             out.stride(1), seg.tables, seg.tables.shape[1], seg.q_tiles, seg.q_tiles.shape[0], seg.tile_size,
+             seg.cu, seg.start, H, G, D1, Dv, bs, scale, float(softcap or 0.0), coef, every, r1, r2, talk, sink)
+        if Tp >= T:
+            return out
+        q1, out, T = q1[Tp:], out[Tp:], T - Tp
     row_seg, positions = seg.row_seg[Tp:], seg.positions[Tp:]
     HB = _heads_per_block(H, Dk, talk is not None)
     # few rows (decoding): deal a row's 64-key tiles out to several workgroups so that ~2 per CU

@@ -124,6 +124,37 @@ def test_fresh_latent_rows(H, tile, lens, extra, dtype, ulp):
         fresh_latent_attention(*args, out, seg, 0.07)
 
 
+@pytest.mark.parametrize("dtype,ulp", DTYPES)
+@pytest.mark.parametrize("lens,starts,bs,tile", [
+    ([15, 16, 17, 1, 33], [0, 0, 3, 31, 64], 16, 128), ([130, 64], [0, 35], 12, 64), ([20, 3], [560, 0], 1, 128)])
+@pytest.mark.parametrize("H,G,opts", [(1, 1, ()), (8, 2, ("cap", "r", "sink", "temp")), (12, 3, ("sink",)), (16, 4, ("r",)),
+                                      (16, 8, ("cap",)), (24, 6, ("cap", "r", "sink", "temp")), (32, 8, ("temp", "r"))])
+def test_mixed_head_tiles(H, G, opts, lens, starts, bs, tile, dtype, ulp):
+    D = 128
+    g = torch.Generator().manual_seed(H + bs)
+    T, seg, (k, v) = portions(lens + [1], starts + [40], bs, g, (G, D), (G, D))
+    seg.tile_rows, seg.tile_size = T - 1, tile             # (the last row is a decoded one)
+    seg.q_tiles = torch.tensor(tile_list(seg.cu.tolist(), len(lens), tile), dtype=torch.int32, device="cuda").view(-1, 2)
+    k, v = k.to(dtype).cuda(), v.to(dtype).cuda()
+    q = torch.randn(T, H * D + 8, generator=g).to(dtype).cuda()[:, :H * D].view(T, H, D)
+    f = lambda *s: torch.rand(*s, generator=g).cuda()  # noqa: E731
+    kw = dict(talk=torch.eye(H).cuda() + 0.3 * (f(H, H) - 0.5), softcap=4.0 if "cap" in opts else 0.0,
+              q_temp=(0.3, 16) if "temp" in opts else None, r1=f(H) if "r" in opts else None,
+              r2=f(H) if "r" in opts else None, sink=2 * f(H) - 1 if "sink" in opts else None)
+    import lumen.ops._seqmix as sm
+    calls, real = [], sm.call
+    sm.call = lambda n, *a: (calls.append(n), real(n, *a))[1]
+    try:
+        out = torch.full((T, H, D), float("nan"), dtype=dtype, device="cuda")
+        row_attention(q, None, k, v, D, out, seg, H, G, 0.1, **kw)
+    finally:
+        sm.call = real
+    assert calls == ["sm_talk_tiles", "sm_row_attn"]
+    ref = torch.zeros(T, H, D, device="cuda")
+    row_attention_ref(q.float(), None, k.float(), v.float(), D, ref, seg, H, G, 0.1, **kw)
+    close(out, ref, ulp)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_fresh_and_cached_prompts_agree(dtype):
     """One engine step of whole prompts (expanded keys) against the same prompts in two portions (the cached latent):

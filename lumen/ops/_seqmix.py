@@ -44,6 +44,9 @@ SIGNATURES = {
     "sm_win_attn_tiles": "iplppppl" "pi" "pi" "pp" "iiii" "ff" "p" "iii" "ipi",
     "sm_fresh_tiles": "i" "plplplpl" "p" "pii" "pp" "iiii" "f",
     "sm_talk_tiles": "i" "pll" "pp" "pll" "pi" "pii" "pp" "iiiii" "fffi" "pppp",
+    "sm_expert_sort": "pppppiii",
+    "sm_expert_act": "iplp" "ppppp" "iiiiii" "iii" "ffff",
+    "sm_expert_down": "ippp" "pp" "ppp" "iiiiii",
     "sm_row_norm_write": "iplpppppiiif",
     "sm_layer_norm": "iippfpppiif",
     "sm_embed_pos": "ipppppiiii",
@@ -96,6 +99,8 @@ def _load():
         lib.sm_fresh_tiles_ok.restype = ctypes.c_int
         lib.sm_talk_tiles_ok.argtypes = [ctypes.c_int] * 5
         lib.sm_talk_tiles_ok.restype = ctypes.c_int
+        lib.sm_expert_ok.argtypes = [ctypes.c_int] * 7
+        lib.sm_expert_ok.restype = ctypes.c_int
         lib.sm_row_attn_lds.argtypes = [ctypes.c_int, ctypes.c_int]
         lib.sm_row_attn_lds.restype = ctypes.c_int
         lib.sm_latent_attn_ok.argtypes = [ctypes.c_int] * 5
@@ -148,6 +153,11 @@ def fresh_tiles_ok(dt: int, D1: int, Dr: int, Dv: int) -> bool:
 def talk_tiles_ok(dt: int, H: int, G: int, D: int, Dv: int) -> bool:
     """Does the prompt attention with mixed heads have a kernel for this dtype code / heads / sizes?"""
     return bool(_load().sm_talk_tiles_ok(dt, H, G, D, Dv))
+
+
+def expert_ok(dt: int, T: int, W: int, E: int, top: int, ff: int, ffs: int) -> bool:
+    """Do the products over chosen experts have kernels for this dtype code and these sizes?"""
+    return bool(_load().sm_expert_ok(dt, T, W, E, top, ff, ffs))
 
 
 def row_attn_lds(HB: int, Dk: int) -> int:

@@ -17,6 +17,9 @@ projections side by side in one [W, E * ff + ffs] weight):
 * ``moe_grouped_mm``: the same arithmetic on the library's grouped GEMM (16-bit dtypes): the
   sorted (row, expert) pairs have a static count, the group offsets stay on the device, nothing
   synchronises and a layer's experts are three launches.
+* ``moe_chosen``: the (row, expert) pairs sorted by expert on the device, both products on HIP kernels
+  (``csrc/seqmix/expert_gemm.hip``) that gather the rows themselves.  16-bit steps of more than a few rows take it,
+  decode graphs included; the other forms serve fp32, sizes without kernels and the few-row steps.
 """
 from __future__ import annotations
 
@@ -26,7 +29,7 @@ from typing import Optional, Union
 import torch
 import torch.nn.functional as F
 
-from .gemm import THIN_MAX_K, _plain, _thin, project, row_bias_ok, thin_ok, weights_ok
+from .gemm import THIN_BATCH_MAX_W, THIN_MAX_K, THIN_MAX_M, _here, _plain, _thin, project, row_bias_ok, thin_ok, weights_ok
 
 
 def route_topk_ref(z: torch.Tensor, top: int) -> torch.Tensor:
@@ -356,6 +359,55 @@ def moe_grouped_mm(h, wts, gu_w, down_w, E: int, top: int, ff: int, ffs: int, ac
     return out.to(h.dtype)
 
 
+def chosen_ok(h, wts, gu_w, down_w, E: int, top: int, ff: int, ffs: int, act="silu", gated: bool = True,
+              weigh: str = "output") -> bool:
+    """Can ``moe_chosen`` run these operands?"""
+    from ._seqmix import DT, expert_ok, use_seqmix
+
+    if not (h.is_cuda and h.dim() == 2 and h.dtype in (torch.bfloat16, torch.float16) and use_seqmix(h)):
+        return False
+    (T, W), k, N = h.shape, 2 if gated else 1, E * ff + ffs
+    return (T > 0 and h.stride(1) == 1 and h.stride(0) % 8 == 0 and h.stride(0) >= W and T * h.stride(0) < 1 << 31
+            and tuple(gu_w.shape) == (k * N, W) and tuple(down_w.shape) == (W, N)
+            and gu_w.dtype == down_w.dtype == h.dtype and gu_w.is_contiguous() and down_w.is_contiguous()
+            and gu_w.device == down_w.device == h.device and weights_ok(wts, h, E)
+            and (h.data_ptr() | gu_w.data_ptr() | down_w.data_ptr()) % 16 == 0
+            and 2 * max(ff, ffs) * W < 1 << 31 and 256 * N < 1 << 31 and 128 * max(ff, ffs) < 1 << 31
+            and (gated or isinstance(act, str) and weigh == "output")
+            and expert_ok(DT[h.dtype], T, W, E, top, ff, ffs) and _plain(h, gu_w, down_w, wts) and _here(h))
+
+
+def moe_chosen(h, wts, gu_w, down_w, E: int, top: int, ff: int, ffs: int, act="silu", gated: bool = True,
+               weigh: str = "output") -> torch.Tensor:
+    """The weighted sum of each row's chosen experts (+ the shared one) on the rows that chose them: HIP kernels that
+    read the rows where they lie and the counts on the device (seqmix/expert_gemm.hip).  A row has at most ``top``
+    non-zero weights.  Results of an expert stay fp32 until their sum is rounded."""
+    from ._seqmix import DT, call
+
+    if weigh not in ("output", "input"):
+        raise ValueError(f"unknown place of the routing weight {weigh!r}")
+    if not chosen_ok(h, wts, gu_w, down_w, E, top, ff, ffs, act, gated, weigh):
+        raise ValueError("chosen experts: rows, stacked weights and routing weights do not fit the kernels")
+    T, W = h.shape
+    dev, dt = h.device, DT[h.dtype]
+    n = T * top
+    ints = torch.empty(2 * n + E + 1, dtype=torch.int32, device=dev)
+    idx, place, off = ints[:n], ints[n:2 * n], ints[2 * n:]
+    wt = torch.empty(n, dtype=torch.float32, device=dev)
+    call("sm_expert_sort", wts, off, idx, wt, place, T, E, top)
+    a = torch.empty(n, ff, dtype=h.dtype, device=dev)
+    a_s = torch.empty(T, ffs, dtype=h.dtype, device=dev) if ffs else None
+    code, c = (GATE_ACTS[act], (0.0,) * 4) if isinstance(act, str) else (
+        4, (act.limit, act.limit_shared, act.slope, act.shift))
+    call("sm_expert_act", dt, h, h.stride(0), gu_w, off, idx, wt, a, a_s, T, W, E, top, ff, ffs, int(gated), code,
+         int(weigh == "input"), *c)
+    y = torch.empty(n, W, dtype=torch.float32, device=dev)
+    y_s = torch.empty(T, W, dtype=torch.float32, device=dev) if ffs else None
+    out = torch.empty(T, W, dtype=h.dtype, device=dev)
+    call("sm_expert_down", dt, a, a_s, down_w, off, place, y, y_s, out, T, W, E, top, ff, ffs)
+    return out
+
+
 # When the grouped form pays.  Measured on MI355X (bf16, 16 experts, widths 1024 - 4096, 512 - 16384
 # rows): the two stacked GEMMs of the dense form run at ~850 TFLOP/s, the grouped GEMMs at ~300, and
 # sorting the (row, expert) pairs costs ~0.4 - 0.8 ms per layer whatever the size.  The grouped form does
@@ -373,6 +425,16 @@ def grouped_pays(rows: int, E: int, top: int, expert_weights: int) -> bool:
     return rows * (E - GROUPED_RATE_RATIO * top) * expert_weights >= GROUPED_MIN_SAVING
 
 
+# Up to 32 rows the activation forms in the thin GEMM's epilogue and experts no row chose are not read; up to 64 the
+# thin GEMM still has the smaller stacks (width 1024, 8 experts of 704, top 2, 48 rows: 32 us against 39).  Beyond, at
+# the widths 1024 - 4096 and with 8 or 16 experts, dense -> chosen in us: 33 rows 240 -> 149 (4096) and 51 -> 44 (1536),
+# 80 rows 168 -> 156 and 52 -> 46, 256 rows 206 -> 167 and 67 -> 51; the one exception is width 2048 with 8 experts at 80 -
+# 160 rows, 52 -> 55.  Against the library's grouped product: 4096 rows 2721 -> 1685 (16 of 2816, width 4096).
+def chosen_pays(rows: int, gu_w: torch.Tensor) -> bool:
+    """Do ``rows`` rows run faster on their chosen experts' own rows than on all experts?"""
+    return rows > THIN_MAX_M or rows > THIN_ACT_MAX_M and gu_w.numel() > THIN_BATCH_MAX_W
+
+
 def moe(h, wts, gu_w, down_w, E: int, top: int, ff: int, ffs: int, act="silu",
         gated: bool = True, weigh: str = "output") -> torch.Tensor:
     """Weighted sum of each row's chosen experts (+ the shared expert): [T, W] in h's dtype.
@@ -380,6 +442,8 @@ def moe(h, wts, gu_w, down_w, E: int, top: int, ff: int, ffs: int, act="silu",
     expert in ``gu_w`` (``act`` also a ``ClampedGate``); else W_down act(W_up h) with the up rows
     alone.  ``weigh`` = "input": an expert sees its weight times h instead of weighing in with its
     output (gated experts)."""
+    if chosen_pays(h.shape[0], gu_w) and chosen_ok(h, wts, gu_w, down_w, E, top, ff, ffs, act, gated, weigh):
+        return moe_chosen(h, wts, gu_w, down_w, E, top, ff, ffs, act, gated, weigh)
     grouped = (grouped_pays(h.shape[0], E, top, (2 if gated else 1) * ff * h.shape[1])
                and not (h.is_cuda and torch.cuda.is_current_stream_capturing()))
     if grouped and grouped_mm_ok(h, ff):

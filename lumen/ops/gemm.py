@@ -138,6 +138,39 @@ def _thin(x, w, bias=None, out_dtype=None, blocks=None) -> torch.Tensor:
     return y
 
 
+ROW_MAX_K = 8192          # K a workgroup of seqmix/row_gemv.hip holds
+
+
+def row_norm_ok(x: torch.Tensor, norm_w: torch.Tensor, res: Optional[torch.Tensor], w: torch.Tensor,
+                gated: bool = False) -> bool:
+    """Can ``row_norm_linear`` run: one row, everything contiguous, of one 16-bit type and on one device?"""
+    xs = x.shape
+    if len(xs) != 2 or xs[0] != 1 or not x.is_cuda or w.dim() != 2:
+        return False
+    K, (N, Kw), dt = xs[1], w.shape, x.dtype
+    if (K != Kw or K % 8 or not 0 < K <= ROW_MAX_K or N % 4 or N == 0 or dt != w.dtype
+            or dt not in (torch.bfloat16, torch.float16) or tuple(norm_w.shape) != (K,)):
+        return False
+    ts = (x, norm_w, w) if res is None else (x, norm_w, w, res)
+    return (all(t.dtype == dt and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in ts)
+            and (res is None or res.shape == xs) and _plain(*ts) and _here(x) and use_native(x))
+
+
+def row_norm_linear(x: torch.Tensor, norm_w: torch.Tensor, eps: float, res: Optional[torch.Tensor],
+                    w: torch.Tensor, gated: bool = False) -> tuple:
+    """(y, s) of one row: s = x + ``res`` (x itself without one), y = w rms_norm(s) -- ``gated``: silu(first half) *
+    second half of it.  For operands that ``row_norm_ok`` has let pass."""
+    from ._seqmix import DT, call, use_seqmix
+
+    use_seqmix(x)
+    K, N = x.shape[1], w.shape[0]
+    F = N // 2 if gated else N
+    y = torch.empty((1, F), device=x.device, dtype=x.dtype)
+    s = torch.empty_like(x) if res is not None else x
+    call("sm_row_gemv", DT[x.dtype], x, res, norm_w, s if res is not None else None, w, y, K, F, int(gated), eps)
+    return y, s
+
+
 # Split-K GEMM (kernels/split_gemm.hip): long contractions over a few hundred rows, whose output has too few
 # tiles to fill the chip.  us, library -> split: K = 11008, N = 4096, rows 72 / 256 / 512 / 1000: 41 -> 32, 51 ->
 # 35, 72 -> 50, 113 -> 87; K = 22016 at 512: 139 (tuned) -> 91; K = 32000 at 512: 290 -> 123; K = 11264, N = 2048 at

@@ -34,7 +34,7 @@ from ..ops.activation import swiglu
 from ..ops.embedding import embedding
 from ..ops.attention import (flash_attention_fresh, flash_attention_paged, paged_decode,
                              rope_write_kv)
-from ..ops.gemm import linear_nt, swiglu_linear_nt
+from ..ops.gemm import linear_nt, row_norm_linear, row_norm_ok, swiglu_linear_nt
 from ..ops.moe import THIN_ACT_MAX_M, thin_act, thin_act_ok
 from ..ops.norm import rms_norm
 from ..ops.rope import rope_tables
@@ -248,8 +248,11 @@ class ModelRunner:
         ml = self.lora if lora_ids is not None else None
         masks = {n: ml.mask(lora_ids, n) for n in (1, 2, 3)} if ml is not None else None
         for i, L in enumerate(self.w.layers):
-            y, res = rms_norm(h, L.ln1, cfg.rms_norm_eps, res)
-            qkv = linear_nt(y, L.qkv)
+            if T == 1 and ml is None and row_norm_ok(h, L.ln1, res, L.qkv):
+                qkv, res = row_norm_linear(h, L.ln1, cfg.rms_norm_eps, res, L.qkv)
+            else:
+                y, res = rms_norm(h, L.ln1, cfg.rms_norm_eps, res)
+                qkv = linear_nt(y, L.qkv)
             if mark is not None and i == 0:
                 mark.record()   # split decode: the second half starts here
             if ml is not None:
@@ -260,6 +263,10 @@ class ModelRunner:
             a = self._allreduce(linear_nt(o, L.o))
             if ml is not None:
                 ml.apply(i, "o", o, a, masks, self._allreduce)
+            if T == 1 and ml is None and row_norm_ok(a, L.ln2, res, L.gate_up):
+                act, res = row_norm_linear(a, L.ln2, cfg.rms_norm_eps, res, L.gate_up, gated=True)
+                h = self._allreduce(linear_nt(act, L.down))
+                continue
             y2, res = rms_norm(a, L.ln2, cfg.rms_norm_eps, res)
             if (T <= THIN_ACT_MAX_M and ml is None and DECODE_SPLIT_MIN == 0 and use_native(y2)
                     and thin_act_ok(y2, None, L.gate_up, 0, 0, self.w.F)):
@@ -411,8 +418,11 @@ class ModelRunner:
                                 max_context, self.scale, self.decode_partition(N)).view(N, nh * D)
 
         h, res = self._layers(h, positions, slots, attn, lora_ids, mark=mark)
-        y, _ = rms_norm(h, self.w.norm, self.cfg.rms_norm_eps, res)
-        logits = linear_nt(y, self.w.lm_head)
+        if N == 1 and row_norm_ok(h, self.w.norm, res, self.w.lm_head):
+            logits, _ = row_norm_linear(h, self.w.norm, self.cfg.rms_norm_eps, res, self.w.lm_head)
+        else:
+            y, _ = rms_norm(h, self.w.norm, self.cfg.rms_norm_eps, res)
+            logits = linear_nt(y, self.w.lm_head)
         return self._vocab_gather(logits) if gather else logits
 
     def decode_partition(self, n_seqs: int) -> int:

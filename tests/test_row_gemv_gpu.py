@@ -1,0 +1,45 @@
+"""The norm, one row's projection and its activation in one launch (seqmix/row_gemv.hip): the separate kernels' result
+over K that ends inside a step or a wave's share, few and many rows, with and without a residual."""
+import pytest
+import torch
+
+from lumen.ops.activation import swiglu
+from lumen.ops.gemm import row_norm_linear, row_norm_ok
+from lumen.ops.norm import rms_norm
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype,ulp", [(torch.bfloat16, 2.0 ** -8), (torch.float16, 2.0 ** -11)])
+@pytest.mark.parametrize("K,N", [(8, 4), (520, 12), (1024, 4096), (1536, 100), (2048, 20000), (2056, 64), (3072, 52), (4096, 6000),
+                                 (4104, 32), (6144, 24), (8192, 4100)])
+@pytest.mark.parametrize("gated,with_res", [(False, True), (True, True), (True, False), (False, False)])
+def test_row_norm_linear(K, N, gated, with_res, dtype, ulp):
+    g = torch.Generator().manual_seed(K + N)
+    f = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    x, w, nw = f(1, K).to(dtype).cuda(), (f(N, K) * K ** -0.5).to(dtype).cuda(), (1 + 0.1 * f(K)).to(dtype).cuda()
+    res = (3 * f(1, K)).to(dtype).cuda() if with_res else None
+    with torch.no_grad():
+        assert row_norm_ok(x, nw, res, w, gated)
+        y, s = row_norm_linear(x, nw, 1e-5, res, w, gated)
+        yn, sn = rms_norm(x, nw, 1e-5, res)
+    assert torch.equal(s, sn)
+    ref = yn.double() @ w.double().t()                        # (the normed row rounds as the norm kernel's)
+    if gated:
+        ref = torch.nn.functional.silu(ref[:, :N // 2]) * ref[:, N // 2:]
+    assert y.shape == ref.shape
+    # the result's rounding (the type's unit roundoff, 2^-8 or 2^-11 of each entry: half the spacing 2^-7 or 2^-10 of
+    # numbers from 1 on) and the fp32 sums of K products of rms 1 / sqrt(K)
+    assert ((y.double() - ref).abs() <= 1.01 * ulp * ref.abs() + 2e-5 * max(1.0, float(ref.abs().max()))).all()
+
+
+def test_refusals():
+    x, w, nw = (torch.ones(*s, dtype=torch.bfloat16, device="cuda") for s in ((1, 64), (8, 64), (64,)))
+    with torch.no_grad():
+        assert row_norm_ok(x, nw, None, w)
+        big = torch.ones(1, 8200, dtype=torch.bfloat16, device="cuda")
+        for bad in ((x.expand(2, 64), nw, None, w), (x, nw.float(), None, w), (x, nw, None, w[:6]), (x, nw[:32], None, w),
+                    (x, nw, x.half(), w), (x, nw, None, w.t().contiguous().t()), (x.cpu(), nw, None, w),
+                    (big, big[0], None, big.expand(8, -1).contiguous())):
+            assert not row_norm_ok(*bad)
+    assert not row_norm_ok(x.clone().requires_grad_(), nw, None, w)

@@ -84,7 +84,8 @@ void lumen_set_rms_lds(int, int);
 hipError_t lumen_paged_attention_decode(int, void*, const void*, const void*, const void*,
                                         const int*, const int*, int, int, int, int, int, int, int,
                                         float, float*, float*, void*, int, unsigned*, int, int,
-                                        int, hipStream_t);
+                                        int, const int*, const float*, const float*,
+                                        const long long*, hipStream_t);
 hipError_t lumen_kv_dequant(int, const void*, const void*, void*, void*, const int*, int,
                             const int*, int, int, int, int, int, hipStream_t);
 hipError_t lumen_reshape_and_cache(int, const void*, const void*, void*, void*, const long long*,
@@ -735,10 +736,21 @@ void paged_attention_decode(at::Tensor& out, const at::Tensor& q, const at::Tens
                             const at::Tensor& context_lens, int64_t num_kv_heads, int64_t block_size,
                             int64_t max_blocks_per_seq, double scale, at::Tensor& tmp_m,
                             at::Tensor& tmp_l, at::Tensor& tmp_o, int64_t partition_size,
-                            const std::optional<at::Tensor>& counters, int64_t one_pass) {
+                            const std::optional<at::Tensor>& counters, int64_t one_pass,
+                            const std::optional<at::Tensor>& pos, const std::optional<at::Tensor>& cos_t,
+                            const std::optional<at::Tensor>& sin_t, const std::optional<at::Tensor>& slots) {
   if (!q.is_cuda()) throw std::invalid_argument("lumen: q must be a GPU tensor");
   need_cuda(out, "out");
   const int num_seqs = static_cast<int>(q.size(0));
+  // the step's own tokens: q is the q part of its fused q|k|v rows, which the kernel reads on
+  if (pos.has_value()) {
+    if (!cos_t || !sin_t || !slots || pos->scalar_type() != at::kInt || slots->scalar_type() != at::kLong ||
+        cos_t->scalar_type() != at::kFloat || sin_t->scalar_type() != at::kFloat || pos->numel() < num_seqs ||
+        slots->numel() < num_seqs || q.stride(0) < (q.size(1) + 2 * num_kv_heads) * q.size(2))
+      throw std::invalid_argument("lumen: paged_attention_decode of new tokens: int32 positions, int64 slots, "
+                                  "fp32 rotary tables, q in its q|k|v rows");
+    need_cuda(*pos, "pos"); need_cuda(*cos_t, "cos"); need_cuda(*sin_t, "sin"); need_cuda(*slots, "slots");
+  }
   const int nh = static_cast<int>(q.size(1));
   const int D = static_cast<int>(q.size(2));
   // q may be a view into the fused qkv rows: heads contiguous, rows at any multiple of D
@@ -764,6 +776,8 @@ void paged_attention_decode(at::Tensor& out, const at::Tensor& q, const at::Tens
                                      tmp_m.data_ptr<float>(), tmp_l.data_ptr<float>(),
                                      tmp_o.data_ptr(), static_cast<int>(partition_size), cnt,
                                      static_cast<int>(one_pass), is_fp8(k_cache) ? 1 : 0, qldh,
+                                     pos ? pos->data_ptr<int>() : nullptr, ptr<float>(cos_t), ptr<float>(sin_t),
+                                     slots ? reinterpret_cast<const long long*>(slots->data_ptr<int64_t>()) : nullptr,
                                      cur_stream()),
         "paged_attention_decode");
 }
@@ -1097,7 +1111,12 @@ PYBIND11_MODULE(_C, m) {
     lumen_set_rms_lds(static_cast<int>(f), static_cast<int>(b));
   });
   m.def("rope_cache_write", &rope_cache_write);
-  m.def("paged_attention_decode", &paged_attention_decode);
+  m.def("paged_attention_decode", &paged_attention_decode, py::arg("out"), py::arg("q"), py::arg("k_cache"),
+        py::arg("v_cache"), py::arg("block_tables"), py::arg("context_lens"), py::arg("num_kv_heads"),
+        py::arg("block_size"), py::arg("max_blocks_per_seq"), py::arg("scale"), py::arg("tmp_m"), py::arg("tmp_l"),
+        py::arg("tmp_o"), py::arg("partition_size"), py::arg("counters"), py::arg("one_pass"),
+        py::arg("pos") = py::none(), py::arg("cos") = py::none(), py::arg("sin") = py::none(),
+        py::arg("slots") = py::none());
   m.def("reshape_and_cache", &reshape_and_cache);
   m.def("sample", &sample, py::arg("logits"), py::arg("temperature"), py::arg("top_p"),
         py::arg("top_k"), py::arg("seed"), py::arg("offset"), py::arg("out_tokens"),

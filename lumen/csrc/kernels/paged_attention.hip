@@ -1,4 +1,4 @@
-// Paged-KV decode attention + KV-cache write (serving half of the north star).
+// Paged-KV decode attention + KV-cache write.
 //
 // Reference behaviour: the reference only declares vLLM 0.6.0 serving (README.md:10,16,
 // requirements.txt:17-18); vLLM's PagedAttention v1/v2 reads K/V through per-sequence block
@@ -340,6 +340,48 @@ __device__ __forceinline__ void pa_fence_reg(R& a, R& b) {
   }
 }
 
+typedef __bf16 pa_bf16x2 __attribute__((ext_vector_type(2)));
+
+// the sum of 8 products of a 16-bit row piece with the query's, fp32 (bf16: both rows as they are, products exact;
+// fp16: mixed fmas, since the dot instruction need not keep subnormals)
+template <typename T>
+__device__ __forceinline__ float pa_dot8(const uint4& k, const uint4& q) {
+  float s = 0.f;
+  if constexpr (std::is_same<T, bf16>::value) {
+    const unsigned kk[4] = {k.x, k.y, k.z, k.w}, qq[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      s = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(pa_bf16x2, kk[j]),
+                                          __builtin_bit_cast(pa_bf16x2, qq[j]), s, false);
+  } else {
+    const T *a = reinterpret_cast<const T*>(&k), *b = reinterpret_cast<const T*>(&q);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s = fmaf(to_f32(a[j]), to_f32(b[j]), s);
+  }
+  return s;
+}
+
+// a cached row piece as 16-bit values (every fp8 value is one of bf16's and fp16's)
+template <typename T, typename KT, typename R>
+__device__ __forceinline__ uint4 pa_row16(const R& r) {
+  if constexpr (std::is_same<KT, fp8>::value) {
+    float f[8];
+    cvt8kv<T, KT>(r, f);
+    return make_uint4(pk2<T>(f[0], f[1]), pk2<T>(f[2], f[3]), pk2<T>(f[4], f[5]), pk2<T>(f[6], f[7]));
+  } else {
+    return r;
+  }
+}
+
+// A decode step's own tokens (the NEW form): rows' positions, rotary tables, cache slots (< 0: not written).
+struct PaNew {
+  const int* pos;
+  const float *cos_t, *sin_t;
+  void *kc, *vc;
+  const long long* slots;
+  int swap;                    // grid (kv head, sequence) instead of (sequence, kv head)
+};
+
 // UNI (block_size == rows per workgroup step, the launcher checks): row t = base + u * NGR + grp
 // of an iteration lies in block (base / BS + u) at offset grp, so the block ids are
 // workgroup-uniform -- scalar loads issued one iteration ahead -- instead of a per-lane block
@@ -348,13 +390,17 @@ __device__ __forceinline__ void pa_fence_reg(R& a, R& b) {
 // PF (with UNI): software-pipelined -- iteration i+1's K / V pieces are issued before iteration
 // i's softmax / P.V work, so every wave keeps two iterations of loads in flight (a pure nt read
 // stream reaches 7.1 TB/s on this chip with 8 x 16 B per lane in flight, profiles/r5_decode)
-template <typename T, int D, int G, typename KT = T, bool UNI = false, bool PF = false>
+// NEW: q is the step's fused q|k|v rows as projected, and the last token of every context is the step's own,
+// not yet cached.  The workgroup turns its query heads itself, walks the cached rows, and the one
+// whose partition ends the context turns the key, writes key and value into the cache and takes them from
+// registers: the rotary-and-cache kernel of a decode step (4 us of launch a layer) is gone.
+template <typename T, int D, int G, typename KT = T, bool UNI = false, bool PF = false, bool NEW = false>
 __global__ void __launch_bounds__(256) pa_decode1_kernel(
     T* __restrict__ out, const T* __restrict__ q, const KT* __restrict__ kc,
     const KT* __restrict__ vc, const int* __restrict__ block_tables,
     const int* __restrict__ context_lens, int nh, int qldh, int nkv, int BS, int max_blocks, int max_parts,
     float scale, float* __restrict__ tmp_m, float* __restrict__ tmp_l, float* __restrict__ tmp_o,
-    int PART) {
+    int PART, PaNew fresh) {
   constexpr int LPT = D / 8;        // lanes per cache row (8 elements each)
   constexpr int NGR = 256 / LPT;    // row groups per workgroup
   // K and V rows in flight per lane, loaded raw and converted at use: 4 of 16-bit rows (16 bytes
@@ -365,20 +411,46 @@ __global__ void __launch_bounds__(256) pa_decode1_kernel(
   constexpr int U = F8 ? 8 : 4;
   using Raw = typename std::conditional<F8, uint2, uint4>::type;
   __shared__ float wst[4][G][D + 2];  // per-wave merged state: acc[D], m, l
-  const int seq = blockIdx.x, kvh = blockIdx.y, part = blockIdx.z;
+  const int seq = fresh.swap ? blockIdx.y : blockIdx.x, kvh = fresh.swap ? blockIdx.x : blockIdx.y, part = blockIdx.z;
   const int ctx = context_lens[seq];
   const int start = part * PART;
   if (start >= ctx) return;
-  const int end = min(ctx, start + PART);
+  const int end = min(NEW ? ctx - 1 : ctx, start + PART);    // the cached rows'
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int grp = tid / LPT, d0 = (tid % LPT) * 8;
-  float qv[G][8];
+  // NEW: the turned pair of a head row's 8 elements and those half a head away, rounded as the row stores them
+  // (explicit fmas, as in rope_cache_kernel: bit-identical)
+  const auto tables = [&](float (&cs)[8], float (&sn)[8]) {
+    const size_t at = static_cast<size_t>(fresh.pos[seq]) * (D / 2) + d0 % (D / 2);
+    load8(fresh.cos_t + at, cs);
+    load8(fresh.sin_t + at, sn);
+  };
+  const auto turn = [&](float (&v)[8], const float (&cs)[8], const float (&sn)[8], bool round) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float o = __shfl_xor(v[j], LPT / 2, 64);
+      v[j] = d0 < D / 2 ? fmaf(v[j], cs[j], -(o * sn[j])) : fmaf(v[j], cs[j], o * sn[j]);
+      if (round) v[j] = to_f32(from_f32<T>(v[j]));
+    }
+  };
+  float cs[8], sn[8];
+  if constexpr (NEW) tables(cs, sn);
+  uint4 qv[G];
 #pragma unroll
   for (int h = 0; h < G; ++h) {
-    load8(q + (static_cast<size_t>(seq) * qldh + kvh * G + h) * D + d0, qv[h]);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) qv[h][j] *= scale;
+    const T* row = q + (static_cast<size_t>(seq) * qldh + kvh * G + h) * D + d0;
+    qv[h] = *reinterpret_cast<const uint4*>(row);
+    if constexpr (NEW) {
+      float f[8];
+      cvt8kv<T, T>(qv[h], f);
+      turn(f, cs, sn, true);
+      store8(reinterpret_cast<T*>(&qv[h]), f);
+    }
   }
+  const auto score = [&](int h, const uint4& k) __attribute__((always_inline)) {
+    const float s = pa_dot8<T>(k, qv[h]);
+    return (LPT == 16 ? pa_red16(s) : wave_sum_width<LPT>(s)) * scale;
+  };
   const int* bt = block_tables + static_cast<size_t>(seq) * max_blocks;
   const size_t head_off = static_cast<size_t>(kvh) * BS * D;
   const size_t blk_stride = static_cast<size_t>(nkv) * BS * D;
@@ -390,31 +462,50 @@ __global__ void __launch_bounds__(256) pa_decode1_kernel(
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[h][j] = 0.f;
   }
-  // one iteration's online-softmax update from its raw K / V pieces (rows t0 + u * NGR)
-  const auto consume = [&](int t0, const Raw (&kraw)[U], const Raw (&vraw)[U]) {
+  // Online-softmax update from the raw K / V pieces of rows t0 + u * NGR, four at a time: their scores of a head
+  // meet its state together, one maximum and one rescaling for all.  Rows past the end count as -inf, and their
+  // values (another sequence's, or none's) as zero.  (Row by row, with fp32 products and a rescaling each, groups
+  // of query heads were bound by the vector units: 256 sequences x 8 heads of 4 queries 95 -> 86 us.)
+  constexpr int R = 4;
+  const auto consume4 = [&](int t0, const Raw* kraw, const Raw* vraw) __attribute__((always_inline)) {
+    float p[G][R];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int t = t0 + u * NGR;
-      float kr[8], vr[8];
-      cvt8kv<T, KT>(kraw[u], kr);
-      cvt8kv<T, KT>(vraw[u], vr);
+    for (int u = 0; u < R; ++u) {
+      const uint4 k = pa_row16<T, KT>(kraw[u]);
 #pragma unroll
       for (int h = 0; h < G; ++h) {
-        float s = 0.f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) s += kr[j] * qv[h][j];
-        s = LPT == 16 ? pa_red16(s) : wave_sum_width<LPT>(s);
-        if (t < end) {  // uniform within the row group
-          const float mn = fmaxf(m[h], s);
-          const float al = __expf(m[h] - mn);  // m = -inf on the first row: al = 0
-          const float p = __expf(s - mn);
-          l[h] = l[h] * al + p;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) acc[h][j] = acc[h][j] * al + p * vr[j];
-          m[h] = mn;
-        }
+        const float s = score(h, k);
+        p[h][u] = t0 + u * NGR < end ? s : -INFINITY;
       }
     }
+#pragma unroll
+    for (int h = 0; h < G; ++h) {
+      const float mx = fmaxf(fmaxf(fmaxf(p[h][0], p[h][1]), fmaxf(p[h][2], p[h][3])), m[h]);
+      const float mb = mx == -INFINITY ? 0.f : mx;   // (a group without a row yet)
+      const float al = __expf(m[h] - mb);
+      m[h] = mx;
+#pragma unroll
+      for (int u = 0; u < R; ++u) p[h][u] = __expf(p[h][u] - mb);
+      l[h] = l[h] * al + ((p[h][0] + p[h][1]) + (p[h][2] + p[h][3]));
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[h][j] *= al;
+    }
+    const bool whole = t0 - grp + R * NGR <= end;
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      Raw r = vraw[u];
+      if (!whole && t0 + u * NGR >= end) r = Raw{};
+      float vr[8];
+      cvt8kv<T, KT>(r, vr);
+#pragma unroll
+      for (int h = 0; h < G; ++h)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[h][j] = fmaf(p[h][u], vr[j], acc[h][j]);
+    }
+  };
+  const auto consume = [&](int t0, const Raw (&kraw)[U], const Raw (&vraw)[U]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < U; c += R) consume4(t0 + c * NGR, kraw + c, vraw + c);
   };
   int nbid[U];
   if constexpr (UNI) {
@@ -453,12 +544,12 @@ __global__ void __launch_bounds__(256) pa_decode1_kernel(
     // q must land before the first asm load issues: a later compiler-inserted wait for it
     // would be vmcnt(0) and drain the prefetched set too
 #pragma unroll
-    for (int h = 0; h < G; ++h)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(qv[h][j]));
+    for (int h = 0; h < G; ++h) asm volatile("" : "+v"(qv[h].x), "+v"(qv[h].y), "+v"(qv[h].z), "+v"(qv[h].w));
     Raw kA[U], vA[U], kB[U], vB[U];
-    issue(nbid, kA, vA);
-    ids(start + step, nbid);
+    if (start < end) {               // (NEW: a partition of the new token alone has no rows to ask for)
+      issue(nbid, kA, vA);
+      ids(start + step, nbid);
+    }
     for (int base = start; base < end; base += 2 * step) {
       const int b1 = base + step;
       const bool more1 = b1 < end;
@@ -506,6 +597,38 @@ __global__ void __launch_bounds__(256) pa_decode1_kernel(
       }
     }
     consume(t0, kraw, vraw);
+  }
+  if constexpr (NEW) {
+    if (ctx - 1 < start + PART && wid == 0) {      // this partition ends the context
+      float kf[8], vf[8];
+      const T* row = q + (static_cast<size_t>(seq) * qldh + nh + kvh) * D + d0;
+      load8(row, kf);
+      load8(row + static_cast<size_t>(nkv) * D, vf);
+      tables(cs, sn);      // (loaded again: registers held over the walk would cost it waves)
+      turn(kf, cs, sn, !F8);
+      Raw rk, rv;                                  // as the cache holds them
+      store8kv<T, KT>(reinterpret_cast<KT*>(&rk), kf);
+      store8kv<T, KT>(reinterpret_cast<KT*>(&rv), vf);
+      cvt8kv<T, KT>(rv, vf);
+      const long long slot = fresh.slots[seq];
+      if (slot >= 0 && grp == 0) {
+        const size_t dst = ((static_cast<size_t>(slot / BS) * nkv + kvh) * BS + slot % BS) * D + d0;
+        *reinterpret_cast<Raw*>(static_cast<KT*>(fresh.kc) + dst) = rk;
+        *reinterpret_cast<Raw*>(static_cast<KT*>(fresh.vc) + dst) = rv;
+      }
+#pragma unroll
+      for (int h = 0; h < G; ++h) {
+        const float s = score(h, pa_row16<T, KT>(rk));
+        if (grp == 0) {
+          const float mn = fmaxf(m[h], s), mb = mn == -INFINITY ? 0.f : mn;
+          const float al = __expf(m[h] - mb), p = __expf(s - mb);
+          l[h] = l[h] * al + p;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) acc[h][j] = acc[h][j] * al + p * vf[j];
+          m[h] = mn;
+        }
+      }
+    }
   }
   // merge the 64 / LPT row groups of each wave (lanes d0-aligned at xor 16, 32, ...)
 #pragma unroll
@@ -697,18 +820,29 @@ template <typename T, int D, int G, typename KT>
 static void launch_pa_uni(bool pf, dim3 grid, hipStream_t st, void* out, const void* q,
                           const void* kc, const void* vc, const int* bt, const int* cl, int nh,
                           int qldh, int nkv, int BS, int max_blocks, int max_parts, float scale,
-                          float* tm, float* tl, void* to, int PART) {
+                          float* tm, float* tl, void* to, int PART, const PaNew& fresh) {
+  const bool is_new = fresh.pos != nullptr;
   if constexpr (pa_pf_ok<D, G>()) {
     if (pf) {
+      if (is_new)
+        hipLaunchKernelGGL((pa_decode1_kernel<T, D, G, KT, true, true, true>), grid, dim3(256), 0, st,
+                           (T*)out, (const T*)q, (const KT*)kc, (const KT*)vc, bt, cl, nh, qldh, nkv,
+                           BS, max_blocks, max_parts, scale, tm, tl, (float*)to, PART, fresh);
+      else
       hipLaunchKernelGGL((pa_decode1_kernel<T, D, G, KT, true, true>), grid, dim3(256), 0, st,
                          (T*)out, (const T*)q, (const KT*)kc, (const KT*)vc, bt, cl, nh, qldh, nkv,
-                         BS, max_blocks, max_parts, scale, tm, tl, (float*)to, PART);
+                         BS, max_blocks, max_parts, scale, tm, tl, (float*)to, PART, fresh);
       return;
     }
   }
-  hipLaunchKernelGGL((pa_decode1_kernel<T, D, G, KT, true>), grid, dim3(256), 0, st, (T*)out,
-                     (const T*)q, (const KT*)kc, (const KT*)vc, bt, cl, nh, qldh, nkv, BS,
-                     max_blocks, max_parts, scale, tm, tl, (float*)to, PART);
+  if (is_new)
+    hipLaunchKernelGGL((pa_decode1_kernel<T, D, G, KT, true, false, true>), grid, dim3(256), 0, st, (T*)out,
+                       (const T*)q, (const KT*)kc, (const KT*)vc, bt, cl, nh, qldh, nkv, BS,
+                       max_blocks, max_parts, scale, tm, tl, (float*)to, PART, fresh);
+  else
+    hipLaunchKernelGGL((pa_decode1_kernel<T, D, G, KT, true>), grid, dim3(256), 0, st, (T*)out,
+                       (const T*)q, (const KT*)kc, (const KT*)vc, bt, cl, nh, qldh, nkv, BS,
+                       max_blocks, max_parts, scale, tm, tl, (float*)to, PART, fresh);
 }
 
 template <typename T, int D>
@@ -716,25 +850,26 @@ static void launch_pa_g(int G, dim3 grid, size_t smem, hipStream_t st, void* out
                         const void* kc, const void* vc, const int* bt, const int* cl, int nh,
                         int qldh, int nkv, int BS, int max_blocks, int max_parts, float scale,
                         float* tm,
-                        float* tl, void* to, int PART, unsigned* cnt, int one_pass, bool fp8kv) {
+                        float* tl, void* to, int PART, unsigned* cnt, int one_pass, bool fp8kv,
+                        const PaNew& fresh) {
   // one_pass 2: the uniform-block-id variant where the block size equals the rows per step
   const bool uni = one_pass >= 2 && BS == 256 / (D / 8) && PART % BS == 0;
   const bool pf = uni && one_pass == 3;
 #define LUMEN_PA_G(GG)                                                                         \
   if (fp8kv && uni)                                                                             \
     launch_pa_uni<T, D, GG, fp8>(pf, grid, st, out, q, kc, vc, bt, cl, nh, qldh, nkv, BS,        \
-                                 max_blocks, max_parts, scale, tm, tl, to, PART);                \
+                                 max_blocks, max_parts, scale, tm, tl, to, PART, fresh);         \
   else if (fp8kv)                                                                               \
     hipLaunchKernelGGL((pa_decode1_kernel<T, D, GG, fp8>), grid, dim3(256), 0, st, (T*)out,     \
                        (const T*)q, (const fp8*)kc, (const fp8*)vc, bt, cl, nh, qldh, nkv, BS,        \
-                       max_blocks, max_parts, scale, tm, tl, (float*)to, PART);                 \
+                       max_blocks, max_parts, scale, tm, tl, (float*)to, PART, fresh);          \
   else if (uni)                                                                                 \
     launch_pa_uni<T, D, GG, T>(pf, grid, st, out, q, kc, vc, bt, cl, nh, qldh, nkv, BS,          \
-                               max_blocks, max_parts, scale, tm, tl, to, PART);                  \
+                               max_blocks, max_parts, scale, tm, tl, to, PART, fresh);           \
   else if (one_pass)                                                                            \
     hipLaunchKernelGGL((pa_decode1_kernel<T, D, GG>), grid, dim3(256), 0, st, (T*)out,          \
                        (const T*)q, (const T*)kc, (const T*)vc, bt, cl, nh, qldh, nkv, BS, max_blocks, \
-                       max_parts, scale, tm, tl, (float*)to, PART);                             \
+                       max_parts, scale, tm, tl, (float*)to, PART, fresh);                      \
   else                                                                                          \
     hipLaunchKernelGGL((pa_decode_kernel<T, D, GG>), grid, dim3(256), smem, st, (T*)out,       \
                        (const T*)q, (const T*)kc, (const T*)vc, bt, cl, nh, qldh, nkv, BS, max_blocks, \
@@ -751,16 +886,23 @@ static hipError_t launch_pa(void* out, const void* q, const void* kc, const void
                             const int* bt, const int* cl, int nseq, int nh, int nkv, int D, int BS,
                             int max_blocks, int max_parts, float scale, float* tm, float* tl,
                             void* to, int PART, unsigned* cnt, int one_pass, int fp8kv,
-                            int qldh, hipStream_t st) {
+                            int qldh, PaNew fresh, hipStream_t st) {
   const int G = nh / nkv;
+  const bool uni = one_pass >= 2 && BS == 256 / (D / 8) && PART % BS == 0;
+  if (fresh.pos != nullptr && !uni) return hipErrorInvalidValue;
+  // Which workgroups run together: those of all kv heads of a few sequences, whose rows of a block follow each other in
+  // memory, once there are workgroups for it (us, bf16 unless said, one head of all sequences -> all heads of a few: 256
+  // sequences of 72 - 578, 32 heads 242 -> 233, 8 of 4 queries 81 -> 77, 32 in fp8 142 -> 126; 64 of 128 - 1025 x 32 119 ->
+  // 106); below, sequences first spread better over the XCDs (32 x 8 15.3 and 16.0, 8 x 4 10.1 and 11.5)
+  fresh.swap = uni && nseq < 65536 && static_cast<long long>(nseq) * nkv >= 512;
   if (fp8kv && one_pass == 0) one_pass = 1;  // the fp8 cache: single-pass kernels only
   if (G != 1 && G != 2 && G != 4 && G != 8) return hipErrorInvalidValue;
-  dim3 grid(nseq, nkv, max_parts);
+  const dim3 grid = fresh.swap ? dim3(nkv, nseq, max_parts) : dim3(nseq, nkv, max_parts);
   const size_t smem = (static_cast<size_t>(G) * PART + 4 * G * D + 2 * G + 8) * sizeof(float);
-  if (D == 128) launch_pa_g<T, 128>(G, grid, smem, st, out, q, kc, vc, bt, cl, nh, qldh, nkv, BS, max_blocks, max_parts, scale, tm, tl, to, PART, cnt, one_pass, fp8kv != 0);
-  else if (D == 64) launch_pa_g<T, 64>(G, grid, smem, st, out, q, kc, vc, bt, cl, nh, qldh, nkv, BS, max_blocks, max_parts, scale, tm, tl, to, PART, cnt, one_pass, fp8kv != 0);
-  else if (D == 256) launch_pa_g<T, 256>(G, grid, smem, st, out, q, kc, vc, bt, cl, nh, qldh, nkv, BS, max_blocks, max_parts, scale, tm, tl, to, PART, cnt, one_pass, fp8kv != 0);
-  else if (D == 32) launch_pa_g<T, 32>(G, grid, smem, st, out, q, kc, vc, bt, cl, nh, qldh, nkv, BS, max_blocks, max_parts, scale, tm, tl, to, PART, cnt, one_pass, fp8kv != 0);
+  if (D == 128) launch_pa_g<T, 128>(G, grid, smem, st, out, q, kc, vc, bt, cl, nh, qldh, nkv, BS, max_blocks, max_parts, scale, tm, tl, to, PART, cnt, one_pass, fp8kv != 0, fresh);
+  else if (D == 64) launch_pa_g<T, 64>(G, grid, smem, st, out, q, kc, vc, bt, cl, nh, qldh, nkv, BS, max_blocks, max_parts, scale, tm, tl, to, PART, cnt, one_pass, fp8kv != 0, fresh);
+  else if (D == 256) launch_pa_g<T, 256>(G, grid, smem, st, out, q, kc, vc, bt, cl, nh, qldh, nkv, BS, max_blocks, max_parts, scale, tm, tl, to, PART, cnt, one_pass, fp8kv != 0, fresh);
+  else if (D == 32) launch_pa_g<T, 32>(G, grid, smem, st, out, q, kc, vc, bt, cl, nh, qldh, nkv, BS, max_blocks, max_parts, scale, tm, tl, to, PART, cnt, one_pass, fp8kv != 0, fresh);
   else return hipErrorInvalidValue;
   if (max_parts > 1 && (cnt == nullptr || one_pass)) {  // unfused merge: second kernel
     dim3 g2(nseq, nh), b2(128);
@@ -780,22 +922,27 @@ extern "C" hipError_t lumen_paged_attention_decode(int dtype, void* out, const v
                                                    int max_parts, float scale, float* tmp_m,
                                                    float* tmp_l, void* tmp_o, int PART,
                                                    unsigned* counters, int one_pass,
-                                                   int fp8kv, int qldh, hipStream_t st) {
-  // counters: nullptr = merge split contexts in a second kernel; else >= nseq * nkv zeroed
+                                                   int fp8kv, int qldh, const int* pos,
+                                                   const float* cos_t, const float* sin_t,
+                                                   const long long* slots, hipStream_t st) {
+  // pos (or null): the last token of every context is the step's own, see the kernel's NEW form; q is then
+  // the fused q|k|v rows and the caches are written.  counters: nullptr = merge split contexts in a second kernel; else >= nseq * nkv zeroed
   // arrival counters (left zeroed again) and the last partition to finish merges in place.
   if (nseq == 0) return hipSuccess;
   // qldh: q row stride in heads (nh for a contiguous [nseq, nh, D] q; the fused qkv row's
   // head count when q is read in place from it)
-  if (nh % nkv != 0 || nh / nkv > lumen::kMaxGroup || PART <= 0 || qldh < nh)
+  if (nh % nkv != 0 || nh / nkv > lumen::kMaxGroup || PART <= 0 || qldh < nh ||
+      (pos != nullptr && (qldh < nh + 2 * nkv || !cos_t || !sin_t || !slots)))
     return hipErrorInvalidValue;
+  const lumen::PaNew fresh{pos, cos_t, sin_t, const_cast<void*>(kc), const_cast<void*>(vc), slots, 0};
   if (dtype == lumen::kBF16)
     return lumen::launch_pa<lumen::bf16>(out, q, kc, vc, block_tables, context_lens, nseq, nh,
                                          nkv, D, BS, max_blocks, max_parts, scale, tmp_m, tmp_l,
-                                         tmp_o, PART, counters, one_pass, fp8kv, qldh, st);
+                                         tmp_o, PART, counters, one_pass, fp8kv, qldh, fresh, st);
   if (dtype == lumen::kF16)
     return lumen::launch_pa<lumen::fp16>(out, q, kc, vc, block_tables, context_lens, nseq, nh,
                                          nkv, D, BS, max_blocks, max_parts, scale, tmp_m, tmp_l,
-                                         tmp_o, PART, counters, one_pass, fp8kv, qldh, st);
+                                         tmp_o, PART, counters, one_pass, fp8kv, qldh, fresh, st);
   return hipErrorInvalidValue;
 }
 

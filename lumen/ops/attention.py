@@ -76,28 +76,56 @@ def paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     num_seqs, nh, D = q.shape
     nb, nkv, bs, _ = k_cache.shape
     if use_native(q):
-        max_parts = max(1, math.ceil(max_context / partition_size))
-        out = torch.empty(num_seqs, nh, D, device=q.device, dtype=q.dtype)
-        if max_parts > 1:
-            tm = torch.empty(num_seqs, nh, max_parts, device=q.device, dtype=torch.float32)
-            tl = torch.empty_like(tm)
-            to = torch.empty(num_seqs, nh, max_parts, D, device=q.device, dtype=torch.float32)
-        else:
-            tm = torch.empty(1, 1, 1, device=q.device, dtype=torch.float32)
-            tl, to = tm, tm
         one = PA_ONE_PASS if one_pass is None else int(one_pass)
-        fused = bool(fused_merge) and not one
-        cnt = (_pa_counters(q.device, num_seqs * nkv) if fused and max_parts > 1
-               else None)
+        fused = bool(fused_merge) and not one and max_context > partition_size
+        cnt = _pa_counters(q.device, num_seqs * nkv) if fused else None
         # q read in place when its heads are contiguous (a view into the fused qkv rows):
         # no per-layer copy of the decode rows' q
         qk = q if (q.stride(2) == 1 and q.stride(1) == D and q.stride(0) % D == 0
                    and q.data_ptr() % 16 == 0) else q.contiguous()
-        native().paged_attention_decode(out, qk, k_cache, v_cache, block_tables,
-                                        context_lens, nkv, bs, block_tables.shape[1], scale, tm,
-                                        tl, to, partition_size, cnt, one)
-        return out
+        return _paged_native(qk, k_cache, v_cache, block_tables, context_lens, max_context, scale,
+                             partition_size, cnt, one)
     return paged_decode_ref(q, k_cache, v_cache, block_tables, context_lens, scale)
+
+
+def _paged_native(q, k_cache, v_cache, block_tables, context_lens, max_context, scale, partition_size, cnt, one,
+                  new=()) -> torch.Tensor:
+    num_seqs, nh, D = q.shape
+    nkv, bs = k_cache.shape[1], k_cache.shape[2]
+    max_parts = max(1, math.ceil(max_context / partition_size))
+    out = torch.empty(num_seqs, nh, D, device=q.device, dtype=q.dtype)
+    if max_parts > 1:
+        tm = torch.empty(num_seqs, nh, max_parts, device=q.device, dtype=torch.float32)
+        tl = torch.empty_like(tm)
+        to = torch.empty(num_seqs, nh, max_parts, D, device=q.device, dtype=torch.float32)
+    else:
+        tm = torch.empty(1, 1, 1, device=q.device, dtype=torch.float32)
+        tl, to = tm, tm
+    native().paged_attention_decode(out, q, k_cache, v_cache, block_tables, context_lens, nkv, bs,
+                                    block_tables.shape[1], scale, tm, tl, to, partition_size, cnt, one, *new)
+    return out
+
+
+def paged_decode_new_ok(qkv: torch.Tensor, k_cache: torch.Tensor, nh: int, partition_size: int) -> bool:
+    """Can ``paged_decode_new`` run: the kernels whose workgroups step over whole cache blocks, 16-bit rows."""
+    _, nkv, bs, D = k_cache.shape
+    return (PA_ONE_PASS >= 2 and use_native(qkv) and D in (32, 64, 128, 256) and bs == 2048 // D
+            and partition_size % bs == 0 and qkv.dim() == 2 and qkv.shape[1] >= (nh + 2 * nkv) * D
+            and qkv.stride(1) == 1 and qkv.stride(0) % D == 0
+            and qkv.data_ptr() % 16 == 0 and k_cache.is_contiguous())
+
+
+def paged_decode_new(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, positions: torch.Tensor,
+                     cos_t: torch.Tensor, sin_t: torch.Tensor, slots: torch.Tensor, block_tables: torch.Tensor,
+                     context_lens: torch.Tensor, max_context: int, nh: int, scale: float,
+                     partition_size: int = 512) -> torch.Tensor:
+    """``rope_write_kv`` and ``paged_decode`` of a pure decode step in one launch: row i of the fused ``qkv`` is the
+    token at cache row ``context_lens[i] - 1`` of its sequence.  q and k are turned on the way (``qkv`` is left as it
+    is), k and v written to ``slots`` (< 0: not).  For calls that ``paged_decode_new_ok`` has let pass."""
+    nkv, D = k_cache.shape[1], k_cache.shape[3]
+    q = qkv.as_strided((qkv.shape[0], nh, D), (qkv.stride(0), D, 1))
+    return _paged_native(q, k_cache, v_cache, block_tables, context_lens, max_context, scale, partition_size,
+                         None, PA_ONE_PASS, (positions.to(torch.int32), cos_t, sin_t, slots.to(torch.int64)))
 
 
 def paged_decode_ref(q, k_cache, v_cache, block_tables, context_lens, scale):

@@ -33,6 +33,7 @@ from ..ops._native import native, use_native
 from ..ops.activation import swiglu
 from ..ops.embedding import embedding
 from ..ops.attention import (flash_attention_fresh, flash_attention_paged, paged_decode,
+                             paged_decode_new, paged_decode_new_ok,
                              rope_write_kv)
 from ..ops.gemm import linear_nt, row_norm_linear, row_norm_ok, swiglu_linear_nt
 from ..ops.moe import THIN_ACT_MAX_M, thin_act, thin_act_ok
@@ -240,7 +241,12 @@ class ModelRunner:
                 dist.all_reduce(x, group=self.tp_group)
         return x
 
-    def _layers(self, h, positions, slots, attn_fn, lora_ids=None, mark=None):
+    def _rotate_write(self, qkv, positions, slots, i):
+        rope_write_kv(qkv, positions, self.w.nh, self.w.nkv, self.cfg.head_dim, self.cos, self.sin,
+                      self.k_cache[i], self.v_cache[i], slots)
+
+    def _layers(self, h, positions, slots, attn_fn, lora_ids=None, mark=None, rotate=True):
+        # rotate: turn q and k and write k and v before attn_fn (False: attn_fn does)
         cfg = self.cfg
         res = None
         T = h.shape[0]
@@ -257,8 +263,8 @@ class ModelRunner:
                 mark.record()   # split decode: the second half starts here
             if ml is not None:
                 ml.apply(i, "qkv", y, qkv, masks)
-            rope_write_kv(qkv, positions, self.w.nh, self.w.nkv, D, self.cos, self.sin,
-                          self.k_cache[i], self.v_cache[i], slots)
+            if rotate:
+                self._rotate_write(qkv, positions, slots, i)
             o = attn_fn(qkv, i)
             a = self._allreduce(linear_nt(o, L.o))
             if ml is not None:
@@ -412,12 +418,18 @@ class ModelRunner:
         N = tokens.shape[0]
         nh, D = self.w.nh, self.cfg.head_dim
 
-        def attn(qkv, i):
-            q = qkv[:, :self.q_size].reshape(N, nh, D)
-            return paged_decode(q, self.k_cache[i], self.v_cache[i], block_tables, context_lens,
-                                max_context, self.scale, self.decode_partition(N)).view(N, nh * D)
+        part = self.decode_partition(N)
 
-        h, res = self._layers(h, positions, slots, attn, lora_ids, mark=mark)
+        def attn(qkv, i):
+            k, v = self.k_cache[i], self.v_cache[i]
+            if paged_decode_new_ok(qkv, k, nh, part):
+                return paged_decode_new(qkv, k, v, positions, self.cos, self.sin, slots, block_tables, context_lens,
+                                        max_context, nh, self.scale, part).view(N, nh * D)
+            self._rotate_write(qkv, positions, slots, i)
+            q = qkv[:, :self.q_size].reshape(N, nh, D)
+            return paged_decode(q, k, v, block_tables, context_lens, max_context, self.scale, part).view(N, nh * D)
+
+        h, res = self._layers(h, positions, slots, attn, lora_ids, mark=mark, rotate=False)
         if N == 1 and row_norm_ok(h, self.w.norm, res, self.w.lm_head):
             logits, _ = row_norm_linear(h, self.w.norm, self.cfg.rms_norm_eps, res, self.w.lm_head)
         else:

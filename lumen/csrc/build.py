@@ -40,7 +40,7 @@ def ext_path() -> str:
 # values to and fro (moves in the assembly, default -> with the option: lora_v3 5080 -> 590,
 # head_scan_chunk16 7675 -> 1938).  Where it measured faster: the LoRA gradients of 8 x 512 tokens, width
 # 4096, dy3 40.7 -> 33.8 us and dxa3 46.6 -> 35.8; the 16-token scans of one 512-token prompt 59.0 -> 54.8 us; recurrent_chunk
-# 318 -> 293 (delta, 8 x 512 tokens).
+# 318 -> 293 (delta, 8 x 512 tokens, of its four-wave form).
 # The others are equal or slower (row_attention.hip's latent_attn_kernel 24.6 -> 32.1 us).
 MFMA_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 MFMA_FORM_FILES = ("lora_v3.hip", "head_scan_chunk16.hip", "recurrent_chunk.hip", "split_gemm.hip",

@@ -19,13 +19,21 @@
 // operands are staged there once for the four waves and read 16 bytes at a time.  All products are
 // fp32 matrix instructions; decays are fp32, their products fp64.
 // The read-outs leave in fp32; the per-head norm and gate follow in gated_rms (rms_group.hip).
-// Measured (8 portions of 512 tokens, width 2048, bf16; the norm kernel's 17 us included): delta, 16 heads
-// of 128: 1000 -> 310 us; wkv, 32 heads of 64: 460 -> 119 us.  A chunk is now a chain of three barriers
-// -- decays and sums, scaled rows, products -- with one wave per SIMD at this size.
+//
+// A chunk's decays and sums, its scaled rows and its small matrices do not need the state: producer waves build the
+// next chunk's (three stages, a barrier after each, the rows after it in flight) while the column waves run the one
+// before, in two LDS buffers.  With all of it done by the same four waves, one after the other, a step was 21 thousand
+// cycles (delta, heads of 128: exponentials and divisions 5.8, scaled rows 3.3, the matrices and the 16-row
+// substitution 4.9, the state's products 7); it is 16 now, bound by what
+// the three waves of a SIMD issue: matrix instructions 5.6 of it.
+// Measured (width 2048, bf16, the norm kernel's 17 us included), four waves -> this, us: delta, 16 heads of 128: 8
+// portions of 512 tokens 305 -> 245, one of 512 281 -> 216, 32 of 128 311 -> 252; 8 heads of 256 512 -> 452; 64 of 32 185
+// -> 173; wkv, 32 heads of 64: 137 -> 124, 117 -> 97, 106 -> 100; 8 heads of 256 338 -> 280.  (Token by token: 1000 and 460.)
 // Error against float64 (512 tokens, heads of 32 - 256): the read-outs are as far off as the serial walk's
-// (1.66e-3, the bf16 result's rounding), the state a little less (delta 0.86e-7, serial 0.88e-7; wkv 0.60e-7,
-// serial 0.62e-7).  That takes the decays' products in float64 (in fp32: + 0.1e-7) and care with the sums
+// (1.66e-3, the bf16 result's rounding), the state a little less (delta 0.86e-7, serial 0.90e-7; wkv 0.62e-7,
+// serial 0.65e-7).  That takes the decays' products in float64 (in fp32: + 0.1e-7) and care with the sums
 // (see the state's update; term by term 1.4e-7 and 0.9e-7), which cost 20 us of the delta scan.
+// (Both products of an update in one accumulator: 0.94e-7.)
 //
 // Range: P_t and 1 / P_16 must stay finite, and so must the masked entries' factors.  A wkv chunk ends
 // before the token that would take some channel's P below 2^-100, so a decay beyond that (0 too) is alone in
@@ -33,8 +41,8 @@
 // stay above 2^-70.  r and k that scaled rows could not hold as normal numbers (kLarge, kTiny*), infinities and
 // NaN run one token at a time, so that earlier tokens stay as they are; wkv values below kSmall make the
 // chunk end at 2^-40.  A chunk of one token costs what one of sixteen does: decays up to e^-50 a token (wkv,
-// 8 x 512 tokens, 32 heads of 64, log decays -e^N(1, 1) at the fast end) take 770 us, the
-// serial walk 460.
+// 8 x 512 tokens, 32 heads of 64, log decays -e^N(1, 1) at the fast end) took 770 us with the four-wave form, the
+// serial walk 460; decays a token of -e^N(0..2, 0.6) 492 with the four-wave form, 460 here.
 #include "seqmix.h"
 
 using namespace lumen;
@@ -49,10 +57,8 @@ __device__ __forceinline__ f32x4 mma(float a, float b, f32x4 c) {
 
 constexpr int kC = 16;                 // tokens per chunk
 constexpr int LP = 20;                 // row stride of the chunk matrices in LDS
-constexpr float kMinP = 0x1p-100f;     // smallest product of a chunk's decays, and a group's share of it
-template <int NG> constexpr float kGroupP() {
-  return NG == 1 ? 0x1p-100f : NG == 2 ? 0x1p-50f : NG == 4 ? 0x1p-25f : 0x1p-12f;
-}
+constexpr int kCol = 4;                 // column waves of a workgroup
+constexpr float kMinP = 0x1p-100f;     // smallest product of a chunk's decays
 
 // |x| as bits, whose order is that of the values (infinities and NaN last)
 __device__ __forceinline__ unsigned mag(float x) { return __builtin_bit_cast(unsigned, x) & 0x7fffffffu; }
@@ -75,6 +81,26 @@ template <typename T> struct ScanArgs {
   float decay_scale, key_eps;
 };
 
+// e^x for x up to 88 (more: as 88; below -200: 0) from the hardware's 2^t, the rounding of t made good; and 1 / (1 +
+// e^-x) with one refinement of the hardware's reciprocal.  As near as expf and an exact division (state's error against
+// float64 unchanged), at a third of their instructions, which bounded the producers (5.8 -> 4.8 thousand cycles a chunk).
+__device__ __forceinline__ float exp_near(float x) {
+  constexpr float kL = 1.44269502f, kLlo = 1.92596299e-8f;     // log2(e) = kL + kLlo
+  x = x < -200.f ? -200.f : x > 88.f ? 88.f : x;               // (NaN stays)
+  const float t = x * kL, lo = fmaf(x, kLlo, fmaf(x, kL, -t));
+  const float r = __builtin_amdgcn_exp2f(t);
+  return fmaf(r, lo * 0.693147182f, r);
+}
+__device__ __forceinline__ float sigmoid_near(float x) {
+  const float d = 1.f + exp_near(-x), r = __builtin_amdgcn_rcpf(d);
+  return fmaf(fmaf(-d, r, 1.f), r, r);
+}
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <int CTRL> __device__ __forceinline__ float dpp(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL,
                                                                0xF, 0xF, false));
@@ -89,50 +115,35 @@ __device__ __forceinline__ float sum16(float v) {        // over the 16 lanes of
   return v + dpp<0x140>(v);
 }
 
-// KB: key channels in blocks of 16
-template <typename T, int KB, bool DELTA>
-__global__ void __launch_bounds__(256)
+// KB: key channels in blocks of 16; kProd: producer waves
+template <typename T, int KB, bool DELTA, int kProd>
+__global__ void __launch_bounds__(64 * (kCol + kProd))
 scan_chunk_kernel(const ScanArgs<T> a) {
   constexpr int DKP = 16 * KB, LK = DKP + 4;
-  constexpr int NG = 256 / DKP, TG = kC / NG;            // staging: token groups, tokens of each
+  constexpr int NG = 64 * kProd / DKP, TG = kC / NG;     // staging: token groups, tokens of each
   constexpr int NM = DELTA ? 4 : 1;
-  __shared__ __attribute__((aligned(16))) float s_r[kC * LK], s_k[kC * LK];
-  __shared__ __attribute__((aligned(16))) float s_u[DELTA ? kC * LK : 4], s_b[DELTA ? kC * LK : 4];
-  __shared__ __attribute__((aligned(16))) float s_m[NM][kC * LP];
-  __shared__ __attribute__((aligned(16))) float s_P[DKP], s_iP[DKP], s_red[kC][KB];
+  static_assert(NG * TG == kC && NM <= kProd, "staging");
+  struct Buf {                                           // a chunk as the column waves read it
+    float r[kC * LK], k[kC * LK], u[DELTA ? kC * LK : 4], b[DELTA ? kC * LK : 4];
+    float m[NM][kC * LP], P[DKP];
+  };
+  __shared__ __attribute__((aligned(16))) Buf s_buf[2];
+  __shared__ __attribute__((aligned(16))) float s_iP[DKP], s_red[kC][KB];
   __shared__ double s_gp[NG][DKP];
   __shared__ float s_tok[kC];
   __shared__ int s_n[2], s_low[2], s_small[2];
   const int sg = blockIdx.x, hd = blockIdx.y;
   const int r0 = a.cu[sg], len = a.cu[sg + 1] - r0;
   if (len <= 0) return;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lr = lane & 15, lg = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool col = w < kCol;                                     // else: a producer
   const int D = a.D, col0 = hd * D;
-  const int j = (blockIdx.z * 4 + w) * 16 + lr;                  // this lane's value column
-  const bool on = j < D;
-  const int ch = tid % DKP, tg = tid / DKP;                      // staging: channel, token group
-  const bool chan = ch < D;
-  const float w0 = chan ? a.w0[col0 + ch] : 0.f, ub = chan ? a.ub[col0 + ch] : 0.f;
-
-  f32x4 S[KB];
-  float* st = a.state + ((long long)a.slot[sg] * a.H + hd) * D * D + j;
-  const bool fresh = a.start[sg] == 0;
-#pragma unroll
-  for (int b = 0; b < KB; ++b)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int i = 16 * b + 4 * lg + e;
-      S[b][e] = (!fresh && on && i < D) ? st[(long long)i * D] : 0.f;
-    }
-
-  // the chunk at t0, as loaded: this thread's channel of its tokens, this lane's values (4 lg + e).  Rows
-  // past the portion repeat its last one, channels past D the last one: blanked where they are used.
-  T pr[TG], pk[TG], pw[TG], pa[TG], pv[4];
-  const int chc = min(ch, D - 1), jc = min(j, D - 1);
-  // the token of a lane's e-th value: an inner index of every product with V
-  const auto tok_of = [&](int e) { return DELTA ? 4 * lg + e : 4 * e + lg; };
+  const int j = (blockIdx.z * kCol + w) * 16 + lr;               // a column wave's lane: its value column
+  const bool on = col && j < D;
   // row t + i of `base`'s chunk at t0, column c (uniform base, 32-bit byte offset from the chunk's first row,
-  // so the rows that are left count up to a chunk's; i known when compiled)
+  // so the rows that are left count up to a chunk's; i known when compiled).  Rows past the portion repeat its
+  // last one, channels past D the last one: blanked where they are used.
   const auto get = [&](const T* base, long long ld, int t0, int t, int i, int c)
                        __attribute__((always_inline)) {
     const unsigned step = (unsigned)ld, last = (unsigned)min(len - 1 - t0, kC - 1) * step;
@@ -140,6 +151,15 @@ scan_chunk_kernel(const ScanArgs<T> a) {
     return *reinterpret_cast<const T*>(
         reinterpret_cast<const char*>(base + (long long)(r0 + t0) * ld + col0) + at * (unsigned)sizeof(T));
   };
+
+  // ---------------- the producers ----------------
+  const int ptid = col ? 0 : tid - 64 * kCol;
+  const int ch = ptid % DKP, tg = ptid / DKP;                    // channel, token group
+  const bool chan = ch < D;
+  const int chc = min(ch, D - 1);
+  const float w0 = chan ? a.w0[col0 + ch] : 0.f, ub = chan ? a.ub[col0 + ch] : 0.f;
+  T pr[TG], pk[TG], pw[TG], pa[TG];                              // the chunk to build, as loaded
+  float rv[TG], kv[TG], wv[TG], av[TG], tok[TG];
   const auto fetch = [&](int t0) __attribute__((always_inline)) {
 #pragma unroll
     for (int q = 0; q < TG; ++q) {
@@ -148,86 +168,51 @@ scan_chunk_kernel(const ScanArgs<T> a) {
       pw[q] = get(a.wl, a.ldw, t0, tg * TG, q, chc);
       if (DELTA) pa[q] = get(a.al, a.lda, t0, tg * TG, q, chc);
     }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) pv[e] = get(a.v, a.ldv, t0, tok_of(0), DELTA ? e : 4 * e, jc);
   };
-  if (tid < 2) { s_n[tid] = kC; s_low[tid] = s_small[tid] = 0; }
-  fetch(0);
-  __syncthreads();
-  for (int t0 = 0, par = 0; t0 < len; par ^= 1) {
-    // ---- decays, removal rates, the channel sums of every token ----
-    float rv[TG], kv[TG], wv[TG], av[TG];
-    {
-      unsigned top = 0u, low = ~0u, lim = 0u;   // r and k: largest, smallest - 1; the others: largest
-      double gp = 1.;
+  // decays, removal rates, the channel sums of every token
+  const auto decays = [&](int t0, int par) __attribute__((always_inline)) {
+    unsigned top = 0u, low = ~0u, lim = 0u;   // r and k: largest, smallest - 1; the others: largest
+    double gp = 1.;
 #pragma unroll
-      for (int q = 0; q < TG; ++q) {
-        const bool live = t0 + tg * TG + q < len && chan;
-        rv[q] = chan ? to_f32(pr[q]) : 0.f;
-        kv[q] = chan ? to_f32(pk[q]) : 0.f;
-        const float zl = to_f32(pw[q]), z = zl + w0;
-        const float d = DELTA ? expf(-a.decay_scale * sigmoid_f(z)) : expf(-expf(z));
-        wv[q] = live ? d : 1.f;
-        gp *= wv[q];
-        const unsigned mr = mag(rv[q]), mk = mag(kv[q]);
-        top = max(top, max(mr, mk));
-        low = min(low, min(mr - 1u, mk - 1u));   // (0 is as good as large)
-        lim = max(lim, mag(zl));
-        if (DELTA) {
-          const float al = to_f32(pa[q]);
-          lim = max(lim, mag(al));
-          av[q] = live ? sigmoid_f(al + ub) : 0.f;
-        }
-        const float s = sum16(DELTA ? kv[q] * kv[q] : rv[q] * ub * kv[q]);
-        if (lr == 0) s_red[tg * TG + q][ch >> 4] = s;
+    for (int q = 0; q < TG; ++q) {
+      const bool live = t0 + tg * TG + q < len && chan;
+      rv[q] = chan ? to_f32(pr[q]) : 0.f;
+      kv[q] = chan ? to_f32(pk[q]) : 0.f;
+      const float zl = to_f32(pw[q]), z = zl + w0;
+      const float d = DELTA ? exp_near(-a.decay_scale * sigmoid_near(z)) : exp_near(-exp_near(z));
+      wv[q] = live ? d : 1.f;
+      gp *= wv[q];
+      const unsigned mr = mag(rv[q]), mk = mag(kv[q]);
+      top = max(top, max(mr, mk));
+      low = min(low, min(mr - 1u, mk - 1u));   // (0 is as good as large)
+      lim = max(lim, mag(zl));
+      if (DELTA) {
+        const float al = to_f32(pa[q]);
+        lim = max(lim, mag(al));
+        av[q] = live ? sigmoid_near(al + ub) : 0.f;
       }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) lim = max(lim, mag(to_f32(pv[e])));
-      s_gp[tg][ch] = gp;
-      if (top > kLarge || low < (DELTA ? kTinyDelta : kTinyWkv) - 1u || lim >= kInf)
-        atomicMin(&s_n[par], 1);
-      if (!DELTA && low < kSmall - 1u) s_small[par] = 1;
-      // no group's product below its share of the range: no chunk product leaves it
-      if (!DELTA && !(gp >= kGroupP<NG>())) s_low[par] = 1;
+      const float s = sum16(DELTA ? kv[q] * kv[q] : rv[q] * ub * kv[q]);
+      if (lr == 0) s_red[tg * TG + q][ch >> 4] = s;
     }
-    __syncthreads();
-    // the tokens' sums, a lane for each of the wave's, handed round
-    float tok[TG];
-    {
-      float v = 0.f;
+    s_gp[tg][ch] = gp;
+    if (top > kLarge || low < (DELTA ? kTinyDelta : kTinyWkv) - 1u || lim >= kInf)
+      atomicMin(&s_n[par], 1);
+    if (!DELTA && low < kSmall - 1u) s_small[par] = 1;
+  };
+  // the tokens' sums, a lane for each of the wave's, handed round
+  const auto tokens = [&]() __attribute__((always_inline)) {
+    float v = 0.f;
 #pragma unroll
-      for (int b = 0; b < KB; ++b) v += s_red[tg * TG + lane % TG][b];
-      if (DELTA) v = 1.f / sqrtf(v + a.key_eps);
+    for (int b = 0; b < KB; ++b) v += s_red[tg * TG + lane % TG][b];
+    if (DELTA) v = 1.f / sqrtf(v + a.key_eps);
 #pragma unroll
-      for (int q = 0; q < TG; ++q) {
-        tok[q] = lane_f(v, q);
-        if (DKP < 64) tok[q] = lane < 32 ? tok[q] : lane_f(v, 32 + q);
-      }
+    for (int q = 0; q < TG; ++q) {
+      tok[q] = lane_f(v, q);
+      if (DKP < 64) tok[q] = lane < 32 ? tok[q] : lane_f(v, 32 + q);
     }
-    if (s_n[par] < kC || s_low[par] || s_small[par]) {   // a shorter chunk (one decision for the workgroup)
-      if (!DELTA) {                      // where does a channel's product leave the range?
-        const float least = s_small[par] ? kSmallP : kMinP;
-        double p = 1.;
-        for (int g = 0; g < tg; ++g) p *= s_gp[g][ch];
-#pragma unroll
-        for (int q = 0; q < TG; ++q) {
-          p *= wv[q];
-          if (p < least && tg * TG + q > 0) atomicMin(&s_n[par], tg * TG + q);
-        }
-      }
-      __syncthreads();
-      double p = 1.;                     // the rows that are left for the next chunk decay nothing
-#pragma unroll
-      for (int q = 0; q < TG; ++q) {
-        if (tg * TG + q >= s_n[par]) wv[q] = 1.f;
-        p *= wv[q];
-      }
-      s_gp[tg][ch] = p;
-      __syncthreads();
-    }
-    const int n = __builtin_amdgcn_readfirstlane(min(s_n[par], len - t0));
-    if (tid == 0) { s_n[par ^ 1] = kC; s_low[par ^ 1] = s_small[par ^ 1] = 0; }
-    // ---- the scaled rows ----
+  };
+  // the scaled rows of a chunk of n tokens; true: some channel's product leaves the range
+  const auto rows = [&](Buf& B, int n, float least) __attribute__((always_inline)) {
     double P = 1., Q = 1.;               // decay of the token groups before and after this one
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
@@ -239,8 +224,8 @@ scan_chunk_kernel(const ScanArgs<T> a) {
     for (int q = TG - 1; q >= 0; --q) {  // decayed to the chunk's end
       const int at = (tg * TG + q) * LK + ch;
       const bool live = tg * TG + q < n;
-      s_k[at] = live ? (float)(kv[q] * Q) : 0.f;
-      if (DELTA) s_b[at] = live ? (float)(kv[q] * tok[q] * av[q] * Q) : 0.f;
+      B.k[at] = live ? (float)(kv[q] * Q) : 0.f;
+      if (DELTA) B.b[at] = live ? (float)(kv[q] * tok[q] * av[q] * Q) : 0.f;
       Q *= wv[q];
     }
 #pragma unroll
@@ -249,104 +234,138 @@ scan_chunk_kernel(const ScanArgs<T> a) {
       const bool live = t < n;
       const float P0 = (float)P;
       P *= wv[q];
-      s_r[at] = live ? rv[q] * (DELTA ? (float)P : P0) : 0.f;
-      if (DELTA) s_u[at] = live ? kv[q] * tok[q] * P0 : 0.f;
+      B.r[at] = live ? rv[q] * (DELTA ? (float)P : P0) : 0.f;
+      if (DELTA) B.u[at] = live ? kv[q] * tok[q] * P0 : 0.f;
       else if (ch == 0) s_tok[t] = tok[q];
     }
-    if (tg == NG - 1) {
-      s_P[ch] = (float)P;
-      s_iP[ch] = 1.f / (float)P;                // (one token: only entries that are masked out see it)
+    if (tg != NG - 1) return false;
+    B.P[ch] = (float)P;
+    s_iP[ch] = 1.f / (float)P;           // (one token: only entries that are masked out see it)
+    return !DELTA && !((float)P >= least);
+  };
+  // chunk matrices, one per wave: U K^T, U B^T (then inverted), R K^T, R B^T
+  const auto matrices = [&](Buf& B, int n) __attribute__((always_inline)) {
+    const int pw_ = w - kCol;
+    if (pw_ >= NM) return;
+    const float* x = (DELTA && pw_ < 2 ? B.u : B.r) + lr * LK + 4 * lg;
+    const float* y = (DELTA && (pw_ & 1) ? B.b : B.k) + lr * LK + 4 * lg;
+    f32x4 c[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int b = 0; b < KB; ++b) {
+      const float4 xa = *reinterpret_cast<const float4*>(x + 16 * b);
+      const float4 ya = *reinterpret_cast<const float4*>(y + 16 * b);
+      const float4 ip = *reinterpret_cast<const float4*>(&s_iP[16 * b + 4 * lg]);
+      c[0] = mma(xa.x * ip.x, ya.x, c[0]);
+      c[1] = mma(xa.y * ip.y, ya.y, c[1]);
+      c[2] = mma(xa.z * ip.z, ya.z, c[2]);
+      c[3] = mma(xa.w * ip.w, ya.w, c[3]);
+      if (KB > 8 && b % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
-    f32x4 V;
+    const f32x4 acc = (c[0] + c[1]) + (c[2] + c[3]);
+    float* m = B.m[pw_];
+    float z[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) V[e] = tok_of(e) < n ? to_f32(pv[e]) : 0.f;
-    const int next = t0 + n;
-    if (next < len) fetch(next);         // in flight during the products
-    __syncthreads();
-    // ---- chunk matrices, one per wave: U K^T, U B^T (then inverted), R K^T, R B^T ----
-    if (w < NM) {
-      const float* x = (DELTA && w < 2 ? s_u : s_r) + lr * LK + 4 * lg;
-      const float* y = (DELTA && (w & 1) ? s_b : s_k) + lr * LK + 4 * lg;
-      f32x4 c[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) c[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int b = 0; b < KB; ++b) {
-        const float4 xa = *reinterpret_cast<const float4*>(x + 16 * b);
-        const float4 ya = *reinterpret_cast<const float4*>(y + 16 * b);
-        const float4 ip = *reinterpret_cast<const float4*>(&s_iP[16 * b + 4 * lg]);
-        c[0] = mma(xa.x * ip.x, ya.x, c[0]);
-        c[1] = mma(xa.y * ip.y, ya.y, c[1]);
-        c[2] = mma(xa.z * ip.z, ya.z, c[2]);
-        c[3] = mma(xa.w * ip.w, ya.w, c[3]);
-      }
-      const f32x4 acc = (c[0] + c[1]) + (c[2] + c[3]);
-      float* m = s_m[w];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i = 4 * lg + e;        // row: token t; column lr: token s
-        float z = i < n && (DELTA && w >= 2 ? lr <= i : lr < i) ? acc[e] : 0.f;
-        if (!DELTA && lr == i && i < n) z = s_tok[i];
-        m[i * LP + lr] = z;
-      }
-      if (DELTA && w == 1) {             // (I + M)^-1, a lane per column
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        float t[kC];
-#pragma unroll
-        for (int i = 0; i < kC; ++i) {
-          float s = 0.f;
-#pragma unroll
-          for (int q = 0; q < kC; q += 4)
-            if (q < i) {
-              const float4 xr = *reinterpret_cast<const float4*>(&m[i * LP + q]);
-              s += xr.x * t[q];
-              if (q + 1 < i) s += xr.y * t[q + 1];
-              if (q + 2 < i) s += xr.z * t[q + 2];
-              if (q + 3 < i) s += xr.w * t[q + 3];
-            }
-          t[i] = i == lr ? 1.f : i > lr ? -s : 0.f;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (lane < 16) {
-#pragma unroll
-          for (int i = 0; i < kC; ++i) m[i * LP + lr] = t[i];
-        }
-      }
+    for (int e = 0; e < 4; ++e) {
+      const int i = 4 * lg + e;          // row: token t; column lr: token s
+      z[e] = i < n && (DELTA && pw_ >= 2 ? lr <= i : lr < i) ? acc[e] : 0.f;
+      if (!DELTA && lr == i && i < n) z[e] = s_tok[i];
     }
-    // ---- what the old state gives (four sums each: a quarter of the chain, and of its error) ----
-    f32x4 O, C = {0.f, 0.f, 0.f, 0.f};
-    {
-      f32x4 o[4], c[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = c[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int e = 0; e < 4; ++e) m[(4 * lg + e) * LP + lr] = z[e];
+    if (DELTA && pw_ == 1) {
+      // (I + M)^-1 = D - D C D: D the inverses of the diagonal 8 x 8 blocks (a lane per column, substitution),
+      // C the block below them.  (Substitution over all sixteen rows: 3800 cycles, a fifth of the step; here 1000.)
+      wave_lds_fence();
+      const int hb = lr >> 3;
+      const float* d = m + 8 * hb * (LP + 1);
+      float4 x[8][2];
 #pragma unroll
-      for (int b = 0; b < KB; ++b) {
-        const float4 x = *reinterpret_cast<const float4*>(&s_r[lr * LK + 16 * b + 4 * lg]);
-        o[0] = mma(x.x, S[b][0], o[0]);
-        o[1] = mma(x.y, S[b][1], o[1]);
-        o[2] = mma(x.z, S[b][2], o[2]);
-        o[3] = mma(x.w, S[b][3], o[3]);
-        if (DELTA) {
-          const float4 u = *reinterpret_cast<const float4*>(&s_u[lr * LK + 16 * b + 4 * lg]);
-          c[0] = mma(u.x, S[b][0], c[0]);
-          c[1] = mma(u.y, S[b][1], c[1]);
-          c[2] = mma(u.z, S[b][2], c[2]);
-          c[3] = mma(u.w, S[b][3], c[3]);
-        }
+      for (int i = 1; i < 8; ++i) {
+        x[i][0] = *reinterpret_cast<const float4*>(d + i * LP);
+        if (i > 4) x[i][1] = *reinterpret_cast<const float4*>(d + i * LP + 4);
       }
-      O = (o[0] + o[1]) + (o[2] + o[3]);
-      if (DELTA) C = (c[0] + c[1]) + (c[2] + c[3]);
+      float4 cr = *reinterpret_cast<const float4*>(m + lr * LP + 4 * lg);
+      if (!(lr >= 8 && lg < 2)) cr = make_float4(0.f, 0.f, 0.f, 0.f);
+      float t[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float v = 0.f;
+#pragma unroll
+        for (int q = 0; q < i; ++q) {
+          const float4 r4 = x[i][q >> 2];
+          v += (q % 4 == 0 ? r4.x : q % 4 == 1 ? r4.y : q % 4 == 2 ? r4.z : r4.w) * t[q];
+        }
+        t[i] = (i == (lr & 7) ? 1.f : 0.f) - v;      // (0 above the diagonal: every term is)
+      }
+      wave_lds_fence();
+      if (lg < 2) {                      // lane group 0: D's blocks; 1: zeros where C was
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (lg == 0) m[(8 * hb + i) * LP + lr] = t[i];
+          else if (lr < 8) m[(8 + i) * LP + lr] = 0.f;
+      }
+      wave_lds_fence();
+      const float4 da = *reinterpret_cast<const float4*>(m + lr * LP + 4 * lg);
+      f32x4 db, X = {0.f, 0.f, 0.f, 0.f}, Y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) db[e] = m[(4 * lg + e) * LP + lr];
+      X = mma(cr.x, db[0], X);
+      X = mma(cr.y, db[1], X);
+      X = mma(cr.z, db[2], X);
+      X = mma(cr.w, db[3], X);
+      Y = mma(da.x, X[0], Y);
+      Y = mma(da.y, X[1], Y);
+      Y = mma(da.z, X[2], Y);
+      Y = mma(da.w, X[3], Y);
+      wave_lds_fence();
+#pragma unroll
+      for (int e = 0; e < 4; ++e) m[(4 * lg + e) * LP + lr] = db[e] - Y[e];
     }
-    __syncthreads();                     // chunk matrices complete
+  };
+
+  // ---------------- the column waves ----------------
+  f32x4 S[KB], V, O, C;
+  T pv[4];
+  float* st = a.state + ((long long)a.slot[sg] * a.H + hd) * D * D + j;
+  const int jc = min(j, D - 1);
+  // the token of a lane's e-th value: an inner index of every product with V
+  const auto tok_of = [&](int e) { return DELTA ? 4 * lg + e : 4 * e + lg; };
+  const auto fetch_v = [&](int t0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) pv[e] = get(a.v, a.ldv, t0, tok_of(0), DELTA ? e : 4 * e, jc);
+  };
+  // what the old state gives (four sums each: a quarter of the chain, and of its error)
+  const auto old_state = [&](const Buf& B) __attribute__((always_inline)) {
+    f32x4 o[4], c[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = c[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int b = 0; b < KB; ++b) {
+      const float4 x = *reinterpret_cast<const float4*>(&B.r[lr * LK + 16 * b + 4 * lg]);
+      o[0] = mma(x.x, S[b][0], o[0]);
+      o[1] = mma(x.y, S[b][1], o[1]);
+      o[2] = mma(x.z, S[b][2], o[2]);
+      o[3] = mma(x.w, S[b][3], o[3]);
+      if (DELTA) {
+        const float4 u = *reinterpret_cast<const float4*>(&B.u[lr * LK + 16 * b + 4 * lg]);
+        c[0] = mma(u.x, S[b][0], c[0]);
+        c[1] = mma(u.y, S[b][1], c[1]);
+        c[2] = mma(u.z, S[b][2], c[2]);
+        c[3] = mma(u.w, S[b][3], c[3]);
+      }
+      if (KB > 8 && b % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+    O = (o[0] + o[1]) + (o[2] + o[3]);
+    if (DELTA) C = (c[0] + c[1]) + (c[2] + c[3]);
+  };
+  const auto read_out = [&](const Buf& B, int t0, int n) __attribute__((always_inline)) {
     const auto small = [&](int m, const f32x4& x, f32x4 acc) {
       float4 y;
-      if (DELTA) y = *reinterpret_cast<const float4*>(&s_m[m][lr * LP + 4 * lg]);
+      if (DELTA) y = *reinterpret_cast<const float4*>(&B.m[m][lr * LP + 4 * lg]);
       else {
-        const float* r = &s_m[m][lr * LP + lg];
+        const float* r = &B.m[m][lr * LP + lg];
         y = make_float4(r[0], r[4], r[8], r[12]);
       }
       acc = mma(y.x, x[0], acc);
@@ -372,21 +391,23 @@ scan_chunk_kernel(const ScanArgs<T> a) {
       for (int e = 0; e < 4; ++e)
         if (4 * lg + e < n) o[(unsigned)(4 * lg) * HD + (unsigned)e * HD + (unsigned)j] = O[e];
     }
-    // ---- the state moves on.  wkv: decayed, then the tokens' terms in order, the last (and least decayed)
-    // ones last, so that a fast channel sees few roundings.  Delta: what the chunk adds is summed apart, in
-    // fours, and meets the state in one rounding; added term by term to it the error was 1.4 - 1.6 times
-    // the serial walk's ----
+  };
+  // The state moves on.  wkv: decayed, then the tokens' terms in order, the last (and least decayed)
+  // ones last, so that a fast channel sees few roundings.  Delta: what the chunk adds is summed apart, in
+  // fours, and meets the state in one rounding; added term by term to it the error was 1.4 - 1.6 times
+  // the serial walk's.
+  const auto new_state = [&](const Buf& B, int b0, int b1) __attribute__((always_inline)) {
 #pragma unroll
-    for (int b = 0; b < KB; ++b) {
-      const float4 P = *reinterpret_cast<const float4*>(&s_P[16 * b + 4 * lg]);
+    for (int b = b0; b < b1; ++b) {
+      const float4 P = *reinterpret_cast<const float4*>(&B.P[16 * b + 4 * lg]);
       const float p[4] = {P.x, P.y, P.z, P.w};
       if (DELTA) {
         f32x4 d[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-          d[e] = mma(s_k[(4 * lg + e) * LK + 16 * b + lr], V[e], zero) +
-                 mma(s_b[(4 * lg + e) * LK + 16 * b + lr], C[e], zero);
+          d[e] = mma(B.k[(4 * lg + e) * LK + 16 * b + lr], V[e], zero) +
+                 mma(B.b[(4 * lg + e) * LK + 16 * b + lr], C[e], zero);
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e)
@@ -396,10 +417,106 @@ scan_chunk_kernel(const ScanArgs<T> a) {
         for (int e = 0; e < 4; ++e) S[b][e] *= p[e];
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          S[b] = mma(s_k[(4 * e + lg) * LK + 16 * b + lr], V[e], S[b]);
+          S[b] = mma(B.k[(4 * e + lg) * LK + 16 * b + lr], V[e], S[b]);
       }
+      if (KB > 8 && b % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
-    t0 = next;
+  };
+
+  // Step: the producers build the chunk at tb while the column waves run the one before it, [tc, tc + nc).  Both
+  // meet at the same barriers: what decides about more of them lies in LDS before the second.
+  if (tid < 2) { s_n[tid] = kC; s_low[tid] = s_small[tid] = 0; }
+  const auto shorter = [&](int par) { return s_n[par] < kC || s_low[par]; };
+  const auto count = [&](int par, int tb) { return __builtin_amdgcn_readfirstlane(min(s_n[par], len - tb)); };
+  if (!col) {
+    fetch(0);
+    __syncthreads();
+    for (int tb = 0, par = 0;; par ^= 1) {
+      const bool build = tb < len;
+      Buf& B = s_buf[par];
+      if (build) decays(tb, par);
+      __syncthreads();
+      if (build) {
+        tokens();
+        if (rows(B, min(kC, len - tb), s_small[par] ? kSmallP : kMinP)) s_low[par] = 1;
+        if (tb + kC < len) fetch(tb + kC);   // in flight from here on, unless the chunk is shorter
+      }
+      __syncthreads();
+      if (build && shorter(par)) {
+        if (!DELTA) {                    // where does a channel's product leave the range?
+          const float least = s_small[par] ? kSmallP : kMinP;
+          double p = 1.;
+          for (int g = 0; g < tg; ++g) p *= s_gp[g][ch];
+#pragma unroll
+          for (int q = 0; q < TG; ++q) {
+            p *= wv[q];
+            if (p < least && tg * TG + q > 0) atomicMin(&s_n[par], tg * TG + q);
+          }
+        }
+        __syncthreads();
+        const int n = count(par, tb);
+        double p = 1.;                   // the rows that are left for the next chunk decay nothing
+#pragma unroll
+        for (int q = 0; q < TG; ++q) {
+          if (tg * TG + q >= n) wv[q] = 1.f;
+          p *= wv[q];
+        }
+        s_gp[tg][ch] = p;
+        __syncthreads();
+        rows(B, n, 0.f);
+        if (tb + n < len) fetch(tb + n);
+        __syncthreads();
+      }
+      const int n = build ? count(par, tb) : 0;
+      if (ptid == 0) { s_n[par ^ 1] = kC; s_low[par ^ 1] = s_small[par ^ 1] = 0; }
+      if (build) matrices(B, n);
+      __syncthreads();
+      if (!build) return;
+      tb += n;
+    }
+  }
+  const bool fresh = a.start[sg] == 0;
+#pragma unroll
+  for (int b = 0; b < KB; ++b)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int i = 16 * b + 4 * lg + e;
+      S[b][e] = (!fresh && on && i < D) ? st[(long long)i * D] : 0.f;
+    }
+  fetch_v(0);
+  __syncthreads();
+  for (int tb = 0, tc = 0, nc = 0, par = 0;; par ^= 1) {
+    const bool build = tb < len;
+    const Buf& A = s_buf[par ^ 1];
+    if (nc > 0) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) V[e] = tok_of(e) < nc ? to_f32(pv[e]) : 0.f;
+    }
+    if (build && tb > 0) fetch_v(tb);
+    if (nc > 0) old_state(A);
+    if (build) {                         // a value that no other row may meet: its chunk is one token long
+      unsigned lim = 0u;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) lim = max(lim, mag(to_f32(pv[e])));
+      if (lim >= kInf) atomicMin(&s_n[par], 1);
+    }
+    // (nothing of this waits for the producers: cut so that the matrix units are not wanted by all at once)
+    if (nc > 0) read_out(A, tc, nc);
+    __syncthreads();
+    if (nc > 0) new_state(A, 0, KB / 2);
+    __syncthreads();
+    if (build && shorter(par)) {
+      __syncthreads();
+      __syncthreads();
+      __syncthreads();
+    }
+    const int n = build ? count(par, tb) : 0;
+    if (nc > 0) new_state(A, KB / 2, KB);
+    __syncthreads();
+    if (!build) break;
+    tc = tb;
+    nc = n;
+    tb += n;
   }
   if (on) {
 #pragma unroll
@@ -414,11 +531,16 @@ scan_chunk_kernel(const ScanArgs<T> a) {
 
 template <typename T, bool DELTA>
 hipError_t launch(const ScanArgs<T>& a, int n_seg, hipStream_t st) {
-  const dim3 grid(n_seg, a.H, (a.D + 63) / 64);
-  if (a.D <= 32) scan_chunk_kernel<T, 2, DELTA><<<grid, 256, 0, st>>>(a);
-  else if (a.D <= 64) scan_chunk_kernel<T, 4, DELTA><<<grid, 256, 0, st>>>(a);
-  else if (a.D <= 128) scan_chunk_kernel<T, 8, DELTA><<<grid, 256, 0, st>>>(a);
-  else scan_chunk_kernel<T, 16, DELTA><<<grid, 256, 0, st>>>(a);
+  const dim3 grid(n_seg, a.H, (a.D + 16 * kCol - 1) / (16 * kCol));
+#define GO(KB, NP) scan_chunk_kernel<T, KB, DELTA, NP><<<grid, 64 * (kCol + NP), 0, st>>>(a)
+  // Eight producer waves keep up with the column waves; four, where two such workgroups fit a CU and there are so many
+  // (wkv, 32 portions of 128 x 32 heads of 64: 126 -> 99 us, delta, 8 of 512 x 64 of 32: 257 -> 171; heads of 128 not: 246 -> 261)
+  const bool few = (long long)grid.x * grid.y * grid.z <= 256;
+  if (a.D <= 32) { if (few) GO(2, 8); else GO(2, 4); }
+  else if (a.D <= 64) { if (few) GO(4, 8); else GO(4, 4); }
+  else if (a.D <= 128) GO(8, 8);
+  else GO(16, 8);
+#undef GO
   return hipGetLastError();
 }
 

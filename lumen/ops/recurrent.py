@@ -119,7 +119,7 @@ def _check_state(state, H, D):
 
 
 # The chunked kernel takes the prompt portions of 16-bit steps: sixteen tokens per matrix step against ~2 us
-# per token of the serial walk (8 portions of 512 tokens, delta rule, 16 heads of 128: 1000 -> 310 us).  Decoded
+# per token of the serial walk (8 portions of 512 tokens, delta rule, 16 heads of 128: 1000 -> 245 us).  Decoded
 # rows are one token each, and fp32 models keep the serial order of the sums.
 CHUNK_MAX_STRIDE = 1 << 26       # elements between rows (32-bit offsets within a chunk)
 DELTA_CHUNK_MAX_DECAY = 3.0      # e^(-16 decay_scale), a chunk's smallest decay product, in fp32's range

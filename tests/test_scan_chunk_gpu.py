@@ -206,3 +206,29 @@ def test_state_is_no_further_from_float64_than_the_serial_walk(kind, D, monkeypa
                        for i, S in enumerate(want)))
     # measured over 36 portions: 0.94 - 1.0 of the serial walk's on average, +- 0.05 for one draw
     assert err[0] <= 1.1 * err[1], err
+
+
+@pytest.mark.parametrize("kind", ["wkv", "delta"])
+@pytest.mark.parametrize("H,D,n", [(9, 64, 30), (5, 20, 60), (3, 128, 90), (2, 256, 3)])
+def test_more_workgroups_than_compute_units_and_one_key_for_all_rows(kind, H, D, n):
+    """Grids of over 256 workgroups (fewer producer waves for the smaller heads), and rows that all carry one key with
+    nearly whole removal: the chunk's triangular matrix is full, its powers grow though its inverse does not."""
+    g = torch.Generator().manual_seed(D)
+    pieces = [15 + 7 * (i % 3) for i in range(n)]
+    starts = [i % 2 for i in range(n)]
+    cu, seg = batch(pieces, 0, starts)
+    x = rows(cu[-1], H, D, torch.bfloat16, g, 0)
+    x[1][:] = x[1][:1].clone()
+    x[4][:] = 4.0
+    w0 = torch.full((H * D,), -6.0).cuda()
+    ub, nw = torch.zeros(H * D).cuda(), torch.ones(H * D).cuda()
+    state = torch.randn(n, H, D, D, generator=g).cuda()
+    before = state.clone()
+    y = run(kind, x, w0, ub, nw, state, seg, H, D)
+    for s in list(range(0, n, 7)) + [n - 1]:
+        a, b, slot = cu[s], cu[s + 1], n - 1 - s
+        want, S = exact(kind, [t[a:b] for t in x], w0, ub, nw, before[slot].cpu().double() * (starts[s] > 0), H, D)
+        # as above: one rounding of the result, fp32 sums
+        err = (y[a:b].cpu().double() - want).abs()
+        assert (err <= want.abs() * 2.0 ** -8 + 2e-5 * want.abs().max()).all(), (s, err.max())
+        assert (state[slot].cpu().double() - S).norm() <= 2e-6 * S.norm()

@@ -18,28 +18,12 @@
 //                  (an expert whose INPUT is weighted); fp32 math.
 //   sm_scaled_act  act(up) over stacked up blocks of experts without a gate, scaled the same way.
 //   sm_write_k     rows of the key projection into the paged key cache by slot.
-#include "seqmix.h"
+#include "route.h"
 
 using namespace lumen;
 
 namespace {
 
-constexpr int kMaxPerLane = 16;   // experts <= 1024
-
-// wave-wide arg-max of (value, index) pairs, ties to the lowest index; every lane gets the result
-__device__ __forceinline__ void wave_argmax(float& bv, int& bi) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(bv, o, 64);
-    const int oi = __shfl_xor(bi, o, 64);
-    if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-  }
-}
-
-constexpr int kNone = 0x7fffffff;
-
-// LDS per wave: c [E] (the choice ranks; -inf once an expert is chosen or its group dropped) and
-// rank [n_groups] (-inf once a group is kept)
 __global__ void __launch_bounds__(256)
 route_groups_kernel(const float* __restrict__ z, const float* __restrict__ corr,
                     float* __restrict__ out, int T, int E, int top, int n_groups, int keep,
@@ -49,85 +33,8 @@ route_groups_kernel(const float* __restrict__ z, const float* __restrict__ corr,
   const int row = blockIdx.x * 4 + wv;
   if (row >= T) return;                              // whole waves leave; no block barrier below
   float* c = s_all + wv * (E + n_groups);
-  float* rank = c + E;
-  const float* zr = z + (long long)row * E;
-  float* orow = out + (long long)row * E;
-  // the scores: sigmoids, or the softmax over all experts (maximum and sum wave-wide, fp32)
-  float smax = 0.f, sinv = 1.f;
-  if (softmax) {
-    smax = -INFINITY;
-    for (int e = lane; e < E; e += 64) smax = fmaxf(smax, zr[e]);
-    smax = wave_max(smax);
-    float ssum = 0.f;
-    for (int e = lane; e < E; e += 64) ssum += expf(zr[e] - smax);
-    sinv = 1.f / wave_sum(ssum);
-  }
-  const auto score = [&](int e) {
-    return softmax ? expf(zr[e] - smax) * sinv : sigmoid_f(zr[e]);
-  };
-  for (int e = lane; e < E; e += 64) {
-    c[e] = score(e) + (corr != nullptr ? corr[e] : 0.f);
-    orow[e] = 0.f;
-  }
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  if (n_groups > 1 && keep < n_groups) {
-    const int per = E / n_groups;
-    // a group's rank: its `rank_top` largest c summed, one lane per group
-    for (int g = lane; g < n_groups; g += 64) {
-      float sum = 0.f;
-      int taken[4] = {-1, -1, -1, -1};               // rank_top <= 4
-      for (int r = 0; r < rank_top && r < per; ++r) {
-        float bv = -INFINITY;
-        int bi = -1;
-        for (int k = 0; k < per; ++k) {
-          bool used = false;
-          for (int q = 0; q < r; ++q) used |= taken[q] == k;
-          if (!used && (bi < 0 || c[g * per + k] > bv)) { bv = c[g * per + k]; bi = k; }
-        }
-        taken[r] = bi;
-        sum += bv;
-      }
-      rank[g] = sum;
-    }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    for (int it = 0; it < keep; ++it) {
-      float bv = -INFINITY;
-      int bi = kNone;
-      for (int g = lane; g < n_groups; g += 64)
-        if (rank[g] > bv || (rank[g] == bv && g < bi && rank[g] != -INFINITY)) { bv = rank[g]; bi = g; }
-      wave_argmax(bv, bi);
-      if (bi == kNone) break;
-      if (lane == 0) rank[bi] = -INFINITY;           // kept: marked by -inf
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    }
-    for (int e = lane; e < E; e += 64)
-      if (rank[e / per] != -INFINITY) c[e] = -INFINITY;   // its group was not kept
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  }
-  float den = 0.f;
-  int mine[16];                                      // top <= E <= 1024: a lane wins <= 16 rounds
-  int n_mine = 0;
-  for (int it = 0; it < top; ++it) {
-    float bv = -INFINITY;
-    int bi = kNone;
-    for (int e = lane; e < E; e += 64)
-      if (c[e] > bv) { bv = c[e]; bi = e; }          // ascending e: ties keep the lowest index
-    wave_argmax(bv, bi);
-    if (bi == kNone) break;                          // fewer than `top` eligible experts
-    den += score(bi);
-    if ((bi & 63) == lane) {
-      c[bi] = -INFINITY;
-      if (n_mine < 16) mine[n_mine++] = bi;
-    }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  }
-  const float k = normalize ? scale / (den + sum_eps) : scale;
-  for (int q = 0; q < n_mine; ++q) orow[mine[q]] = score(mine[q]) * k;
+  route_groups_row(z + (long long)row * E, corr, out + (long long)row * E, c, c + E, lane, E, top, n_groups, keep,
+                   rank_top, scale, sum_eps, softmax, normalize);
 }
 
 template <typename T>
@@ -169,46 +76,9 @@ scaled_act_v8(const T* __restrict__ u, const float* __restrict__ wts, T* __restr
 
 __global__ void __launch_bounds__(256)
 route_topk_kernel(const float* __restrict__ z, float* __restrict__ out, int T, int E, int top) {
-  const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (row >= T) return;
-  const float* zr = z + (long long)row * E;
-  float val[kMaxPerLane];
-  unsigned sel = 0;
-#pragma unroll
-  for (int q = 0; q < kMaxPerLane; ++q) {
-    const int e = lane + 64 * q;
-    val[q] = e < E ? zr[e] : -INFINITY;
-  }
-  float m0 = 0.f, den = 0.f;
-  for (int it = 0; it < top; ++it) {
-    float bv = -INFINITY;
-    int bi = 0x7fffffff;
-#pragma unroll
-    for (int q = 0; q < kMaxPerLane; ++q) {
-      const int e = lane + 64 * q;
-      if (e < E && !((sel >> q) & 1u) && (val[q] > bv || (val[q] == bv && e < bi))) {
-        bv = val[q];
-        bi = e;
-      }
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ov = __shfl_xor(bv, o, 64);
-      const int oi = __shfl_xor(bi, o, 64);
-      if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-    }
-    if (bi == 0x7fffffff) break;         // fewer than `top` finite candidates
-    if (it == 0) m0 = bv;
-    den += expf(bv - m0);
-    if ((bi & 63) == lane) sel |= 1u << (bi >> 6);
-  }
-  float* orow = out + (long long)row * E;
-#pragma unroll
-  for (int q = 0; q < kMaxPerLane; ++q) {
-    const int e = lane + 64 * q;
-    if (e < E) orow[e] = ((sel >> q) & 1u) ? expf(val[q] - m0) / den : 0.f;
-  }
+  route_topk_row(z + (long long)row * E, out + (long long)row * E, threadIdx.x & 63, E, top);
 }
 
 template <typename T>

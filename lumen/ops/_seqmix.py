@@ -52,6 +52,7 @@ SIGNATURES = {
     "sm_layer_norm": "iippfpppiif",
     "sm_embed_pos": "ipppppiiii",
     "sm_route_groups": "pppiiiiiiffii",
+    "sm_route_rows": "ii" "pp" "pl" "ppp" "ppp" "ppp" "iii" "f" "iiiiii" "ff" "p",
     "sm_rotary_write": "iplppppiiiiipii",
     "sm_min_gru": "iplpppppppiifppii",
     "sm_diff_combine": "ipplpiiiifff",

@@ -122,6 +122,103 @@ def route_groups(z: torch.Tensor, correction: Optional[torch.Tensor], top: int, 
     return out
 
 
+# Few rows: the norm before the experts, the router's product and the routing in one launch (seqmix/route_rows.hip, a
+# workgroup per row, which reads the router for itself; more rows or experts are better off with the product on
+# matrix cores).
+ROUTE_MAX_M, ROUTE_MAX_E, ROUTE_MAX_W = 64, 64, 8192
+
+
+def _route_rows_ok(h: torch.Tensor, router: torch.Tensor, bias, correction, top: int, groups: int, keep: int,
+                   rank_top: int) -> bool:
+    """``h``: the normed rows, or the sublayer's output that the stream takes before the norm."""
+    if h.dim() != 2 or not 0 < h.shape[0] <= ROUTE_MAX_M or not h.is_cuda or router.dim() != 2:
+        return False
+    (E, W), dt = router.shape, h.dtype
+    if (W != h.shape[1] or W % 8 or not 0 < W <= ROUTE_MAX_W or not 0 < E <= ROUTE_MAX_E or dt != router.dtype
+            or dt not in (torch.bfloat16, torch.float16) or router.device != h.device or not router.is_contiguous()
+            or not row_bias_ok(bias, h, E) or not _plain(h, router) or not _here(h)):
+        return False
+    if bias is not None and not _plain(bias) or correction is not None and not (
+            correction.dtype == torch.float32 and correction.is_contiguous() and correction.numel() == E
+            and correction.device == h.device and _plain(correction)):
+        return False
+    if groups and (E % groups or not 1 <= keep <= groups or top > keep * (E // groups) or not 1 <= rank_top <= 4):
+        return False
+    return (1 <= top <= E and h.stride(1) == 1 and h.stride(0) % 8 == 0 and h.stride(0) >= W
+            and (h.data_ptr() | router.data_ptr()) % 16 == 0)
+
+
+def _stream_ok(x: torch.Tensor, y: torch.Tensor, rows: tuple, ones: tuple = ()) -> bool:
+    """Can the fused form take ``y`` into the fp32 stream ``x``, with norms' ``rows`` of [W] and single values?"""
+    if not (x.dtype == torch.float32 and x.shape == y.shape and x.is_contiguous() and y.is_contiguous()
+            and x.device == y.device and x.data_ptr() % 16 == 0 and _plain(x)):
+        return False
+    return (all(t.dtype == torch.float32 and t.device == x.device and _plain(t) for t in rows + ones)
+            and all(t.is_contiguous() and t.numel() == x.shape[1] and t.data_ptr() % 16 == 0 for t in rows)
+            and all(t.numel() == 1 for t in ones))
+
+
+def _route_rows(kind, x, y, h, norm, post, eps, router, bias, top, groups=0, keep=0, rank_top=1, softmax=False,
+                normalize=True, scale=1.0, sum_eps=0.0, correction=None) -> torch.Tensor:
+    from ._seqmix import DT, call, use_seqmix
+
+    use_seqmix(h)
+    T, W = h.shape
+    E = router.shape[0]
+    out = torch.empty(T, E, dtype=torch.float32, device=h.device)
+    call("sm_route_rows", DT[h.dtype], kind, x, y, h, h.stride(0), *norm, *post, router, bias, out, T, W, E, eps, top,
+         groups, keep, rank_top, int(softmax), int(bool(normalize)), scale, sum_eps, correction)
+    return out
+
+
+_NONE3 = (None, None, None)
+
+
+def routed_topk(h: torch.Tensor, router: torch.Tensor, bias: Optional[torch.Tensor], top: int) -> torch.Tensor:
+    """``route_topk`` of ``router_logits``."""
+    if _route_rows_ok(h, router, bias, None, top, 0, 0, 1):
+        return _route_rows(0, None, None, h, _NONE3, _NONE3, 0.0, router, bias, top)
+    return route_topk(router_logits(h, router, bias), top)
+
+
+def routed_groups(h: torch.Tensor, router: torch.Tensor, correction: Optional[torch.Tensor], top: int, n_groups: int,
+                  keep: int, scale: float = 1.0, sum_eps: float = 1e-20, rank_top: int = 2,
+                  score: str = "sigmoid", normalize: bool = True) -> torch.Tensor:
+    """``route_groups`` of ``router_logits``."""
+    if score in ("sigmoid", "softmax") and _route_rows_ok(h, router, None, correction, top, n_groups, keep, rank_top):
+        return _route_rows(0, None, None, h, _NONE3, _NONE3, 0.0, router, None, top, n_groups, keep, rank_top,
+                           score == "softmax", normalize, scale, sum_eps, correction)
+    return route_groups(router_logits(h, router), correction, top, n_groups, keep, scale, sum_eps, rank_top, score,
+                        normalize)
+
+
+def residual_rms_routed(x: torch.Tensor, y: torch.Tensor, w: torch.Tensor, eps: float, router: torch.Tensor, top: int,
+                        normalize: bool = True) -> tuple:
+    """``residual_rms`` into the experts' input h, and its routing by sigmoid scores (``route_groups`` of one
+    group): (h, weights)."""
+    from .norm import residual_rms
+
+    if _route_rows_ok(y, router, None, None, top, 1, 1, 1) and _stream_ok(x, y, (w,)):
+        h = torch.empty_like(y)
+        return h, _route_rows(1, x, y, h, (w, None, None), _NONE3, eps, router, None, top, 1, 1, 1, False, normalize,
+                              1.0, 1e-20)
+    h = residual_rms(x, y, w, eps)
+    return h, route_groups(router_logits(h, router), None, top, 1, 1, normalize=normalize)
+
+
+def dyt_residual_routed(x: torch.Tensor, y: torch.Tensor, post, pre, router: torch.Tensor,
+                        bias: Optional[torch.Tensor], top: int, dtype: torch.dtype) -> tuple:
+    """``dyt_residual`` into the experts' input h, and its routing over the ``top`` logits: (x, h, weights)."""
+    from .norm import dyt_residual
+
+    if y.dtype == dtype and _route_rows_ok(y, router, bias, None, top, 0, 0, 1) \
+            and _stream_ok(x, y, (*post[:2], *pre[:2]), (post[2], pre[2])):
+        h = torch.empty_like(y)
+        return x, h, _route_rows(2, x, y, h, pre, post, 0.0, router, bias, top)
+    x, h = dyt_residual(x, y, post, pre, dtype)
+    return x, h, route_topk(router_logits(h, router, bias), top)
+
+
 GATE_ACTS = {"silu": 0, "relu": 1, "gelu_tanh": 2, "relu2": 3}
 _ACT_FN = {"silu": F.silu, "relu": F.relu, "gelu_tanh": lambda z: F.gelu(z, approximate="tanh"),
            "relu2": lambda z: F.relu(z) ** 2}

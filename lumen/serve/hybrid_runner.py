@@ -50,7 +50,8 @@ from ..ops.attention import (chunk_sink_attention, diff_head_combine, fresh_late
 from ..ops.conv import dyt_canon, short_conv
 from ..ops.embedding import embed_positions, embed_scaled, gated_token_slice, soft_cap
 from ..ops.gemm import project
-from ..ops.moe import ClampedGate, feed_forward, moe, route_groups, route_topk, router_logits
+from ..ops.moe import (ClampedGate, dyt_residual_routed, feed_forward, moe, residual_rms_routed, routed_groups,
+                       router_logits)
 from ..ops.norm import (SPLIT, depth_mix_norm, dyt, dyt_residual, embed_rms, gated_rms_norm,
                         group_rms_norm, group_rms_residual, hyper_mix, hyper_start, parts_rms,
                         residual_rms, scaled_residual_layer_norm, weight_layer_norm)
@@ -283,13 +284,13 @@ def run_layers(w: HybridWeights, st: HybridState, tokens: torch.Tensor, seg: Seg
         if f is None:
             x, _ = dyt_residual(x, y, L.norms["norm1b"], None, dt)
         else:
-            x, h2 = dyt_residual(x, y, L.norms["norm1b"], L.norms["norm2"], dt)
             if f["E"]:
                 # the router in fp32, on the (possibly 16-bit rounded) normed row
-                z = router_logits(h2, f["router"], f["router_b"])
-                y2 = moe(h2, route_topk(z, f["top"]), f["gu"], f["down"], f["E"], f["top"],
-                         f["ff"], f["ffs"])
+                x, h2, r = dyt_residual_routed(x, y, L.norms["norm1b"], L.norms["norm2"], f["router"], f["router_b"],
+                                               f["top"], dt)
+                y2 = moe(h2, r, f["gu"], f["down"], f["E"], f["top"], f["ff"], f["ffs"])
             else:
+                x, h2 = dyt_residual(x, y, L.norms["norm1b"], L.norms["norm2"], dt)
                 y2 = feed_forward(h2, f["gu"], f["down"], f["ffs"])
             x, _ = dyt_residual(x, y2, L.norms["norm2b"], None, dt)
         if observe is not None:
@@ -638,8 +639,8 @@ def run_fanopel_layers(w: FanopelWeights, st: FanopelState, tokens: torch.Tensor
         else:
             x, h2 = scaled_residual_layer_norm(x, y, c, f["norm"], eps, dt)
             # the router in fp32, on the (possibly 16-bit rounded) normed row
-            r = route_groups(router_logits(h2, f["router"]), f["correction"], f["top"], f["groups"],
-                             f["keep"], f["scale"], f["sum_eps"], f["rank_top"])
+            r = routed_groups(h2, f["router"], f["correction"], f["top"], f["groups"], f["keep"], f["scale"],
+                              f["sum_eps"], f["rank_top"])
             y2 = moe(h2, r, f["up"], f["down"], f["E"], f["top"], f["ff"], 0, "relu2", gated=False)
             x, h = scaled_residual_layer_norm(x, y2, c, nxt, eps, dt)
         if observe is not None:
@@ -898,8 +899,8 @@ def run_foderax_layers(w: FoderaxWeights, st: FoderaxState, tokens: torch.Tensor
         f = L.ff
         if f is not None:
             # the router in fp32, on the (possibly 16-bit rounded) normed row
-            r = route_groups(router_logits(h, f["router"]), None, f["top"], f["groups"], f["keep"],
-                             1.0, rank_top=1, score="softmax", normalize=False)
+            r = routed_groups(h, f["router"], None, f["top"], f["groups"], f["keep"], 1.0, rank_top=1,
+                              score="softmax", normalize=False)
             ys.append(moe(h, r, f["up"], f["down"], f["E"], f["top"], f["ff"], 0, "relu2",
                           gated=False))
             scales.append(f["ls2"])
@@ -1312,11 +1313,12 @@ def _tazulix_mixer(L: TazulixLayerW, w: TazulixWeights, st: TazulixState, n: int
     return project(y, L.w["o"])
 
 
-def _tazulix_ff(f: dict, h) -> torch.Tensor:
+def _tazulix_ff(f: dict, x, y, eps: float) -> torch.Tensor:
+    """The mixer's output ``y`` joins the stream ``x``; the feed-forward of the normed rows."""
     if not f["E"]:
-        return feed_forward(h, f["up"], f["down"], f["ff"], "relu2", gated=False)
+        return feed_forward(residual_rms(x, y, f["norm"], eps), f["up"], f["down"], f["ff"], "relu2", gated=False)
     # the router in fp32, on the (possibly 16-bit rounded) normed row
-    r = route_groups(router_logits(h, f["router"]), None, f["top"], 1, 1, normalize=False)
+    h, r = residual_rms_routed(x, y, f["norm"], eps, f["router"], f["top"], normalize=False)
     return moe(h, r, f["gu"], f["down"], f["E"], f["top"], f["ff"], f["ffs"], f["act"],
                weigh="input")
 
@@ -1344,8 +1346,7 @@ def run_tazulix_layers(w: TazulixWeights, st: TazulixState, tokens: torch.Tensor
         if L.ff is None:
             h = residual_rms(x, y, want(n + 1), eps)
         else:
-            h = residual_rms(x, y, L.ff["norm"], eps)
-            h = residual_rms(x, _tazulix_ff(L.ff, h), want(n + 1), eps)
+            h = residual_rms(x, _tazulix_ff(L.ff, x, y, eps), want(n + 1), eps)
         if observe is not None:
             observe(n, x)
     return x

@@ -1,0 +1,175 @@
+// What a decode step's latent-attention layer does around its attention, two launches instead of four.
+//
+//   sm_latent_in     a row of z = [query latent Q | latent R | rotated key part Dr]: the cache row as sm_latent_write
+//                    forms it, and rms(z[:Q]) * wq.  One workgroup for each of the two, per row: as a wave of a
+//                    four-row workgroup the write took 10 us for 64 rows, most of it one wave's chain of loads.
+//   sm_latent_query  the query in the latent space, qa[h] = q[h, :D] uk[h] (uk held [H][R][D], so both operands are
+//                    rows along D), and the rotated part of every head turned in place.  A wave takes 16
+//                    latent columns of a head and 64 rows, fragments straight from L2 (2 MB of weights, 16 KB of
+//                    queries a head; nothing is worth staging for one product each), all loads in flight at once.
+// Bound by latency.  64 rows x 16 heads, D = 128, R = 512, in a decode step, us: write and norm 10.1 + 4.5 -> 6.2; batched
+// library product and rotation 5.1 + 4.5 -> 7.0.
+#include "seqmix.h"
+
+using namespace lumen;
+
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+template <typename T> __device__ __forceinline__ f32x4 mma(uint4 a, uint4 b, f32x4 c);
+template <> __device__ __forceinline__ f32x4 mma<bf16>(uint4 a, uint4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+template <> __device__ __forceinline__ f32x4 mma<fp16>(uint4 a, uint4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+
+constexpr int kThreads = 256;
+
+template <typename T> struct InArgs {
+  const T* z; long long ldz;
+  const float *wq, *wn, *inv_freq;
+  const int* positions; const long long* slots;
+  T *cache, *vt, *qn;
+  int bs, Q, R, Dr, dims;
+  float eps;
+};
+
+template <typename T>
+__global__ void __launch_bounds__(kThreads) latent_in_kernel(const InArgs<T> a) {
+  __shared__ float s_red[kThreads / 64];
+  const int t = blockIdx.x, tid = threadIdx.x;
+  const T* zr = a.z + (long long)t * a.ldz;
+  const bool query = blockIdx.y == 1;
+  const long long s = query ? 0 : a.slots[t];
+  if (s < 0) return;                                   // (the whole workgroup)
+  const T* x = query ? zr : zr + a.Q;
+  const int n = query ? a.Q : a.R;
+  const float* w = query ? a.wq : a.wn;
+  float ss = 0.f;
+  for (int c = tid; c < n; c += kThreads) {
+    const float v = to_f32(x[c]);
+    ss += v * v;
+  }
+  const float inv = 1.f / sqrtf(block_sum<kThreads>(ss, s_red) / (float)n + a.eps);
+  T* dst = query ? a.qn + (long long)t * a.Q : a.cache + s * (a.R + a.Dr);
+  T* dt = !query && a.vt ? a.vt + (s / a.bs) * (long long)a.R * a.bs + s % a.bs : nullptr;
+  for (int c = tid; c < n; c += kThreads) {
+    const T v = from_f32<T>(to_f32(x[c]) * inv * w[c]);
+    dst[c] = v;
+    if (dt) dt[(long long)c * a.bs] = v;
+  }
+  if (query) return;
+  const float pos = (float)a.positions[t];
+  for (int pr = tid; pr < a.dims / 2; pr += kThreads) {
+    float sn, cs;
+    sincosf(pos * a.inv_freq[pr], &sn, &cs);
+    const float u = to_f32(x[a.R + 2 * pr]), v = to_f32(x[a.R + 2 * pr + 1]);
+    dst[a.R + 2 * pr] = from_f32<T>(u * cs - v * sn);
+    dst[a.R + 2 * pr + 1] = from_f32<T>(v * cs + u * sn);
+  }
+  for (int c = a.dims + tid; c < a.Dr; c += kThreads) dst[a.R + c] = x[a.R + c];
+}
+
+template <typename T> struct QueryArgs {
+  T* q; long long ldq; int ldh;             // rows; head h of a row at column h * ldh
+  const T* w;                               // [H][R][D]
+  T* out;                                   // [H][Tn][R]
+  int Tn, R, off, dims;                     // rotated part: columns off .. off + dims - 1 of a head
+  const float* inv_freq; const int* positions;
+};
+
+// KS: steps of 32 along D
+template <typename T, int KS>
+__global__ void __launch_bounds__(256) latent_query_kernel(const QueryArgs<T> a) {
+  constexpr int D = 32 * KS;
+  const int h = blockIdx.y, t0 = blockIdx.z * 64;
+  if ((int)blockIdx.x * 64 >= a.R) {                   // the last column of workgroups: the rotation
+    const int half = a.dims / 2, n = min(64, a.Tn - t0) * half;
+    for (int i = threadIdx.x; i < n; i += 256) {
+      const int t = t0 + i / half, pr = i % half;
+      float sn, cs;
+      sincosf((float)a.positions[t] * a.inv_freq[pr], &sn, &cs);
+      T* p = a.q + (long long)t * a.ldq + h * a.ldh + a.off + 2 * pr;
+      const float u = to_f32(p[0]), v = to_f32(p[1]);
+      p[0] = from_f32<T>(u * cs - v * sn);
+      p[1] = from_f32<T>(v * cs + u * sn);
+    }
+    return;
+  }
+  const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
+  const int r0 = blockIdx.x * 64 + 16 * (threadIdx.x >> 6);
+  const T* wr = a.w + ((long long)h * a.R + r0 + lr) * D + 8 * lg;
+  uint4 x[KS], y[4][KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) x[s] = *reinterpret_cast<const uint4*>(wr + 32 * s);
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (t0 + 16 * j < a.Tn) {
+      const T* qr = a.q + (long long)min(t0 + 16 * j + lr, a.Tn - 1) * a.ldq + h * a.ldh + 8 * lg;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) y[j][s] = *reinterpret_cast<const uint4*>(qr + 32 * s);
+    }
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (t0 + 16 * j < a.Tn) {
+      f32x4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < KS; ++s) c = mma<T>(x[s], y[j][s], c);
+      const int t = t0 + 16 * j + lr;                  // lane (lr, lg): row t, columns r0 + 4 lg ..
+      if (t < a.Tn)
+        *reinterpret_cast<uint2*>(a.out + ((long long)h * a.Tn + t) * a.R + r0 + 4 * lg) =
+            make_uint2(pk2<T>(c[0], c[1]), pk2<T>(c[2], c[3]));
+    }
+}
+
+}  // namespace
+
+extern "C" {
+
+// z [rows][>= Q + R + Dr] at stride ldz, any 16-bit or fp32 type; qn [rows][Q]; the rest as sm_latent_write.
+hipError_t sm_latent_in(int dt, const void* z, long long ldz, const float* wq, void* qn, const float* wn,
+                        const float* inv_freq, const int* positions, const long long* slots, void* cache, void* vt,
+                        int bs, int rows, int Q, int R, int Dr, int dims, float eps, hipStream_t st) {
+  if (rows == 0) return hipSuccess;
+  if (rows < 0 || Q < 1 || R < 1 || Dr < 0 || dims < 0 || dims % 2 || dims > Dr || bs < 1 || ldz < Q + R + Dr)
+    return hipErrorInvalidValue;
+#define CALL(T)                                                                                                 \
+  latent_in_kernel<T><<<dim3(rows, 2), kThreads, 0, st>>>(InArgs<T>{(const T*)z, ldz, wq, wn, inv_freq, positions, \
+                                                            slots, (T*)cache, (T*)vt, (T*)qn, bs, Q, R, Dr, dims, eps})
+  SM_DISPATCH(dt, CALL)
+#undef CALL
+  return hipGetLastError();
+}
+
+// q [rows] at stride ldq, heads at stride ldh (both % 8); w [H][R][D]; out [H][rows][R].  16-bit, D in 64, 128, 192 or
+// 256, R % 64 == 0, 16-byte bases; the rotated part, if any, lies behind a head's first D columns.
+hipError_t sm_latent_query(int dt, void* q, long long ldq, int ldh, const void* w, void* out, int rows, int H, int D,
+                           int R, int off, int dims, const float* inv_freq, const int* positions, hipStream_t st) {
+  if (rows == 0) return hipSuccess;
+  if (rows < 0 || rows > 64 * 65535 || H < 1 || H > 65535 || R < 64 || R % 64 || ldh < D || ldh % 8 || ldq % 8 ||
+      ldq < (long long)(H - 1) * ldh + D || dims < 0 || dims % 2 ||
+      (dims > 0 && (off < D || off + dims > ldh || !inv_freq || !positions ||
+                    ldq < (long long)(H - 1) * ldh + off + dims)) ||
+      ((uintptr_t)q | (uintptr_t)w | (uintptr_t)out) % 16 || (dt != kBF16 && dt != kF16))
+    return hipErrorInvalidValue;
+  const dim3 grid(R / 64 + (dims > 0), H, (rows + 63) / 64);
+#define GO(T, KS)                                                                                                   \
+  latent_query_kernel<T, KS><<<grid, 256, 0, st>>>(QueryArgs<T>{(T*)q, ldq, ldh, (const T*)w, (T*)out, rows, R, off, \
+                                                                 dims, inv_freq, positions})
+#define GO_T(T)                            \
+  if (D == 64) GO(T, 2);                   \
+  else if (D == 128) GO(T, 4);             \
+  else if (D == 192) GO(T, 6);             \
+  else if (D == 256) GO(T, 8);             \
+  else return hipErrorInvalidValue
+  if (dt == kBF16) { GO_T(bf16); } else { GO_T(fp16); }
+#undef GO_T
+#undef GO
+  return hipGetLastError();
+}
+
+}  // extern "C"

@@ -52,6 +52,9 @@ SIGNATURES = {
     "sm_layer_norm": "iippfpppiif",
     "sm_embed_pos": "ipppppiiii",
     "sm_route_groups": "pppiiiiiiffii",
+    "sm_latent_in": "iplpp" "pppp" "pp" "iiiiii" "f",
+    "sm_latent_query": "iplipp" "iiiiii" "pp",
+    "sm_thin_gate": "iplpp" "iii" "plp",
     "sm_route_rows": "ii" "pp" "pl" "ppp" "ppp" "ppp" "iii" "f" "iiiiii" "ff" "p",
     "sm_rotary_write": "iplppppiiiiipii",
     "sm_min_gru": "iplpppppppiifppii",

@@ -675,6 +675,54 @@ def latent_write(z: torch.Tensor, w_norm: torch.Tensor, inv_freq: torch.Tensor,
          vt, own, cache.shape[1], z.shape[0], R, Dr, dims, eps)
 
 
+LATENT_STEP_MAX_T = 512      # rows; more fill the chip with a wave per row
+
+
+def latent_inputs(z: torch.Tensor, Q: int, wq: torch.Tensor, w_norm: torch.Tensor, inv_freq: Optional[torch.Tensor],
+                  positions: torch.Tensor, slots: torch.Tensor, cache: torch.Tensor, R: int, dims: int, eps: float,
+                  vt: Optional[torch.Tensor] = None, own: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``latent_write`` of z[:, Q:] and the RMS norm of the query latent z[:, :Q] with ``wq``, which is returned: one
+    launch for a step of few rows (HIP ``csrc/seqmix/latent_step.hip``)."""
+    from ._seqmix import DT, call, use_seqmix
+    from .norm import group_rms_norm
+
+    T, Dr = z.shape[0], z.shape[1] - Q - R
+    if (own is not None or not 0 < T <= LATENT_STEP_MAX_T or not use_seqmix(z) or z.stride(1) != 1 or cache.dtype != z.dtype
+            or not cache.is_contiguous() or cache.shape[-1] != R + Dr or dims > Dr or dims % 2 or wq.numel() != Q
+            or wq.dtype != torch.float32 or not wq.is_contiguous()
+            or vt is not None and (tuple(vt.shape) != (cache.shape[0], R, cache.shape[1]) or vt.dtype != cache.dtype
+                                   or not vt.is_contiguous())):
+        latent_write(z[:, Q:], w_norm, inv_freq, positions, slots, cache, R, dims, eps, vt, own)
+        return group_rms_norm(z[:, :Q], wq, 1, eps, z.dtype)
+    qn = torch.empty(T, Q, dtype=z.dtype, device=z.device)
+    call("sm_latent_in", DT[z.dtype], z, z.stride(0), wq, qn, w_norm, inv_freq, positions, slots, cache, vt,
+         cache.shape[1], T, Q, R, Dr, dims, eps)
+    return qn
+
+
+def latent_query(q: torch.Tensor, uk: torch.Tensor, ukT: torch.Tensor, D: int, positions: torch.Tensor,
+                 dims: int = 0, inv_freq: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """q [T, H, D + Dr], a decode step's queries: their first ``dims`` columns behind D turned in place (see
+    ``rotate_interleaved_``), and their first D in the latent space, [H, T, R] = q[:, h, :D] uk[h].  ``ukT`` [H, R, D]:
+    ``uk`` [H, D, R] with both last dimensions exchanged."""
+    from ._seqmix import DT, call, use_seqmix
+    from .gemm import _here, _plain
+    from .rope import rotate_interleaved_
+
+    T, H, N = q.shape
+    R = ukT.shape[1]
+    if (not 0 < T <= LATENT_STEP_MAX_T or not use_seqmix(q) or q.dtype not in (torch.bfloat16, torch.float16)
+            or D not in (64, 128, 192, 256) or R % 64 or N % 8 or q.stride(2) != 1 or q.stride(1) != N
+            or q.stride(0) % 8 or ukT.dtype != q.dtype or tuple(ukT.shape) != (H, R, D) or not ukT.is_contiguous()
+            or (q.data_ptr() | ukT.data_ptr()) % 16 or not _plain(q, ukT) or not _here(q)):
+        if dims:
+            rotate_interleaved_(q.view(T, H * N), positions, H, N, D, dims, inv_freq)
+        return torch.bmm(q[:, :, :D].transpose(0, 1), uk)
+    out = torch.empty(H, T, R, dtype=q.dtype, device=q.device)
+    call("sm_latent_query", DT[q.dtype], q, q.stride(0), N, ukT, out, T, H, D, R, D, dims, inv_freq, positions)
+    return out
+
+
 def fresh_latent_ok(dtype: torch.dtype, seg, D: int, Dr: int, Dv: int) -> bool:
     """Can ``fresh_latent_attention`` run the step's prompt portions?"""
     from ._seqmix import DT, fresh_tiles_ok

@@ -48,6 +48,25 @@ def gated_token_slice(z: torch.Tensor, table: torch.Tensor, tokens: torch.Tensor
     return out
 
 
+def gated_token_project(x: torch.Tensor, w: torch.Tensor, table: torch.Tensor, tokens: torch.Tensor,
+                        col0: int) -> torch.Tensor:
+    """``gated_token_slice`` of x @ w^T; few rows gate the projection's fp32 sums in its epilogue
+    (HIP ``csrc/seqmix/thin_gemm.hip``)."""
+    from ._seqmix import DT, call
+    from .gemm import _plain, project, thin_ok
+
+    dim = w.shape[0]
+    if (thin_ok(x, w, gemv=False) and 0 <= col0 and table.dim() == 2 and col0 + dim <= table.shape[1]
+            and table.stride(1) == 1 and table.dtype == x.dtype and table.device == x.device
+            and tokens.dtype == torch.int64 and tokens.is_contiguous() and tokens.numel() == x.shape[0]
+            and tokens.device == x.device and _plain(table)):
+        out = torch.empty(x.shape[0], dim, dtype=x.dtype, device=x.device)
+        call("sm_thin_gate", DT[x.dtype], x, x.stride(0), w, out, x.shape[0], dim, x.shape[1], table[:, col0:],
+             table.stride(0), tokens)
+        return out
+    return gated_token_slice(project(x, w), table, tokens, col0)
+
+
 def embed_positions_ref(tokens, positions, table, pos_table):
     return table[tokens].float() + pos_table[positions.long()].float()
 

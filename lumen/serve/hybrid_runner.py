@@ -44,11 +44,11 @@ from ..models.config import ModelConfig
 from ..models.gedatar import DELTA_DECAY, DELTA_KEY_EPS
 from ..ops.attention import (chunk_sink_attention, diff_head_combine, fresh_latent_attention,
                              fresh_latent_ok, head_norm_rotary_write,
-                             head_norm_write, latent_write, row_attention,
+                             head_norm_write, latent_inputs, latent_query, row_attention,
                              row_norm_rotary_write, row_norm_write, transposed_values_ok,
                              write_key_cache)
 from ..ops.conv import dyt_canon, short_conv
-from ..ops.embedding import embed_positions, embed_scaled, gated_token_slice, soft_cap
+from ..ops.embedding import embed_positions, embed_scaled, gated_token_project, soft_cap
 from ..ops.gemm import project
 from ..ops.moe import (ClampedGate, dyt_residual_routed, feed_forward, moe, residual_rms_routed, routed_groups,
                        router_logits)
@@ -372,6 +372,7 @@ class DalavikWeights:
                     L.w["uq"] = t(x + "uq").detach()
                     L.w["ukv"] = torch.cat([t(x + "uk"), t(x + "uv")], 0).contiguous()
                     L.w["uk"] = L.w["ukv"][:H * D].view(H, D, R)                     # q_h @ uk[h]
+                    L.w["ukT"] = L.w["uk"].transpose(1, 2).contiguous()
                     L.w["uvT"] = t(x + "uv").detach().view(H, Dv, R).transpose(1, 2).contiguous()
                     L.w["inv_freq"] = interleaved_inv_freq(m["rot"]["dims"], m["rot"]["base"], dev)
                 else:
@@ -452,12 +453,15 @@ def run_dalavik_layers(w: DalavikWeights, st: DalavikState, tokens: torch.Tensor
             if L.kv_layer == i:
                 # the step's own cache rows, for this layer's fresh prompts and those of borrowing layers
                 own[i] = torch.empty(T, R + Dr, dtype=dt, device=x.device) if fresh else None
-                latent_write(z[:, Q:], L.w["dkv_norm"], L.w["inv_freq"], seg.positions,
-                             seg.cache_slots, st.lat[i], R, m["rot"]["dims"], eps, st.latT[i], own[i])
+                qn = latent_inputs(z, Q, L.w["dq_norm"], L.w["dkv_norm"], L.w["inv_freq"], seg.positions,
+                                   seg.cache_slots, st.lat[i], R, m["rot"]["dims"], eps, st.latT[i], own[i])
+            else:
+                qn = group_rms_norm(z[:, :Q], L.w["dq_norm"], 1, eps, dt)
             cache = st.lat[L.kv_layer]
-            q = project(group_rms_norm(z[:, :Q], L.w["dq_norm"], 1, eps, dt), L.w["uq"])
-            rotate_interleaved_(q, seg.positions, H, D + Dr, D, m["rot"]["dims"], L.w["inv_freq"])
+            q = project(qn, L.w["uq"])
             q3 = q.view(T, H, D + Dr)
+            if fresh:
+                rotate_interleaved_(q, seg.positions, H, D + Dr, D, m["rot"]["dims"], L.w["inv_freq"])
             o = torch.empty(T, H, Dv, dtype=dt, device=x.device)
             if fresh:
                 c = own[L.kv_layer][:fresh]
@@ -467,7 +471,8 @@ def run_dalavik_layers(w: DalavikWeights, st: DalavikState, tokens: torch.Tensor
             if fresh < T:
                 n, sg = T - fresh, seg.decoded() if fresh else seg
                 q3, od = q3[fresh:], o[fresh:]
-                qa = torch.bmm(q3[:, :, :D].transpose(0, 1), L.w["uk"])          # [H, T, R]
+                qa = latent_query(q3, L.w["uk"], L.w["ukT"], D, seg.positions, 0 if fresh else m["rot"]["dims"],
+                                  L.w["inv_freq"])                               # [H, T, R]
                 ol = torch.empty(H, n, R, dtype=dt, device=x.device)
                 row_attention(qa.transpose(0, 1), q3[:, :, D:], cache, cache, R, ol.transpose(0, 1),
                               sg, H, 1, float(m["scale"]), vt=st.latT[L.kv_layer])
@@ -493,7 +498,7 @@ def run_dalavik_layers(w: DalavikWeights, st: DalavikState, tokens: torch.Tensor
             xb = xc if cast is not None else x
         sd = L.side
         if sd is not None:
-            g = gated_token_slice(project(xb, sd["gate"]), w.side_embed, tokens, sd["col0"])
+            g = gated_token_project(xb, sd["gate"], w.side_embed, tokens, sd["col0"])
             x, xc = group_rms_residual(x, project(g, sd["proj"]), sd["norm"], 1, eps, cast)
             xb = xc if cast is not None else x
         if observe is not None:
@@ -750,6 +755,7 @@ class FoderaxWeights:
                     L.w["dq_norm"], L.w["dkv_norm"] = f32(x + "dq.norm"), f32(x + "dkv.norm")
                     L.w["uq"] = t(x + "uq").detach()
                     L.w["uk"] = t(x + "uk").detach().view(H, D, R)                   # q_h @ uk[h]
+                    L.w["ukT"] = L.w["uk"].transpose(1, 2).contiguous()
                     L.w["uvT"] = t(x + "uv").detach().view(H, Dv, R).transpose(1, 2).contiguous()
                     L.w["sink"] = f32(x + "sink")
                     L.w["o"] = t(x + "o").detach()
@@ -871,10 +877,9 @@ def run_foderax_layers(w: FoderaxWeights, st: FoderaxState, tokens: torch.Tensor
         elif L.kind == "latent_attention":
             H, D, Dv, R, Q = m["heads"], m["dim"], m["vdim"], m["kv_rank"], m["q_rank"]
             z = project(h, L.w["in"])
-            latent_write(z[:, Q:Q + R], L.w["dkv_norm"], None, seg.positions, seg.cache_slots,
-                         st.lat[i], R, 0, eps, st.latT[i])
-            q = project(group_rms_norm(z[:, :Q], L.w["dq_norm"], 1, eps, dt), L.w["uq"])
-            qa = torch.bmm(q.view(T, H, D).transpose(0, 1), L.w["uk"])          # [H, T, R]
+            q = project(latent_inputs(z[:, :Q + R], Q, L.w["dq_norm"], L.w["dkv_norm"], None, seg.positions,
+                                      seg.cache_slots, st.lat[i], R, 0, eps, st.latT[i]), L.w["uq"])
+            qa = latent_query(q.view(T, H, D), L.w["uk"], L.w["ukT"], D, seg.positions)          # [H, T, R]
             ol = torch.empty(H, T, R, dtype=dt, device=dev)
             row_attention(qa.transpose(0, 1), None, st.lat[i], st.lat[i], R, ol.transpose(0, 1),
                           seg, H, 1, float(m["scale"]), sink=L.w["sink"], vt=st.latT[i],

@@ -1,4 +1,4 @@
-// What a decode step's latent-attention layer does around its attention, two launches instead of four.
+// What a decode step's latent-attention layer does around its attention, three launches instead of six.
 //
 //   sm_latent_in     a row of z = [query latent Q | latent R | rotated key part Dr]: the cache row as sm_latent_write
 //                    forms it, and rms(z[:Q]) * wq.  One workgroup for each of the two, per row: as a wave of a
@@ -7,8 +7,11 @@
 //                    rows along D), and the rotated part of every head turned in place.  A wave takes 16
 //                    latent columns of a head and 64 rows, fragments straight from L2 (2 MB of weights, 16 KB of
 //                    queries a head; nothing is worth staging for one product each), all loads in flight at once.
+//   sm_latent_out    the partial sums of sm_latent_attn weighed together (or its finished rows), rounded, and expanded:
+//                    o[h] = uv[h] ol[h].  A workgroup takes 16 rows of a head; a wave asks for its 16 output columns'
+//                    weights (all of R), joins in the sums, which meet in LDS, and multiplies.
 // Bound by latency.  64 rows x 16 heads, D = 128, R = 512, in a decode step, us: write and norm 10.1 + 4.5 -> 6.2; batched
-// library product and rotation 5.1 + 4.5 -> 7.0.
+// library product and rotation 5.1 + 4.5 -> 7.0; sums of 8 splits and library product 4.9 + 12.7 -> 10.9.
 #include "seqmix.h"
 
 using namespace lumen;
@@ -126,6 +129,77 @@ __global__ void __launch_bounds__(256) latent_query_kernel(const QueryArgs<T> a)
     }
 }
 
+template <typename T> struct OutArgs {
+  const float *ml, *part; int nsplit;       // of sm_latent_attn; nsplit 1: x
+  const T* x; long long xr, xh;             // finished rows [Tn][H][R] at these strides
+  const T* gate; long long gater;
+  const T* uv;                              // [H][Dv][R]
+  T* o; long long orow, oh;
+  int Tn, H, Dv;
+};
+
+// KS: steps of 32 along R; a wave per 16 of Dv
+template <typename T, int KS>
+__global__ void __launch_bounds__(1024) latent_out_kernel(const OutArgs<T> a) {
+  constexpr int R = 32 * KS, LD = R + 8;               // (16-byte pieces of 16 rows: no bank conflicts)
+  __shared__ __attribute__((aligned(16))) T s_x[16 * LD];
+  __shared__ float s_w[16][64];
+  const int h = blockIdx.y, t0 = blockIdx.x * 16, n = min(16, a.Tn - t0);
+  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4, w = tid >> 6;
+  uint4 u[KS];
+  const T* ur = a.uv + ((long long)h * a.Dv + 16 * w + lr) * R + 8 * lg;
+#pragma unroll
+  for (int s = 0; s < KS; ++s) u[s] = *reinterpret_cast<const uint4*>(ur + 32 * s);
+  if (a.nsplit > 1) {
+    for (int i = w; i < n; i += (int)blockDim.x >> 6) {    // lane s weighs split s
+      const long long base = ((long long)(t0 + i) * a.H + h) * a.nsplit;
+      const float ms = lane < a.nsplit ? a.ml[2 * (base + lane)] : -INFINITY;
+      const float ls = lane < a.nsplit ? a.ml[2 * (base + lane) + 1] : 0.f;
+      const float M = wave_max(ms);
+      const float e = ms == -INFINITY ? 0.f : expf(ms - M);
+      float L = wave_sum(ls * e);
+      if (a.gate != nullptr) L *= 1.f + expf(-to_f32(a.gate[(long long)(t0 + i) * a.gater + h]));   // / sigmoid
+      s_w[i][lane] = e / L;
+    }
+    __syncthreads();
+  }
+  for (int x = tid; x < n * (R / 4); x += blockDim.x) {
+    const int i = x / (R / 4), c = 4 * (x % (R / 4));
+    if (a.nsplit > 1) {
+      const float* p = a.part + ((long long)(t0 + i) * a.H + h) * a.nsplit * R + c;
+      float v[4] = {0.f, 0.f, 0.f, 0.f};
+      const auto add = [&](const float4& y, float k) {
+        v[0] += y.x * k; v[1] += y.y * k; v[2] += y.z * k; v[3] += y.w * k;
+      };
+      int s = 0;
+      for (; s + 4 <= a.nsplit; s += 4) {
+        float4 y[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) y[q] = *reinterpret_cast<const float4*>(p + (long long)(s + q) * R);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) add(y[q], s_w[i][s + q]);
+      }
+      for (; s < a.nsplit; ++s) add(*reinterpret_cast<const float4*>(p + (long long)s * R), s_w[i][s]);
+      store4<T>(s_x + i * LD + c, v);
+    } else {
+      *reinterpret_cast<uint2*>(s_x + i * LD + c) =
+          *reinterpret_cast<const uint2*>(a.x + (long long)(t0 + i) * a.xr + h * a.xh + c);
+    }
+  }
+  __syncthreads();
+  f32x4 c0 = {0.f, 0.f, 0.f, 0.f}, c1 = c0;
+  const T* xr = s_x + min(lr, n - 1) * LD + 8 * lg;
+#pragma unroll
+  for (int s = 0; s < KS; s += 2) {
+    c0 = mma<T>(u[s], *reinterpret_cast<const uint4*>(xr + 32 * s), c0);
+    c1 = mma<T>(u[s + 1], *reinterpret_cast<const uint4*>(xr + 32 * s + 32), c1);
+  }
+  c0 += c1;
+  if (lr < n)                                          // lane (lr, lg): row t0 + lr, columns 16 w + 4 lg ..
+    *reinterpret_cast<uint2*>(a.o + (long long)(t0 + lr) * a.orow + h * a.oh + 16 * w + 4 * lg) =
+        make_uint2(pk2<T>(c0[0], c0[1]), pk2<T>(c0[2], c0[3]));
+}
+
 }  // namespace
 
 extern "C" {
@@ -165,6 +239,32 @@ hipError_t sm_latent_query(int dt, void* q, long long ldq, int ldh, const void* 
   else if (D == 128) GO(T, 4);             \
   else if (D == 192) GO(T, 6);             \
   else if (D == 256) GO(T, 8);             \
+  else return hipErrorInvalidValue
+  if (dt == kBF16) { GO_T(bf16); } else { GO_T(fp16); }
+#undef GO_T
+#undef GO
+  return hipGetLastError();
+}
+
+// The rows of sm_latent_attn: ml, part of nsplit > 1 splits (gate as there), or with nsplit 1 x at strides xr, xh (% 4, 8-byte
+// base).  uv [H][Dv][R], Dv % 16 == 0 up to 256, R 64, 128, 256 or 512; o at strides orow, oh (% 4, 8-byte base).
+hipError_t sm_latent_out(int dt, const float* ml, const float* part, int nsplit, const void* x, long long xr,
+                         long long xh, const void* gate, long long gater, const void* uv, void* o, long long orow,
+                         long long oh, int rows, int H, int Dv, int R, hipStream_t st) {
+  if (rows == 0) return hipSuccess;
+  if (rows < 0 || H < 1 || H > 65535 || Dv < 16 || Dv % 16 || Dv > 256 || nsplit < 1 || nsplit > 64 || !uv || !o ||
+      (uintptr_t)uv % 16 || (uintptr_t)o % 8 || orow % 4 || oh % 4 || (dt != kBF16 && dt != kF16) ||
+      (nsplit > 1 ? !ml || !part || (uintptr_t)part % 16 : !x || (uintptr_t)x % 8 || xr % 4 || xh % 4))
+    return hipErrorInvalidValue;
+  const dim3 grid((rows + 15) / 16, H);
+#define GO(T, KS)                                                                                                 \
+  latent_out_kernel<T, KS><<<grid, 4 * Dv, 0, st>>>(OutArgs<T>{ml, part, nsplit, (const T*)x, xr, xh, (const T*)gate, \
+                                                               gater, (const T*)uv, (T*)o, orow, oh, rows, H, Dv})
+#define GO_T(T)                            \
+  if (R == 64) GO(T, 2);                   \
+  else if (R == 128) GO(T, 4);             \
+  else if (R == 256) GO(T, 8);             \
+  else if (R == 512) GO(T, 16);            \
   else return hipErrorInvalidValue
   if (dt == kBF16) { GO_T(bf16); } else { GO_T(fp16); }
 #undef GO_T

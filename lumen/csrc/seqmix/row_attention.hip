@@ -1000,7 +1000,7 @@ hipError_t sm_latent_attn(int dt, const void* q1, long long q1r, long long q1h, 
   if (!sm_latent_attn_ok(dt, Dv, D1 + D2, D1, bs) || nsplit < 1 || nsplit > 64 ||
       (nsplit > 1 && (!ws_ml || !ws_o)) || krow % 8 || !al(kc) || !al(vt) || !al(q1) || q1r % 8 ||
       q1h % 8 || (D2 > 0 && (!q2 || !al(q2) || q2r % 8 || q2h % 8)) || our % 4 || ouh % 4 ||
-      (uintptr_t)out % 8)
+      (uintptr_t)out % 8 || (!out && nsplit == 1))
     return hipErrorInvalidValue;
 #define CALL(TT)                                                                              \
   {                                                                                           \
@@ -1011,7 +1011,7 @@ hipError_t sm_latent_attn(int dt, const void* q1, long long q1r, long long q1h, 
                       nullptr, 1, nsplit, ws_ml, ws_o};                                       \
     hipError_t e = launch_latent_attn<TT>(a, (const TT*)vt, T, st);                           \
     if (e != hipSuccess) return e;                                                            \
-    if (nsplit > 1)                                                                           \
+    if (nsplit > 1 && out)      /* (without: the caller adds the splits, sm_latent_out) */     \
       row_attn_combine_kernel<TT><<<dim3(T, H), 256, 0, st>>>(                                \
           ws_ml, ws_o, (TT*)out, our, ouh, H, Dv, nsplit, (const TT*)gate, gater);            \
     return hipGetLastError();                                                                 \

@@ -1034,12 +1034,25 @@ def _heads_per_block(H: int, Dk: int, need_all: bool) -> int:
 LATENT_TILE_ROWS = 2048      # rows x 16-head blocks from which prompt portions take the tiled latent kernel
 
 
+def _expand_ok(expand: tuple, q1: torch.Tensor, T: int, H: int, R: int) -> bool:
+    """Does sm_latent_out take these rows?"""
+    from .gemm import _here, _plain
+
+    uv, o = expand
+    return (T <= LATENT_STEP_MAX_T and R in (64, 128, 256, 512) and uv.dim() == 3 and uv.shape[0] == H
+            and uv.shape[2] == R and uv.shape[1] % 16 == 0 and 0 < uv.shape[1] <= 256 and uv.is_contiguous()
+            and uv.data_ptr() % 16 == 0 and uv.dtype == q1.dtype == o.dtype and tuple(o.shape) == (T, H, uv.shape[1])
+            and o.stride(2) == 1 and o.stride(0) % 4 == 0 and o.stride(1) % 4 == 0 and o.data_ptr() % 8 == 0
+            and _plain(q1, uv) and _here(q1))
+
+
 def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Tensor,
                   vcache: torch.Tensor, Dv: int, out: torch.Tensor, seg, H: int, G: int,
                   scale: float, softcap: float = 0.0, q_temp=None, r1=None, r2=None, talk=None,
                   sink=None, vt: Optional[torch.Tensor] = None, slopes=None, window: int = 0,
                   keep_first: int = 0, gate: Optional[torch.Tensor] = None,
-                  sigmoid_bias: Optional[torch.Tensor] = None, v_div: int = 1) -> torch.Tensor:
+                  sigmoid_bias: Optional[torch.Tensor] = None, v_div: int = 1,
+                  expand: Optional[tuple] = None) -> torch.Tensor:
     """Causal attention of every row of a step against paged caches.
 
     q1 [T, H, D1] and (optionally) q2 [T, H, D2] are views with arbitrary row / head strides;
@@ -1062,7 +1075,8 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
     heads) -- several score maps over the same values.  ``vt`` [blocks, Dv, block]: a per-block
     transposed copy of the values (``latent_write`` keeps one); with it, one key/value head,
     values that are a prefix of the key rows and a 16-bit dtype, the whole kernel runs on the
-    matrix cores.
+    matrix cores.  ``expand`` = (uv [H, Dv', Dv], o [T, H, Dv']): where the latent kernel serves all rows of a small
+    step, they go through ``uv`` into ``o``, which is then returned, and ``out`` is left unwritten.
 
     Several kernels serve it.  The prompt portions of a step (``seg.q_tiles``) go to the tiled
     matrix-core kernel of ``csrc/seqmix/window_attention.hip`` when the keys and values have caches
@@ -1140,12 +1154,18 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
         if nsplit > 1:
             ws_ml = torch.empty(T * H * nsplit * 2, dtype=torch.float32, device=q1.device)
             ws_o = torch.empty(T * H * nsplit * Dv, dtype=torch.float32, device=q1.device)
+        fused = expand is not None and full is out and _expand_ok(expand, q1, T, H, Dv)
         call("sm_latent_attn", DT[q1.dtype], q1, q1.stride(0), q1.stride(1), D1,
              q2, q2.stride(0) if q2 is not None else 0, q2.stride(1) if q2 is not None else 0, D2,
-             kcache, krow, vt, Dv, out, out.stride(0), out.stride(1),
+             kcache, krow, vt, Dv, None if fused and nsplit > 1 else out, out.stride(0), out.stride(1),
              seg.tables, seg.tables.shape[1], row_seg, positions, T, H, bs,
              scale, float(softcap or 0.0), coef, every, r1, r2, sink,
              gate, gate.stride(0) if gate is not None else 0, nsplit, ws_ml, ws_o)
+        if fused:
+            uv, o = expand
+            call("sm_latent_out", DT[q1.dtype], ws_ml, ws_o, nsplit, out, out.stride(0), out.stride(1), gate,
+                 gate.stride(0) if gate is not None else 0, uv, o, o.stride(0), o.stride(1), T, H, uv.shape[1], Dv)
+            return o
         return full
     # a step's prompt portions: tiles of consecutive rows of one segment on the matrix cores, when
     # nothing needs all heads of a (row, key) pair at once and the kernel has the head size; the

@@ -373,7 +373,8 @@ class DalavikWeights:
                     L.w["ukv"] = torch.cat([t(x + "uk"), t(x + "uv")], 0).contiguous()
                     L.w["uk"] = L.w["ukv"][:H * D].view(H, D, R)                     # q_h @ uk[h]
                     L.w["ukT"] = L.w["uk"].transpose(1, 2).contiguous()
-                    L.w["uvT"] = t(x + "uv").detach().view(H, Dv, R).transpose(1, 2).contiguous()
+                    L.w["uv"] = t(x + "uv").detach().view(H, Dv, R)
+                    L.w["uvT"] = L.w["uv"].transpose(1, 2).contiguous()
                     L.w["inv_freq"] = interleaved_inv_freq(m["rot"]["dims"], m["rot"]["base"], dev)
                 else:
                     L.w["qkv"] = torch.cat([t(x + n) for n in "qkv"], 0).contiguous()
@@ -474,9 +475,10 @@ def run_dalavik_layers(w: DalavikWeights, st: DalavikState, tokens: torch.Tensor
                 qa = latent_query(q3, L.w["uk"], L.w["ukT"], D, seg.positions, 0 if fresh else m["rot"]["dims"],
                                   L.w["inv_freq"])                               # [H, T, R]
                 ol = torch.empty(H, n, R, dtype=dt, device=x.device)
-                row_attention(qa.transpose(0, 1), q3[:, :, D:], cache, cache, R, ol.transpose(0, 1),
-                              sg, H, 1, float(m["scale"]), vt=st.latT[L.kv_layer])
-                torch.bmm(ol, L.w["uvT"], out=od.transpose(0, 1))
+                got = row_attention(qa.transpose(0, 1), q3[:, :, D:], cache, cache, R, ol.transpose(0, 1),
+                                    sg, H, 1, float(m["scale"]), vt=st.latT[L.kv_layer], expand=(L.w["uv"], od))
+                if got is not od:
+                    torch.bmm(ol, L.w["uvT"], out=od.transpose(0, 1))
         else:
             H, G, D, Dv = m["heads"], m["kv_heads"], m["dim"], m["vdim"]
             qkv = project(xb, L.w["qkv"], L.w["qkv_b"])
@@ -756,7 +758,8 @@ class FoderaxWeights:
                     L.w["uq"] = t(x + "uq").detach()
                     L.w["uk"] = t(x + "uk").detach().view(H, D, R)                   # q_h @ uk[h]
                     L.w["ukT"] = L.w["uk"].transpose(1, 2).contiguous()
-                    L.w["uvT"] = t(x + "uv").detach().view(H, Dv, R).transpose(1, 2).contiguous()
+                    L.w["uv"] = t(x + "uv").detach().view(H, Dv, R)
+                    L.w["uvT"] = L.w["uv"].transpose(1, 2).contiguous()
                     L.w["sink"] = f32(x + "sink")
                     L.w["o"] = t(x + "o").detach()
                     L.w["scales"] = [ls1]
@@ -881,11 +884,12 @@ def run_foderax_layers(w: FoderaxWeights, st: FoderaxState, tokens: torch.Tensor
                                       seg.cache_slots, st.lat[i], R, 0, eps, st.latT[i]), L.w["uq"])
             qa = latent_query(q.view(T, H, D), L.w["uk"], L.w["ukT"], D, seg.positions)          # [H, T, R]
             ol = torch.empty(H, T, R, dtype=dt, device=dev)
-            row_attention(qa.transpose(0, 1), None, st.lat[i], st.lat[i], R, ol.transpose(0, 1),
-                          seg, H, 1, float(m["scale"]), sink=L.w["sink"], vt=st.latT[i],
-                          gate=z[:, Q + R:Q + R + H])
             o = torch.empty(T, H, Dv, dtype=dt, device=dev)
-            torch.bmm(ol, L.w["uvT"], out=o.transpose(0, 1))
+            got = row_attention(qa.transpose(0, 1), None, st.lat[i], st.lat[i], R, ol.transpose(0, 1),
+                                seg, H, 1, float(m["scale"]), sink=L.w["sink"], vt=st.latT[i],
+                                gate=z[:, Q + R:Q + R + H], expand=(L.w["uv"], o))
+            if got is not o:
+                torch.bmm(ol, L.w["uvT"], out=o.transpose(0, 1))
             ys = [project(o.view(T, H * Dv), L.w["o"])]
         else:
             H, G, D, Dv = m["heads"], m["kv_heads"], m["dim"], m["vdim"]

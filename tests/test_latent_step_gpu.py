@@ -75,3 +75,43 @@ def test_gated_token_slice(T, W, dim, cols, dt):
         near(got, want, dt, 2 * ULP[dt])                  # (separate launches round the product as well)
     with pytest.raises(ValueError):
         gated_token_project(x, w, table, tok, cols - dim + 1)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,H,R,Dr,Dv,ctx,gated", [(1, 16, 512, 64, 128, 700, False), (17, 4, 512, 64, 64, 130, True),
+                                                   (64, 16, 512, 0, 256, 40, True), (40, 16, 256, 32, 16, 300, False),
+                                                   (300, 32, 512, 64, 48, 9, True), (5, 2, 512, 64, 24, 90, True)])
+def test_sums_and_expansion(T, H, R, Dr, Dv, ctx, gated, dt):
+    """Many splits of the keys, few, one; a size that keeps the separate product (24 columns)."""
+    from lumen.ops.attention import row_attention, transposed_values_ok
+    from lumen.ops.segments import SegBatch
+
+    g = torch.Generator(device="cuda").manual_seed(T)
+    r = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    bs, i32 = 16, dict(dtype=torch.int32, device="cuda")
+    assert transposed_values_ok(dt, R, Dr, bs, "cuda")
+    lens = torch.randint(1, ctx + 1, (T,), generator=torch.Generator().manual_seed(T))
+    lens[0] = ctx
+    per = (ctx + bs - 1) // bs
+    tables = torch.randperm(64 * per)[torch.arange(T * per) % (64 * per)].view(T, per).to(**i32)
+    cache = r(64 * per, bs, R + Dr).to(dt)
+    vt = cache[:, :, :R].transpose(1, 2).contiguous()
+    pos = (lens - 1).to(**i32)
+    ar = torch.arange(T + 1, **i32)
+    seg = SegBatch(ar, ar[:T], pos, ar[:T], pos, tables, None)
+    qa, q2 = r(H, T, R).to(dt), r(T, H, Dr).to(dt) if Dr else None
+    gate = r(T, H).to(dt) if gated else None
+    uv = (r(H, Dv, R) / R ** 0.5).to(dt)
+    kw = dict(vt=vt, gate=gate, sink=r(H) if gated else None)
+    ol = torch.empty(H, T, R, dtype=dt, device="cuda")
+    row_attention(qa.transpose(0, 1), q2, cache, cache, R, ol.transpose(0, 1), seg, H, 1, 0.05, **kw)
+    o = torch.zeros(T, H, Dv + 4, dtype=dt, device="cuda")[:, :, :Dv]
+    out = torch.empty_like(ol).transpose(0, 1)
+    got = row_attention(qa.transpose(0, 1), q2, cache, cache, R, out, seg, H, 1, 0.05, expand=(uv, o), **kw)
+    assert (got is o) == (Dv % 16 == 0)
+    if got is o:
+        # the same rows, their last bit apart where the splits' sum ends differently, through sums of R products
+        want = torch.matmul(ol.double(), uv.double().transpose(1, 2).contiguous()).transpose(0, 1)
+        near(o, want, dt, ULP[dt])
+    else:
+        assert torch.equal(got.transpose(0, 1), ol)

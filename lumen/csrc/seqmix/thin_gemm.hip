@@ -35,7 +35,8 @@
 //   dense 2048 -> 5632 (gated): 1 row 18.3 / 28.8 us, 8 rows 22.8 / 31.8, 32 rows 27.9 / 35.8
 //   16 experts of 1408, top 3, and a shared one: 1 row 17.5 / 113.9, 8 rows 49.3 / 122.3, 32 rows 88.2 /
 //   144.6; width 4096, experts of 2816: 8 rows 189.4 / 269.6, 32 rows 248.4 / 406.8
-// The gated form (thin_gate) multiplies gelu(sum) with a row of a per-token table: a launch of 4 us less per layer.
+// The gated form (thin_gate) multiplies gelu(sum) with a row of a per-token table: a launch of 4 us less per layer; thin_tail
+// turns a projection's last columns (tanh) or copies them into a cache, likewise.
 // From 33 rows on every tile re-reads more x than W, so the widest matrices stay with the library
 // there; at M = 1 the GEMV stays ahead on long rows (ops/gemm.py has the rule).
 #include "seqmix.h"
@@ -97,8 +98,12 @@ struct ThinArgs {
   GateForm form;
   // plain form (or null): y = gelu_tanh(x W^T) * table[token of the row], columns alike
   const void* table; long long ldt; const long long* tokens;
+  // plain form: tanh of the columns from tanh_from on; the columns from cache_from on once more, as rounded, to row
+  // slots[m] (>= 0) of a cache
+  int tanh_from; void* cache; long long ldc; int cache_from; const long long* slots;
 };
 
+constexpr int kNoTanh = 0x7fffffff;
 constexpr int kMaxWts = 2048;     // routing weights held in LDS (M * E)
 
 // the i-th set bit of a mask
@@ -296,6 +301,17 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] = gelu_tanh_f(v[e]) * to_f32(e4[e]);
         }
+        if (n + 3 >= p.tanh_from) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e >= p.tanh_from) v[e] = tanhf(v[e]);
+        }
+        if (p.cache != nullptr && n >= p.cache_from) {
+          const long long sl = p.slots[m];
+          if (sl >= 0)
+            *reinterpret_cast<uint2*>((T*)p.cache + sl * p.ldc + (n - p.cache_from)) =
+                make_uint2(pk2<T>(v[0], v[1]), pk2<T>(v[2], v[3]));
+        }
         if (p.out32)
           *reinterpret_cast<f32x4*>((float*)p.y + (long long)m * p.ldy + n) = v;
         else
@@ -397,6 +413,7 @@ hipError_t sm_thin_gemm(int dt, const void* x, long long ldx, const void* W, con
                          ffs < 0 || ffs % 64 || (long long)E * ff + ffs != K))
     return hipErrorInvalidValue;
   ThinArgs p{};
+  p.tanh_from = kNoTanh;
   p.x = x; p.W = W; p.bias = bias; p.y = y;
   p.M = M; p.N = N; p.K = K; p.ldx = ldx; p.ldy = ldy; p.out32 = out32;
   if (wts != nullptr) { p.wts = wts; p.E = E; p.ff = ff; p.ffs = ffs; p.sparse = 1; }
@@ -413,9 +430,30 @@ hipError_t sm_thin_gate(int dt, const void* x, long long ldx, const void* W, voi
       !tokens || ldt < N || 64LL * K * 2 >= (1LL << 32) || 64LL * ldx * 2 >= (1LL << 32))
     return hipErrorInvalidValue;
   ThinArgs p{};
+  p.tanh_from = kNoTanh;
   p.x = x; p.W = W; p.y = y;
   p.M = M; p.N = N; p.K = K; p.ldx = ldx; p.ldy = N;
   p.table = table; p.ldt = ldt; p.tokens = tokens;
+  if (dt == kBF16) return pick<bf16>(p, st);
+  if (dt == kF16) return pick<fp16>(p, st);
+  return hipErrorInvalidValue;
+}
+
+// y [M, N] = x @ W^T, the columns from tanh_from on through tanh, those from cache_from on (cache given)
+// also to row slots[m] >= 0 of cache, rows at stride ldc.  cache_from, ldc % 4, cache at 8 bytes; the rest as above.
+hipError_t sm_thin_tail(int dt, const void* x, long long ldx, const void* W, void* y, int M, int N, int K, int tanh_from,
+                        void* cache, long long ldc, int cache_from, const long long* slots, hipStream_t st) {
+  if (M == 0 || N == 0) return hipSuccess;
+  if (M < 0 || M > 64 || N < 4 || N % 4 || K < BK || K % BK || ldx < K || ldx % 8 || !aligned(x, W, y) ||
+      tanh_from < 0 || 64LL * K * 2 >= (1LL << 32) || 64LL * ldx * 2 >= (1LL << 32) ||
+      (cache && (!slots || cache_from < 0 || cache_from % 4 || cache_from >= N || ldc % 4 || ldc < N - cache_from ||
+                 (uintptr_t)cache % 8)))
+    return hipErrorInvalidValue;
+  ThinArgs p{};
+  p.tanh_from = kNoTanh;
+  p.x = x; p.W = W; p.y = y;
+  p.M = M; p.N = N; p.K = K; p.ldx = ldx; p.ldy = N;
+  p.tanh_from = tanh_from; p.cache = cache; p.ldc = ldc; p.cache_from = cache_from; p.slots = slots;
   if (dt == kBF16) return pick<bf16>(p, st);
   if (dt == kF16) return pick<fp16>(p, st);
   return hipErrorInvalidValue;
@@ -439,6 +477,7 @@ hipError_t sm_thin_act(int dt, const void* x, long long ldx, const void* W, cons
   if (sparse && (E < 1 || ff % 64 || ffs % 64)) return hipErrorInvalidValue;
   if (64LL * K * 2 >= (1LL << 32) || 64LL * ldx * 2 >= (1LL << 32)) return hipErrorInvalidValue;
   ThinArgs p{};
+  p.tanh_from = kNoTanh;
   p.x = x; p.W = W; p.y = y;
   p.M = M; p.N = (int)out; p.K = K; p.ldx = ldx; p.ldy = out;
   p.wts = wts; p.E = E; p.ff = ff; p.ffs = ffs; p.sparse = sparse;

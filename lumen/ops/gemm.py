@@ -231,6 +231,44 @@ def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = Non
     return F.linear(x, w, bias)
 
 
+def _thin_tail(x, w, tanh_from: int = 1 << 30, cache=None, cache_from: int = 0, slots=None) -> torch.Tensor:
+    from ._seqmix import DT, call, use_seqmix
+
+    use_seqmix(x)
+    (M, K), N = x.shape, w.shape[0]
+    y = torch.empty((M, N), device=x.device, dtype=x.dtype)
+    call("sm_thin_tail", DT[x.dtype], x, x.stride(0), w, y, M, N, K, tanh_from, cache,
+         N - cache_from if cache is not None else 0, cache_from, slots)
+    return y
+
+
+def project_tanh(x: torch.Tensor, w: torch.Tensor, start: int = 0) -> torch.Tensor:
+    """x @ w^T and the tanh of its columns from ``start`` on: (the columns before, which are left as they are and are
+    only valid there; the tanh's) as views or tensors of their own.  Few rows form it in the epilogue, from the fp32 sums."""
+    if 0 <= start < w.shape[0] and thin_ok(x, w):
+        y = _thin_tail(x, w, tanh_from=start)
+        return y[:, :start], y[:, start:]
+    y = project(x, w)
+    return y[:, :start], torch.tanh(y[:, start:])
+
+
+def project_write_keys(x: torch.Tensor, w: torch.Tensor, cache: torch.Tensor, slots: torch.Tensor,
+                       start: int) -> torch.Tensor:
+    """x @ w^T, whose columns from ``start`` on also go to the rows ``slots`` (-1: none) of the paged key cache
+    [blocks, block, heads, dim] (``write_key_cache``); few rows do so in the epilogue."""
+    from .attention import write_key_cache
+
+    GD = cache.shape[2] * cache.shape[3]
+    if (thin_ok(x, w) and start % 4 == 0 and 0 <= start and w.shape[0] - start == GD and GD % 4 == 0
+            and cache.is_contiguous() and cache.dtype == x.dtype and cache.device == x.device
+            and slots.dtype == torch.int64 and slots.is_contiguous() and slots.numel() == x.shape[0]
+            and slots.device == x.device and cache.data_ptr() % 8 == 0 and _plain(cache)):
+        return _thin_tail(x, w, cache=cache, cache_from=start, slots=slots)
+    y = project(x, w)
+    write_key_cache(y[:, start:], cache, slots)
+    return y
+
+
 # Decode batches 5..256: the decode-batch MFMA GEMM (kernels/decode_gemm.hip) where the measured
 # plan table (configs/kernels/decode_gemm_plans.json, written by lumen/bench/decode_gemm_probe.py) has
 # a winning (BM, BN, split-K) for the shape, hipBLASLt with the tuned table otherwise.  (Two

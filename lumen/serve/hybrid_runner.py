@@ -38,18 +38,16 @@ from dataclasses import dataclass, field, replace
 from typing import Dict, List, Optional
 
 import torch
-import torch.nn.functional as F
 
 from ..models.config import ModelConfig
 from ..models.gedatar import DELTA_DECAY, DELTA_KEY_EPS
 from ..ops.attention import (chunk_sink_attention, diff_head_combine, fresh_latent_attention,
                              fresh_latent_ok, head_norm_rotary_write,
                              head_norm_write, latent_inputs, latent_query, row_attention,
-                             row_norm_rotary_write, row_norm_write, transposed_values_ok,
-                             write_key_cache)
+                             row_norm_rotary_write, row_norm_write, transposed_values_ok)
 from ..ops.conv import dyt_canon, short_conv
 from ..ops.embedding import embed_positions, embed_scaled, gated_token_project, soft_cap
-from ..ops.gemm import project
+from ..ops.gemm import project, project_tanh, project_write_keys
 from ..ops.moe import (ClampedGate, dyt_residual_routed, feed_forward, moe, residual_rms_routed, routed_groups,
                        router_logits)
 from ..ops.norm import (SPLIT, depth_mix_norm, dyt, dyt_residual, embed_rms, gated_rms_norm,
@@ -254,28 +252,29 @@ def run_layers(w: HybridWeights, st: HybridState, tokens: torch.Tensor, seg: Seg
     cfg = w.cfg
     dt = w.dtype
     eps = cfg.rms_norm_eps
-    x = F.embedding(tokens, w.embed).float()
+    tokens = tokens.long().contiguous()
+    x = embed_scaled(tokens, w.embed, 1.0, torch.empty(tokens.shape[0], cfg.hidden_size, dtype=torch.float32,
+                                                       device=tokens.device))
     for i, L in enumerate(w.layers):
         m = L.m
         h = dyt_canon(x, L.norms["norm1"], L.canon, st.tail[i], seg, dt)
         if L.kind == "attention":
             H, G, D = m["heads"], m["kv_heads"], m["dim"]
-            qk = project(h, L.w["qk"])
-            write_key_cache(qk[:, H * D:], st.keys[i], seg.cache_slots)
+            qk = project_write_keys(h, L.w["qk"], st.keys[i], seg.cache_slots, H * D)
             o = chunk_sink_attention(qk[:, :H * D], st.keys[i], seg, H, G, D, float(m["scale"]),
                                      int(m["mask"]["size"]), eps, sink=True)
         elif L.kind == "wkv":
             H, D = m["heads"], m["dim"]
             mix = token_shift(h, L.w["mu"], st.prev[i], seg)
             rkvg = torch.bmm(mix[:4], L.w["rkvg"])
-            wl = project(torch.tanh(project(mix[4], L.w["w1"])), L.w["w2"])
+            wl = project(project_tanh(mix[4], L.w["w1"])[1], L.w["w2"])
             o = wkv_scan(rkvg[0], rkvg[1], rkvg[2], wl, rkvg[3], L.w["w0"], L.w["u"], L.w["norm"],
                          st.S[i], seg, H, D, eps)
         else:
             H, D = m["heads"], m["dim"]
             HD = H * D
-            z = project(h, L.w["in"])
-            wl = project(torch.tanh(z[:, 5 * HD:]), L.w["w2"])
+            z, wl = project_tanh(h, L.w["in"], 5 * HD)
+            wl = project(wl, L.w["w2"])
             o = delta_scan(z[:, :HD], z[:, HD:2 * HD], z[:, 2 * HD:3 * HD], wl,
                            z[:, 4 * HD:5 * HD], z[:, 3 * HD:4 * HD], L.w["w0"], L.w["a_b"],
                            L.w["norm"], st.S[i], seg, H, D, eps, DELTA_DECAY, DELTA_KEY_EPS)
@@ -440,8 +439,8 @@ def run_dalavik_layers(w: DalavikWeights, st: DalavikState, tokens: torch.Tensor
     dt = w.dtype
     eps, groups = cfg.rms_norm_eps, cfg.norm_groups
     T = tokens.shape[0]
-    xb = F.embedding(tokens, w.embed).to(dt)      # (the rows as stored are their own copy in `dt`)
-    x = xb.float()
+    tokens = tokens.long().contiguous()
+    x, _, xb = embed_rms(tokens, w.embed, 1.0, None, eps, rows=True)      # (the table's rows are their own copy in `dt`)
     cast = dt if dt != torch.float32 else None
     own: Dict[int, Optional[torch.Tensor]] = {}
     for i, L in enumerate(w.layers):

@@ -25,6 +25,121 @@ constexpr int kMaxD = 256;
 // step each (8 rows x 16 heads: 20.2 us with four and un-unrolled loads, 17.7 with eight)
 constexpr int kRowWaves = 8;
 
+// 16-bit rows of LPT = D / 8 lanes, LPT a power of two: a key is loaded once, 16 bytes a lane, for its score, its
+// square and its value.  (The form below reads a key row per lane for the scores -- 64 rows apart -- and all of them once
+// more for the values: 8 rows x 16 heads, 512 keys, 17.9 us in a decode step, bound by those reads' latency; here 12.1.)
+// kStep keys per lane group and step, the next step's in flight; every group keeps its own (max, sum, accumulator),
+// which meet in the wave and then in LDS.  Rows past the last key repeat it and count for nothing.
+constexpr int kStep = 8;
+
+template <int CTRL> __device__ __forceinline__ float row_dpp(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+}
+
+template <typename T, int LPT>
+__device__ __forceinline__ float key_dot(const uint4& a, const uint4& b) {
+  float s = 0.f;
+  if constexpr (__is_same(T, bf16)) {
+    const unsigned x[4] = {a.x, a.y, a.z, a.w}, y[4] = {b.x, b.y, b.z, b.w};
+    typedef __bf16 two __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      s = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(two, x[j]), __builtin_bit_cast(two, y[j]), s, false);
+  } else {                                   // (mixed fmas: the dot instruction need not keep subnormals)
+    const T *x = reinterpret_cast<const T*>(&a), *y = reinterpret_cast<const T*>(&b);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s = fmaf(to_f32(x[j]), to_f32(y[j]), s);
+  }
+  s += row_dpp<0xB1>(s);
+  s += row_dpp<0x4E>(s);
+  if (LPT > 4) s += row_dpp<0x141>(s);
+  if (LPT > 8) s += row_dpp<0x140>(s);
+  if (LPT > 16) s += __shfl_xor(s, 16, 64);
+  return s;
+}
+
+template <typename T, int LPT>
+__global__ void __launch_bounds__(64 * kRowWaves)
+chunk_row_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ cache, T* __restrict__ out,
+                 const int* __restrict__ tables, int maxb, const int* __restrict__ row_seg,
+                 const int* __restrict__ positions, int H, int G, int bs, float scale, float eps, int chunk, int sink) {
+  constexpr int D = 8 * LPT, KPW = 64 / LPT, KS = KPW * kRowWaves;      // keys a step of the workgroup per load
+  const int t = blockIdx.x, hd = blockIdx.y, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int g = hd / (H / G), grp = lane / LPT, part = lane % LPT;
+  const int pos = positions[t], lo = chunk > 0 ? (pos / chunk) * chunk : 0;
+  const int* tbl = tables + (long long)row_seg[t] * maxb;
+  __shared__ float s_acc[kRowWaves][D], s_m[kRowWaves], s_l[kRowWaves];
+  const int first = lo + w * KPW + grp;
+  uint4 nxt[kStep];
+  const auto load = [&](int j0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < kStep; ++u) {
+      const unsigned j = (unsigned)min(j0 + u * KS, pos), b = j / (unsigned)bs;
+      nxt[u] = *reinterpret_cast<const uint4*>(cache + (((long long)tbl[b] * bs + (j - b * bs)) * G + g) * D + 8 * part);
+    }
+  };
+  load(first);
+  const uint4 qv = *reinterpret_cast<const uint4*>(q + (long long)t * ldq + hd * D + 8 * part);
+  const float qn = scale / sqrtf(key_dot<T, LPT>(qv, qv) / D + eps);
+  const bool sinks = sink && w == 0 && grp == 0;          // the sink: a key of score 0 without a value
+  float m = sinks ? 0.f : -INFINITY, l = sinks ? 1.f : 0.f, acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int j0 = first; __any(j0 <= pos); j0 += kStep * KS) {
+    uint4 k[kStep];
+    float p[kStep], mx = m;
+#pragma unroll
+    for (int u = 0; u < kStep; ++u) k[u] = nxt[u];
+    if (__any(j0 + kStep * KS <= pos)) load(j0 + kStep * KS);
+#pragma unroll
+    for (int u = 0; u < kStep; ++u) {
+      const float s = key_dot<T, LPT>(k[u], qv) * qn * rsqrtf(key_dot<T, LPT>(k[u], k[u]) * (1.f / D) + eps);
+      p[u] = j0 + u * KS <= pos ? s : -INFINITY;
+      mx = fmaxf(mx, p[u]);
+    }
+    const float mb = mx == -INFINITY ? 0.f : mx, al = expf(m - mb);
+    m = mx;
+    l *= al;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] *= al;
+#pragma unroll
+    for (int u = 0; u < kStep; ++u) {
+      p[u] = expf(p[u] - mb);
+      l += p[u];
+      const T* v = reinterpret_cast<const T*>(&k[u]);
+      if (j0 + u * KS <= pos) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = fmaf(p[u], to_f32(v[e]), acc[e]);
+      }
+    }
+  }
+#pragma unroll
+  for (int o = LPT; o < 64; o <<= 1) {
+    const float m2 = __shfl_xor(m, o, 64), l2 = __shfl_xor(l, o, 64), M = fmaxf(m, m2);
+    const float a1 = m == -INFINITY ? 0.f : expf(m - M), a2 = m2 == -INFINITY ? 0.f : expf(m2 - M);
+    l = l * a1 + l2 * a2;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = acc[e] * a1 + __shfl_xor(acc[e], o, 64) * a2;
+    m = M;
+  }
+  if (lane < LPT) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s_acc[w][8 * part + e] = acc[e];
+    if (lane == 0) { s_m[w] = m; s_l[w] = l; }
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < D) {
+    float mt = -INFINITY, lt = 0.f, o = 0.f;
+#pragma unroll
+    for (int x = 0; x < kRowWaves; ++x) mt = fmaxf(mt, s_m[x]);
+#pragma unroll
+    for (int x = 0; x < kRowWaves; ++x) {
+      const float f = s_m[x] == -INFINITY ? 0.f : expf(s_m[x] - mt);
+      lt += s_l[x] * f;
+      o += s_acc[x][threadIdx.x] * f;
+    }
+    out[((long long)t * H + hd) * D + threadIdx.x] = from_f32<T>(o / lt);
+  }
+}
+
 template <typename T>
 __global__ void __launch_bounds__(64 * kRowWaves)
 chunk_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ cache,
@@ -570,6 +685,21 @@ hipError_t sm_chunk_attn(int dt, const void* q, long long ldq, const void* cache
   if (T == 0) return hipSuccess;
   if (D < 1 || D > kMaxD || G < 1 || H % G || bs < 1 || chunk < 0) return hipErrorInvalidValue;
   const dim3 grid(T, H);
+  if ((dt == kBF16 || dt == kF16) && (D == 32 || D == 64 || D == 128 || D == 256) && ldq % 8 == 0 &&
+      ((uintptr_t)q | (uintptr_t)cache) % 16 == 0) {
+#define ROW(TT, LPT)                                                                                                \
+  chunk_row_kernel<TT, LPT><<<grid, 64 * kRowWaves, 0, st>>>((const TT*)q, ldq, (const TT*)cache, (TT*)out, tables, \
+                                                             maxb, row_seg, positions, H, G, bs, scale, eps, chunk, sink)
+#define ROWS(TT)                 \
+  if (D == 32) ROW(TT, 4);       \
+  else if (D == 64) ROW(TT, 8);  \
+  else if (D == 128) ROW(TT, 16); \
+  else ROW(TT, 32)
+    if (dt == kBF16) { ROWS(bf16); } else { ROWS(fp16); }
+#undef ROWS
+#undef ROW
+    return hipGetLastError();
+  }
 #define CALL(TT) chunk_attn_kernel<TT><<<grid, 64 * kRowWaves, 0, st>>>((const TT*)q, ldq, (const TT*)cache, (TT*)out, tables, maxb, row_seg, positions, H, G, D, bs, scale, eps, chunk, sink)
   SM_DISPATCH(dt, CALL)
 #undef CALL

@@ -68,8 +68,11 @@ __global__ void __launch_bounds__(256, 2) row_gemv_kernel(const RowGemvArgs<T> a
     const long long row = GATED ? wave + (long long)(n >> 1) * waves + (n & 1 ? a.F : 0) : wave + (long long)n * waves;
     const T* p = a.W + row * a.K;
 #pragma unroll
-    for (int u = 0; u < KS; ++u)
-      o[u] = u + 1 < KS || 512 * u + 8 * lane < a.K ? ntload(p + 512 * u + 8 * lane) : z;
+    for (int u = 0; u < KS; ++u) {
+      // (the last step that K reaches may end within it, and need not be the last of KS)
+      if (512 * (u + 1) <= a.K) o[u] = ntload(p + 512 * u + 8 * lane);
+      else o[u] = 512 * u + 8 * lane < a.K ? ntload(p + 512 * u + 8 * lane) : z;
+    }
   };
 #pragma unroll
   for (int d = 0; d < D - 1; ++d)

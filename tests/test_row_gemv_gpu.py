@@ -43,3 +43,22 @@ def test_refusals():
                     (big, big[0], None, big.expand(8, -1).contiguous())):
             assert not row_norm_ok(*bad)
     assert not row_norm_ok(x.clone().requires_grad_(), nw, None, w)
+
+
+@pytest.mark.parametrize("K", [8, 264, 512, 1032, 2104, 2560, 3080, 4616, 5640, 6152, 7176])
+@pytest.mark.parametrize("gated", [False, True])
+def test_nothing_behind_a_row_is_read(K, gated):
+    """K well below what the kernel's form is built for: the weights lie in a larger buffer of NaN."""
+    g = torch.Generator().manual_seed(K)
+    N = 24
+    buf = torch.full((N + 40, K), float("nan"), dtype=torch.bfloat16, device="cuda")
+    w = buf[:N]
+    w.copy_(torch.randn(N, K, generator=g) * K ** -0.5)
+    x, nw = torch.randn(1, K, generator=g).bfloat16().cuda(), torch.ones(K, dtype=torch.bfloat16, device="cuda")
+    with torch.no_grad():
+        assert row_norm_ok(x, nw, None, w, gated)
+        y, _ = row_norm_linear(x, nw, 1e-5, None, w, gated)
+        ref = rms_norm(x, nw, 1e-5, None)[0].double() @ w.double().t()
+    if gated:
+        ref = torch.nn.functional.silu(ref[:, :N // 2]) * ref[:, N // 2:]
+    assert ((y.double() - ref).abs() <= 1.01 * 2.0 ** -8 * ref.abs() + 2e-5 * max(1.0, float(ref.abs().max()))).all()

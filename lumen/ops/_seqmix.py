@@ -55,6 +55,9 @@ SIGNATURES = {
     "sm_latent_in": "iplpp" "pppp" "pp" "iiiiii" "f",
     "sm_latent_query": "iplipp" "iiiiii" "pp",
     "sm_latent_out": "ippi" "pll" "pl" "p" "pll" "iiii",
+    "sm_mid_slabs": "iplpp" "iiii",
+    "sm_mid_act": "iplpp" "iiiii" "ffff",
+    "sm_slab_rms": "ipippp" "iii" "f",
     "sm_thin_tail": "iplpp" "iiii" "plip",
     "sm_thin_gate": "iplpp" "iii" "plp",
     "sm_route_rows": "ii" "pp" "pl" "ppp" "ppp" "ppp" "iii" "f" "iiiiii" "ff" "p",

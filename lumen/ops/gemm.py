@@ -138,6 +138,37 @@ def _thin(x, w, bias=None, out_dtype=None, blocks=None) -> torch.Tensor:
     return y
 
 
+MID_MAX_M = 64            # rows seqmix/mid_gemm.hip takes
+
+
+def mid_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Can the kernels of seqmix/mid_gemm.hip multiply x [M, K] with w [N, K]^T?"""
+    xs, ws = x.shape, w.shape
+    if len(xs) != 2 or not 1 < xs[0] <= MID_MAX_M or len(ws) != 2 or not x.is_cuda:
+        return False
+    K, (N, Kw), dt = xs[1], ws, x.dtype
+    if (K != Kw or K % 128 or not 0 < K < THIN_MAX_K or N % 4 or N == 0 or dt != w.dtype
+            or dt not in (torch.bfloat16, torch.float16) or x.device != w.device or not w.is_contiguous()):
+        return False
+    ld, one = x.stride()
+    return (one == 1 and ld % 8 == 0 and K <= ld < THIN_MAX_LD and (x.data_ptr() | w.data_ptr()) % 16 == 0
+            and _plain(x, w) and _here(x))
+
+
+def mid_slabs(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """fp32 sums of x @ w^T over S slices of K, [S, M, N], for operands that ``mid_ok`` has let pass.  A workgroup per
+    CU, at most eight slices (us with the norm that adds them, 64 rows: 2048 x 5632 in 4 / 8 / 16 slices 14.1 / 12.4 / 14.9,
+    1024 x 2816 10.1 / 8.6 / 9.8, 4096 x 11264 in 2 / 4 / 8 36.2 / 26.7 / 29.0, 3072 x 8448 in 4 / 5 / 8 20.7 / 19.7 / 22.3)."""
+    from ._seqmix import DT, call, use_seqmix
+
+    use_seqmix(x)
+    (M, K), N = x.shape, w.shape[0]
+    S = max(1, min(8, 256 // -(-N // 64), K // 128))
+    y = torch.empty(S, M, N, dtype=torch.float32, device=x.device)
+    call("sm_mid_slabs", DT[x.dtype], x, x.stride(0), w, y, M, N, K, S)
+    return y
+
+
 ROW_MAX_K = 8192          # K a workgroup of seqmix/row_gemv.hip holds
 
 

@@ -29,7 +29,8 @@ from typing import Optional, Union
 import torch
 import torch.nn.functional as F
 
-from .gemm import THIN_BATCH_MAX_W, THIN_MAX_K, THIN_MAX_M, _here, _plain, _thin, project, row_bias_ok, thin_ok, weights_ok
+from .gemm import (MID_MAX_M, THIN_BATCH_MAX_W, THIN_MAX_K, THIN_MAX_M, _here, _plain, _thin, mid_ok, project, row_bias_ok,
+                   thin_ok, weights_ok)
 
 
 def route_topk_ref(z: torch.Tensor, top: int) -> torch.Tensor:
@@ -371,6 +372,31 @@ def _thin_act(h, gu_w, wts, E, ff, ffs, act="silu", gated=True, weigh="output", 
     return out
 
 
+def mid_act_ok(h: torch.Tensor, gu_w: torch.Tensor, ff: int, act="silu", gated: bool = True) -> bool:
+    """Should ``mid_act`` run a dense first projection and its activation?  In the measured range, widths of 1024 on: from 33 rows on, where a round of tiles of
+    32 (ungated 64) columns is enough (us with the activation, 64 rows, before -> now: 5632 x 2048 20.3 -> 15.7, 2816 x
+    1024 13.0 -> 8.8, 4224 x 1536 17.3 -> 12.1; 264 tiles, 8448 x 3072, 34.9 -> 38.1); from 17 on if the tiles also fill half
+    the chip (17 rows: 132 tiles 11.6 -> 10.2, 176 14.5 -> 13.5, 88 6.2 -> 7.8)."""
+    M = h.shape[0]
+    tiles = -(-ff // (32 if gated else 64))
+    return (16 < M <= MID_MAX_M and 0 < tiles <= 256 and (M > THIN_ACT_MAX_M or tiles >= 128) and ff % 4 == 0
+            and h.shape[-1] >= 1024 and (gated or isinstance(act, str)) and gu_w.shape[0] == (2 if gated else 1) * ff
+            and (ff + 64) * h.shape[-1] < 1 << 31 and mid_ok(h, gu_w))
+
+
+def mid_act(h, gu_w, ff: int, act="silu", gated: bool = True) -> torch.Tensor:
+    """act(gate) * up (or act) of h @ gu_w^T, [M, ff], from the fp32 sums, for operands that ``mid_act_ok`` has let pass."""
+    from ._seqmix import DT, call, use_seqmix
+
+    use_seqmix(h)
+    M, K = h.shape
+    out = torch.empty((M, ff), dtype=h.dtype, device=h.device)
+    code, c = (GATE_ACTS[act], (0.0,) * 4) if isinstance(act, str) else (
+        4, (act.limit, act.limit_shared, act.slope, act.shift))
+    call("sm_mid_act", DT[h.dtype], h, h.stride(0), gu_w, out, M, ff, K, int(gated), code, *c)
+    return out
+
+
 def moe_dense(h, wts, gu_w, down_w, E: int, ff: int, ffs: int, act="silu", gated: bool = True,
               weigh: str = "output", top: Optional[int] = None) -> torch.Tensor:
     """``top`` (optional): every row has at most that many non-zero weights."""
@@ -391,9 +417,17 @@ def moe_dense(h, wts, gu_w, down_w, E: int, ff: int, ffs: int, act="silu", gated
 def feed_forward(h, gu_w, down_w, ff: int, act="silu", gated: bool = True) -> torch.Tensor:
     """Dense feed-forward W_down (act(W_gate h) * W_up h) ([gate | up] rows stacked in ``gu_w``), or
     without a gate W_down act(W_up h)."""
-    if h.shape[0] <= THIN_ACT_MAX_M and thin_act_ok(h, None, gu_w, 0, 0, ff, act, gated):
-        return project(_thin_act(h, gu_w, None, 0, 0, ff, act, gated), down_w)
-    return project(_act(project(h, gu_w), None, 0, 0, ff, act, gated, "output"), down_w)
+    return project(ff_act(h, gu_w, ff, act, gated), down_w)
+
+
+def ff_act(h, gu_w, ff: int, act="silu", gated: bool = True) -> torch.Tensor:
+    """The first half of ``feed_forward``: act(W_gate h) * W_up h, or act(W_up h)."""
+    if h.dim() == 2 and h.shape[0] <= MID_MAX_M:
+        if mid_act_ok(h, gu_w, ff, act, gated):
+            return mid_act(h, gu_w, ff, act, gated)
+        if h.shape[0] <= THIN_ACT_MAX_M and thin_act_ok(h, None, gu_w, 0, 0, ff, act, gated):
+            return _thin_act(h, gu_w, None, 0, 0, ff, act, gated)
+    return _act(project(h, gu_w), None, 0, 0, ff, act, gated, "output")
 
 
 def moe_grouped(h, wts, gu_w, down_w, E: int, ff: int, ffs: int, act="silu", gated: bool = True,

@@ -184,6 +184,27 @@ def group_rms_residual(x: torch.Tensor, y: torch.Tensor, w: torch.Tensor, groups
     return x, xb
 
 
+def project_group_rms(x: torch.Tensor, a: torch.Tensor, proj: torch.Tensor, w: torch.Tensor, groups: int, eps: float,
+                      cast=None) -> tuple:
+    """``group_rms_residual`` of y = a @ proj^T.  2 - 64 rows: the projection's fp32 sums over slices of K meet in the
+    norm (``csrc/seqmix/mid_gemm.hip``; us, both launches, before -> now: 8 rows 2048 x 5632 12.3 -> 10.3, 2048 x 2048 8.6 ->
+    7.7, 64 rows 21.7 -> 12.4, 11.8 -> 9.7, 2048 x 128 6.7 -> 5.9, 4096 x 11264 40.7 -> 26.7)."""
+    from ._seqmix import DT, call
+    from .gemm import _plain, mid_ok, mid_slabs, project
+
+    N = proj.shape[0]
+    if (mid_ok(a, proj) and N <= 8192 and N % groups == 0 and (N // groups) % 256 == 0 and x.shape == (a.shape[0], N)
+            and x.dtype == torch.float32 and x.is_contiguous() and x.device == a.device and x.data_ptr() % 16 == 0
+            and w.dtype == torch.float32 and w.is_contiguous() and w.numel() == N and w.device == a.device
+            and w.data_ptr() % 16 == 0 and cast in (None, torch.float32, torch.bfloat16, torch.float16) and _plain(x, w)):
+        y = mid_slabs(a, proj)
+        xb = torch.empty(x.shape, dtype=cast, device=x.device) if cast not in (None, torch.float32) else None
+        call("sm_slab_rms", DT[cast if xb is not None else torch.float32], y, y.shape[0], w, x, xb, x.shape[0], N, groups,
+             eps)
+        return x, xb
+    return group_rms_residual(x, project(a, proj), w, groups, eps, cast)
+
+
 # ---- layer norm with a weight (and optionally a shift), fused with a scaled residual add ----------
 # LN(x) = (x - mean) / sqrt(mean((x - mean)^2) + eps) * w (+ b).  The fp32 residual stream takes a
 # sublayer's output multiplied by a constant, x += mult * y, and the same pass produces the next

@@ -48,11 +48,11 @@ from ..ops.attention import (chunk_sink_attention, diff_head_combine, fresh_late
 from ..ops.conv import dyt_canon, short_conv
 from ..ops.embedding import embed_positions, embed_scaled, gated_token_project, soft_cap
 from ..ops.gemm import project, project_tanh, project_write_keys
-from ..ops.moe import (ClampedGate, dyt_residual_routed, feed_forward, moe, residual_rms_routed, routed_groups,
+from ..ops.moe import (ClampedGate, dyt_residual_routed, feed_forward, ff_act, moe, residual_rms_routed, routed_groups,
                        router_logits)
 from ..ops.norm import (SPLIT, depth_mix_norm, dyt, dyt_residual, embed_rms, gated_rms_norm,
-                        group_rms_norm, group_rms_residual, hyper_mix, hyper_start, parts_rms,
-                        residual_rms, scaled_residual_layer_norm, weight_layer_norm)
+                        group_rms_norm, hyper_mix, hyper_start, parts_rms,
+                        project_group_rms, residual_rms, scaled_residual_layer_norm, weight_layer_norm)
 from ..ops.recurrent import delta_scan, head_scan, min_gru_scan, token_shift, wkv_scan
 from ..ops.rope import rotary_write, rotate_interleaved_
 from ..ops.segments import SegBatch, whole_prompts, whole_sequences
@@ -489,18 +489,17 @@ def run_dalavik_layers(w: DalavikWeights, st: DalavikState, tokens: torch.Tensor
                           float(m["scale"]), float(m.get("softcap") or 0.0),
                           (float(qt["coef"]), int(qt["every"])) if qt else None,
                           L.w["r1"], L.w["r2"], L.w["talk"], L.w["sink"])
-        y = project(o.view(T, H * Dv), L.w["o"])
-        x, xc = group_rms_residual(x, y, L.norm1, groups, eps, cast)
+        x, xc = project_group_rms(x, o.view(T, H * Dv), L.w["o"], L.norm1, groups, eps, cast)
         xb = xc if cast is not None else x
         f = L.ff
         if f is not None:
-            y = feed_forward(xb, f["gu"], f["down"], f["ff"], "relu")
-            x, xc = group_rms_residual(x, y, f["norm"], groups, eps, cast)
+            a = ff_act(xb, f["gu"], f["ff"], "relu")
+            x, xc = project_group_rms(x, a, f["down"], f["norm"], groups, eps, cast)
             xb = xc if cast is not None else x
         sd = L.side
         if sd is not None:
             g = gated_token_project(xb, sd["gate"], w.side_embed, tokens, sd["col0"])
-            x, xc = group_rms_residual(x, project(g, sd["proj"]), sd["norm"], 1, eps, cast)
+            x, xc = project_group_rms(x, g, sd["proj"], sd["norm"], 1, eps, cast)
             xb = xc if cast is not None else x
         if observe is not None:
             observe(i, x)

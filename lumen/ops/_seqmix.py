@@ -48,6 +48,7 @@ SIGNATURES = {
     "sm_expert_act": "iplp" "ppppp" "iiiiii" "iii" "ffff",
     "sm_expert_down": "ippp" "pp" "ppp" "iiiiii",
     "sm_row_gemv": "ipppppp" "iii" "f",
+    "sm_row_stream": "ippppppp" "iiii" "f",
     "sm_row_norm_write": "iplpppppiiif",
     "sm_layer_norm": "iippfpppiif",
     "sm_embed_pos": "ipppppiiii",

@@ -202,6 +202,39 @@ def row_norm_linear(x: torch.Tensor, norm_w: torch.Tensor, eps: float, res: Opti
     return y, s
 
 
+def row_stream_ok(x: torch.Tensor, y: Optional[torch.Tensor], norm_w: torch.Tensor, w: torch.Tensor,
+                  bias: Optional[torch.Tensor] = None) -> bool:
+    """Can ``row_stream_linear`` run: one fp32 row ``x`` and its norm's weight, ``y``, ``w`` and ``bias`` of one 16-bit type?"""
+    xs = x.shape
+    if len(xs) != 2 or xs[0] != 1 or not x.is_cuda or w.dim() != 2 or w.dtype not in (torch.bfloat16, torch.float16):
+        return False
+    K, (N, Kw), dt = xs[1], w.shape, w.dtype
+    if K != Kw or K % 8 or not 0 < K <= ROW_MAX_K or N == 0 or tuple(norm_w.shape) != (K,) \
+            or x.dtype != torch.float32 or norm_w.dtype != torch.float32:
+        return False
+    ts = (x, norm_w, w) if y is None else (x, norm_w, w, y)
+    return (all(t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in ts)
+            and (y is None or y.shape == xs and y.dtype == dt)
+            and (bias is None or row_bias_ok(bias, w, N) and _plain(bias)) and _plain(*ts) and _here(x) and use_native(x))
+
+
+def row_stream_linear(x: torch.Tensor, y: Optional[torch.Tensor], norm_w: torch.Tensor, eps: float, w: torch.Tensor,
+                      bias: Optional[torch.Tensor] = None, act: Optional[str] = None, out32: bool = False) -> tuple:
+    """(z, s) of one row of an fp32 stream that a sublayer's output ``y`` joins: s = x + y (x itself without one), z = act(w
+    rms_norm(s) + bias), in w's type or (``out32``) fp32.  For operands that ``row_stream_ok`` has let pass.  (HIP
+    ``csrc/seqmix/row_gemv.hip``.)"""
+    from ._seqmix import DT, call, use_seqmix
+    from .moe import GATE_ACTS
+
+    use_seqmix(x)
+    K, N = x.shape[1], w.shape[0]
+    z = torch.empty((1, N), device=x.device, dtype=torch.float32 if out32 else w.dtype)
+    s = torch.empty_like(x) if y is not None else x
+    call("sm_row_stream", DT[w.dtype], x, y, norm_w, s if y is not None else None, w, bias, z, K, N,
+         -1 if act is None else GATE_ACTS[act], int(out32), eps)
+    return z, s
+
+
 # Split-K GEMM (kernels/split_gemm.hip): long contractions over a few hundred rows, whose output has too few
 # tiles to fill the chip.  us, library -> split: K = 11008, N = 4096, rows 72 / 256 / 512 / 1000: 41 -> 32, 51 ->
 # 35, 72 -> 50, 113 -> 87; K = 22016 at 512: 139 (tuned) -> 91; K = 32000 at 512: 290 -> 123; K = 11264, N = 2048 at

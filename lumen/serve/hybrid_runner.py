@@ -47,7 +47,7 @@ from ..ops.attention import (chunk_sink_attention, diff_head_combine, fresh_late
                              row_norm_rotary_write, row_norm_write, transposed_values_ok)
 from ..ops.conv import dyt_canon, short_conv
 from ..ops.embedding import embed_positions, embed_scaled, gated_token_project, soft_cap
-from ..ops.gemm import project, project_tanh, project_write_keys
+from ..ops.gemm import project, project_tanh, project_write_keys, row_stream_linear, row_stream_ok
 from ..ops.moe import (ClampedGate, dyt_residual_routed, feed_forward, ff_act, moe, residual_rms_routed, routed_groups,
                        router_logits)
 from ..ops.norm import (SPLIT, depth_mix_norm, dyt, dyt_residual, embed_rms, gated_rms_norm,
@@ -1270,6 +1270,8 @@ class TazulixWeights:
         return run_tazulix_layers(self, st, tokens, seg, observe)
 
     def head(self, x: torch.Tensor) -> torch.Tensor:
+        if row_stream_ok(x, None, self.final, self.lm_head):
+            return row_stream_linear(x, None, self.final, self.cfg.rms_norm_eps, self.lm_head, out32=True)[0]
         h = group_rms_norm(x, self.final, 1, self.cfg.rms_norm_eps, self.dtype)
         return router_logits(h, self.lm_head)     # fp32 logits from the 16-bit (or fp32) operands
 
@@ -1297,22 +1299,20 @@ class TazulixState:
                                                        dtype=torch.float32, device=device))
 
 
-def _tazulix_mixer(L: TazulixLayerW, w: TazulixWeights, st: TazulixState, n: int, h, seg):
-    """Pass ``n``'s mixer on its normed input h [T, W]."""
+def _tazulix_mixer(L: TazulixLayerW, w: TazulixWeights, st: TazulixState, n: int, z, seg):
+    """Pass ``n``'s mixer on the projection z of its normed input."""
     m, dt, eps = L.m, w.dtype, w.cfg.rms_norm_eps
-    T = h.shape[0]
+    T = z.shape[0]
     H, D, Dv = m["heads"], m["dim"], m["vdim"]
     if L.kind == "attention":
         G = m["kv_heads"]
-        z = project(h, L.w["in"], L.w["in_b"])
         row_norm_rotary_write(z, L.w["q.norm"], L.w["k.norm"], seg.positions, seg.cache_slots,
                               st.k[n], st.v[n], H, G, D, Dv, L.rot_dims, L.w["inv_freq"], L.amp,
                               eps)
-        o = torch.empty(T, H, Dv, dtype=dt, device=h.device)
+        o = torch.empty(T, H, Dv, dtype=dt, device=z.device)
         row_attention(z[:, :H * D].view(T, H, D), None, st.k[n], st.v[n], Dv, o, seg, H, G,
                       float(m["scale"]))
         return project(o.view(T, H * Dv), L.w["o"])
-    z = project(h, L.w["in"])
     q0, k0, v0, g0 = L.cols
     y = head_scan(z[:, q0:q0 + H * D], z[:, k0:k0 + H * D], z[:, v0:v0 + H * Dv], st.S[n], seg, H,
                   D, Dv, L.w["log_decay"], silu_in=True)
@@ -1320,13 +1320,16 @@ def _tazulix_mixer(L: TazulixLayerW, w: TazulixWeights, st: TazulixState, n: int
     return project(y, L.w["o"])
 
 
-def _tazulix_ff(f: dict, x, y, eps: float) -> torch.Tensor:
-    """The mixer's output ``y`` joins the stream ``x``; the feed-forward of the normed rows."""
+def _tazulix_ff(f: dict, x, y, eps: float) -> tuple:
+    """The mixer's output ``y`` joins the stream ``x``; the feed-forward of the normed rows.  (The stream, the result.)"""
     if not f["E"]:
-        return feed_forward(residual_rms(x, y, f["norm"], eps), f["up"], f["down"], f["ff"], "relu2", gated=False)
+        if row_stream_ok(x, y, f["norm"], f["up"]):
+            a, x = row_stream_linear(x, y, f["norm"], eps, f["up"], act="relu2")
+            return x, project(a, f["down"])
+        return x, feed_forward(residual_rms(x, y, f["norm"], eps), f["up"], f["down"], f["ff"], "relu2", gated=False)
     # the router in fp32, on the (possibly 16-bit rounded) normed row
     h, r = residual_rms_routed(x, y, f["norm"], eps, f["router"], f["top"], normalize=False)
-    return moe(h, r, f["gu"], f["down"], f["E"], f["top"], f["ff"], f["ffs"], f["act"],
+    return x, moe(h, r, f["gu"], f["down"], f["E"], f["top"], f["ff"], f["ffs"], f["act"],
                weigh="input")
 
 
@@ -1345,15 +1348,22 @@ def run_tazulix_layers(w: TazulixWeights, st: TazulixState, tokens: torch.Tensor
     looped = any(w.starts)
     x, h, e = embed_rms(tokens, w.embed, w.scale, want(0), eps, rows=looped)
     p = router_logits(e, w.loop_e) if looped else None
+    z = None                                  # the next pass's projection, where the norm came with it
     for n, i in enumerate(w.runs):
         L = w.layers[i]
         if w.starts[n]:
             x, h = parts_rms(router_logits(h, w.loop_x), p, w.scale, L.norm1, eps, w.dtype)
-        y = _tazulix_mixer(L, w, st, n, h, seg)
-        if L.ff is None:
-            h = residual_rms(x, y, want(n + 1), eps)
-        else:
-            h = residual_rms(x, _tazulix_ff(L.ff, x, y, eps), want(n + 1), eps)
+        y = _tazulix_mixer(L, w, st, n, project(h, L.w["in"], L.w.get("in_b")) if z is None else z, seg)
+        z = None
+        if L.ff is not None:
+            x, y = _tazulix_ff(L.ff, x, y, eps)
+        nxt = want(n + 1)
+        if isinstance(nxt, torch.Tensor) and x.shape[0] == 1:
+            M = w.layers[w.runs[n + 1]].w
+            if row_stream_ok(x, y, nxt, M["in"], M.get("in_b")):
+                z, x = row_stream_linear(x, y, nxt, eps, M["in"], M.get("in_b"))
+        if z is None:
+            h = residual_rms(x, y, nxt, eps)
         if observe is not None:
             observe(n, x)
     return x

@@ -62,3 +62,33 @@ def test_nothing_behind_a_row_is_read(K, gated):
     if gated:
         ref = torch.nn.functional.silu(ref[:, :N // 2]) * ref[:, N // 2:]
     assert ((y.double() - ref).abs() <= 1.01 * 2.0 ** -8 * ref.abs() + 2e-5 * max(1.0, float(ref.abs().max()))).all()
+
+
+@pytest.mark.parametrize("dtype,ulp", [(torch.bfloat16, 2.0 ** -8), (torch.float16, 2.0 ** -11)])
+@pytest.mark.parametrize("K,N", [(8, 3), (520, 12), (1024, 4096), (2048, 20000), (2104, 65), (3072, 52), (5640, 32), (8192, 4100)])
+def test_row_of_a_stream(K, N, dtype, ulp):
+    """An fp32 row that a sublayer's output joins, or alone; bias, activation, fp32 results."""
+    from lumen.ops.gemm import row_stream_linear, row_stream_ok
+
+    g = torch.Generator().manual_seed(K + N)
+    f = lambda *s: torch.randn(*s, generator=g).cuda()  # noqa: E731
+    x, y, nw, w, b = 3 * f(1, K), f(1, K).to(dtype), 1 + 0.1 * f(K), (f(N, K) * K ** -0.5).to(dtype), f(N).to(dtype)
+    for yy, bias, act, out32 in ((y, None, None, False), (y, b, "relu2", False), (None, None, None, True), (y, b, "silu", True)):
+        keep = x.clone()
+        with torch.no_grad():
+            assert row_stream_ok(x, yy, nw, w, bias)
+            z, s = row_stream_linear(x, yy, nw, 1e-6, w, bias, act, out32)
+        assert torch.equal(x, keep) and (s is x if yy is None else torch.equal(s, x + yy.float()))
+        n = s.double() / torch.sqrt(s.double().square().mean(-1, keepdim=True) + 1e-6) * nw.double()
+        # the normed row is rounded once: a neighbour of the float64 one where they lie on both sides of a tie
+        ref = n.float().to(dtype).double() @ w.double().t()
+        flip = ulp * 2.0 ** -10 * (n.abs() @ w.double().abs().t())
+        ref = ref + (0 if bias is None else bias.double())
+        if act:
+            ref = torch.relu(ref) ** 2 if act == "relu2" else torch.nn.functional.silu(ref)
+        assert z.dtype == (torch.float32 if out32 else dtype)
+        tol = (0 if out32 else 1.01 * ulp * ref.abs()) + (2e-5 + 4 * flip.max()) * max(1.0, float(ref.abs().max()))
+        assert ((z.double() - ref).abs() <= tol).all(), (z.double() - ref).abs().max()
+    assert not row_stream_ok(x, y.float(), nw, w) and not row_stream_ok(x.to(dtype), y, nw, w)
+    assert not row_stream_ok(x, y, nw.to(dtype), w) and not row_stream_ok(x, y, nw, w, b[:-1])
+    assert not row_stream_ok(x.expand(2, K), None, nw, w)

@@ -509,31 +509,35 @@ def chosen_ok(h, wts, gu_w, down_w, E: int, top: int, ff: int, ffs: int, act="si
 
 
 def moe_chosen(h, wts, gu_w, down_w, E: int, top: int, ff: int, ffs: int, act="silu", gated: bool = True,
-               weigh: str = "output") -> torch.Tensor:
+               weigh: str = "output", checked: bool = False) -> torch.Tensor:
     """The weighted sum of each row's chosen experts (+ the shared one) on the rows that chose them: HIP kernels that
     read the rows where they lie and the counts on the device (seqmix/expert_gemm.hip).  A row has at most ``top``
-    non-zero weights.  Results of an expert stay fp32 until their sum is rounded."""
+    non-zero weights.  Results of an expert stay fp32 until their sum is rounded.  ``checked``: ``chosen_ok`` has let
+    these operands pass."""
     from ._seqmix import DT, call
 
     if weigh not in ("output", "input"):
         raise ValueError(f"unknown place of the routing weight {weigh!r}")
-    if not chosen_ok(h, wts, gu_w, down_w, E, top, ff, ffs, act, gated, weigh):
+    if not (checked or chosen_ok(h, wts, gu_w, down_w, E, top, ff, ffs, act, gated, weigh)):
         raise ValueError("chosen experts: rows, stacked weights and routing weights do not fit the kernels")
     T, W = h.shape
     dev, dt = h.device, DT[h.dtype]
     n = T * top
-    ints = torch.empty(2 * n + E + 1, dtype=torch.int32, device=dev)
-    idx, place, off = ints[:n], ints[n:2 * n], ints[2 * n:]
-    wt = torch.empty(n, dtype=torch.float32, device=dev)
+    # one buffer for what lies between the launches, its parts by address (short prompts wait for the host)
+    sizes = (n * ff * 2, T * ffs * 2, n * W * 4, T * W * 4 if ffs else 0, 4 * n, 4 * n, 4 * n, 4 * (E + 1))
+    at = [0]
+    for b in sizes:
+        at.append(at[-1] + (b + 255 & ~255))
+    ws = torch.empty(at[-1], dtype=torch.uint8, device=dev)
+    p0 = ws.data_ptr()
+    a, a_s, y, y_s, idx, place, wt, off = (p0 + o for o in at[:-1])
+    if not ffs:
+        a_s = y_s = None
     call("sm_expert_sort", wts, off, idx, wt, place, T, E, top)
-    a = torch.empty(n, ff, dtype=h.dtype, device=dev)
-    a_s = torch.empty(T, ffs, dtype=h.dtype, device=dev) if ffs else None
     code, c = (GATE_ACTS[act], (0.0,) * 4) if isinstance(act, str) else (
         4, (act.limit, act.limit_shared, act.slope, act.shift))
     call("sm_expert_act", dt, h, h.stride(0), gu_w, off, idx, wt, a, a_s, T, W, E, top, ff, ffs, int(gated), code,
          int(weigh == "input"), *c)
-    y = torch.empty(n, W, dtype=torch.float32, device=dev)
-    y_s = torch.empty(T, W, dtype=torch.float32, device=dev) if ffs else None
     out = torch.empty(T, W, dtype=h.dtype, device=dev)
     call("sm_expert_down", dt, a, a_s, down_w, off, place, y, y_s, out, T, W, E, top, ff, ffs)
     return out
@@ -574,7 +578,7 @@ def moe(h, wts, gu_w, down_w, E: int, top: int, ff: int, ffs: int, act="silu",
     alone.  ``weigh`` = "input": an expert sees its weight times h instead of weighing in with its
     output (gated experts)."""
     if chosen_pays(h.shape[0], gu_w) and chosen_ok(h, wts, gu_w, down_w, E, top, ff, ffs, act, gated, weigh):
-        return moe_chosen(h, wts, gu_w, down_w, E, top, ff, ffs, act, gated, weigh)
+        return moe_chosen(h, wts, gu_w, down_w, E, top, ff, ffs, act, gated, weigh, True)
     grouped = (grouped_pays(h.shape[0], E, top, (2 if gated else 1) * ff * h.shape[1])
                and not (h.is_cuda and torch.cuda.is_current_stream_capturing()))
     if grouped and grouped_mm_ok(h, ff):

@@ -336,6 +336,8 @@ class DalavikWeights:
     into one GEMM, the per-head up projections are laid out for batched GEMMs, norm weights and
     the attention's per-head constants are fp32."""
 
+    asks_fresh = True          # latent attention of whole prompts
+
     def __init__(self, model, tp_rank: int = 0, tp_size: int = 1):
         if tp_size != 1:
             raise NotImplementedError("Dalavik models are served at tensor-parallel size 1")
@@ -1408,7 +1410,9 @@ class HybridRunner(ModelRunner):
     @torch.no_grad()
     def execute(self, inp: StepInput) -> torch.Tensor:
         seg = inp.seg
-        if not seg.fresh and whole_prompts(inp.cu_seqlens, inp.kv_lens, seg.tile_rows):
+        # (short prompts wait for the host: asked where a layer makes use of it)
+        if getattr(self.w, "asks_fresh", False) and not seg.fresh \
+                and whole_prompts(inp.cu_seqlens, inp.kv_lens, seg.tile_rows):
             seg = replace(seg, fresh=True)
         x = self.w.run_layers(self.state, inp.tokens, seg, self.observe)
         if inp.extra_rows is not None and inp.extra_rows.numel():

@@ -329,6 +329,7 @@ class DalavikLayerW:
     ff: Optional[dict] = None       # gu [2 ff, W], down [W, ff], ff, norm
     side: Optional[dict] = None     # gate [d, W], proj [W, d], norm [W], col0
     kv_layer: int = -1              # latent attention: the layer whose cache rows it reads
+    readers: Dict[int, tuple] = field(default_factory=dict)   # an owner's: {layer: (dim, rot_dim, vdim)} reading its rows
 
 
 class DalavikWeights:
@@ -365,6 +366,7 @@ class DalavikWeights:
                     H, D, Dv, R = m["heads"], m["dim"], m["vdim"], m["kv_rank"]
                     own = m.get("kv_from") is None
                     L.kv_layer = i if own else int(m["kv_from"])
+                    (L if own else self.layers[L.kv_layer]).readers[i] = (D, m["rot_dim"], Dv)
                     L.w["down"] = (torch.cat([t(x + "dq"), t(x + "dkv")], 0).contiguous()
                                    if own else t(x + "dq").detach())
                     L.w["dq_norm"] = f32(x + "dq.norm")
@@ -453,8 +455,10 @@ def run_dalavik_layers(w: DalavikWeights, st: DalavikState, tokens: torch.Tensor
             z = project(xb, L.w["down"])
             fresh = seg.tile_rows if fresh_latent_ok(dt, seg, D, Dr, Dv) else 0
             if L.kv_layer == i:
-                # the step's own cache rows, for this layer's fresh prompts and those of borrowing layers
-                own[i] = torch.empty(T, R + Dr, dtype=dt, device=x.device) if fresh else None
+                # the step's own cache rows, for the fresh prompts of this layer and of borrowing layers,
+                # whose heads may have other sizes
+                keep = any(fresh_latent_ok(dt, seg, *d) for d in L.readers.values())
+                own[i] = torch.empty(T, R + Dr, dtype=dt, device=x.device) if keep else None
                 qn = latent_inputs(z, Q, L.w["dq_norm"], L.w["dkv_norm"], L.w["inv_freq"], seg.positions,
                                    seg.cache_slots, st.lat[i], R, m["rot"]["dims"], eps, st.latT[i], own[i])
             else:
@@ -480,6 +484,8 @@ def run_dalavik_layers(w: DalavikWeights, st: DalavikState, tokens: torch.Tensor
                                     sg, H, 1, float(m["scale"]), vt=st.latT[L.kv_layer], expand=(L.w["uv"], od))
                 if got is not od:
                     torch.bmm(ol, L.w["uvT"], out=od.transpose(0, 1))
+            if i == max(w.layers[L.kv_layer].readers):
+                own.pop(L.kv_layer, None)
         else:
             H, G, D, Dv = m["heads"], m["kv_heads"], m["dim"], m["vdim"]
             qkv = project(xb, L.w["qkv"], L.w["qkv_b"])

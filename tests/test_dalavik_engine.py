@@ -143,6 +143,26 @@ def test_whole_prompt_matches_oracle(device, name):
     check(m(torch.tensor(toks, device=device))[0].cpu(), want)
 
 
+@pytest.mark.parametrize("sizes", [(64, 128), (128, 64), (128, 128), (64, 64)])
+def test_borrower_with_heads_of_its_own(sizes, monkeypatch):
+    """A whole prompt where the owner of a cache and its borrower differ in whether they expand fresh prompts: the
+    borrower's expanded form takes the owner's rows."""
+    import lumen.serve.hybrid_runner as R
+
+    cfg = _cfg("mixed", 90, 48, 1, 0, 1e-5, [
+        _lat(2, sizes[0], 64, sizes[0], 40, 24, 0.1, 777.0, 8, None),
+        _lat(1, sizes[1], 64, sizes[1], 40, 16, 0.1, 777.0, 8, _ff(24), kv_from=0)])
+    m = DalavikForCausalLM(cfg, dtype=torch.float32, device="cpu")
+    m.init_weights(seed=4)
+    expanded, real = [], R.fresh_latent_attention
+    monkeypatch.setattr(R, "fresh_latent_ok",     # (as on the GPU)
+                        lambda dtype, seg, D, Dr, Dv, *a: seg.fresh and (D, Dr, Dv) == (128, 64, 128))
+    monkeypatch.setattr(R, "fresh_latent_attention", lambda *a: (expanded.append(1), real(*a))[1])
+    toks = tokens(m, 23, 5)
+    check(replay_alone(m, "cpu", toks, [23]), Oracle(m).forward(toks))
+    assert len(expanded) == sizes.count(128)
+
+
 @pytest.mark.parametrize("device", DEVICES)
 def test_residual_stream_after_every_layer(device):
     """The runner's per-layer hook against the oracle's stream: a fault shows at its layer."""

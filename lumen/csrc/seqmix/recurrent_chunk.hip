@@ -81,20 +81,6 @@ template <typename T> struct ScanArgs {
   float decay_scale, key_eps;
 };
 
-// e^x for x up to 88 (more: as 88; below -200: 0) from the hardware's 2^t, the rounding of t made good; and 1 / (1 +
-// e^-x) with one refinement of the hardware's reciprocal.  As near as expf and an exact division (state's error against
-// float64 unchanged), at a third of their instructions, which bounded the producers (5.8 -> 4.8 thousand cycles a chunk).
-__device__ __forceinline__ float exp_near(float x) {
-  constexpr float kL = 1.44269502f, kLlo = 1.92596299e-8f;     // log2(e) = kL + kLlo
-  x = x < -200.f ? -200.f : x > 88.f ? 88.f : x;               // (NaN stays)
-  const float t = x * kL, lo = fmaf(x, kLlo, fmaf(x, kL, -t));
-  const float r = __builtin_amdgcn_exp2f(t);
-  return fmaf(r, lo * 0.693147182f, r);
-}
-__device__ __forceinline__ float sigmoid_near(float x) {
-  const float d = 1.f + exp_near(-x), r = __builtin_amdgcn_rcpf(d);
-  return fmaf(fmaf(-d, r, 1.f), r, r);
-}
 __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();

@@ -16,6 +16,39 @@ __device__ __forceinline__ float dyt_f(float x, float alpha, float w, float b) {
   return tanhf(alpha * x) * w + b;
 }
 
+// As near to the exact values as expf, logf, tanhf and an exact division, from the hardware's 2^t, log2 and
+// reciprocal with their roundings made good: at a third of the instructions, for the inner loops that those bound.
+// e^x for x up to 88 (more: as 88; below -200: 0)
+__device__ __forceinline__ float exp_near(float x) {
+  constexpr float kL = 1.44269502f, kLlo = 1.92596299e-8f;     // log2(e) = kL + kLlo
+  x = x < -200.f ? -200.f : x > 88.f ? 88.f : x;               // (NaN stays)
+  const float t = x * kL, lo = fmaf(x, kLlo, fmaf(x, kL, -t));
+  const float r = __builtin_amdgcn_exp2f(t);
+  return fmaf(r, lo * 0.693147182f, r);
+}
+// 1 / d for 1 <= d < 2^127
+__device__ __forceinline__ float recip_near(float d) {
+  const float r = __builtin_amdgcn_rcpf(d);
+  return fmaf(fmaf(-d, r, 1.f), r, r);
+}
+__device__ __forceinline__ float sigmoid_near(float x) { return recip_near(1.f + exp_near(-x)); }
+// ln x for normal x
+__device__ __forceinline__ float log_near(float x) {
+  constexpr float kL = 0.693147182f, kLlo = -1.90465421e-9f;   // ln 2 = kL + kLlo
+  const float y = __builtin_amdgcn_logf(x), r = y * kL;
+  return r + fmaf(y, kLlo, fmaf(y, kL, -r));
+}
+// tanh x: near 0 an odd polynomial (least squares in x^2, weighted to an even relative error of 3e-10), else through
+// one exponential
+__device__ __forceinline__ float tanh_near(float x) {
+  const float z = x * x;
+  float p = fmaf(z, -0.00665356684f, 0.0213016998f);
+  p = fmaf(z, p, -0.0538999699f);
+  p = fmaf(z, p, 0.133329704f);
+  p = fmaf(z, p, -0.333333284f);
+  return z < 0.25f ? fmaf(x, z * p, x) : 1.f - 2.f * recip_near(1.f + exp_near(2.f * x));
+}
+
 // four consecutive elements as one vector access (16 bytes of fp32, 8 bytes of a 16-bit type)
 template <typename T> __device__ __forceinline__ void load4(const T* __restrict__ p, float (&o)[4]) {
   const uint2 raw = *reinterpret_cast<const uint2*>(p);

@@ -723,12 +723,13 @@ def latent_query(q: torch.Tensor, uk: torch.Tensor, ukT: torch.Tensor, D: int, p
     return out
 
 
-def fresh_latent_ok(dtype: torch.dtype, seg, D: int, Dr: int, Dv: int) -> bool:
-    """Can ``fresh_latent_attention`` run the step's prompt portions?"""
+def fresh_latent_ok(dtype: torch.dtype, seg, D: int, Dr: int, Dv: int, R: int = 0) -> bool:
+    """Can ``fresh_latent_attention`` run the step's prompt portions?  ``R``: columns before the shared key part in
+    its rows (the kernel reads them in 16-byte chunks)."""
     from ._seqmix import DT, fresh_tiles_ok
 
     return (seg.fresh and seg.q_tiles is not None and seg.tile_rows > 0 and seg.cu.is_cuda
-            and dtype in (torch.bfloat16, torch.float16) and fresh_tiles_ok(DT[dtype], D, Dr, Dv))
+            and dtype in (torch.bfloat16, torch.float16) and R % 8 == 0 and fresh_tiles_ok(DT[dtype], D, Dr, Dv))
 
 
 def fresh_latent_attention_ref(q, k, kr, v, out, seg, scale):

@@ -329,7 +329,7 @@ class DalavikLayerW:
     ff: Optional[dict] = None       # gu [2 ff, W], down [W, ff], ff, norm
     side: Optional[dict] = None     # gate [d, W], proj [W, d], norm [W], col0
     kv_layer: int = -1              # latent attention: the layer whose cache rows it reads
-    readers: Dict[int, tuple] = field(default_factory=dict)   # an owner's: {layer: (dim, rot_dim, vdim)} reading its rows
+    readers: Dict[int, tuple] = field(default_factory=dict)   # an owner's: {layer: (dim, rot_dim, vdim, kv_rank)} reading its rows
 
 
 class DalavikWeights:
@@ -366,7 +366,7 @@ class DalavikWeights:
                     H, D, Dv, R = m["heads"], m["dim"], m["vdim"], m["kv_rank"]
                     own = m.get("kv_from") is None
                     L.kv_layer = i if own else int(m["kv_from"])
-                    (L if own else self.layers[L.kv_layer]).readers[i] = (D, m["rot_dim"], Dv)
+                    (L if own else self.layers[L.kv_layer]).readers[i] = (D, m["rot_dim"], Dv, R)
                     L.w["down"] = (torch.cat([t(x + "dq"), t(x + "dkv")], 0).contiguous()
                                    if own else t(x + "dq").detach())
                     L.w["dq_norm"] = f32(x + "dq.norm")
@@ -453,7 +453,7 @@ def run_dalavik_layers(w: DalavikWeights, st: DalavikState, tokens: torch.Tensor
             H, D, Dr, Dv, R, Q = (m["heads"], m["dim"], m["rot_dim"], m["vdim"], m["kv_rank"],
                                   m["q_rank"])
             z = project(xb, L.w["down"])
-            fresh = seg.tile_rows if fresh_latent_ok(dt, seg, D, Dr, Dv) else 0
+            fresh = seg.tile_rows if fresh_latent_ok(dt, seg, D, Dr, Dv, R) else 0
             if L.kv_layer == i:
                 # the step's own cache rows, for the fresh prompts of this layer and of borrowing layers,
                 # whose heads may have other sizes

@@ -491,6 +491,17 @@ def test_bf16_close_to_oracle_and_cut_invariant(name):
     check_rounding(cut, whole)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rank", [100, 104])
+def test_latent_rank_and_rotated_part_alignment(rank):
+    """A fresh prompt where the shared key part of a cache row does and does not begin on 16 bytes."""
+    cfg = _cfg("rank", 90, 64, 1, 0, 1e-5, [_lat(2, 128, 64, 128, rank, 24, 0.07, 777.0, 8, _ff(32))])
+    m = DalavikForCausalLM(cfg, dtype=torch.bfloat16, device="cuda")
+    m.init_weights(seed=6)
+    toks = tokens(m, 70, 7)
+    check_rounding(replay_alone(m, "cuda", toks, [1000]), oracle(m).forward(toks))
+
+
 def check_rounding(got, want, rms=2.5e-2, worst=0.12):
     """16-bit activations: the error's root mean square and its maximum over all logits, as
     fractions of the logits' spread."""

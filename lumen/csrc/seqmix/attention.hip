@@ -603,6 +603,53 @@ tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ c
     __syncthreads();
   }
   l += __shfl_xor(l, 32, 64);
+  // A hidden key has weight 0, but 0 times an infinite or NaN value is NaN: channels that are not finite are formed
+  // again, key by key over what the row sees (m and l stand).
+  bool odd = false;
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) odd |= !(fabsf(O[db][r]) < INFINITY);
+  if (__builtin_expect(__any(odd && qv), 0)) {
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db) {
+      f32x16 o;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[r] = 0.f;
+      for (int j = wlo_min; j <= wpos_max; ++j) {
+        const int jb = j / bs;
+        const T* kp = cache + (((long long)tbl[jb] * bs + (j - jb * bs)) * G + g) * D;
+        float s = 0.f, k2 = 0.f;
+#pragma unroll
+        for (int kk = 0; kk < D / 16; ++kk) {
+          __builtin_amdgcn_sched_barrier(0);       // (one load at a time: registers)
+          float x[8];
+          load8<T>(kp + 16 * kk + 8 * hi, x);
+          uint4 qk = qreg[kk];
+          asm volatile("" : "+v"(qk.x), "+v"(qk.y), "+v"(qk.z), "+v"(qk.w));   // (converted here, not ahead of the loop)
+          const T* y = reinterpret_cast<const T*>(&qk);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            s = fmaf(x[e], to_f32(y[e]), s);
+            k2 = fmaf(x[e], x[e], k2);
+          }
+        }
+        s += __shfl_xor(s, 32, 64);
+        k2 += __shfl_xor(k2, 32, 64);
+        const float p = __expf(s * qn / sqrtf(k2 / D + eps) - m);
+        if (j > pos || j < lo) continue;
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+          float v[4];
+          load4<T>(kp + 32 * db + 8 * q4 + 4 * hi, v);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[4 * q4 + e] = fmaf(p, v[e], o[4 * q4 + e]);
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) O[db][r] = fabsf(O[db][r]) < INFINITY ? O[db][r] : o[r];
+    }
+  }
   if (qv) {
     const float inv = 1.f / l;
     T* op = out + ((long long)qrow * H + hd) * D;

@@ -67,6 +67,28 @@ template <> __device__ __forceinline__ void store4<float>(float* __restrict__ p,
   *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
 }
 
+// infinities and NaN among 16-bit values
+template <typename T> struct OddBits {            // exponents of all ones and their lowest bit, in both halves
+  static constexpr unsigned E = 0x7c007c00u, one = 0x04000400u;
+};
+template <> struct OddBits<bf16> { static constexpr unsigned E = 0x7f807f80u, one = 0x00800080u; };
+template <typename T> __device__ __forceinline__ unsigned odd2(unsigned v) {      // bits 15 and 31
+  return ((v & OddBits<T>::E) + OddBits<T>::one) & 0x80008000u;
+}
+template <typename T> __device__ __forceinline__ bool odd8(const uint4& v) {
+  return (odd2<T>(v.x) | odd2<T>(v.y) | odd2<T>(v.z) | odd2<T>(v.w)) != 0;
+}
+template <typename T> __device__ __forceinline__ unsigned finite2(unsigned v) { return v & ~((odd2<T>(v) >> 15) * 0xffffu); }
+template <typename T> __device__ __forceinline__ uint4 finite8(const uint4& v) {
+  return make_uint4(finite2<T>(v.x), finite2<T>(v.y), finite2<T>(v.z), finite2<T>(v.w));
+}
+// the infinities and NaN of four consecutive 16-bit values, 0 elsewhere
+template <typename T> __device__ __forceinline__ void odd4(const T* p, float (&o)[4]) {
+  load4<T>(p, o);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = fabsf(o[e]) < INFINITY ? 0.f : o[e];
+}
+
 // the gate's activation: 0 SiLU, 1 ReLU, 2 tanh-GELU, 3 squared ReLU
 __device__ __forceinline__ float gate_act(float g, int act) {
   if (act == 3) {

@@ -14,6 +14,9 @@
 //   3. wave w takes the softmax of its heads with lane (row, 8 keys): exactly the operand of O^T += V^T P^T, so
 //      the weights feed it from registers, as a 16-bit head plus a 16-bit remainder; the values lie row-major in LDS
 //      (LDS-DMA, issued before step 1) and are read transposed (ds_read_b64_tr_b16).
+// A hidden key has weight 0, but 0 times an infinite or NaN value is NaN: in the tiles where some row's keys end (a
+// workgroup's last one or two) such values are blanked in LDS, and added at the end to the rows that do see them (a
+// weight is positive, so the value itself is the result).
 // The score of (key, head, row) lies at ((key Hp + (head ^ head/4 ^ key/4 ^ key/16) mod 4 in the low bits) 16 + row):
 // all three steps touch four different groups of 16 banks at a time.
 // Bound by the chain of tiles at two waves per SIMD (~13000 cycles per 32 keys, a third of it the shaping's
@@ -87,7 +90,7 @@ __global__ void __launch_bounds__(512, 2) talk_tile_kernel(const TalkArgs<T> a) 
   extern __shared__ __attribute__((aligned(16))) char smem[];
   float* s_s = reinterpret_cast<float*>(smem);                         // [kKeys][Hp][16]
   char* s_v = smem + kKeys * Hp * 16 * 4;                              // [G][kKeys][256 bytes]
-  int* s_tbl = reinterpret_cast<int*>(s_v + a.G * kKeys * 256);        // [kTbl]
+  int* s_tbl = reinterpret_cast<int*>(s_v + a.G * kKeys * 256);        // [kTbl], then: were values blanked?
   const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // every tile's last rows first: consecutive workgroups belong to different tiles
@@ -103,6 +106,7 @@ __global__ void __launch_bounds__(512, 2) talk_tile_kernel(const TalkArgs<T> a) 
   const bool in_lds = nblk <= kTbl;
   if (in_lds)
     for (int i = threadIdx.x; i < nblk; i += 512) s_tbl[i] = tbl[i];
+  if (threadIdx.x == 0) s_tbl[kTbl] = 0;
   // heads past the last one: scores of zero, never written again
   for (int i = threadIdx.x; i < kKeys * Hp * 4; i += 512)
     reinterpret_cast<f32x4*>(s_s)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -241,6 +245,15 @@ __global__ void __launch_bounds__(512, 2) talk_tile_kernel(const TalkArgs<T> a) 
     }
     // the values have landed for every wave (the next tile's keys, asked for after them, too)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (j0 + kKeys - 1 > first + p0) {                  // some row's keys end here: infinite values of the wave's
+      for (int gv = 0; gv < a.G; ++gv) {                // value rows are blanked
+        uint4* vp = reinterpret_cast<uint4*>(s_v + (gv * kKeys + 4 * w) * 256 + 16 * lo);
+        if (odd8<T>(*vp)) {
+          *vp = finite8<T>(*vp);
+          s_tbl[kTbl] = 1;
+        }
+      }
+    }
     __syncthreads();
     // 3. softmax and values of the wave's heads
     if (on) {
@@ -293,6 +306,20 @@ __global__ void __launch_bounds__(512, 2) talk_tile_kernel(const TalkArgs<T> a) 
     }
     __syncthreads();
   }
+  if (s_tbl[kTbl] != 0 && on) {                          // what was blanked, for the rows that see it
+    for (int j = (first + p0 + 1) / kKeys * kKeys; j <= pos; ++j) {      // (from the first such tile on)
+      const T* vr = a.vc + (cache_row(j) * a.G + g) * kD + 4 * lg;
+#pragma unroll
+      for (int n = 0; n < 8; ++n) {
+        float v[4];
+        odd4<T>(vr + 16 * n, v);
+#pragma unroll
+        for (int x = 0; x < HPW; ++x)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) O[x][n][i] += v[i];
+      }
+    }
+  }
   // O[x][n][i]: channel 16 n + 4 lg + i of head hw + x, row lr
 #pragma unroll
   for (int x = 0; x < HPW; ++x) {
@@ -311,7 +338,7 @@ __global__ void __launch_bounds__(512, 2) talk_tile_kernel(const TalkArgs<T> a) 
 
 inline int heads_per_wave(int H) { return H <= 8 ? 1 : H <= 16 ? 2 : 4; }
 inline size_t talk_lds(int H, int G) {
-  return (size_t)kKeys * ((H + 15) / 16 * 16) * 16 * 4 + (size_t)G * kKeys * 256 + kTbl * 4;
+  return (size_t)kKeys * ((H + 15) / 16 * 16) * 16 * 4 + (size_t)G * kKeys * 256 + (kTbl + 4) * 4;
 }
 
 template <typename T>

@@ -24,7 +24,8 @@
 // before), two LDS buffers leave one barrier per tile, 64 keys share its exchanges, and the accumulators follow
 // the maximum only when it rises by kRise.  Measured (us, tiles of 32 keys, one buffer -> now; bf16, heads of
 // 128, soft cap): 1 x 512 rows x 32 heads 55 -> 33, 8 x 512 x 16 91 -> 43, 14 of 63 - 509 x 16 110 -> 58, 1 x 4096 x 32
-// (window 1024) 380 -> 168; heads of 64 44 -> 23, of 256 191 -> 113, values of 256 169 -> 101.
+// (window 1024) 380 -> 168; heads of 64 44 -> 23, of 256 191 -> 113, values of 256 169 -> 101; the look for infinite
+// results at the end, which later came to it, 1 - 2 us (8 x 512 x 16 43.9 -> 45.5).
 //
 // Per wave (32 queries) and 32 keys, with v_mfma_f32_32x32x16:
 //   S^T = K Q^T      keys on the accumulator rows, queries on the columns (lane & 31): a lane
@@ -71,6 +72,16 @@ template <> __device__ __forceinline__ void unpack2<fp16>(unsigned v, float& a, 
   const lumen_f16x2 h = __builtin_bit_cast(lumen_f16x2, v);
   a = static_cast<float>(h[0]);
   b = static_cast<float>(h[1]);
+}
+
+// s + the products of 8 16-bit values at k with those of q
+template <typename T> __device__ __forceinline__ float dot8(const T* k, const uint4& q, float s) {
+  float x[8];
+  load8<T>(k, x);
+  const T* y = reinterpret_cast<const T*>(&q);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) s = fmaf(x[e], to_f32(y[e]), s);
+  return s;
 }
 
 constexpr float kRise = 5.f;      // log of the largest weight a tile may form before its maximum moves the reference
@@ -385,6 +396,55 @@ win_tile_attn_kernel(const WinTileArgs<T> a) {
     k0 = kn;
   }
   l += __shfl_xor(l, 32, 64);
+  // A hidden key has weight 0, but 0 times an infinite or NaN value is NaN: channels that are not finite are formed
+  // again, key by key over what the row sees (m and l stand).
+  bool odd = false;
+#pragma unroll
+  for (int db = 0; db < DV / 32; ++db)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) odd |= !(fabsf(O[db][r]) < INFINITY);
+  if (__builtin_expect(__any(odd && qv), 0)) {
+#pragma unroll
+    for (int db = 0; db < DV / 32; ++db) {
+      f32x16 o;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[r] = 0.f;
+      for (int j = kfirst; j <= wpos_max; ++j) {
+        if (window > 0 && j >= keep) j = max(j, wpos_min - window + 1);
+        const T *kp, *kr, *vp;
+        if constexpr (FRESH) {
+          kp = a.kc + (seg_r0 + j) * a.ldk + g * (D - kDr);
+          kr = a.kr + (seg_r0 + j) * a.ldr - (D - kDr);
+          vp = a.vc + (seg_r0 + j) * a.ldv + gv * DV;
+        } else {
+          const int jb = j / bs;
+          const long long row = (long long)tbl[jb] * bs + (j - jb * bs);
+          kp = kr = a.kc + (row * a.G + g) * D;
+          vp = a.vc + (row * Gv + gv) * DV;
+        }
+        float s = 0.f;
+#pragma unroll
+        for (int kk = 0; kk < D / 16; ++kk) {
+          __builtin_amdgcn_sched_barrier(0);     // (one load at a time: registers)
+          s = dot8<T>((FRESH && 16 * kk >= D - kDr ? kr : kp) + 16 * kk + 8 * hi, qreg[kk], s);
+        }
+        s = (s + __shfl_xor(s, 32, 64)) * a.scale;
+        if (cap > 0.f) s = cap * tanh_exp(s * rcap);
+        s -= slope * (float)(pos - j);
+        const float p = a.sigb != nullptr ? 1.f / (1.f + __expf(-(s + sbias))) : __expf(s - m);
+        if (j > pos || (window > 0 && pos - j >= window && j >= keep)) continue;
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+          float v[4];
+          load4<T>(vp + 32 * db + 8 * q4 + 4 * hi, v);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[4 * q4 + e] = fmaf(p, v[e], o[4 * q4 + e]);
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) O[db][r] = fabsf(O[db][r]) < INFINITY ? O[db][r] : o[r];
+    }
+  }
   if (qv) {
     float inv = a.sigb != nullptr ? 1.f : 1.f / l;   // l > 0: a row always sees its own key
     if (a.gate != nullptr) inv *= sigmoid_f(to_f32(a.gate[(long long)qrow * a.gater + hd]));

@@ -155,6 +155,62 @@ def test_mixed_head_tiles(H, G, opts, lens, starts, bs, tile, dtype, ulp):
     close(out, ref, ulp)
 
 
+ODD = {5: (0, float("inf")), 37: (9, float("-inf")), 100: (21, float("nan"))}     # position: channel, value
+
+
+def odd_rows(run, v, seg, window=0):
+    """``run`` before and after values of some tokens became infinite or NaN: the rows that see such a token are lost in
+    its channel, the others keep what they had (formed again there), and other channels their bits."""
+    before = run().clone()
+    assert torch.isfinite(before).all()
+    lost = torch.zeros_like(before, dtype=torch.bool)
+    for j, (ch, x) in ODD.items():
+        v(j)[..., ch] = x
+        p = seg.positions[:before.shape[0]]
+        lost[(p >= j) & ((window == 0) | (p - j < window)), :, ch] = True
+    after, other = run(), ~lost.any(1).any(0)
+    assert torch.equal(after[:, :, other], before[:, :, other]) and not torch.isfinite(after[lost]).any()
+    close(after[~lost], before[~lost], 2.0 ** -8 if before.dtype == torch.bfloat16 else 2.0 ** -11)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kind,H,G,D,Dv,window", [
+    ("window", 4, 2, 128, 128, 0), ("window", 2, 2, 64, 128, 20), ("window", 2, 1, 128, 256, 0), ("talk", 8, 2, 128, 128, 0),
+    ("talk", 16, 4, 128, 128, 0), ("talk", 24, 6, 128, 128, 0), ("fresh", 3, 3, 128, 128, 0)])
+def test_infinite_values_of_hidden_tokens(kind, H, G, D, Dv, window, dtype):
+    g = torch.Generator().manual_seed(H)
+    T, seg, (k, v) = portions([131], [0], 16, g, (G, D), (G, Dv))
+    f = lambda *s: torch.randn(*s, generator=g).to(dtype).cuda()  # noqa: E731
+    k, v, out = k.to(dtype).cuda(), v.to(dtype).cuda(), torch.zeros(T, H, Dv, dtype=dtype, device="cuda")
+    if kind == "fresh":
+        from lumen.ops.attention import fresh_latent_attention
+        seg.fresh = True
+        q, k, kr, v = f(T, H, D + 64), f(T, H, D), f(T, 64), f(T, H, Dv)
+        return odd_rows(lambda: fresh_latent_attention(q, k, kr, v, out, seg, 0.07), lambda j: v[j], seg)
+    q, talk = f(T, H, D), torch.eye(H).cuda() + 0.1 if kind == "talk" else None
+    odd_rows(lambda: row_attention(q, None, k, v, Dv, out, seg, H, G, 0.1, talk=talk, window=window),
+             lambda j: v[seg.tables[0, j // 16].item(), j % 16], seg, window)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,G,D,chunk", [(4, 2, 128, 0), (2, 1, 96, 50), (2, 2, 256, 0), (2, 2, 64, 128)])
+def test_infinite_keys_of_hidden_tokens(H, G, D, chunk, dtype):
+    """Keys that are their own values: whole rows that see such a token are lost, the others keep what they had."""
+    g = torch.Generator().manual_seed(H)
+    T, seg, (k,) = portions([131], [0], 16, g, (G, D))
+    k, q = k.to(dtype).cuda(), torch.randn(T, H * D, generator=g).to(dtype).cuda()
+    run = lambda: chunk_sink_attention(q, k, seg, H, G, D, 0.3, chunk, 1e-6).view(T, -1)  # noqa: E731
+    before = run()
+    lost = torch.zeros(T, dtype=torch.bool, device="cuda")
+    for j, x in ((37, float("inf")), (70, float("nan"))):
+        k[seg.tables[0, j // 16].item(), j % 16] = x
+        p = seg.positions
+        lost |= (p >= j) & ((chunk == 0) | (p // max(chunk, 1) == j // max(chunk, 1)))
+    after = run()
+    assert torch.isnan(after[lost]).all() and 0 < int(lost.sum()) < T
+    close(after[~lost], before[~lost], 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_fresh_and_cached_prompts_agree(dtype):
     """One engine step of whole prompts (expanded keys) against the same prompts in two portions (the cached latent):

@@ -12,18 +12,21 @@
 //   2. wave w mixes the heads of its 4 keys: S' = talk S per key with v_mfma_f32_16x16x4_f32 -- the products stay
 //      in fp32 -- in place;
 //   3. wave w takes the softmax of its heads with lane (row, 8 keys): exactly the operand of O^T += V^T P^T, so
-//      the weights feed it from registers, as a 16-bit head plus a 16-bit remainder; the values lie row-major in LDS
+//      the weights feed it from registers, the fp32 ones in three 16-bit parts; the values lie row-major in LDS
 //      (LDS-DMA, issued before step 1) and are read transposed (ds_read_b64_tr_b16).
 // A hidden key has weight 0, but 0 times an infinite or NaN value is NaN: in the tiles where some row's keys end (a
 // workgroup's last one or two) such values are blanked in LDS, and added at the end to the rows that do see them (a
 // weight is positive, so the value itself is the result).
 // The score of (key, head, row) lies at ((key Hp + (head ^ head/4 ^ key/4 ^ key/16) mod 4 in the low bits) 16 + row):
 // all three steps touch four different groups of 16 banks at a time.
-// Bound by the chain of tiles at two waves per SIMD (~13000 cycles per 32 keys, a third of it the shaping's
+// Bound by the chain of tiles at two waves per SIMD (~14000 cycles per 32 keys, a third of it the shaping's
 // transcendentals).  Measured against the row kernel (us, bf16, one key head per four heads, everything on): 16 heads,
-// 14 prompts of 63 - 509 tokens 515 -> 97, 1 x 512 148 -> 91, 1 x 200 48 -> 43, 1 x 128 30 -> 30, 1 x 24 22 -> 15; 8
-// heads, 1 x 2048 755 -> 248; 32 heads, 8 of 32 - 256 316 -> 119, 1 x 2048 5248 -> 856, 1 x 80 57 -> 54: prompts of every
+// 14 prompts of 63 - 509 tokens 515 -> 107, 1 x 512 148 -> 101, 1 x 200 48 -> 47, 1 x 128 30 -> 30, 1 x 24 22 -> 15; 8
+// heads, 1 x 2048 755 -> 275; 32 heads, 8 of 32 - 256 316 -> 130, 1 x 2048 5248 -> 930, 1 x 80 57 -> 58: prompts of every
 // length take it.
+// Error: the row kernel's.  Share of results that are not float64's rounded, row kernel / here: bf16 0.0003 / 0.0003,
+// fp16 0.0022 / 0.0022.  (Two parts and the hardware's exponential, logarithm and reciprocal as they are: 0.0025 and
+// 0.0115, at 100 us for the 14 prompts; three parts alone 104; expf, logf and tanhf 117, with the same error.)
 #include "seqmix.h"
 
 using namespace lumen;
@@ -50,6 +53,19 @@ template <> struct Mfma<fp16> {
 };
 
 constexpr int kD = 128, kRows = 16, kKeys = 32, kTbl = 512;
+// fp16: weights up to e^kRise times this fit, and the parts of small ones stay above its subnormals' grain
+template <typename T> constexpr float kUp = 1.f;
+template <> constexpr float kUp<fp16> = 128.f;
+template <typename T> __device__ __forceinline__ void unpack2(unsigned u, float& a, float& b);
+template <> __device__ __forceinline__ void unpack2<bf16>(unsigned u, float& a, float& b) {
+  a = __uint_as_float(u << 16);
+  b = __uint_as_float(u & 0xffff0000u);
+}
+template <> __device__ __forceinline__ void unpack2<fp16>(unsigned u, float& a, float& b) {
+  const auto h = __builtin_bit_cast(lumen_f16x2, u);
+  a = static_cast<float>(h[0]);
+  b = static_cast<float>(h[1]);
+}
 constexpr float kRise = 5.f;      // log of the largest weight a tile may form before its maximum moves the reference
 
 template <typename T> struct TalkArgs {
@@ -76,11 +92,6 @@ __device__ __forceinline__ void dma16(const void* src, const char* lds_wave_base
   const unsigned m0 = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(
       reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const char*)(lds_wave_base))));
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(m0) : "memory", "m0");
-}
-
-// tanh through one exponential: 1 - 2 / (1 + e^(2x)); exact limits at both ends
-__device__ __forceinline__ float tanh_exp(float x) {
-  return 1.f - 2.f * __builtin_amdgcn_rcpf(1.f + __expf(2.f * x));
 }
 
 // HPW: heads of a wave (consecutive ones of one key head); MT: 16-head blocks of the mixing
@@ -205,7 +216,7 @@ __global__ void __launch_bounds__(512, 2) talk_tile_kernel(const TalkArgs<T> a) 
 #pragma unroll
           for (int b = 0; b < 2; ++b)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) c[b][i] = cap * tanh_exp(c[b][i] * rcap);
+            for (int i = 0; i < 4; ++i) c[b][i] = cap * tanh_near(c[b][i] * rcap);
         }
         if (a.r1 != nullptr) {
 #pragma unroll
@@ -213,7 +224,7 @@ __global__ void __launch_bounds__(512, 2) talk_tile_kernel(const TalkArgs<T> a) 
 #pragma unroll
             for (int i = 0; i < 4; ++i) {              // (keys past the row's position are masked below)
               const float d = (float)max(pos - (j0 + 16 * b + 4 * lg + i), 0);
-              c[b][i] -= r1 * __logf(1.f + r2 * d);
+              c[b][i] -= r1 * log_near(1.f + r2 * d);
             }
         }
 #pragma unroll
@@ -272,24 +283,33 @@ __global__ void __launch_bounds__(512, 2) talk_tile_kernel(const TalkArgs<T> a) 
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
         if (__any(mx > m[x] + kRise)) {
           const float mn = mx > m[x] + kRise ? mx : m[x];
-          const float corr = mn == m[x] ? 1.f : __expf(m[x] - mn);
+          const float corr = mn == m[x] ? 1.f : exp_near(m[x] - mn);
           l[x] *= corr;
           m[x] = mn;
 #pragma unroll
           for (int n = 0; n < 8; ++n) O[x][n] *= corr;
         }
         const float ms = m[x] == -INFINITY ? 0.f : m[x];
-        float hi[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          p[e] = __expf(p[e] - ms);
+          p[e] = exp_near(p[e] - ms);
           l[x] += p[e];
-          hi[e] = to_f32(from_f32<T>(p[e]));
         }
-        const uint4 ph = make_uint4(pk2<T>(hi[0], hi[1]), pk2<T>(hi[2], hi[3]), pk2<T>(hi[4], hi[5]),
-                                    pk2<T>(hi[6], hi[7]));
-        const uint4 pl = make_uint4(pk2<T>(p[0] - hi[0], p[1] - hi[1]), pk2<T>(p[2] - hi[2], p[3] - hi[3]),
-                                    pk2<T>(p[4] - hi[4], p[5] - hi[5]), pk2<T>(p[6] - hi[6], p[7] - hi[7]));
+        uint4 part[3];                                   // the fp32 weights in three 16-bit parts: all of their bits
+#pragma unroll
+        for (int y = 0; y < 3; ++y) {
+          unsigned u[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if (y == 0) { p[2 * e] *= kUp<T>; p[2 * e + 1] *= kUp<T>; }
+            u[e] = pk2<T>(p[2 * e], p[2 * e + 1]);
+            float h0, h1;
+            unpack2<T>(u[e], h0, h1);
+            p[2 * e] -= h0;
+            p[2 * e + 1] -= h1;
+          }
+          part[y] = make_uint4(u[0], u[1], u[2], u[3]);
+        }
         // lane (lr, lg) of operand n: channel 16 n + lr, keys 8 lg .. 8 lg + 7, from rows 8 lg + lr / 4 (+ 4)
         const char* vb = s_v + g * kKeys * 256;
         const int r = 8 * xg + (xr >> 2), half = 8 * (xr & 1);
@@ -299,8 +319,8 @@ __global__ void __launch_bounds__(512, 2) talk_tile_kernel(const TalkArgs<T> a) 
           const uint2 v0 = tr_read(vb + r * 256 + ((ch ^ vswz(r)) << 4) + half);
           const uint2 v1 = tr_read(vb + (r + 4) * 256 + ((ch ^ vswz(r + 4)) << 4) + half);
           const uint4 av = make_uint4(v0.x, v0.y, v1.x, v1.y);
-          O[x][n] = Mfma<T>::run(av, ph, O[x][n]);
-          O[x][n] = Mfma<T>::run(av, pl, O[x][n]);
+#pragma unroll
+          for (int y = 0; y < 3; ++y) O[x][n] = Mfma<T>::run(av, part[2 - y], O[x][n]);
         }
       }
     }
@@ -327,7 +347,7 @@ __global__ void __launch_bounds__(512, 2) talk_tile_kernel(const TalkArgs<T> a) 
     sum += __shfl_xor(sum, 16, 64);
     sum += __shfl_xor(sum, 32, 64);
     if (hw + x >= a.H || first + lr >= end) continue;
-    const float inv = 1.f / sum;
+    const float inv = 1.f / (sum * kUp<T>);
     T* op = a.out + (long long)row * a.our + (long long)(hw + x) * a.ouh + 4 * lg;
 #pragma unroll
     for (int n = 0; n < 8; ++n)

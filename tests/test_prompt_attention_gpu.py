@@ -155,6 +155,31 @@ def test_mixed_head_tiles(H, G, opts, lens, starts, bs, tile, dtype, ulp):
     close(out, ref, ulp)
 
 
+@pytest.mark.parametrize("dtype,share", [(torch.bfloat16, 0.001), (torch.float16, 0.005)])
+@pytest.mark.parametrize("H,G", [(8, 2), (16, 4), (32, 8)])
+def test_mixed_head_tiles_hold_fp32_weights(H, G, dtype, share):
+    """Scores, weights and sums in fp32: hardly a result but float64's rounded.  A relative error e of a result before
+    it is rounded misses that for a share of ~ 2 e / (the type's half ulp): fp32's (a few 2^-24, over sums of 63 keys) 0.03
+    and 0.2 %; weights of ~16 bits leave 0.25 and 1.2 %.  (Sizes whose shares were seen to be that.)"""
+    T, D = 63, 128
+    g = torch.Generator().manual_seed(H)
+    _, seg, (k, v) = portions([T], [0], 16, g, (G, D), (G, D))
+    k, v = k.to(dtype).cuda(), v.to(dtype).cuda()
+    q, f = torch.randn(T, H, D, generator=g).to(dtype).cuda(), lambda *s: torch.rand(*s, generator=g).cuda()
+    talk, r1, r2, sink = torch.eye(H).cuda() + 0.3 * (f(H, H) - 0.5), f(H), f(H), f(H)
+    out = torch.empty(T, H, D, dtype=dtype, device="cuda")
+    row_attention(q, None, k, v, D, out, seg, H, G, 0.088, 50.0, (0.3, 16), r1, r2, talk, sink)
+    at = torch.arange(T, device="cuda")
+    K, V = (x[seg.tables[0].long()[at // 16], at % 16].double().repeat_interleave(H // G, 1) for x in (k, v))
+    s = torch.einsum("thd,jhd->htj", q.double(), K) * 0.088 * (1 + 0.3 * torch.log((at + 1) // 16 + 1.0).double())[:, None]
+    s = 50 * torch.tanh(s / 50) - r1.double()[:, None, None] * torch.log(
+        1 + r2.double()[:, None, None] * (at[:, None] - at).clamp(min=0))
+    s = torch.einsum("ij,jtk->itk", talk.double(), s).masked_fill(at[:, None] < at, -float("inf"))
+    e = torch.exp(s)
+    ref = torch.einsum("htj,jhd->thd", e / (e.sum(-1, keepdim=True) + torch.exp(sink.double())[:, None, None]), V)
+    assert (out != ref.to(dtype)).double().mean() < share
+
+
 ODD = {5: (0, float("inf")), 37: (9, float("-inf")), 100: (21, float("nan"))}     # position: channel, value
 
 

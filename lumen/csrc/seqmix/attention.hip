@@ -29,7 +29,8 @@ constexpr int kRowWaves = 8;
 // square and its value.  (The form below reads a key row per lane for the scores -- 64 rows apart -- and all of them once
 // more for the values: 8 rows x 16 heads, 512 keys, 17.9 us in a decode step, bound by those reads' latency; here 12.1.)
 // kStep keys per lane group and step, the next step's in flight; every group keeps its own (max, sum, accumulator),
-// which meet in the wave and then in LDS.  Rows past the last key repeat it and count for nothing.
+// which meet in the wave and then in LDS.  Rows past the last key repeat it and count for nothing.  (rsqrtf: 0.9 ulp at
+// most where 1 / sqrtf has 1.5.  Results that are not float64's rounded: bf16 0.07 -> 0.02 %, fp16 0.57 -> 0.28.)
 constexpr int kStep = 8;
 
 template <int CTRL> __device__ __forceinline__ float row_dpp(float v) {

@@ -27,8 +27,9 @@
 // substitution 4.9, the state's products 7); it is 16 now, bound by what
 // the three waves of a SIMD issue: matrix instructions 5.6 of it.
 // Measured (width 2048, bf16, the norm kernel's 17 us included), four waves -> this, us: delta, 16 heads of 128: 8
-// portions of 512 tokens 305 -> 245, one of 512 281 -> 216, 32 of 128 311 -> 252; 8 heads of 256 512 -> 452; 64 of 32 185
-// -> 173; wkv, 32 heads of 64: 137 -> 124, 117 -> 97, 106 -> 100; 8 heads of 256 338 -> 280.  (Token by token: 1000 and 460.)
+// portions of 512 tokens 305 -> 237, one of 512 281 -> 211, 32 of 128 311 -> 248; 8 heads of 256 512 -> 434; 64 of 32 185
+// -> 172; wkv, 32 heads of 64 whose decays hardly ever cut a chunk: 136 -> 126, 117 -> 99, 106 -> 101; 8 heads of 256 338 ->
+// 281.  (Token by token: 1000 and 460.)
 // Error against float64 (512 tokens, heads of 32 - 256): the read-outs are as far off as the serial walk's
 // (1.66e-3, the bf16 result's rounding), the state a little less (delta 0.86e-7, serial 0.90e-7; wkv 0.62e-7,
 // serial 0.65e-7).  That takes the decays' products in float64 (in fp32: + 0.1e-7) and care with the sums
@@ -40,9 +41,12 @@
 // its chunk, where nothing is divided by it; the delta rule's decays, at least e^-decay_scale per token,
 // stay above 2^-70.  r and k that scaled rows could not hold as normal numbers (kLarge, kTiny*), infinities and
 // NaN run one token at a time, so that earlier tokens stay as they are; wkv values below kSmall make the
-// chunk end at 2^-40.  A chunk of one token costs what one of sixteen does: decays up to e^-50 a token (wkv,
-// 8 x 512 tokens, 32 heads of 64, log decays -e^N(1, 1) at the fast end) took 770 us with the four-wave form, the
-// serial walk 460; decays a token of -e^N(0..2, 0.6) 492 with the four-wave form, 460 here.
+// chunk end at 2^-40.
+// A chunk that turns out to leave the range costs rows formed and asked for twice, and two more barriers; where the two
+// before it did, its place is found before the rows (one more barrier).  us, four waves -> rows always twice, three
+// more barriers -> this, 8 x 512 tokens, 32 heads of 64, the kernel alone: decays a token of -e^N(0..2, 0.6), all chunks cut,
+// 478 -> 442 -> 301; a head of which 31 - 49 of 39 - 51 chunks are cut 207 -> 222 -> 180; none cut 119 -> 107 -> 109.
+// Decays up to e^-50 a token, chunks of one: 770 with the four-wave form.
 #include "seqmix.h"
 
 using namespace lumen;
@@ -115,7 +119,7 @@ scan_chunk_kernel(const ScanArgs<T> a) {
   };
   __shared__ __attribute__((aligned(16))) Buf s_buf[2];
   __shared__ __attribute__((aligned(16))) float s_iP[DKP], s_red[kC][KB];
-  __shared__ double s_gp[NG][DKP];
+  __shared__ double s_gp[NG][DKP], s_gt[DELTA ? 1 : kC][DELTA ? 1 : DKP];   // a token group's decay; up to each token (`cut`)
   __shared__ float s_tok[kC];
   __shared__ int s_n[2], s_low[2], s_small[2];
   const int sg = blockIdx.x, hd = blockIdx.y;
@@ -197,14 +201,32 @@ scan_chunk_kernel(const ScanArgs<T> a) {
       if (DKP < 64) tok[q] = lane < 32 ? tok[q] : lane_f(v, 32 + q);
     }
   };
-  // the scaled rows of a chunk of n tokens; true: some channel's product leaves the range
-  const auto rows = [&](Buf& B, int n, float least) __attribute__((always_inline)) {
+  // where does a channel's product leave the range?  The chunk ends before that token
+  const auto cut = [&](int par) __attribute__((always_inline)) {
+    if constexpr (DELTA) return;
+    const float least = s_small[par] ? kSmallP : kMinP;
+    double before = 1., p = 1.;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) before *= g < tg ? s_gp[g][ch] : 1.;
+    int first = kC;
+#pragma unroll
+    for (int q = 0; q < TG; ++q) {
+      p *= wv[q];
+      s_gt[tg * TG + q][ch] = p;
+      if (first == kC && before * p < least) first = tg * TG + q;
+    }
+    if (first < kC && !(before < least)) atomicMin(&s_n[par], max(first, 1));
+  };
+  // The scaled rows of a chunk of n tokens (ALL: as many as there are, at most kC); rows that are left for the next
+  // chunk decay nothing.  Returns whether some channel's product leaves the range (ALL).
+  const auto rows = [&](auto all, Buf& B, int n, float least) __attribute__((always_inline)) {
+    constexpr bool ALL = decltype(all)::value;
+    const int tc = ALL ? NG - 1 : (n - 1) / TG;          // the group that the chunk ends in
     double P = 1., Q = 1.;               // decay of the token groups before and after this one
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
-      const double q = s_gp[g][ch];
-      P *= g < tg ? q : 1.;
-      Q *= g > tg ? q : 1.;
+      P *= g < tg ? s_gp[g][ch] : 1.;
+      Q *= g > tg && g <= tc ? (ALL || DELTA || g < tc ? s_gp[g][ch] : s_gt[n - 1][ch]) : 1.;
     }
 #pragma unroll
     for (int q = TG - 1; q >= 0; --q) {  // decayed to the chunk's end
@@ -212,22 +234,22 @@ scan_chunk_kernel(const ScanArgs<T> a) {
       const bool live = tg * TG + q < n;
       B.k[at] = live ? (float)(kv[q] * Q) : 0.f;
       if (DELTA) B.b[at] = live ? (float)(kv[q] * tok[q] * av[q] * Q) : 0.f;
-      Q *= wv[q];
+      Q *= ALL || live ? wv[q] : 1.f;
     }
 #pragma unroll
     for (int q = 0; q < TG; ++q) {       // decayed from the chunk's start
       const int t = tg * TG + q, at = t * LK + ch;
       const bool live = t < n;
       const float P0 = (float)P;
-      P *= wv[q];
+      P *= ALL || live ? wv[q] : 1.f;
       B.r[at] = live ? rv[q] * (DELTA ? (float)P : P0) : 0.f;
       if (DELTA) B.u[at] = live ? kv[q] * tok[q] * P0 : 0.f;
       else if (ch == 0) s_tok[t] = tok[q];
     }
-    if (tg != NG - 1) return false;
+    if (tg != tc) return false;
     B.P[ch] = (float)P;
     s_iP[ch] = 1.f / (float)P;           // (one token: only entries that are masked out see it)
-    return !DELTA && !((float)P >= least);
+    return !DELTA && ALL && !((float)P >= least);
   };
   // chunk matrices, one per wave: U K^T, U B^T (then inverted), R K^T, R B^T
   const auto matrices = [&](Buf& B, int n) __attribute__((always_inline)) {
@@ -412,53 +434,62 @@ scan_chunk_kernel(const ScanArgs<T> a) {
   // Step: the producers build the chunk at tb while the column waves run the one before it, [tc, tc + nc).  Both
   // meet at the same barriers: what decides about more of them lies in LDS before the second.
   if (tid < 2) { s_n[tid] = kC; s_low[tid] = s_small[tid] = 0; }
-  const auto shorter = [&](int par) { return s_n[par] < kC || s_low[par]; };
   const auto count = [&](int par, int tb) { return __builtin_amdgcn_readfirstlane(min(s_n[par], len - tb)); };
+  // A wkv chunk's rows are formed as if all of it stayed in range, and again if it does not -- unless the two before were
+  // cut (a head with a fast channel cuts most of its chunks): then the place is found first.  The delta rule's length
+  // is known before its rows.
   if (!col) {
-    fetch(0);
-    __syncthreads();
-    for (int tb = 0, par = 0;; par ^= 1) {
+    int tb = 0, par = 0, cuts = 0;
+    // one step; false: it was the last
+    const auto step = [&](auto cutting) __attribute__((always_inline)) {
+      constexpr bool CUT = decltype(cutting)::value;
       const bool build = tb < len;
       Buf& B = s_buf[par];
       if (build) decays(tb, par);
       __syncthreads();
+      int n = min(kC, len - tb);
       if (build) {
+        if (CUT) {
+          cut(par);
+          __syncthreads();
+        }
         tokens();
-        if (rows(B, min(kC, len - tb), s_small[par] ? kSmallP : kMinP)) s_low[par] = 1;
-        if (tb + kC < len) fetch(tb + kC);   // in flight from here on, unless the chunk is shorter
+        if (DELTA || CUT) {
+          n = count(par, tb);
+          rows(std::false_type{}, B, n, 0.f);
+        } else if (rows(std::true_type{}, B, n, s_small[par] ? kSmallP : kMinP)) {
+          s_low[par] = 1;
+        }
+        if (tb + n < len) fetch(tb + n);       // in flight from here on, unless the chunk is shorter
       }
       __syncthreads();
-      if (build && shorter(par)) {
-        if (!DELTA) {                    // where does a channel's product leave the range?
-          const float least = s_small[par] ? kSmallP : kMinP;
-          double p = 1.;
-          for (int g = 0; g < tg; ++g) p *= s_gp[g][ch];
-#pragma unroll
-          for (int q = 0; q < TG; ++q) {
-            p *= wv[q];
-            if (p < least && tg * TG + q > 0) atomicMin(&s_n[par], tg * TG + q);
-          }
-        }
+      if (!DELTA && !CUT && build && (s_n[par] < kC || s_low[par])) {
+        cut(par);
         __syncthreads();
-        const int n = count(par, tb);
-        double p = 1.;                   // the rows that are left for the next chunk decay nothing
-#pragma unroll
-        for (int q = 0; q < TG; ++q) {
-          if (tg * TG + q >= n) wv[q] = 1.f;
-          p *= wv[q];
-        }
-        s_gp[tg][ch] = p;
-        __syncthreads();
-        rows(B, n, 0.f);
+        n = count(par, tb);
+        rows(std::false_type{}, B, n, 0.f);
         if (tb + n < len) fetch(tb + n);
         __syncthreads();
       }
-      const int n = build ? count(par, tb) : 0;
+      cuts = !DELTA && n < min(kC, len - tb) ? cuts + 1 : 0;
       if (ptid == 0) { s_n[par ^ 1] = kC; s_low[par ^ 1] = s_small[par ^ 1] = 0; }
       if (build) matrices(B, n);
       __syncthreads();
-      if (!build) return;
       tb += n;
+      par ^= 1;
+      return build;
+    };
+    fetch(0);
+    __syncthreads();
+    for (;;) {                           // (two loops: with the choice inside, a step that is not cut took 0.2 us more)
+      do
+        if (!step(std::false_type{})) return;
+      while (cuts < 2);
+      if constexpr (!DELTA) {
+        do
+          if (!step(std::true_type{})) return;
+        while (cuts > 0);
+      }
     }
   }
   const bool fresh = a.start[sg] == 0;
@@ -471,7 +502,7 @@ scan_chunk_kernel(const ScanArgs<T> a) {
     }
   fetch_v(0);
   __syncthreads();
-  for (int tb = 0, tc = 0, nc = 0, par = 0;; par ^= 1) {
+  for (int tb = 0, tc = 0, nc = 0, par = 0, cuts = 0;; par ^= 1) {
     const bool build = tb < len;
     const Buf& A = s_buf[par ^ 1];
     if (nc > 0) {
@@ -489,14 +520,15 @@ scan_chunk_kernel(const ScanArgs<T> a) {
     // (nothing of this waits for the producers: cut so that the matrix units are not wanted by all at once)
     if (nc > 0) read_out(A, tc, nc);
     __syncthreads();
+    if (build && cuts > 1) __syncthreads();
     if (nc > 0) new_state(A, 0, KB / 2);
     __syncthreads();
-    if (build && shorter(par)) {
-      __syncthreads();
+    if (!DELTA && build && cuts < 2 && (s_n[par] < kC || s_low[par])) {
       __syncthreads();
       __syncthreads();
     }
     const int n = build ? count(par, tb) : 0;
+    cuts = !DELTA && n < min(kC, len - tb) ? cuts + 1 : 0;
     if (nc > 0) new_state(A, KB / 2, KB);
     __syncthreads();
     if (!build) break;

@@ -108,6 +108,37 @@ def test_wkv_decays_from_none_to_total(H, D):
     assert (state[0].cpu().double() - S).norm() <= 2e-6 * S.norm()
 
 
+@pytest.mark.parametrize("H,D", [(2, 64), (1, 32), (1, 200)])
+@pytest.mark.parametrize("T", [160, 161, 175])
+def test_wkv_runs_of_cut_chunks(H, D, T):
+    """Stretches whose chunks stay in range, whose every chunk is cut, and with single cuts; rows of one token and the end
+    within a cut stretch; a row that is not finite among them."""
+    g = torch.Generator().manual_seed(T + D)
+    cu, seg = batch([T, 1, 2], 0, [0, 5, 0])
+    x = rows(T + 3, H, D, torch.bfloat16, g, 0)
+    z = torch.full((T + 3, H * D), -4.0)
+    z[30:75, 7::16] = 2.0                      # e^-7.4 a token: 9 of them to a chunk
+    z[95, 1] = z[97, 9] = z[120, 3] = 4.5      # one total decay in a chunk
+    z[T - 25:, ::8] = 3.0                      # 3 to a chunk, up to the end and in the short portions
+    x[3] = z.bfloat16().cuda()
+    w0, ub, nw = torch.zeros(H * D).cuda(), torch.randn(H * D, generator=g).cuda(), torch.ones(H * D).cuda()
+    state = torch.randn(3, H, D, D, generator=g).cuda()
+    before = state.clone()
+    y = run("wkv", x, w0, ub, nw, state, seg, H, D)
+    for s, (a, b) in enumerate(zip(cu, cu[1:])):
+        S0 = before[2 - s].cpu().double() * (s == 1)
+        want, S = exact("wkv", [t[a:b] for t in x], w0, ub, nw, S0, H, D)
+        err = (y[a:b].cpu().double() - want).abs()
+        assert (err <= want.abs() * 2.0 ** -8 + 2e-5 * want.abs().max()).all()
+        assert (state[2 - s].cpu().double() - S).norm() <= 2e-6 * S.norm()
+    clean, at = y.clone(), 50
+    x[2][at, 3] = float("inf")
+    y = run("wkv", x, w0, ub, nw, before.clone(), seg, H, D)
+    torch.testing.assert_close(y[:at], clean[:at], rtol=2.0 ** -7, atol=1e-4)
+    torch.testing.assert_close(y[:T, D:], clean[:T, D:], rtol=2.0 ** -7, atol=1e-4)
+    assert not torch.isfinite(y[at + 1, :D]).all()
+
+
 @pytest.mark.parametrize("kind", ["wkv", "delta"])
 def test_a_row_that_is_not_finite_spoils_no_earlier_row(kind):
     H, D = 2, 64

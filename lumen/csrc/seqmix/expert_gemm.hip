@@ -17,10 +17,10 @@
 //  * XCDs take consecutive tiles, an expert's row tiles within a weight panel first: a panel comes from HBM once.
 // Bound by the loop at one wave per SIMD (1.0 us a step where split_gemm.hip takes 0.73: an expert's pairs are
 // fetched again for every few panels) and by each tile's own prologue and epilogue; under ~200 rows by reading the
-// weights once.  Measured (us, a whole layer of experts, dense form -> here; bf16, width 2048, experts of 1408): 8
-// experts, top 2, and a shared one: 4096 rows 534 -> 283, 512 90 -> 60, 256 62 -> 56, 100 52 -> 54; 16, top 3, shared:
-// 4096 1130 -> 371, 512 166 -> 99, 64 149 -> 79; 16 ungated, top 4: 4096 810 -> 298, 8192 at width 4096 2721 (grouped
-// library product) -> 1685.  Error against float64 2.3e-3 where the dense form has 3.5e-3: nothing is rounded between the
+// weights once.  Measured (us, a whole layer of experts, dense form -> here; bf16, width 2048, experts of 1408, weights that
+// the last-level cache holds; ops/moe.py has few rows with weights from HBM): 8 experts, top 2, and a shared one: 4096 rows
+// 534 -> 283, 512 90 -> 60, 256 62 -> 56; 16, top 3, shared: 4096 1130 -> 371, 512 166 -> 99, 64 149 -> 79; 16 ungated,
+// top 4: 4096 810 -> 298, 8192 at width 4096 2721 (grouped library product) -> 1685.  Error against float64 2.3e-3 where the dense form has 3.5e-3: nothing is rounded between the
 // products and the activation, nor before the sum.
 #include "seqmix.h"
 

@@ -18,8 +18,8 @@ projections side by side in one [W, E * ff + ffs] weight):
   sorted (row, expert) pairs have a static count, the group offsets stay on the device, nothing
   synchronises and a layer's experts are three launches.
 * ``moe_chosen``: the (row, expert) pairs sorted by expert on the device, both products on HIP kernels
-  (``csrc/seqmix/expert_gemm.hip``) that gather the rows themselves.  16-bit steps of more than a few rows take it,
-  decode graphs included; the other forms serve fp32, sizes without kernels and the few-row steps.
+  (``csrc/seqmix/expert_gemm.hip``) that gather the rows themselves.  16-bit steps of more than a few rows take it
+  (``chosen_pays``), decode graphs included; the other forms serve fp32, sizes without kernels and the few-row steps.
 """
 from __future__ import annotations
 
@@ -561,12 +561,26 @@ def grouped_pays(rows: int, E: int, top: int, expert_weights: int) -> bool:
 
 
 # Up to 32 rows the activation forms in the thin GEMM's epilogue and experts no row chose are not read; up to 64 the
-# thin GEMM still has the smaller stacks (width 1024, 8 experts of 704, top 2, 48 rows: 32 us against 39).  Beyond, at
-# the widths 1024 - 4096 and with 8 or 16 experts, dense -> chosen in us: 33 rows 240 -> 149 (4096) and 51 -> 44 (1536),
-# 80 rows 168 -> 156 and 52 -> 46, 256 rows 206 -> 167 and 67 -> 51; the one exception is width 2048 with 8 experts at 80 -
-# 160 rows, 52 -> 55.  Against the library's grouped product: 4096 rows 2721 -> 1685 (16 of 2816, width 4096).
-def chosen_pays(rows: int, gu_w: torch.Tensor) -> bool:
-    """Do ``rows`` rows run faster on their chosen experts' own rows than on all experts?"""
+# thin GEMM still has the smaller stacks (width 1024, 8 experts of 704, top 2, 48 rows: 32 us against 39).  Beyond, a layer's
+# time from weights in HBM, dense -> chosen in us (bf16, experts of 2.75 / 4 of the width):
+#   16 experts  width 1024: 72 rows 53 -> 46, 256 63 -> 50;  1536: 118 -> 64, 158 -> 69;  2048, top 3 and a shared one: 33 rows
+#               156 -> 90, 72 100 -> 91, 512 167 -> 99;  4096: 8192 rows 2721 (the library's grouped product) -> 1685
+#   8 experts   width 4096: 33 rows 243 -> 153, 72 169 -> 154;  3072: 152 -> 103, 110 -> 103
+#               but 1024: 72 rows 39 -> 43, 160 43 -> 44, 320 55 -> 46;  1536: 72 55 -> 61, 160 60 -> 61, 192 77 -> 63;  2048: 33
+#               62 -> 68, 72 61 -> 69, 160 69 -> 70, 192 71 -> 72, 256 76 -> 74, 512 96 -> 79
+#   4 experts   width 2048, top 1: 72 rows 38 -> 58, 512 64 -> 68, 768 81 -> 68;  4096: 72 86 -> 104, 256 112 -> 115, 320 126 -> 118
+# A tile of rows per expert costs the same at any width, and few experts leave the dense product little to spare: they
+# take their own rows from where that pays.  (Widths below 1024, which no served layer has: not measured, by row count alone.)
+CHOSEN_MANY_EXPERTS, CHOSEN_WIDE = 16, 3072
+
+
+def chosen_pays(rows: int, gu_w: torch.Tensor, E: int) -> bool:
+    """Do ``rows`` rows run faster on their chosen experts' own rows than on all ``E`` experts?"""
+    W = gu_w.shape[1]
+    if E < CHOSEN_MANY_EXPERTS and W >= 1024:
+        least = (0 if E >= 8 else 256) if W >= CHOSEN_WIDE else (160 if E >= 8 else 512)
+        if rows <= least:
+            return False
     return rows > THIN_MAX_M or rows > THIN_ACT_MAX_M and gu_w.numel() > THIN_BATCH_MAX_W
 
 
@@ -577,7 +591,7 @@ def moe(h, wts, gu_w, down_w, E: int, top: int, ff: int, ffs: int, act="silu",
     expert in ``gu_w`` (``act`` also a ``ClampedGate``); else W_down act(W_up h) with the up rows
     alone.  ``weigh`` = "input": an expert sees its weight times h instead of weighing in with its
     output (gated experts)."""
-    if chosen_pays(h.shape[0], gu_w) and chosen_ok(h, wts, gu_w, down_w, E, top, ff, ffs, act, gated, weigh):
+    if chosen_pays(h.shape[0], gu_w, E) and chosen_ok(h, wts, gu_w, down_w, E, top, ff, ffs, act, gated, weigh):
         return moe_chosen(h, wts, gu_w, down_w, E, top, ff, ffs, act, gated, weigh, True)
     grouped = (grouped_pays(h.shape[0], E, top, (2 if gated else 1) * ff * h.shape[1])
                and not (h.is_cuda and torch.cuda.is_current_stream_capturing()))

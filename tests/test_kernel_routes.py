@@ -253,3 +253,11 @@ def test_decode_plans_are_read_for_calls_that_can_use_one(monkeypatch, tmp_path)
     monkeypatch.setattr(torch.Tensor, "is_cuda", True)
     monkeypatch.setattr(gemm, "DGEMM", False)
     assert gemm.dg_plan(x, w) is None
+
+
+@pytest.mark.parametrize("E,W,ff,most", [(8, 1024, 704, 160), (8, 2048, 1408, 160), (4, 2048, 1408, 512), (4, 4096, 2816, 256),
+                                         (8, 4096, 2816, 32), (16, 1024, 704, 64), (16, 2048, 1408, 32), (8, 256, 128, 64)])
+def test_experts_own_rows_from_where_they_pay(E, W, ff, most):
+    """``most``: the most rows that all experts serve; a few experts of a narrow layer serve more of them."""
+    gu = torch.empty(2 * E * ff, W, device="meta")
+    assert not M.chosen_pays(most, gu, E) and M.chosen_pays(most + 1, gu, E)

@@ -65,6 +65,37 @@ def test_new_tokens(D, nh, nkv, dt, fp8):
         assert torch.equal(got[0], v)
 
 
+@pytest.mark.parametrize("D,nh,nkv,dt,fp8", [
+    (128, 8, 8, torch.bfloat16, False), (128, 32, 8, torch.bfloat16, True), (64, 16, 8, torch.float16, False),
+    (128, 8, 8, torch.float16, False), (32, 8, 8, torch.float16, False), (256, 8, 8, torch.float16, False)])
+@pytest.mark.parametrize("part", [128, 512])
+def test_large_batches_walk_the_heads_first(D, nh, nkv, dt, fp8, part):
+    """From 512 (sequence, key head) pairs on the grid's axes change places: ragged contexts over several partitions, with
+    and without the step's own tokens; a few of the sequences alone, which keep the other grid, give the same bits."""
+    from lumen.ops.attention import paged_decode, paged_decode_new, paged_decode_ref, rope_write_kv
+
+    lens = [1 + (i * 97) % 701 for i in range(64)]                   # 64 x 8 pairs; a few x 8
+    qkv, kc, vc, bt, cl, pos, slots, cos, sin = _case(D, nh, nkv, lens, dt, fp8, 3)
+    scale, few = 1 / math.sqrt(D), 9
+    x, k2, v2 = qkv.clone(), kc.clone(), vc.clone()
+    rope_write_kv(x, pos, nh, nkv, D, cos, sin, k2, v2, slots)
+    q = x[:, :nh * D].view(len(lens), nh, D)
+    ref = paged_decode_ref(q.float(), k2.float(), v2.float(), bt, cl, scale)
+    for n in (len(lens), few):
+        k1, v1 = kc.clone(), vc.clone()
+        got = paged_decode_new(qkv[:n], k1, v1, pos[:n], cos, sin, slots[:n], bt[:n], cl[:n], 701, nh, scale, part)
+        old = paged_decode(q[:n], k2, v2, bt[:n], cl[:n], 701, scale, part)
+        if n > few:
+            assert torch.equal(k1.view(torch.uint8), k2.view(torch.uint8))
+            assert torch.equal(v1.view(torch.uint8), v2.view(torch.uint8))
+            all_new, all_old = got, old
+        for y in (got, old):
+            # the result's rounding and the weights' and sums' in fp32, relative to the largest entry
+            err = (y.float() - ref[:n]).abs().max() / ref.abs().max()
+            assert err < (2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11) * 1.1
+    assert torch.equal(got, all_new[:few]) and torch.equal(old, all_old[:few])
+
+
 def test_refused():
     """Rows the kernel cannot take stay with the two-launch form; what does not fit is an error."""
     from lumen.ops.attention import paged_decode_new_ok

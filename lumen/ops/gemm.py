@@ -172,8 +172,7 @@ def mid_slabs(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 ROW_MAX_K = 8192          # K a workgroup of seqmix/row_gemv.hip holds
 
 
-def row_norm_ok(x: torch.Tensor, norm_w: torch.Tensor, res: Optional[torch.Tensor], w: torch.Tensor,
-                gated: bool = False) -> bool:
+def row_norm_ok(x: torch.Tensor, norm_w: torch.Tensor, res: Optional[torch.Tensor], w: torch.Tensor) -> bool:
     """Can ``row_norm_linear`` run: one row, everything contiguous, of one 16-bit type and on one device?"""
     xs = x.shape
     if len(xs) != 2 or xs[0] != 1 or not x.is_cuda or w.dim() != 2:
@@ -306,7 +305,7 @@ def _thin_tail(x, w, tanh_from: int = 1 << 30, cache=None, cache_from: int = 0, 
     return y
 
 
-def project_tanh(x: torch.Tensor, w: torch.Tensor, start: int = 0) -> torch.Tensor:
+def project_tanh(x: torch.Tensor, w: torch.Tensor, start: int = 0) -> tuple:
     """x @ w^T and the tanh of its columns from ``start`` on: (the columns before, which are left as they are and are
     only valid there; the tanh's) as views or tensors of their own.  Few rows form it in the epilogue, from the fp32 sums."""
     if 0 <= start < w.shape[0] and thin_ok(x, w):

@@ -175,13 +175,6 @@ def _route_rows(kind, x, y, h, norm, post, eps, router, bias, top, groups=0, kee
 _NONE3 = (None, None, None)
 
 
-def routed_topk(h: torch.Tensor, router: torch.Tensor, bias: Optional[torch.Tensor], top: int) -> torch.Tensor:
-    """``route_topk`` of ``router_logits``."""
-    if _route_rows_ok(h, router, bias, None, top, 0, 0, 1):
-        return _route_rows(0, None, None, h, _NONE3, _NONE3, 0.0, router, bias, top)
-    return route_topk(router_logits(h, router, bias), top)
-
-
 def routed_groups(h: torch.Tensor, router: torch.Tensor, correction: Optional[torch.Tensor], top: int, n_groups: int,
                   keep: int, scale: float = 1.0, sum_eps: float = 1e-20, rank_top: int = 2,
                   score: str = "sigmoid", normalize: bool = True) -> torch.Tensor:

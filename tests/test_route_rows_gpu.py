@@ -3,8 +3,7 @@ import pytest
 import torch
 
 from lumen.ops import moe
-from lumen.ops.moe import (dyt_residual_routed, residual_rms_routed, route_groups_ref, route_topk_ref, routed_groups,
-                           routed_topk)
+from lumen.ops.moe import dyt_residual_routed, residual_rms_routed, route_groups_ref, route_topk_ref, routed_groups
 from lumen.ops.norm import dyt_residual, residual_rms
 
 pytestmark = pytest.mark.gpu
@@ -33,16 +32,16 @@ def _same(got, want, top):
 @pytest.mark.parametrize("T,W,E,top", [(1, 8, 1, 1), (5, 520, 3, 2), (64, 2048, 16, 3), (2, 1024, 64, 8),
                                        (7, 4096, 33, 4), (3, 8192, 9, 9), (1, 2056, 8, 2)])
 def test_given_rows(T, W, E, top, dt, calls):
-    r, h, R, b = _rows(T, W, E, dt)
+    r, h, R, _ = _rows(T, W, E, dt)
     z = h.double() @ R.double().t()
-    _same(routed_topk(h, R, b, top), route_topk_ref(z + b.double(), top).double(), top)
-    _same(routed_topk(torch.cat([h, h], 1)[:, :W], R, None, top), route_topk_ref(z, top).double(), top)
     corr = 0.1 * r(E)
     G = 3 if E % 3 == 0 else 1
     for score, norm in (("sigmoid", True), ("softmax", False)):
         k = min(top, max(1, G - 1) * (E // G))
         got = routed_groups(h, R, corr, k, G, max(1, G - 1), 2.0, 1e-20, 2, score, norm)
         _same(got, route_groups_ref(z.float(), corr, k, G, max(1, G - 1), 2.0, 1e-20, 2, score, norm).double(), k)
+        assert torch.equal(got, routed_groups(torch.cat([h, h], 1)[:, :W], R, corr, k, G, max(1, G - 1), 2.0, 1e-20, 2, score,
+                                              norm))
     assert calls == [0] * 4
 
 
@@ -69,12 +68,11 @@ def test_with_the_norm(T, W, E, top, dt, calls):
 
 
 def test_other_rows_keep_the_separate_launches(calls):
-    r, h, R, b = _rows(4, 64, 8, torch.bfloat16)
-    for hh, RR, bb in ((h[:, ::2], R[:, :32].contiguous(), b), (h.float(), R.float(), b.float()),
-                       (torch.cat([h] * 17), R, b), (h, r(72, 64).bfloat16(), None)):
-        z = hh.double() @ RR.double().t()
-        z = z if bb is None else z + bb.double()
-        _same(routed_topk(hh, RR, bb, 2), route_topk_ref(z, 2).double(), 2)
+    r, h, R, _ = _rows(4, 64, 8, torch.bfloat16)
+    for hh, RR in ((h[:, ::2], R[:, :32].contiguous()), (h.float(), R.float()), (torch.cat([h] * 17), R),
+                   (h, r(72, 64).bfloat16())):
+        z = (hh.double() @ RR.double().t()).float()
+        _same(routed_groups(hh, RR, None, 2, 1, 1), route_groups_ref(z, None, 2, 1, 1, 1.0).double(), 2)
     assert calls == []
     with pytest.raises(ValueError):
         routed_groups(h, R, None, 2, 3, 1)

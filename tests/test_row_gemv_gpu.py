@@ -20,7 +20,7 @@ def test_row_norm_linear(K, N, gated, with_res, dtype, ulp):
     x, w, nw = f(1, K).to(dtype).cuda(), (f(N, K) * K ** -0.5).to(dtype).cuda(), (1 + 0.1 * f(K)).to(dtype).cuda()
     res = (3 * f(1, K)).to(dtype).cuda() if with_res else None
     with torch.no_grad():
-        assert row_norm_ok(x, nw, res, w, gated)
+        assert row_norm_ok(x, nw, res, w)
         y, s = row_norm_linear(x, nw, 1e-5, res, w, gated)
         yn, sn = rms_norm(x, nw, 1e-5, res)
     assert torch.equal(s, sn)
@@ -56,7 +56,7 @@ def test_nothing_behind_a_row_is_read(K, gated):
     w.copy_(torch.randn(N, K, generator=g) * K ** -0.5)
     x, nw = torch.randn(1, K, generator=g).bfloat16().cuda(), torch.ones(K, dtype=torch.bfloat16, device="cuda")
     with torch.no_grad():
-        assert row_norm_ok(x, nw, None, w, gated)
+        assert row_norm_ok(x, nw, None, w)
         y, _ = row_norm_linear(x, nw, 1e-5, None, w, gated)
         ref = rms_norm(x, nw, 1e-5, None)[0].double() @ w.double().t()
     if gated:

@@ -431,7 +431,7 @@ __global__ void __launch_bounds__(256) pa_decode1_kernel(
       const float o = __shfl_xor(v[j], LPT / 2, 64);
       v[j] = d0 < D / 2 ? fmaf(v[j], cs[j], -(o * sn[j])) : fmaf(v[j], cs[j], o * sn[j]);
       // (fp32 first, as there: fp16's mixed fma would round once where that rounds twice, a last bit at ties)
-      asm volatile("" : "+v"(v[j]));
+      if constexpr (std::is_same<T, fp16>::value) asm("" : "+v"(v[j]));
       if (round) v[j] = to_f32(from_f32<T>(v[j]));
     }
   };

@@ -13,7 +13,7 @@
 // ... of the output and walks the tile's keys (coalesced rows).  Scores, norms and the softmax
 // are fp32.  The mask bounds a row's keys by `chunk`, so decode reads at most chunk keys and a
 // split over the keys is not needed.
-#include "seqmix.h"
+#include "mma.h"
 
 using namespace lumen;
 
@@ -303,38 +303,6 @@ chunk_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ 
 //                    (two products), which keeps ~16 mantissa bits of the fp32 weights.
 // Accumulator layout of the 32x32 products: lane l, register 4j + i = row 8j + 4(l >> 5) + i,
 // column l & 31; operand lanes hold k = 8(l >> 5) + 0..7.
-constexpr float kRise = 5.f;      // log of the largest weight a tile may form before its maximum moves the reference
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef __bf16 bf16x8v __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8v __attribute__((ext_vector_type(8)));
-
-template <typename T> struct Mma32;
-template <> struct Mma32<bf16> {
-  static __device__ __forceinline__ f32x16 run(uint4 a, uint4 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8v, a),
-                                                   __builtin_bit_cast(bf16x8v, b), c, 0, 0, 0);
-  }
-};
-template <> struct Mma32<fp16> {
-  static __device__ __forceinline__ f32x16 run(uint4 a, uint4 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8v, a),
-                                                  __builtin_bit_cast(f16x8v, b), c, 0, 0, 0);
-  }
-};
-
-// the two halves of a packed 16-bit pair as fp32 (bf16: a shift and a mask)
-template <typename T> __device__ __forceinline__ void unpack2(unsigned v, float& a, float& b);
-template <> __device__ __forceinline__ void unpack2<bf16>(unsigned v, float& a, float& b) {
-  a = __uint_as_float(v << 16);
-  b = __uint_as_float(v & 0xffff0000u);
-}
-template <> __device__ __forceinline__ void unpack2<fp16>(unsigned v, float& a, float& b) {
-  const lumen_f16x2 h = __builtin_bit_cast(lumen_f16x2, v);
-  a = static_cast<float>(h[0]);
-  b = static_cast<float>(h[1]);
-}
-
 template <typename T>
 __device__ __forceinline__ float sumsq8(uint4 v) {
   const unsigned w[4] = {v.x, v.y, v.z, v.w};

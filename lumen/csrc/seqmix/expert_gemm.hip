@@ -22,28 +22,11 @@
 // 534 -> 283, 512 90 -> 60, 256 62 -> 56; 16, top 3, shared: 4096 1130 -> 371, 512 166 -> 99, 64 149 -> 79; 16 ungated,
 // top 4: 4096 810 -> 298, 8192 at width 4096 2721 (grouped library product) -> 1685.  Error against float64 2.3e-3 where the dense form has 3.5e-3: nothing is rounded between the
 // products and the activation, nor before the sum.
-#include "seqmix.h"
+#include "mma.h"
 
 using namespace lumen;
 
 namespace {
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-template <typename T> struct Mfma;
-template <> struct Mfma<bf16> {
-  static __device__ __forceinline__ f32x4 run(uint4 a, uint4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  }
-};
-template <> struct Mfma<fp16> {
-  static __device__ __forceinline__ f32x4 run(uint4 a, uint4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
-                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  }
-};
 
 constexpr int BM = 128, BN = 256, BK = 64, ROWB = 128;   // pairs, weight rows; a stage row is 64 elements
 constexpr int NI = 8, MJ = 4;                            // fragments of a wave: 128 weight rows x 64 pairs
@@ -53,14 +36,6 @@ constexpr int kMaxE = 64;
 
 __device__ __forceinline__ int swz(int r) { return (r >> 1) & 7; }
 
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0xF70);
-}
-__device__ __forceinline__ void dma16(const void* base, unsigned off, unsigned lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :: "v"(off), "s"(base), "s"(lds) : "memory", "m0");
-}
 __device__ __forceinline__ void done_reading() {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();

@@ -12,23 +12,11 @@
 //                    weights (all of R), joins in the sums, which meet in LDS, and multiplies.
 // Bound by latency.  64 rows x 16 heads, D = 128, R = 512, in a decode step, us: write and norm 10.1 + 4.5 -> 6.2; batched
 // library product and rotation 5.1 + 4.5 -> 7.0; sums of 8 splits and library product 4.9 + 12.7 -> 10.9.
-#include "seqmix.h"
+#include "mma.h"
 
 using namespace lumen;
 
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-template <typename T> __device__ __forceinline__ f32x4 mma(uint4 a, uint4 b, f32x4 c);
-template <> __device__ __forceinline__ f32x4 mma<bf16>(uint4 a, uint4 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-template <> __device__ __forceinline__ f32x4 mma<fp16>(uint4 a, uint4 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
 
 constexpr int kThreads = 256;
 
@@ -121,7 +109,7 @@ __global__ void __launch_bounds__(256) latent_query_kernel(const QueryArgs<T> a)
     if (t0 + 16 * j < a.Tn) {
       f32x4 c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int s = 0; s < KS; ++s) c = mma<T>(x[s], y[j][s], c);
+      for (int s = 0; s < KS; ++s) c = Mfma<T>::run(x[s], y[j][s], c);
       const int t = t0 + 16 * j + lr;                  // lane (lr, lg): row t, columns r0 + 4 lg ..
       if (t < a.Tn)
         *reinterpret_cast<uint2*>(a.out + ((long long)h * a.Tn + t) * a.R + r0 + 4 * lg) =
@@ -191,8 +179,8 @@ __global__ void __launch_bounds__(1024) latent_out_kernel(const OutArgs<T> a) {
   const T* xr = s_x + min(lr, n - 1) * LD + 8 * lg;
 #pragma unroll
   for (int s = 0; s < KS; s += 2) {
-    c0 = mma<T>(u[s], *reinterpret_cast<const uint4*>(xr + 32 * s), c0);
-    c1 = mma<T>(u[s + 1], *reinterpret_cast<const uint4*>(xr + 32 * s + 32), c1);
+    c0 = Mfma<T>::run(u[s], *reinterpret_cast<const uint4*>(xr + 32 * s), c0);
+    c1 = Mfma<T>::run(u[s + 1], *reinterpret_cast<const uint4*>(xr + 32 * s + 32), c1);
   }
   c0 += c1;
   if (lr < n)                                          // lane (lr, lg): row t0 + lr, columns 16 w + 4 lg ..

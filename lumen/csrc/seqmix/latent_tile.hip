@@ -23,28 +23,11 @@
 // hence the rule in ops/attention.py.  A tile costs a wave ~5.9 us, twice its matrix instructions' time: one
 // wave per SIMD, whose softmax and masks do not overlap its products.  Eight waves of one row each were
 // slower (231 us): operand reads double and the accumulators spill.
-#include "seqmix.h"
+#include "mma.h"
 
 using namespace lumen;
 
 namespace {
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-template <typename T> struct Mfma;
-template <> struct Mfma<bf16> {
-  static __device__ __forceinline__ f32x4 run(uint4 a, uint4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  }
-};
-template <> struct Mfma<fp16> {
-  static __device__ __forceinline__ f32x4 run(uint4 a, uint4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
-                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  }
-};
 
 constexpr int kRows = 8;          // rows of a workgroup (two per wave)
 constexpr int kKeys = 32;         // keys per tile

@@ -13,39 +13,15 @@
 // 12.3 -> 10.3, 8.6 -> 7.7, 8.4 -> 7.3, 25.8 -> 24.2, 19.1 -> 17.4); gate, up and activation 5632 x 2048 20.3 -> 15.7, 2816 x 1024
 // 13.0 -> 8.8; without a gate 5632 x 2048 16.9 -> 13.6, 11264 x 4096 31.3 -> 27.2.  One round of tiles only: a workgroup
 // fills a CU's LDS, so 264 tiles (gated 8448 x 3072) take two, 34.9 -> 38.1, and stay with the separate launches.
-#include "seqmix.h"
+#include "mma.h"
 
 using namespace lumen;
 
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-template <typename T> __device__ __forceinline__ f32x4 mma(uint4 a, uint4 b, f32x4 c);
-template <> __device__ __forceinline__ f32x4 mma<bf16>(uint4 a, uint4 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-template <> __device__ __forceinline__ f32x4 mma<fp16>(uint4 a, uint4 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
-
 constexpr int BM = 64, BN = 64, BK = 128, ROWB = 2 * BK;     // a row of a stage: 16 chunks of 16 bytes
 constexpr int STAGE = (BM + BN) * ROWB, D = 4;               // 32 KiB
 constexpr int PIECES = STAGE / 1024 / 4;                     // LDS-DMA instructions of a wave and stage
-
-template <int N> __device__ __forceinline__ void wait_vm() {
-  static_assert(N >= 0 && N < 64, "vmcnt");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0xF70);
-}
-
-// LDS-DMA of 16 bytes per lane (uniform base, 32-bit lane offset, M0: the wave's 1-KiB piece).  Inline asm, so that
-// this kernel's own counted waits order it.
-__device__ __forceinline__ void dma16(const void* base, unsigned off, unsigned lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :: "v"(off), "s"(base), "s"(lds) : "memory", "m0");
-}
 
 struct MidArgs {
   const void *x, *W;
@@ -116,7 +92,7 @@ __global__ void __launch_bounds__(256, 1) mid_kernel(const MidArgs p) {
 #pragma unroll
     for (int s = 0; s < BK / 32; ++s)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] = mma<T>(a[s][i], b[s], acc[i]);
+      for (int i = 0; i < 4; ++i) acc[i] = Mfma<T>::run(a[s][i], b[s], acc[i]);
   }
   const int m = 16 * wid + lr;         // lane (lr, lg): row m, columns 16 i + 4 lg .. of the tile
   if (m >= p.M) return;

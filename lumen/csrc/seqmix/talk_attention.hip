@@ -27,46 +27,18 @@
 // Error: the row kernel's.  Share of results that are not float64's rounded, row kernel / here: bf16 0.0003 / 0.0003,
 // fp16 0.0022 / 0.0022.  (Two parts and the hardware's exponential, logarithm and reciprocal as they are: 0.0025 and
 // 0.0115, at 100 us for the 14 prompts; three parts alone 104; expf, logf and tanhf 117, with the same error.)
-#include "seqmix.h"
+#include "mma.h"
 
 using namespace lumen;
 
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-template <typename T> struct Mfma;
-template <> struct Mfma<bf16> {
-  static __device__ __forceinline__ f32x4 run(uint4 a, uint4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  }
-};
-template <> struct Mfma<fp16> {
-  static __device__ __forceinline__ f32x4 run(uint4 a, uint4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
-                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  }
-};
-
 constexpr int kD = 128, kRows = 16, kKeys = 32, kTbl = 512;
 // fp16: weights up to e^kRise times this fit, and the parts of small ones stay above its subnormals' grain
 template <typename T> constexpr float kUp = 1.f;
 template <> constexpr float kUp<fp16> = 128.f;
-template <typename T> __device__ __forceinline__ void unpack2(unsigned u, float& a, float& b);
-template <> __device__ __forceinline__ void unpack2<bf16>(unsigned u, float& a, float& b) {
-  a = __uint_as_float(u << 16);
-  b = __uint_as_float(u & 0xffff0000u);
-}
-template <> __device__ __forceinline__ void unpack2<fp16>(unsigned u, float& a, float& b) {
-  const auto h = __builtin_bit_cast(lumen_f16x2, u);
-  a = static_cast<float>(h[0]);
-  b = static_cast<float>(h[1]);
-}
-constexpr float kRise = 5.f;      // log of the largest weight a tile may form before its maximum moves the reference
 
 template <typename T> struct TalkArgs {
   const T* q; long long qr, qh;

@@ -39,41 +39,17 @@
 // turns a projection's last columns (tanh) or copies them into a cache, likewise.
 // From 33 rows on every tile re-reads more x than W, so the widest matrices stay with the library
 // there; at M = 1 the GEMV stays ahead on long rows (ops/gemm.py has the rule).
-#include "seqmix.h"
+#include "mma.h"
 
 using namespace lumen;
 
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-template <typename T> struct Mfma;
-template <> struct Mfma<bf16> {
-  static __device__ __forceinline__ f32x4 run(uint4 a, uint4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  }
-};
-template <> struct Mfma<fp16> {
-  static __device__ __forceinline__ f32x4 run(uint4 a, uint4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
-                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  }
-};
 
 constexpr int BK = 64, ROWB = 128;   // k per stage, bytes of an image row
 
 // 16-byte chunk c of image row r lives at chunk c ^ swz(r): a fragment read (16 rows at one chunk)
 // touches 16 different bank slots
 __device__ __forceinline__ int swz(int r) { return (r >> 1) & 7; }
-
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  static_assert(N >= 0 && N < 64, "vmcnt");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0xF70);
-}
 
 // LDS-DMA of 16 bytes per lane (wave-uniform base + 32-bit lane offset) as inline asm, so that the
 // compiler does not drain the ring before the next fragment read; the counted waits below order it

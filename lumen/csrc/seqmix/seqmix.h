@@ -16,8 +16,10 @@ __device__ __forceinline__ float dyt_f(float x, float alpha, float w, float b) {
   return tanhf(alpha * x) * w + b;
 }
 
-// As near to the exact values as expf, logf, tanhf and an exact division, from the hardware's 2^t, log2 and
-// reciprocal with their roundings made good: at a third of the instructions, for the inner loops that those bound.
+// expf, logf, tanhf and an exact division from the hardware's 2^t, log2 and reciprocal with their roundings made good,
+// at a third of the instructions, for the inner loops that those bound.  Largest error in units of the last place,
+// the library's -> here (4 M values each): e^x, -80 .. 5: 0.85 -> 1.25 (the hardware's form as it is 62); ln, 1 .. 500: 2.3 -> 2.1;
+// tanh 1.4 -> 2.2; sigmoid, -60 .. 60: 2.5 -> 3.4 (58).
 // e^x for x up to 88 (more: as 88; below -200: 0)
 __device__ __forceinline__ float exp_near(float x) {
   constexpr float kL = 1.44269502f, kLlo = 1.92596299e-8f;     // log2(e) = kL + kLlo
@@ -39,14 +41,14 @@ __device__ __forceinline__ float log_near(float x) {
   return r + fmaf(y, kLlo, fmaf(y, kL, -r));
 }
 // tanh x: near 0 an odd polynomial (least squares in x^2, weighted to an even relative error of 3e-10), else through
-// one exponential
+// one exponential of |x|
 __device__ __forceinline__ float tanh_near(float x) {
   const float z = x * x;
   float p = fmaf(z, -0.00665356684f, 0.0213016998f);
   p = fmaf(z, p, -0.0538999699f);
   p = fmaf(z, p, 0.133329704f);
   p = fmaf(z, p, -0.333333284f);
-  return z < 0.25f ? fmaf(x, z * p, x) : 1.f - 2.f * recip_near(1.f + exp_near(2.f * x));
+  return z < 0.25f ? fmaf(x, z * p, x) : copysignf(1.f - 2.f * recip_near(1.f + exp_near(2.f * fabsf(x))), x);
 }
 
 // four consecutive elements as one vector access (16 bytes of fp32, 8 bytes of a 16-bit type)

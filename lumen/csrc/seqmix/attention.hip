@@ -574,12 +574,12 @@ tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ c
   l += __shfl_xor(l, 32, 64);
   // A hidden key has weight 0, but 0 times an infinite or NaN value is NaN: channels that are not finite are formed
   // again, key by key over what the row sees (m and l stand).
-  bool odd = false;
+  float odd[4] = {0.f, 0.f, 0.f, 0.f};             // (0 times a finite number stays 0)
 #pragma unroll
   for (int db = 0; db < D / 32; ++db)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) odd |= !(fabsf(O[db][r]) < INFINITY);
-  if (__builtin_expect(__any(odd && qv), 0)) {
+    for (int r = 0; r < 16; ++r) odd[r & 3] = fmaf(O[db][r], 0.f, odd[r & 3]);
+  if (__builtin_expect(__any(odd[0] + odd[1] + odd[2] + odd[3] != 0.f && qv), 0)) {
 #pragma unroll
     for (int db = 0; db < D / 32; ++db) {
       f32x16 o;

@@ -25,7 +25,8 @@
 // the maximum only when it rises by kRise.  Measured (us, tiles of 32 keys, one buffer -> now; bf16, heads of
 // 128, soft cap): 1 x 512 rows x 32 heads 55 -> 33, 8 x 512 x 16 91 -> 43, 14 of 63 - 509 x 16 110 -> 58, 1 x 4096 x 32
 // (window 1024) 380 -> 168; heads of 64 44 -> 23, of 256 191 -> 113, values of 256 169 -> 101; the look for infinite
-// results at the end, which later came to it, 1 - 2 us (8 x 512 x 16 43.9 -> 45.5).
+// results at the end, which later came to it, 0.1 - 1.3 us (8 x 512 x 16 39.0 -> 39.7, 1 x 64 9.2 -> 9.5; with a comparison
+// per result 0.3 - 1.9).  A portion of few keys pays for a whole tile of 64 (1 x 16 7.4 -> 9.0, 64 x 5 x 32 heads 22 -> 31).
 //
 // Per wave (32 queries) and 32 keys, with v_mfma_f32_32x32x16:
 //   S^T = K Q^T      keys on the accumulator rows, queries on the columns (lane & 31): a lane
@@ -368,12 +369,12 @@ win_tile_attn_kernel(const WinTileArgs<T> a) {
   l += __shfl_xor(l, 32, 64);
   // A hidden key has weight 0, but 0 times an infinite or NaN value is NaN: channels that are not finite are formed
   // again, key by key over what the row sees (m and l stand).
-  bool odd = false;
+  float odd[4] = {0.f, 0.f, 0.f, 0.f};             // (0 times a finite number stays 0)
 #pragma unroll
   for (int db = 0; db < DV / 32; ++db)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) odd |= !(fabsf(O[db][r]) < INFINITY);
-  if (__builtin_expect(__any(odd && qv), 0)) {
+    for (int r = 0; r < 16; ++r) odd[r & 3] = fmaf(O[db][r], 0.f, odd[r & 3]);
+  if (__builtin_expect(__any(odd[0] + odd[1] + odd[2] + odd[3] != 0.f && qv), 0)) {
 #pragma unroll
     for (int db = 0; db < DV / 32; ++db) {
       f32x16 o;

@@ -676,6 +676,12 @@ def latent_write(z: torch.Tensor, w_norm: torch.Tensor, inv_freq: torch.Tensor,
 
 
 LATENT_STEP_MAX_T = 512      # rows; more fill the chip with a wave per row
+# Multiply-adds up to which the small kernels of the absorbed query and of the expansion are ahead of the library's batched
+# product with the rotation, or the splits' sums, beside it (us, library and kernel, latent 512, heads of 128): query, 16 heads
+# 64 rows 7.6 and 5.4, 128 7.9 and 7.9, 256 8.9 and 10.6; 32 heads 64 8.1 and 8.1, 128 9.2 and 10.7; 64 heads 32 9.0 and 7.4, 64 9.6
+# and 10.9; heads of 192, 16 of them, 64 7.6 and 6.7, 128 8.5 and 10.3.  Attention and expansion: 16 heads 256 57.9 and 47.2, 384
+# 62.4 and 60.8, 512 65.3 and 68.2; 64 heads 64 46.6 and 41.4, 128 52.7 and 57.4.
+LATENT_QUERY_MAX, LATENT_EXPAND_MAX = 1 << 27, 1 << 28
 
 
 def latent_inputs(z: torch.Tensor, Q: int, wq: torch.Tensor, w_norm: torch.Tensor, inv_freq: Optional[torch.Tensor],
@@ -711,8 +717,8 @@ def latent_query(q: torch.Tensor, uk: torch.Tensor, ukT: torch.Tensor, D: int, p
 
     T, H, N = q.shape
     R = ukT.shape[1]
-    if (not 0 < T <= LATENT_STEP_MAX_T or not use_seqmix(q) or q.dtype not in (torch.bfloat16, torch.float16)
-            or D not in (64, 128, 192, 256) or R % 64 or N % 8 or q.stride(2) != 1 or q.stride(1) != N
+    if (not 0 < T <= LATENT_STEP_MAX_T or T * H * D * R > LATENT_QUERY_MAX or not use_seqmix(q)
+            or q.dtype not in (torch.bfloat16, torch.float16) or D not in (64, 128, 192, 256) or R % 64 or N % 8 or q.stride(2) != 1 or q.stride(1) != N
             or q.stride(0) % 8 or ukT.dtype != q.dtype or tuple(ukT.shape) != (H, R, D) or not ukT.is_contiguous()
             or (q.data_ptr() | ukT.data_ptr()) % 16 or not _plain(q, ukT) or not _here(q)):
         if dims:
@@ -1041,6 +1047,7 @@ def _expand_ok(expand: tuple, q1: torch.Tensor, T: int, H: int, R: int) -> bool:
 
     uv, o = expand
     return (T <= LATENT_STEP_MAX_T and R in (64, 128, 256, 512) and uv.dim() == 3 and uv.shape[0] == H
+            and T * H * R * uv.shape[1] <= LATENT_EXPAND_MAX
             and uv.shape[2] == R and uv.shape[1] % 16 == 0 and 0 < uv.shape[1] <= 256 and uv.is_contiguous()
             and uv.data_ptr() % 16 == 0 and uv.dtype == q1.dtype == o.dtype and tuple(o.shape) == (T, H, uv.shape[1])
             and o.stride(2) == 1 and o.stride(0) % 4 == 0 and o.stride(1) % 4 == 0 and o.data_ptr() % 8 == 0

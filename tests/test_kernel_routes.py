@@ -261,3 +261,25 @@ def test_experts_own_rows_from_where_they_pay(E, W, ff, most):
     """``most``: the most rows that all experts serve; a few experts of a narrow layer serve more of them."""
     gu = torch.empty(2 * E * ff, W, device="meta")
     assert not M.chosen_pays(most, gu, E) and M.chosen_pays(most + 1, gu, E)
+
+
+def test_latent_products_of_many_rows_keep_the_library(launched, monkeypatch):
+    from lumen.ops import attention as A
+
+    def run(T, H, D, R):
+        launched.clear()
+        q, uk = torch.zeros(T, H, D + 64, **BF), torch.zeros(H, D, R, **BF)
+        assert A.latent_query(q, uk, uk.transpose(1, 2).contiguous(), D, torch.zeros(T, **i32)).shape == (H, T, R)
+        return len(launched)
+
+    i32 = dict(dtype=torch.int32)
+    assert [run(*s) for s in ((1, 64, 128, 512), (128, 16, 128, 512), (129, 16, 128, 512), (64, 64, 128, 512), (512, 4, 128, 512),
+                              (512, 16, 64, 128))] == [1, 1, 0, 0, 1, 1]
+    monkeypatch.setattr(gemm, "_here", lambda *a: True)
+
+    def expand(T, H, R, Dv):
+        uv, o = torch.zeros(H, Dv, R, **BF), torch.zeros(T, H, Dv, **BF)
+        return A._expand_ok((uv, o), torch.zeros(1, **BF), T, H, R)
+
+    assert [expand(*s) for s in ((1, 64, 512, 128), (256, 16, 512, 128), (257, 16, 512, 128), (64, 64, 512, 128), (65, 64, 512, 128),
+                                 (512, 4, 512, 128))] == [True, True, False, True, False, True]

@@ -129,14 +129,26 @@ def route_groups(z: torch.Tensor, correction: Optional[torch.Tensor], top: int, 
 ROUTE_MAX_M, ROUTE_MAX_E, ROUTE_MAX_W = 64, 64, 8192
 
 
+def _route_rows_pay(rows: int, W: int, E: int, normed: bool) -> bool:
+    """A workgroup reads the whole router, and few rows have few workgroups: a large one is better read by the thin GEMM
+    (us, separate launches and one, 1 / 16 / 32 / 64 rows.  Given rows, experts x width: 64 x 2048 7.6 and 7.8, 8.1 and 8.0, -, 10.5
+    and 8.1; 64 x 3072 8.4 and 10.4, 8.8 and 10.8, 9.9 and 10.7, 12.2 and 10.8; 64 x 8192 10.3 and 16.3, 12.7 and 17.1, -, 21.1 and 17.1; 48 x
+    4096 9.2 and 9.5, 9.5 and 9.9, 11.0 and 9.8, 13.9 and 9.9; 32 x 6144 9.2 and 10.4, 11.2 and 10.8, 13.4 and 10.8, 17.5 and 10.8.
+    With the norm: 64 x 4096 13.1 and 12.0 for one; 64 x 8192 15.3 and 17.8, -, 21.5 and 18.8)."""
+    if normed:
+        return E * W <= 1 << 18 or rows >= E // 2
+    return E * W < 3 << 16 or rows >= E - 16
+
+
 def _route_rows_ok(h: torch.Tensor, router: torch.Tensor, bias, correction, top: int, groups: int, keep: int,
-                   rank_top: int) -> bool:
-    """``h``: the normed rows, or the sublayer's output that the stream takes before the norm."""
+                   rank_top: int, normed: bool = False) -> bool:
+    """``h``: the normed rows, or (``normed``: the launch norms) the sublayer's output that the stream takes first."""
     if h.dim() != 2 or not 0 < h.shape[0] <= ROUTE_MAX_M or not h.is_cuda or router.dim() != 2:
         return False
     (E, W), dt = router.shape, h.dtype
     if (W != h.shape[1] or W % 8 or not 0 < W <= ROUTE_MAX_W or not 0 < E <= ROUTE_MAX_E or dt != router.dtype
             or dt not in (torch.bfloat16, torch.float16) or router.device != h.device or not router.is_contiguous()
+            or not _route_rows_pay(h.shape[0], W, E, normed)
             or not row_bias_ok(bias, h, E) or not _plain(h, router) or not _here(h)):
         return False
     if bias is not None and not _plain(bias) or correction is not None and not (
@@ -192,7 +204,7 @@ def residual_rms_routed(x: torch.Tensor, y: torch.Tensor, w: torch.Tensor, eps: 
     group): (h, weights)."""
     from .norm import residual_rms
 
-    if _route_rows_ok(y, router, None, None, top, 1, 1, 1) and _stream_ok(x, y, (w,)):
+    if _route_rows_ok(y, router, None, None, top, 1, 1, 1, True) and _stream_ok(x, y, (w,)):
         h = torch.empty_like(y)
         return h, _route_rows(1, x, y, h, (w, None, None), _NONE3, eps, router, None, top, 1, 1, 1, False, normalize,
                               1.0, 1e-20)
@@ -205,7 +217,7 @@ def dyt_residual_routed(x: torch.Tensor, y: torch.Tensor, post, pre, router: tor
     """``dyt_residual`` into the experts' input h, and its routing over the ``top`` logits: (x, h, weights)."""
     from .norm import dyt_residual
 
-    if y.dtype == dtype and _route_rows_ok(y, router, bias, None, top, 0, 0, 1) \
+    if y.dtype == dtype and _route_rows_ok(y, router, bias, None, top, 0, 0, 1, True) \
             and _stream_ok(x, y, (*post[:2], *pre[:2]), (post[2], pre[2])):
         h = torch.empty_like(y)
         return x, h, _route_rows(2, x, y, h, pre, post, 0.0, router, bias, top)

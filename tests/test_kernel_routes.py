@@ -283,3 +283,11 @@ def test_latent_products_of_many_rows_keep_the_library(launched, monkeypatch):
 
     assert [expand(*s) for s in ((1, 64, 512, 128), (256, 16, 512, 128), (257, 16, 512, 128), (64, 64, 512, 128), (65, 64, 512, 128),
                                  (512, 4, 512, 128))] == [True, True, False, True, False, True]
+
+
+@pytest.mark.parametrize("normed,sizes", [
+    (False, ((1, 2048, 64, 1), (47, 3072, 64, 0), (48, 3072, 64, 1), (1, 8192, 64, 0), (1, 8192, 16, 1), (15, 6144, 32, 0),
+             (16, 6144, 32, 1), (7, 4096, 33, 1))),
+    (True, ((1, 4096, 64, 1), (31, 8192, 64, 0), (32, 8192, 64, 1), (1, 8192, 32, 1)))])
+def test_large_routers_of_few_rows_keep_the_thin_gemm(normed, sizes):
+    assert [M._route_rows_pay(T, W, E, normed) for T, W, E, _ in sizes] == [bool(s[3]) for s in sizes]

@@ -21,9 +21,9 @@
 // all three steps touch four different groups of 16 banks at a time.
 // Bound by the chain of tiles at two waves per SIMD (~14000 cycles per 32 keys, a third of it the shaping's
 // transcendentals).  Measured against the row kernel (us, bf16, one key head per four heads, everything on): 16 heads,
-// 14 prompts of 63 - 509 tokens 515 -> 107, 1 x 512 148 -> 101, 1 x 200 48 -> 47, 1 x 128 30 -> 30, 1 x 24 22 -> 15; 8
-// heads, 1 x 2048 755 -> 275; 32 heads, 8 of 32 - 256 316 -> 130, 1 x 2048 5248 -> 930, 1 x 80 57 -> 58: prompts of every
-// length take it.
+// 14 prompts of 63 - 509 tokens 515 -> 107, 1 x 512 148 -> 101, 1 x 24 22 -> 15; 8 heads, 1 x 2048 755 -> 275; 32 heads, 8
+// of 32 - 256 316 -> 130, 1 x 2048 5248 -> 930.  Few rows behind many keys have short work in a long chain and stay with
+// the row kernel (16 heads, 16 rows behind 1024 keys: 31 us there, 198 here).
 // Error: the row kernel's.  Share of results that are not float64's rounded, row kernel / here: bf16 0.0003 / 0.0003,
 // fp16 0.0022 / 0.0022.  (Two parts and the hardware's exponential, logarithm and reciprocal as they are: 0.0025 and
 // 0.0115, at 100 us for the 14 prompts; three parts alone 104; expf, logf and tanhf 117, with the same error.)

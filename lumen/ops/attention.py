@@ -1041,6 +1041,18 @@ def _heads_per_block(H: int, Dk: int, need_all: bool) -> int:
 LATENT_TILE_ROWS = 2048      # rows x 16-head blocks from which prompt portions take the tiled latent kernel
 
 
+def _talk_tiles_pay(seg, block: int) -> bool:
+    """Mixed heads: do the prompt portions go to the tiles?  A tile walks its rows' keys in one chain, so its launch takes
+    the longest portion's keys, whatever the rows are; the row kernel takes the pairs of rows and keys and, up to 256 rows,
+    deals a row's keys out.  They meet where the pairs make 256 to 320 rows of the longest portion's keys (us, row kernel
+    and tiles, 8 / 16 / 32 heads: 2 rows behind 512 keys 20 and 74, 30 and 101, 58 and 231; 16 x 16 rows behind 1024 94 and 145,
+    187 and 209, 414 and 496; 64 x 5 rows 190 and 157, 338 and 210, 839 and 487; 256 rows behind 4096 377 and 617, 677 and 838, 1565
+    and 1977; 512 732 and 652, 1311 and 884, 3070 and 2084; whole prompts of 256 rows 31 and 40, 52 and 56, 111 and 128; 320 56 and
+    48, 98 and 67, 222 and 156).  Short chains cost the launch (a prompt of 96 rows 19 and 19, 30 and 27, 57 and 57)."""
+    pairs, longest = seg.prompt_keys(block)
+    return longest <= 96 or pairs > 256 * longest
+
+
 def _expand_ok(expand: tuple, q1: torch.Tensor, T: int, H: int, R: int) -> bool:
     """Does sm_latent_out take these rows?"""
     from .gemm import _here, _plain
@@ -1196,6 +1208,7 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
         gate = gate[Tp:] if gate is not None else None
     # mixed heads: 16 rows and all heads of a tile on the matrix cores
     elif (talk is not None and seg.q_tiles is not None and seg.tile_rows > 0 and q2 is None and slopes is None
+            and _talk_tiles_pay(seg, bs)
             and window == 0 and gate is None and sigmoid_bias is None and v_div == 1
             and vcache is not kcache and krow == G * D1 and vrow == G * Dv
             and q1.dtype in (torch.bfloat16, torch.float16) and talk_tiles_ok(DT[q1.dtype], H, G, D1, Dv)

@@ -28,6 +28,8 @@ class SegBatch:
     tile_rows: int = 0
     tile_size: int = 64       # rows per tile of q_tiles (TILE_ROWS when they were cut)
     fresh: bool = False       # every portion starts at position 0: its keys are rows of this step
+    # the portions' (pairs of rows and keys, keys of the longest), where the host has counted them
+    keys: Optional[tuple] = None
 
     @property
     def S(self) -> int:
@@ -45,12 +47,20 @@ class SegBatch:
             return self.S - (self.T - self.tile_rows), self.tile_rows
         return (0, 0) if self.S == self.T else (self.S, self.T)
 
+    def prompt_keys(self, block: int) -> tuple:
+        """The prompt portions' (pairs of rows and keys, keys of the longest): ``keys``, or what the width of the tables
+        of cache blocks of ``block`` rows allows."""
+        if self.keys is not None:
+            return self.keys
+        longest = self.tables.shape[1] * block
+        return self.portions()[1] * longest, longest
+
     def decoded(self) -> "SegBatch":
         """The rows after the prompt portions, with the step's segments, offsets and tables: what a row's
         attention reads (``row_seg``, ``positions``, ``tables``, ``cache_slots``)."""
         n = self.tile_rows
         return replace(self, row_seg=self.row_seg[n:], positions=self.positions[n:], q_tiles=None, tile_rows=0,
-                       fresh=False, cache_slots=None if self.cache_slots is None else self.cache_slots[n:])
+                       fresh=False, keys=None, cache_slots=None if self.cache_slots is None else self.cache_slots[n:])
 
 
 import os
@@ -70,8 +80,19 @@ def tile_list(cu, n_segments: int, rows: int = 0):
 def whole_prompts(cu, kv_lens, tile_rows: int) -> bool:
     """Do the portions of row offsets ``cu`` (host ints) that make a step's first ``tile_rows`` rows all start at
     position 0, i.e. has each as many rows as its sequence has keys (``kv_lens``, host)?"""
+    return _portions(cu, kv_lens, tile_rows) and all(b - a == n for a, b, n in zip(cu, cu[1:], kv_lens))
+
+
+def portion_keys(cu, kv_lens, tile_rows: int) -> Optional[tuple]:
+    """(pairs of rows and keys, keys of the longest) of these portions, None where the host does not know them."""
+    if not _portions(cu, kv_lens, tile_rows):
+        return None
+    return sum((b - a) * int(n) for a, b, n in zip(cu, cu[1:], kv_lens)), int(max(kv_lens))
+
+
+def _portions(cu, kv_lens, tile_rows: int) -> bool:
     return (tile_rows > 0 and kv_lens is not None and cu is not None and len(cu) == len(kv_lens) + 1
-            and cu[-1] == tile_rows and all(b - a == n for a, b, n in zip(cu, cu[1:], kv_lens)))
+            and cu[-1] == tile_rows)
 
 
 def whole_sequences(lengths, device, slots=None, block_size: int = 16) -> SegBatch:
@@ -95,4 +116,4 @@ def whole_sequences(lengths, device, slots=None, block_size: int = 16) -> SegBat
     return SegBatch(torch.tensor(cu, **i32),
                     torch.tensor(list(slots) if slots is not None else list(range(S)), **i32),
                     torch.zeros(S, **i32), row_seg, pos, tables, torch.cat(cache_slots),
-                    torch.tensor(tile_list(cu, S), **i32).view(-1, 2), cu[-1], TILE_ROWS, True)
+                    torch.tensor(tile_list(cu, S), **i32).view(-1, 2), cu[-1], TILE_ROWS, True, portion_keys(cu, list(lengths), cu[-1]))

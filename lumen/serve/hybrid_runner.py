@@ -55,7 +55,7 @@ from ..ops.norm import (SPLIT, depth_mix_norm, dyt, dyt_residual, embed_rms, gat
                         project_group_rms, residual_rms, scaled_residual_layer_norm, weight_layer_norm)
 from ..ops.recurrent import delta_scan, head_scan, min_gru_scan, token_shift, wkv_scan
 from ..ops.rope import rotary_write, rotate_interleaved_
-from ..ops.segments import SegBatch, whole_prompts, whole_sequences
+from ..ops.segments import SegBatch, portion_keys, whole_prompts, whole_sequences
 from .model_runner import ModelRunner, StepInput, fill_step
 
 
@@ -337,7 +337,7 @@ class DalavikWeights:
     into one GEMM, the per-head up projections are laid out for batched GEMMs, norm weights and
     the attention's per-head constants are fp32."""
 
-    asks_fresh = True          # latent attention of whole prompts
+    asks_fresh = True          # latent attention of whole prompts; keys of the portions: mixed heads
 
     def __init__(self, model, tp_rank: int = 0, tp_size: int = 1):
         if tp_size != 1:
@@ -1417,9 +1417,9 @@ class HybridRunner(ModelRunner):
     def execute(self, inp: StepInput) -> torch.Tensor:
         seg = inp.seg
         # (short prompts wait for the host: asked where a layer makes use of it)
-        if getattr(self.w, "asks_fresh", False) and not seg.fresh \
-                and whole_prompts(inp.cu_seqlens, inp.kv_lens, seg.tile_rows):
-            seg = replace(seg, fresh=True)
+        if getattr(self.w, "asks_fresh", False):
+            host = (inp.cu_seqlens, inp.kv_lens, seg.tile_rows)
+            seg = replace(seg, fresh=seg.fresh or whole_prompts(*host), keys=seg.keys or portion_keys(*host))
         x = self.w.run_layers(self.state, inp.tokens, seg, self.observe)
         if inp.extra_rows is not None and inp.extra_rows.numel():
             self.extra_logits = self._logits_rows(x, inp.extra_rows)

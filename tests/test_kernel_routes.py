@@ -263,6 +263,35 @@ def test_experts_own_rows_from_where_they_pay(E, W, ff, most):
     assert not M.chosen_pays(most, gu, E) and M.chosen_pays(most + 1, gu, E)
 
 
+@pytest.mark.parametrize("lens,starts,width,tiles", [
+    ([2], [510], 32, False), ([128] * 2, [1000] * 2, 71, False), ([256], [0], 16, False), ([320], [0], 20, True), ([80] * 3, [0] * 3, 5, True),
+    ([5] * 64, [1000] * 64, 63, True), ([5] * 64, [200] * 63 + [8000], 501, False), ([300] * 2, [0] * 2, 600, True), ([16], [0], 600, True)])
+def test_mixed_heads_of_few_rows_behind_many_keys(launched, monkeypatch, lens, starts, width, tiles):
+    """A tile's chain is as long as the longest portion: short portions behind long contexts keep the row kernel."""
+    from lumen.ops.attention import row_attention
+    from lumen.ops.segments import SegBatch, portion_keys, tile_list
+
+    monkeypatch.setattr(_seqmix, "talk_tiles_ok", lambda *a: True)
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    T, S, H, D = cu[-1], len(lens), 2, 128
+    i32 = dict(dtype=torch.int32)
+    row = torch.repeat_interleave(torch.arange(S), torch.tensor(lens)).int()
+    seg = SegBatch(torch.tensor(cu, **i32), torch.arange(S, **i32), torch.tensor(starts, **i32), row, torch.zeros(T, **i32),
+                   torch.zeros(S, width, **i32), None, torch.tensor(tile_list(cu, S), **i32).view(-1, 2), T, 128)
+    q, k, v = torch.zeros(T, H, D, **BF), torch.zeros(1, 16, H, D, **BF), torch.zeros(1, 16, H, D, **BF)
+    kv = [a + b for a, b in zip(lens, starts)]
+    name = "sm_talk_tiles" if tiles else "sm_row_attn"
+    for keys in (portion_keys(cu, kv, T), None):                # (without the host's count: by the tables' width)
+        seg.keys, uneven = keys, width * 16 > 2 * max(kv) or max(kv) > 2 * min(kv)
+        row_attention(q, None, k, v, D, torch.zeros(T, H, D, **BF), seg, H, H, 0.1, talk=torch.eye(H))
+        if keys is not None or not uneven:
+            assert [n for n, _ in launched] == [name]
+        launched.clear()
+    assert portion_keys(cu, kv, T + 1) is None and portion_keys(None, kv, T) is None and portion_keys(cu, None, T) is None
+
+
 def test_latent_products_of_many_rows_keep_the_library(launched, monkeypatch):
     from lumen.ops import attention as A
 

@@ -134,6 +134,7 @@ def test_mixed_head_tiles(H, G, opts, lens, starts, bs, tile, dtype, ulp):
     g = torch.Generator().manual_seed(H + bs)
     T, seg, (k, v) = portions(lens + [1], starts + [40], bs, g, (G, D), (G, D))
     seg.tile_rows, seg.tile_size = T - 1, tile             # (the last row is a decoded one)
+    seg.keys = (T, 1)                                      # (the tiles' edges, also where they are not the faster kernel)
     seg.q_tiles = torch.tensor(tile_list(seg.cu.tolist(), len(lens), tile), dtype=torch.int32, device="cuda").view(-1, 2)
     k, v = k.to(dtype).cuda(), v.to(dtype).cuda()
     q = torch.randn(T, H * D + 8, generator=g).to(dtype).cuda()[:, :H * D].view(T, H, D)
@@ -205,6 +206,7 @@ def odd_rows(run, v, seg, window=0):
 def test_infinite_values_of_hidden_tokens(kind, H, G, D, Dv, window, dtype):
     g = torch.Generator().manual_seed(H)
     T, seg, (k, v) = portions([131], [0], 16, g, (G, D), (G, Dv))
+    seg.keys = (T, 1)                                      # (mixed heads: the tiles)
     f = lambda *s: torch.randn(*s, generator=g).to(dtype).cuda()  # noqa: E731
     k, v, out = k.to(dtype).cuda(), v.to(dtype).cuda(), torch.zeros(T, H, Dv, dtype=dtype, device="cuda")
     if kind == "fresh":

@@ -287,9 +287,13 @@ chunk_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ 
 // keys the tile can see (from the first row's chunk start to the last row's position) are visited KT = 64
 // at a time (32 for heads over 128), staged in LDS twice (row-major for the scores, transposed for the value
 // pass) and shared by the waves.  Bound by the chain of tiles at two waves per SIMD; the loads of a tile leave
-// together one tile ahead and two buffers leave one barrier per tile, as in window_attention.hip.  us, tiles of
-// 32 keys, one buffer -> now (bf16, heads of 128): 8 x 512 rows x 16 heads 83 -> 39, 1 x 200 28 -> 20, 32 of 12 -
-// 100 25 -> 15, 1 x 4096 x 32 (chunk 1024) 284 -> 123; heads of 64 45 -> 28, 96 49 -> 34, 256 113 -> 109.
+// together one tile ahead and two buffers leave one barrier per tile, as in window_attention.hip.  Heads over 128 have
+// no registers left: one buffer, value addresses formed where they are used and queries read again by the look at the
+// end keep the spills out of the loop (us, two buffers -> one, 8 heads of 256 / 192: 8 x 512 rows 93 -> 84 / 54 -> 49, chunks of
+// 128 39 -> 36 / 24 -> 21, 1 x 200 42 -> 41 / 27 -> 24).  us, tiles of 32 keys, one buffer -> now (bf16, heads of 128): 8 x 512
+// rows x 16 heads 82 -> 43, 1 x 200 29 -> 21, 32 x 50 16 -> 12, 1 x 1024 x 32 109 -> 64; heads of 64 47 -> 31, 96 50 -> 38, 192 54
+// -> 49, 256 93 -> 84.  A portion of few keys pays for a whole tile of 64 (1 x 2 8.0 -> 8.9; 64 x 5 rows x 32 heads 22 -> 29;
+// a second form of the tile for 32 keys 29, and 8 x 512 46).
 // Per wave (32 queries) and 32 keys, with v_mfma_f32_32x32x16:
 //   S^T = K Q^T      keys on the accumulator rows, queries on the columns (lane & 31): a lane
 //                    owns ONE query, so its running max / sum / correction are plain scalars;
@@ -317,7 +321,7 @@ __device__ __forceinline__ float sumsq8(uint4 v) {
 }
 
 // (register budget: left to itself the compiler takes > 300 registers and runs one wave per SIMD.  Two waves
-// for heads of 96 and 128, where three spill; of 256 two with spills are ahead of one without, 109 us against 135)
+// for heads of 96 and 128, where three spill; of 256 two with spills are ahead of one without)
 template <typename T, int D, int NW, int KT>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 3 : 2)))
 tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ cache,
@@ -327,9 +331,10 @@ tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ c
                  int chunk, int sink) {
   constexpr int QT = 32 * NW, LK = D + 8, LT = KT + 8, NV = D / 8, SB = KT / 32;
   // two buffers: a tile is stored while the one before it is read, one barrier per tile
-  __shared__ __align__(16) T s_kb[2][KT * LK];    // key tile, row-major
-  __shared__ __align__(16) T s_tb[2][D * LT];     // key tile, transposed [d][key]
-  __shared__ float s_nb[2][KT];                   // 1 / rms of the tile's keys (power-of-two D / 8)
+  constexpr int NB = D <= 128 ? 2 : 1;
+  __shared__ __align__(16) T s_kb[NB][KT * LK];   // key tile, row-major
+  __shared__ __align__(16) T s_tb[NB][D * LT];    // key tile, transposed [d][key]
+  __shared__ float s_nb[NB][KT];                  // 1 / rms of the tile's keys (power-of-two D / 8)
   constexpr int kTbl = 512;                   // block-table entries of the visible keys, in LDS
   __shared__ int s_tbl[kTbl];
   constexpr bool kStagedNorm = (NV & (NV - 1)) == 0 && NV <= 64;
@@ -548,11 +553,12 @@ tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ c
       const uint4 bl = make_uint4(pl[0], pl[1], pl[2], pl[3]);
 #pragma unroll
       for (int db = 0; db < D / 32; ++db) {
-        // quads 4 s2 + hi and 4 s2 + 2 + hi of row 32 db + c, under the store's permutation: both low
-        // bits lie in t0 / t1, the others in the instruction's offset
-        const int at = 32 * db * LT + 32 * (s2 >> 1) + 16 * ((s2 & 1) ^ (db & 1));
-        const uint2 a0 = *reinterpret_cast<const uint2*>(s_t + t0 + at);
-        const uint2 a1 = *reinterpret_cast<const uint2*>(s_t + t1 + at);
+        // quads 4 s2 + hi and 4 s2 + 2 + hi of row 32 db + c, under the store's permutation: both low bits lie in t0 /
+        // t1, the others in the instruction's offset (heads over 128: formed here, those take no registers)
+        const int sw = ((32 * db + c) >> 3) & 7, at = 32 * db * LT + 32 * (s2 >> 1) + 16 * ((s2 & 1) ^ (db & 1));
+        const T* row = s_t + (32 * db + c) * LT;
+        const uint2 a0 = *reinterpret_cast<const uint2*>(D <= 128 ? s_t + t0 + at : row + 4 * ((4 * s2 + hi) ^ sw));
+        const uint2 a1 = *reinterpret_cast<const uint2*>(D <= 128 ? s_t + t1 + at : row + 4 * ((4 * s2 + 2 + hi) ^ sw));
         const uint4 a = make_uint4(a0.x, a0.y, a1.x, a1.y);
         O[db] = Mma32<T>::run(a, bh, O[db]);
         O[db] = Mma32<T>::run(a, bl, O[db]);
@@ -561,15 +567,25 @@ tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ c
   };
 
   prefetch(kbeg);
-  commit(kbeg, s_kb[0], s_tb[0], s_nb[0]);
-  __builtin_amdgcn_s_waitcnt(0xF70);       // vmcnt(0): or the loop's first product would wait, every time, for
-  __syncthreads();                         // the queries, and with them for the tile just asked for
-  for (int k0 = kbeg, cur = 0; k0 <= kend; k0 += KT, cur ^= 1) {
-    const bool more = k0 + KT <= kend;
-    if (more) prefetch(k0 + KT);
-    tile(k0, s_kb[cur], s_tb[cur], s_nb[cur]);
-    if (more) commit(k0 + KT, s_kb[cur ^ 1], s_tb[cur ^ 1], s_nb[cur ^ 1]);
-    __syncthreads();
+  if constexpr (NB == 1) {
+    for (int k0 = kbeg; k0 <= kend; k0 += KT) {
+      __syncthreads();                       // the tile before has been read
+      commit(k0, s_kb[0], s_tb[0], s_nb[0]);
+      __syncthreads();
+      if (k0 + KT <= kend) prefetch(k0 + KT);
+      tile(k0, s_kb[0], s_tb[0], s_nb[0]);
+    }
+  } else {
+    commit(kbeg, s_kb[0], s_tb[0], s_nb[0]);
+    __builtin_amdgcn_s_waitcnt(0xF70);     // vmcnt(0): or the loop's first product would wait, every time, for
+    __syncthreads();                       // the queries, and with them for the tile just asked for
+    for (int k0 = kbeg, cur = 0; k0 <= kend; k0 += KT, cur ^= 1) {
+      const bool more = k0 + KT <= kend;
+      if (more) prefetch(k0 + KT);
+      tile(k0, s_kb[cur], s_tb[cur], s_nb[cur]);
+      if (more) commit(k0 + KT, s_kb[cur ^ 1], s_tb[cur ^ 1], s_nb[cur ^ 1]);
+      __syncthreads();
+    }
   }
   l += __shfl_xor(l, 32, 64);
   // A hidden key has weight 0, but 0 times an infinite or NaN value is NaN: channels that are not finite are formed
@@ -579,6 +595,7 @@ tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ c
   for (int db = 0; db < D / 32; ++db)
 #pragma unroll
     for (int r = 0; r < 16; ++r) odd[r & 3] = fmaf(O[db][r], 0.f, odd[r & 3]);
+  const long long qat = (long long)(qv ? qrow : row0) * ldq + hd * D;      // (heads over 128: q is read again)
   if (__builtin_expect(__any(odd[0] + odd[1] + odd[2] + odd[3] != 0.f && qv), 0)) {
 #pragma unroll
     for (int db = 0; db < D / 32; ++db) {
@@ -594,7 +611,7 @@ tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ c
           __builtin_amdgcn_sched_barrier(0);       // (one load at a time: registers)
           float x[8];
           load8<T>(kp + 16 * kk + 8 * hi, x);
-          uint4 qk = qreg[kk];
+          uint4 qk = D <= 128 ? qreg[kk] : *reinterpret_cast<const uint4*>(q + qat + 16 * kk + 8 * hi);
           asm volatile("" : "+v"(qk.x), "+v"(qk.y), "+v"(qk.z), "+v"(qk.w));   // (converted here, not ahead of the loop)
           const T* y = reinterpret_cast<const T*>(&qk);
 #pragma unroll

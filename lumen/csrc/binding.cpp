@@ -72,8 +72,8 @@ hipError_t lumen_skinny_gemm(int, const void*, const void*, void*, int, int, int
                              long long, hipStream_t);
 hipError_t lumen_decode_gemm(int, const void*, const void*, void*, float*, int*, int, int, int,
                              long long, long long, int, int, int, int, int, hipStream_t);
-hipError_t lumen_split_gemm(int, const void*, long long, const void*, long long, void*, long long,
-                            float*, int, int, int, int, hipStream_t);
+hipError_t lumen_tile_gemm(int, const void*, long long, const void*, long long, const void*, void*, long long, float*,
+                           int, int, int, int, int, hipStream_t);
 hipError_t lumen_mlp_gemm(int, int, const void*, long long, const void*, long long, void*, long long,
                           void*, long long, const void*, long long, int, int, int, int, int, float*,
                           int*, int, hipStream_t);
@@ -251,22 +251,38 @@ void skinny_gemm(const at::Tensor& x, const at::Tensor& w, at::Tensor& y) {
         "skinny_gemm");
 }
 
-// x @ w^T in s slices of K (kernels/split_gemm.hip); the slabs are the call's own
-at::Tensor split_gemm(const at::Tensor& x, const at::Tensor& w, int64_t s) {
+// x @ w^T (+ bias) on 256 x 32 ni tiles, in s slices of K (kernels/tile_gemm.hip), into `out` or a new tensor; the slabs
+// are the call's own
+at::Tensor tile_product(const at::Tensor& x, const at::Tensor& w, const std::optional<at::Tensor>& bias, int64_t ni,
+                        int64_t s, const std::optional<at::Tensor>& out) {
   if (!x.is_cuda() || !w.is_cuda() || x.device() != w.device())
-    throw std::invalid_argument("lumen: split_gemm needs tensors of one GPU");
+    throw std::invalid_argument("lumen: tile_gemm needs tensors of one GPU");
   if (x.dim() != 2 || w.dim() != 2 || x.stride(1) != 1 || w.stride(1) != 1 ||
-      x.size(1) != w.size(1) || x.scalar_type() != w.scalar_type() || s < 2)
-    throw std::invalid_argument("lumen: split_gemm shape/layout mismatch");
-  const int64_t M = x.size(0), N = w.size(0), tiles = (M + 255) / 256 * ((N + 127) / 128);
-  at::Tensor y = at::empty({M, N}, x.options());
-  at::Tensor ws = at::empty({s * tiles * 32768}, x.options().dtype(at::kFloat));
-  check(lumen_split_gemm(dcode(w), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(),
-                         N, ws.data_ptr<float>(), static_cast<int>(M),
-                         static_cast<int>(N), static_cast<int>(x.size(1)), static_cast<int>(s),
-                         cur_stream()),
-        "split_gemm");
+      x.size(1) != w.size(1) || x.scalar_type() != w.scalar_type() || s < 1 || ni < 3 || ni > 6)
+    throw std::invalid_argument("lumen: tile_gemm shape/layout mismatch");
+  const int64_t M = x.size(0), N = w.size(0), tiles = (M + 255) / 256 * ((N + 32 * ni - 1) / (32 * ni));
+  if (bias && (bias->dim() != 1 || bias->size(0) != N || !bias->is_contiguous() ||
+               bias->scalar_type() != w.scalar_type() || bias->device() != w.device()))
+    throw std::invalid_argument("lumen: tile_gemm bias mismatch");
+  if (out && (out->dim() != 2 || out->size(0) != M || out->size(1) != N || out->stride(1) != 1 ||
+              out->scalar_type() != w.scalar_type() || out->device() != w.device()))
+    throw std::invalid_argument("lumen: tile_gemm output mismatch");
+  at::Tensor y = out ? *out : at::empty({M, N}, x.options()), ws;
+  if (s > 1) ws = at::empty({s * tiles * 8192 * ni}, x.options().dtype(at::kFloat));
+  check(lumen_tile_gemm(dcode(w), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0),
+                        bias ? bias->data_ptr() : nullptr, y.data_ptr(), y.stride(0),
+                        s > 1 ? ws.data_ptr<float>() : nullptr, static_cast<int>(M), static_cast<int>(N),
+                        static_cast<int>(x.size(1)), static_cast<int>(s), static_cast<int>(ni), cur_stream()),
+        "tile_gemm");
   return y;
+}
+at::Tensor tile_gemm(const at::Tensor& x, const at::Tensor& w, int64_t ni, const std::optional<at::Tensor>& bias,
+                     const std::optional<at::Tensor>& out) {
+  return tile_product(x, w, bias, ni, 1, out);
+}
+at::Tensor split_gemm(const at::Tensor& x, const at::Tensor& w, int64_t s) {
+  if (s < 2) throw std::invalid_argument("lumen: split_gemm takes two slices or more");
+  return tile_product(x, w, std::nullopt, 4, s, std::nullopt);
 }
 
 // decode-batch MFMA GEMM (kernels/decode_gemm.hip): y = x @ w^T with block tile (bm, bn) and
@@ -1098,6 +1114,8 @@ PYBIND11_MODULE(_C, m) {
   m.def("transpose2d", &transpose2d);
   m.def("skinny_gemm", &skinny_gemm);
   m.def("skinny_swiglu_gemm", &skinny_swiglu_gemm);
+  m.def("tile_gemm", &tile_gemm, py::arg("x"), py::arg("w"), py::arg("ni"), py::arg("bias") = py::none(),
+        py::arg("out") = py::none());
   m.def("split_gemm", &split_gemm);
   m.def("decode_gemm", &decode_gemm);
   m.def("mlp_gemm", &mlp_gemm, py::arg("epi"), py::arg("x"), py::arg("w"), py::arg("c"),

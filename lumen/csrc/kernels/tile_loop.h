@@ -1,0 +1,184 @@
+// The main loop of products x w^T on tiles of 256 rows of x and 32 NI rows of w (16-bit operands, fp32 sums), one workgroup of
+// four waves per CU; the kernels around it choose the rows and write the results.
+//
+//  * A wave owns 128 x 16 NI results.  Operands come by LDS-DMA in stages of 64 k, two to three steps ahead under
+//    counted waits; one barrier per step.  x has three LDS slots, w three where they fit into 160 KiB and two otherwise: then
+//    w's DMA goes out in the second half of a step and x's in the first, where the CU's one address path would be busy
+//    all of the second half with both (256 x 192: 0.88 -> 0.80 us a step).
+//  * Between two products stands at most one other thing, a fragment read or a DMA: in groups of eight products
+//    behind their reads the matrix core waited for the issue (256 x 128: 0.82 -> 0.75 us a step, 256 x 256 1.27 -> 1.0).
+//  * The accumulators are named as accumulation registers in the products' assembly.  The compiler, left to place them, splits
+//    128 and more over both files and moves them to and fro, or spills (256 x 256).
+// On 128 CUs a 256 x 256 step takes 0.95 us, 0.85 being the matrix core's; on all 256 the clock falls with the power of random
+// operands: 1.25 us, as in the library (zeros: 0.98; products alone: 2.04 PFLOP/s random, 2.41 zeros).
+#pragma once
+#include "common.h"
+
+namespace lumen {
+namespace tile {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+
+// c += a b.  The compiler sees the operands' waits but not the matrix core's latency: whoever reads c by other means goes
+// through settle() and hold() first.
+template <typename T>
+__device__ __forceinline__ void mfma(f32x4& c, uint4 a, uint4 b) {
+  if constexpr (__is_same(T, bf16))
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c)
+                 : "v"(__builtin_bit_cast(bf16x8, a)), "v"(__builtin_bit_cast(bf16x8, b)));
+  else
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c)
+                 : "v"(__builtin_bit_cast(f16x8, a)), "v"(__builtin_bit_cast(f16x8, b)));
+}
+// the last products have left the matrix core
+__device__ __forceinline__ void settle() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
+// a read of c is not moved ahead of this
+__device__ __forceinline__ void hold(f32x4& c) { asm volatile("" : "+a"(c)); }
+
+constexpr int BM = 256, BK = 64, ROWB = 128;             // a row of a stage is 64 elements, 128 bytes
+constexpr int MJ = 8;                                    // 16-row fragments of a wave's x: 128 rows
+constexpr int XB = BM * ROWB;
+constexpr int CUS = 256;
+
+template <int NI>
+struct Shape {
+  static constexpr int BN = 32 * NI, WB = BN * ROWB;
+  static constexpr int NST = 3 * (XB + WB) <= 160 * 1024 ? 3 : 2;        // slots of w
+  static constexpr int LDS = 3 * XB + NST * WB;
+  static constexpr int PIECES = 8 + NI;                  // 1-KiB LDS-DMA pieces of a wave and stage: 8 of x, NI of w
+};
+
+// 16-byte chunk c of stage row r lies at chunk c ^ swz(r): a fragment read (16 rows at one chunk) and an
+// LDS-DMA piece (8 whole rows) are both conflict free
+__device__ __forceinline__ int swz(int r) { return (r >> 1) & 7; }
+
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  static_assert(N >= 0 && N < 64, "vmcnt");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0xF70);
+}
+
+// LDS-DMA of 16 bytes per lane into the wave's 1-KiB piece (M0: its LDS address).  Inline asm, so that
+// the waits of the loop's own counting order it.
+__device__ __forceinline__ void dma16(const void* base, unsigned off, unsigned lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               :: "v"(off), "s"(base), "s"(lds) : "memory", "m0");
+}
+
+// this wave's fragment reads have arrived, and every wave's: their stage may be overwritten
+__device__ __forceinline__ void done_reading() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// Block b of n -> unit: blocks go to the XCDs in turn, XCD x takes consecutive units.
+__device__ __forceinline__ int unit_of(int b, int n) {
+  const int xcd = b & 7, q8 = n >> 3, r8 = n & 7;
+  return (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (b >> 3);
+}
+// Tile -> (row tile, column tile): `group` row tiles by all column tiles, row tiles first, so that the 32 tiles an XCD holds at
+// a time read a few panels of both operands from its L2.
+__device__ __forceinline__ void tile_at(int tile, int tiles_m, int tiles_n, int group, int& tm, int& tn) {
+  const int gsz = group * tiles_n, g = tile / gsz, gr = min(group, tiles_m - g * group), in = tile - g * gsz;
+  tn = in / gr;
+  tm = g * group + in - tn * gr;
+}
+
+// W row of a wave's 16 NI -> column: the fragments of a pair give a lane 8 consecutive columns (the last of an odd
+// number of fragments 4)
+template <int NI>
+__device__ __forceinline__ int colperm(int w) {
+  if ((w & ~31) + 32 > 16 * NI) return w;
+  return (w & ~31) | (((w >> 2) & 3) << 3) | (((w >> 4) & 1) << 2) | (w & 3);
+}
+
+// acc[i][j] = products of fragments i of w and j of x over nk stages (64 k each) from xb and wb, to which off[q] is the
+// lane's byte offset of the wave's piece q: stage rows 8 (wid + 4 q) + lane / 8 of x for q < 8, of w from piece 8 on, chunk
+// (lane & 7) ^ swz(row).  Lane (lr, lg) holds row 16 j + lr of its wave's x, rows 16 i + 4 lg .. + 3 of its w.
+template <typename T, int NI>
+__device__ __forceinline__ void products(char* lds, const char* xb, const char* wb, int nk,
+                                         const unsigned (&off)[Shape<NI>::PIECES], f32x4 (&acc)[NI][MJ]) {
+  constexpr int NST = Shape<NI>::NST, WB = Shape<NI>::WB, PIECES = Shape<NI>::PIECES;
+  // pieces [PB, PIECES) of a stage go out behind a second half's products, [0, PB) behind the first half's
+  constexpr int PB = NST == 2 ? 8 : PIECES - PIECES / 2, A = NST;
+  struct Slot { int x, w; };
+  const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const unsigned lds0 = (unsigned)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds);
+  auto issue = [&](int t, Slot slot, int q0, int q1) __attribute__((always_inline)) {
+    const char *xs = xb + (long long)t * (BK * 2), *ws = wb + (long long)t * (BK * 2);
+    const unsigned dx = __builtin_amdgcn_readfirstlane(lds0 + slot.x * XB + wid * 1024);
+    const unsigned dw = __builtin_amdgcn_readfirstlane(lds0 + 3 * XB + slot.w * WB + wid * 1024);
+#pragma unroll
+    for (int q = q0; q < q1; ++q) dma16(q < 8 ? xs : ws, off[q], q < 8 ? dx + q * 4096 : dw + (q - 8) * 4096);
+  };
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < MJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f}, hold(acc[i][j]);
+  settle();                                              // (and the products find the zeros written)
+  uint4 fa[2][NI], fb[2][MJ];
+  const int rb0 = (128 * (wid >> 1) + lr) * ROWB, ra0 = (16 * NI * (wid & 1) + lr) * ROWB;
+  // fragments u0 .. u1 - 1 of half h of a stage (w's, then x's)
+  auto frags = [&](int h, Slot slot, int u0, int u1) __attribute__((always_inline)) {
+    const int c = ((4 * h + lg) ^ swz(lr)) << 4;
+    const char *px = lds + slot.x * XB + c, *pw = lds + 3 * XB + slot.w * WB + c;
+#pragma unroll
+    for (int u = u0; u < u1; ++u)
+      if (u < NI) fa[h][u] = *reinterpret_cast<const uint4*>(pw + ra0 + u * 16 * ROWB);
+      else fb[h][u - NI] = *reinterpret_cast<const uint4*>(px + rb0 + (u - NI) * 16 * ROWB);
+  };
+  // the products of half h; between them the reads of the other half's fragments (from stage slot fs, in the first
+  // three quarters) and pieces q0 .. q1 - 1 of stage `t` into slot `ds` (t < 0: none)
+  auto half = [&](int h, Slot fs, int t, Slot ds, int q0, int q1) __attribute__((always_inline)) {
+    constexpr int U = NI * MJ, R = NI + MJ, UR = U * 3 / 4;
+    const int P = q1 - q0;
+#pragma unroll
+    for (int j = 0; j < MJ; ++j)
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int n = j * NI + i;
+        mfma<T>(acc[i][j], fa[h][i], fb[h][j]);
+        frags(1 - h, fs, min(R, (n * R + UR - 1) / UR), min(R, ((n + 1) * R + UR - 1) / UR));
+        if (t >= 0) issue(t, ds, q0 + n * P / U, q0 + (n + 1) * P / U);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+  };
+  auto after = [](Slot s) __attribute__((always_inline)) {
+    return Slot{s.x == 2 ? 0 : s.x + 1, s.w == NST - 1 ? 0 : s.w + 1};
+  };
+  // Step t multiplies stage t; at its start the first half's fragments are in registers.  Behind the first
+  // half's products it reads the second half's and sends for pieces [0, PB) of stage t + 2; then stage t + 1 has to be
+  // there, and every wave done with stage t.  NST 3: its slots take the other pieces of stage t + 3 behind the second
+  // half's products.  NST 2: its w slot takes the w pieces of stage t + 2.
+  Slot s0{0, 0}, s1{1, 1}, s2 = after(s1);
+  issue(0, s0, 0, PIECES);
+  if (nk > 1) issue(1, s1, 0, PIECES);
+  if (NST == 3 && nk > 2) issue(2, s2, PB, PIECES);
+  if (NST == 3 && nk > 2) wait_vm<2 * PIECES - PB>(); else if (nk > 1) wait_vm<PIECES>(); else wait_vm<0>();
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  frags(0, s0, 0, NI + MJ);
+  int t = 0;
+  for (; t + A < nk; ++t) {
+    half(0, s0, t + 2, s2, 0, PB);
+    wait_vm<NST == 3 ? PIECES : PB>();
+    done_reading();
+    half(1, s1, t + A, NST == 3 ? s0 : Slot{s2.x, s0.w}, PB, PIECES);
+    s0 = s1, s1 = s2, s2 = after(s2);
+  }
+  for (; t < nk; ++t) {                                  // the last stages
+    half(0, s0, t + 2 < nk ? t + 2 : -1, s2, 0, PB);
+    if (NST == 3 && t + 2 < nk) wait_vm<PIECES>(); else wait_vm<0>();
+    done_reading();
+    half(1, s1, -1, s2, 0, 0);                           // (the last step reads a slot that holds an earlier stage: unused)
+    s0 = s1, s1 = s2, s2 = after(s2);
+  }
+  settle();
+}
+
+}  // namespace tile
+}  // namespace lumen

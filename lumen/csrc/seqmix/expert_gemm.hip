@@ -7,7 +7,7 @@
 //
 // The dense form (two library products over ALL experts, ops/moe.py) does E / top times the work; the library's
 // grouped product runs at 300 TFLOP/s.  Here a workgroup takes 128 pairs of one expert and 256 rows of its weights,
-// both products on the loop of kernels/split_gemm.hip (three LDS stages of 64 k by LDS-DMA under counted waits, one
+// both products on a loop like that of kernels/tile_loop.h (three LDS stages of 64 k by LDS-DMA under counted waits, one
 // barrier a step, four waves of 64 pairs x 128 weight rows):
 //  * the rows of a tile are gathered by the DMA's source addresses; no sorted copy of h exists;
 //  * a wave's 128 weight rows of the first product are 64 gate rows and their 64 up rows, so the activation with the
@@ -15,7 +15,7 @@
 //  * counts stay on the device: the grid is sized for the most tiles the step can have and the surplus leaves at once.
 //    Nothing synchronises, nothing depends on host-visible counts (a capture may hold it);
 //  * XCDs take consecutive tiles, an expert's row tiles within a weight panel first: a panel comes from HBM once.
-// Bound by the loop at one wave per SIMD (1.0 us a step where split_gemm.hip takes 0.73: an expert's pairs are
+// Bound by the loop at one wave per SIMD (1.0 us a step where kernels/tile_loop.h takes 0.7: an expert's pairs are
 // fetched again for every few panels) and by each tile's own prologue and epilogue; under ~200 rows by reading the
 // weights once.  Measured (us, a whole layer of experts, dense form -> here; bf16, width 2048, experts of 1408, weights that
 // the last-level cache holds; ops/moe.py has few rows with weights from HBM): 8 experts, top 2, and a shared one: 4096 rows

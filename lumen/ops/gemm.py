@@ -3,7 +3,7 @@
 Up to 64 rows the projection is a stream of the weight matrix: the HIP kernels
 ``seqmix/thin_gemm.hip`` (1 - 64 rows) and ``kernels/skinny_gemm.hip`` (1 row) run it where they
 measured faster than a library GEMM; long contractions over some more rows are cut along K
-(``kernels/split_gemm.hip``).  The rest (and CPU tensors) goes to ``torch.matmul`` (hipBLASLt with the
+(``kernels/tile_gemm.hip``), and products whose result is about one round of its tiles go there whole.  The rest (and CPU tensors) goes to ``torch.matmul`` (hipBLASLt with the
 tuned table)."""
 from __future__ import annotations
 
@@ -234,7 +234,7 @@ def row_stream_linear(x: torch.Tensor, y: Optional[torch.Tensor], norm_w: torch.
     return z, s
 
 
-# Split-K GEMM (kernels/split_gemm.hip): long contractions over a few hundred rows, whose output has too few
+# Split-K GEMM (kernels/tile_gemm.hip): long contractions over a few hundred rows, whose output has too few
 # tiles to fill the chip.  us, library -> split: K = 11008, N = 4096, rows 72 / 256 / 512 / 1000: 41 -> 32, 51 ->
 # 35, 72 -> 50, 113 -> 87; K = 22016 at 512: 139 (tuned) -> 91; K = 32000 at 512: 290 -> 123; K = 11264, N = 2048 at
 # 320 / 1000: 48 -> 32, 72 -> 51.  Below K = 8192 the slabs cost what the split gains (K = 4096 at 512 rows: 28.2
@@ -258,11 +258,7 @@ def split_slices(x: torch.Tensor, w: torch.Tensor) -> int:
             or dt not in (torch.bfloat16, torch.float16) or x.device != w.device
             or not _plain(x, w) or not _here(x) or not use_native(x)):
         return 0
-    (lx, ex), (lw, ew) = x.stride(), w.stride()
-    if (ex != 1 or ew != 1 or lx % 8 or lw % 8 or not K <= lx <= 1 << 22 or not K <= lw <= 1 << 22
-            or (x.data_ptr() | w.data_ptr()) % 16):
-        return 0
-    return S
+    return S if _aligned(x, w, K) else 0
 
 
 def split_linear(x: torch.Tensor, w: torch.Tensor, S: int) -> torch.Tensor:
@@ -271,10 +267,75 @@ def split_linear(x: torch.Tensor, w: torch.Tensor, S: int) -> torch.Tensor:
     return native().split_gemm(x, w, S)
 
 
+# One round of 256 x 32 ni tiles (kernels/tile_gemm.hip) where some ni makes the result about one wave of the chip.  At
+# 0.85 of the tiles' area filled it is as fast as the library or faster over 350 shapes of 300 - 8000 rows, K 512 - 22016,
+# both types, tuned solutions included (us, library -> tiles: 4010 x 2048 x 2048 32.4 -> 31.3, x 5632 75 -> 72, x 11264 161
+# -> 143, 4010 x 2560 x 2048 44 -> 37, 2048 x 4096 x 11008 160 -> 143, 1000 x 8192 x 2048 34.7 -> 32.3, 512 x 22528 x
+# 4096 89 -> 84; worst 1280 x 8192 x 5632, filled 0.83, 96 -> 105).  Where N is no multiple of 1024 the library's own tiles fill
+# badly too: from 0.75 on (4010 x 2112 x 2048 42 -> 34, 3000 x 2112 x 2048 36 -> 29, 700 x 11264 x 2048 45 -> 36;
+# worst 3000 x 1536 x 2048, 0.73, 23.2 -> 24.4).
+TILE_MIN_M, TILE_MIN_K, TILE_CUS = 256, 512, 256
+TILE_FILL, TILE_FILL_ODD = 0.85, 0.75
+TILE_MIN_MN = int(TILE_FILL_ODD * TILE_CUS * 8192 * 3)     # fewer results than any such round has (asked first: host time)
+
+
+def tile_columns(M: int, N: int, K: int) -> int:
+    """``ni`` of the 256 x 32 ni tiles on which x [M, K] @ w [N, K]^T should run (0: leave it to the library)."""
+    if M < TILE_MIN_M or K < TILE_MIN_K:
+        return 0
+    tm = -(-M // 256)
+    for ni in (3, 4, 5, 6):
+        if tm * -(-N // (32 * ni)) <= TILE_CUS:
+            fill = M * N / (TILE_CUS * 8192 * ni)
+            return ni if fill >= TILE_FILL or N % 1024 and fill >= TILE_FILL_ODD else 0
+    return 0
+
+
+def _aligned(x: torch.Tensor, w: torch.Tensor, K: int) -> bool:
+    (lx, ex), (lw, ew) = x.stride(), w.stride()
+    return (ex == 1 and ew == 1 and lx % 8 == 0 and lw % 8 == 0 and K <= lx <= 1 << 22 and K <= lw <= 1 << 22
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+
+
+def tile_ok(x: torch.Tensor, w: torch.Tensor) -> int:
+    """``tile_columns`` of x @ w^T, 0 where the kernel cannot run it."""
+    xs, ws = x.shape, w.shape
+    if len(xs) != 2 or len(ws) != 2 or not x.is_cuda:
+        return 0
+    (M, K), (N, Kw), dt = xs, ws, x.dtype
+    ni = tile_columns(M, N, K)
+    if (not ni or K != Kw or K % 64 or N % 4 or K >= 1 << 22 or dt != w.dtype
+            or dt not in (torch.bfloat16, torch.float16) or x.device != w.device
+            or not _plain(x, w) or not _here(x) or not use_native(x) or not _aligned(x, w, K)):
+        return 0
+    return ni
+
+
+def tile_linear(x: torch.Tensor, w: torch.Tensor, ni: int, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x [M, K] @ w [N, K]^T (+ ``bias`` [N]) on 256 x 32 ni tiles, rounded once.  Callers take ``ni`` from ``tile_ok``."""
+    return native().tile_gemm(x, w, ni, bias)
+
+
 def matmul_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """x @ w[N, K]^T: the split-K GEMM where it is the faster one, else ``torch.matmul``."""
-    S = split_slices(x, w)
-    return split_linear(x, w, S) if S else torch.matmul(x, w.t())
+    """x @ w[N, K]^T: the split-K GEMM or one round of tiles where they are the faster ones, else ``torch.matmul``."""
+    xs = x.shape
+    if len(xs) == 2:                               # (short prompts wait for the host)
+        S = split_slices(x, w) if xs[1] >= SPLIT_MIN_K else 0
+        if S:
+            return split_linear(x, w, S)
+        ni = tile_ok(x, w) if xs[0] * w.shape[0] >= TILE_MIN_MN else 0
+        if ni:
+            return tile_linear(x, w, ni)
+    return torch.matmul(x, w.t())
+
+
+def _mm_into(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor) -> None:
+    """y = x @ w^T into a column view of operands that ``_split_plan`` has let pass."""
+    ni = tile_ok(x, w)
+    if ni and y.stride(0) % 4 == 0 and y.data_ptr() % 8 == 0:
+        native().tile_gemm(x, w, ni, None, y)
+    else:
+        torch.mm(x, w.t(), out=y)
 
 
 def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -282,9 +343,12 @@ def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = Non
     one row of a large matrix), the library otherwise."""
     xs = x.shape
     if len(xs) == 2 and xs[0] > THIN_MAX_M:            # (first: short prompts are bound by the host)
-        if bias is None and (xs[1] >= SPLIT_MIN_K or xs[0] * w.shape[0] >= MIN_CUT) and x.is_cuda:
+        MN = xs[0] * w.shape[0]
+        if bias is None and (xs[1] >= SPLIT_MIN_K or MN >= TILE_MIN_MN) and x.is_cuda:
             return mm_nt(x, w)
-        return F.linear(x, w, bias)
+        ni = (tile_ok(x, w) if MN >= TILE_MIN_MN and bias is not None and row_bias_ok(bias, x, w.shape[0]) and _plain(bias)
+              and bias.data_ptr() % 8 == 0 else 0)
+        return tile_linear(x, w, ni, bias) if ni else F.linear(x, w, bias)
     if thin_ok(x, w) and (bias is None or row_bias_ok(bias, x, w.shape[0]) and _plain(bias)):
         return _thin(x, w, bias)
     if bias is None and len(xs) == 2 and xs[0] == 1 and _plain(x, w) and _here(x) and skinny_ok(x, w):
@@ -461,7 +525,7 @@ def split_cols(M: int, N: int) -> int:
 # 637 -> 490, x 11008 407 -> 266, 4010 x 11264 x 2048 162 -> 141, 1300 x 22016 x 4096 299 -> 207, 300 x 95744 x
 # 4096 325 -> 238, 8000 x 11008 x 4096 627 -> 477.  Taking the columns that fill the waves nearest instead
 # (39 of 43 at 3100 rows x 11008: 507 of 512 tiles) sends the main part back to stream-K: 354 -> 369, with 38
-# columns 218.  With one whole wave it is even (2305 x 12288 173 -> 172): left whole.
+# columns 218.  With one whole wave it is even (2305 x 12288 173 -> 172): left whole here.
 # Where the row tiles do not divide 256, every wave of the main part leaves 256 mod tm tiles to the rest.  Up to 8
 # waves that costs less than stream-K does even when the rest passes one wave (4874 x 22016: 734 -> 647, 5100 x
 # 22016 x 2048 in fp16 369 -> 379); from 9 on it does not (5100 x 32000 897 -> 1032, 7300 x 25344 580 -> 644):
@@ -485,6 +549,17 @@ def wave_cols(M: int, N: int, K: int) -> int:
         return 0
     rest = tail + waves * (SPLIT_CUS % tm)
     return n1 if waves <= WAVE_SPILL_MAX or rest <= SPLIT_CUS else 0
+
+
+def round_cols(M: int, N: int, K: int) -> int:
+    """Column count of the one whole wave of 256 x 256 tiles in an [M, N] output whose rest is one round of narrow tiles of
+    kernels/tile_gemm.hip (0: no cut).  us, whole -> cut: 2048 x 11264 x 2048 88 -> 82, 4010 x 5632 x 4096 158 -> 142, 4096 x 6144 x
+    5632 215 -> 205; 43 such shapes 0.99 - 1.15 times as fast, mean 1.05.  Rests of wider tiles (ni 5 - 6): 0.94 - 1.03."""
+    tm, tn = -(-M // SPLIT_TILE), -(-N // SPLIT_TILE)
+    if M < WAVE_MIN_M or tm > WAVE_MAX_TM or N % 8 or K < WAVE_MIN_K or tm * tn // SPLIT_CUS != 1:
+        return 0
+    n1 = SPLIT_CUS // tm * SPLIT_TILE
+    return n1 if n1 < N and tile_columns(M, N - n1, K) in (3, 4) else 0
 
 
 _tuned: dict = {"n": -1, "sigs": {}}
@@ -524,7 +599,7 @@ def _split_plan(x: torch.Tensor, w: torch.Tensor) -> int:
             and w.stride(1) == 1):
         return 0
     (M, K), N = xs, ws[0]
-    n1, n2 = split_cols(M, N), wave_cols(M, N, K)
+    n1, n2 = split_cols(M, N), wave_cols(M, N, K) or round_cols(M, N, K)
     if not (n1 or n2):
         return 0
     # the first where both parts have tuned solutions, the second where neither the whole nor the parts
@@ -564,7 +639,7 @@ def mm_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         return matmul_nt(x, w)
     y = torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=x.dtype)
     torch.mm(x, w[:n1].t(), out=y[:, :n1])
-    torch.mm(x, w[n1:].t(), out=y[:, n1:])
+    _mm_into(x, w[n1:], y[:, n1:])
     return y
 
 

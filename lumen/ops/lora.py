@@ -22,7 +22,7 @@ import torch
 import torch.nn.functional as F
 
 from ._native import DTYPE_CODE, native, use_native
-from .gemm import mm_nt
+from .gemm import matmul_nt, mm_nt
 
 Seg = Tuple[int, int, int, int]
 
@@ -526,7 +526,7 @@ class _LoraLinear(torch.autograd.Function):
         W = weight_fn() if fold is None else None
 
         def gemm():
-            y_ = torch.matmul(x2d, W.t())
+            y_ = matmul_nt(x2d, W)
             if bias is not None:
                 y_.add_(bias)
             return y_
@@ -539,7 +539,7 @@ class _LoraLinear(torch.autograd.Function):
             Z = _zeros(T, R, device=x2d.device, train=ctx.train)
             _lora3_down(x2d, A, Z, p, seed)
             native().lora3_z_tail(Z, xe, K, FOLD_KP)
-            y = torch.matmul(xe, fold.t())
+            y = matmul_nt(xe, fold)
             if bias is not None:
                 y.add_(bias)
             rope_done = False

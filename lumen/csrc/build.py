@@ -252,7 +252,7 @@ def seqmix_path() -> str:
 def seqmix_sources() -> list:
     d = os.path.join(HERE, "seqmix")
     return sorted(glob.glob(os.path.join(d, "*.hip")) + glob.glob(os.path.join(d, "*.h"))
-                  + [os.path.join(HERE, "kernels", "common.h")])
+                  + [os.path.join(HERE, "kernels", h) for h in ("common.h", "tile_loop.h")])
 
 
 def seqmix_digest() -> str:

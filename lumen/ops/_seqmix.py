@@ -58,6 +58,7 @@ SIGNATURES = {
     "sm_latent_out": "ippi" "pll" "pl" "p" "pll" "iiii",
     "sm_mid_slabs": "iplpp" "iiii",
     "sm_mid_act": "iplpp" "iiiii" "ffff",
+    "sm_tile_act": "iplpp" "iiiiii" "i" "fff",
     "sm_slab_rms": "ipippp" "iii" "f",
     "sm_thin_tail": "iplpp" "iiii" "plip",
     "sm_thin_gate": "iplpp" "iii" "plp",

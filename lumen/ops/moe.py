@@ -402,6 +402,65 @@ def mid_act(h, gu_w, ff: int, act="silu", gated: bool = True) -> torch.Tensor:
     return out
 
 
+def act_rounds(M: int, ff: int) -> tuple:
+    """Column ranges (c0, c1, ni) of the launches of ``tile_act``: whole rounds of 256 workgroups on tiles of 256 rows by 128
+    columns, the rest on one round of the narrowest tiles that make it one."""
+    tm = -(-M // 256)
+    per = 256 // tm * 128                          # columns of a round
+    if per == 0:
+        return ()
+    c = ff // per * per
+    out = [(0, c, 8)] if c else []
+    if c < ff:
+        out.append((c, ff, next(ni for ni in (4, 6, 8) if tm * -(-(ff - c) // (16 * ni)) <= 256)))
+    return tuple(out)
+
+
+# Which products with a gated activation ``tile_act`` runs (us, product and pass before -> now, bf16): width 2048, ff 5632: 300 rows
+# 33.6 -> 27.7, 1000 52.8 -> 42.3, 4010 179 -> 156, 8000 337 -> 291; 1024, 2816: 512 20.9 -> 16.5, 4010 69 -> 49; 4096, 11008: 256 68 ->
+# 63, 1000 172 -> 159, 4010 574 -> 538.  It needs the more of the tiles' area filled the longer a product is, as the library cuts
+# long products of few tiles along K: over 370 sizes of 130 - 8000 rows and widths 512 - 4096 it is 0.95 - 1.99 times as fast under
+# this rule, 1.22 in the mean (left out: 300 rows, width 4096, filled 0.54, 78 -> 80; 1290 rows, 0.68, 235 -> 248; 220, ff 3000, width 2048, 0.16, 20 -> 25).
+ACT_TILE_FILL, ACT_TILE_FILL_MANY = 8192, 6000             # K over the filled share, up to 256 rows and above
+
+
+def _act_tiles_pay(M: int, ff: int, K: int) -> bool:
+    tm = -(-M // 256)
+    cells = sum(256 * 256 * 16 * ni * -(-(tm * -(-(c1 - c0) // (16 * ni))) // 256) for c0, c1, ni in act_rounds(M, ff))
+    return M * ff * (ACT_TILE_FILL if M <= 256 else ACT_TILE_FILL_MANY) >= K * cells > 0
+
+
+def tile_act_ok(h: torch.Tensor, gu_w: torch.Tensor, ff: int, act="silu", gated: bool = True) -> bool:
+    """Can and should ``tile_act`` run a dense first projection and its activation?"""
+    xs, ws = h.shape, gu_w.shape
+    if len(xs) != 2 or not h.is_cuda or not gated or not MID_MAX_M < xs[0] <= 65536 or len(ws) != 2:
+        return False
+    (M, K), dt = xs, h.dtype
+    if M * ff < 512 * K:                           # less than the rule asks of one round (first: short prompts wait for the host)
+        return False
+    if (ws[0] != 2 * ff or ws[1] != K or K % 64 or K == 0 or ff % 8 or ff == 0 or 4 * ff * K >= 1 << 32 or dt != gu_w.dtype
+            or dt not in (torch.bfloat16, torch.float16) or gu_w.device != h.device or not gu_w.is_contiguous()
+            or not _act_tiles_pay(M, ff, K)):
+        return False
+    ld, one = h.stride()
+    return (one == 1 and ld % 8 == 0 and K <= ld <= 1 << 22 and (h.data_ptr() | gu_w.data_ptr()) % 16 == 0
+            and _plain(h, gu_w) and _here(h))
+
+
+def tile_act(h, gu_w, ff: int, act="silu") -> torch.Tensor:
+    """act(gate) * up of h @ gu_w^T, [M, ff], from the fp32 sums, for operands that ``tile_act_ok`` has let pass.  (HIP
+    ``csrc/seqmix/tile_act.hip``.)"""
+    from ._seqmix import DT, call, use_seqmix
+
+    use_seqmix(h)
+    M, K = h.shape
+    out = torch.empty((M, ff), dtype=h.dtype, device=h.device)
+    code, c = (GATE_ACTS[act], (0.0,) * 3) if isinstance(act, str) else (4, (act.limit_shared, act.slope, act.shift))
+    for c0, c1, ni in act_rounds(M, ff):
+        call("sm_tile_act", DT[h.dtype], h, h.stride(0), gu_w, out, M, K, ff, c0, c1, ni, code, *c)
+    return out
+
+
 def moe_dense(h, wts, gu_w, down_w, E: int, ff: int, ffs: int, act="silu", gated: bool = True,
               weigh: str = "output", top: Optional[int] = None) -> torch.Tensor:
     """``top`` (optional): every row has at most that many non-zero weights."""
@@ -432,6 +491,8 @@ def ff_act(h, gu_w, ff: int, act="silu", gated: bool = True) -> torch.Tensor:
             return mid_act(h, gu_w, ff, act, gated)
         if h.shape[0] <= THIN_ACT_MAX_M and thin_act_ok(h, None, gu_w, 0, 0, ff, act, gated):
             return _thin_act(h, gu_w, None, 0, 0, ff, act, gated)
+    elif tile_act_ok(h, gu_w, ff, act, gated):
+        return tile_act(h, gu_w, ff, act)
     return _act(project(h, gu_w), None, 0, 0, ff, act, gated, "output")
 
 

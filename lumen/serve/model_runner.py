@@ -36,7 +36,7 @@ from ..ops.attention import (flash_attention_fresh, flash_attention_paged, paged
                              paged_decode_new, paged_decode_new_ok,
                              rope_write_kv)
 from ..ops.gemm import linear_nt, row_norm_linear, row_norm_ok, swiglu_linear_nt
-from ..ops.moe import MID_MAX_M, THIN_ACT_MAX_M, mid_act, mid_act_ok, thin_act, thin_act_ok
+from ..ops.moe import MID_MAX_M, THIN_ACT_MAX_M, mid_act, mid_act_ok, thin_act, thin_act_ok, tile_act, tile_act_ok
 from ..ops.norm import rms_norm
 from ..ops.rope import rope_tables
 
@@ -284,6 +284,9 @@ class ModelRunner:
             if T <= MID_MAX_M and ml is None and DECODE_SPLIT_MIN == 0 and use_native(y2) \
                     and mid_act_ok(y2, L.gate_up, self.w.F):
                 h = self._allreduce(linear_nt(mid_act(y2, L.gate_up, self.w.F), L.down))
+                continue
+            if ml is None and DECODE_SPLIT_MIN == 0 and use_native(y2) and tile_act_ok(y2, L.gate_up, self.w.F):
+                h = self._allreduce(linear_nt(tile_act(y2, L.gate_up, self.w.F), L.down))
                 continue
             gu = linear_nt(y2, L.gate_up)
             if ml is not None:

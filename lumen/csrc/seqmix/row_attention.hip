@@ -633,8 +633,13 @@ row_attn_kernel(const RowAttnArgs<T> a) {
 //      the weights of one head; the accumulator's column is the head, so the running correction is
 //      lane-local and nothing is merged across waves at the end.
 // Scores, maxima, sums and the accumulator are fp32.
-template <typename T, int NT>   // NT: 16-channel tiles per wave, Dv = 64 NT
-__global__ void __launch_bounds__(64 * kWaves)
+//
+// A decode step costs the chain of its loads: position, table, 18 steps of key fragments, 4 of values, each waited for.
+// DEEP sends for four steps of keys while four are multiplied, and for the first values with the first keys: 64 rows of 500
+// tokens, 16 heads over 512 + 64, 26.6 -> 23.3 us, one row 17.5 -> 15.1.  It takes registers: many rows of small ranks, whose workgroups hide each other's loads, keep the form
+// without (1024 rows of 250 tokens over 256 + 32: 34 us, DEEP 50).
+template <typename T, int NT, bool DEEP>   // NT: 16-channel tiles per wave, Dv = 64 NT
+__global__ void __launch_bounds__(64 * kWaves, DEEP ? 2 : 1)
 latent_attn_kernel(const RowAttnArgs<T> a, const T* __restrict__ vt) {
   extern __shared__ float smem[];
   constexpr int kPRow = 128 + 8;                 // weights per head in LDS: 128 keys + padding
@@ -676,6 +681,40 @@ latent_attn_kernel(const RowAttnArgs<T> a, const T* __restrict__ vt) {
 #pragma unroll
   for (int n = 0; n < NT; ++n) O[n] = f32x4v{0.f, 0.f, 0.f, 0.f};
   const T* qp = s_qb + hd * (Dkp + kQPad);
+  // key fragments of kCh steps of 32 channels: one chunk is loaded while the one before it is multiplied
+  constexpr int kCh = DEEP ? 4 : 1;
+  uint4 ka[kCh], kb[kCh], kc[kCh], kd[kCh], vv[DEEP ? 2 : 1][NT];
+  const T *kp0 = a.kc, *kp1 = a.kc;
+  const auto keys = [&](int jw) {                          // the rows of the lane's keys (addressable ones)
+    const int k0 = min(jw + hd, pos), k1 = min(jw + 16 + hd, pos);
+    kp0 = a.kc + ((long long)tbl[k0 / a.bs] * a.bs + k0 % a.bs) * a.krow + 8 * kg;
+    kp1 = a.kc + ((long long)tbl[k1 / a.bs] * a.bs + k1 % a.bs) * a.krow + 8 * kg;
+  };
+  const auto load = [&](uint4 (&x)[kCh], uint4 (&y)[kCh], int d0) {
+#pragma unroll
+    for (int c = 0; c < kCh; ++c)
+      if (d0 + 32 * c < Dkp) {
+        const bool in = d0 + 32 * c + 8 * kg < Dk;         // (past the key: zeros)
+        x[c] = in ? *reinterpret_cast<const uint4*>(kp0 + d0 + 32 * c) : make_uint4(0u, 0u, 0u, 0u);
+        y[c] = in ? *reinterpret_cast<const uint4*>(kp1 + d0 + 32 * c) : make_uint4(0u, 0u, 0u, 0u);
+      }
+  };
+  const auto values = [&](uint4 (&v)[NT], int jb) {        // the lane's 8 keys from jb on, its channels
+    const int k = min(jb, pos);
+    const T* vp = vt + ((long long)tbl[k / a.bs] * a.Dv) * a.bs + jb % a.bs;
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+      v[n] = *reinterpret_cast<const uint4*>(vp + (long long)((w * NT + n) * 16 + hd) * a.bs);
+  };
+  if (128 * (int)blockIdx.z + 32 * w <= pos) {
+    keys(128 * blockIdx.z + 32 * w);
+    if (DEEP) load(ka, kb, 0);
+  }
+  const auto ahead = [&](int j0) {                         // the first two steps' values of a tile
+    if (DEEP && j0 <= pos) values(vv[0], j0 + 8 * kg);
+    if (DEEP && j0 + 32 <= pos) values(vv[DEEP], j0 + 32 + 8 * kg);
+  };
+  ahead(128 * blockIdx.z);
   __syncthreads();
 
   for (int j0 = 128 * blockIdx.z; j0 <= pos; j0 += 128 * a.nsplit) {
@@ -683,22 +722,30 @@ latent_attn_kernel(const RowAttnArgs<T> a, const T* __restrict__ vt) {
     const int jw = j0 + 32 * w;
     float sc[2][4];
     float mx = -INFINITY;
+    f32x4v c0 = {0.f, 0.f, 0.f, 0.f}, c1 = {0.f, 0.f, 0.f, 0.f};
     if (jw <= pos) {
-      f32x4v c0 = {0.f, 0.f, 0.f, 0.f}, c1 = {0.f, 0.f, 0.f, 0.f};
-      const int k0 = min(jw + hd, pos), k1 = min(jw + 16 + hd, pos);        // addressable keys
-      const T* kp0 = a.kc + ((long long)tbl[k0 / a.bs] * a.bs + k0 % a.bs) * a.krow;
-      const T* kp1 = a.kc + ((long long)tbl[k1 / a.bs] * a.bs + k1 % a.bs) * a.krow;
-      for (int d0 = 0; d0 < Dkp; d0 += 32) {
-        const int d = d0 + 8 * kg;
-        uint4 a0 = make_uint4(0u, 0u, 0u, 0u), a1 = a0;
-        if (d < Dk) {
-          a0 = *reinterpret_cast<const uint4*>(kp0 + d);
-          a1 = *reinterpret_cast<const uint4*>(kp1 + d);
+      const auto mul = [&](const uint4 (&x)[kCh], const uint4 (&y)[kCh], int d0) {
+#pragma unroll
+        for (int c = 0; c < kCh; ++c)
+          if (d0 + 32 * c < Dkp) {
+            const uint4 bv = *reinterpret_cast<const uint4*>(qp + d0 + 32 * c + 8 * kg);
+            c0 = Mma16<T>::run(x[c], bv, c0);
+            c1 = Mma16<T>::run(y[c], bv, c1);
+          }
+      };
+      if (!DEEP)
+        for (int d0 = 0; d0 < Dkp; d0 += 32) {
+          load(ka, kb, d0);
+          mul(ka, kb, d0);
         }
-        const uint4 bv = *reinterpret_cast<const uint4*>(qp + d);
-        c0 = Mma16<T>::run(a0, bv, c0);
-        c1 = Mma16<T>::run(a1, bv, c1);
+      else for (int d0 = 0; d0 < Dkp; d0 += 64 * kCh) {
+        if (d0 + 32 * kCh < Dkp) load(kc, kd, d0 + 32 * kCh);
+        mul(ka, kb, d0);
+        if (d0 + 64 * kCh < Dkp) load(ka, kb, d0 + 64 * kCh);
+        if (d0 + 32 * kCh < Dkp) mul(kc, kd, d0 + 32 * kCh);
       }
+    }
+    if (jw <= pos) {
 #pragma unroll
       for (int sb = 0; sb < 2; ++sb) {
 #pragma unroll
@@ -750,13 +797,13 @@ latent_attn_kernel(const RowAttnArgs<T> a, const T* __restrict__ vt) {
     // 3. O^T += V^T P^T for the wave's channels over the tile's keys
     l_run = l_run * corr + (s_l[hd] + s_l[16 + hd]) + (s_l[32 + hd] + s_l[48 + hd]);
     m_run = mn;
+#pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       const int jb = j0 + 32 * ks + 8 * kg;                // the lane's 8 keys
-      if (j0 + 32 * ks > pos) break;
+      if (j0 + 32 * ks > pos) continue;
       const uint4 bh = *reinterpret_cast<const uint4*>(s_ph + hd * kPRow + 32 * ks + 8 * kg);
       const uint4 bl = *reinterpret_cast<const uint4*>(s_pl + hd * kPRow + 32 * ks + 8 * kg);
-      const int ka = min(jb, pos);
-      const T* vp = vt + ((long long)tbl[ka / a.bs] * a.Dv) * a.bs + jb % a.bs;
+      if (!DEEP) values(vv[0], jb);
       // keys past the row's position carry weight 0 but may hold anything: blank them
       const int nv = pos - jb + 1;                         // visible keys among the lane's 8
       uint4 mk = make_uint4(~0u, ~0u, ~0u, ~0u);
@@ -768,13 +815,19 @@ latent_attn_kernel(const RowAttnArgs<T> a, const T* __restrict__ vt) {
       }
 #pragma unroll
       for (int n = 0; n < NT; ++n) {
-        const int dv = (w * NT + n) * 16 + hd;             // as A operand: the lane's channel
-        uint4 av = *reinterpret_cast<const uint4*>(vp + (long long)dv * a.bs);
+        uint4 av = vv[DEEP ? ks & 1 : 0][n];                          // as A operand: the lane's channel
         av.x &= mk.x; av.y &= mk.y; av.z &= mk.z; av.w &= mk.w;
         O[n] = Mma16<T>::run(av, bh, O[n]);
         O[n] = Mma16<T>::run(av, bl, O[n]);
       }
+      if (DEEP && ks < 2 && j0 + 32 * (ks + 2) <= pos) values(vv[DEEP ? ks & 1 : 0], jb + 64);
     }
+    const int jn = j0 + 128 * a.nsplit + 32 * w;           // the next tile's first keys
+    if (jn <= pos) {
+      keys(jn);
+      if (DEEP) load(ka, kb, 0);
+    }
+    ahead(j0 + 128 * a.nsplit);
   }
   // O[n][i] = O^T[channel (w NT + n) 16 + 4 kg + i][head hd]
   if (head_on) {
@@ -813,15 +866,19 @@ template <typename T>
 hipError_t launch_latent_attn(const RowAttnArgs<T>& a, const T* vt, int Tn, hipStream_t st) {
   const size_t lds = latent_attn_lds(a.D1 + a.D2, sizeof(T));
   const dim3 grid(Tn, (a.H + 15) / 16, a.nsplit);
+  // two workgroups of the deep form fit a CU, as of the other one at ranks of 384 and more.  Up to 192 the forms are even.
+  const bool deep = (long long)grid.x * grid.y * grid.z <= 512;
+#define LATENT(N, D) latent_attn_kernel<T, N, D><<<grid, 64 * kWaves, lds, st>>>(a, vt)
   switch (a.Dv / 64) {
-    case 1: latent_attn_kernel<T, 1><<<grid, 64 * kWaves, lds, st>>>(a, vt); break;
-    case 2: latent_attn_kernel<T, 2><<<grid, 64 * kWaves, lds, st>>>(a, vt); break;
-    case 3: latent_attn_kernel<T, 3><<<grid, 64 * kWaves, lds, st>>>(a, vt); break;
-    case 4: latent_attn_kernel<T, 4><<<grid, 64 * kWaves, lds, st>>>(a, vt); break;
-    case 6: latent_attn_kernel<T, 6><<<grid, 64 * kWaves, lds, st>>>(a, vt); break;
-    case 8: latent_attn_kernel<T, 8><<<grid, 64 * kWaves, lds, st>>>(a, vt); break;
+    case 1: LATENT(1, false); break;
+    case 2: LATENT(2, false); break;
+    case 3: LATENT(3, false); break;
+    case 4: if (deep) LATENT(4, true); else LATENT(4, false); break;
+    case 6: LATENT(6, true); break;
+    case 8: LATENT(8, true); break;
     default: return hipErrorInvalidValue;
   }
+#undef LATENT
   return hipGetLastError();
 }
 template <>

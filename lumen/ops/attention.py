@@ -1227,8 +1227,12 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
     tiles = (seg.tables.shape[1] * kcache.shape[1] + 63) // 64
     if window > 0:                     # a row visits the window's tiles and the kept first ones
         tiles = min(tiles, (window + 63) // 64 + 1 + (keep_first + 63) // 64)
-    while talk is None and HB > 4 and T * ((H + HB - 1) // HB) * tiles < 512:
-        HB //= 2                       # fewer heads per workgroup: more workgroups
+    # fewer heads per workgroup: more workgroups, and a shorter chain in each.  Tables of a server's longest context count
+    # many tiles whatever the rows hold, so few rows are told by their blocks (us, 16 heads of 128 over 4, 8 rows, 16 heads
+    # a workgroup -> 4: 250 tokens 27 -> 14, 4000 45 -> 37; 16 rows -> 8: 250 30 -> 20, 1000 31 -> 23, 4000 50 -> 52; 64 rows of
+    # 4000 would go 152 -> 179)
+    while talk is None and HB > 4 and (T * ((H + HB - 1) // HB) * tiles < 512 or 2 * T * ((H + HB - 1) // HB) <= 32):
+        HB //= 2
     blocks = T * ((H + HB - 1) // HB)
     nsplit = max(1, min(tiles, 32, 512 // max(blocks, 1)))
     ws_ml = ws_o = None

@@ -73,7 +73,7 @@ hipError_t lumen_skinny_gemm(int, const void*, const void*, void*, int, int, int
 hipError_t lumen_decode_gemm(int, const void*, const void*, void*, float*, int*, int, int, int,
                              long long, long long, int, int, int, int, int, hipStream_t);
 hipError_t lumen_tile_gemm(int, const void*, long long, const void*, long long, const void*, void*, long long, float*,
-                           int, int, int, int, int, hipStream_t);
+                           int, int, int, int, int, int, int, hipStream_t);
 hipError_t lumen_mlp_gemm(int, int, const void*, long long, const void*, long long, void*, long long,
                           void*, long long, const void*, long long, int, int, int, int, int, float*,
                           int*, int, hipStream_t);
@@ -251,16 +251,16 @@ void skinny_gemm(const at::Tensor& x, const at::Tensor& w, at::Tensor& y) {
         "skinny_gemm");
 }
 
-// x @ w^T (+ bias) on 256 x 32 ni tiles, in s slices of K (kernels/tile_gemm.hip), into `out` or a new tensor; the slabs
+// x @ w^T (+ bias) on 32 mj x 32 ni tiles, in s slices of K (kernels/tile_gemm.hip), into `out` or a new tensor; the slabs
 // are the call's own
 at::Tensor tile_product(const at::Tensor& x, const at::Tensor& w, const std::optional<at::Tensor>& bias, int64_t ni,
-                        int64_t s, const std::optional<at::Tensor>& out) {
+                        int64_t mj, bool turned, int64_t s, const std::optional<at::Tensor>& out) {
   if (!x.is_cuda() || !w.is_cuda() || x.device() != w.device())
     throw std::invalid_argument("lumen: tile_gemm needs tensors of one GPU");
   if (x.dim() != 2 || w.dim() != 2 || x.stride(1) != 1 || w.stride(1) != 1 ||
-      x.size(1) != w.size(1) || x.scalar_type() != w.scalar_type() || s < 1 || ni < 3 || ni > 6)
+      x.size(1) != w.size(1) || x.scalar_type() != w.scalar_type() || s < 1 || ni < 1 || ni > 8 || mj < 1 || mj > 8)
     throw std::invalid_argument("lumen: tile_gemm shape/layout mismatch");
-  const int64_t M = x.size(0), N = w.size(0), tiles = (M + 255) / 256 * ((N + 32 * ni - 1) / (32 * ni));
+  const int64_t M = x.size(0), N = w.size(0), tiles = (M + 32 * mj - 1) / (32 * mj) * ((N + 32 * ni - 1) / (32 * ni));
   if (bias && (bias->dim() != 1 || bias->size(0) != N || !bias->is_contiguous() ||
                bias->scalar_type() != w.scalar_type() || bias->device() != w.device()))
     throw std::invalid_argument("lumen: tile_gemm bias mismatch");
@@ -268,21 +268,22 @@ at::Tensor tile_product(const at::Tensor& x, const at::Tensor& w, const std::opt
               out->scalar_type() != w.scalar_type() || out->device() != w.device()))
     throw std::invalid_argument("lumen: tile_gemm output mismatch");
   at::Tensor y = out ? *out : at::empty({M, N}, x.options()), ws;
-  if (s > 1) ws = at::empty({s * tiles * 8192 * ni}, x.options().dtype(at::kFloat));
+  if (s > 1) ws = at::empty({s * tiles * 1024 * mj * ni}, x.options().dtype(at::kFloat));
   check(lumen_tile_gemm(dcode(w), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0),
                         bias ? bias->data_ptr() : nullptr, y.data_ptr(), y.stride(0),
                         s > 1 ? ws.data_ptr<float>() : nullptr, static_cast<int>(M), static_cast<int>(N),
-                        static_cast<int>(x.size(1)), static_cast<int>(s), static_cast<int>(ni), cur_stream()),
+                        static_cast<int>(x.size(1)), static_cast<int>(s), static_cast<int>(ni), static_cast<int>(mj),
+                        turned ? 1 : 0, cur_stream()),
         "tile_gemm");
   return y;
 }
 at::Tensor tile_gemm(const at::Tensor& x, const at::Tensor& w, int64_t ni, const std::optional<at::Tensor>& bias,
-                     const std::optional<at::Tensor>& out) {
-  return tile_product(x, w, bias, ni, 1, out);
+                     const std::optional<at::Tensor>& out, int64_t mj, bool turned) {
+  return tile_product(x, w, bias, ni, mj, turned, 1, out);
 }
-at::Tensor split_gemm(const at::Tensor& x, const at::Tensor& w, int64_t s) {
+at::Tensor split_gemm(const at::Tensor& x, const at::Tensor& w, int64_t s, int64_t mj, bool turned) {
   if (s < 2) throw std::invalid_argument("lumen: split_gemm takes two slices or more");
-  return tile_product(x, w, std::nullopt, 4, s, std::nullopt);
+  return tile_product(x, w, std::nullopt, 4, mj, turned, s, std::nullopt);
 }
 
 // decode-batch MFMA GEMM (kernels/decode_gemm.hip): y = x @ w^T with block tile (bm, bn) and
@@ -1115,8 +1116,8 @@ PYBIND11_MODULE(_C, m) {
   m.def("skinny_gemm", &skinny_gemm);
   m.def("skinny_swiglu_gemm", &skinny_swiglu_gemm);
   m.def("tile_gemm", &tile_gemm, py::arg("x"), py::arg("w"), py::arg("ni"), py::arg("bias") = py::none(),
-        py::arg("out") = py::none());
-  m.def("split_gemm", &split_gemm);
+        py::arg("out") = py::none(), py::arg("mj") = 8, py::arg("turned") = false);
+  m.def("split_gemm", &split_gemm, py::arg("x"), py::arg("w"), py::arg("s"), py::arg("mj") = 8, py::arg("turned") = false);
   m.def("decode_gemm", &decode_gemm);
   m.def("mlp_gemm", &mlp_gemm, py::arg("epi"), py::arg("x"), py::arg("w"), py::arg("c"),
         py::arg("act") = py::none(), py::arg("gu") = py::none(), py::arg("group_m") = 4,

@@ -1,15 +1,19 @@
-// y = x w^T (+ bias) of 65 - some thousand rows on 256 x (32 NI) tiles (tile_loop.h), where the library's tiles fill the chip
-// badly: the caller takes NI 3 - 6 so that one round of workgroups covers the result, and cuts long contractions into S
-// slices where even that leaves CUs idle.
+// y = x w^T (+ bias) of 17 - some thousand rows on 32 mj x 32 ni tiles (tile_loop.h), where the library's tiles fill the chip
+// badly: the caller takes mj 2, 4 or 8 by the rows and ni so that one round of workgroups covers the result, and cuts long
+// contractions into S slices where even that leaves CUs idle.
 //  * XCDs take consecutive (slice, tile) pairs, `group` row tiles by all columns, so an L2 holds few panels;
 //  * slices leave fp32 slabs in the order of the lanes' registers (whole-line stores) and a second kernel adds
-//    them in slice order: 7 us for 32 MB.
-// Measured (bf16, us, library -> here, weights from HBM): S = 1: 4010 x 2048 x 2048 32.4 -> 31.3, x 5632 75 -> 72, 2048 x 4096 x
-// 11008 160 -> 143; 4010 x 2112 x 2048 42 -> 34 (NI 5), 4010 x 1536 x 2048 26.9 -> 26.6 (NI 3), 1000 x 11264 x 2048 49 -> 43 (NI 6).
-// Sliced: 512 x 4096 x 22016 235 -> 97, x 11008 79 -> 54; 256 x 4096 x 11008 53 -> 39; 1000 x 2048 x 11264 63 -> 51.
-// Bound by the power of the products and of the operands' way through LDS (tile_loop.h), and by 5 - 8 us in which all CUs
-// write their results at once (4 TB/s).  A form that runs several tiles a workgroup without a gap, stores under the next
-// tile's products, was faster for 2.75 and 4 rounds of 256 x 128 tiles (93 -> 80, 124 -> 118) but not for 256 x 256 ones.
+//    them in slice order: 7 us for 32 MB;
+//  * `turned`: column tiles start their walk of k at different stages, for rows of w that meet in the same memory channels.
+// Measured (bf16, us, library or thin kernel -> here, weights from HBM): 256-row tiles, S = 1: 4010 x 2048 x 2048 32.4 -> 31.3, x 5632
+// 75 -> 72, 2048 x 4096 x 11008 160 -> 143; 4010 x 2112 x 2048 42 -> 34 (ni 5), 4010 x 1536 x 2048 26.9 -> 26.6 (ni 3), 1000 x 11264 x 2048
+// 49 -> 43 (ni 6).  Sliced: 512 x 4096 x 22016 235 -> 97, x 11008 79 -> 54.  Few rows: 64 x 32000 x 4096 61 -> 48.5 (5.4 TB/s of weights),
+// 100 x 22016 x 4096 49 -> 41, 256 x 8192 x 4096 42.5 -> 31.9; sliced 64 x 2048 x 11264 32.7 -> 19.5, 128 x 4096 x 11008 39 -> 29.  A decode
+// step of 4 layers of width 4096 at 48 rows 651 -> 550, at 112 rows 805 -> 725.  The lines are in ops/gemm.py.
+// From some hundred rows on bound by the power of the products and of the operands' way through LDS (tile_loop.h), and by 5 - 8 us in
+// which all CUs write their results at once (4 TB/s); below by w's way from HBM.  A form that runs several tiles a
+// workgroup without a gap, stores under the next tile's products, was faster for 2.75 and 4 rounds of 256 x 128 tiles (93 -> 80, 124
+// -> 118) but not for 256 x 256 ones.
 #include "tile_loop.h"
 
 namespace lumen {
@@ -21,7 +25,8 @@ struct GemmArgs {
   void* y; long long ldy;
   const void* bias;
   float* ws;
-  int M, N, K, tiles_m, tiles_n, group, S, wide;         // wide: y's rows can be written 16 bytes at a time
+  int M, N, K, tiles_m, tiles_n, group, S;
+  int wide, turned;          // y's rows can be written 16 bytes at a time; column tiles start at different k
 };
 
 template <typename T>
@@ -52,10 +57,11 @@ __device__ __forceinline__ void put(const GemmArgs& a, int m, int n, int i, f32x
   if (more) *reinterpret_cast<uint2*>(p + 4) = hi;
 }
 
-template <typename T, int NI>
+template <typename T, int NI, int MJ, bool APART>
 __global__ void __launch_bounds__(256, 1) tile_gemm_kernel(const GemmArgs a) {
-  constexpr int BN = Shape<NI>::BN, PIECES = Shape<NI>::PIECES;
-  __shared__ __attribute__((aligned(16))) char lds[Shape<NI>::LDS];
+  using S = Shape<NI, MJ>;
+  constexpr int BM = S::BM, BN = S::BN, PIECES = S::PIECES;
+  __shared__ __attribute__((aligned(16))) char lds[S::LDS];
   const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tiles = a.tiles_m * a.tiles_n, v = unit_of(blockIdx.x, gridDim.x);
@@ -70,13 +76,13 @@ __global__ void __launch_bounds__(256, 1) tile_gemm_kernel(const GemmArgs a) {
   unsigned off[PIECES];                                  // (rows past the edge read the last row: never stored)
 #pragma unroll
   for (int q = 0; q < PIECES; ++q) {
-    const int r = 8 * (wid + 4 * (q < 8 ? q : q - 8)) + (lane >> 3), c = (lane & 7) ^ swz(r);
+    const int r = 8 * (wid + 4 * (q < MJ ? q : q - MJ)) + (lane >> 3), c = (lane & 7) ^ swz(r);
     const int col = r / (16 * NI) * (16 * NI) + colperm<NI>(r % (16 * NI));
-    off[q] = q < 8 ? (unsigned)min(r, a.M - m0 - 1) * (unsigned)(2 * a.ldx) + 16 * c
+    off[q] = q < MJ ? (unsigned)min(r, a.M - m0 - 1) * (unsigned)(2 * a.ldx) + 16 * c
                    : (unsigned)min(col, a.N - n0 - 1) * (unsigned)(2 * a.ldw) + 16 * c;
   }
   f32x4 acc[NI][MJ];
-  products<T, NI>(lds, xb, wb, nk, off, acc);
+  products<T, NI, MJ, APART>(lds, xb, wb, nk, APART && a.turned ? (int)(13u * tn % nk) : 0, off, acc);
   if (a.S > 1) {
     f32x4* o = (f32x4*)a.ws + (((long long)slice * tiles + tile) * 4 + wid) * (NI * MJ * 64) + lane;
 #pragma unroll
@@ -87,7 +93,7 @@ __global__ void __launch_bounds__(256, 1) tile_gemm_kernel(const GemmArgs a) {
   }
 #pragma unroll
   for (int j = 0; j < MJ; ++j) {
-    const int m = m0 + 128 * (wid >> 1) + 16 * j + lr;
+    const int m = m0 + 16 * MJ * (wid >> 1) + 16 * j + lr;
 #pragma unroll
     for (int i = 0; i < NI; i += 2) {
       constexpr int last = NI - 1;
@@ -100,15 +106,16 @@ __global__ void __launch_bounds__(256, 1) tile_gemm_kernel(const GemmArgs a) {
 }
 
 // y = the sum of the S slabs, which lie in the order of the lanes that wrote them; a wave sums a pair of fragments
-template <typename T, int NI>
+template <typename T, int NI, int MJ>
 __global__ void __launch_bounds__(256) tile_sum_kernel(const GemmArgs a) {
+  using S = Shape<NI, MJ>;
   constexpr int NP = (NI + 1) / 2;
   const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
   const int f = blockIdx.x * 4 + (threadIdx.x >> 6);     // (tile, wave, j, pair)
   const int i = 2 * (f % NP), j = f / NP % MJ, wid = f / (NP * MJ) % 4, tile = f / (NP * MJ * 4);
   int tm, tn;
   tile_at(tile, a.tiles_m, a.tiles_n, a.group, tm, tn);
-  const int m = tm * BM + 128 * (wid >> 1) + 16 * j + lr;
+  const int m = tm * S::BM + 16 * MJ * (wid >> 1) + 16 * j + lr;
   if (m >= a.M) return;
   const bool pair = i + 1 < NI;
   const f32x4* p = (const f32x4*)a.ws + ((long long)(tile * 4 + wid) * (NI * MJ) + j * NI + i) * 64 + lane;
@@ -118,7 +125,7 @@ __global__ void __launch_bounds__(256) tile_sum_kernel(const GemmArgs a) {
     s += p[k * plane];
     if (pair) r += p[k * plane + 64];
   }
-  put<T, NI>(a, m, tn * Shape<NI>::BN + 16 * (NI * (wid & 1) + i) + (pair ? 8 : 4) * lg, i, s, r);
+  put<T, NI>(a, m, tn * S::BN + 16 * (NI * (wid & 1) + i) + (pair ? 8 : 4) * lg, i, s, r);
 }
 
 }  // namespace tile
@@ -126,31 +133,46 @@ __global__ void __launch_bounds__(256) tile_sum_kernel(const GemmArgs a) {
 
 extern "C" {
 
-// y [M, N] = x [M, K] w [N, K]^T + bias [N] (or null), 16-bit, rows at ldx, ldw, ldy, on 256 x 32 ni tiles, K in S slices; ws (S
-// > 1): S * tiles * 8192 ni fp32.  K % 64 == 0, N % 4 == 0, rows of x and w at 16-byte addresses, of y and bias at 8-byte ones.
+// y [M, N] = x [M, K] w [N, K]^T + bias [N] (or null), 16-bit, rows at ldx, ldw, ldy, on 32 mj x 32 ni tiles, K in S slices; ws (S
+// > 1): S * tiles * 1024 mj ni fp32; turned: column tiles start at different k.  K % 64 == 0, N % 4 == 0, rows of x and w at 16-byte addresses, of y and bias at 8-byte ones.
 hipError_t lumen_tile_gemm(int dt, const void* x, long long ldx, const void* w, long long ldw, const void* bias, void* y,
-                           long long ldy, float* ws, int M, int N, int K, int S, int ni, hipStream_t st) {
+                           long long ldy, float* ws, int M, int N, int K, int S, int ni, int mj, int turned, hipStream_t st) {
   using namespace lumen;
   using namespace lumen::tile;
   if ((long long)M * N == 0) return hipSuccess;
   if (K <= 0 || K % BK || N % 4 || S < 1 || S > K / BK || ldx % 8 || ldw % 8 || ldy % 4 || ldx < K ||
       ldw < K || ldy < N || ldx > (1 << 22) || ldw > (1 << 22) || (S > 1 && !ws) || (dt != kF16 && dt != kBF16) ||
-      ((uintptr_t)x | (uintptr_t)w | (uintptr_t)ws) % 16 || ((uintptr_t)y | (uintptr_t)bias) % 8 || ni < 3 || ni > 6 ||
-      (S > 1 && ni != 4) || (long long)(K / BK) * S >= (1LL << 31))
+      ((uintptr_t)x | (uintptr_t)w | (uintptr_t)ws) % 16 || ((uintptr_t)y | (uintptr_t)bias) % 8 ||
+      (S > 1 && (ni != 4 || (mj != 2 && mj != 4 && mj != 8))) || (long long)(K / BK) * S >= (1LL << 31))
     return hipErrorInvalidValue;
-  const long long tm = (M + BM - 1) / BM, tn = (N + 32 * ni - 1) / (32 * ni), tiles = tm * tn;
+  const int BM = 32 * mj;
+  const long long tm = (M + BM - 1LL) / BM, tn = (N + 32 * ni - 1) / (32 * ni), tiles = tm * tn;
   if (tiles * S >= (1 << 20)) return hipErrorInvalidValue;
   const GemmArgs a{x, ldx, w, ldw, y, ldy, bias, ws, M, N, K, (int)tm, (int)tn, (int)(tm < 4 ? tm : 4), S,
-                   ldy % 8 == 0 && (uintptr_t)y % 16 == 0};
-#define GO(NI)                                                                                            \
-  if (dt == kBF16) tile_gemm_kernel<bf16, NI><<<(int)tiles * S, 256, 0, st>>>(a);                         \
-  else tile_gemm_kernel<fp16, NI><<<(int)tiles * S, 256, 0, st>>>(a);
-  if (ni == 3) { GO(3) } else if (ni == 4) { GO(4) } else if (ni == 5) { GO(5) } else { GO(6) }
+                   ldy % 8 == 0 && (uintptr_t)y % 16 == 0, turned};
+  const int grid = (int)tiles * S;
+  // (256 rows in step without the walk's arithmetic: 4010 x 2048 x 5632 78.3 -> 76.5 us)
+  switch (10 * mj + ni + (mj == 8 && turned ? 100 : 0)) {
+#define GO(MJ, NI, APART)                                                                                       \
+  case 10 * MJ + NI + (MJ == 8 && APART ? 100 : 0):                                                             \
+    if (dt == kBF16) tile_gemm_kernel<bf16, NI, MJ, APART><<<grid, 256, 0, st>>>(a);                            \
+    else tile_gemm_kernel<fp16, NI, MJ, APART><<<grid, 256, 0, st>>>(a);                                        \
+    break;
+    GO(2, 1, true) GO(2, 2, true) GO(2, 3, true) GO(2, 4, true) GO(2, 5, true) GO(2, 6, true) GO(2, 8, true)
+    GO(4, 2, true) GO(4, 3, true) GO(4, 4, true) GO(4, 5, true) GO(4, 6, true) GO(4, 8, true)
+    GO(8, 3, false) GO(8, 4, false) GO(8, 5, false) GO(8, 6, false) GO(8, 3, true) GO(8, 4, true)
 #undef GO
+    default: return hipErrorInvalidValue;
+  }
   if (S > 1) {
-    const int blocks = (int)tiles * 2 * MJ;              // NI 4: two pairs, MJ rows, four waves a tile, four to a block
-    if (dt == kBF16) tile_sum_kernel<bf16, 4><<<blocks, 256, 0, st>>>(a);
-    else tile_sum_kernel<fp16, 4><<<blocks, 256, 0, st>>>(a);
+    const int blocks = (int)tiles * 2 * mj;              // NI 4: two pairs, mj rows' fragments, four waves a tile, four to a block
+#define GO(MJ)                                                                    \
+  case MJ:                                                                        \
+    if (dt == kBF16) tile_sum_kernel<bf16, 4, MJ><<<blocks, 256, 0, st>>>(a);     \
+    else tile_sum_kernel<fp16, 4, MJ><<<blocks, 256, 0, st>>>(a);                 \
+    break;
+    switch (mj) { GO(2) GO(4) GO(8) }
+#undef GO
   }
   return hipGetLastError();
 }

@@ -1,10 +1,14 @@
-// The main loop of products x w^T on tiles of 256 rows of x and 32 NI rows of w (16-bit operands, fp32 sums), one workgroup of
+// The main loop of products x w^T on tiles of 32 MJ rows of x and 32 NI rows of w (16-bit operands, fp32 sums), one workgroup of
 // four waves per CU; the kernels around it choose the rows and write the results.
 //
-//  * A wave owns 128 x 16 NI results.  Operands come by LDS-DMA in stages of 64 k, two to three steps ahead under
-//    counted waits; one barrier per step.  x has three LDS slots, w three where they fit into 160 KiB and two otherwise: then
-//    w's DMA goes out in the second half of a step and x's in the first, where the CU's one address path would be busy
-//    all of the second half with both (256 x 192: 0.88 -> 0.80 us a step).
+//  * A wave owns 16 MJ x 16 NI results.  Operands come by LDS-DMA in stages of 64 k under counted waits, as many steps
+//    ahead as fit into 160 KiB (six at most); one barrier per step.  256 x 192 and wider keep three slots of x and two of
+//    w: then w's DMA goes out in the second half of a step and x's in the first, where the CU's one address path would be
+//    busy all of the second half with both (256 x 192: 0.88 -> 0.80 us a step).
+//  * With w from HBM few-row tiles wait for bytes: a CU takes 97 B/ns from L2 and 60 of lines from HBM, however many are in
+//    flight (48 KB do), so the tile is as narrow in x as the rows are.  Rows of w some KB apart, read a stage at
+//    a time by all workgroups in step, meet in the same memory channels: the caller may have a tile start its walk of k
+//    elsewhere (`turn`; a bare stream of rows 8 KB apart 5.0 -> 5.6 TB/s, 4 KB apart 4.45 -> 5.45).
 //  * Between two products stands at most one other thing, a fragment read or a DMA: in groups of eight products
 //    behind their reads the matrix core waited for the issue (256 x 128: 0.82 -> 0.75 us a step, 256 x 256 1.27 -> 1.0).
 //  * The accumulators are named as accumulation registers in the products' assembly.  The compiler, left to place them, splits
@@ -37,17 +41,16 @@ __device__ __forceinline__ void settle() { asm volatile("s_nop 15\n\ts_nop 15" :
 // a read of c is not moved ahead of this
 __device__ __forceinline__ void hold(f32x4& c) { asm volatile("" : "+a"(c)); }
 
-constexpr int BM = 256, BK = 64, ROWB = 128;             // a row of a stage is 64 elements, 128 bytes
-constexpr int MJ = 8;                                    // 16-row fragments of a wave's x: 128 rows
-constexpr int XB = BM * ROWB;
+constexpr int BK = 64, ROWB = 128;                       // a row of a stage is 64 elements, 128 bytes
 constexpr int CUS = 256;
 
-template <int NI>
+template <int NI, int MJ>
 struct Shape {
-  static constexpr int BN = 32 * NI, WB = BN * ROWB;
-  static constexpr int NST = 3 * (XB + WB) <= 160 * 1024 ? 3 : 2;        // slots of w
-  static constexpr int LDS = 3 * XB + NST * WB;
-  static constexpr int PIECES = 8 + NI;                  // 1-KiB LDS-DMA pieces of a wave and stage: 8 of x, NI of w
+  static constexpr int BM = 32 * MJ, BN = 32 * NI, XB = BM * ROWB, WB = BN * ROWB;
+  static constexpr int FIT = 160 * 1024 / (XB + WB);
+  static constexpr int NST = FIT < 6 ? FIT : 6, NSX = NST < 3 ? 3 : NST;         // slots of w and x
+  static constexpr int LDS = NSX * XB + NST * WB;
+  static constexpr int PIECES = MJ + NI;                 // 1-KiB LDS-DMA pieces of a wave and stage: MJ of x, NI of w
 };
 
 // 16-byte chunk c of stage row r lies at chunk c ^ swz(r): a fragment read (16 rows at one chunk) and an
@@ -58,6 +61,14 @@ template <int N>
 __device__ __forceinline__ void wait_vm() {
   static_assert(N >= 0 && N < 64, "vmcnt");
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0xF70);
+}
+
+// all but the last r (R at most) stages have arrived
+template <int R, int PIECES>
+__device__ __forceinline__ void wait_stages(int r) {
+  if constexpr (R <= 0) wait_vm<0>();
+  else if (r >= R) wait_vm<R * PIECES>();
+  else wait_stages<R - 1, PIECES>(r);
 }
 
 // LDS-DMA of 16 bytes per lane into the wave's 1-KiB piece (M0: its LDS address).  Inline asm, so that
@@ -96,24 +107,27 @@ __device__ __forceinline__ int colperm(int w) {
 }
 
 // acc[i][j] = products of fragments i of w and j of x over nk stages (64 k each) from xb and wb, to which off[q] is the
-// lane's byte offset of the wave's piece q: stage rows 8 (wid + 4 q) + lane / 8 of x for q < 8, of w from piece 8 on, chunk
-// (lane & 7) ^ swz(row).  Lane (lr, lg) holds row 16 j + lr of its wave's x, rows 16 i + 4 lg .. + 3 of its w.
-template <typename T, int NI>
-__device__ __forceinline__ void products(char* lds, const char* xb, const char* wb, int nk,
-                                         const unsigned (&off)[Shape<NI>::PIECES], f32x4 (&acc)[NI][MJ]) {
-  constexpr int NST = Shape<NI>::NST, WB = Shape<NI>::WB, PIECES = Shape<NI>::PIECES;
+// lane's byte offset of the wave's piece q: stage rows 8 (wid + 4 q) + lane / 8 of x for q < MJ, of w from piece MJ on, chunk
+// (lane & 7) ^ swz(row).  APART: the walk starts at stage `turn` < nk and comes round to it.  Lane (lr, lg) holds row 16 j + lr of its
+// wave's x, rows 16 i + 4 lg .. + 3 of its w.
+template <typename T, int NI, int MJ, bool APART = false>
+__device__ __forceinline__ void products(char* lds, const char* xb, const char* wb, int nk, int turn,
+                                         const unsigned (&off)[Shape<NI, MJ>::PIECES], f32x4 (&acc)[NI][MJ]) {
+  using S = Shape<NI, MJ>;
+  constexpr int NSX = S::NSX, NST = S::NST, XB = S::XB, WB = S::WB, PIECES = S::PIECES;
   // pieces [PB, PIECES) of a stage go out behind a second half's products, [0, PB) behind the first half's
-  constexpr int PB = NST == 2 ? 8 : PIECES - PIECES / 2, A = NST;
+  constexpr int PB = NST == 2 ? MJ : PIECES - PIECES / 2, F = NSX - 1;
   struct Slot { int x, w; };
   const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const unsigned lds0 = (unsigned)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds);
   auto issue = [&](int t, Slot slot, int q0, int q1) __attribute__((always_inline)) {
-    const char *xs = xb + (long long)t * (BK * 2), *ws = wb + (long long)t * (BK * 2);
+    const int u = APART ? (t + turn < nk ? t + turn : t + turn - nk) : t;
+    const char *xs = xb + (long long)u * (BK * 2), *ws = wb + (long long)u * (BK * 2);
     const unsigned dx = __builtin_amdgcn_readfirstlane(lds0 + slot.x * XB + wid * 1024);
-    const unsigned dw = __builtin_amdgcn_readfirstlane(lds0 + 3 * XB + slot.w * WB + wid * 1024);
+    const unsigned dw = __builtin_amdgcn_readfirstlane(lds0 + NSX * XB + slot.w * WB + wid * 1024);
 #pragma unroll
-    for (int q = q0; q < q1; ++q) dma16(q < 8 ? xs : ws, off[q], q < 8 ? dx + q * 4096 : dw + (q - 8) * 4096);
+    for (int q = q0; q < q1; ++q) dma16(q < MJ ? xs : ws, off[q], q < MJ ? dx + q * 4096 : dw + (q - MJ) * 4096);
   };
 #pragma unroll
   for (int i = 0; i < NI; ++i)
@@ -121,11 +135,11 @@ __device__ __forceinline__ void products(char* lds, const char* xb, const char* 
     for (int j = 0; j < MJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f}, hold(acc[i][j]);
   settle();                                              // (and the products find the zeros written)
   uint4 fa[2][NI], fb[2][MJ];
-  const int rb0 = (128 * (wid >> 1) + lr) * ROWB, ra0 = (16 * NI * (wid & 1) + lr) * ROWB;
+  const int rb0 = (16 * MJ * (wid >> 1) + lr) * ROWB, ra0 = (16 * NI * (wid & 1) + lr) * ROWB;
   // fragments u0 .. u1 - 1 of half h of a stage (w's, then x's)
   auto frags = [&](int h, Slot slot, int u0, int u1) __attribute__((always_inline)) {
     const int c = ((4 * h + lg) ^ swz(lr)) << 4;
-    const char *px = lds + slot.x * XB + c, *pw = lds + 3 * XB + slot.w * WB + c;
+    const char *px = lds + slot.x * XB + c, *pw = lds + NSX * XB + slot.w * WB + c;
 #pragma unroll
     for (int u = u0; u < u1; ++u)
       if (u < NI) fa[h][u] = *reinterpret_cast<const uint4*>(pw + ra0 + u * 16 * ROWB);
@@ -148,34 +162,37 @@ __device__ __forceinline__ void products(char* lds, const char* xb, const char* 
       }
   };
   auto after = [](Slot s) __attribute__((always_inline)) {
-    return Slot{s.x == 2 ? 0 : s.x + 1, s.w == NST - 1 ? 0 : s.w + 1};
+    return Slot{s.x == NSX - 1 ? 0 : s.x + 1, s.w == NST - 1 ? 0 : s.w + 1};
   };
   // Step t multiplies stage t; at its start the first half's fragments are in registers.  Behind the first
-  // half's products it reads the second half's and sends for pieces [0, PB) of stage t + 2; then stage t + 1 has to be
-  // there, and every wave done with stage t.  NST 3: its slots take the other pieces of stage t + 3 behind the second
+  // half's products it reads the second half's and sends for pieces [0, PB) of stage t + F; then stage t + 1 has to be
+  // there, and every wave done with stage t.  NST > 2: its slots take the other pieces of stage t + NST behind the second
   // half's products.  NST 2: its w slot takes the w pieces of stage t + 2.
-  Slot s0{0, 0}, s1{1, 1}, s2 = after(s1);
-  issue(0, s0, 0, PIECES);
-  if (nk > 1) issue(1, s1, 0, PIECES);
-  if (NST == 3 && nk > 2) issue(2, s2, PB, PIECES);
-  if (NST == 3 && nk > 2) wait_vm<2 * PIECES - PB>(); else if (nk > 1) wait_vm<PIECES>(); else wait_vm<0>();
+  Slot s0{0, 0}, s1{1, 1}, sf{F, F % NST};               // slots of stages t, t + 1, t + F
+#pragma unroll
+  for (int u = 0; u < F; ++u)
+    if (u < nk) issue(u, Slot{u, u % NST}, 0, PIECES);
+  constexpr int first = (F - 1) * PIECES;                // what may be missing behind stage 0
+  if (NST > 2 && nk > F) issue(F, sf, PB, PIECES), wait_vm<first + (NST > 2 ? PIECES - PB : 0)>();
+  else if (nk >= F) wait_vm<first>();
+  else wait_vm<0>();
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   frags(0, s0, 0, NI + MJ);
   int t = 0;
-  for (; t + A < nk; ++t) {
-    half(0, s0, t + 2, s2, 0, PB);
-    wait_vm<NST == 3 ? PIECES : PB>();
+  for (; t + NST < nk; ++t) {
+    half(0, s0, t + F, sf, 0, PB);
+    wait_vm<(NST > 2 ? first : PB)>();
     done_reading();
-    half(1, s1, t + A, NST == 3 ? s0 : Slot{s2.x, s0.w}, PB, PIECES);
-    s0 = s1, s1 = s2, s2 = after(s2);
+    half(1, s1, t + NST, NST > 2 ? s0 : Slot{sf.x, s0.w}, PB, PIECES);
+    s0 = s1, s1 = after(s1), sf = after(sf);
   }
   for (; t < nk; ++t) {                                  // the last stages
-    half(0, s0, t + 2 < nk ? t + 2 : -1, s2, 0, PB);
-    if (NST == 3 && t + 2 < nk) wait_vm<PIECES>(); else wait_vm<0>();
+    half(0, s0, t + F < nk ? t + F : -1, sf, 0, PB);
+    wait_stages<NST == 2 ? 0 : F - 1, PIECES>(nk - 2 - t);
     done_reading();
-    half(1, s1, -1, s2, 0, 0);                           // (the last step reads a slot that holds an earlier stage: unused)
-    s0 = s1, s1 = s2, s2 = after(s2);
+    half(1, s1, -1, s1, 0, 0);                           // (the last step reads a slot that holds an earlier stage: unused)
+    s0 = s1, s1 = after(s1), sf = after(sf);
   }
   settle();
 }

@@ -13,6 +13,8 @@ using namespace lumen;
 
 namespace {
 
+constexpr int MJ = 8, BM = 32 * MJ;                      // rows of a tile
+
 struct ActArgs {
   const void* x; long long ldx;
   const void* w;               // [2 ff, K] contiguous
@@ -42,29 +44,29 @@ __device__ __forceinline__ float gated(const GateForm& f, float g, float u) {
 
 template <typename T, int NI, int ACT>
 __global__ void __launch_bounds__(256, 1) tile_act_kernel(const ActArgs a) {
-  using tile::Shape;
   using tile::hold;
-  constexpr int PIECES = Shape<NI>::PIECES, MJ = tile::MJ, CT = 16 * NI;         // CT: result columns of a tile
-  __shared__ __attribute__((aligned(16))) char lds[Shape<NI>::LDS];
+  using S = tile::Shape<NI, MJ>;
+  constexpr int PIECES = S::PIECES, CT = 16 * NI;        // CT: result columns of a tile
+  __shared__ __attribute__((aligned(16))) char lds[S::LDS];
   const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int tm, tn;
   tile::tile_at(tile::unit_of(blockIdx.x, gridDim.x), a.tiles_m, a.tiles_n, a.group, tm, tn);
-  const int m0 = tm * tile::BM, n0 = a.c0 + tn * CT;
+  const int m0 = tm * BM, n0 = a.c0 + tn * CT;
   unsigned off[PIECES];                                  // (rows past the edge read the last row: never stored)
 #pragma unroll
   for (int q = 0; q < PIECES; ++q) {
-    const int r = 8 * (wid + 4 * (q < 8 ? q : q - 8)) + (lane >> 3), c = (lane & 7) ^ tile::swz(r);
+    const int r = 8 * (wid + 4 * (q < MJ ? q : q - MJ)) + (lane >> 3), c = (lane & 7) ^ tile::swz(r);
     const int col = min(n0 + r / (16 * NI) * (8 * NI) + col_of<NI>(r % (16 * NI)), a.c1 - 1);
-    off[q] = q < 8 ? (unsigned)min(r, a.M - m0 - 1) * (unsigned)(2 * a.ldx) + 16 * c
+    off[q] = q < MJ ? (unsigned)min(r, a.M - m0 - 1) * (unsigned)(2 * a.ldx) + 16 * c
                    : (unsigned)(col + ((r >> 4) & 1 ? a.ff : 0)) * (unsigned)(2 * a.K) + 16 * c;
   }
   tile::f32x4 acc[NI][MJ];
-  tile::products<T, NI>(lds, (const char*)a.x + (long long)m0 * a.ldx * 2, (const char*)a.w, a.K / tile::BK, off, acc);
+  tile::products<T, NI, MJ>(lds, (const char*)a.x + (long long)m0 * a.ldx * 2, (const char*)a.w, a.K / tile::BK, 0, off, acc);
   // lane (lr, lg) holds row 16 j + lr, columns col_of(16 i + 4 lg ..), of gate (i even) and up (i odd)
 #pragma unroll
   for (int j = 0; j < MJ; ++j) {
-    const int m = m0 + 128 * (wid >> 1) + 16 * j + lr;
+    const int m = m0 + 16 * MJ * (wid >> 1) + 16 * j + lr;
 #pragma unroll
     for (int i = 0; i < NI; i += 4) {
       constexpr int last = NI - 1;
@@ -101,7 +103,7 @@ hipError_t sm_tile_act(int dt, const void* x, long long ldx, const void* w, void
       ldx % 8 || ldx < K || ldx > (1 << 22) || 4LL * ff * K >= (1LL << 32) || (dt != kF16 && dt != kBF16) || act < 0 || act > 4 ||
       ((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) % 16 || (ni != 4 && ni != 6 && ni != 8))
     return hipErrorInvalidValue;
-  const long long tm = (M + tile::BM - 1LL) / tile::BM, tn = (c1 - c0 + 16 * ni - 1) / (16 * ni);
+  const long long tm = (M + BM - 1LL) / BM, tn = (c1 - c0 + 16 * ni - 1) / (16 * ni);
   if (tm * tn >= (1 << 20)) return hipErrorInvalidValue;
   const ActArgs a{x, ldx, w, y, M, ff, K, c0, c1, (int)tm, (int)tn, (int)(tm < 4 ? tm : 4),
                   GateForm{act, 0, limit, limit, slope, shift}};

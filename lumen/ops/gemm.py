@@ -2,9 +2,9 @@
 
 Up to 64 rows the projection is a stream of the weight matrix: the HIP kernels
 ``seqmix/thin_gemm.hip`` (1 - 64 rows) and ``kernels/skinny_gemm.hip`` (1 row) run it where they
-measured faster than a library GEMM; long contractions over some more rows are cut along K
-(``kernels/tile_gemm.hip``), and products whose result is about one round of its tiles go there whole.  The rest (and CPU tensors) goes to ``torch.matmul`` (hipBLASLt with the
-tuned table)."""
+measured faster than a library GEMM; from 17 rows on wide results, results of about one round of its tiles, and long
+contractions, cut along K, run on ``kernels/tile_gemm.hip``.  The rest (and CPU tensors) goes to ``torch.matmul``
+(hipBLASLt with the tuned table)."""
 from __future__ import annotations
 
 import os
@@ -234,27 +234,69 @@ def row_stream_linear(x: torch.Tensor, y: Optional[torch.Tensor], norm_w: torch.
     return z, s
 
 
-# Split-K GEMM (kernels/tile_gemm.hip): long contractions over a few hundred rows, whose output has too few
-# tiles to fill the chip.  us, library -> split: K = 11008, N = 4096, rows 72 / 256 / 512 / 1000: 41 -> 32, 51 ->
-# 35, 72 -> 50, 113 -> 87; K = 22016 at 512: 139 (tuned) -> 91; K = 32000 at 512: 290 -> 123; K = 11264, N = 2048 at
-# 320 / 1000: 48 -> 32, 72 -> 51.  Below K = 8192 the slabs cost what the split gains (K = 4096 at 512 rows: 28.2
-# and 28.4; K = 5632, N = 2048 at 200: 19.2 and 21.5).  Over 128 tiles a slice would be less than half of K
-# on more workgroups than CUs; under 128 workgroups most CUs idle.
-SPLIT_MIN_M, SPLIT_MIN_K, SPLIT_MAX_S = 65, 8192, 8
+# Split-K GEMM (kernels/tile_gemm.hip): contractions whose output has too few tiles to fill the chip.  Tiles of 128 columns
+# and 64 rows, from 65 rows on 128, from some 200 on 256.  us, library or thin kernel -> split:
+#  * 241 rows and more, K from 8192 on: K = 11008, N = 4096, rows 256 / 512 / 1000: 51 -> 35, 72 -> 50, 113 -> 87; K = 22016 at 512:
+#    139 (tuned) -> 91; K = 32000 at 512: 290 -> 123; K = 11264, N = 2048 at 320 / 1000: 48 -> 32, 72 -> 51.  Below, the slabs cost
+#    what the split gains (K = 4096 at 512 rows: 28.2 and 28.4).
+#  * 33 - 64 rows (256-row tiles were no gain): 64 x 2048 x 11264 32.7 -> 19.5, x 8192 23.9 -> 16.4, 64 x 4096 x 11008 33.3 -> 25.4, 48 x
+#    3072 x 5632 17.7 -> 15.6 (33 x 4096 x 5632 16.2 -> 17.8); 17 - 32 rows from K = 11008 on: 24 x 2048 x 11264 21.5 -> 18.4 (3072 x 8448 17.5 -> 18.3).  Shorter K where
+#    neither the thin kernel nor few_tiles takes the width: 64 x 5120 x 4096 24.5 -> 16.5, 6144 x 3072 21.1 -> 15.7; but 64 x 4096 x
+#    4096 14.4 -> 14.9, 2048 x 5632 13.6 -> 13.2, 8192 x 4096 18.9 -> 20.1.
+#  * 65 - 128 rows (256-row tiles -> 128): 128 x 4096 x 11008 39.2 -> 29.1, 72 x 2048 x 8192 23.0 -> 18.5; library -> here 128 x 4096 x 5632
+#    33.6 -> 21.7, 72 x 4096 x 4096 22.1 -> 17.9, 100 x 8192 x 4096 25.1 -> 23.9; but 2048 x 5632 13.9 -> 16.4, 3072 x 4096 14.5 -> 16.4.
+#  * 129 - 240 rows: 180 x 4096 x 11008 44.4 -> 34.6, 180 x 3072 x 5632 26.8 -> 21.3, 224 x 6144 x 4096 38.7 -> 27.9; 180 x 6144 x 4096 even.
+# Over 128 tiles a slice would be less than half of K on more workgroups than CUs; under 128 workgroups most CUs idle.
+# Walks apart (few_tiles) for up to 256 rows of 4096 columns and more: 64 x 8192 x 8192 40.0 -> 33.1, 4096 x 11008 26.7 -> 25.4, worst
+# 4096 x 8192 21.3 -> 22.3.
+SPLIT_MIN_K, SPLIT_FEW_K, SPLIT_MAX_S, SPLIT_FEW_M = 8192, 3072, 8, 240
+
+
+def split_plan(M: int, N: int, K: int) -> int:
+    """The split-K GEMM's form for x [M, K] @ w [N, K]^T: S slices + 16 mj + 256 for walks apart (mj 8, in step: S alone), or 0."""
+    if M < FEW_MIN_M or K < (SPLIT_FEW_K if M <= SPLIT_FEW_M else SPLIT_MIN_K):
+        return 0
+    if M <= 32:
+        if K < 11008 or not 4096 <= N <= 8192:
+            return 0
+    elif K >= SPLIT_MIN_K:
+        if N > 8192 if M <= 64 else N < 2048 and M <= SPLIT_FEW_M:
+            return 0
+    else:
+        wide = 4096 < N < FEW_MIN_N
+        if M <= 64:
+            pays = wide or K >= 5632 and 3072 <= N <= 4096 and M > 40
+        elif M <= 128:
+            pays = wide or (K >= 5632 and N >= 3072 or K >= 4096 and N >= 4096) and N <= 8192
+        else:
+            pays = K >= 4096 and (wide or N == 4096) or K >= 5632 and 3072 <= N < FEW_MIN_N
+        if not pays:
+            return 0
+    mj = 2 if M <= 64 else 4 if M <= 128 or N <= (5376 if M <= 192 else 2048 if K >= SPLIT_MIN_K or M > SPLIT_FEW_M else 4096) else 8
+    if M > SPLIT_FEW_M:
+        mj = 8
+    tiles = -(-M // (32 * mj)) * -(-N // 128)
+    if not 0 < tiles <= 128:
+        return 0
+    S = min(SPLIT_MAX_S if M > SPLIT_FEW_M else 12, TILE_CUS // tiles)
+    if tiles * S < 128:
+        return 0
+    apart = 256 if M <= 256 and N >= 4096 else 0
+    return S + apart + 16 * mj if apart or mj < 8 else S
 
 
 def split_slices(x: torch.Tensor, w: torch.Tensor) -> int:
-    """Slices of K in which the split-K GEMM should run x [M, K] @ w [N, K]^T (0: leave it to the library)."""
+    """``split_plan`` of x [M, K] @ w [N, K]^T of 65 rows and more, 0 where the kernel cannot run it (leave it to the others)."""
+    return _slices(x, w) if x.shape[0] > THIN_MAX_M else 0
+
+
+def _slices(x: torch.Tensor, w: torch.Tensor) -> int:
     xs = x.shape
-    if len(xs) != 2 or xs[1] < SPLIT_MIN_K or w.dim() != 2 or not x.is_cuda:
+    if len(xs) != 2 or xs[1] < SPLIT_FEW_K or w.dim() != 2 or not x.is_cuda:
         return 0                                   # (nearly every call: as little host time as can be)
-    (M, K), (N, Kw) = xs, w.shape
-    tiles = -(-M // 256) * -(-N // 128)
-    if not (M >= SPLIT_MIN_M and K == Kw and 0 < tiles <= 128):
-        return 0
-    S = min(SPLIT_MAX_S, 256 // tiles)
-    dt = x.dtype
-    if (tiles * S < 128 or K % 64 or N % 4 or K >= 1 << 22 or dt != w.dtype
+    (M, K), (N, Kw), dt = xs, w.shape, x.dtype
+    S = split_plan(M, N, K)
+    if (not S or K != Kw or K % 64 or N % 4 or K >= 1 << 22 or dt != w.dtype
             or dt not in (torch.bfloat16, torch.float16) or x.device != w.device
             or not _plain(x, w) or not _here(x) or not use_native(x)):
         return 0
@@ -262,9 +304,9 @@ def split_slices(x: torch.Tensor, w: torch.Tensor) -> int:
 
 
 def split_linear(x: torch.Tensor, w: torch.Tensor, S: int) -> torch.Tensor:
-    """x [M, K] @ w [N, K]^T in S slices of K, their fp32 sums added in order and rounded once.  Callers
+    """x [M, K] @ w [N, K]^T in slices of K, their fp32 sums added in order and rounded once.  Callers
     take S from ``split_slices``."""
-    return native().split_gemm(x, w, S)
+    return native().split_gemm(x, w, S & 15, S >> 4 & 15 or 8, S > 255)
 
 
 # One round of 256 x 32 ni tiles (kernels/tile_gemm.hip) where some ni makes the result about one wave of the chip.  At
@@ -276,7 +318,6 @@ def split_linear(x: torch.Tensor, w: torch.Tensor, S: int) -> torch.Tensor:
 # worst 3000 x 1536 x 2048, 0.73, 23.2 -> 24.4).
 TILE_MIN_M, TILE_MIN_K, TILE_CUS = 256, 512, 256
 TILE_FILL, TILE_FILL_ODD = 0.85, 0.75
-TILE_MIN_MN = int(TILE_FILL_ODD * TILE_CUS * 8192 * 3)     # fewer results than any such round has (asked first: host time)
 
 
 def tile_columns(M: int, N: int, K: int) -> int:
@@ -291,6 +332,71 @@ def tile_columns(M: int, N: int, K: int) -> int:
     return 0
 
 
+# Up to 256 rows of wide matrices, and 96- and 160-column tiles above (us, library or thin kernel -> here, bf16, weights
+# from HBM; K where nothing is said 4096).  A tile takes 64 rows, from 65 on 128, for the widest from 177 on 256, and the
+# narrowest number of columns that makes the result one round of workgroups.
+#  * Tiles of one column start their walk of k apart where rows of w lie a multiple of 4 KiB apart: in step, all tiles would
+#    read a stage of their rows from the same memory channels (in step / apart: 40 x 24576 45.9 / 38.8, x 2048 26.0 / 21.4, x
+#    6144 71.6 / 57.0; x 3072 30.5 / 31.0).  The library and the thin kernel walk in step, so this is where most is gained.
+#    From 257 rows on x costs more than w and is better read in step.
+#  * 17 - 64 rows, from three quarters of a round on (32 columns: nine tenths): 40 x 8192 18.4 -> 16.7, 24576 47.5 -> 38.8, 32000 61 -> 48, 64000 124 -> 98, 32000
+#    x 2048 33.6 -> 27.7, 24576 x 1024 19.4 -> 13.2.  Not less than that (40 x 4096 12.6 -> 15.2).  Long K in step only with 32
+#    or 96 columns (40 x 8192 x 2816 19.9 -> 13.3, 24576 x 5120 51.2 -> 48.8; 64 x 14336 x 5120 33.3 -> 36.1, 7680 x 5632 25.2
+#    -> 26.6, 32000 x 5120 63.6 -> 67.4).  Up to 32 rows the thin kernel keeps 32-column tiles of long K (20 x 8192 14.7 -> 15.9) and what takes
+#    128 - 192 columns (20 x 32000 x 2048 26.5 -> 27.4).
+#  * 65 - 128 rows, from nine tenths of a round on, up to K = 2048 three quarters: 100 x 22016 49.1 -> 41.3, 32000 64 -> 51, 64000
+#    132 -> 104, 12288 x 1024 12.1 -> 10.3; not long K in step (32000 x 2816 39.3 -> 39.5, 128 x 22016 x 2816 32.8 -> 35.2).
+#  * 177 - 256 rows as 2 x 64- or 96-column tiles: 256 x 8192 42.5 -> 31.9, x 12288 x 2048 28.5 -> 22.3, 180 x 12288 40.6 -> 33.8, 8192
+#    27.5 -> 27.1; as 256 x 96: 200 x 22016 60.8 -> 56.1, x 1024 22.4 -> 19.5, x 5120 even.  At
+#    130 - 160 rows the second row tile is mostly padding (161 x 24576 x 1024 19.8 -> 21.8).
+#  * above: 1000 x 3072 32.3 -> 29.0, 500 x 5120 38.1 -> 34.6, 1000 x 5120 50.3 -> 46.3, x 1024 19.2 -> 15.8; long K even (512 x 5120 x
+#    5632 49.1 -> 49.5), other widths are the library's (512 x 8192 41.7 -> 42.8, 768 x 6144 x 2816 33.9 -> 34.2).
+FEW_MIN_M, FEW_MIN_N, FEW_MIN_MN = 17, 7168, 1 << 21
+FEW_NI = {2: (1, 2, 3, 4, 5, 6, 8), 4: (2, 3, 4, 5, 6, 8), 8: (3, 4, 5, 6)}
+
+
+def _round(M: int, N: int, mj: int) -> tuple:
+    """(ni, filled share of its rounds) of the narrowest 32 mj x 32 ni tiles that are one round, else the widest."""
+    tm = -(-M // (32 * mj))
+    for ni in FEW_NI[mj]:
+        tiles = tm * -(-N // (32 * ni))
+        if tiles <= TILE_CUS:
+            break
+    return ni, tiles / (-(-tiles // TILE_CUS) * TILE_CUS)
+
+
+def few_tiles(M: int, N: int, K: int) -> int:
+    """The tiles on which x [M, K] @ w [N, K]^T should run beside ``tile_columns``: ni + 16 mj + 256 for walks apart, or 0."""
+    if M < FEW_MIN_M or K < 1024 or K >= SPLIT_MIN_K:
+        return 0
+    if M > 256:
+        if K > 4096 or M * N > TILE_CUS * 4096 * 5:    # (first: short prompts and training steps wait for the host)
+            return 0
+        tm, lead = -(-M // 128), 0.8 * TILE_CUS * 4096
+        if tm * -(-N // 96) <= TILE_CUS < tm * -(-N // 64):
+            return 3 + 64 if M * N >= 3 * lead else 0
+        if tm * -(-N // 160) <= TILE_CUS < tm * -(-N // 128):
+            return 5 + 64 if M * N >= 5 * (lead if K <= 2048 else 0.95 * TILE_CUS * 4096) else 0
+        return 0
+    apart = 256 if K % 2048 == 0 else 0
+    free = apart or K <= 2048                          # not held up by what the others read
+    if M <= 64:
+        ni, fill = _round(M, N, 2)
+        pays = fill >= (0.88 if ni == 1 else 0.72) and (free or ni in (1, 3)) and (
+            K <= (3072 if M <= 32 else 4096) if ni == 1 else M > 32 or ni <= 3 or ni == 8)
+        return ni + 32 + apart if pays else 0
+    if M <= 128:
+        ni, fill = _round(M, N, 4)
+        return ni + 64 + apart if free and N <= 65536 and fill >= (0.72 if K <= 2048 else 0.88) else 0
+    if M <= 176:
+        return 0
+    ni, fill = _round(M, N, 4)
+    if ni <= 3:
+        return ni + 64 + apart if fill >= 0.88 else 0
+    ni, fill = _round(M, N, 8)
+    return ni + 128 + apart if ni == 3 and fill >= 0.88 and (apart or K <= 4608) else 0
+
+
 def _aligned(x: torch.Tensor, w: torch.Tensor, K: int) -> bool:
     (lx, ex), (lw, ew) = x.stride(), w.stride()
     return (ex == 1 and ew == 1 and lx % 8 == 0 and lw % 8 == 0 and K <= lx <= 1 << 22 and K <= lw <= 1 << 22
@@ -298,12 +404,12 @@ def _aligned(x: torch.Tensor, w: torch.Tensor, K: int) -> bool:
 
 
 def tile_ok(x: torch.Tensor, w: torch.Tensor) -> int:
-    """``tile_columns`` of x @ w^T, 0 where the kernel cannot run it."""
+    """``tile_columns`` or ``few_tiles`` of x @ w^T, 0 where the kernel cannot run it."""
     xs, ws = x.shape, w.shape
     if len(xs) != 2 or len(ws) != 2 or not x.is_cuda:
         return 0
     (M, K), (N, Kw), dt = xs, ws, x.dtype
-    ni = tile_columns(M, N, K)
+    ni = tile_columns(M, N, K) or few_tiles(M, N, K)
     if (not ni or K != Kw or K % 64 or N % 4 or K >= 1 << 22 or dt != w.dtype
             or dt not in (torch.bfloat16, torch.float16) or x.device != w.device
             or not _plain(x, w) or not _here(x) or not use_native(x) or not _aligned(x, w, K)):
@@ -312,18 +418,19 @@ def tile_ok(x: torch.Tensor, w: torch.Tensor) -> int:
 
 
 def tile_linear(x: torch.Tensor, w: torch.Tensor, ni: int, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """x [M, K] @ w [N, K]^T (+ ``bias`` [N]) on 256 x 32 ni tiles, rounded once.  Callers take ``ni`` from ``tile_ok``."""
-    return native().tile_gemm(x, w, ni, bias)
+    """x [M, K] @ w [N, K]^T (+ ``bias`` [N]) on 256 x 32 ni tiles or ``few_tiles``', rounded once.  Callers take ``ni`` from
+    ``tile_ok``."""
+    return native().tile_gemm(x, w, ni & 15, bias, None, ni >> 4 & 15 or 8, ni > 255)
 
 
 def matmul_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x @ w[N, K]^T: the split-K GEMM or one round of tiles where they are the faster ones, else ``torch.matmul``."""
     xs = x.shape
     if len(xs) == 2:                               # (short prompts wait for the host)
-        S = split_slices(x, w) if xs[1] >= SPLIT_MIN_K else 0
+        S = split_slices(x, w) if xs[1] >= SPLIT_FEW_K else 0
         if S:
             return split_linear(x, w, S)
-        ni = tile_ok(x, w) if xs[0] * w.shape[0] >= TILE_MIN_MN else 0
+        ni = tile_ok(x, w) if xs[0] * w.shape[0] >= FEW_MIN_MN or w.shape[0] >= FEW_MIN_N else 0
         if ni:
             return tile_linear(x, w, ni)
     return torch.matmul(x, w.t())
@@ -333,9 +440,13 @@ def _mm_into(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor) -> None:
     """y = x @ w^T into a column view of operands that ``_split_plan`` has let pass."""
     ni = tile_ok(x, w)
     if ni and y.stride(0) % 4 == 0 and y.data_ptr() % 8 == 0:
-        native().tile_gemm(x, w, ni, None, y)
+        native().tile_gemm(x, w, ni & 15, None, y, ni >> 4 & 15 or 8, ni > 255)
     else:
         torch.mm(x, w.t(), out=y)
+
+
+def _bias_ok(bias: torch.Tensor, x: torch.Tensor, w: torch.Tensor) -> bool:
+    return row_bias_ok(bias, x, w.shape[0]) and _plain(bias) and bias.data_ptr() % 8 == 0
 
 
 def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -343,12 +454,19 @@ def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = Non
     one row of a large matrix), the library otherwise."""
     xs = x.shape
     if len(xs) == 2 and xs[0] > THIN_MAX_M:            # (first: short prompts are bound by the host)
-        MN = xs[0] * w.shape[0]
-        if bias is None and (xs[1] >= SPLIT_MIN_K or MN >= TILE_MIN_MN) and x.is_cuda:
+        many = xs[0] * w.shape[0] >= FEW_MIN_MN or w.shape[0] >= FEW_MIN_N
+        if bias is None and (xs[1] >= SPLIT_FEW_K or many) and x.is_cuda:
             return mm_nt(x, w)
-        ni = (tile_ok(x, w) if MN >= TILE_MIN_MN and bias is not None and row_bias_ok(bias, x, w.shape[0]) and _plain(bias)
-              and bias.data_ptr() % 8 == 0 else 0)
+        ni = tile_ok(x, w) if many and bias is not None and _bias_ok(bias, x, w) else 0
         return tile_linear(x, w, ni, bias) if ni else F.linear(x, w, bias)
+    if len(xs) == 2 and xs[0] >= FEW_MIN_M and w.shape[0] >= FEW_MIN_N:
+        ni = tile_ok(x, w) if bias is None or _bias_ok(bias, x, w) else 0
+        if ni:
+            return tile_linear(x, w, ni, bias)
+    elif len(xs) == 2 and bias is None and xs[0] >= FEW_MIN_M and xs[1] >= SPLIT_FEW_K:
+        S = _slices(x, w)
+        if S:
+            return split_linear(x, w, S)
     if thin_ok(x, w) and (bias is None or row_bias_ok(bias, x, w.shape[0]) and _plain(bias)):
         return _thin(x, w, bias)
     if bias is None and len(xs) == 2 and xs[0] == 1 and _plain(x, w) and _here(x) and skinny_ok(x, w):
@@ -645,7 +763,14 @@ def mm_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 def linear_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x [M, K] @ w[N, K]^T -> [M, N]."""
-    M = x.shape[0]
+    M, K = x.shape
+    if FEW_MIN_M <= M <= SPLIT_FEW_M:                  # (before the planned shapes: 128 x 4096 x 11008 39 -> 29 us)
+        S = _slices(x, w) if K >= SPLIT_FEW_K else 0
+        if S:
+            return split_linear(x, w, S)
+        ni = tile_ok(x, w) if w.shape[0] >= FEW_MIN_N else 0
+        if ni:
+            return tile_linear(x, w, ni)
     if M <= THIN_MAX_M:
         if thin_ok(x, w) and use_native(x):
             return _thin(x, w)

@@ -29,7 +29,7 @@ from typing import Optional, Union
 import torch
 import torch.nn.functional as F
 
-from .gemm import (MID_MAX_M, THIN_BATCH_MAX_W, THIN_MAX_K, THIN_MAX_M, _here, _plain, _thin, mid_ok, project, row_bias_ok,
+from .gemm import (MID_MAX_M, THIN_BATCH_MAX_W, THIN_MAX_K, THIN_MAX_M, _here, _plain, _thin, few_tiles, mid_ok, project, row_bias_ok,
                    thin_ok, weights_ok)
 
 
@@ -421,12 +421,17 @@ def act_rounds(M: int, ff: int) -> tuple:
 # 63, 1000 172 -> 159, 4010 574 -> 538.  It needs the more of the tiles' area filled the longer a product is, as the library cuts
 # long products of few tiles along K: over 370 sizes of 130 - 8000 rows and widths 512 - 4096 it is 0.95 - 1.99 times as fast under
 # this rule, 1.22 in the mean (left out: 300 rows, width 4096, filled 0.54, 78 -> 80; 1290 rows, 0.68, 235 -> 248; 220, ff 3000, width 2048, 0.16, 20 -> 25).
+# Up to 256 rows the product has tiles of 128 rows, and up to 224 walks of k apart, which are worth more than the pass (192 x 5632 x
+# 2048 28.8 here, 23.7 with the pass, 224 x 11008 x 4096 62.9 and 61.0; 256 x 11264 x 4096 61.2 and 65.6).
 ACT_TILE_FILL, ACT_TILE_FILL_MANY = 8192, 6000             # K over the filled share, up to 256 rows and above
 
 
 def _act_tiles_pay(M: int, ff: int, K: int) -> bool:
     tm = -(-M // 256)
     cells = sum(256 * 256 * 16 * ni * -(-(tm * -(-(c1 - c0) // (16 * ni))) // 256) for c0, c1, ni in act_rounds(M, ff))
+    few = few_tiles(M, 2 * ff, K) if M <= 256 else 0
+    if few and (M <= 224 or few >> 4 & 15 == 4):
+        return False
     return M * ff * (ACT_TILE_FILL if M <= 256 else ACT_TILE_FILL_MANY) >= K * cells > 0
 
 

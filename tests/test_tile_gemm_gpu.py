@@ -83,3 +83,89 @@ def test_routes():
     for c in (0, n1 - 8, n1, 5616):
         want, tol = bound(x[:64], w[c:c + 16], None, torch.float16)
         assert ((y[:64, c:c + 16].double().cpu() - want).abs() <= tol).all()
+
+
+# 64- and 128-row tiles: one row and one past a tile, columns past one, fewer stages of k than the ring has and more, walks apart
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("mj,ni", [(2, 1), (2, 2), (2, 3), (2, 4), (2, 5), (2, 6), (2, 8), (4, 2), (4, 3), (4, 4), (4, 5), (4, 6), (4, 8),
+                                   (8, 3), (8, 4)])
+@pytest.mark.parametrize("M,N,K,lead,bias", [(64, 512, 64, 0, False), (65, 260, 384, 8, True), (17, 1004, 448, 0, True),
+                                             (129, 100, 128, 64, False), (257, 36, 1088, 0, True)])
+def test_row_tiles(M, N, K, lead, bias, mj, ni, dt):
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K + lead, generator=g).to(dt).to(dev)[:, :K]
+    w = torch.randn(N, K + lead, generator=g).to(dt).to(dev)[:, :K]
+    b = torch.randn(N, generator=g).to(dt).to(dev) if bias else None
+    want, tol = bound(x, w, b, dt)
+    for apart in (False, True):
+        y = torch.full((M, N + 16), 7.0, dtype=dt, device=dev)
+        native().tile_gemm(x, w, ni, b, y[:, 4:4 + N], mj, apart)
+        assert ((y[:, 4:4 + N].double().cpu() - want).abs() <= tol).all()
+        assert (y[:, :4] == 7.0).all() and (y[:, 4 + N:] == 7.0).all()
+
+
+def test_few_tiles_rule():
+    forms = {(2, n) for n in (1, 2, 3, 4, 5, 6, 8)} | {(4, n) for n in (2, 3, 4, 5, 6, 8)} | {(8, 3)}
+    for M in (1, 16, 17, 33, 64, 65, 128, 129, 176, 177, 256, 257, 500, 1000, 70000):
+        for N in (64, 4096, 7168, 8192, 12288, 22016, 24576, 32000, 64000, 128256, 1 << 20):
+            for K in (64, 1024, 2048, 2816, 4096, 5632, 8192):
+                code = gemm.few_tiles(M, N, K)
+                if code:
+                    assert 17 <= M and 1024 <= K < 8192 and (code >> 4 & 15, code & 15) in forms
+                    assert (code > 255) == (K % 2048 == 0 and M <= 256)
+                    if M <= 256:                        # asked only for as many columns or results
+                        assert N >= gemm.FEW_MIN_N
+                    assert M * N >= gemm.FEW_MIN_MN or N >= gemm.FEW_MIN_N
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(33, 8192, 2048), (64, 32000, 1024), (20, 22016, 1024), (100, 24576, 2048), (200, 12288, 1024),
+                                   (1000, 3072, 1024)])
+def test_few_route(M, N, K):
+    x, w = torch.randn(M, K, device=dev).bfloat16(), torch.randn(N, K, device=dev).bfloat16()
+    b = torch.randn(N, device=dev).bfloat16()
+    code = gemm.tile_ok(x, w)
+    assert code == gemm.few_tiles(M, N, K) > 0
+    y = native().tile_gemm(x, w, code & 15, None, None, code >> 4 & 15, code > 255)
+    for out in (gemm.linear_nt(x, w), gemm.project(x, w), gemm.matmul_nt(x, w)):
+        assert torch.equal(out, y)
+    assert torch.equal(gemm.project(x, w, b), native().tile_gemm(x, w, code & 15, b, None, code >> 4 & 15, code > 255))
+    for a, c in ((x[:, :-8], w[:, :-8]), (x.float(), w.float()), (x, w.half()), (x[:, 1:], w[:, 1:])):     # the general paths take these
+        assert gemm.tile_ok(a, c) == 0
+
+
+# slabs of 64- and 128-row tiles: the slices' sums over tiles' edges, and the rule's forms
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("mj", [2, 4, 8])
+@pytest.mark.parametrize("M,N,K,S", [(64, 128, 128, 2), (65, 260, 832, 12), (129, 100, 1088, 5), (17, 4, 192, 3), (200, 1000, 448, 2)])
+def test_row_slices(M, N, K, S, mj, dt):
+    g = torch.Generator().manual_seed(M + K)
+    x, w = torch.randn(M, K, generator=g).to(dt).to(dev), torch.randn(N, K, generator=g).to(dt).to(dev)
+    want, tol = bound(x, w, None, dt)
+    for apart in (False, True):
+        assert ((native().split_gemm(x, w, S, mj, apart).double().cpu() - want).abs() <= tol).all()
+
+
+def test_split_plan_rule():
+    for M in (1, 16, 17, 32, 33, 64, 65, 128, 129, 192, 193, 240, 241, 256, 257, 1000, 5000):
+        for N in (4, 1024, 2048, 3072, 4096, 5120, 6144, 8192, 12288, 32000):
+            for K in (64, 2048, 3072, 4096, 5632, 8192, 11264, 32768):
+                code = gemm.split_plan(M, N, K)
+                if code:
+                    S, mj = code & 15, code >> 4 & 15 or 8
+                    tiles = -(-M // (32 * mj)) * -(-N // 128)
+                    assert 2 <= S <= K // 64 and mj in (2, 4, 8) and 128 <= tiles * S <= 256 and K >= 3072
+                    assert code < 256 or M <= 256
+    assert gemm.split_plan(512, 4096, 8192) == 4 and gemm.split_plan(64, 2048, 8192) == 12 + 32
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(64, 4096, 11008), (33, 5120, 4096), (100, 4096, 5632), (180, 3072, 8448)])
+def test_split_route(M, N, K):
+    x, w = torch.randn(M, K, device=dev).bfloat16(), torch.randn(N, K, device=dev).bfloat16()
+    code = gemm.split_plan(M, N, K)
+    y = native().split_gemm(x, w, code & 15, code >> 4 & 15 or 8, code > 255)
+    for out in (gemm.linear_nt(x, w), gemm.project(x, w)):
+        assert torch.equal(out, y)

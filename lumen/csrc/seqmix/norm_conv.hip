@@ -249,12 +249,23 @@ dyt_canon_v4(const float* __restrict__ x, const float* __restrict__ w, const flo
 // channels) -- it reads and writes its own four channels of the tail, so nothing is shared.  (The strip
 // kernel walks 16 rows of different sequences in turn on 1 / 16 of the workgroups and leaves the tail to a
 // second launch: 8 rows of width 2048 11.4 + 4.5 us, here 4.0.)  Segments of more rows are walked in order.
+// A launch costs such a step 4 us and its work next to nothing, so what stands around it is part of it, channel by channel: the
+// sublayer's output y that the stream takes first (null: none), and the token shift of the result with its own tail (mu
+// null: none).  8 rows of width 2048: residual and convolution 4.1 + 4.3 -> 4.3 us, with shift and tail 18.3 -> 6.3.
+template <typename T>
+struct JoinArgs {
+  const T* y; const float *w, *b, *alpha;          // x += DyT(y)
+};
+struct ShiftArgs {
+  const float* mu; float* prev; int n; long long plane;
+};
+
 template <typename TO, int TAPS>
 __global__ void __launch_bounds__(64)
-dyt_canon_rows_v4(const float* __restrict__ x, const float* __restrict__ w,
+dyt_canon_rows_v4(float* __restrict__ x, const JoinArgs<TO> join, const float* __restrict__ w,
                   const float* __restrict__ b, const float* __restrict__ alpha,
                   const float* __restrict__ cw, float* __restrict__ tail, TO* __restrict__ out,
-                  const int* __restrict__ cu, const int* __restrict__ slot,
+                  const ShiftArgs shift, const int* __restrict__ cu, const int* __restrict__ slot,
                   const int* __restrict__ start, int W) {
   constexpr int K = TAPS - 1;
   const int c = 4 * (blockIdx.x * 64 + threadIdx.x), sg = blockIdx.y;
@@ -277,10 +288,25 @@ dyt_canon_rows_v4(const float* __restrict__ x, const float* __restrict__ w,
     for (int j = 0; j < 4; ++j) win[k][j] = 0.f;
     if (p0 - K + k >= 0) load4<float>(tp + (long long)k * W, win[k]);
   }
+  float jw[4], jb[4], ja = 0.f, pv[4] = {0.f, 0.f, 0.f, 0.f};
+  if (join.y != nullptr) {
+    ja = *join.alpha;
+    load4<float>(join.w + c, jw);
+    load4<float>(join.b + c, jb);
+  }
+  float* pp = shift.mu != nullptr ? shift.prev + (long long)slot[sg] * W + c : nullptr;
+  if (pp != nullptr && p0 > 0) load4<float>(pp, pv);
   for (int t = r0; t < r0 + len; ++t) {
     const long long i = (long long)t * W + c;
     float hc[4], o[4];
     load4<float>(x + i, hc);
+    if (join.y != nullptr) {
+      float yv[4];
+      load4<TO>(join.y + i, yv);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) hc[j] += dyt_f(yv[j], ja, jw[j], jb[j]);
+      store4<float>(x + i, hc);
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       hc[j] = dyt_f(hc[j], a, wv[j], bv[j]);
@@ -289,7 +315,21 @@ dyt_canon_rows_v4(const float* __restrict__ x, const float* __restrict__ w,
       for (int d = 1; d <= K; ++d) acc += cwv[j][K - d] * win[K - d][j];
       o[j] = hc[j] + acc;
     }
-    store4<TO>(out + i, o);
+    if (pp == nullptr) {
+      store4<TO>(out + i, o);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] = to_f32(from_f32<TO>(o[j]));       // the shift's input, as stored
+      for (int s = 0; s < shift.n; ++s) {
+        float m4[4], v[4];
+        load4<float>(shift.mu + (long long)s * W + c, m4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = o[j] + (pv[j] - o[j]) * m4[j];
+        store4<TO>(out + s * shift.plane + i, v);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) pv[j] = o[j];
+    }
 #pragma unroll
     for (int k = 0; k + 1 < K; ++k)
 #pragma unroll
@@ -301,6 +341,7 @@ dyt_canon_rows_v4(const float* __restrict__ x, const float* __restrict__ w,
   }
 #pragma unroll
   for (int k = 0; k < K; ++k) store4<float>(tp + (long long)k * W, win[k]);
+  if (pp != nullptr) store4<float>(pp, pv);
 }
 
 template <typename T>
@@ -394,15 +435,21 @@ hipError_t sm_dyt_canon(int dt, const float* x, const float* w, const float* b, 
   return hipGetLastError();
 }
 
-// Norm, convolution and the tail's move over S short segments (decoded rows); W % 4 == 0, taps <= 8.
-hipError_t sm_dyt_canon_rows(int dt, const float* x, const float* w, const float* b,
-                             const float* alpha, const float* cw, float* tail, void* out,
-                             const int* cu, const int* slot, const int* start, int S, int W,
-                             int taps, hipStream_t st) {
+// Norm, convolution and the tail's move over S short segments (decoded rows) of T rows; W % 4 == 0, taps <= 8.  With y [T, W] in
+// out's type (or null) x += DyT(y) first; with mu [nmix, W] (or null) out is [nmix, T, W], the result's token shift, and prev
+// [slots, W] moves on.
+hipError_t sm_dyt_canon_rows(int dt, float* x, const void* y, const float* yw, const float* yb, const float* ya,
+                             const float* w, const float* b, const float* alpha, const float* cw, float* tail,
+                             void* out, const float* mu, float* prev, int nmix, const int* cu, const int* slot,
+                             const int* start, int S, int T, int W, int taps, hipStream_t st) {
   if ((long long)S * W == 0) return hipSuccess;
-  if (taps < 1 || taps > 8 || W % 4 || S > 65535) return hipErrorInvalidValue;
+  if (taps < 1 || taps > 8 || W % 4 || S > 65535 || (y && (!yw || !yb || !ya)) || (mu && (!prev || nmix < 1)))
+    return hipErrorInvalidValue;
   const dim3 grid((W / 4 + 63) / 64, S);
-#define GO(TT, TP) dyt_canon_rows_v4<TT, TP><<<grid, 64, 0, st>>>(x, w, b, alpha, cw, tail, (TT*)out, cu, slot, start, W)
+  const ShiftArgs shift{mu, prev, nmix, (long long)T * W};
+#define GO(TT, TP)                                                                                                   \
+  dyt_canon_rows_v4<TT, TP><<<grid, 64, 0, st>>>(x, JoinArgs<TT>{(const TT*)y, yw, yb, ya}, w, b, alpha, cw, tail,     \
+                                                 (TT*)out, shift, cu, slot, start, W)
 #define CALL(TT)                                                                   \
   switch (taps) {                                                                  \
     case 1: GO(TT, 1); break; case 2: GO(TT, 2); break; case 3: GO(TT, 3); break;  \

@@ -25,10 +25,29 @@ namespace {
 
 constexpr int TB = 8;   // tokens staged per batch
 
+// a's low-rank row times one row of w2, rounded as the product would be stored.  (Its own launch, a library product with K = 16,
+// took a decode step 7.5 us; here the scan of 8 rows x 16 heads takes 1 us more.)
+template <typename T>
+__device__ __forceinline__ float low_rank(const T* a, const T* b, int rank) {
+  float s = 0.f;
+  for (int e = 0; e < rank; e += 8) {
+    if constexpr (sizeof(T) == 2) {
+      const uint4 p = *reinterpret_cast<const uint4*>(a + e), q = *reinterpret_cast<const uint4*>(b + e);
+      const T *pa = reinterpret_cast<const T*>(&p), *qa = reinterpret_cast<const T*>(&q);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s = fmaf(to_f32(pa[j]), to_f32(qa[j]), s);
+    } else {
+      for (int j = 0; j < 8; ++j) s = fmaf(to_f32(a[e + j]), to_f32(b[e + j]), s);
+    }
+  }
+  return to_f32(from_f32<T>(s));
+}
+
 template <typename T, int KT, int KS, bool DELTA>
 __global__ void __launch_bounds__(1024)
 scan_kernel(const T* __restrict__ r, long long ldr, const T* __restrict__ k, long long ldk,
             const T* __restrict__ v, long long ldv, const T* __restrict__ wl, long long ldw,
+            const T* __restrict__ w2, int rank,            // wl's rows are w2's (or null) low-rank factor
             const T* __restrict__ al, long long lda, const T* __restrict__ gl, long long ldg,
             const float* __restrict__ w0, const float* __restrict__ ub,  // u (wkv) / a bias (delta)
             const float* __restrict__ normw, float* __restrict__ state, T* __restrict__ out,
@@ -70,7 +89,8 @@ scan_kernel(const T* __restrict__ r, long long ldr, const T* __restrict__ k, lon
       if (i < D) {
         rv = to_f32(r[row * ldr + col + i]);
         kv = to_f32(k[row * ldk + col + i]);
-        const float z = to_f32(wl[row * ldw + col + i]) + w0[col + i];
+        const float z = (w2 != nullptr ? low_rank(wl + row * ldw, w2 + (long long)(col + i) * rank, rank)
+                                       : to_f32(wl[row * ldw + col + i])) + w0[col + i];
         if (DELTA) {
           wv = expf(-decay_scale * sigmoid_f(z));
           xv = sigmoid_f(to_f32(al[row * lda + col + i]) + ub[col + i]);
@@ -179,7 +199,7 @@ scan_kernel(const T* __restrict__ r, long long ldr, const T* __restrict__ k, lon
 
 template <typename T, bool DELTA>
 hipError_t launch_scan(const void* r, long long ldr, const void* k, long long ldk, const void* v,
-                       long long ldv, const void* wl, long long ldw, const void* al,
+                       long long ldv, const void* wl, long long ldw, const void* w2, int rank, const void* al,
                        long long lda, const void* gl, long long ldg, const float* w0,
                        const float* ub, const float* normw, float* state, void* out,
                        long long ldo, const int* cu, const int* slot, const int* start, int S,
@@ -187,10 +207,11 @@ hipError_t launch_scan(const void* r, long long ldr, const void* k, long long ld
                        hipStream_t st) {
   if (S == 0) return hipSuccess;
   if (D < 1 || D > 256) return hipErrorInvalidValue;
+  if (w2 && (rank < 8 || rank % 8 || ldw % 8 || ldw < rank || ((uintptr_t)wl | (uintptr_t)w2) % 16)) return hipErrorInvalidValue;
   const dim3 grid(S, H);
 #define GO(KT, KS)                                                                               \
   scan_kernel<T, KT, KS, DELTA><<<grid, ((D * KS + 63) / 64) * 64, 0, st>>>(                     \
-      (const T*)r, ldr, (const T*)k, ldk, (const T*)v, ldv, (const T*)wl, ldw, (const T*)al, lda, \
+      (const T*)r, ldr, (const T*)k, ldk, (const T*)v, ldv, (const T*)wl, ldw, (const T*)w2, rank, (const T*)al, lda, \
       (const T*)gl, ldg, w0, ub, normw, state, (T*)out, ldo, cu, slot, start, H, D, eps,         \
       decay_scale, key_eps)
   if (D <= 32) GO(16, 2);
@@ -205,24 +226,25 @@ hipError_t launch_scan(const void* r, long long ldr, const void* k, long long ld
 
 extern "C" {
 
+// wl [rows, H D], or with w2 [H D, rank] (else null) its low-rank factor [rows, rank]: rank % 8 == 0, 16-byte rows
 hipError_t sm_wkv(int dt, const void* r, long long ldr, const void* k, long long ldk,
-                  const void* v, long long ldv, const void* wl, long long ldw, const void* g,
+                  const void* v, long long ldv, const void* wl, long long ldw, const void* w2, int rank, const void* g,
                   long long ldg, const float* w0, const float* u, const float* normw,
                   float* state, void* out, long long ldo, const int* cu, const int* slot,
                   const int* start, int S, int H, int D, float eps, hipStream_t st) {
-#define CALL(T) return launch_scan<T, false>(r, ldr, k, ldk, v, ldv, wl, ldw, nullptr, 0, g, ldg, w0, u, normw, state, out, ldo, cu, slot, start, S, H, D, eps, 0.f, 0.f, st)
+#define CALL(T) return launch_scan<T, false>(r, ldr, k, ldk, v, ldv, wl, ldw, w2, rank, nullptr, 0, g, ldg, w0, u, normw, state, out, ldo, cu, slot, start, S, H, D, eps, 0.f, 0.f, st)
   SM_DISPATCH(dt, CALL)
 #undef CALL
   return hipSuccess;
 }
 
 hipError_t sm_gdelta(int dt, const void* r, long long ldr, const void* k, long long ldk,
-                     const void* v, long long ldv, const void* wl, long long ldw, const void* al,
-                     long long lda, const void* gl, long long ldg, const float* w0,
+                     const void* v, long long ldv, const void* wl, long long ldw, const void* w2, int rank,
+                     const void* al, long long lda, const void* gl, long long ldg, const float* w0,
                      const float* a_b, const float* normw, float* state, void* out,
                      long long ldo, const int* cu, const int* slot, const int* start, int S,
                      int H, int D, float eps, float decay_scale, float key_eps, hipStream_t st) {
-#define CALL(T) return launch_scan<T, true>(r, ldr, k, ldk, v, ldv, wl, ldw, al, lda, gl, ldg, w0, a_b, normw, state, out, ldo, cu, slot, start, S, H, D, eps, decay_scale, key_eps, st)
+#define CALL(T) return launch_scan<T, true>(r, ldr, k, ldk, v, ldv, wl, ldw, w2, rank, al, lda, gl, ldg, w0, a_b, normw, state, out, ldo, cu, slot, start, S, H, D, eps, decay_scale, key_eps, st)
   SM_DISPATCH(dt, CALL)
 #undef CALL
   return hipSuccess;

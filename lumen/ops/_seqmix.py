@@ -26,8 +26,8 @@ SIGNATURES = {
     "sm_canon_tail": "ppppppppiii",
     "sm_token_shift": "ippppppppiii",
     "sm_shift_tail": "ippppii",
-    "sm_wkv": "iplplplplplppppplpppiiif",
-    "sm_gdelta": "iplplplplplplppppplpppiiifff",
+    "sm_wkv": "iplplplplpiplppppplpppiiif",
+    "sm_gdelta": "iplplplplpiplplppppplpppiiifff",
     "sm_write_k": "iplppii",
     "sm_chunk_attn": "iplpppippiiiiiffii",
     "sm_chunk_attn_tiles": "iplpppipippiiiiffiii",
@@ -80,7 +80,7 @@ SIGNATURES = {
     "sm_short_conv": "iplpppp" "pppp" "iii",
     "sm_conv_tail": "iiplpppp" "ppp" "iii",
     "sm_fill_step": "ppippippi" "pp" "ppl" "ppii" "ii",
-    "sm_dyt_canon_rows": "ipppppppppp" "iii",
+    "sm_dyt_canon_rows": "ippppp" "pppppp" "ppi" "ppp" "iiii",
     "sm_latent_tiles": "i" "plli" "plli" "pl" "pi" "pll" "pi" "pii" "pp" "ii" "fffi" "ppp" "pl",
     "sm_scan_chunk": "ii" "plplplplpl" "pppp" "ppp" "iii" "ff",
     "sm_thin_gemm": "iplpppliiii" "piii",

@@ -48,10 +48,39 @@ def dyt_canon_ref(x, norm, conv_w, tail, seg: SegBatch, out_dtype):
     return out.to(out_dtype)
 
 
+def _canon_step(x, norm, conv_w, tail, seg: SegBatch, out_dtype, joined, shift) -> torch.Tensor:
+    """A step of decoded rows in one launch where the kernel takes it, else one after the other."""
+    from ._seqmix import DT, call, use_seqmix
+    from .norm import dyt_residual
+    from .recurrent import token_shift
+
+    (T, W), taps = x.shape, conv_w.shape[1]
+    y, post = joined if joined is not None else (None, (None, None, None))
+    mu, prev = shift if shift is not None else (None, None)
+    if (use_seqmix(x) and seg.portions() == (0, 0) and W % 4 == 0 and taps <= 8 and 0 < seg.S <= 65535
+            and (y is None or y.dtype == out_dtype and y.shape == x.shape and y.is_contiguous())
+            and (tail.dtype == torch.float32 and tail.shape[1:] == (taps - 1, W) or taps == 1)):
+        assert x.dtype == torch.float32 and x.is_contiguous() and conv_w.dtype == torch.float32
+        assert mu is None or mu.dtype == torch.float32 and prev.dtype == torch.float32 and mu.is_contiguous()
+        n = 0 if mu is None else mu.shape[0]
+        out = torch.empty((n, T, W) if n else (T, W), dtype=out_dtype, device=x.device)
+        call("sm_dyt_canon_rows", DT[out_dtype], x, y, post[0], post[1], post[2], norm[0], norm[1], norm[2], conv_w, tail,
+             out, mu, prev, n, seg.cu, seg.slot, seg.start, seg.S, T, W, taps)
+        return out
+    if y is not None:
+        dyt_residual(x, y, post, None, out_dtype)
+    h = dyt_canon(x, norm, conv_w, tail, seg, out_dtype)
+    return h if mu is None else token_shift(h, mu, prev, seg)
+
+
 def dyt_canon(x: torch.Tensor, norm, conv_w: torch.Tensor, tail: torch.Tensor, seg: SegBatch,
-              out_dtype) -> torch.Tensor:
+              out_dtype, joined=None, shift=None) -> torch.Tensor:
+    """The convolution of DyT(x); ``joined`` = (y, its norm): the stream ``x`` takes a sublayer's output in place first
+    (``dyt_residual``); ``shift`` = (mu, prev): the token shift of the result instead (``token_shift``)."""
     from ._seqmix import DT, call, use_seqmix
 
+    if joined is not None or shift is not None:
+        return _canon_step(x, norm, conv_w, tail, seg, out_dtype, joined, shift)
     if not use_seqmix(x):
         return dyt_canon_ref(x, norm, conv_w, tail, seg, out_dtype)
     T, W = x.shape
@@ -60,8 +89,8 @@ def dyt_canon(x: torch.Tensor, norm, conv_w: torch.Tensor, tail: torch.Tensor, s
     assert tail.dtype == torch.float32 and tail.shape[1:] == (max(taps - 1, 0), W) or taps == 1
     out = torch.empty(T, W, dtype=out_dtype, device=x.device)
     if seg.portions() == (0, 0) and W % 4 == 0 and taps <= 8 and 0 < seg.S <= 65535:
-        call("sm_dyt_canon_rows", DT[out_dtype], x, norm[0], norm[1], norm[2], conv_w, tail, out,
-             seg.cu, seg.slot, seg.start, seg.S, W, taps)
+        call("sm_dyt_canon_rows", DT[out_dtype], x, None, None, None, None, norm[0], norm[1], norm[2], conv_w, tail, out,
+             None, None, 0, seg.cu, seg.slot, seg.start, seg.S, T, W, taps)
         return out
     call("sm_dyt_canon", DT[out_dtype], x, norm[0], norm[1], norm[2], conv_w, tail, out, seg.cu,
          seg.slot, seg.start, seg.row_seg, T, W, taps)

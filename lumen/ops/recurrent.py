@@ -145,24 +145,46 @@ def _chunk_portions(r, k, v, wl, al, gl, w0, ub, norm_w, state, out, seg: SegBat
     return P
 
 
-def wkv_scan(r, k, v, wl, g, w0, u, norm_w, state, seg: SegBatch, H: int, D: int, eps: float):
+def _low_rank(r, wl, w2, seg: SegBatch) -> tuple:
+    """(wl, None), wl = its low-rank factor times w2^T, or both as they are where the scan forms the product: a step of
+    decoded rows, 16-bit, 16-byte rows of at most 64 ranks."""
+    from ._seqmix import use_seqmix
+    from .gemm import _plain, project
+
+    if w2 is None:
+        return wl, None
+    rank = w2.shape[1]
+    if (use_seqmix(r) and seg.portions() == (0, 0) and r.dtype in (torch.bfloat16, torch.float16)
+            and wl.dtype == w2.dtype == r.dtype and wl.dim() == 2 and wl.shape[1] == rank and 0 < rank <= 64 and rank % 8 == 0
+            and w2.is_contiguous() and wl.stride(1) == 1 and wl.stride(0) % 8 == 0 and wl.stride(0) >= rank
+            and (wl.data_ptr() | w2.data_ptr()) % 16 == 0 and w2.device == wl.device == r.device and _plain(r, wl, w2)):
+        return wl, w2
+    return project(wl, w2), None
+
+
+def wkv_scan(r, k, v, wl, g, w0, u, norm_w, state, seg: SegBatch, H: int, D: int, eps: float, w2=None):
+    """The wkv recurrence over a step's segments.  With ``w2`` [H D, rank] ``wl`` is its low-rank factor [T, rank]."""
     from ._seqmix import DT, call, use_seqmix
 
+    wl, w2 = _low_rank(r, wl, w2, seg)
     if not use_seqmix(r):
         return wkv_scan_ref(r, k, v, wl, g, w0, u, norm_w, state, seg, H, D, eps)
     _check_state(state, H, D)
     T = r.shape[0]
     out = torch.empty(T, H * D, dtype=r.dtype, device=r.device)
     P = _chunk_portions(r, k, v, wl, None, g, w0, u, norm_w, state, out, seg, H, D, eps, "silu")
-    call("sm_wkv", DT[r.dtype], r, _ld(r), k, _ld(k), v, _ld(v), wl, _ld(wl), g, _ld(g), w0, u,
+    call("sm_wkv", DT[r.dtype], r, _ld(r), k, _ld(k), v, _ld(v), wl, _ld(wl), w2,
+         0 if w2 is None else w2.shape[1], g, _ld(g), w0, u,
          norm_w, state, out, H * D, seg.cu[P:], seg.slot[P:], seg.start[P:], seg.S - P, H, D, eps)
     return out
 
 
 def delta_scan(r, k, v, wl, al, gl, w0, a_b, norm_w, state, seg: SegBatch, H: int, D: int,
-               eps: float, decay_scale: float, key_eps: float):
+               eps: float, decay_scale: float, key_eps: float, w2=None):
+    """The delta rule over a step's segments; ``w2`` as in ``wkv_scan``."""
     from ._seqmix import DT, call, use_seqmix
 
+    wl, w2 = _low_rank(r, wl, w2, seg)
     if not use_seqmix(r):
         return delta_scan_ref(r, k, v, wl, al, gl, w0, a_b, norm_w, state, seg, H, D, eps,
                               decay_scale, key_eps)
@@ -171,7 +193,8 @@ def delta_scan(r, k, v, wl, al, gl, w0, a_b, norm_w, state, seg: SegBatch, H: in
     out = torch.empty(T, H * D, dtype=r.dtype, device=r.device)
     P = _chunk_portions(r, k, v, wl, al, gl, w0, a_b, norm_w, state, out, seg, H, D, eps, "sigmoid",
                         float(decay_scale), float(key_eps))
-    call("sm_gdelta", DT[r.dtype], r, _ld(r), k, _ld(k), v, _ld(v), wl, _ld(wl), al, _ld(al), gl,
+    call("sm_gdelta", DT[r.dtype], r, _ld(r), k, _ld(k), v, _ld(v), wl, _ld(wl), w2,
+         0 if w2 is None else w2.shape[1], al, _ld(al), gl,
          _ld(gl), w0, a_b, norm_w, state, out, H * D, seg.cu[P:], seg.slot[P:], seg.start[P:],
          seg.S - P, H, D, eps, decay_scale, key_eps)
     return out

@@ -53,7 +53,7 @@ from ..ops.moe import (ClampedGate, dyt_residual_routed, feed_forward, ff_act, m
 from ..ops.norm import (SPLIT, depth_mix_norm, dyt, dyt_residual, embed_rms, gated_rms_norm,
                         group_rms_norm, hyper_mix, hyper_start, parts_rms,
                         project_group_rms, residual_rms, scaled_residual_layer_norm, weight_layer_norm)
-from ..ops.recurrent import delta_scan, head_scan, min_gru_scan, token_shift, wkv_scan
+from ..ops.recurrent import delta_scan, head_scan, min_gru_scan, wkv_scan
 from ..ops.rope import rotary_write, rotate_interleaved_
 from ..ops.segments import SegBatch, portion_keys, whole_prompts, whole_sequences
 from .model_runner import ModelRunner, StepInput, fill_step
@@ -255,9 +255,12 @@ def run_layers(w: HybridWeights, st: HybridState, tokens: torch.Tensor, seg: Seg
     tokens = tokens.long().contiguous()
     x = embed_scaled(tokens, w.embed, 1.0, torch.empty(tokens.shape[0], cfg.hidden_size, dtype=torch.float32,
                                                        device=tokens.device))
+    joined = None                                  # the last sublayer's output, which the next layer's norm joins
     for i, L in enumerate(w.layers):
         m = L.m
-        h = dyt_canon(x, L.norms["norm1"], L.canon, st.tail[i], seg, dt)
+        h = dyt_canon(x, L.norms["norm1"], L.canon, st.tail[i], seg, dt, joined,
+                      (L.w["mu"], st.prev[i]) if L.kind == "wkv" else None)
+        joined = None
         if L.kind == "attention":
             H, G, D = m["heads"], m["kv_heads"], m["dim"]
             qk = project_write_keys(h, L.w["qk"], st.keys[i], seg.cache_slots, H * D)
@@ -265,23 +268,22 @@ def run_layers(w: HybridWeights, st: HybridState, tokens: torch.Tensor, seg: Seg
                                      int(m["mask"]["size"]), eps, sink=True)
         elif L.kind == "wkv":
             H, D = m["heads"], m["dim"]
-            mix = token_shift(h, L.w["mu"], st.prev[i], seg)
+            mix = h                                # (five shifted mixes)
             rkvg = torch.bmm(mix[:4], L.w["rkvg"])
-            wl = project(project_tanh(mix[4], L.w["w1"])[1], L.w["w2"])
+            wl = project_tanh(mix[4], L.w["w1"])[1]
             o = wkv_scan(rkvg[0], rkvg[1], rkvg[2], wl, rkvg[3], L.w["w0"], L.w["u"], L.w["norm"],
-                         st.S[i], seg, H, D, eps)
+                         st.S[i], seg, H, D, eps, L.w["w2"])
         else:
             H, D = m["heads"], m["dim"]
             HD = H * D
             z, wl = project_tanh(h, L.w["in"], 5 * HD)
-            wl = project(wl, L.w["w2"])
             o = delta_scan(z[:, :HD], z[:, HD:2 * HD], z[:, 2 * HD:3 * HD], wl,
                            z[:, 4 * HD:5 * HD], z[:, 3 * HD:4 * HD], L.w["w0"], L.w["a_b"],
-                           L.w["norm"], st.S[i], seg, H, D, eps, DELTA_DECAY, DELTA_KEY_EPS)
+                           L.w["norm"], st.S[i], seg, H, D, eps, DELTA_DECAY, DELTA_KEY_EPS, L.w["w2"])
         y = project(o, L.w["o"])
         f = L.ff
         if f is None:
-            x, _ = dyt_residual(x, y, L.norms["norm1b"], None, dt)
+            joined = (y, L.norms["norm1b"])
         else:
             if f["E"]:
                 # the router in fp32, on the (possibly 16-bit rounded) normed row
@@ -291,7 +293,10 @@ def run_layers(w: HybridWeights, st: HybridState, tokens: torch.Tensor, seg: Seg
             else:
                 x, h2 = dyt_residual(x, y, L.norms["norm1b"], L.norms["norm2"], dt)
                 y2 = feed_forward(h2, f["gu"], f["down"], f["ffs"])
-            x, _ = dyt_residual(x, y2, L.norms["norm2b"], None, dt)
+            joined = (y2, L.norms["norm2b"])
+        if observe is not None or i + 1 == len(w.layers):
+            x, _ = dyt_residual(x, *joined, None, dt)
+            joined = None
         if observe is not None:
             observe(i, x)
     return x

@@ -454,8 +454,9 @@ def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = Non
     one row of a large matrix), the library otherwise."""
     xs = x.shape
     if len(xs) == 2 and xs[0] > THIN_MAX_M:            # (first: short prompts are bound by the host)
-        many = xs[0] * w.shape[0] >= FEW_MIN_MN or w.shape[0] >= FEW_MIN_N
-        if bias is None and (xs[1] >= SPLIT_FEW_K or many) and x.is_cuda:
+        (M, K), N = xs, w.shape[0]
+        many = M * N >= FEW_MIN_MN or N >= FEW_MIN_N
+        if bias is None and (many or K >= SPLIT_MIN_K or K >= SPLIT_FEW_K and M <= SPLIT_FEW_M) and x.is_cuda:
             return mm_nt(x, w)
         ni = tile_ok(x, w) if many and bias is not None and _bias_ok(bias, x, w) else 0
         return tile_linear(x, w, ni, bias) if ni else F.linear(x, w, bias)

@@ -285,7 +285,7 @@ class ModelRunner:
                     and mid_act_ok(y2, L.gate_up, self.w.F):
                 h = self._allreduce(linear_nt(mid_act(y2, L.gate_up, self.w.F), L.down))
                 continue
-            if ml is None and DECODE_SPLIT_MIN == 0 and use_native(y2) and tile_act_ok(y2, L.gate_up, self.w.F):
+            if ml is None and use_native(y2) and tile_act_ok(y2, L.gate_up, self.w.F):
                 h = self._allreduce(linear_nt(tile_act(y2, L.gate_up, self.w.F), L.down))
                 continue
             gu = linear_nt(y2, L.gate_up)

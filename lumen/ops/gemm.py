@@ -397,6 +397,24 @@ def few_tiles(M: int, N: int, K: int) -> int:
     return ni + 128 + apart if ni == 3 and fill >= 0.88 and (apart or K <= 4608) else 0
 
 
+# Short products of prompts: the library takes the host 20 us a call (the tuned table is asked), its kernel 9 - 15, so a step of
+# 257 - 1000 rows of width 1024 - 2048 waits for the host whatever the card does; a tile launch takes the host 8 us and the card
+# no more than 18, one round of 128-row tiles whose walk of k is short.  (Above, and at 256 rows and less, where decode steps
+# replay without the host, the kernel's own time counts: 4010 x 576 x 2048 13.2 us in the library, 17 here.)
+SHORT_MK, SHORT_NIK = 1 << 20, 6144
+
+
+def short_tiles(M: int, N: int, K: int) -> int:
+    """The tiles (as ``few_tiles``) of a product that is over before the host has called the library for the next, or 0."""
+    if M <= 256 or M * K > SHORT_MK or K > 2048 or K < 128 or N < 64:
+        return 0
+    tm = -(-M // 128)
+    for ni in (2, 3, 4, 5):
+        if tm * -(-N // (32 * ni)) <= TILE_CUS:
+            return ni + 64 if ni * K <= SHORT_NIK else 0
+    return 0
+
+
 def _aligned(x: torch.Tensor, w: torch.Tensor, K: int) -> bool:
     (lx, ex), (lw, ew) = x.stride(), w.stride()
     return (ex == 1 and ew == 1 and lx % 8 == 0 and lw % 8 == 0 and K <= lx <= 1 << 22 and K <= lw <= 1 << 22
@@ -404,12 +422,12 @@ def _aligned(x: torch.Tensor, w: torch.Tensor, K: int) -> bool:
 
 
 def tile_ok(x: torch.Tensor, w: torch.Tensor) -> int:
-    """``tile_columns`` or ``few_tiles`` of x @ w^T, 0 where the kernel cannot run it."""
+    """``tile_columns``, ``few_tiles`` or ``short_tiles`` of x @ w^T, 0 where the kernel cannot run it."""
     xs, ws = x.shape, w.shape
     if len(xs) != 2 or len(ws) != 2 or not x.is_cuda:
         return 0
     (M, K), (N, Kw), dt = xs, ws, x.dtype
-    ni = tile_columns(M, N, K) or few_tiles(M, N, K)
+    ni = short_tiles(M, N, K) or tile_columns(M, N, K) or few_tiles(M, N, K)
     if (not ni or K != Kw or K % 64 or N % 4 or K >= 1 << 22 or dt != w.dtype
             or dt not in (torch.bfloat16, torch.float16) or x.device != w.device
             or not _plain(x, w) or not _here(x) or not use_native(x) or not _aligned(x, w, K)):
@@ -430,7 +448,8 @@ def matmul_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         S = split_slices(x, w) if xs[1] >= SPLIT_FEW_K else 0
         if S:
             return split_linear(x, w, S)
-        ni = tile_ok(x, w) if xs[0] * w.shape[0] >= FEW_MIN_MN or w.shape[0] >= FEW_MIN_N else 0
+        ni = (tile_ok(x, w) if xs[0] * w.shape[0] >= FEW_MIN_MN or w.shape[0] >= FEW_MIN_N
+              or xs[0] > 256 and xs[0] * xs[1] <= SHORT_MK else 0)
         if ni:
             return tile_linear(x, w, ni)
     return torch.matmul(x, w.t())
@@ -455,7 +474,7 @@ def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = Non
     xs = x.shape
     if len(xs) == 2 and xs[0] > THIN_MAX_M:            # (first: short prompts are bound by the host)
         (M, K), N = xs, w.shape[0]
-        many = M * N >= FEW_MIN_MN or N >= FEW_MIN_N
+        many = M * N >= FEW_MIN_MN or N >= FEW_MIN_N or M > 256 and M * K <= SHORT_MK
         if bias is None and (many or K >= SPLIT_MIN_K or K >= SPLIT_FEW_K and M <= SPLIT_FEW_M) and x.is_cuda:
             return mm_nt(x, w)
         ni = tile_ok(x, w) if many and bias is not None and _bias_ok(bias, x, w) else 0

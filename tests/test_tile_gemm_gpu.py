@@ -169,3 +169,29 @@ def test_split_route(M, N, K):
     y = native().split_gemm(x, w, code & 15, code >> 4 & 15 or 8, code > 255)
     for out in (gemm.linear_nt(x, w), gemm.project(x, w)):
         assert torch.equal(out, y)
+
+
+def test_short_tiles_rule():
+    for M in (1, 256, 257, 300, 512, 1000, 1024, 1025, 4010):
+        for N in (4, 64, 576, 1024, 2048, 5632, 11264):
+            for K in (64, 128, 1024, 1536, 2048, 2112, 4096):
+                code = gemm.short_tiles(M, N, K)
+                if code:
+                    ni = code & 15
+                    assert code >> 4 == 4 and 2 <= ni <= 5 and ni * K <= 6144 and 256 < M and M * K <= 1 << 20
+                    assert -(-M // 128) * -(-N // (32 * ni)) <= 256
+    assert gemm.short_tiles(300, 576, 2048) == 2 + 64 and gemm.short_tiles(256, 576, 2048) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,bias", [(257, 576, 2048, True), (300, 3072, 1024, False), (1000, 100, 128, True), (480, 2048, 2048, False)])
+def test_short_route(M, N, K, bias):
+    x, w = torch.randn(M, K, device=dev).bfloat16(), torch.randn(N, K, device=dev).bfloat16()
+    b = torch.randn(N, device=dev).bfloat16() if bias else None
+    code = gemm.short_tiles(M, N, K)
+    got = gemm.project(x, w, b)
+    assert code and torch.equal(got, native().tile_gemm(x, w, code & 15, b, None, 4, False))
+    want, tol = bound(x, w, b, torch.bfloat16)
+    assert ((got.double().cpu() - want).abs() <= tol).all()
+    w.requires_grad_()                                      # differentiable: the library's
+    assert gemm.project(x, w, b).requires_grad

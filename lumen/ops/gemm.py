@@ -398,15 +398,18 @@ def few_tiles(M: int, N: int, K: int) -> int:
 
 
 # Short products of prompts: the library takes the host 20 us a call (the tuned table is asked), its kernel 9 - 15, so a step of
-# 257 - 1000 rows of width 1024 - 2048 waits for the host whatever the card does; a tile launch takes the host 8 us and the card
-# no more than 18, one round of 128-row tiles whose walk of k is short.  (Above, and at 256 rows and less, where decode steps
-# replay without the host, the kernel's own time counts: 4010 x 576 x 2048 13.2 us in the library, 17 here.)
-SHORT_MK, SHORT_NIK = 1 << 20, 6144
+# 65 - 1000 rows of width 1024 - 2048 waits for the host whatever the card does; a tile launch takes the host 8 us and the card
+# no more than 18, one round of 128-row tiles whose walk of k is short (from K = 2049 on for the down projections of narrow models).  (Above, the kernel's own time counts: 4010 x 576 x
+# 2048 13.2 us in the library, 17 here.  So it does where a decode step of up to 256 rows is captured, to replay without the host:
+# 128 x 2048 x 2048 9.3 us in the library, 11.2 - 13 here.)
+# Steps of 4 layers, us: Llama, 200 tokens of width 1024 663 -> 445, 100 of width 2048 668 -> 528; dalavik 1159 -> 787, 1148 -> 859; silonex 831 ->
+# 608, 824 -> 694; where the card is nearly the longer one (tazulix, 240 of width 2048) 780 -> 774.
+SHORT_MK, SHORT_NIK, SHORT_MAX_K, SHORT_NK = 1 << 20, 6144, 3072, 1 << 22
 
 
 def short_tiles(M: int, N: int, K: int) -> int:
     """The tiles (as ``few_tiles``) of a product that is over before the host has called the library for the next, or 0."""
-    if M <= 256 or M * K > SHORT_MK or K > 2048 or K < 128 or N < 64:
+    if M <= THIN_MAX_M or M * K > SHORT_MK or K > 2048 and (K > SHORT_MAX_K or N * K > SHORT_NK) or K < 128 or N < 64:
         return 0
     tm = -(-M // 128)
     for ni in (2, 3, 4, 5):
@@ -427,7 +430,11 @@ def tile_ok(x: torch.Tensor, w: torch.Tensor) -> int:
     if len(xs) != 2 or len(ws) != 2 or not x.is_cuda:
         return 0
     (M, K), (N, Kw), dt = xs, ws, x.dtype
-    ni = short_tiles(M, N, K) or tile_columns(M, N, K) or few_tiles(M, N, K)
+    ni = tile_columns(M, N, K) or few_tiles(M, N, K)
+    if not ni:
+        ni = short_tiles(M, N, K)
+        if ni and M <= 256 and torch.cuda.is_current_stream_capturing():
+            return 0
     if (not ni or K != Kw or K % 64 or N % 4 or K >= 1 << 22 or dt != w.dtype
             or dt not in (torch.bfloat16, torch.float16) or x.device != w.device
             or not _plain(x, w) or not _here(x) or not use_native(x) or not _aligned(x, w, K)):
@@ -449,7 +456,7 @@ def matmul_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         if S:
             return split_linear(x, w, S)
         ni = (tile_ok(x, w) if xs[0] * w.shape[0] >= FEW_MIN_MN or w.shape[0] >= FEW_MIN_N
-              or xs[0] > 256 and xs[0] * xs[1] <= SHORT_MK else 0)
+              or xs[1] <= SHORT_MAX_K and THIN_MAX_M < xs[0] and xs[0] * xs[1] <= SHORT_MK else 0)
         if ni:
             return tile_linear(x, w, ni)
     return torch.matmul(x, w.t())
@@ -474,7 +481,7 @@ def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = Non
     xs = x.shape
     if len(xs) == 2 and xs[0] > THIN_MAX_M:            # (first: short prompts are bound by the host)
         (M, K), N = xs, w.shape[0]
-        many = M * N >= FEW_MIN_MN or N >= FEW_MIN_N or M > 256 and M * K <= SHORT_MK
+        many = M * N >= FEW_MIN_MN or N >= FEW_MIN_N or K <= SHORT_MAX_K and M * K <= SHORT_MK
         if bias is None and (many or K >= SPLIT_MIN_K or K >= SPLIT_FEW_K and M <= SPLIT_FEW_M) and x.is_cuda:
             return mm_nt(x, w)
         ni = tile_ok(x, w) if many and bias is not None and _bias_ok(bias, x, w) else 0

@@ -64,7 +64,7 @@ def test_routes():
     x, w = torch.randn(4010, 512, device=dev).bfloat16(), torch.randn(2112, 512, device=dev).bfloat16()
     b = torch.randn(2112, device=dev).bfloat16()
     assert gemm.tile_ok(x, w) == 5
-    for a, c in ((x[:200], w), (x.float(), w.float()), (x.cpu(), w.cpu()), (x, w.t().contiguous().t()), (x.half(), w),
+    for a, c in ((x[:64], w), (x.float(), w.float()), (x.cpu(), w.cpu()), (x, w.t().contiguous().t()), (x.half(), w),
                  (x[:, 1:449], w[:, 1:449]), (x.clone().requires_grad_(), w), (x[:, :500], w[:, :500])):
         assert gemm.tile_ok(a, c) == 0
     want, tol = bound(x, w, b, torch.bfloat16)
@@ -172,19 +172,19 @@ def test_split_route(M, N, K):
 
 
 def test_short_tiles_rule():
-    for M in (1, 256, 257, 300, 512, 1000, 1024, 1025, 4010):
+    for M in (1, 64, 65, 256, 257, 300, 512, 1000, 1024, 1025, 4010):
         for N in (4, 64, 576, 1024, 2048, 5632, 11264):
-            for K in (64, 128, 1024, 1536, 2048, 2112, 4096):
+            for K in (64, 128, 1024, 1536, 2048, 2112, 3072, 4096):
                 code = gemm.short_tiles(M, N, K)
                 if code:
                     ni = code & 15
-                    assert code >> 4 == 4 and 2 <= ni <= 5 and ni * K <= 6144 and 256 < M and M * K <= 1 << 20
+                    assert code >> 4 == 4 and 2 <= ni <= 5 and ni * K <= 6144 and 64 < M and M * K <= 1 << 20
                     assert -(-M // 128) * -(-N // (32 * ni)) <= 256
-    assert gemm.short_tiles(300, 576, 2048) == 2 + 64 and gemm.short_tiles(256, 576, 2048) == 0
+    assert gemm.short_tiles(300, 576, 2048) == 2 + 64 and gemm.short_tiles(64, 576, 2048) == 0
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K,bias", [(257, 576, 2048, True), (300, 3072, 1024, False), (1000, 100, 128, True), (480, 2048, 2048, False)])
+@pytest.mark.parametrize("M,N,K,bias", [(65, 576, 2048, True), (200, 2048, 1024, False), (257, 576, 2048, True), (300, 3072, 1024, False), (1000, 100, 128, True), (480, 2048, 2048, False)])
 def test_short_route(M, N, K, bias):
     x, w = torch.randn(M, K, device=dev).bfloat16(), torch.randn(N, K, device=dev).bfloat16()
     b = torch.randn(N, device=dev).bfloat16() if bias else None

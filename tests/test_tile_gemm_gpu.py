@@ -195,3 +195,26 @@ def test_short_route(M, N, K, bias):
     assert ((got.double().cpu() - want).abs() <= tol).all()
     w.requires_grad_()                                      # differentiable: the library's
     assert gemm.project(x, w, b).requires_grad
+
+
+def test_short_slices_rule():
+    for M in (64, 65, 128, 300, 372, 373, 682, 1000):
+        for N in (4, 1000, 1024, 2048, 3072, 4096):
+            for K in (2048, 3072, 3136, 4224, 5632, 8128, 8192):
+                code = gemm.short_slices(M, N, K)
+                if code:
+                    S = code & 15
+                    assert code >> 4 == 4 and 2 <= S <= K // 64 and 64 < M and M * K <= 1 << 21 and 3072 < K < 8192
+                    assert -(-M // 128) * -(-N // 128) * S <= 256
+    assert gemm.short_slices(300, 2048, 5632) == 5 + 64
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(65, 2048, 5632), (300, 2048, 5632), (400, 1024, 3200)])
+def test_short_slices_route(M, N, K):
+    x, w = torch.randn(M, K, device=dev).bfloat16(), torch.randn(N, K, device=dev).bfloat16()
+    code = gemm.short_slices(M, N, K)
+    want, tol = bound(x, w, None, torch.bfloat16)
+    for got in (gemm.project(x, w), gemm.linear_nt(x, w)):
+        assert code and torch.equal(got, native().split_gemm(x, w, code & 15, 4, False))
+        assert ((got.double().cpu() - want).abs() <= tol).all()

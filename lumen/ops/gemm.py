@@ -803,10 +803,10 @@ def mm_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 
 def linear_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """x [M, K] @ w[N, K]^T -> [M, N]."""
-    M, K = x.shape
-    if FEW_MIN_M <= M <= SPLIT_FEW_M:                  # (before the planned shapes: 128 x 4096 x 11008 39 -> 29 us)
-        S = _slices(x, w) if K >= SPLIT_FEW_K else 0
+    """x [M, K] @ w[N, K]^T -> [M, N]; operands of other dimensions as ``torch.matmul`` takes them."""
+    M = x.shape[0]
+    if x.dim() == 2 and FEW_MIN_M <= M <= SPLIT_FEW_M:     # (before the planned shapes: 128 x 4096 x 11008 39 -> 29 us)
+        S = _slices(x, w) if x.shape[1] >= SPLIT_FEW_K else 0
         if S:
             return split_linear(x, w, S)
         ni = tile_ok(x, w) if w.shape[0] >= FEW_MIN_N else 0

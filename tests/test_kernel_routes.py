@@ -320,3 +320,10 @@ def test_latent_products_of_many_rows_keep_the_library(launched, monkeypatch):
     (True, ((1, 4096, 64, 1), (31, 8192, 64, 0), (32, 8192, 64, 1), (1, 8192, 32, 1)))])
 def test_large_routers_of_few_rows_keep_the_thin_gemm(normed, sizes):
     assert [M._route_rows_pay(T, W, E, normed) for T, W, E, _ in sizes] == [bool(s[3]) for s in sizes]
+
+
+@pytest.mark.parametrize("lead", [(), (2,), (2, 3), (300, 2), (100, 2), (2, 3, 4)])
+def test_products_of_rows_in_any_number_of_dimensions(lead):
+    x, w = torch.randn(*lead, 8), torch.randn(5, 8)
+    for f in (gemm.linear_nt, gemm.matmul_nt, gemm.mm_nt, gemm.project):
+        assert torch.allclose(f(x, w), x @ w.t(), atol=1e-5)

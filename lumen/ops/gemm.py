@@ -8,6 +8,8 @@ contractions, cut along K, run on ``kernels/tile_gemm.hip``.  The rest (and CPU 
 from __future__ import annotations
 
 import os
+import threading
+from contextlib import contextmanager
 from typing import Optional
 
 import torch
@@ -296,10 +298,8 @@ def _slices(x: torch.Tensor, w: torch.Tensor) -> int:
         return 0                                   # (nearly every call: as little host time as can be)
     (M, K), (N, Kw), dt = xs, w.shape, x.dtype
     S = split_plan(M, N, K)
-    if not S:
+    if not S and not (_step.decoded and M <= REPLAY_MAX_M):
         S = short_slices(M, N, K)
-        if S and M <= 256 and torch.cuda.is_current_stream_capturing():
-            return 0
     if (not S or K != Kw or K % 64 or N % 4 or K >= 1 << 22 or dt != w.dtype
             or dt not in (torch.bfloat16, torch.float16) or x.device != w.device
             or not _plain(x, w) or not _here(x) or not use_native(x)):
@@ -404,11 +404,31 @@ def few_tiles(M: int, N: int, K: int) -> int:
 # Short products of prompts: the library takes the host 20 us a call (the tuned table is asked), its kernel 9 - 15, so a step of
 # 65 - 1000 rows of width 1024 - 2048 waits for the host whatever the card does; a tile launch takes the host 8 us and the card
 # no more than 18, one round of 128-row tiles whose walk of k is short (from K = 2049 on for the down projections of narrow models).  (Above, the kernel's own time counts: 4010 x 576 x
-# 2048 13.2 us in the library, 17 here.  So it does where a decode step of up to 256 rows is captured, to replay without the host:
-# 128 x 2048 x 2048 9.3 us in the library, 11.2 - 13 here.)
+# 2048 13.2 us in the library, 17 here.  So it does in a step of decoded rows, which a graph replays without the host:
+# 128 x 2048 x 2048 9.3 us in the library, 11.2 - 13 here: see ``decoded_rows``.)
 # Steps of 4 layers, us: Llama, 200 tokens of width 1024 663 -> 445, 100 of width 2048 668 -> 528; dalavik 1159 -> 787, 1148 -> 859; silonex 831 ->
 # 608, 824 -> 694; where the card is nearly the longer one (tazulix, 240 of width 2048) 780 -> 774.
 SHORT_MK, SHORT_NIK, SHORT_MAX_K, SHORT_NK = 1 << 20, 6144, 3072, 1 << 22
+REPLAY_MAX_M = 256        # the most decoded rows a graph replays
+
+
+class _Step(threading.local):
+    decoded = False
+
+
+_step = _Step()
+
+
+@contextmanager
+def decoded_rows():
+    """Products of this thread belong to a step of decoded rows.  The caller says so for the eager step, the warm-up of a
+    capture and the capture alike, so all of them run the same kernels (and round alike), and the library has seen each
+    of its products before one is captured."""
+    before, _step.decoded = _step.decoded, True
+    try:
+        yield
+    finally:
+        _step.decoded = before
 
 
 def short_tiles(M: int, N: int, K: int) -> int:
@@ -445,10 +465,8 @@ def tile_ok(x: torch.Tensor, w: torch.Tensor) -> int:
         return 0
     (M, K), (N, Kw), dt = xs, ws, x.dtype
     ni = tile_columns(M, N, K) or few_tiles(M, N, K)
-    if not ni:
+    if not ni and not (_step.decoded and M <= REPLAY_MAX_M):
         ni = short_tiles(M, N, K)
-        if ni and M <= 256 and torch.cuda.is_current_stream_capturing():
-            return 0
     if (not ni or K != Kw or K % 64 or N % 4 or K >= 1 << 22 or dt != w.dtype
             or dt not in (torch.bfloat16, torch.float16) or x.device != w.device
             or not _plain(x, w) or not _here(x) or not use_native(x) or not _aligned(x, w, K)):

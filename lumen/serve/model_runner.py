@@ -35,7 +35,7 @@ from ..ops.embedding import embedding
 from ..ops.attention import (flash_attention_fresh, flash_attention_paged, paged_decode,
                              paged_decode_new, paged_decode_new_ok,
                              rope_write_kv)
-from ..ops.gemm import linear_nt, row_norm_linear, row_norm_ok, swiglu_linear_nt
+from ..ops.gemm import decoded_rows, linear_nt, row_norm_linear, row_norm_ok, swiglu_linear_nt
 from ..ops.moe import MID_MAX_M, THIN_ACT_MAX_M, mid_act, mid_act_ok, thin_act, thin_act_ok, tile_act, tile_act_ok
 from ..ops.norm import rms_norm
 from ..ops.rope import rope_tables
@@ -460,7 +460,8 @@ class ModelRunner:
     def decode(self, inp: StepInput) -> torch.Tensor:
         N = inp.tokens.shape[0]
         if not self.use_graphs or N > self.graph_buckets[-1]:
-            return self._decode_input(inp)
+            with decoded_rows():
+                return self._decode_input(inp)
         bucket = next(b for b in self.graph_buckets if b >= N)
         g = self._graphs.get(bucket)
         if g is None:
@@ -511,14 +512,14 @@ class ModelRunner:
         if s is None:
             s = self._warm_stream = torch.cuda.Stream()
         s.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(s):
+        with torch.cuda.stream(s), decoded_rows():
             for _ in range(2):  # warm up (allocator, hipBLASLt heuristics) outside capture
                 self._decode_static(st)
         torch.cuda.current_stream().wait_stream(s)
         graph = torch.cuda.CUDAGraph()
         if self._graph_pool is None:
             self._graph_pool = torch.cuda.graph_pool_handle()
-        with torch.cuda.graph(graph, pool=self._graph_pool):
+        with torch.cuda.graph(graph, pool=self._graph_pool), decoded_rows():
             out = self._decode_static(st)
         self._graphs[bucket] = (graph, st, out)
         return self._graphs[bucket]

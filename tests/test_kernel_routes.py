@@ -1,4 +1,6 @@
 """Which calls the kernels of few rows and of decode steps take, and what happens to the ones they cannot."""
+from contextlib import nullcontext
+
 import pytest
 import torch
 
@@ -327,3 +329,59 @@ def test_products_of_rows_in_any_number_of_dimensions(lead):
     x, w = torch.randn(*lead, 8), torch.randn(5, 8)
     for f in (gemm.linear_nt, gemm.matmul_nt, gemm.mm_nt, gemm.project):
         assert torch.allclose(f(x, w), x @ w.t(), atol=1e-5)
+
+
+def test_decoded_rows_take_the_same_products_eager_warmed_up_and_captured(monkeypatch):
+    """The caller says that a step's rows are decoded; whether the stream is being captured is not asked."""
+    from types import SimpleNamespace
+
+    from lumen.serve.model_runner import ModelRunner
+
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    for name in ("_plain", "_here", "use_native"):
+        monkeypatch.setattr(gemm, name, lambda *a: True)
+    x, w, down = (torch.empty(*s, device="meta", **BF) for s in ((100, 1024), (2048, 1024), (1024, 3200)))
+    long, most = torch.empty(100, 3200, device="meta", **BF), torch.empty(300, 1024, device="meta", **BF)
+    seen = []
+
+    def routes(*a, **k):
+        seen.append((gemm.tile_ok(x, w), gemm.split_slices(long, down), gemm.tile_ok(most, w)))
+
+    for capturing in (False, True):
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+        routes()
+        with gemm.decoded_rows():
+            routes()
+    routes()
+    prompt, decoded = seen[0], seen[1]
+    assert all(prompt) and decoded == (0, 0, prompt[2]) and seen == [prompt, decoded] * 2 + [prompt]
+
+    seen.clear()
+    run = SimpleNamespace(use_graphs=False, _decode_input=routes)
+    ModelRunner.decode(run, SimpleNamespace(tokens=x))
+    within = lambda *a, **k: nullcontext()  # noqa: E731
+    stream = SimpleNamespace(wait_stream=lambda s: None)
+    for name, v in (("stream", within), ("graph", within), ("Stream", lambda: stream), ("current_stream", lambda: stream),
+                    ("CUDAGraph", object), ("graph_pool_handle", object)):
+        monkeypatch.setattr(torch.cuda, name, v)
+    run = SimpleNamespace(_static_inputs=lambda b: {}, _decode_static=routes, _graph_pool=None, _graphs={})
+    ModelRunner._capture(run, 128)
+    assert len(seen) == 4 and set(seen) == {decoded}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M_,N,K", [(100, 2048, 1024), (128, 1024, 3200)])
+def test_captured_products_are_the_warm_ups(M_, N, K):
+    x, w = torch.randn(M_, K, device="cuda").bfloat16(), torch.randn(N, K, device="cuda").bfloat16()
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side), gemm.decoded_rows():
+        want = [f(x, w) for f in (gemm.project, gemm.linear_nt)]
+    torch.cuda.current_stream().wait_stream(side)
+    with torch.cuda.graph(graph), gemm.decoded_rows():
+        got = [f(x, w) for f in (gemm.project, gemm.linear_nt)]
+    for _ in range(3):
+        for y in got:
+            y.zero_()
+        graph.replay()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))

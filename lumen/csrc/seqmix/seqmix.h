@@ -34,6 +34,20 @@ __device__ __forceinline__ float recip_near(float d) {
   return fmaf(fmaf(-d, r, 1.f), r, r);
 }
 __device__ __forceinline__ float sigmoid_near(float x) { return recip_near(1.f + exp_near(-x)); }
+// g / (1 + e^-z) as expf and a division give it, in the half of their instructions: e^-z from the hardware's 2^f, |f| <= 1/2, the
+// quotient from its reciprocal and one remainder.  Largest error in units of the last place (mean square) over 16 M values, |g| up to 88, silu_f -> here:
+// 2.72 (0.441) -> 2.72 (0.442); g sigmoid_f(1.7 g) -> here 2.65 (0.473) -> 2.18 (0.401).  KEEP: NaN z with a g that is none.
+template <bool KEEP>
+__device__ __forceinline__ float logistic_gate(float g, float z) {
+  constexpr float kL = 1.44269502f, kLlo = 1.92596299e-8f;     // log2(e) = kL + kLlo
+  float x = -z;                                                // beyond +-200 as there: e^x is 0 or infinite
+  x = !KEEP ? __builtin_amdgcn_fmed3f(x, -200.f, 200.f) : x < -200.f ? -200.f : x > 200.f ? 200.f : x;
+  const float n = rintf(x * kL), f = fmaf(x, kLlo, fmaf(x, kL, -n));
+  const float e = __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), (int)n);
+  const float d = fmaf(e, 0.25f, 0.25f), r = __builtin_amdgcn_rcpf(d), g4 = 0.25f * g;     // (a quarter: the reciprocal is no denormal)
+  const float q = g4 * r, rest = fmaf(-d, q, g4);
+  return rest == rest ? fmaf(rest, r, q) : q;                  // (no remainder where g or d is infinite)
+}
 // ln x for normal x
 __device__ __forceinline__ float log_near(float x) {
   constexpr float kL = 0.693147182f, kLlo = -1.90465421e-9f;   // ln 2 = kL + kLlo

@@ -416,13 +416,14 @@ def act_rounds(M: int, ff: int) -> tuple:
     return tuple(out)
 
 
-# Which products with a gated activation ``tile_act`` runs (us, product and pass before -> now, bf16): width 2048, ff 5632: 300 rows
-# 33.6 -> 27.7, 1000 52.8 -> 42.3, 4010 179 -> 156, 8000 337 -> 291; 1024, 2816: 512 20.9 -> 16.5, 4010 69 -> 49; 4096, 11008: 256 68 ->
-# 63, 1000 172 -> 159, 4010 574 -> 538.  It needs the more of the tiles' area filled the longer a product is, as the library cuts
-# long products of few tiles along K: over 370 sizes of 130 - 8000 rows and widths 512 - 4096 it is 0.95 - 1.99 times as fast under
-# this rule, 1.22 in the mean (left out: 300 rows, width 4096, filled 0.54, 78 -> 80; 1290 rows, 0.68, 235 -> 248; 220, ff 3000, width 2048, 0.16, 20 -> 25).
+# Which products with a gated activation ``tile_act`` runs (us, product and pass -> here, bf16): width 2048, ff 5632: 300 rows
+# 34.8 -> 26.4, 1000 51.3 -> 42.0, 4010 165 -> 148, 8000 314 -> 291; 1024, 2816: 512 18.4 -> 16.2, 4010 61 -> 48; 4096, 11008: 256 64 ->
+# 62, 1000 164 -> 151, 4010 553 -> 526.  It needs the more of the tiles' area filled the longer a product is, as the library cuts
+# long products of few tiles along K: over 98 sizes of 130 - 8000 rows and widths 512 - 4096 it is 0.90 - 1.76 times as fast under
+# this rule, 1.19 in the mean (worst: 224 rows, ff 4224, width 1536 18.4 -> 20.5, 1290 x 5632 x 2048 72.7 -> 78.0; left out: 300 rows,
+# width 4096, filled 0.54, 78 -> 80; 1290 rows, 0.68, 235 -> 248; 220, ff 3000, width 2048, 0.16, 20 -> 25).
 # Up to 256 rows the product has tiles of 128 rows, and up to 224 walks of k apart, which are worth more than the pass (192 x 5632 x
-# 2048 28.8 here, 23.7 with the pass, 224 x 11008 x 4096 62.9 and 61.0; 256 x 11264 x 4096 61.2 and 65.6).
+# 2048 28.8 here, 23.7 with the pass, 224 x 11008 x 4096 62.9 and 61.0; 256 x 11264 x 4096 60.3 and 63.0).
 ACT_TILE_FILL, ACT_TILE_FILL_MANY = 8192, 6000             # K over the filled share, up to 256 rows and above
 
 

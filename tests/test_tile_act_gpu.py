@@ -52,6 +52,25 @@ def test_tile_act(act, dt):
         assert ((y.double().cpu() - want).abs() <= tol).all(), (M, ff)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("act", ["silu", moe.ClampedGate(8.0, 8.0, 1.0, 1.0)])
+def test_activation_is_rounded_from_full_fp32(act, dt):
+    """Rows of one 1, so gate and up are exact.  The exponential is off by 2 units of 2^-24, the sum, the division and two
+    products and a sum by one each: what lies 8 units and more from the middle of two 16-bit values is rounded to the nearer one."""
+    K, ff = 64, 8192
+    g = torch.Generator().manual_seed(5)
+    x = torch.eye(K, dtype=dt, device=dev)
+    w = torch.cat([torch.rand(ff, K, generator=g) * 18 - 15, torch.randn(ff, K, generator=g) * 4]).to(dt).to(dev)
+    want = reference(x, w, act)
+    near = want.to(dt)
+    step = 2.0 ** torch.frexp(want.abs())[1].double() * torch.finfo(dt).eps / 2       # between neighbours
+    apart = (step / 2 - (near.double() - want).abs()) / want.abs() > 8 * 2.0 ** -24
+    apart &= want.abs() > 2 * torch.finfo(dt).tiny
+    assert apart.double().mean() > 0.8
+    assert (moe.tile_act(x, w, ff, act).cpu()[apart] == near[apart]).all()
+
+
 def test_rounds_cover_the_columns_once():
     for M in (1, 65, 256, 257, 300, 1500, 4010, 8000, 20000, 65536):
         for ff in (8, 104, 1408, 2816, 5632, 11008, 14336):

@@ -145,17 +145,19 @@ def _chunk_portions(r, k, v, wl, al, gl, w0, ub, norm_w, state, out, seg: SegBat
     return P
 
 
-def _low_rank(r, wl, w2, seg: SegBatch) -> tuple:
-    """(wl, None), wl = its low-rank factor times w2^T, or both as they are where the scan forms the product: a step of
-    decoded rows, 16-bit, 16-byte rows of at most 64 ranks."""
+def _low_rank(r, wl, w2, seg: SegBatch, HD: int) -> tuple:
+    """(wl, None), wl = its low-rank factor times w2^T [rank, HD], or both as they are where the scan forms the product: a
+    step of decoded rows, 16-bit, 16-byte rows of at most 64 ranks."""
     from ._seqmix import use_seqmix
     from .gemm import _plain, project
 
     if w2 is None:
         return wl, None
+    if w2.dim() != 2 or wl.dim() != 2 or w2.shape[0] != HD or wl.shape != (r.shape[0], w2.shape[1]):
+        raise ValueError(f"decay of {r.shape[0]} rows x {HD}: factors {tuple(wl.shape)} and {tuple(w2.shape)} do not form it")
     rank = w2.shape[1]
     if (use_seqmix(r) and seg.portions() == (0, 0) and r.dtype in (torch.bfloat16, torch.float16)
-            and wl.dtype == w2.dtype == r.dtype and wl.dim() == 2 and wl.shape[1] == rank and 0 < rank <= 64 and rank % 8 == 0
+            and wl.dtype == w2.dtype == r.dtype and 0 < rank <= 64 and rank % 8 == 0
             and w2.is_contiguous() and wl.stride(1) == 1 and wl.stride(0) % 8 == 0 and wl.stride(0) >= rank
             and (wl.data_ptr() | w2.data_ptr()) % 16 == 0 and w2.device == wl.device == r.device and _plain(r, wl, w2)):
         return wl, w2
@@ -166,7 +168,7 @@ def wkv_scan(r, k, v, wl, g, w0, u, norm_w, state, seg: SegBatch, H: int, D: int
     """The wkv recurrence over a step's segments.  With ``w2`` [H D, rank] ``wl`` is its low-rank factor [T, rank]."""
     from ._seqmix import DT, call, use_seqmix
 
-    wl, w2 = _low_rank(r, wl, w2, seg)
+    wl, w2 = _low_rank(r, wl, w2, seg, H * D)
     if not use_seqmix(r):
         return wkv_scan_ref(r, k, v, wl, g, w0, u, norm_w, state, seg, H, D, eps)
     _check_state(state, H, D)
@@ -184,7 +186,7 @@ def delta_scan(r, k, v, wl, al, gl, w0, a_b, norm_w, state, seg: SegBatch, H: in
     """The delta rule over a step's segments; ``w2`` as in ``wkv_scan``."""
     from ._seqmix import DT, call, use_seqmix
 
-    wl, w2 = _low_rank(r, wl, w2, seg)
+    wl, w2 = _low_rank(r, wl, w2, seg, H * D)
     if not use_seqmix(r):
         return delta_scan_ref(r, k, v, wl, al, gl, w0, a_b, norm_w, state, seg, H, D, eps,
                               decay_scale, key_eps)

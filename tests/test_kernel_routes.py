@@ -385,3 +385,28 @@ def test_captured_products_are_the_warm_ups(M_, N, K):
             y.zero_()
         graph.replay()
         assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("scan", ["wkv", "delta"])
+def test_low_rank_decay_of_another_shape_is_not_read(launched, scan):
+    """The scan reads row c of the second factor for channel c: one with fewer rows would be read past its end."""
+    from lumen.ops import recurrent as R
+    from lumen.ops.segments import SegBatch
+
+    T, H, D = 3, 2, 64
+    i32 = dict(dtype=torch.int32)
+    at = torch.arange(T, **i32)
+    seg = SegBatch(torch.arange(T + 1, **i32), at, at, at, at, None, None)
+    x, w0, state = torch.zeros(T, H * D, **BF), torch.zeros(H * D), torch.zeros(T, H, D, D)
+
+    def run(wl, w2):
+        if scan == "wkv":
+            return R.wkv_scan(x, x, x, wl, x, w0, w0, w0, state, seg, H, D, 1e-5, w2)
+        return R.delta_scan(x, x, x, wl, x, x, w0, w0, w0, state, seg, H, D, 1e-5, 1.0, 1e-5, w2)
+
+    wl, w2 = torch.zeros(T, 16, **BF), torch.zeros(H * D, 16, **BF)
+    for a, b in ((wl, w2[:-1]), (wl, w2[:64]), (wl[:2], w2), (wl[:, :8], w2), (wl, w2.flatten())):
+        with pytest.raises(ValueError):
+            run(a, b)
+    assert not launched
+    assert run(wl, w2).shape == (T, H * D) and len(launched) == 1

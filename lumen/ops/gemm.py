@@ -341,7 +341,8 @@ def tile_columns(M: int, N: int, K: int) -> int:
 # narrowest number of columns that makes the result one round of workgroups.
 #  * Tiles of one column start their walk of k apart where rows of w lie a multiple of 4 KiB apart: in step, all tiles would
 #    read a stage of their rows from the same memory channels (in step / apart: 40 x 24576 45.9 / 38.8, x 2048 26.0 / 21.4, x
-#    6144 71.6 / 57.0; x 3072 30.5 / 31.0).  The library and the thin kernel walk in step, so this is where most is gained.
+#    6144 71.6 / 57.0; x 3072 30.5 / 31.0; columns of a wider matrix go by its rows: 24576 x 2816 of rows of 4096 33.6 / 28.7, x 4096 of rows
+#    of 4224 38.3 / 38.8).  The library and the thin kernel walk in step, so this is where most is gained.
 #    From 257 rows on x costs more than w and is better read in step.
 #  * 17 - 64 rows, from three quarters of a round on (32 columns: nine tenths): 40 x 8192 18.4 -> 16.7, 24576 47.5 -> 38.8, 32000 61 -> 48, 64000 124 -> 98, 32000
 #    x 2048 33.6 -> 27.7, 24576 x 1024 19.4 -> 13.2.  Not less than that (40 x 4096 12.6 -> 15.2).  Long K in step only with 32
@@ -369,8 +370,9 @@ def _round(M: int, N: int, mj: int) -> tuple:
     return ni, tiles / (-(-tiles // TILE_CUS) * TILE_CUS)
 
 
-def few_tiles(M: int, N: int, K: int) -> int:
-    """The tiles on which x [M, K] @ w [N, K]^T should run beside ``tile_columns``: ni + 16 mj + 256 for walks apart, or 0."""
+def few_tiles(M: int, N: int, K: int, ld: Optional[int] = None) -> int:
+    """The tiles on which x [M, K] @ w [N, K]^T should run beside ``tile_columns``: ni + 16 mj + 256 for walks apart, or 0.  ``ld``:
+    elements from one row of w to the next (K)."""
     if M < FEW_MIN_M or K < 1024 or K >= SPLIT_MIN_K:
         return 0
     if M > 256:
@@ -382,7 +384,7 @@ def few_tiles(M: int, N: int, K: int) -> int:
         if tm * -(-N // 160) <= TILE_CUS < tm * -(-N // 128):
             return 5 + 64 if M * N >= 5 * (lead if K <= 2048 else 0.95 * TILE_CUS * 4096) else 0
         return 0
-    apart = 256 if K % 2048 == 0 else 0
+    apart = 256 if (ld or K) % 2048 == 0 else 0
     free = apart or K <= 2048                          # not held up by what the others read
     if M <= 64:
         ni, fill = _round(M, N, 2)
@@ -464,7 +466,7 @@ def tile_ok(x: torch.Tensor, w: torch.Tensor) -> int:
     if len(xs) != 2 or len(ws) != 2 or not x.is_cuda:
         return 0
     (M, K), (N, Kw), dt = xs, ws, x.dtype
-    ni = tile_columns(M, N, K) or few_tiles(M, N, K)
+    ni = tile_columns(M, N, K) or few_tiles(M, N, K, w.stride(0))
     if not ni and not (_step.decoded and M <= REPLAY_MAX_M):
         ni = short_tiles(M, N, K)
     if (not ni or K != Kw or K % 64 or N % 4 or K >= 1 << 22 or dt != w.dtype

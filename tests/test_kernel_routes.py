@@ -410,3 +410,15 @@ def test_low_rank_decay_of_another_shape_is_not_read(launched, scan):
             run(a, b)
     assert not launched
     assert run(wl, w2).shape == (T, H * D) and len(launched) == 1
+
+
+@pytest.mark.parametrize("rows,K,apart", [(4096, 4096, True), (4096, 2048, True), (4096, 1024, True), (2176, 2048, False), (3072, 2048, False),
+                                          (4224, 4096, False), (2048, 1088, True)])
+def test_walks_apart_follow_the_distance_of_rows(monkeypatch, rows, K, apart):
+    """Rows a multiple of 4 KiB apart meet in the same memory channels, however many of their columns are read."""
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    for name in ("_plain", "_here", "use_native"):
+        monkeypatch.setattr(gemm, name, lambda *a: True)
+    x, w = torch.empty(40, K, device="meta", **BF), torch.empty(24576, rows, device="meta", **BF)[:, :K]
+    code = gemm.tile_ok(x, w)
+    assert code and (code > 255) == apart

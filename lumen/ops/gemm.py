@@ -520,14 +520,13 @@ def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = Non
             return mm_nt(x, w)
         ni = tile_ok(x, w) if many and bias is not None and _bias_ok(bias, x, w) else 0
         return tile_linear(x, w, ni, bias) if ni else F.linear(x, w, bias)
-    if len(xs) == 2 and xs[0] >= FEW_MIN_M and w.shape[0] >= FEW_MIN_N:
-        ni = tile_ok(x, w) if bias is None or _bias_ok(bias, x, w) else 0
-        if ni:
-            return tile_linear(x, w, ni, bias)
-    elif len(xs) == 2 and bias is None and xs[0] >= FEW_MIN_M and xs[1] >= SPLIT_FEW_K:
-        S = _slices(x, w)
+    if len(xs) == 2 and xs[0] >= FEW_MIN_M:            # (as in ``linear_nt``)
+        S = _slices(x, w) if bias is None and xs[1] >= SPLIT_FEW_K else 0
         if S:
             return split_linear(x, w, S)
+        ni = tile_ok(x, w) if w.shape[0] >= FEW_MIN_N and (bias is None or _bias_ok(bias, x, w)) else 0
+        if ni:
+            return tile_linear(x, w, ni, bias)
     if thin_ok(x, w) and (bias is None or row_bias_ok(bias, x, w.shape[0]) and _plain(bias)):
         return _thin(x, w, bias)
     if bias is None and len(xs) == 2 and xs[0] == 1 and _plain(x, w) and _here(x) and skinny_ok(x, w):

@@ -422,3 +422,21 @@ def test_walks_apart_follow_the_distance_of_rows(monkeypatch, rows, K, apart):
     x, w = torch.empty(40, K, device="meta", **BF), torch.empty(24576, rows, device="meta", **BF)[:, :K]
     code = gemm.tile_ok(x, w)
     assert code and (code > 255) == apart
+
+
+def test_served_stacks_and_llama_take_the_same_products(monkeypatch):
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    for name in ("_plain", "_here", "use_native", "thin_ok"):
+        monkeypatch.setattr(gemm, name, lambda *a: True)
+    for name in ("split_linear", "tile_linear", "_thin"):
+        monkeypatch.setattr(gemm, name, lambda x, w, *a, name=name: (name, a[0] if a else None))
+    split = 0
+    for M_ in (17, 32, 33, 40, 64):
+        x = {K: torch.empty(M_, K, device="meta", **BF) for K in (1024, 3072, 4096, 5632, 8192, 11008, 16384)}
+        for K in x:
+            for N in (2048, 4096, 5120, 7168, 7680, 8192, 12288, 32000):
+                w = torch.empty(N, K, device="meta", **BF)
+                got, want = gemm.project(x[K], w), gemm.linear_nt(x[K], w)
+                assert got[0] == want[0] and (got[1] or 0) == (want[1] or 0), (M_, N, K)
+                split += got[0] == "split_linear" and N >= gemm.FEW_MIN_N
+    assert split

@@ -162,7 +162,8 @@ def test_split_plan_rule():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(64, 4096, 11008), (33, 5120, 4096), (100, 4096, 5632), (180, 3072, 8448)])
+@pytest.mark.parametrize("M,N,K", [(64, 4096, 11008), (33, 5120, 4096), (100, 4096, 5632), (180, 3072, 8448),
+                                   (64, 8192, 8192)])
 def test_split_route(M, N, K):
     x, w = torch.randn(M, K, device=dev).bfloat16(), torch.randn(N, K, device=dev).bfloat16()
     code = gemm.split_plan(M, N, K)

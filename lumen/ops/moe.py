@@ -436,12 +436,14 @@ def _act_tiles_pay(M: int, ff: int, K: int) -> bool:
     return M * ff * (ACT_TILE_FILL if M <= 256 else ACT_TILE_FILL_MANY) >= K * cells > 0
 
 
-def tile_act_ok(h: torch.Tensor, gu_w: torch.Tensor, ff: int, act="silu", gated: bool = True) -> bool:
-    """Can and should ``tile_act`` run a dense first projection and its activation?"""
+def tile_act_ok(h: torch.Tensor, gu_w: torch.Tensor, ff: int, act="silu", gated: bool = True,
+                rows: Optional[int] = None) -> bool:
+    """Can and should ``tile_act`` run a dense first projection and its activation?  ``rows``: those of the batch that h is a
+    part of, which decide, so that the parts round as the whole does."""
     xs, ws = h.shape, gu_w.shape
-    if len(xs) != 2 or not h.is_cuda or not gated or not MID_MAX_M < xs[0] <= 65536 or len(ws) != 2:
+    if len(xs) != 2 or not h.is_cuda or not gated or not MID_MAX_M < (rows or xs[0]) <= 65536 or len(ws) != 2:
         return False
-    (M, K), dt = xs, h.dtype
+    M, K, dt = rows or xs[0], xs[1], h.dtype
     if M * ff < 512 * K:                           # less than the rule asks of one round (first: short prompts wait for the host)
         return False
     if (ws[0] != 2 * ff or ws[1] != K or K % 64 or K == 0 or ff % 8 or ff == 0 or 4 * ff * K >= 1 << 32 or dt != gu_w.dtype

@@ -245,8 +245,8 @@ class ModelRunner:
         rope_write_kv(qkv, positions, self.w.nh, self.w.nkv, self.cfg.head_dim, self.cos, self.sin,
                       self.k_cache[i], self.v_cache[i], slots)
 
-    def _layers(self, h, positions, slots, attn_fn, lora_ids=None, mark=None, rotate=True):
-        # rotate: turn q and k and write k and v before attn_fn (False: attn_fn does)
+    def _layers(self, h, positions, slots, attn_fn, lora_ids=None, mark=None, rotate=True, rows=None):
+        # rotate: turn q and k and write k and v before attn_fn (False: attn_fn does); rows: of the batch that h is a half of
         cfg = self.cfg
         res = None
         T = h.shape[0]
@@ -276,8 +276,8 @@ class ModelRunner:
             y2, res = rms_norm(a, L.ln2, cfg.rms_norm_eps, res)
             if (T <= THIN_ACT_MAX_M and ml is None and DECODE_SPLIT_MIN == 0 and use_native(y2)
                     and thin_act_ok(y2, None, L.gate_up, 0, 0, self.w.F)):
-                # few decode rows: the activation in the gate|up projection's epilogue (not for the halves
-                # of a split batch, which round the projection like the whole batch does)
+                # few decode rows: the activation in the gate|up projection's epilogue (not where batches are split,
+                # whose halves round the projection like the whole batch does)
                 act = thin_act(y2, L.gate_up, None, 0, 0, self.w.F)
                 h = self._allreduce(linear_nt(act, L.down))
                 continue
@@ -285,7 +285,7 @@ class ModelRunner:
                     and mid_act_ok(y2, L.gate_up, self.w.F):
                 h = self._allreduce(linear_nt(mid_act(y2, L.gate_up, self.w.F), L.down))
                 continue
-            if ml is None and use_native(y2) and tile_act_ok(y2, L.gate_up, self.w.F):
+            if ml is None and use_native(y2) and tile_act_ok(y2, L.gate_up, self.w.F, rows=rows):
                 h = self._allreduce(linear_nt(tile_act(y2, L.gate_up, self.w.F), L.down))
                 continue
             gu = linear_nt(y2, L.gate_up)
@@ -410,17 +410,17 @@ class ModelRunner:
         outs = [None, None]
         a = slice(0, hN)
         outs[0] = self._decode_rows(tokens[a], positions[a], slots[a], block_tables[a],
-                                    context_lens[a], max_context, None, True, mark=first)
+                                    context_lens[a], max_context, None, True, mark=first, rows=N)
         side.wait_event(first)
         with torch.cuda.stream(side):
             b = slice(hN, N)
             outs[1] = self._decode_rows(tokens[b], positions[b], slots[b], block_tables[b],
-                                        context_lens[b], max_context, None, True)
+                                        context_lens[b], max_context, None, True, rows=N)
         cur.wait_stream(side)
         return torch.cat(outs, 0)
 
     def _decode_rows(self, tokens, positions, slots, block_tables, context_lens, max_context,
-                     lora_ids=None, gather: bool = True, mark=None):
+                     lora_ids=None, gather: bool = True, mark=None, rows=None):
         h = embedding(tokens, self.w.embed)
         N = tokens.shape[0]
         nh, D = self.w.nh, self.cfg.head_dim
@@ -436,7 +436,7 @@ class ModelRunner:
             q = qkv[:, :self.q_size].reshape(N, nh, D)
             return paged_decode(q, k, v, block_tables, context_lens, max_context, self.scale, part).view(N, nh * D)
 
-        h, res = self._layers(h, positions, slots, attn, lora_ids, mark=mark, rotate=False)
+        h, res = self._layers(h, positions, slots, attn, lora_ids, mark=mark, rotate=False, rows=rows)
         if N == 1 and row_norm_ok(h, self.w.norm, res, self.w.lm_head):
             logits, _ = row_norm_linear(h, self.w.norm, self.cfg.rms_norm_eps, res, self.w.lm_head)
         else:

@@ -292,3 +292,33 @@ def test_split_decode_two_streams_matches(monkeypatch):
             assert ((a - b).norm() / b.norm()).item() < 1e-2
         same = sum(int(x == y) for a, b in zip(o0, o1) for x, y in zip(a, b))
         assert same >= 0.95 * sum(len(a) for a in o0), (graphs, same)
+
+
+def test_halves_of_a_split_batch_form_the_activation_as_the_whole(monkeypatch):
+    """256 rows take the product with the activation in its epilogue (gate and up unrounded); 128 alone would not."""
+    import lumen.serve.model_runner as mr
+    from lumen.models import build_model
+    from lumen.ops.moe import tile_act_ok
+    from lumen.serve.engine import EngineConfig, LLMEngine
+
+    dev, N = torch.device("cuda", 0), 256
+    m = build_model("small-llama", dtype=torch.bfloat16, device=dev, init="random", seed=4)
+    r = LLMEngine(EngineConfig(model="small-llama", device="cuda", max_model_len=64, block_size=16, num_blocks=N,
+                               use_graphs=False, max_num_seqs=N), model=m.eval()).runner
+    rows, real = [], mr.tile_act
+    monkeypatch.setattr(mr, "tile_act", lambda h, *a: (rows.append(h.shape[0]), real(h, *a))[1])
+    i32 = dict(dtype=torch.int32, device=dev)
+    at = torch.arange(N, device=dev)
+    args = (at % r.cfg.vocab_size, torch.zeros(N, **i32), 16 * at, at.int().view(N, 1), torch.ones(N, **i32), 16)
+    w = r.w.layers[0].gate_up
+    assert not tile_act_ok(torch.empty(N // 2, w.shape[1], device=dev, dtype=w.dtype), w, r.w.F)
+    with torch.no_grad():
+        whole = r._decode_eager(*args).float()
+        layers = len(r.w.layers)
+        assert rows == [N] * layers
+        monkeypatch.setattr(mr, "DECODE_SPLIT_MIN", 32)
+        rows.clear()
+        halves = r._decode_eager(*args).float()
+        torch.cuda.synchronize()
+    assert rows == [N // 2] * (2 * layers)
+    assert ((halves - whole).norm() / whole.norm()).item() < 1e-2

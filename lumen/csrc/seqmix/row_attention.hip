@@ -377,6 +377,15 @@ row_attn_kernel(const RowAttnArgs<T> a) {
                         : to_f32(a.q2[(long long)t * a.q2r + (long long)h * a.q2h + (d - a.D1)]);
     }
   }
+  const TileWalk walk(pos, a.window, a.keep);
+  if ((int)blockIdx.z >= walk.count && a.nsplit > 1 && a.sigb == nullptr) {      // no tile: row_attn_combine reads no values
+    if ((int)threadIdx.x < nh) {
+      const long long slot = ((long long)t * a.H + h0 + threadIdx.x) * a.nsplit + blockIdx.z;
+      a.ws_ml[2 * slot] = -INFINITY;
+      a.ws_ml[2 * slot + 1] = -1.f;
+    }
+    return;
+  }
   float temp = 1.f;
   if (a.tevery > 0 && a.tcoef != 0.f)
     temp = 1.f + a.tcoef * logf((float)((pos + 1) / a.tevery) + 1.f);
@@ -407,7 +416,6 @@ row_attn_kernel(const RowAttnArgs<T> a) {
   __syncthreads();
 
   int buf = 0;
-  const TileWalk walk(pos, a.window, a.keep);
   for (int tv = blockIdx.z; tv < walk.count; tv += a.nsplit, buf ^= 1) {
     const int j0 = walk.key0(tv);
     const int j = j0 + lane;
@@ -887,8 +895,8 @@ hipError_t launch_latent_attn<float>(const RowAttnArgs<float>&, const float*, in
 }
 
 // out[t, h] = sum_s acc_s exp(m_s - M) / sum_s l_s exp(m_s - M), M = max_s m_s: the splits of a
-// row's keys merged; a split that saw no key has (m, l) = (-inf, 0) and drops out.  With a gate
-// the head's output is multiplied by sigmoid(gate[t, h]).
+// row's keys merged; a split that saw no key has (m, l) = (-inf, 0) and drops out, the last ones that had no tile
+// (-inf, -1) and no values at all.  With a gate the head's output is multiplied by sigmoid(gate[t, h]).
 template <typename T>
 __global__ void __launch_bounds__(256)
 row_attn_combine_kernel(const float* __restrict__ ws_ml, const float* __restrict__ ws_o,
@@ -897,9 +905,12 @@ row_attn_combine_kernel(const float* __restrict__ ws_ml, const float* __restrict
   const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63;
   const long long base = ((long long)t * H + h) * nsplit;
   __shared__ float s_w[64];
+  __shared__ int s_n;
   if (threadIdx.x < 64) {                                // nsplit <= 64: lane s weighs split s
     const float ms = lane < nsplit ? ws_ml[2 * (base + lane)] : -INFINITY;
     const float ls = lane < nsplit ? ws_ml[2 * (base + lane) + 1] : 0.f;
+    const int n = __popcll(__ballot(lane < nsplit && !(ls < 0.f)));
+    if (lane == 0) s_n = n;
     const float M = wave_max(ms);
     const float e = ms == -INFINITY ? 0.f : expf(ms - M);
     float L = wave_sum(ls * e);
@@ -908,9 +919,10 @@ row_attn_combine_kernel(const float* __restrict__ ws_ml, const float* __restrict
   }
   __syncthreads();
   T* op = out + (long long)t * our + (long long)h * ouh;
+  const int n = s_n;
   for (int d = threadIdx.x; d < Dv; d += 256) {
     float o = 0.f;
-    for (int s = 0; s < nsplit; ++s) o += ws_o[(base + s) * Dv + d] * s_w[s];
+    for (int s = 0; s < n; ++s) o += ws_o[(base + s) * Dv + d] * s_w[s];
     op[d] = from_f32<T>(o);
   }
 }

@@ -1229,12 +1229,15 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
         tiles = min(tiles, (window + 63) // 64 + 1 + (keep_first + 63) // 64)
     # fewer heads per workgroup: more workgroups, and a shorter chain in each.  Tables of a server's longest context count
     # many tiles whatever the rows hold, so few rows are told by their blocks (us, 16 heads of 128 over 4, 8 rows, 16 heads
-    # a workgroup -> 4: 250 tokens 27 -> 14, 4000 45 -> 37; 16 rows -> 8: 250 30 -> 20, 1000 31 -> 23, 4000 50 -> 52; 64 rows of
+    # a workgroup -> 4: 250 tokens 26 -> 12, 4000 52 -> 34; 16 rows -> 8: 250 30 -> 18, 1000 30 -> 22, 4000 58 -> 46; 64 rows of
     # 4000 would go 152 -> 179)
     while talk is None and HB > 4 and (T * ((H + HB - 1) // HB) * tiles < 512 or 2 * T * ((H + HB - 1) // HB) <= 32):
         HB //= 2
     blocks = T * ((H + HB - 1) // HB)
-    nsplit = max(1, min(tiles, 32, 512 // max(blocks, 1)))
+    # up to 32 blocks of few heads: 32 splits, as long rows would else pay for the halved heads with longer chains (16 rows of 4000,
+    # 16 / 32 splits: 62 / 46; 8 heads over 2 46 / 34, where one block a row took 38; splits past a row's last tile cost 0 - 0.2).
+    # Of 16 heads fewer workgroups fit a CU: 32 rows of 4000 77 / 81.
+    nsplit = max(1, min(tiles, 32, (1024 if talk is None and HB <= 8 and blocks <= 32 else 512) // max(blocks, 1)))
     ws_ml = ws_o = None
     if nsplit > 1:
         ws_ml = torch.empty(T * H * nsplit * 2, dtype=torch.float32, device=q1.device)

@@ -440,3 +440,19 @@ def test_served_stacks_and_llama_take_the_same_products(monkeypatch):
                 assert got[0] == want[0] and (got[1] or 0) == (want[1] or 0), (M_, N, K)
                 split += got[0] == "split_linear" and N >= gemm.FEW_MIN_N
     assert split
+
+
+@pytest.mark.parametrize("T,H,heads,splits", [(16, 8, 4, 32), (16, 16, 8, 32), (8, 16, 4, 32), (14, 16, 8, 32), (1, 16, 4, 32), (32, 16, 16, 16),
+                                              (64, 16, 16, 8), (64, 8, 8, 8)])
+def test_halved_heads_of_few_rows_keep_as_many_splits(launched, T, H, heads, splits):
+    """Behind a server's tables: rows of 4000 tokens on half the heads and half the splits took longer than before either."""
+    from lumen.ops.attention import row_attention
+    from lumen.ops.segments import SegBatch
+
+    i32 = dict(dtype=torch.int32)
+    at = torch.arange(T, **i32)
+    seg = SegBatch(torch.arange(T + 1, **i32), at, at, at, at, torch.zeros(T, 256, **i32), None)
+    q, kv = torch.zeros(T, H, 128, **BF), torch.zeros(1, 16, H, 128, **BF)
+    row_attention(q, None, kv, kv.clone(), 128, torch.zeros(T, H, 128, **BF), seg, H, H, 0.1)
+    (name, a), = launched
+    assert name == "sm_row_attn" and a[-3] == splits and a[24] == heads

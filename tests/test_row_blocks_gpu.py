@@ -50,6 +50,33 @@ def test_few_rows(T, H, G, dt):
         close(out[t], want, vv.abs().max(), dt)
 
 
+@pytest.mark.parametrize("sink,window", [(False, 0), (True, 0), (False, 100), (True, 200)])
+@pytest.mark.parametrize("T,H,G", [(16, 8, 2), (1, 16, 4), (5, 4, 4)])
+def test_splits_past_a_rows_last_tile_are_not_read(T, H, G, sink, window):
+    """32 splits for rows of 1 - 30 tiles, in memory that held NaN."""
+    g = torch.Generator().manual_seed(T + window)
+    ctx = [(1, 64, 65, 1900, 128, 129, 700, 640)[t % 8] for t in range(T)]
+    seg, nb, tables = step(ctx, g)
+    dt = torch.bfloat16
+    q, k, v = (torch.randn(*s, generator=g).to(dt) for s in ((T, H, 128), (nb, 16, G, 128), (nb, 16, G, 128)))
+    s = torch.randn(H, generator=g)
+    out = torch.empty(T, H, 128, dtype=dt, device=dev)
+    qd, kd, vd, sd = q.to(dev), k.to(dev), v.to(dev), s.to(dev)
+    for n in (T * H * 32 * 2, T * H * 32 * 128):
+        torch.full((n,), float("nan"), device=dev)         # freed at once: the workspaces lie here
+    row_attention(qd, None, kd, vd, 128, out, seg, H, G, 0.088, sink=sd if sink else None, window=window)
+    for t, n in enumerate(ctx):
+        at = torch.arange(max(0, n - window) if window else 0, n)
+        rows = tables[t].long()[at // 16] * 16 + at % 16
+        kk, vv = k.view(-1, G, 128)[rows].double(), v.view(-1, G, 128)[rows].double()
+        want = []
+        for h in range(H):
+            z = 0.088 * (kk[:, h * G // H] @ q[t, h].double())
+            z = torch.cat([z, s[h:h + 1].double()]) if sink else z
+            want.append(torch.softmax(z, 0)[:len(at)] @ vv[:, h * G // H])
+        close(out[t], torch.stack(want), vv.abs().max(), dt)
+
+
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("T,H,R,D2", [(1, 16, 512, 64), (9, 16, 256, 32), (600, 3, 256, 32), (5, 20, 384, 64), (7, 4, 512, 8),
                                       (6, 16, 192, 64), (600, 2, 64, 0)])

@@ -574,10 +574,11 @@ def project_write_keys(x: torch.Tensor, w: torch.Tensor, cache: torch.Tensor, sl
     return y
 
 
-# Decode batches 5..256: the decode-batch MFMA GEMM (kernels/decode_gemm.hip) where the measured
-# plan table (configs/kernels/decode_gemm_plans.json, written by lumen/bench/decode_gemm_probe.py) has
-# a winning (BM, BN, split-K) for the shape, hipBLASLt with the tuned table otherwise.  (Two
-# earlier hand-written attempts lost, scripts/probes/: 32-row M tiles, and all-M-rows tiles over
+# Decode batches 5..256 that neither the few-row nor the tiled kernels take: the decode-batch MFMA GEMM
+# (kernels/decode_gemm.hip) where the measured plan table (configs/kernels/decode_gemm_plans.json or LUMEN_DGEMM_PLANS, written
+# by lumen/bench/decode_gemm_probe.py) has a (BM, BN, split-K) that beats the library's kernel, hipBLASLt with the tuned table
+# otherwise (256 x 5120 x 5120: 51.2 -> 37.5 us; at the other shapes of Llama-2-7B and -13B the tiled kernels are 1.05 - 1.3 times as
+# fast as its best form, or the library is).  (Two earlier hand-written attempts lost, scripts/probes/: 32-row M tiles, and all-M-rows tiles over
 # all of K whose every workgroup pulled the whole x through its CU's load path.)
 DG_BMS = (64, 128, 192, 256)
 DG_BNS = {256: (64, 96, 128, 160), 192: (64, 96, 128), 128: (64, 96, 128, 192, 256),
@@ -824,7 +825,7 @@ def mm_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 def linear_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x [M, K] @ w[N, K]^T -> [M, N]; operands of other dimensions as ``torch.matmul`` takes them."""
     M = x.shape[0]
-    if x.dim() == 2 and FEW_MIN_M <= M <= SPLIT_FEW_M:     # (before the planned shapes: 128 x 4096 x 11008 39 -> 29 us)
+    if x.dim() == 2 and FEW_MIN_M <= M <= SPLIT_FEW_M:     # (before the planned shapes: 128 x 4096 x 11008 38 -> 28 us)
         S = _slices(x, w) if x.shape[1] >= SPLIT_FEW_K else 0
         if S:
             return split_linear(x, w, S)

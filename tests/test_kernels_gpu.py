@@ -933,17 +933,33 @@ def test_decode_gemm_variants(bm):
 
 
 @pytest.mark.parametrize("N,K", [(12288, 4096), (4096, 4096), (22016, 4096), (4096, 11008),
-                                 (32000, 4096)])
+                                 (32000, 4096), (5120, 5120)])
 @pytest.mark.parametrize("M", [64, 100, 200, 256])
 def test_decode_gemm_planned_shapes(N, K, M):
-    """linear_nt on the serving shapes of Llama-2-7B: the planned decode GEMM (or hipBLASLt where
-    the plan table has no win) matches an f32 matmul."""
-    from lumen.ops.gemm import dg_plan, linear_nt
+    """linear_nt on the serving shapes of Llama-2-7B and -13B: the planned decode GEMM (or the few-row and
+    tiled kernels or hipBLASLt where the plan table has no win) matches an f32 matmul; a plan of the
+    table is also run as such."""
+    from lumen.ops.gemm import decode_gemm, dg_plan, linear_nt
 
     x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
     w = (torch.randn(N, K, device=DEV) * 0.02).to(torch.bfloat16)
-    y = linear_nt(x, w)
-    assert rel(y, x.float() @ w.float().t()) < 1e-2, dg_plan(x, w)
+    y, plan = linear_nt(x, w), dg_plan(x, w)
+    assert rel(y, x.float() @ w.float().t()) < 1e-2, plan
+    if plan is not None:
+        assert rel(decode_gemm(x, w, *plan), x.float() @ w.float().t()) < 1e-2, plan
+    assert (plan is not None) == ((N, K) == (5120, 5120) and M > 192)
+
+
+def test_every_plan_of_the_table_is_one_that_linear_nt_runs():
+    from lumen.ops import gemm
+
+    for (N, K, bm), p in gemm.dg_plans().items():
+        x = torch.randn(bm, K, device=DEV).to(torch.bfloat16)
+        w = (torch.randn(N, K, device=DEV) * 0.02).to(torch.bfloat16)
+        assert gemm.dg_plan(x, w) == (bm,) + p
+        y = gemm.decode_gemm(x, w, bm, *p)
+        with gemm.decoded_rows():
+            assert torch.equal(gemm.linear_nt(x, w), y)
 
 
 @pytest.mark.parametrize("N,F", [(4096, 11008), (1024, 2752)])

@@ -73,13 +73,19 @@ def test_activation_is_rounded_from_full_fp32(act, dt):
 
 def test_rounds_cover_the_columns_once():
     for M in (1, 65, 256, 257, 300, 1500, 4010, 8000, 20000, 65536):
-        for ff in (8, 104, 1408, 2816, 5632, 11008, 14336):
-            at = 0
-            for c0, c1, ni in moe.act_rounds(M, ff):
-                assert c0 == at < c1 and c0 % 8 == 0 and ni in (4, 6, 8)
-                assert ni == 8 and c0 == 0 and c1 < ff or -(-M // 256) * -(-(c1 - c0) // (16 * ni)) <= 256 or c1 % 128 == 0
+        tm = -(-M // 256)
+        for ff in (8, 104, 1408, 2816, 5632, 5640, 11000, 11008, 14336):
+            at, rounds = 0, moe.act_rounds(M, ff)
+            for k, (c0, c1, ni) in enumerate(rounds):
+                assert c0 == at < c1 and c0 % 8 == 0
+                whole = 256 // tm * 128                                  # columns of a whole round of 128-column tiles
+                if (c1 - c0) % whole == 0:
+                    assert ni == 8 and k == 0
+                else:                                                    # the rest: one round, of the narrowest tiles that make it one
+                    fits = [n for n in (4, 6, 8) if tm * -(-(c1 - c0) // (16 * n)) <= 256]
+                    assert c1 == ff and ni == fits[0]
                 at = c1
-            assert at == ff
+            assert at == ff and len(rounds) <= 2
     assert moe.act_rounds(70000, 5632) == () and not moe._act_tiles_pay(70000, 5632, 2048)
     assert moe._act_tiles_pay(4010, 5632, 2048) and not moe._act_tiles_pay(300, 11264, 4096)
 

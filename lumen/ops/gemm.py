@@ -249,8 +249,12 @@ def row_stream_linear(x: torch.Tensor, y: Optional[torch.Tensor], norm_w: torch.
 #    33.6 -> 21.7, 72 x 4096 x 4096 22.1 -> 17.9, 100 x 8192 x 4096 25.1 -> 23.9; but 2048 x 5632 13.9 -> 16.4, 3072 x 4096 14.5 -> 16.4.
 #  * 129 - 240 rows: 180 x 4096 x 11008 44.4 -> 34.6, 180 x 3072 x 5632 26.8 -> 21.3, 224 x 6144 x 4096 38.7 -> 27.9; 180 x 6144 x 4096 even.
 # Over 128 tiles a slice would be less than half of K on more workgroups than CUs; under 128 workgroups most CUs idle.
-# Walks apart (few_tiles) for up to 256 rows of 4096 columns and more: 64 x 8192 x 8192 40.0 -> 33.1, 4096 x 11008 26.7 -> 25.4, worst
-# 4096 x 8192 21.3 -> 22.3.
+# Walks apart (as in few_tiles) for up to 256 rows of 4096 columns and more.  Slices already start at different k, and which K
+# still meet in the same channels was not to be told from the rows' distance (us, in step / apart: 64 x 8192 x 8192 40.1 / 33.2, 64 x 6144 x 11008
+# 39.4 / 32.3, but x 11264 32.7 / 33.3, 256 x 6144 x 14336 57.0 / 60.1, x 4096 x 8192 31.1 / 33.1): over 280 sizes of K 3072 - 14336 apart is
+# 0.94 - 1.22 times as fast, 1.016 in the mean, and under 4096 columns even but for K = 11008 (80 sizes, 1.018).
+# Between the sizes above: 255 drawn ones of 17 - 256 rows, K 3072 - 14400 1.34 times as fast as the better of the thin kernel and the library
+# in the mean, three of them below 0.97 (worst 66 x 4512 x 4096 16.6 -> 19.6).
 SPLIT_MIN_K, SPLIT_FEW_K, SPLIT_MAX_S, SPLIT_FEW_M = 8192, 3072, 8, 240
 
 
@@ -274,9 +278,8 @@ def split_plan(M: int, N: int, K: int) -> int:
             pays = K >= 4096 and (wide or N == 4096) or K >= 5632 and 3072 <= N < FEW_MIN_N
         if not pays:
             return 0
-    mj = 2 if M <= 64 else 4 if M <= 128 or N <= (5376 if M <= 192 else 2048 if K >= SPLIT_MIN_K or M > SPLIT_FEW_M else 4096) else 8
-    if M > SPLIT_FEW_M:
-        mj = 8
+    mj = (8 if M > SPLIT_FEW_M else 2 if M <= 64 else
+          4 if M <= 128 or N <= (5376 if M <= 192 else 2048 if K >= SPLIT_MIN_K else 4096) else 8)
     tiles = -(-M // (32 * mj)) * -(-N // 128)
     if not 0 < tiles <= 128:
         return 0
@@ -356,6 +359,8 @@ def tile_columns(M: int, N: int, K: int) -> int:
 #    130 - 160 rows the second row tile is mostly padding (161 x 24576 x 1024 19.8 -> 21.8).
 #  * above: 1000 x 3072 32.3 -> 29.0, 500 x 5120 38.1 -> 34.6, 1000 x 5120 50.3 -> 46.3, x 1024 19.2 -> 15.8; long K even (512 x 5120 x
 #    5632 49.1 -> 49.5), other widths are the library's (512 x 8192 41.7 -> 42.8, 768 x 6144 x 2816 33.9 -> 34.2).
+# Between the sizes above: 245 drawn ones of 17 - 256 rows, 7168 - 66000 columns and K 1024 - 8128 1.14 times as fast as the better of the thin
+# kernel and the library in the mean, one of them below 0.97 (250 x 12048 x 7936 71.9 -> 75.8).
 FEW_MIN_M, FEW_MIN_N, FEW_MIN_MN = 17, 7168, 1 << 21
 FEW_NI = {2: (1, 2, 3, 4, 5, 6, 8), 4: (2, 3, 4, 5, 6, 8), 8: (3, 4, 5, 6)}
 
@@ -403,8 +408,8 @@ def few_tiles(M: int, N: int, K: int, ld: Optional[int] = None) -> int:
     return ni + 128 + apart if ni == 3 and fill >= 0.88 and (apart or K <= 4608) else 0
 
 
-# Short products of prompts: the library takes the host 20 us a call (the tuned table is asked), its kernel 9 - 15, so a step of
-# 65 - 1000 rows of width 1024 - 2048 waits for the host whatever the card does; a tile launch takes the host 8 us and the card
+# Short products of prompts: the library takes the host 18 us a call (19 - 21 with a tuned table, which is asked), its kernel 5 - 17, so a
+# step of 65 - 1000 rows of width 1024 - 2048 waits for the host whatever the card does; a tile launch takes the host 8 us and the card
 # no more than 18, one round of 128-row tiles whose walk of k is short (from K = 2049 on for the down projections of narrow models).  (Above, the kernel's own time counts: 4010 x 576 x
 # 2048 13.2 us in the library, 17 here.  So it does in a step of decoded rows, which a graph replays without the host:
 # 128 x 2048 x 2048 9.3 us in the library, 11.2 - 13 here: see ``decoded_rows``.)

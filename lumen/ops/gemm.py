@@ -471,7 +471,7 @@ def tile_ok(x: torch.Tensor, w: torch.Tensor) -> int:
     if len(xs) != 2 or len(ws) != 2 or not x.is_cuda:
         return 0
     (M, K), (N, Kw), dt = xs, ws, x.dtype
-    ni = tile_columns(M, N, K) or few_tiles(M, N, K, w.stride(0))
+    ni = tile_columns(M, N, K) or (few_tiles(M, N, K, w.stride(0)) if M > 256 or N >= FEW_MIN_N else 0)
     if not ni and not (_step.decoded and M <= REPLAY_MAX_M):
         ni = short_tiles(M, N, K)
     if (not ni or K != Kw or K % 64 or N % 4 or K >= 1 << 22 or dt != w.dtype

@@ -958,8 +958,15 @@ def test_every_plan_of_the_table_is_one_that_linear_nt_runs():
         w = (torch.randn(N, K, device=DEV) * 0.02).to(torch.bfloat16)
         assert gemm.dg_plan(x, w) == (bm,) + p
         y = gemm.decode_gemm(x, w, bm, *p)
+        graph = torch.cuda.CUDAGraph()
         with gemm.decoded_rows():
             assert torch.equal(gemm.linear_nt(x, w), y)
+            with torch.cuda.graph(graph):
+                out = gemm.linear_nt(x, w)
+        for _ in range(3):                             # (the tile counters are left at zero)
+            out.zero_()
+            graph.replay()
+            assert torch.equal(out, y) and torch.equal(gemm.linear_nt(x, w), y)
 
 
 @pytest.mark.parametrize("N,F", [(4096, 11008), (1024, 2752)])

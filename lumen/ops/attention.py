@@ -1238,6 +1238,11 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
     # 16 / 32 splits: 62 / 46; 8 heads over 2 46 / 34, where one block a row took 38; splits past a row's last tile cost 0 - 0.2).
     # Of 16 heads fewer workgroups fit a CU: 32 rows of 4000 77 / 81.
     nsplit = max(1, min(tiles, 32, (1024 if talk is None and HB <= 8 and blocks <= 32 else 512) // max(blocks, 1)))
+    # step_attention.hip (its conditions are the launcher's): a workgroup serves a row and key head, or all heads of a row when
+    # they are mixed.  Workgroups of 3 and 2 a CU: half or twice as many splits are 2 - 20 % slower at 16 - 64 rows, and even below.
+    if (D1 == Dv == 128 and q2 is None and H // G in (2, 4, 8) and v_div == 1 and sigmoid_bias is None
+            and krow == vrow == G * 128 and q1.dtype != torch.float32):
+        nsplit = max(1, min(tiles, 64, 1024 // (T * G) if talk is None else 512 // T))
     ws_ml = ws_o = None
     if nsplit > 1:
         ws_ml = torch.empty(T * H * nsplit * 2, dtype=torch.float32, device=q1.device)

@@ -1,0 +1,55 @@
+"""Attention of decoded rows with heads of 128 (step_attention.hip) with every score shaping it takes, against the torch reference in
+fp32, at the edges of its groups of 16 keys and tiles of 64, in caches whose other rows hold NaN."""
+import pytest
+import torch
+
+from lumen.ops.attention import row_attention, row_attention_ref
+from lumen.ops.segments import SegBatch
+
+pytestmark = pytest.mark.gpu
+CTX = (1, 15, 16, 17, 63, 64, 65, 127, 129, 300, 700)
+
+
+def step(ctx, bs, g, device="cpu"):
+    need = [-(-c // bs) for c in ctx]
+    free = torch.randperm(sum(need) + 2, generator=g).tolist()
+    tables = torch.zeros(len(ctx), max(need) + 3, dtype=torch.int32)
+    for t, n in enumerate(need):
+        tables[t, :n] = torch.tensor([free.pop() for _ in range(n)], dtype=torch.int32)
+    i32 = dict(dtype=torch.int32)
+    seq, pos = torch.arange(len(ctx), **i32), torch.tensor(ctx, **i32) - 1
+    return SegBatch(torch.arange(len(ctx) + 1, **i32), seq, pos, seq, pos, tables, None), sum(need) + 2
+
+
+def on_gpu(seg):
+    c = lambda x: None if x is None else x.cuda()  # noqa: E731
+    return SegBatch(c(seg.cu), c(seg.slot), c(seg.start), c(seg.row_seg), c(seg.positions), c(seg.tables), None)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kind", ["plain", "cap_window", "bias_sink_gate", "slopes_keep", "talk", "talk_window"])
+@pytest.mark.parametrize("T,H,G,bs", [(11, 16, 4, 16), (1, 8, 2, 16), (11, 12, 6, 32), (11, 16, 2, 8), (3, 32, 8, 16), (300, 4, 2, 16)])
+def test_shapings(T, H, G, bs, kind, dt):
+    g = torch.Generator().manual_seed(H + T)
+    ctx = [CTX[(t + (5 if T == 1 else 0)) % len(CTX)] if T < 100 else 1 + t % 70 for t in range(T)]
+    seg, nb = step(ctx, bs, g)
+    k, v = (torch.full((nb * bs, G, 128), float("nan")).to(dt) for _ in range(2))
+    for t, n in enumerate(ctx):
+        rows = seg.tables[t].long()[torch.arange(n) // bs] * bs + torch.arange(n) % bs
+        k[rows], v[rows] = (torch.randn(n, G, 128, generator=g).to(dt) for _ in range(2))
+    k, v = k.view(nb, bs, G, 128), v.view(nb, bs, G, 128)
+    q = torch.randn(T, H * 128 + 24, generator=g).to(dt)[:, :H * 128]            # rows of a wider projection
+    rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    kw = {"plain": {}, "cap_window": dict(softcap=3.0, window=100),
+          "bias_sink_gate": dict(r1=rnd(H).abs(), r2=rnd(H).abs(), sink=rnd(H), gate=rnd(T, H).to(dt), q_temp=(0.4, 32)),
+          "slopes_keep": dict(slopes=0.02 * rnd(H).abs(), window=70, keep_first=5),
+          "talk": dict(softcap=5.0, r1=rnd(H).abs(), r2=rnd(H).abs(), sink=rnd(H), q_temp=(0.4, 32), talk=torch.eye(H) + 0.2 * rnd(H, H)),
+          "talk_window": dict(talk=torch.eye(H) + 0.2 * rnd(H, H), window=90, keep_first=3)}[kind]
+    want = row_attention_ref(q.view(T, H, 128), None, k, v, 128, torch.empty(T, H, 128), seg, H, G, 0.088, **kw)
+    out = torch.empty(T, H, 128, dtype=dt, device="cuda")
+    kw = {n: x.cuda() if torch.is_tensor(x) else x for n, x in kw.items()}
+    row_attention(q.cuda().view(T, H, 128), None, k.cuda(), v.cuda(), 128, out, on_gpu(seg), H, G, 0.088, **kw)
+    # one rounding of the result; scores of size <= 32, mixed by rows of 1-norm <= 8, to a few units of fp32's last place in weights
+    # and sums over values of size <= 5 (a score's error of 8 x 32 x 2^-23 x 16 is one of 2^-11 in its weight at the most)
+    tol = want.abs() * torch.finfo(dt).eps / 2 + 5.0 * (2.0 ** -11 if "talk" in kind else 2.0 ** -14)
+    assert ((out.float().cpu() - want).abs() <= tol).all()

@@ -11,7 +11,8 @@
 //                    o[h] = uv[h] ol[h].  A workgroup takes 16 rows of a head; a wave asks for its 16 output columns'
 //                    weights (all of R), joins in the sums, which meet in LDS, and multiplies.
 // Bound by latency.  64 rows x 16 heads, D = 128, R = 512, in a decode step, us: write and norm 10.1 + 4.5 -> 6.2; batched
-// library product and rotation 5.1 + 4.5 -> 7.0; sums of 8 splits and library product 4.9 + 12.7 -> 10.9.
+// library product and rotation 5.1 + 4.5 -> 7.0; sums of 8 splits and library product 4.9 + 12.7 -> 6.5 (10.9 with
+// 16 rows a workgroup and sums of splits without keys).
 #include "mma.h"
 
 using namespace lumen;
@@ -123,7 +124,7 @@ template <typename T> struct OutArgs {
   const T* gate; long long gater;
   const T* uv;                              // [H][Dv][R]
   T* o; long long orow, oh;
-  int Tn, H, Dv;
+  int Tn, H, Dv, rows;                      // rows: of a workgroup
 };
 
 // KS: steps of 32 along R; a wave per 16 of Dv
@@ -132,7 +133,8 @@ __global__ void __launch_bounds__(1024) latent_out_kernel(const OutArgs<T> a) {
   constexpr int R = 32 * KS, LD = R + 8;               // (16-byte pieces of 16 rows: no bank conflicts)
   __shared__ __attribute__((aligned(16))) T s_x[16 * LD];
   __shared__ float s_w[16][64];
-  const int h = blockIdx.y, t0 = blockIdx.x * 16, n = min(16, a.Tn - t0);
+  __shared__ int s_n[16];
+  const int h = blockIdx.y, t0 = blockIdx.x * a.rows, n = min(a.rows, a.Tn - t0);
   const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4, w = tid >> 6;
   uint4 u[KS];
   const T* ur = a.uv + ((long long)h * a.Dv + 16 * w + lr) * R + 8 * lg;
@@ -143,6 +145,8 @@ __global__ void __launch_bounds__(1024) latent_out_kernel(const OutArgs<T> a) {
       const long long base = ((long long)(t0 + i) * a.H + h) * a.nsplit;
       const float ms = lane < a.nsplit ? a.ml[2 * (base + lane)] : -INFINITY;
       const float ls = lane < a.nsplit ? a.ml[2 * (base + lane) + 1] : 0.f;
+      const int live = __popcll(__ballot(lane < a.nsplit && !(ls < 0.f)));   // (the last ones had no key: no sums)
+      if (lane == 0) s_n[i] = live;
       const float M = wave_max(ms);
       const float e = ms == -INFINITY ? 0.f : expf(ms - M);
       float L = wave_sum(ls * e);
@@ -159,15 +163,16 @@ __global__ void __launch_bounds__(1024) latent_out_kernel(const OutArgs<T> a) {
       const auto add = [&](const float4& y, float k) {
         v[0] += y.x * k; v[1] += y.y * k; v[2] += y.z * k; v[3] += y.w * k;
       };
+      const int live = s_n[i];
       int s = 0;
-      for (; s + 4 <= a.nsplit; s += 4) {
+      for (; s + 4 <= live; s += 4) {
         float4 y[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) y[q] = *reinterpret_cast<const float4*>(p + (long long)(s + q) * R);
 #pragma unroll
         for (int q = 0; q < 4; ++q) add(y[q], s_w[i][s + q]);
       }
-      for (; s < a.nsplit; ++s) add(*reinterpret_cast<const float4*>(p + (long long)s * R), s_w[i][s]);
+      for (; s < live; ++s) add(*reinterpret_cast<const float4*>(p + (long long)s * R), s_w[i][s]);
       store4<T>(s_x + i * LD + c, v);
     } else {
       *reinterpret_cast<uint2*>(s_x + i * LD + c) =
@@ -244,10 +249,14 @@ hipError_t sm_latent_out(int dt, const float* ml, const float* part, int nsplit,
       (uintptr_t)uv % 16 || (uintptr_t)o % 8 || orow % 4 || oh % 4 || (dt != kBF16 && dt != kF16) ||
       (nsplit > 1 ? !ml || !part || (uintptr_t)part % 16 : !x || (uintptr_t)x % 8 || xr % 4 || xh % 4))
     return hipErrorInvalidValue;
-  const dim3 grid((rows + 15) / 16, H);
+  // rows of a workgroup: 16, fewer where that leaves CUs idle, as the sums of 16 rows and a head's weights are 300 KB to
+  // fetch for one (16 rows -> fewer, us with the attention: 8 rows of 16 heads 16.7 -> 14.1, 16 of 8 18.8 -> 13.8, 64 of 16 25.8 -> 21.3)
+  int per = 16;
+  while (per > 1 && (long long)((rows + per - 1) / per) * H < 256) per /= 2;
+  const dim3 grid((rows + per - 1) / per, H);
 #define GO(T, KS)                                                                                                 \
   latent_out_kernel<T, KS><<<grid, 4 * Dv, 0, st>>>(OutArgs<T>{ml, part, nsplit, (const T*)x, xr, xh, (const T*)gate, \
-                                                               gater, (const T*)uv, (T*)o, orow, oh, rows, H, Dv})
+                                                               gater, (const T*)uv, (T*)o, orow, oh, rows, H, Dv, per})
 #define GO_T(T)                            \
   if (R == 64) GO(T, 2);                   \
   else if (R == 128) GO(T, 4);             \

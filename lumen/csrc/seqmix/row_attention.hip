@@ -293,7 +293,7 @@ template <typename T, int HPW, bool MMA>
 __global__ void __launch_bounds__(64 * kWaves)
 row_attn_kernel(const RowAttnArgs<T> a) {
   extern __shared__ float smem[];
-  const int t = xcd_row(blockIdx.x, gridDim.x), lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int t = row_of(a, blockIdx.x, gridDim.x), lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int h0 = blockIdx.y * a.HB;
   const int nh = min(a.HB, a.H - h0);
   const int Dk = a.D1 + a.D2;
@@ -598,21 +598,38 @@ row_attn_kernel(const RowAttnArgs<T> a) {
 //      lane-local and nothing is merged across waves at the end.
 // Scores, maxima, sums and the accumulator are fp32.
 //
-// A decode step costs the chain of its loads: position, table, 18 steps of key fragments, 4 of values, each waited for.
-// DEEP sends for four steps of keys while four are multiplied, and for the first values with the first keys: 64 rows of 500
-// tokens, 16 heads over 512 + 64, 26.6 -> 23.3 us, one row 17.5 -> 15.1.  It takes registers: many rows of small ranks, whose workgroups hide each other's loads, keep the form
-// without (1024 rows of 250 tokens over 256 + 32: 34 us, DEEP 50).
-template <typename T, int NT, bool DEEP>   // NT: 16-channel tiles per wave, Dv = 64 NT
-__global__ void __launch_bounds__(64 * kWaves, DEEP ? 2 : 1)
+// A workgroup whose split holds no key of its row: (max, sum) = (-inf, -1), and no values
+template <typename T>
+__device__ __forceinline__ bool latent_no_tile(const RowAttnArgs<T>& a, int t, int pos, int h0, int nh, int tile) {
+  if (tile * (int)blockIdx.z <= pos || a.nsplit == 1) return false;
+  if ((int)threadIdx.x < nh) {
+    const long long slot = ((long long)t * a.H + h0 + threadIdx.x) * a.nsplit + blockIdx.z;
+    a.ws_ml[2 * slot] = -INFINITY;
+    a.ws_ml[2 * slot + 1] = -1.f;
+  }
+  return true;
+}
+// Of a lane's 8 keys the first n are seen: keys past the row's position carry weight 0 but may hold anything
+__device__ __forceinline__ uint4 seen_mask(int n) {
+  if (n >= 8) return make_uint4(~0u, ~0u, ~0u, ~0u);
+  const unsigned e = n <= 0 ? 0u : (unsigned)n;
+  const unsigned long long lo = e >= 4 ? ~0ull : (e == 0 ? 0ull : ((1ull << (16 * e)) - 1));
+  const unsigned long long hi = e <= 4 ? 0ull : ((1ull << (16 * (e - 4))) - 1);
+  return make_uint4((unsigned)lo, (unsigned)(lo >> 32), (unsigned)hi, (unsigned)(hi >> 32));
+}
+
+template <typename T, int NT>   // NT: 16-channel tiles per wave, Dv = 64 NT
+__global__ void __launch_bounds__(64 * kWaves)
 latent_attn_kernel(const RowAttnArgs<T> a, const T* __restrict__ vt) {
   extern __shared__ float smem[];
   constexpr int kPRow = 128 + 8;                 // weights per head in LDS: 128 keys + padding
-  const int t = xcd_row(blockIdx.x, gridDim.x), lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int t = row_of(a, blockIdx.x, gridDim.x), lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int h0 = blockIdx.y * 16;
   const int nh = min(16, a.H - h0);
   const int Dk = a.D1 + a.D2;
   const int Dkp = (Dk + 31) / 32 * 32;
   const int pos = a.positions[t];
+  if (latent_no_tile(a, t, pos, h0, nh, 128)) return;
   const int* tbl = a.tables + (long long)a.row_seg[t] * a.maxb;
   const int hd = lane & 15, kg = lane >> 4;
   T* s_qb = reinterpret_cast<T*>(smem);                               // [16][Dkp + pad]
@@ -645,40 +662,6 @@ latent_attn_kernel(const RowAttnArgs<T> a, const T* __restrict__ vt) {
 #pragma unroll
   for (int n = 0; n < NT; ++n) O[n] = f32x4v{0.f, 0.f, 0.f, 0.f};
   const T* qp = s_qb + hd * (Dkp + kQPad);
-  // key fragments of kCh steps of 32 channels: one chunk is loaded while the one before it is multiplied
-  constexpr int kCh = DEEP ? 4 : 1;
-  uint4 ka[kCh], kb[kCh], kc[kCh], kd[kCh], vv[DEEP ? 2 : 1][NT];
-  const T *kp0 = a.kc, *kp1 = a.kc;
-  const auto keys = [&](int jw) {                          // the rows of the lane's keys (addressable ones)
-    const int k0 = min(jw + hd, pos), k1 = min(jw + 16 + hd, pos);
-    kp0 = a.kc + ((long long)tbl[k0 / a.bs] * a.bs + k0 % a.bs) * a.krow + 8 * kg;
-    kp1 = a.kc + ((long long)tbl[k1 / a.bs] * a.bs + k1 % a.bs) * a.krow + 8 * kg;
-  };
-  const auto load = [&](uint4 (&x)[kCh], uint4 (&y)[kCh], int d0) {
-#pragma unroll
-    for (int c = 0; c < kCh; ++c)
-      if (d0 + 32 * c < Dkp) {
-        const bool in = d0 + 32 * c + 8 * kg < Dk;         // (past the key: zeros)
-        x[c] = in ? *reinterpret_cast<const uint4*>(kp0 + d0 + 32 * c) : make_uint4(0u, 0u, 0u, 0u);
-        y[c] = in ? *reinterpret_cast<const uint4*>(kp1 + d0 + 32 * c) : make_uint4(0u, 0u, 0u, 0u);
-      }
-  };
-  const auto values = [&](uint4 (&v)[NT], int jb) {        // the lane's 8 keys from jb on, its channels
-    const int k = min(jb, pos);
-    const T* vp = vt + ((long long)tbl[k / a.bs] * a.Dv) * a.bs + jb % a.bs;
-#pragma unroll
-    for (int n = 0; n < NT; ++n)
-      v[n] = *reinterpret_cast<const uint4*>(vp + (long long)((w * NT + n) * 16 + hd) * a.bs);
-  };
-  if (128 * (int)blockIdx.z + 32 * w <= pos) {
-    keys(128 * blockIdx.z + 32 * w);
-    if (DEEP) load(ka, kb, 0);
-  }
-  const auto ahead = [&](int j0) {                         // the first two steps' values of a tile
-    if (DEEP && j0 <= pos) values(vv[0], j0 + 8 * kg);
-    if (DEEP && j0 + 32 <= pos) values(vv[DEEP], j0 + 32 + 8 * kg);
-  };
-  ahead(128 * blockIdx.z);
   __syncthreads();
 
   for (int j0 = 128 * blockIdx.z; j0 <= pos; j0 += 128 * a.nsplit) {
@@ -688,25 +671,16 @@ latent_attn_kernel(const RowAttnArgs<T> a, const T* __restrict__ vt) {
     float mx = -INFINITY;
     f32x4v c0 = {0.f, 0.f, 0.f, 0.f}, c1 = {0.f, 0.f, 0.f, 0.f};
     if (jw <= pos) {
-      const auto mul = [&](const uint4 (&x)[kCh], const uint4 (&y)[kCh], int d0) {
-#pragma unroll
-        for (int c = 0; c < kCh; ++c)
-          if (d0 + 32 * c < Dkp) {
-            const uint4 bv = *reinterpret_cast<const uint4*>(qp + d0 + 32 * c + 8 * kg);
-            c0 = Mma16<T>::run(x[c], bv, c0);
-            c1 = Mma16<T>::run(y[c], bv, c1);
-          }
-      };
-      if (!DEEP)
-        for (int d0 = 0; d0 < Dkp; d0 += 32) {
-          load(ka, kb, d0);
-          mul(ka, kb, d0);
-        }
-      else for (int d0 = 0; d0 < Dkp; d0 += 64 * kCh) {
-        if (d0 + 32 * kCh < Dkp) load(kc, kd, d0 + 32 * kCh);
-        mul(ka, kb, d0);
-        if (d0 + 64 * kCh < Dkp) load(ka, kb, d0 + 64 * kCh);
-        if (d0 + 32 * kCh < Dkp) mul(kc, kd, d0 + 32 * kCh);
+      const int k0 = min(jw + hd, pos), k1 = min(jw + 16 + hd, pos);       // the rows of the lane's keys (addressable ones)
+      const T* kp0 = a.kc + ((long long)tbl[k0 / a.bs] * a.bs + k0 % a.bs) * a.krow + 8 * kg;
+      const T* kp1 = a.kc + ((long long)tbl[k1 / a.bs] * a.bs + k1 % a.bs) * a.krow + 8 * kg;
+      for (int d0 = 0; d0 < Dkp; d0 += 32) {
+        const bool in = d0 + 8 * kg < Dk;                  // (past the key: zeros)
+        const uint4 x = in ? *reinterpret_cast<const uint4*>(kp0 + d0) : make_uint4(0u, 0u, 0u, 0u);
+        const uint4 y = in ? *reinterpret_cast<const uint4*>(kp1 + d0) : make_uint4(0u, 0u, 0u, 0u);
+        const uint4 bv = *reinterpret_cast<const uint4*>(qp + d0 + 8 * kg);
+        c0 = Mma16<T>::run(x, bv, c0);
+        c1 = Mma16<T>::run(y, bv, c1);
       }
     }
     if (jw <= pos) {
@@ -767,31 +741,21 @@ latent_attn_kernel(const RowAttnArgs<T> a, const T* __restrict__ vt) {
       if (j0 + 32 * ks > pos) continue;
       const uint4 bh = *reinterpret_cast<const uint4*>(s_ph + hd * kPRow + 32 * ks + 8 * kg);
       const uint4 bl = *reinterpret_cast<const uint4*>(s_pl + hd * kPRow + 32 * ks + 8 * kg);
-      if (!DEEP) values(vv[0], jb);
-      // keys past the row's position carry weight 0 but may hold anything: blank them
-      const int nv = pos - jb + 1;                         // visible keys among the lane's 8
-      uint4 mk = make_uint4(~0u, ~0u, ~0u, ~0u);
-      if (nv < 8) {
-        const unsigned e = nv <= 0 ? 0u : (unsigned)nv;
-        const unsigned long long lo = e >= 4 ? ~0ull : (e == 0 ? 0ull : ((1ull << (16 * e)) - 1));
-        const unsigned long long hi = e <= 4 ? 0ull : ((1ull << (16 * (e - 4))) - 1);
-        mk = make_uint4((unsigned)lo, (unsigned)(lo >> 32), (unsigned)hi, (unsigned)(hi >> 32));
-      }
+      const int k = min(jb, pos);
+      const T* vp = vt + ((long long)tbl[k / a.bs] * a.Dv) * a.bs + jb % a.bs;
+      uint4 vv[NT];
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+        vv[n] = *reinterpret_cast<const uint4*>(vp + (long long)((w * NT + n) * 16 + hd) * a.bs);
+      const uint4 mk = seen_mask(pos - jb + 1);
 #pragma unroll
       for (int n = 0; n < NT; ++n) {
-        uint4 av = vv[DEEP ? ks & 1 : 0][n];                          // as A operand: the lane's channel
+        uint4 av = vv[n];                                    // as A operand: the lane's channel
         av.x &= mk.x; av.y &= mk.y; av.z &= mk.z; av.w &= mk.w;
         O[n] = Mma16<T>::run(av, bh, O[n]);
         O[n] = Mma16<T>::run(av, bl, O[n]);
       }
-      if (DEEP && ks < 2 && j0 + 32 * (ks + 2) <= pos) values(vv[DEEP ? ks & 1 : 0], jb + 64);
     }
-    const int jn = j0 + 128 * a.nsplit + 32 * w;           // the next tile's first keys
-    if (jn <= pos) {
-      keys(jn);
-      if (DEEP) load(ka, kb, 0);
-    }
-    ahead(j0 + 128 * a.nsplit);
   }
   // O[n][i] = O^T[channel (w NT + n) 16 + 4 kg + i][head hd]
   if (head_on) {
@@ -821,27 +785,200 @@ latent_attn_kernel(const RowAttnArgs<T> a, const T* __restrict__ vt) {
   }
 }
 
+// The same for few rows, whose step costs the chain of its loads: position, table, keys, values.  W waves share a tile of 16 W keys;
+// a wave's 16 keys (18 pieces of 16 bytes a lane for 512 + 64 channels) and its part of the channels' values over all of
+// the tile's keys (16 pieces) are asked for together and wait in registers.  Splits without a key of their row store no sums.
+// A graph of caches rotated through 700 MB, merge and expansion included, four waves that load four steps ahead -> here, us, 16
+// heads over 512 + 64: 1 row of 331 keys 20.9 -> 14.0, 8 rows of 62 - 500 27.6 -> 14.1, 64 of 64 - 514 31.1 -> 21.3, 200 of 62 - 500
+// 56.8 -> 43.8, 600 of 37 - 300 86 -> 55 (from 200 rows on most of it by where the rows run, RowAttnArgs::own); over 256 + 32, 64 rows
+// 20.7 -> 15.3.
+template <typename T, int NT, int KS, int W>   // Dv = 64 NT, keys of KS steps of 32 channels
+__global__ void __launch_bounds__(64 * W, 2)
+latent_row_kernel(const RowAttnArgs<T> a, const T* __restrict__ vt) {
+  constexpr int Dkp = 32 * KS, LQ = Dkp + kQPad, TILE = 16 * W, kPRow = TILE + 8, NV = 4 * NT / W, VS = W / 2, NTH = 64 * W;
+  __shared__ __attribute__((aligned(16))) T s_qb[16 * LQ];
+  __shared__ __attribute__((aligned(16))) T s_ph[16 * kPRow], s_pl[16 * kPRow];
+  __shared__ float s_m[W][16], s_l[W][16];
+  const int t = row_of(a, blockIdx.x, gridDim.x), lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h0 = blockIdx.y * 16, nh = min(16, a.H - h0), Dk = a.D1 + a.D2;
+  const int pos = a.positions[t];
+  const int* tbl = a.tables + (long long)a.row_seg[t] * a.maxb;
+  const int hd = lane & 15, kg = lane >> 4;
+  // queries: pieces of 8 channels, Dkp / 8 a head
+  constexpr int NQ = (16 * Dkp / 8 + NTH - 1) / NTH;
+  uint4 qv[NQ];
+#pragma unroll
+  for (int i = 0; i < NQ; ++i) {
+    const int c = threadIdx.x + NTH * i, hl = c / (Dkp / 8), d = (c % (Dkp / 8)) * 8;
+    qv[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (hl < nh && d < Dk)
+      qv[i] = d < a.D1 ? *reinterpret_cast<const uint4*>(a.q1 + (long long)t * a.q1r + (long long)(h0 + hl) * a.q1h + d)
+                       : *reinterpret_cast<const uint4*>(a.q2 + (long long)t * a.q2r + (long long)(h0 + hl) * a.q2h + (d - a.D1));
+  }
+  if (latent_no_tile(a, t, pos, h0, nh, TILE)) return;
+  float temp = 1.f;
+  if (a.tevery > 0 && a.tcoef != 0.f)
+    temp = 1.f + a.tcoef * logf((float)((pos + 1) / a.tevery) + 1.f);
+  const float qscale = a.scale * temp;
+  const bool head_on = hd < nh;
+  const int h = h0 + (head_on ? hd : 0);
+  const bool sk = a.sink != nullptr && blockIdx.z == 0;
+  float m_run = sk ? a.sink[h] : -INFINITY, l_run = sk ? 1.f : 0.f;
+  const float r1 = a.r1 ? a.r1[h] : 0.f, r2 = a.r1 ? a.r2[h] : 0.f;
+  f32x4v O[NV];
+#pragma unroll
+  for (int n = 0; n < NV; ++n) O[n] = f32x4v{0.f, 0.f, 0.f, 0.f};
+  const int ch0 = (w * NV) * 16 + hd;                      // the lane's first channel as A operand
+  for (int j0 = TILE * blockIdx.z; j0 <= pos; j0 += TILE * a.nsplit) {
+    const int jw = j0 + 16 * w, jk = min(jw + hd, pos);
+    int vb[VS];
+    const int kb = tbl[jk / a.bs];
+#pragma unroll
+    for (int s = 0; s < VS; ++s) vb[s] = tbl[min(j0 + 32 * s + 8 * kg, pos) / a.bs];
+    const T* kp = a.kc + ((long long)kb * a.bs + jk % a.bs) * a.krow + 8 * kg;
+    uint4 k[KS], v[VS][NV];
+#pragma unroll
+    for (int s = 0; s < KS; ++s)                           // (only the last step may pass the key's end)
+      k[s] = s + 1 < KS || 32 * s + 8 * kg < Dk ? *reinterpret_cast<const uint4*>(kp + 32 * s) : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+    for (int s = 0; s < VS; ++s) {
+      const T* vp = vt + ((long long)vb[s] * a.Dv + ch0) * a.bs + (j0 + 32 * s + 8 * kg) % a.bs;
+#pragma unroll
+      for (int n = 0; n < NV; ++n) v[s][n] = *reinterpret_cast<const uint4*>(vp + (long long)(16 * n) * a.bs);
+    }
+    if (j0 == TILE * (int)blockIdx.z) {
+#pragma unroll
+      for (int i = 0; i < NQ; ++i) {
+        const int c = threadIdx.x + NTH * i;
+        if (c < 16 * Dkp / 8) *reinterpret_cast<uint4*>(s_qb + c / (Dkp / 8) * LQ + (c % (Dkp / 8)) * 8) = qv[i];
+      }
+      __syncthreads();
+    }
+    // 1. scores of the wave's 16 keys: c[i] = S^T[key 4 kg + i][head hd]
+    f32x4v c = {0.f, 0.f, 0.f, 0.f}, c1 = c;
+    const T* qp = s_qb + hd * LQ + 8 * kg;
+#pragma unroll
+    for (int s = 0; s + 1 < KS; s += 2) {
+      c = Mma16<T>::run(k[s], *reinterpret_cast<const uint4*>(qp + 32 * s), c);
+      c1 = Mma16<T>::run(k[s + 1], *reinterpret_cast<const uint4*>(qp + 32 * s + 32), c1);
+    }
+    if (KS % 2) c = Mma16<T>::run(k[KS - 1], *reinterpret_cast<const uint4*>(qp + 32 * KS - 32), c);
+    c += c1;
+    float sc[4], mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int j = jw + 4 * kg + i;
+      float sv = c[i] * qscale;
+      if (a.softcap > 0.f) sv = a.softcap * tanhf(sv / a.softcap);
+      if (a.r1 != nullptr) sv -= r1 * logf(1.f + r2 * (float)(pos - j));
+      sc[i] = j <= pos ? sv : -INFINITY;
+      mx = fmaxf(mx, sc[i]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if (kg == 0) s_m[w][hd] = mx;
+    __syncthreads();
+    // 2. the tile's maximum per head, the weights of the wave's keys into LDS
+    float mn = m_run;                                      // finite: key j0 is visible
+#pragma unroll
+    for (int q = 0; q < W; ++q) mn = fmaxf(mn, s_m[q][hd]);
+    const float corr = expf(m_run - mn);
+    float ls = 0.f, ph[4], pl[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float pv = sc[i] == -INFINITY ? 0.f : expf(sc[i] - mn);
+      ls += pv;
+      ph[i] = to_f32(from_f32<T>(pv));
+      pl[i] = pv - ph[i];
+    }
+    const int col = 16 * w + 4 * kg;
+    *reinterpret_cast<uint2*>(s_ph + hd * kPRow + col) = make_uint2(pk2<T>(ph[0], ph[1]), pk2<T>(ph[2], ph[3]));
+    *reinterpret_cast<uint2*>(s_pl + hd * kPRow + col) = make_uint2(pk2<T>(pl[0], pl[1]), pk2<T>(pl[2], pl[3]));
+    ls += __shfl_xor(ls, 16, 64);
+    ls += __shfl_xor(ls, 32, 64);
+    if (kg == 0) s_l[w][hd] = ls;
+#pragma unroll
+    for (int n = 0; n < NV; ++n) O[n] *= corr;
+    __syncthreads();
+    // 3. O^T += V^T P^T for the wave's channels over the tile's keys
+    l_run *= corr;
+#pragma unroll
+    for (int q = 0; q < W; ++q) l_run += s_l[q][hd];
+    m_run = mn;
+#pragma unroll
+    for (int s = 0; s < VS; ++s) {
+      if (j0 + 32 * s > pos) continue;
+      const uint4 bh = *reinterpret_cast<const uint4*>(s_ph + hd * kPRow + 32 * s + 8 * kg);
+      const uint4 bl = *reinterpret_cast<const uint4*>(s_pl + hd * kPRow + 32 * s + 8 * kg);
+      const uint4 mk = seen_mask(pos - (j0 + 32 * s + 8 * kg) + 1);
+#pragma unroll
+      for (int n = 0; n < NV; ++n) {
+        uint4 av = v[s][n];
+        av.x &= mk.x; av.y &= mk.y; av.z &= mk.z; av.w &= mk.w;
+        O[n] = Mma16<T>::run(av, bh, O[n]);
+        O[n] = Mma16<T>::run(av, bl, O[n]);
+      }
+    }
+  }
+  // O[n][i] = O^T[channel (w NV + n) 16 + 4 kg + i][head hd]
+  if (!head_on) return;
+  if (a.nsplit == 1) {
+    float inv = 1.f / l_run;
+    if (a.gate != nullptr) inv *= sigmoid_f(to_f32(a.gate[(long long)t * a.gater + h]));
+    T* op = a.out + (long long)t * a.our + (long long)h * a.ouh;
+#pragma unroll
+    for (int n = 0; n < NV; ++n)
+      *reinterpret_cast<uint2*>(op + (w * NV + n) * 16 + 4 * kg) =
+          make_uint2(pk2<T>(O[n][0] * inv, O[n][1] * inv), pk2<T>(O[n][2] * inv, O[n][3] * inv));
+  } else {
+    const long long slot = ((long long)t * a.H + h) * a.nsplit + blockIdx.z;
+    if (w == 0 && kg == 0) {
+      a.ws_ml[2 * slot] = m_run;
+      a.ws_ml[2 * slot + 1] = l_run;
+    }
+#pragma unroll
+    for (int n = 0; n < NV; ++n)
+      *reinterpret_cast<float4*>(a.ws_o + slot * a.Dv + (w * NV + n) * 16 + 4 * kg) = make_float4(O[n][0], O[n][1], O[n][2], O[n][3]);
+  }
+}
+
 inline size_t latent_attn_lds(int Dk, int esz) {
   return (size_t)16 * ((Dk + 31) / 32 * 32 + kQPad) * esz + 2 * (size_t)16 * (128 + 8) * esz +
          2 * kWaves * 16 * sizeof(float);
 }
 
+// Rows times blocks of 16 heads up to which a workgroup takes 64 keys instead of 128: a CU fetches 60 B/ns, so few workgroups want
+// few keys each, and many the fewer partial sums (64 / 128 keys, us: 1 row 14.0 / 17.1, 16 rows of 8 heads 18.8 / 21.4, 32 of 16
+// 18.3 / 20.3, 64 of 16 23.3 / 21.3, of 2000 keys 51 / 53)
+constexpr int kLatentNarrow = 32;
+
 template <typename T>
 hipError_t launch_latent_attn(const RowAttnArgs<T>& a, const T* vt, int Tn, hipStream_t st) {
   const size_t lds = latent_attn_lds(a.D1 + a.D2, sizeof(T));
   const dim3 grid(Tn, (a.H + 15) / 16, a.nsplit);
-  // two workgroups of the deep form fit a CU, as of the other one at ranks of 384 and more.  Up to 192 the forms are even.
-  const bool deep = (long long)grid.x * grid.y * grid.z <= 512;
-#define LATENT(N, D) latent_attn_kernel<T, N, D><<<grid, 64 * kWaves, lds, st>>>(a, vt)
+  const int ks = (a.D1 + a.D2 + 31) / 32;
+  const bool few = (long long)grid.x * grid.y * grid.z <= 512, narrow = (long long)grid.x * grid.y <= kLatentNarrow;
+#define LATENT(N) latent_attn_kernel<T, N><<<grid, 64 * kWaves, lds, st>>>(a, vt)
+#define ROW(N, KS)                                                                        \
+  if (narrow) latent_row_kernel<T, N, KS, 4><<<grid, 256, 0, st>>>(a, vt);                \
+  else latent_row_kernel<T, N, KS, 8><<<grid, 512, 0, st>>>(a, vt)
+#define ROWS(N)                                  \
+  if (ks == 2 * N) { ROW(N, 2 * N); }            \
+  else if (ks == 2 * N + 1) { ROW(N, 2 * N + 1); } \
+  else if (ks == 2 * N + 2) { ROW(N, 2 * N + 2); } \
+  else LATENT(N)
   switch (a.Dv / 64) {
-    case 1: LATENT(1, false); break;
-    case 2: LATENT(2, false); break;
-    case 3: LATENT(3, false); break;
-    case 4: if (deep) LATENT(4, true); else LATENT(4, false); break;
-    case 6: LATENT(6, true); break;
-    case 8: LATENT(8, true); break;
+    case 1: LATENT(1); break;
+    case 2: LATENT(2); break;
+    case 3: LATENT(3); break;
+    case 4: if (few) { ROWS(4); } else { LATENT(4); } break;
+    case 6: ROWS(6); break;
+    case 8: ROWS(8); break;
     default: return hipErrorInvalidValue;
   }
+#undef ROWS
+#undef ROW
 #undef LATENT
   return hipGetLastError();
 }
@@ -1022,8 +1159,8 @@ hipError_t sm_latent_attn(int dt, const void* q1, long long q1r, long long q1h, 
                           long long ouh, const int* tables, int maxb, const int* row_seg,
                           const int* positions, int T, int H, int bs, float scale, float softcap,
                           float tcoef, int tevery, const float* r1, const float* r2,
-                          const float* sink, const void* gate, long long gater, int nsplit,
-                          float* ws_ml, float* ws_o, hipStream_t st) {
+                          const float* sink, const void* gate, long long gater, int own,
+                          int nsplit, float* ws_ml, float* ws_o, hipStream_t st) {
   if (T == 0) return hipSuccess;
   const auto al = [](const void* p) { return (uintptr_t)p % 16 == 0; };
   if (!sm_latent_attn_ok(dt, Dv, D1 + D2, D1, bs) || nsplit < 1 || nsplit > 64 ||
@@ -1037,7 +1174,7 @@ hipError_t sm_latent_attn(int dt, const void* q1, long long q1r, long long q1h, 
                       (const TT*)kc, krow, (const TT*)kc, krow, Dv, (TT*)out, our, ouh,       \
                       tables, maxb, row_seg, positions, H, 1, 16, bs, scale, softcap, tcoef,  \
                       tevery, r1, r2, nullptr, sink, nullptr, 0, 0, (const TT*)gate, gater,   \
-                      nullptr, 1, nsplit, ws_ml, ws_o};                                       \
+                      nullptr, 1, own, nsplit, ws_ml, ws_o};                                  \
     hipError_t e = launch_latent_attn<TT>(a, (const TT*)vt, T, st);                           \
     if (e != hipSuccess) return e;                                                            \
     if (nsplit > 1 && out)      /* (without: the caller adds the splits, sm_latent_out) */     \
@@ -1061,8 +1198,8 @@ hipError_t sm_row_attn(int dt, const void* q1, long long q1r, long long q1h, int
                        int bs, float scale, float softcap, float tcoef, int tevery,
                        const float* r1, const float* r2, const float* talk, const float* sink,
                        const float* slopes, int window, int keep, const void* gate,
-                       long long gater, const float* sigb, int vdiv, int nsplit, float* ws_ml,
-                       float* ws_o, hipStream_t st) {
+                       long long gater, const float* sigb, int vdiv, int own, int nsplit,
+                       float* ws_ml, float* ws_o, hipStream_t st) {
   if (T == 0) return hipSuccess;
   if (nsplit < 1 || nsplit > 64 || (nsplit > 1 && (!ws_ml || !ws_o))) return hipErrorInvalidValue;
   if (vdiv < 1 || G % vdiv != 0 || (sigb && sink)) return hipErrorInvalidValue;
@@ -1075,7 +1212,7 @@ hipError_t sm_row_attn(int dt, const void* q1, long long q1r, long long q1h, int
                       (const TT*)kc, krow, (const TT*)vc, vrow, Dv, (TT*)out, our, ouh,       \
                       tables, maxb, row_seg, positions, H, G, HB, bs, scale, softcap, tcoef,  \
                       tevery, r1, r2, talk, sink, slopes, window, keep, (const TT*)gate,      \
-                      gater, sigb, vdiv, nsplit, ws_ml, ws_o};                                \
+                      gater, sigb, vdiv, own, nsplit, ws_ml, ws_o};                                \
     return launch_row_attn<TT>(a, T, st);                                                     \
   }
   SM_DISPATCH(dt, CALL)

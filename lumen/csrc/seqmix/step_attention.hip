@@ -124,7 +124,7 @@ step_attn_kernel(const RowAttnArgs<T> a) {
   __shared__ float s_c[4][HP];
   __shared__ __attribute__((aligned(16))) float s_o[4][HP][D];
   __shared__ float s_m[4][HP], s_l[4][HP];
-  const int t = xcd_row(blockIdx.x, gridDim.x), g = blockIdx.y, z = blockIdx.z;
+  const int t = row_of(a, blockIdx.x, gridDim.x), g = blockIdx.y, z = blockIdx.z;
   const int lane = threadIdx.x & 63, lr = lane & 15, kg = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int pos = a.positions[t];
@@ -279,7 +279,7 @@ template <typename T, int HP>
 __global__ void __launch_bounds__(512, 2)
 talk_attn_kernel(const RowAttnArgs<T> a) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
-  const int t = xcd_row(blockIdx.x, gridDim.x), z = blockIdx.z, H = a.H, ld = H + 4;
+  const int t = row_of(a, blockIdx.x, gridDim.x), z = blockIdx.z, H = a.H, ld = H + 4;
   const int lane = threadIdx.x & 63, lr = lane & 15, kg = lane >> 4;
   const int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // the wave's key head
   float* s_sc = smem;

@@ -38,9 +38,9 @@ SIGNATURES = {
     "sm_rotate_heads": "iplliiippi",
     "sm_latent_write": "iplpppppppiiiiif",
     "sm_head_norm_write": "iplpppppiiiiif",
-    "sm_latent_attn": "i" "plli" "plli" "pl" "pi" "pll" "pi" "pp" "iii" "fffi" "ppp" "pl" "ipp",
+    "sm_latent_attn": "i" "plli" "plli" "pl" "pi" "pll" "pi" "pp" "iii" "fffi" "ppp" "pl" "iipp",
     "sm_row_attn": "i" "plli" "plli" "pl" "pli" "pll" "pi" "pp" "iiiii" "fffi" "pppp" "piipl"
-                   "pi" "ipp",
+                   "pi" "iipp",
     "sm_win_attn_tiles": "iplppppl" "pi" "pi" "pp" "iiii" "ff" "p" "iii" "ipi",
     "sm_fresh_tiles": "i" "plplplpl" "p" "pii" "pp" "iiii" "f",
     "sm_talk_tiles": "i" "pll" "pp" "pll" "pi" "pii" "pp" "iiiii" "fffi" "pppp",

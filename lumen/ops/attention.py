@@ -1038,6 +1038,7 @@ def _heads_per_block(H: int, Dk: int, need_all: bool) -> int:
     return hb
 
 
+LATENT_NARROW = 32           # rows x 16-head blocks up to which row_attention.hip takes 64 keys a workgroup (kLatentNarrow there)
 LATENT_TILE_ROWS = 2048      # rows x 16-head blocks from which prompt portions take the tiled latent kernel
 
 
@@ -1137,6 +1138,7 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
     coef, every = (float(q_temp[0]), int(q_temp[1])) if q_temp is not None else (0.0, 0)
     bs = kcache.shape[1]
     al8 = lambda x: x.data_ptr() % 16 == 0 and x.stride(0) % 8 == 0 and x.stride(1) % 8 == 0  # noqa: E731
+    own = int(seg.cu.shape[0] - 1 == T)                  # decoded rows: every one a sequence of its own
     if (vt is not None and G == 1 and talk is None and vcache is kcache and D1 >= Dv
             and slopes is None and window == 0 and sigmoid_bias is None
             and (gate is None or gate.stride(1) == 1)
@@ -1168,8 +1170,9 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
         else:
             full = out
         blocks = T * ((H + 15) // 16)
-        tiles = (seg.tables.shape[1] * bs + 127) // 128
-        nsplit = max(1, min(tiles, 32, 512 // max(blocks, 1)))
+        keys = 64 if blocks <= LATENT_NARROW else 128             # (a workgroup's tile: the launcher's rule)
+        tiles = (seg.tables.shape[1] * bs + keys - 1) // keys
+        nsplit = max(1, min(tiles, 64 if keys == 64 else 32, 512 // max(blocks, 1)))
         ws_ml = ws_o = None
         if nsplit > 1:
             ws_ml = torch.empty(T * H * nsplit * 2, dtype=torch.float32, device=q1.device)
@@ -1180,7 +1183,7 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
              kcache, krow, vt, Dv, None if fused and nsplit > 1 else out, out.stride(0), out.stride(1),
              seg.tables, seg.tables.shape[1], row_seg, positions, T, H, bs,
              scale, float(softcap or 0.0), coef, every, r1, r2, sink,
-             gate, gate.stride(0) if gate is not None else 0, nsplit, ws_ml, ws_o)
+             gate, gate.stride(0) if gate is not None else 0, own, nsplit, ws_ml, ws_o)
         if fused:
             uv, o = expand
             call("sm_latent_out", DT[q1.dtype], ws_ml, ws_o, nsplit, out, out.stride(0), out.stride(1), gate,
@@ -1253,7 +1256,7 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
          seg.tables, seg.tables.shape[1], row_seg, positions, T, H, G, HB,
          kcache.shape[1], scale, float(softcap or 0.0), coef, every, r1, r2, talk, sink,
          slopes, window, keep_first, gate, gate.stride(0) if gate is not None else 0,
-         sigmoid_bias, v_div, nsplit, ws_ml, ws_o)
+         sigmoid_bias, v_div, own, nsplit, ws_ml, ws_o)
     return out
 
 

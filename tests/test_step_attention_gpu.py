@@ -1,5 +1,6 @@
-"""Attention of decoded rows with heads of 128 (step_attention.hip) with every score shaping it takes, against the torch reference in
-fp32, at the edges of its groups of 16 keys and tiles of 64, in caches whose other rows hold NaN."""
+"""Attention of decoded rows, heads of 128 (step_attention.hip) and latent rows (row_attention.hip), with every score shaping they
+take, against the torch reference in fp32, at the edges of their groups of 16 keys and tiles of 64 and 128, in caches whose other
+rows hold NaN."""
 import pytest
 import torch
 
@@ -53,3 +54,43 @@ def test_shapings(T, H, G, bs, kind, dt):
     # and sums over values of size <= 5 (a score's error of 8 x 32 x 2^-23 x 16 is one of 2^-11 in its weight at the most)
     tol = want.abs() * torch.finfo(dt).eps / 2 + 5.0 * (2.0 ** -11 if "talk" in kind else 2.0 ** -14)
     assert ((out.float().cpu() - want).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shaped,gated", [(False, False), (True, False), (True, True)])
+@pytest.mark.parametrize("T,H,R,D2,bs", [(3, 16, 512, 64, 16), (33, 16, 512, 64, 16), (17, 20, 512, 0, 8), (11, 5, 256, 32, 32),
+                                         (40, 16, 256, 64, 16), (11, 16, 384, 32, 16), (40, 3, 384, 0, 16), (40, 16, 512, 40, 16)])
+def test_latent_rows(T, H, R, D2, bs, shaped, gated, dt):
+    """Tiles of 64 keys (up to 32 rows x 16 heads) and of 128; with and without the expansion of the merged sums."""
+    g = torch.Generator().manual_seed(T + R)
+    ctx = [CTX[t % len(CTX)] for t in range(T)]
+    seg, nb = step(ctx, bs, g)
+    D = R + D2
+    c = torch.full((nb * bs, D), float("nan")).to(dt)
+    for t, n in enumerate(ctx):
+        c[seg.tables[t].long()[torch.arange(n) // bs] * bs + torch.arange(n) % bs] = torch.randn(n, D, generator=g).to(dt)
+    c = c.view(nb, bs, D)
+    q = torch.randn(T, H, D, generator=g).to(dt)
+    uv = (torch.randn(H, 64, R, generator=g) / R ** 0.5).to(dt)
+    rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    kw = dict(softcap=4.0, r1=rnd(H).abs(), r2=rnd(H).abs(), sink=rnd(H), q_temp=(0.4, 32)) if shaped else {}
+    kw["gate"] = rnd(T, H).to(dt) if gated else None
+    q1, q2 = q[:, :, :R], q[:, :, R:] if D2 else None
+    want = row_attention_ref(q1, q2, c, c, R, torch.empty(T, H, R), seg, H, 1, 0.04, **kw)
+    kw = {n: x.cuda() if torch.is_tensor(x) else x for n, x in kw.items()}
+    qd, cd = q.cuda(), c.cuda()
+    args = (qd[:, :, :R], qd[:, :, R:] if D2 else None, cd, cd, R)
+    kw["vt"] = c[:, :, :R].transpose(1, 2).contiguous().cuda()
+    out = torch.empty(T, H, R, dtype=dt, device="cuda")
+    row_attention(*args, out, on_gpu(seg), H, 1, 0.04, **kw)
+    # as above, weights in two 16-bit parts: 16 bits of them for bf16
+    tol = want.abs() * torch.finfo(dt).eps / 2 + 5.0 * 2.0 ** -13
+    assert ((out.float().cpu() - want).abs() <= tol).all()
+    o = torch.empty(T, H, 64, dtype=dt, device="cuda")
+    got = row_attention(*args, out.clone(), on_gpu(seg), H, 1, 0.04, expand=(uv.cuda(), o), **kw)
+    if got is o:                                           # the expansion of the rounded rows, rounded once more
+        w2 = torch.einsum("thr,hvr->thv", out.float().cpu(), uv.float())
+        mag = torch.einsum("thr,hvr->thv", out.float().cpu().abs(), uv.float().abs())
+        tol = w2.abs() * torch.finfo(dt).eps / 2 + mag * (2.0 ** -20 + torch.finfo(dt).eps / 8)
+        assert ((o.float().cpu() - w2).abs() <= tol).all()
+    assert (got is o) == (R in (256, 512))

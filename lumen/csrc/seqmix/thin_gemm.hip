@@ -21,8 +21,8 @@
 // (F.linear) and for M = 1 the rows-per-lane GEMV of kernels/skinny_gemm.hip:
 //   M = 8:  2048 x 2048 3.9 / 8.4, 11264 x 2048 10.1 / 16.3, 2048 x 5632 8.3 / 11.6, 32000 x 2048 23.8 /
 //           33.2, 4096 x 4096 7.8 / 12.9, 22528 x 4096 31.5 / 51.9 (5.9 TB/s), 4096 x 11264 17.5 / 20.7
-//   M = 32: 4.8 / 8.6, 12.5 / 16.3, 12.4 / 15.6, 25.5 / 27.4, 9.5 / 12.7, 37.8 / 42.9, 24.7 / 27.3
-//   M = 64: 6.5 / 9.0, 15.3 / 17.6, 17.4 / 18.4, 29.4 / 27.9, 13.3 / 14.3, 52.0 / 45.1, 33.9 / 34.9
+//   M = 32: 4.8 / 8.6, 12.5 / 16.3, 10.3 / 15.6, 25.5 / 27.4, 9.5 / 12.7, 37.8 / 42.9, 24.7 / 27.3
+//   M = 64: 6.1 / 9.0, 15.3 / 17.6, 12.0 / 18.4, 29.4 / 27.9, 13.3 / 14.3, 52.0 / 45.1, 33.9 / 34.9
 //   M = 1:  3.8 / 8.3 (GEMV 4.4), 9.8 / 16.1 (10.5), 7.3 / 11.7 (6.6), 22.4 / 32.0 (22.9), 7.5 / 12.1
 //           (8.1), 30.7 / 51.6 (28.5), 17.2 / 20.6 (17.2)
 // The activation form (thin_act): a workgroup's tile is 16 activation columns -- their gate rows and
@@ -88,7 +88,7 @@ __device__ __forceinline__ int nth_bit(unsigned long long m, int i) {
   return __builtin_ctzll(m);
 }
 
-// XP: pieces of 8 x rows (1, 2, 4, 8: M <= 8, 16, 32, 64).  ACT: 0 plain, 1 activation of RT = 1 row
+// XP: pieces of 8 x rows (1, 2, 4, 8: groups of up to 8, 16, 32, 64 rows, blockIdx.y names the group).  ACT: 0 plain, 1 activation of RT = 1 row
 // tile (no gate), 2 gated (RT = 2: the tile's gate rows, its up rows).
 template <typename T, int RT, int XP, int NW, int D, int ACT>
 __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
@@ -106,7 +106,8 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
   char* ring = lds + wid * D * SB;
   char* part = lds + NW * D * SB;                  // [2][NW][PB]: this tile's and the last one's
   float* wts = reinterpret_cast<float*>(part + 2 * NW * PB);
-  const T* x = (const T*)p.x;
+  const int m0 = blockIdx.y * (8 * XP), M = min(p.M - m0, 8 * XP);       // this workgroup's rows
+  const T* x = (const T*)p.x + (long long)m0 * p.ldx;
   const T* W = (const T*)p.W;
 
   // experts some row chose (every one of them unless `sparse`)
@@ -114,13 +115,13 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
   int n_chosen = 0;
   if (WTS > 0 && p.E > 0) {
     if (p.wts != nullptr) {
-      for (int i = threadIdx.x; i < p.M * p.E; i += 64 * NW) wts[i] = p.wts[i];
+      for (int i = threadIdx.x; i < M * p.E; i += 64 * NW) wts[i] = p.wts[m0 * p.E + i];
       __syncthreads();
     }
     if (p.sparse) {
       bool on = false;
       if (lane < p.E)
-        for (int m = 0; m < p.M; ++m) on |= !(wts[m * p.E + lane] == 0.f);
+        for (int m = 0; m < M; ++m) on |= !(wts[m * p.E + lane] == 0.f);
       chosen = __ballot(on);
       n_chosen = __popcll(chosen);
     }
@@ -184,7 +185,7 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
 #pragma unroll
     for (int q = 0; q < XP; ++q) {
       const int r = 8 * q + rr;
-      dma16(x, ((unsigned)min(r, p.M - 1) * (unsigned)p.ldx + kk + 8 * (c ^ swz(r))) * 2u,
+      dma16(x, ((unsigned)min(r, M - 1) * (unsigned)p.ldx + kk + 8 * (c ^ swz(r))) * 2u,
             img + WB + 8 * q * ROWB);
     }
     put = put + 1 == D ? 0 : put + 1;
@@ -265,8 +266,8 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
       for (int q = wid; q < RT * MT; q += NW) {
         const int i = q / MT, j = q - i * MT;
         f32x4 v = sum(q);
-        const int m = 16 * j + lr, n = t * RT * 16 + 16 * i + 4 * lg;
-        if (m >= p.M || n >= p.N) continue;
+        const int m = m0 + 16 * j + lr, n = t * RT * 16 + 16 * i + 4 * lg;
+        if (m >= p.M || 16 * j + lr >= M || n >= p.N) continue;
         if (p.bias != nullptr) {
           const T* b = (const T*)p.bias + n;
 #pragma unroll
@@ -300,7 +301,7 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
       for (int j = wid; j < MT; j += NW) {
         const int m = 16 * j + lr;
         f32x4 g = sum(j), u = ACT == 2 ? sum(MT + j) : f32x4{1.f, 1.f, 1.f, 1.f};
-        if (m >= p.M) continue;
+        if (m >= M) continue;
         const float w = e < p.E ? wts[m * p.E + e] : 1.f;
         float o[4];
 #pragma unroll
@@ -308,7 +309,7 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
           o[i] = w == 0.f ? 0.f
                  : ACT == 2 ? gated_f(g[i], u[i], w, e == p.E, p.form)
                             : gate_act(g[i], p.form.act) * w;
-        *reinterpret_cast<uint2*>((T*)p.y + (long long)m * p.ldy + e * p.ff + col + 4 * lg) =
+        *reinterpret_cast<uint2*>((T*)p.y + (long long)(m0 + m) * p.ldy + e * p.ff + col + 4 * lg) =
             make_uint2(pk2<T>(o[0], o[1]), pk2<T>(o[2], o[3]));
       }
     }
@@ -319,25 +320,29 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
 template <typename T, int RT, int XP, int NW, int D, int ACT = 0>
 hipError_t run(ThinArgs p, int per_cu, hipStream_t st) {
   p.tiles = ACT ? (p.E * p.ff + p.ffs) / 16 : (p.N + 16 * RT - 1) / (16 * RT);
-  const int grid = p.tiles < 256 * per_cu ? p.tiles : 256 * per_cu;
+  const dim3 grid(p.tiles < 256 * per_cu ? p.tiles : 256 * per_cu, (p.M + 8 * XP - 1) / (8 * XP));
   thin_kernel<T, RT, XP, NW, D, ACT><<<grid, 64 * NW, 0, st>>>(p);
   return hipGetLastError();
 }
 
 // The tile.  One 16-row tile per step of four waves (two workgroups share a CU) is best or within 3 %
-// everywhere at M <= 16, except that long rows of a matrix with few tiles want eight waves (2048 x
-// 5632: 8.3 vs 8.4 - 9 us) and the widest long-row matrices want 32-row tiles (22528 x 4096: 31.5 vs
-// 32.8 us, x read half as often).  Above 16 rows x costs as much as W: many tiles take 64 rows per x
-// fragment (11264 x 2048 at M = 64: 15.3 vs 18.7 us with 32), few tiles need the waves on K instead
-// (2048 x 2048: 6.5 us with 16-row tiles of four waves).
+// everywhere at M <= 16, except that long rows of a matrix with few tiles, and few tiles of any kind, want eight waves (2048 x
+// 5632: 8.3 vs 8.4 - 9 us, 256 x 4096: 4.6 vs 5.5) and the widest long-row matrices want 32-row tiles (22528 x 4096: 31.5 vs
+// 32.8 us, x read half as often).  Above 16 rows x costs as much as W: many tiles take all rows of x, 64 to an x
+// fragment (11264 x 2048 at M = 64: 15.3 vs 18.7 us with 32); where that leaves CUs idle the rows are cut into groups of 32 or
+// 16, each with workgroups of its own that hold more of W in flight.  All rows -> groups, us, 64 rows: 128 x 2048 6.1 -> 3.8, 256 x
+// 4096 9.5 -> 4.9 (16 and eight waves; of 32 4.7, 6.9), 2048 x 2048 7.8 -> 6.1, 2048 x 5632 17.1 -> 12.0 (32), 3072 x 2048 8.1 -> 7.5
+// (32, 32-row tiles; 16-row ones 9.6), 4096 x 4096 14.2 -> 13.8, 6144 x 2048 13.3 -> 11.8; 32 rows: 128 x 2048 4.5 -> 3.6, 2048 x 2048
+// 6.2 -> 5.1, 2048 x 5632 12.4 -> 10.3 (16; 3072 x 2048 would go 6.5 -> 7.0).
 template <typename T>
 hipError_t pick(const ThinArgs& p, hipStream_t st) {
-  const bool wide = p.N >= 8192;
+  const bool wide = p.N >= 8192, tiny = p.N <= 256;
   if (p.M <= 8) {
     if (wide && p.K >= 4096) return run<T, 2, 1, 4, 4>(p, 1, st);
-    if (!wide && p.K >= 4608) return run<T, 1, 1, 8, 4>(p, 2, st);
+    if (!wide && (p.K >= 4608 || tiny)) return run<T, 1, 1, 8, 4>(p, 2, st);
     return run<T, 1, 1, 4, 4>(p, 2, st);
   }
+  if (tiny && p.E == 0) return run<T, 1, 2, 8, 4>(p, 1, st);
   if (p.M <= 16) {
     if (wide && p.K >= 4096) return run<T, 2, 2, 4, 4>(p, 1, st);
     return run<T, 1, 2, 4, 4>(p, 2, st);
@@ -345,10 +350,12 @@ hipError_t pick(const ThinArgs& p, hipStream_t st) {
   if (p.M <= 32) {
     if (wide && p.K >= 4096) return run<T, 2, 4, 4, 3>(p, 1, st);
     if (wide) return run<T, 4, 4, 2, 3>(p, 1, st);
+    if (p.N <= 2112 && p.E == 0) return run<T, 1, 2, 4, 4>(p, 2, st);    // rows in groups of 16
     return run<T, 1, 4, 4, 3>(p, 2, st);
   }
   if (wide) return run<T, 4, 8, 2, 3>(p, 1, st);
-  return run<T, 1, 8, 4, 3>(p, 1, st);
+  if (p.N <= 2048) return run<T, 1, 4, 4, 3>(p, 2, st);                  // in groups of 32
+  return run<T, 2, 4, 4, 3>(p, 1, st);
 }
 
 template <typename T>

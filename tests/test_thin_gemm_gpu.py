@@ -142,3 +142,16 @@ def test_one_row_of_a_wide_model_skips_experts():
     # each activation may round to the other side (2^-7 of it at most, two neighbours), then the result rounds
     slack = (a.abs() @ down.double().nan_to_num().abs().t()) * 2.0 ** -7
     assert ((y.double() - ref).abs() <= slack + ref.abs() * 2.0 ** -8).all()
+
+
+@pytest.mark.parametrize("dtype,bits", [(torch.bfloat16, 8), (torch.float16, 11)])
+@pytest.mark.parametrize("M", [9, 17, 31, 33, 49, 64])
+@pytest.mark.parametrize("N,K", [(256, 4096), (260, 192), (2112, 320), (2116, 320), (2052, 128), (5000, 192)])
+def test_rows_in_groups(M, N, K, dtype, bits):
+    """Few tiles: the rows are cut into groups of 16 or 32 with workgroups of their own."""
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x = torch.randn(M, K + 8, device="cuda", generator=g).to(dtype)[:, :K]
+    w = (torch.randn(N, K, device="cuda", generator=g) / K ** 0.5).to(dtype)
+    y, exact = thin_linear(x, w), x.double() @ w.double().t()
+    acc, ulp = bound(x, w, bits)
+    assert ((y.double() - exact).abs() <= acc + exact.abs() * ulp + 1e-30).all()

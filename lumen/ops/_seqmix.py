@@ -76,6 +76,7 @@ SIGNATURES = {
     "sm_row_norm_rotary": "ipl" "ppppppp" "iiiiii" "ff",
     "sm_stream_rms": "ipi" "ppifp" "p" "pppf" "ppi" "iif",
     "sm_head_scan_chunk": "ii" "plplplplpl" "pppp" "pp" "ppp" "iiiiiiff",
+    "sm_head_scan_ahead": "ii" "plplplplpl" "pppp" "pp" "ppp" "iiiiiiff" "pi",
     "sm_head_scan_step": "ii" "plplplplpl" "pppp" "pp" "ppp" "iiiiiiff",
     "sm_short_conv": "iplpppp" "pppp" "iii",
     "sm_conv_tail": "iiplpppp" "ppp" "iii",
@@ -119,6 +120,8 @@ def _load():
         lib.sm_latent_attn_ok.restype = ctypes.c_int
         lib.sm_latent_tiles_ok.argtypes = [ctypes.c_int] * 6
         lib.sm_latent_tiles_ok.restype = ctypes.c_int
+        lib.sm_head_scan_ahead_bytes.argtypes = [ctypes.c_int] * 5
+        lib.sm_head_scan_ahead_bytes.restype = ctypes.c_longlong
         lib.sm_min_gru_sub.argtypes = []
         lib.sm_min_gru_sub.restype = ctypes.c_int
         _lib = lib
@@ -185,6 +188,11 @@ def latent_attn_ok(dt: int, Dv: int, Dk: int, D1: int, bs: int) -> bool:
 def latent_tiles_ok(dt: int, Dv: int, Dk: int, D1: int, bs: int, max_blocks: int) -> bool:
     """Does the latent attention have a kernel that shares key tiles among rows for these sizes?"""
     return bool(_load().sm_latent_tiles_ok(dt, Dv, Dk, D1, bs, max_blocks))
+
+
+def head_scan_ahead_bytes(delta: bool, Dk: int, H: int, rep: int, chunks: int) -> int:
+    """Workspace of the scan whose chunks are built ahead for a step of ``chunks`` chunks; 0: no such kernel."""
+    return int(_load().sm_head_scan_ahead_bytes(int(delta), Dk, H, rep, chunks))
 
 
 def min_gru_sub() -> int:

@@ -269,7 +269,7 @@ def min_gru_scan(zxg: torch.Tensor, b_z: torch.Tensor, b_x: torch.Tensor, state:
 # l = -exp(A_log) dt (the delta rule uses dt in the decay only).  The delta rule first makes q and k
 # unit vectors, x / sqrt(sum x^2 + key_eps), and multiplies q by ``q_scale``.  Decays, step sizes,
 # unit vectors and the state are fp32; the read-out is returned in fp32.
-# (HIP: ``csrc/seqmix/head_scan_chunk.hip`` and, for bf16, ``head_scan_chunk16.hip`` for prompt
+# (HIP: ``csrc/seqmix/head_scan_chunk.hip`` and, for bf16, ``head_scan_chunk16.hip`` and ``head_scan_ahead.hip`` for prompt
 # portions, ``head_scan_step.hip`` for decoded rows.)
 def head_scan_ref(q, k, v, state, seg: SegBatch, H, rep, Dk, Dv, decay, beta=None, skip=None,
                   silu_in=False, key_eps=0.0, q_scale=1.0):
@@ -312,6 +312,14 @@ def head_scan_ref(q, k, v, state, seg: SegBatch, H, rep, Dk, Dv, decay, beta=Non
     return out.reshape(T, H * Dv)
 
 
+# The scan whose chunks are built ahead (head_scan_ahead.hip): where sequences x heads x 32-column blocks leave CUs idle, a chunk of
+# the chain takes 1.7 us instead of 4.4 (delta rule), 1.3 instead of 2.8.  Chunk producers in each workgroup -> ahead, us, width 4096:
+# 1 x 512 rows delta 79 -> 46, constant decays 52 -> 34, state-space 47 -> 36; 1 x 2048 286 -> 135, 187 -> 101, 173 -> 104; 1 x 96 21 -> 18,
+# 15.5 -> 13.6, 15.8 -> 15.3.  Two rounds of workgroups (4 x 512) would go 81 -> 87, 55 -> 72, 67 -> 110, 64 rows a sequence 13.0 -> 13.7.
+AHEAD_MIN_ROWS, AHEAD_MAX_BLOCKS = 96, 256
+AHEAD_MAX_BYTES = 1 << 28        # of its workspace, 0.8 MB a chunk at width 4096
+
+
 def head_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.Tensor,
               seg: SegBatch, H: int, Dk: int, Dv: int, decay, beta=None, skip=None, rep: int = 1,
               silu_in: bool = False, key_eps: float = 0.0, q_scale: float = 1.0) -> torch.Tensor:
@@ -320,7 +328,7 @@ def head_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.Te
     an fp32 tensor [H] of constant log decays, or (logits [T, H], A_log [H], dt_bias [H]).  ``beta``
     [T, H] (write-strength logits) selects the delta rule, without ``skip``.  ``silu_in``: q, k and v
     pass through silu as they are read (q and k rounded to their dtype again).  Returns the read-outs [T, H * Dv] in fp32."""
-    from ._seqmix import DT, call, use_seqmix
+    from ._seqmix import DT, call, head_scan_ahead_bytes, use_seqmix
 
     if H % rep:
         raise ValueError(f"{H} heads do not share q / k in groups of {rep}")
@@ -347,9 +355,18 @@ def head_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.Te
             _ld(al) if al is not None else 0, beta, _ld(beta) if beta is not None else 0, A_log,
             dt_bias, decay if const else None, skip, state, out)
     tail = (H, rep, Dk, Dv, int(bool(silu_in)), key_eps, q_scale)
-    P, _ = seg.portions()
+    P, rows = seg.portions()
     if P:
-        call("sm_head_scan_chunk", *head, seg.cu, seg.slot, seg.start, P, *tail)
+        chunks = (rows + 31 * P) // 32
+        size = 0
+        if (rows >= AHEAD_MIN_ROWS * P and P * H * ((Dv + 31) // 32) <= AHEAD_MAX_BLOCKS and q.dtype == torch.bfloat16
+                and Dv % 8 == 0 and v.data_ptr() % 16 == 0 and 0 < _ld(v) < 1 << 25 and _ld(v) % 8 == 0):
+            size = head_scan_ahead_bytes(beta is not None, Dk, H, rep, chunks)
+        if 0 < size <= AHEAD_MAX_BYTES:
+            ws = torch.empty(size, dtype=torch.uint8, device=q.device)
+            call("sm_head_scan_ahead", *head, seg.cu, seg.slot, seg.start, P, *tail, ws, chunks)
+        else:
+            call("sm_head_scan_chunk", *head, seg.cu, seg.slot, seg.start, P, *tail)
     if seg.S > P:
         call("sm_head_scan_step", *head, seg.cu[P:], seg.slot[P:], seg.start[P:], seg.S - P, *tail)
     return out

@@ -66,6 +66,52 @@ __global__ void __launch_bounds__(kThreads) latent_in_kernel(const InArgs<T> a) 
   for (int c = a.dims + tid; c < a.Dr; c += kThreads) dst[a.R + c] = x[a.R + c];
 }
 
+// 16-bit rows of up to 2048 aligned entries: eight a thread, everything asked for at once (1536 + 512 + 64 entries, 64 rows
+// 3.73 -> 3.12 us, 4096 rows 22.8 -> 19.0)
+template <typename T>
+__global__ void __launch_bounds__(kThreads) latent_in_wide(const InArgs<T> a) {
+  __shared__ float s_red[kThreads / 64];
+  const int t = blockIdx.x, c = 8 * threadIdx.x;
+  const T* zr = a.z + (long long)t * a.ldz;
+  const bool query = blockIdx.y == 1;
+  const long long s = query ? 0 : a.slots[t];
+  const T* x = query ? zr : zr + a.Q;
+  const int n = query ? a.Q : a.R, pr = threadIdx.x;
+  const bool on = c < n, turns = !query && pr < a.dims / 2;
+  float v[8], w[8], ss = 0.f, u0 = 0.f, u1 = 0.f, f = 0.f;
+  load8<T>(x + (on ? c : 0), v);
+  load8<float>((query ? a.wq : a.wn) + (on ? c : 0), w);
+  if (turns) {
+    u0 = to_f32(x[a.R + 2 * pr]);
+    u1 = to_f32(x[a.R + 2 * pr + 1]);
+    f = (float)a.positions[t] * a.inv_freq[pr];
+  }
+  if (s < 0) return;                                   // (the whole workgroup)
+#pragma unroll
+  for (int e = 0; e < 8; ++e) ss += on ? v[e] * v[e] : 0.f;
+  const float inv = 1.f / sqrtf(block_sum<kThreads>(ss, s_red) / (float)n + a.eps);
+  T* dst = query ? a.qn + (long long)t * a.Q : a.cache + s * (a.R + a.Dr);
+  if (on) {
+    T o[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = from_f32<T>(v[e] * inv * w[e]);
+    *reinterpret_cast<uint4*>(dst + c) = *reinterpret_cast<const uint4*>(o);
+    if (!query && a.vt) {
+      T* dt = a.vt + (s / a.bs) * (long long)a.R * a.bs + s % a.bs;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) dt[(long long)(c + e) * a.bs] = o[e];
+    }
+  }
+  if (query) return;
+  if (turns) {
+    float sn, cs;
+    sincosf(f, &sn, &cs);
+    dst[a.R + 2 * pr] = from_f32<T>(u0 * cs - u1 * sn);
+    dst[a.R + 2 * pr + 1] = from_f32<T>(u1 * cs + u0 * sn);
+  }
+  for (int i = a.dims + threadIdx.x; i < a.Dr; i += kThreads) dst[a.R + i] = x[a.R + i];
+}
+
 template <typename T> struct QueryArgs {
   T* q; long long ldq; int ldh;             // rows; head h of a row at column h * ldh
   const T* w;                               // [H][R][D]
@@ -204,6 +250,19 @@ hipError_t sm_latent_in(int dt, const void* z, long long ldz, const float* wq, v
   if (rows == 0) return hipSuccess;
   if (rows < 0 || Q < 1 || R < 1 || Dr < 0 || dims < 0 || dims % 2 || dims > Dr || bs < 1 || ldz < Q + R + Dr)
     return hipErrorInvalidValue;
+  const auto al = [](const void* p) { return (uintptr_t)p % 16 == 0; };
+  const bool wide = dt != kF32 && Q % 8 == 0 && R % 8 == 0 && Dr % 8 == 0 && Q <= 8 * kThreads && R <= 8 * kThreads &&
+                    dims / 2 <= kThreads && ldz % 8 == 0 && al(z) && al(wq) && al(wn) && al(qn) && al(cache);
+  if (wide) {
+#define WIDE(T)                                                                                                 \
+  latent_in_wide<T><<<dim3(rows, 2), kThreads, 0, st>>>(InArgs<T>{(const T*)z, ldz, wq, wn, inv_freq, positions, \
+                                                          slots, (T*)cache, (T*)vt, (T*)qn, bs, Q, R, Dr, dims, eps})
+    if (dt == kBF16) WIDE(bf16);
+    else if (dt == kF16) WIDE(fp16);
+    else return hipErrorInvalidValue;
+#undef WIDE
+    return hipGetLastError();
+  }
 #define CALL(T)                                                                                                 \
   latent_in_kernel<T><<<dim3(rows, 2), kThreads, 0, st>>>(InArgs<T>{(const T*)z, ldz, wq, wn, inv_freq, positions, \
                                                             slots, (T*)cache, (T*)vt, (T*)qn, bs, Q, R, Dr, dims, eps})

@@ -155,6 +155,63 @@ gated_rms_kernel(const float* __restrict__ x, const T* __restrict__ g, long long
   }
 }
 
+// The same for aligned groups of at most N x 256 entries a wave, in registers: values, gates and weights are asked for together, as
+// a decoded row costs the chain of its loads (launch after launch, one group: one row of 2048 3.38 -> 2.82 us, of 4096 4.72 -> 3.60;
+// 4096 rows of 2048 15.7 -> 14.6).
+template <typename T, int N>
+__global__ void __launch_bounds__(256)
+gated_rms_wide_kernel(const float* __restrict__ x, const T* __restrict__ g, long long ldg, const float* __restrict__ w,
+                      T* __restrict__ out, int W, int groups, int shared_w, int gate_first, int sigmoid, float eps) {
+  __shared__ float s_part[4];
+  const int r = blockIdx.x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int gs = W / groups;
+  const int wpg = groups >= 4 ? 1 : groups == 1 ? 4 : groups == 2 ? 2 : 1;   // waves per group
+  const int per_pass = 4 / wpg, slot = wv / wpg, sub = wv % wpg;
+  const int gi = blockIdx.y * per_pass + slot;
+  const bool on = gi < groups && slot < per_pass;
+  Raw4<float> x4[N], w4[N];
+  Raw4<T> g4[N];
+  float v[N][4], z[N][4], ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {                // (no branch: entries past the group's end read the row's first)
+    const int c0 = 4 * (lane + 64 * (sub + wpg * i)), c = on && c0 < gs ? c0 : 0, col = on && c0 < gs ? gi * gs + c0 : 0;
+    x4[i].ask(x + (long long)r * W + col);
+    g4[i].ask(g + (long long)r * ldg + col);
+    w4[i].ask(w + (shared_w ? c : col));
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    x4[i].get(v[i]);
+    g4[i].get(z[i]);
+    const bool in = on && 4 * (lane + 64 * (sub + wpg * i)) < gs;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (!in) v[i][e] = 0.f;
+      z[i][e] = sigmoid ? sigmoid_f(z[i][e]) : silu_f(z[i][e]);
+      if (gate_first) v[i][e] *= z[i][e];
+      ss += in ? v[i][e] * v[i][e] : 0.f;
+    }
+  }
+  float tot = wave_sum(ss);
+  if (wpg > 1) {                             // (uniform) waves sharing a group exchange their sums
+    if (lane == 0) s_part[wv] = tot;
+    __syncthreads();
+    tot = 0.f;
+    for (int k = 0; k < wpg; ++k) tot += s_part[slot * wpg + k];
+  }
+  const float inv = 1.f / sqrtf(tot / (float)gs + eps);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int c = 4 * (lane + 64 * (sub + wpg * i)), col = gi * gs + c;
+    if (!on || c >= gs) continue;
+    float ww[4];
+    w4[i].get(ww);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[i][e] = v[i][e] * inv * ww[e] * (gate_first ? 1.f : z[i][e]);
+    store4<T>(out + (long long)r * W + col, v[i]);
+  }
+}
+
 // groups of at most 256 entries (heads): SG lanes of 4 entries each own a (row, group), in registers
 template <typename T>
 __global__ void __launch_bounds__(256)
@@ -202,13 +259,75 @@ __global__ void gate_rows_kernel(const T* __restrict__ z, long long ldz, const T
   }
 }
 
+// The same for groups of at most N x 256 aligned entries a wave, in registers: a workgroup per row and pass over the groups, values,
+// weights and the residual asked for together (launch after launch: 64 rows of 2048, one group 3.27 -> 2.82 us, 16 groups 5.50 -> 2.32;
+// 4096 rows 16.1 -> 15.8, 20.0 -> 17.8).
+template <typename TI, typename TO, int N>
+__global__ void __launch_bounds__(256)
+group_rms_held(const TI* __restrict__ x, long long ldx, const float* __restrict__ w, float* __restrict__ res,
+               TO* __restrict__ out, long long ldo, int W, int groups, float eps) {
+  __shared__ float s_part[4];
+  const int r = blockIdx.x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int gs = W / groups;
+  const int wpg = groups >= 4 ? 1 : groups == 1 ? 4 : groups == 2 ? 2 : 1;   // waves per group
+  const int slot = wv / wpg, sub = wv % wpg, g = blockIdx.y * (4 / wpg) + slot;
+  const bool on = g < groups;
+  Raw4<TI> x4[N];
+  Raw4<float> w4[N], a4[N];
+  float v[N][4], ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {                // (no branch: entries past the group's end read the row's first)
+    const int c = 4 * (lane + 64 * (sub + wpg * i)), col = on && c < gs ? g * gs + c : 0;
+    x4[i].ask(x + (long long)r * ldx + col);
+    w4[i].ask(w + col);
+    a4[i].v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (res) a4[i].ask(res + (long long)r * W + col);
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    x4[i].get(v[i]);
+    const bool in = on && 4 * (lane + 64 * (sub + wpg * i)) < gs;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss += in ? v[i][e] * v[i][e] : 0.f;
+  }
+  float tot = wave_sum(ss);
+  if (wpg > 1) {                             // (uniform) waves sharing a group exchange their sums
+    if (lane == 0) s_part[wv] = tot;
+    __syncthreads();
+    tot = 0.f;
+    for (int k = 0; k < wpg; ++k) tot += s_part[slot * wpg + k];
+  }
+  const float inv = 1.f / sqrtf(tot / (float)gs + eps);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int c = 4 * (lane + 64 * (sub + wpg * i)), col = g * gs + c;
+    if (!on || c >= gs) continue;
+    float ww[4], a[4];
+    w4[i].get(ww);
+    a4[i].get(a);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[i][e] = res ? v[i][e] * inv * ww[e] + a[e] : v[i][e] * inv * ww[e];
+    if (res) store4<float>(res + (long long)r * W + col, v[i]);
+    if (out) store4<TO>(out + (long long)r * ldo + col, v[i]);
+  }
+}
+
 template <typename TI, typename TO>
 hipError_t launch_rms(const void* x, long long ldx, const float* w, float* res, void* out,
                       long long ldo, int rows, int W, int groups, float eps, hipStream_t st) {
   const int gs = W / groups;
   const bool vec = gs % 4 == 0 && ldx % 4 == 0 && ldo % 4 == 0 &&
                    ((uintptr_t)x % 16 == 0) && ((uintptr_t)out % 16 == 0);
-  if (vec)
+  const int wpg = groups >= 4 ? 1 : groups == 1 ? 4 : groups == 2 ? 2 : 1;
+  const int parts = (gs + 256 * wpg - 1) / (256 * wpg), passes = (groups * wpg + 3) / 4;   // parts: 256 entries of a group a wave
+  const dim3 grid(rows, passes);
+  if (vec && passes <= 65535 && parts <= 1)
+    group_rms_held<TI, TO, 1><<<grid, 256, 0, st>>>((const TI*)x, ldx, w, res, (TO*)out, ldo, W, groups, eps);
+  else if (vec && passes <= 65535 && parts <= 2)
+    group_rms_held<TI, TO, 2><<<grid, 256, 0, st>>>((const TI*)x, ldx, w, res, (TO*)out, ldo, W, groups, eps);
+  else if (vec && passes <= 65535 && parts <= 4)
+    group_rms_held<TI, TO, 4><<<grid, 256, 0, st>>>((const TI*)x, ldx, w, res, (TO*)out, ldo, W, groups, eps);
+  else if (vec)
     group_rms_kernel<TI, TO, true><<<rows, 256, 0, st>>>((const TI*)x, ldx, w, res, (TO*)out, ldo,
                                                          W, groups, eps);
   else
@@ -263,6 +382,9 @@ hipError_t sm_gated_rms(int dt, const float* x, const void* g, long long ldg, co
                    (uintptr_t)g % 16 == 0 && (uintptr_t)out % 16 == 0;
   const int gs = W / groups;
   const bool small = vec && gs <= 256 && (uintptr_t)w % 16 == 0 && W % 4 == 0;
+  const int wave_per = groups >= 4 ? 1 : groups == 1 ? 4 : groups == 2 ? 2 : 1, passes = (gs + 256 * wave_per - 1) / (256 * wave_per);
+  // (one pass leaves waves without an entry: many rows of 512, one group, 7.0 us through LDS, 7.6 in registers)
+  const bool wide = vec && (uintptr_t)w % 16 == 0 && (rows <= 1024 || passes > 1);
   int SG = 1;
   while (4 * SG < gs) SG <<= 1;
   const long long items = (long long)rows * groups;
@@ -271,6 +393,15 @@ hipError_t sm_gated_rms(int dt, const float* x, const void* g, long long ldg, co
   if (small)                                                                                    \
     gated_rms_small_kernel<TT><<<blocks, 256, 0, st>>>(x, (const TT*)g, ldg, w, (TT*)out, W,    \
                                 groups, gs, SG, items, shared_w, gate_first, sigmoid, eps);     \
+  else if (wide && passes <= 1)                                                                 \
+    gated_rms_wide_kernel<TT, 1><<<grid, 256, 0, st>>>(x, (const TT*)g, ldg, w, (TT*)out, W,    \
+                                groups, shared_w, gate_first, sigmoid, eps);                    \
+  else if (wide && passes <= 2)                                                                 \
+    gated_rms_wide_kernel<TT, 2><<<grid, 256, 0, st>>>(x, (const TT*)g, ldg, w, (TT*)out, W,    \
+                                groups, shared_w, gate_first, sigmoid, eps);                    \
+  else if (wide && passes <= 4)                                                                 \
+    gated_rms_wide_kernel<TT, 4><<<grid, 256, 0, st>>>(x, (const TT*)g, ldg, w, (TT*)out, W,    \
+                                groups, shared_w, gate_first, sigmoid, eps);                    \
   else if (vec) gated_rms_kernel<TT, true><<<grid, 256, lds, st>>>(x, (const TT*)g, ldg, w, (TT*)out, \
                                                 W, groups, shared_w, gate_first, sigmoid, eps); \
   else gated_rms_kernel<TT, false><<<grid, 256, lds, st>>>(x, (const TT*)g, ldg, w, (TT*)out, W, \

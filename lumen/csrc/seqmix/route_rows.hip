@@ -8,8 +8,11 @@
 //                   sm_route_topk (groups = 0) or sm_route_groups form them.
 //
 // For a few rows each of these was a launch of 4 - 6 us for a few KB.  A workgroup of eight waves takes a row; a wave
-// takes every eighth expert, whose first row it asks for before the norm; the logits meet in LDS and one wave routes.
+// takes every eighth expert, whose first rows (two up to width 4096) it asks for before the norm, as it does for all that the norm
+// takes; the logits meet in LDS and one wave routes.
 // Every row reads the router again (64 KB from L2), which 64 rows still hide.
+// All of the norm's operands are asked for before its sum, and few experts are ranked by counting (route.h): one row of 2048, 8
+// experts 5.2 -> 4.1 us, 16 experts 5.6 -> 4.7.
 // Measured as a decode step's time (bf16, width 2048): one row, three layers of 16 experts 296.6 -> 284.0 us; eight rows,
 // two layers of 8 experts 375.8 -> 368.6.
 #include "route.h"
@@ -58,36 +61,47 @@ __global__ void __launch_bounds__(kThreads) route_rows_kernel(const RouteArgs<T>
   __shared__ float s_z[kMaxE], s_c[2 * kMaxE], s_red[kWaves];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), W = a.W;
   const long long row = blockIdx.x;
-  uint4 r[KS];
-  const auto ask = [&](int e) __attribute__((always_inline)) {
+  constexpr int B = KS <= 8 && (KS <= 4 || std::is_same<T, bf16>::value) ? 2 : 1;   // a wave's experts at a time: what registers hold
+  uint4 r[B][KS];
+  const auto ask = [&](int e, uint4 (&o)[KS]) __attribute__((always_inline)) {
+    if (e >= a.E) return;
 #pragma unroll
     for (int u = 0; u < KS; ++u) {
       const int c = 512 * u + 8 * lane;
-      r[u] = c < W ? *reinterpret_cast<const uint4*>(a.R + (long long)e * W + c) : make_uint4(0, 0, 0, 0);
+      o[u] = c < W ? *reinterpret_cast<const uint4*>(a.R + (long long)e * W + c) : make_uint4(0, 0, 0, 0);
     }
   };
-  if (w < a.E) ask(w);
+#pragma unroll
+  for (int b = 0; b < B; ++b) ask(w + b * kWaves, r[b]);
   if constexpr (KIND > 0) {
     constexpr int N = (KS * 512 + 4 * kThreads - 1) / (4 * kThreads);
-    float v[N][4], sq = 0.f;
+    float v[N][4], y[N][4], nw[N][4], nb[N][4], pw[N][4], pb[N][4], sq = 0.f;
+    Raw4<T> y4[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {                        // (no branch: past the row's end, its first channels again)
+      const int c0 = 4 * (threadIdx.x + i * kThreads), c = c0 < W ? c0 : 0;
+      load4<float>(a.x + row * W + c, v[i]);
+      y4[i].ask(a.y + row * W + c);
+      load4<float>(a.w + c, nw[i]);
+      if constexpr (KIND == 2) {
+        load4<float>(a.pw + c, pw[i]);
+        load4<float>(a.pb + c, pb[i]);
+        load4<float>(a.b + c, nb[i]);
+      }
+    }
     const float ap = KIND == 2 ? *a.pa : 0.f, an = KIND == 2 ? *a.alpha : 0.f;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const int c = 4 * (threadIdx.x + i * kThreads);
       if (c >= W) break;
-      float y[4];
-      load4<float>(a.x + row * W + c, v[i]);
-      load4<T>(a.y + row * W + c, y);
+      y4[i].get(y[i]);
       if constexpr (KIND == 2) {
-        float pw[4], pb[4];
-        load4<float>(a.pw + c, pw);
-        load4<float>(a.pb + c, pb);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) y[e] = dyt_f(y[e], ap, pw[e], pb[e]);
+        for (int e = 0; e < 4; ++e) y[i][e] = dyt_f(y[i][e], ap, pw[i][e], pb[i][e]);
       }
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        v[i][e] += y[e];
+        v[i][e] += y[i][e];
         sq += v[i][e] * v[i][e];
       }
       store4<float>(a.x + row * W + c, v[i]);
@@ -98,17 +112,9 @@ __global__ void __launch_bounds__(kThreads) route_rows_kernel(const RouteArgs<T>
     for (int i = 0; i < N; ++i) {
       const int c = 4 * (threadIdx.x + i * kThreads);
       if (c >= W) break;
-      float nw[4];
-      load4<float>(a.w + c, nw);
-      if constexpr (KIND == 1) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[i][e] = v[i][e] * inv * nw[e];
-      } else {
-        float nb[4];
-        load4<float>(a.b + c, nb);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[i][e] = dyt_f(v[i][e], an, nw[e], nb[e]);
-      }
+      for (int e = 0; e < 4; ++e)
+        v[i][e] = KIND == 1 ? v[i][e] * inv * nw[i][e] : dyt_f(v[i][e], an, nw[i][e], nb[i][e]);
       store4<T>(a.h + row * a.ldh + c, v[i]);
       store4<T>(s_h + c, v[i]);
     }
@@ -121,13 +127,24 @@ __global__ void __launch_bounds__(kThreads) route_rows_kernel(const RouteArgs<T>
     x[u] = make_uint4(0, 0, 0, 0);
     if (c < W) x[u] = *reinterpret_cast<const uint4*>(KIND > 0 ? s_h + c : a.h + row * a.ldh + c);
   }
-  for (int e = w; e < a.E; e += kWaves) {
-    float s[2] = {0.f, 0.f};
+  for (int e = w; e < a.E; e += B * kWaves) {
+    float z[B];
 #pragma unroll
-    for (int u = 0; u < KS; ++u) s[u & 1] = dot8<T>(r[u], x[u], s[u & 1]);
-    if (e + kWaves < a.E) ask(e + kWaves);
-    const float z = wave_sum(s[0] + s[1]);
-    if (lane == 0) s_z[e] = z + (a.bias != nullptr ? to_f32(a.bias[e]) : 0.f);
+    for (int b = 0; b < B; ++b) {
+      float s[2] = {0.f, 0.f};
+      if (e + b * kWaves < a.E) {
+#pragma unroll
+        for (int u = 0; u < KS; ++u) s[u & 1] = dot8<T>(r[b][u], x[u], s[u & 1]);
+      }
+      z[b] = s[0] + s[1];
+      ask(e + (B + b) * kWaves, r[b]);
+    }
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const int f = e + b * kWaves;
+      z[b] = wave_sum(z[b]);
+      if (lane == 0 && f < a.E) s_z[f] = z[b] + (a.bias != nullptr ? to_f32(a.bias[f]) : 0.f);
+    }
   }
   __syncthreads();
   if (w != 0) return;

@@ -76,6 +76,19 @@ template <> __device__ __forceinline__ void load4<float>(const float* __restrict
   const float4 a = *reinterpret_cast<const float4*>(p);
   o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w;
 }
+// the same asked for now and converted where it is used: a conversion waits for its load, also under a branch not yet left
+template <typename T> struct Raw4 {
+  uint2 v;
+  __device__ __forceinline__ void ask(const T* __restrict__ p) { v = *reinterpret_cast<const uint2*>(p); }
+  __device__ __forceinline__ void put(T* __restrict__ p) const { *reinterpret_cast<uint2*>(p) = v; }
+  __device__ __forceinline__ void get(float (&o)[4]) const { load4<T>(reinterpret_cast<const T*>(&v), o); }
+};
+template <> struct Raw4<float> {
+  float4 v;
+  __device__ __forceinline__ void ask(const float* __restrict__ p) { v = *reinterpret_cast<const float4*>(p); }
+  __device__ __forceinline__ void put(float* __restrict__ p) const { *reinterpret_cast<float4*>(p) = v; }
+  __device__ __forceinline__ void get(float (&o)[4]) const { o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w; }
+};
 template <typename T> __device__ __forceinline__ void store4(T* __restrict__ p, const float (&v)[4]) {
   *reinterpret_cast<uint2*>(p) = make_uint2(pk2<T>(v[0], v[1]), pk2<T>(v[2], v[3]));
 }

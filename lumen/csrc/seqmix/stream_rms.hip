@@ -10,8 +10,9 @@
 //                 x, f0, f1, f2 are fp32; y and the embedding table are in the compute dtype.  With
 //                 `rows` the token's table row is also copied out as it is (a GEMM's operand).
 //
-// One workgroup per row, four channels per lane; the new row stays in LDS between the sum of squares
-// and the output.
+// One workgroup per row, four channels per lane.  Rows of up to 4096 aligned channels stay in registers, and everything that the row
+// takes, the norm's weight too, is asked for before the first sum: a decoded row costs its chain of loads (bf16,
+// launch after launch: one row of 2048 3.03 -> 2.72 us, of 4096 4.08 -> 3.29; 4096 rows of 2048 20.9 -> 20.4).  Other rows stay in LDS between the sum of squares and the output.
 #include "seqmix.h"
 
 using namespace lumen;
@@ -109,6 +110,86 @@ __global__ void __launch_bounds__(kThreads) stream_rms_kernel(const StreamArgs<T
   }
 }
 
+// N: 1024-channel parts of a row
+template <typename T, int N>
+__global__ void __launch_bounds__(kThreads) stream_row_kernel(const StreamArgs<T> a) {
+  __shared__ float s_red[kThreads / 64];
+  const int W = a.W;
+  const long long base = (long long)blockIdx.x * W;
+  const T* er = nullptr;
+  if (a.table != nullptr) {
+    long long tok = a.tokens[blockIdx.x];
+    tok = tok < 0 ? 0 : (tok >= a.vocab ? a.vocab - 1 : tok);
+    er = a.table + tok * W;
+  }
+  Raw4<float> x4[N], f0[N], f1[N], f2[N], w4[N];
+  Raw4<T> e4[N], y4[N];
+  const auto each = [&](auto&& f) __attribute__((always_inline)) {      // (past the row's end: its first channels again)
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int c = 4 * (threadIdx.x + i * kThreads);
+      f(i, c < W ? c : 0);
+    }
+  };
+  if (a.keep) each([&](int i, int c) { x4[i].ask(a.x + base + c); });
+  if (a.y != nullptr) each([&](int i, int c) { y4[i].ask(a.y + base + c); });
+  if (a.f0 != nullptr) each([&](int i, int c) { f0[i].ask(a.f0 + base + c); });
+  if (a.f1 != nullptr) each([&](int i, int c) { f1[i].ask(a.f1 + base + c); });
+  if (a.f2 != nullptr) each([&](int i, int c) { f2[i].ask(a.f2 + base + c); });
+  if (a.w != nullptr) each([&](int i, int c) { w4[i].ask(a.w + c); });
+  if (er != nullptr) each([&](int i, int c) { e4[i].ask(er + c); });
+  float v[N][4], sq = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int c = 4 * (threadIdx.x + i * kThreads);
+    if (c >= W) break;
+    const auto add = [&](const auto& r, float k) __attribute__((always_inline)) {
+      float o[4];
+      r.get(o);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[i][e] += k * o[e];
+    };
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[i][e] = 0.f;
+    if (a.keep) x4[i].get(v[i]);
+    if (er != nullptr) {
+      if (a.rows != nullptr) e4[i].put(a.rows + base + c);
+      add(e4[i], a.scale);
+    }
+    if (a.y != nullptr) add(y4[i], 1.f);
+    if (a.f0 != nullptr) add(f0[i], 1.f);
+    if (a.f1 != nullptr) add(f1[i], 1.f);
+    if (a.f2 != nullptr) add(f2[i], a.coef);
+    store4<float>(a.x + base + c, v[i]);
+    if (a.w != nullptr) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sq += v[i][e] * v[i][e];
+    } else if (a.split) {
+      float lo[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float hi = to_f32(from_f32<T>(v[i][e]));
+        lo[e] = v[i][e] - hi;
+        v[i][e] = hi;
+      }
+      store4<T>(a.h + base + c, v[i]);
+      store4<T>(a.h + a.lo + base + c, lo);
+    }
+  }
+  if (a.w == nullptr) return;
+  const float inv = 1.f / sqrtf(block_sum<kThreads>(sq, s_red) / (float)W + a.eps);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int c = 4 * (threadIdx.x + i * kThreads);
+    if (c >= W) break;
+    float ww[4];
+    w4[i].get(ww);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[i][e] = v[i][e] * inv * ww[e];
+    store4<T>(a.h + base + c, v[i]);
+  }
+}
+
 }  // namespace
 
 extern "C" {
@@ -132,7 +213,10 @@ hipError_t sm_stream_rms(int dt, float* x, int keep, const void* table, const lo
   {                                                                                               \
     StreamArgs<T> a{x, keep, (const T*)table, tokens, vocab, scale, (T*)table_rows, (const T*)y,  \
                     f0, f1, f2, coef, w, (T*)h, split, (long long)rows * W, W, eps};              \
-    if (vec) stream_rms_kernel<T, 4><<<rows, kThreads, lds, st>>>(a);                             \
+    if (vec && W <= 1024) stream_row_kernel<T, 1><<<rows, kThreads, 0, st>>>(a);                  \
+    else if (vec && W <= 2048) stream_row_kernel<T, 2><<<rows, kThreads, 0, st>>>(a);             \
+    else if (vec && W <= 4096) stream_row_kernel<T, 4><<<rows, kThreads, 0, st>>>(a);             \
+    else if (vec) stream_rms_kernel<T, 4><<<rows, kThreads, lds, st>>>(a);                        \
     else stream_rms_kernel<T, 1><<<rows, kThreads, lds, st>>>(a);                                 \
   }
   SM_DISPATCH(dt, CALL)

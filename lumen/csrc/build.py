@@ -43,7 +43,7 @@ def ext_path() -> str:
 # 318 -> 293 (delta, 8 x 512 tokens, of its four-wave form).
 # The others are equal or slower (row_attention.hip's latent_attn_kernel 24.6 -> 32.1 us).
 MFMA_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
-MFMA_FORM_FILES = ("lora_v3.hip", "head_scan_chunk16.hip", "head_scan_ahead.hip", "recurrent_chunk.hip", "expert_gemm.hip")
+MFMA_FORM_FILES = ("lora_v3.hip", "head_scan_chunk16.hip", "head_scan_ahead.hip", "recurrent_chunk.hip")
 
 
 # no packed-fp32 instructions (v_pk_*_f32): scalar fp32 code only

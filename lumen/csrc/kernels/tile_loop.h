@@ -109,10 +109,11 @@ __device__ __forceinline__ int colperm(int w) {
 // acc[i][j] = products of fragments i of w and j of x over nk stages (64 k each) from xb and wb, to which off[q] is the
 // lane's byte offset of the wave's piece q: stage rows 8 (wid + 4 q) + lane / 8 of x for q < MJ, of w from piece MJ on, chunk
 // (lane & 7) ^ swz(row).  APART: the walk starts at stage `turn` < nk and comes round to it.  Lane (lr, lg) holds row 16 j + lr of its
-// wave's x, rows 16 i + 4 lg .. + 3 of its w.
-template <typename T, int NI, int MJ, bool APART = false>
+// wave's x, rows 16 i + 4 lg .. + 3 of its w.  HALF: with `odd` the last stage holds 32 k; its lanes of the upper half read the lower
+// one again, which is multiplied once.
+template <typename T, int NI, int MJ, bool APART = false, bool HALF = false>
 __device__ __forceinline__ void products(char* lds, const char* xb, const char* wb, int nk, int turn,
-                                         const unsigned (&off)[Shape<NI, MJ>::PIECES], f32x4 (&acc)[NI][MJ]) {
+                                         const unsigned (&off)[Shape<NI, MJ>::PIECES], f32x4 (&acc)[NI][MJ], bool odd = false) {
   using S = Shape<NI, MJ>;
   constexpr int NSX = S::NSX, NST = S::NST, XB = S::XB, WB = S::WB, PIECES = S::PIECES;
   // pieces [PB, PIECES) of a stage go out behind a second half's products, [0, PB) behind the first half's
@@ -121,13 +122,15 @@ __device__ __forceinline__ void products(char* lds, const char* xb, const char* 
   const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const unsigned lds0 = (unsigned)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds);
+  const unsigned upper = HALF && odd && (((lane >> 2) ^ wid) & 1) ? BK : 0;     // (bytes; chunk (lane & 7) ^ swz(row) >= 4)
   auto issue = [&](int t, Slot slot, int q0, int q1) __attribute__((always_inline)) {
+    const unsigned back = HALF && t == nk - 1 ? upper : 0;
     const int u = APART ? (t + turn < nk ? t + turn : t + turn - nk) : t;
     const char *xs = xb + (long long)u * (BK * 2), *ws = wb + (long long)u * (BK * 2);
     const unsigned dx = __builtin_amdgcn_readfirstlane(lds0 + slot.x * XB + wid * 1024);
     const unsigned dw = __builtin_amdgcn_readfirstlane(lds0 + NSX * XB + slot.w * WB + wid * 1024);
 #pragma unroll
-    for (int q = q0; q < q1; ++q) dma16(q < MJ ? xs : ws, off[q], q < MJ ? dx + q * 4096 : dw + (q - MJ) * 4096);
+    for (int q = q0; q < q1; ++q) dma16(q < MJ ? xs : ws, HALF ? off[q] - back : off[q], q < MJ ? dx + q * 4096 : dw + (q - MJ) * 4096);
   };
 #pragma unroll
   for (int i = 0; i < NI; ++i)
@@ -191,7 +194,7 @@ __device__ __forceinline__ void products(char* lds, const char* xb, const char* 
     half(0, s0, t + F < nk ? t + F : -1, sf, 0, PB);
     wait_stages<NST == 2 ? 0 : F - 1, PIECES>(nk - 2 - t);
     done_reading();
-    half(1, s1, -1, s1, 0, 0);                           // (the last step reads a slot that holds an earlier stage: unused)
+    if (!HALF || !odd || t + 1 < nk) half(1, s1, -1, s1, 0, 0);      // (the last step reads a slot that holds an earlier stage: unused)
     s0 = s1, s1 = after(s1), sf = after(sf);
   }
   settle();

@@ -6,41 +6,32 @@
 //   sm_expert_sum     out[t] = the sum of the row's pairs in expert order and of its shared result, rounded once
 //
 // The dense form (two library products over ALL experts, ops/moe.py) does E / top times the work; the library's
-// grouped product runs at 300 TFLOP/s.  Here a workgroup takes 128 pairs of one expert and 256 rows of its weights,
-// both products on a loop like that of kernels/tile_loop.h (three LDS stages of 64 k by LDS-DMA under counted waits, one
-// barrier a step, four waves of 64 pairs x 128 weight rows):
+// grouped product runs at 300 TFLOP/s.  Here a workgroup takes 64, 128 or 256 pairs of one expert and 256 rows of its weights,
+// both products on the loop of kernels/tile_loop.h:
 //  * the rows of a tile are gathered by the DMA's source addresses; no sorted copy of h exists;
-//  * a wave's 128 weight rows of the first product are 64 gate rows and their 64 up rows, so the activation with the
-//    routing weight is formed from the fp32 sums and the [pairs, 2 ff] intermediate is never stored;
+//  * a wave's weight rows of the first product are alternating fragments of 16 gate rows and their 16 up rows, so the activation
+//    with the routing weight is formed from the fp32 sums and the [pairs, 2 ff] intermediate is never stored;
 //  * counts stay on the device: the grid is sized for the most tiles the step can have and the surplus leaves at once.
 //    Nothing synchronises, nothing depends on host-visible counts (a capture may hold it);
-//  * XCDs take consecutive tiles, an expert's row tiles within a weight panel first: a panel comes from HBM once.
-// Bound by the loop at one wave per SIMD (1.0 us a step where kernels/tile_loop.h takes 0.7: an expert's pairs are
-// fetched again for every few panels) and by each tile's own prologue and epilogue; under ~200 rows by reading the
-// weights once.  Measured (us, a whole layer of experts, dense form -> here; bf16, width 2048, experts of 1408, weights that
-// the last-level cache holds; ops/moe.py has few rows with weights from HBM): 8 experts, top 2, and a shared one: 4096 rows
-// 534 -> 283, 512 90 -> 60, 256 62 -> 56; 16, top 3, shared: 4096 1130 -> 371, 512 166 -> 99, 64 149 -> 79; 16 ungated,
-// top 4: 4096 810 -> 298, 8192 at width 4096 2721 (grouped library product) -> 1685.  Error against float64 2.3e-3 where the dense form has 3.5e-3: nothing is rounded between the
-// products and the activation, nor before the sum.
+//  * XCDs take consecutive tiles, an expert's row tiles within a weight panel first: a panel comes from HBM once;
+//  * a tile occupies its CU, so the time goes by whole rounds of 256 tiles: tiles of 256 pairs run whole rounds, and what is
+//    left over, known on the device, is cut into two or four smaller tiles each where those make one round.
+// Bound by the rounds: a tile of 256 x 256 takes 1.25 us a stage of 64 k, as in the dense products, and 11 us around them (first
+// stages, activation, stores); under ~200 rows by reading the weights once.  Measured (us, a whole layer of experts, weights from
+// HBM, bf16; tiles of 128 pairs alone, on a loop of their own -> here): width 2048, 8 experts of 1408, top 2, and a
+// shared one: 4096 rows 294 -> 247, 2048 172 -> 141, 512 77 -> 74, 160 70 -> 66; 16, top 3, shared: 4096 373 -> 336, 1024 148 ->
+// 127, 256 91 -> 87, 64 84 -> 82; 16 ungated, top 4: 4096 298 -> 251; width 4096, 16 of 2816, top 4: 8192 rows 2370 -> 2026, 300
+// 257 -> 258; dense form: 4096 rows of the first 534, of the second 1130.  Error against float64 2.3e-3 where the dense form has
+// 3.5e-3: nothing is rounded between the products and the activation, nor before the sum.
 #include "mma.h"
+#include "../kernels/tile_loop.h"
 
 using namespace lumen;
 
 namespace {
 
-constexpr int BM = 128, BN = 256, BK = 64, ROWB = 128;   // pairs, weight rows; a stage row is 64 elements
-constexpr int NI = 8, MJ = 4;                            // fragments of a wave: 128 weight rows x 64 pairs
-constexpr int XB = BM * ROWB, STAGE = (BM + BN) * ROWB;  // [pairs | weights]
-constexpr int XP = BM / 32, PIECES = (BM + BN) / 32;     // 1-KiB LDS-DMA pieces of a wave and stage (x's first)
+constexpr int BN = 256, BK = tile::BK;                   // weight rows of a tile
 constexpr int kMaxE = 64;
-
-__device__ __forceinline__ int swz(int r) { return (r >> 1) & 7; }
-
-__device__ __forceinline__ void done_reading() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
 
 struct ExpertArgs {
   const void *x, *xs;          // rows of the experts' (gathered) and of the shared expert's product
@@ -58,49 +49,123 @@ struct ExpertArgs {
 // sigmoid on the exponential and reciprocal units (the results are rounded to 16 bits)
 __device__ __forceinline__ float sigmoid_fast(float x) { return __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
 
-// activation results of pair fragment j: columns of a lane's accumulators (acc[i]: gate, acc[NI / 2 + i]: up)
-template <typename T, int MODE, int ACT>
-__device__ __forceinline__ void put_row(const GateForm& f, const f32x4 (&acc)[NI][MJ], int j, T* o, int c0, int ff,
+// MODE 0: column (of 64) of row r of a wave's 128 weight rows, alternating fragments of 16 gate and their 16 up rows; a
+// lane's fragments of two such pairs hold 8 consecutive columns
+__device__ __forceinline__ int gate_col(int r) {
+  return 32 * (r >> 6) + 8 * ((r >> 2) & 3) + 4 * ((r >> 5) & 1) + (r & 3);
+}
+
+// activation results of pair fragment j (MODE 0: acc[even]: gate, acc[odd]: up)
+template <typename T, int MODE, int NI, int MJ, int ACT>
+__device__ __forceinline__ void put_row(const GateForm& f, tile::f32x4 (&acc)[NI][MJ], int j, T* o, int c0, int ff,
                                         int wn, int lg, float w, bool shared) {
-  constexpr int NO = MODE == 0 ? NI / 2 : NI;
-  const int col0 = c0 + (MODE == 0 ? 64 : 128) * wn + 4 * lg;
   const float wi = f.weigh_in ? w : 1.f, wo = f.weigh_in ? 1.f : w, lim = shared ? f.limit_s : f.limit;
   const auto act = [&](float g) {
     if constexpr (ACT == 0) return g * sigmoid_fast(g);
     else return gate_act(g, ACT);
   };
+  constexpr int STEP = MODE == 0 ? 4 : 2;                // fragments of 8 columns
 #pragma unroll
-  for (int i = 0; i < NO; ++i) {
-    if (col0 + 16 * i >= ff) continue;
-    float r[4];
+  for (int i = 0; i < NI; i += STEP) {
+    const int col = c0 + (MODE == 0 ? 8 : 16) * (NI * wn + i) + 8 * lg;
+    unsigned out[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      float g = acc[i][j][q] * wi;
+    for (int h = 0; h < 2; ++h) {
+      float r[4];
+      tile::f32x4& a0 = acc[i + STEP / 2 * h][j];
+      tile::hold(a0);
       if constexpr (MODE == 1) {
-        r[q] = act(g) * wo;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) r[q] = act(a0[q] * wi) * wo;
       } else {
-        float u = acc[(NI / 2 + i) % NI][j][q] * wi;
-        if constexpr (ACT == 4) {
-          g = fminf(g, lim);
-          u = fminf(fmaxf(u, -lim), lim);
-          r[q] = g * sigmoid_fast(f.slope * g) * (u + f.shift) * wo;
-        } else {
-          r[q] = act(g) * u * wo;
+        tile::f32x4& a1 = acc[i + 2 * h + 1][j];
+        tile::hold(a1);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          float g = a0[q] * wi, u = a1[q] * wi;
+          if constexpr (ACT == 4) {
+            g = fminf(g, lim);
+            u = fminf(fmaxf(u, -lim), lim);
+            r[q] = g * sigmoid_fast(f.slope * g) * (u + f.shift) * wo;
+          } else {
+            r[q] = act(g) * u * wo;
+          }
         }
       }
+      out[2 * h] = pk2<T>(r[0], r[1]);
+      out[2 * h + 1] = pk2<T>(r[2], r[3]);
     }
-    *reinterpret_cast<uint2*>(o + col0 + 16 * i) = make_uint2(pk2<T>(r[0], r[1]), pk2<T>(r[2], r[3]));
+    if (col < ff) *reinterpret_cast<uint4*>(o + col) = make_uint4(out[0], out[1], out[2], out[3]);
   }
 }
 
-// MODE 0: gate and up rows -> activation, 1: up rows alone -> activation, 2: second projection -> fp32
-template <typename T, int MODE>
-__global__ void __launch_bounds__(256, 1) expert_kernel(const ExpertArgs a) {
-  __shared__ __attribute__((aligned(16))) char lds[3 * STAGE];
-  constexpr int CT = MODE == 0 ? BN / 2 : BN;            // result columns of a tile
+// the tile of an expert's (or the shared one's) pairs m0 .. and result columns c0 ..: 32 MJ pairs by 32 NI weight rows.
+// MODE 0: gate and up rows -> activation ACT (GateForm's), 1: up rows alone -> activation, 2: second projection -> fp32.
+// (A choice of the activation at run time makes the compiler copy accumulators, which it does not know to be under way still,
+// between the products; chosen inside the element it also made the epilogue 14000 instructions long.)
+template <typename T, int MODE, int NI, int MJ, int ACT>
+__device__ __forceinline__ void run_tile(const ExpertArgs& a, char* lds, int e, int r0, int rows, int m0, int c0) {
+  constexpr int PIECES = tile::Shape<NI, MJ>::PIECES;
   const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wid >> 1, wn = wid & 1;
+  const bool shared = e == a.E;
+  const int ff = shared ? a.ffs : a.ff;
+  const int nk = MODE == 2 ? (ff + BK - 1) / BK : a.W / BK, N = MODE == 2 ? a.W : ff;
+  const T* x = (const T*)(shared ? a.xs : a.x);
+  const long long ldx = shared ? a.ldxs : a.ldx;
+  const bool gather = MODE != 2 && !shared;
+  const char* xb = (const char*)(x + (gather ? 0 : (long long)(r0 + m0) * ldx));
+  // weights: MODE 0 / 1 row blocks per expert, MODE 2 column blocks
+  const char* wb = (const char*)((const T*)a.w + (MODE == 2 ? (long long)c0 * a.ldw + (long long)e * a.ff
+                                                            : (long long)e * (MODE == 0 ? 2 : 1) * a.ff * a.ldw));
+  unsigned off[PIECES];                                  // (past the edges the last row is read: never stored)
+#pragma unroll
+  for (int q = 0; q < PIECES; ++q) {
+    const int r = 8 * (wid + 4 * (q < MJ ? q : q - MJ)) + (lane >> 3), c = (lane & 7) ^ tile::swz(r);
+    if (q < MJ) {
+      const int i = min(r, rows - m0 - 1);
+      off[q] = (unsigned)(gather ? a.idx[r0 + m0 + i] : i) * (unsigned)(2 * ldx) + 16 * c;
+    } else if (MODE == 0) {
+      const int col = min(c0 + r / (16 * NI) * (8 * NI) + gate_col(r % (16 * NI)), ff - 1);
+      off[q] = (unsigned)(col + ((r >> 4) & 1 ? ff : 0)) * (unsigned)(2 * a.ldw) + 16 * c;
+    } else {
+      const int col = r / (16 * NI) * (16 * NI) + tile::colperm<NI>(r % (16 * NI));
+      off[q] = (unsigned)(MODE == 1 ? min(c0 + col, ff - 1) : min(col, N - c0 - 1)) * (unsigned)(2 * a.ldw) + 16 * c;
+    }
+  }
+  tile::f32x4 acc[NI][MJ];
+  tile::products<T, NI, MJ, false, MODE == 2>(lds, xb, wb, nk, 0, off, acc, MODE == 2 && ff % BK != 0);
+  // lane (lr, lg) holds pair 16 j + lr, weight rows 16 i + 4 lg .. + 3 of its wave's block
+#pragma unroll
+  for (int j = 0; j < MJ; ++j) {
+    const int m = m0 + 16 * MJ * wm + 16 * j + lr;
+    if (m >= rows) continue;
+    if constexpr (MODE == 2) {
+      float* o = (float*)(shared ? a.ys : a.y) + (long long)(r0 + m) * a.W;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int col = c0 + 16 * NI * wn + 32 * (i >> 1) + 8 * lg + 4 * (i & 1);
+        tile::hold(acc[i][j]);
+        if (col < N) *reinterpret_cast<tile::f32x4*>(o + col) = acc[i][j];
+      }
+    } else {
+      const float wt = shared ? 1.f : a.wt[r0 + m];
+      T* o = (T*)(shared ? a.ys : a.y) + (long long)(r0 + m) * ff;
+      put_row<T, MODE, NI, MJ, ACT>(a.form, acc, j, o, c0, ff, wn, lg, wt, shared);
+    }
+  }
+}
+
+// Tiles of 32 MJ pairs and 256 weight rows.  MJ 8: whole rounds of the CUs; what is left over is cut into two or four where that
+// makes one round of smaller tiles.
+template <typename T, int MODE, int MJ, int ACT>
+__global__ void __launch_bounds__(256, 1) expert_kernel(const ExpertArgs a) {
+  constexpr int BM = 32 * MJ, CT = MODE == 0 ? BN / 2 : BN;            // rows and result columns of a tile
+  __shared__ __attribute__((aligned(16))) char lds[MJ == 8 && tile::Shape<8, 4>::LDS > tile::Shape<8, 8>::LDS
+                                                       ? tile::Shape<8, 4>::LDS : tile::Shape<8, MJ>::LDS];
+  static_assert(tile::Shape<4, 4>::LDS <= 163840);
+  const int lane = threadIdx.x & 63;
   // the tile: experts in order (the shared one last), weight panels in order, row tiles within a panel
   const int ce = ((MODE == 2 ? a.W : a.ff) + CT - 1) / CT, cs = a.ffs > 0 ? ((MODE == 2 ? a.W : a.ffs) + CT - 1) / CT : 0;
   const int rows_e = lane < a.E ? a.off[lane + 1] - a.off[lane] : 0;
@@ -111,10 +176,23 @@ __global__ void __launch_bounds__(256, 1) expert_kernel(const ExpertArgs a) {
     if (lane >= o) pre += n;
   }
   const int tiles_e = __builtin_amdgcn_readlane(pre, 63) * ce, ts = (a.T + BM - 1) / BM;
-  const int total = tiles_e + ts * cs;
-  if ((int)blockIdx.x >= total) return;
-  const int xcd = blockIdx.x & 7, q8 = total >> 3, r8 = total & 7;
-  const int v = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + ((int)blockIdx.x >> 3);
+  const int total = tiles_e + ts * cs, b = blockIdx.x;
+  int v, cut = 1, part = 0;
+  if constexpr (MJ == 8) {
+    const int full = total / tile::CUS * tile::CUS, left = total - full;
+    if (b < full) {
+      v = tile::unit_of(b, full);
+    } else {
+      cut = 4 * left <= tile::CUS ? 4 : 2 * left <= tile::CUS ? 2 : 1;
+      if (b - full >= cut * left) return;
+      const int u = tile::unit_of(b - full, cut * left);
+      v = full + u / cut;
+      part = u % cut;
+    }
+  } else {
+    if (b >= total) return;
+    v = tile::unit_of(b, total);
+  }
   int e = a.E, r0 = 0, rows = a.T, u = v - tiles_e, nt = ts;
   if (v < tiles_e) {
     e = __popcll(__ballot(pre * ce <= v));               // (lanes past E hold the total: never counted)
@@ -125,120 +203,17 @@ __global__ void __launch_bounds__(256, 1) expert_kernel(const ExpertArgs a) {
     r0 = a.off[e];
     rows = a.off[e + 1] - r0;
   }
-  const bool shared = e == a.E;
-  const int ff = shared ? a.ffs : a.ff;
   const int tn = u / nt, m0 = (u - tn * nt) * BM, c0 = tn * CT;
-  const int nk = MODE == 2 ? (ff + BK - 1) / BK : a.W / BK, N = MODE == 2 ? a.W : ff;
-  // a contraction of 32 more: the last stage reads its first half twice and multiplies it once
-  const bool odd = MODE == 2 && ff % BK != 0;
-  const T* x = (const T*)(shared ? a.xs : a.x);
-  const long long ldx = shared ? a.ldxs : a.ldx;
-  const bool gather = MODE != 2 && !shared;
-  const char* xb = (const char*)(x + (gather ? 0 : (long long)(r0 + m0) * ldx));
-  // weights: MODE 0 / 1 row blocks per expert, MODE 2 column blocks
-  const char* wb = (const char*)((const T*)a.w + (MODE == 2 ? (long long)c0 * a.ldw + (long long)e * a.ff
-                                                            : (long long)e * (MODE == 0 ? 2 : 1) * a.ff * a.ldw));
-  unsigned off[PIECES];
-#pragma unroll
-  for (int q = 0; q < PIECES; ++q) {
-    const int p = wid + 4 * q, r = 8 * (q < XP ? p : p - BM / 8) + (lane >> 3);
-    const int c = (lane & 7) ^ swz(r);
-    if (q < XP) {
-      const int i = min(r, rows - m0 - 1);
-      off[q] = (unsigned)(gather ? a.idx[r0 + m0 + i] : i) * (unsigned)(2 * ldx) + 16 * c;
-    } else if (MODE == 0) {                              // [64 gate | 64 up] rows of each wave column
-      const int col = min(c0 + 64 * (r >> 7) + (r & 63), ff - 1);
-      off[q] = (unsigned)(col + (r & 64 ? ff : 0)) * (unsigned)(2 * a.ldw) + 16 * c;
-    } else if (MODE == 1) {
-      off[q] = (unsigned)min(c0 + r, ff - 1) * (unsigned)(2 * a.ldw) + 16 * c;
-    } else {
-      off[q] = (unsigned)min(r, N - c0 - 1) * (unsigned)(2 * a.ldw) + 16 * c;
+  if constexpr (MJ == 8) {
+    if (cut > 1) {
+      const int m = m0 + BM / 2 * (part & 1), c = c0 + CT / 2 * (part >> 1);
+      if (m >= rows || c >= (MODE == 2 ? a.W : e == a.E ? a.ffs : a.ff)) return;
+      if (cut == 2) run_tile<T, MODE, 8, 4, ACT>(a, lds, e, r0, rows, m, c0);
+      else run_tile<T, MODE, 4, 4, ACT>(a, lds, e, r0, rows, m, c);
+      return;
     }
   }
-  const unsigned lds0 = (unsigned)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds);
-  const unsigned upper = ((lane >> 2) ^ wid) & 1 ? BK : 0;     // (bytes) the lane's chunk lies in the upper half
-  auto issue = [&](int t, int slot, int q0, int q1) __attribute__((always_inline)) {
-    const unsigned back = odd && t == nk - 1 ? upper : 0;
-    const char *xs = xb + (long long)t * (BK * 2), *wsrc = wb + (long long)t * (BK * 2);
-    const unsigned dst = __builtin_amdgcn_readfirstlane(lds0 + slot * STAGE + wid * 1024);
-#pragma unroll
-    for (int q = q0; q < q1; ++q) dma16(q < XP ? xs : wsrc, MODE == 2 ? off[q] - back : off[q], dst + q * 4096);
-  };
-  f32x4 acc[NI][MJ];
-#pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int j = 0; j < MJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  uint4 fa[2][NI], fb[2][MJ];
-  const int rb0 = (64 * wm + lr) * ROWB, ra0 = XB + (128 * wn + lr) * ROWB;
-  // fragments u0 .. u1 - 1 of half h of a stage (x's, then w's)
-  auto frags = [&](int h, int slot, int u0, int u1) __attribute__((always_inline)) {
-    const char* p = lds + slot * STAGE + (((4 * h + lg) ^ swz(lr)) << 4);
-#pragma unroll
-    for (int i = u0; i < u1; ++i)
-      if (i < MJ) fb[h][i] = *reinterpret_cast<const uint4*>(p + rb0 + i * 16 * ROWB);
-      else fa[h][i - MJ] = *reinterpret_cast<const uint4*>(p + ra0 + (i - MJ) * 16 * ROWB);
-  };
-  // the products of half h; between them the reads of the other half's fragments (from stage slot fs) and
-  // half of the pieces of stage `t` into slot `ds` (t < 0: none)
-  auto half = [&](int h, int fs, int t, int ds) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      if (2 * i < NI + MJ) frags(1 - h, fs, 2 * i, 2 * i + 2);
-      if (t >= 0 && i < PIECES / 2) issue(t, ds, (1 - h) * (PIECES / 2) + i, (1 - h) * (PIECES / 2) + i + 1);
-#pragma unroll
-      for (int j = 0; j < MJ; ++j) acc[i][j] = Mfma<T>::run(fa[h][i], fb[h][j], acc[i][j]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
-  issue(0, 0, 0, PIECES);
-  if (nk > 1) issue(1, 1, 0, PIECES);
-  if (nk > 2) issue(2, 2, 0, PIECES / 2);
-  if (nk > 2) wait_vm<PIECES + PIECES / 2>(); else if (nk > 1) wait_vm<PIECES>(); else wait_vm<0>();
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-  frags(0, 0, 0, NI + MJ);
-  int slot = 0, t = 0;
-  for (; t + 3 < nk; ++t) {
-    const int next = slot == 2 ? 0 : slot + 1, last = slot == 0 ? 2 : slot - 1;
-    half(0, slot, t + 2, last);
-    wait_vm<PIECES>();
-    done_reading();
-    half(1, next, t + 3, slot);
-    slot = next;
-  }
-  for (; t < nk; ++t) {       // the last three stages
-    const int next = slot == 2 ? 0 : slot + 1, last = slot == 0 ? 2 : slot - 1;
-    half(0, slot, t + 2 < nk ? t + 2 : -1, last);
-    if (t + 2 < nk) wait_vm<PIECES>(); else wait_vm<0>();
-    done_reading();
-    if (!odd || t + 1 < nk) half(1, next, -1, 0);     // (the last step reads a slot that holds an earlier stage: unused)
-    slot = next;
-  }
-  // lane (lr, lg) holds pair 16 j + lr, weight rows 16 i + 4 lg .. + 3 of its wave's block
-#pragma unroll
-  for (int j = 0; j < MJ; ++j) {
-    const int m = m0 + 64 * wm + 16 * j + lr;
-    if (m >= rows) continue;
-    if constexpr (MODE == 2) {
-      float* o = (float*)(shared ? a.ys : a.y) + (long long)(r0 + m) * a.W + c0 + 128 * wn + 4 * lg;
-#pragma unroll
-      for (int i = 0; i < NI; ++i)
-        if (c0 + 128 * wn + 16 * i + 4 * lg < N) *reinterpret_cast<f32x4*>(o + 16 * i) = acc[i][j];
-    } else {
-      const float wt = shared ? 1.f : a.wt[r0 + m];
-      T* o = (T*)(shared ? a.ys : a.y) + (long long)(r0 + m) * ff;
-      // (one branch per row: with the choice inside the element the epilogue was 14000 instructions long, and
-      // fetching them took as long as half of the products)
-      switch (a.form.act) {
-        case 0: put_row<T, MODE, 0>(a.form, acc, j, o, c0, ff, wn, lg, wt, shared); break;
-        case 1: put_row<T, MODE, 1>(a.form, acc, j, o, c0, ff, wn, lg, wt, shared); break;
-        case 2: put_row<T, MODE, 2>(a.form, acc, j, o, c0, ff, wn, lg, wt, shared); break;
-        case 3: put_row<T, MODE, 3>(a.form, acc, j, o, c0, ff, wn, lg, wt, shared); break;
-        default: put_row<T, MODE, 4>(a.form, acc, j, o, c0, ff, wn, lg, wt, shared);
-      }
-    }
-  }
+  run_tile<T, MODE, 8, MJ, ACT>(a, lds, e, r0, rows, m0, c0);
 }
 
 // One workgroup per expert e: pairs of experts before e are counted along the way (a row's chosen experts below e
@@ -343,8 +318,41 @@ bool sizes_ok(int dt, int T, int W, int E, int top, int ff, int ffs) {
          top <= E && ff >= 32 && ff % 32 == 0 && ffs >= 0 && ffs % 32 == 0 && (long long)T * top < (1 << 30) &&
          (long long)(2 * E * (long long)ff + 2 * ffs) * W < (1LL << 40);
 }
-long long tiles_of(int T, int E, int top, long long ce, long long cs) {
-  return ((long long)T * top / BM + E) * ce + (long long)((T + BM - 1) / BM) * cs;
+constexpr int kMinRows = 64;                             // of a tile
+// the most tiles of `bm` rows and ce (an expert's) or cs (the shared one's) column tiles
+long long tiles_of(int T, int E, int top, int bm, long long ce, long long cs) {
+  return ((long long)T * top / bm + E) * ce + (long long)((T + bm - 1) / bm) * cs;
+}
+
+// Rows of a tile / 32: the least time of all rounds of the CUs, as far as the sizes tell.  Of T top / E rows each, more or less
+// by their root.  us a tile, by stages of 64 k, as measured (4096 rows, 8 experts of 1408 and a shared one, width 2048: act of 256
+// rows in rounds and a cut one 139 us, of 128 rows 165, of 64 240).
+int pick_rows(int T, int E, int top, int nk, int ce, int cs) {
+  const double r = (double)T * top / E, s = 1.5 * sqrt(r);
+  const auto tiles = [&](int bm) {
+    double n = 0.;
+    for (const double x : {r - s, r, r + s}) n += x <= bm ? 1. : ceil(x / bm);
+    return ceil(n * E / 3. * ce) + (double)((T + bm - 1) / bm) * cs;
+  };
+  const auto rounds = [&](int bm) { return ceil(tiles(bm) / tile::CUS); };
+  const double full = floor(tiles(256) / tile::CUS), left = tiles(256) - full * tile::CUS;
+  const double t4 = 0.72 * nk + 10., t2 = 0.55 * nk + 9., cut = 0.42 * nk + 8., t8 = 1.25 * nk + 11.;
+  const double all8 = full * t8 + (left == 0. ? 0. : 4 * left <= tile::CUS ? cut : 2 * left <= tile::CUS ? t4 : t8);
+  const double all4 = rounds(128) * t4, all2 = rounds(64) * t2;
+  return all8 < all4 && all8 < all2 ? 8 : all4 <= all2 ? 4 : 2;
+}
+
+template <typename T, int MODE, int ACT>
+hipError_t launch(const ExpertArgs& p, int top, int ce, int cs, hipStream_t st) {
+  const int nk = (MODE == 2 ? (p.ff > p.ffs ? p.ff : p.ffs) : p.W) / BK, mj = pick_rows(p.T, p.E, top, nk, ce, cs);
+  // (MJ 8: what is left over may take a round of its own)
+  const unsigned grid = (unsigned)(tiles_of(p.T, p.E, top, 32 * mj, ce, cs) + (mj == 8 ? tile::CUS : 0));
+  switch (mj) {
+    case 2: expert_kernel<T, MODE, 2, ACT><<<grid, 256, 0, st>>>(p); break;
+    case 4: expert_kernel<T, MODE, 4, ACT><<<grid, 256, 0, st>>>(p); break;
+    default: expert_kernel<T, MODE, 8, ACT><<<grid, 256, 0, st>>>(p);
+  }
+  return hipGetLastError();
 }
 
 }  // namespace
@@ -353,7 +361,7 @@ extern "C" {
 
 // T rows, width W, E experts of ff of which a row chooses at most `top`, a shared one of ffs (or 0)
 int sm_expert_ok(int dt, int T, int W, int E, int top, int ff, int ffs) {
-  return sizes_ok(dt, T, W, E, top, ff, ffs) && tiles_of(T, E, top, (W + ff) / 64 + 2, (W + ffs) / 64 + 2) < (1 << 30);
+  return sizes_ok(dt, T, W, E, top, ff, ffs) && tiles_of(T, E, top, kMinRows, (W + ff) / 64 + 2, (W + ffs) / 64 + 2) < (1 << 30);
 }
 
 // wts [T, E] fp32 -> off [E + 1], idx and wt [T top], place [T, top] (a row's pairs in expert order, -1: none)
@@ -371,18 +379,24 @@ hipError_t sm_expert_act(int dt, const void* h, long long ldh, const void* w, co
                          hipStream_t st) {
   if (!sm_expert_ok(dt, T, W, E, top, ff, ffs) || act < 0 || act > (gated ? 4 : 3) || (weigh_in && !gated) ||
       ldh % 8 || ldh < W || (long long)T * ldh >= (1LL << 31) || 2LL * (ff > ffs ? ff : ffs) * W >= (1LL << 31) ||
-      ((uintptr_t)h | (uintptr_t)w) % 16 || ((uintptr_t)a | (uintptr_t)as) % 8)
+      ((uintptr_t)h | (uintptr_t)w | (uintptr_t)a | (uintptr_t)as) % 16)
     return hipErrorInvalidValue;
   const ExpertArgs p{h, h, ldh, ldh, w, W, a, as, off, idx, wt, T, W, E, ff, ffs,
                      GateForm{act, weigh_in, limit, limit_s, slope, shift}};
   const int ct = gated ? BN / 2 : BN;
-  const unsigned grid = (unsigned)tiles_of(T, E, top, (ff + ct - 1) / ct, ffs > 0 ? (ffs + ct - 1) / ct : 0);
-#define GO(TT)                                                          \
-  if (gated) expert_kernel<TT, 0><<<grid, 256, 0, st>>>(p);             \
-  else expert_kernel<TT, 1><<<grid, 256, 0, st>>>(p);
+  const int ce = (ff + ct - 1) / ct, cs = ffs > 0 ? (ffs + ct - 1) / ct : 0;
+#define GO(TT)                                                                    \
+  if (!gated) return act == 0   ? launch<TT, 1, 0>(p, top, ce, cs, st)            \
+                     : act == 1 ? launch<TT, 1, 1>(p, top, ce, cs, st)            \
+                     : act == 2 ? launch<TT, 1, 2>(p, top, ce, cs, st)            \
+                                : launch<TT, 1, 3>(p, top, ce, cs, st);           \
+  return act == 0   ? launch<TT, 0, 0>(p, top, ce, cs, st)                        \
+         : act == 1 ? launch<TT, 0, 1>(p, top, ce, cs, st)                        \
+         : act == 2 ? launch<TT, 0, 2>(p, top, ce, cs, st)                        \
+         : act == 3 ? launch<TT, 0, 3>(p, top, ce, cs, st)                        \
+                    : launch<TT, 0, 4>(p, top, ce, cs, st);
   if (dt == kBF16) { GO(bf16) } else { GO(fp16) }
 #undef GO
-  return hipGetLastError();
 }
 
 // y [T top, W] and ys [T, W] fp32 = a and as by w [W, E ff + ffs]; then out [T, W] their sum per row
@@ -390,16 +404,15 @@ hipError_t sm_expert_down(int dt, const void* a, const void* as, const void* w, 
                           float* y, float* ys, void* out, int T, int W, int E, int top, int ff, int ffs,
                           hipStream_t st) {
   const long long ldw = (long long)E * ff + ffs;
-  if (!sm_expert_ok(dt, T, W, E, top, ff, ffs) || BN * ldw >= (1LL << 31) || (long long)BM * ff >= (1LL << 31) ||
-      (long long)BM * ffs >= (1LL << 31) || ((uintptr_t)a | (uintptr_t)as | (uintptr_t)w | (uintptr_t)y | (uintptr_t)ys) % 16 ||
+  if (!sm_expert_ok(dt, T, W, E, top, ff, ffs) || BN * ldw >= (1LL << 31) || 256LL * ff >= (1LL << 31) ||
+      256LL * ffs >= (1LL << 31) || ((uintptr_t)a | (uintptr_t)as | (uintptr_t)w | (uintptr_t)y | (uintptr_t)ys) % 16 ||
       (uintptr_t)out % 8)
     return hipErrorInvalidValue;
   const ExpertArgs p{a, as, ff, ffs, w, ldw, y, ys, off, nullptr, nullptr, T, W, E, ff, ffs, GateForm{}};
-  const long long c = (W + BN - 1) / BN;
-  const unsigned grid = (unsigned)tiles_of(T, E, top, c, ffs > 0 ? c : 0);
+  const int c = (W + BN - 1) / BN;
   const dim3 sum((unsigned)T, (unsigned)((W + 1023) / 1024));
 #define GO(TT)                                                                                       \
-  expert_kernel<TT, 2><<<grid, 256, 0, st>>>(p);                                                     \
+  if (const hipError_t rc = launch<TT, 2, 0>(p, top, c, ffs > 0 ? c : 0, st)) return rc;         \
   expert_sum_kernel<TT><<<sum, 256, 0, st>>>(y, ffs > 0 ? ys : nullptr, place, (TT*)out, top, W);
   if (dt == kBF16) { GO(bf16) } else { GO(fp16) }
 #undef GO

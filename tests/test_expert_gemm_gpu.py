@@ -1,4 +1,4 @@
-"""Products over the rows that chose an expert (seqmix/expert_gemm.hip) against float64: tiles of 128 pairs and 128 / 256
+"""Products over the rows that chose an expert (seqmix/expert_gemm.hip) against float64: tiles of 64 - 256 pairs and 128 / 256
 columns and their remainders, contractions of 32 more than whole stages, experts nobody or everybody chose, rows with
 fewer choices than `top`, several thousand rows, row strides, every activation, replays of a captured call."""
 import pytest
@@ -75,6 +75,23 @@ def test_chosen_experts(T, W, E, top, ff, ffs, act, gated, weigh, skew, dtype):
     assert torch.equal(M.moe_chosen(wide[:, :W], wts, gu, down, *args), out)
     if not ffs and T > 1:
         assert not out[T // 2].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,W,E,top,ff,ffs,act,gated,weigh", [
+    (100, 192, 8, 2, 544, 480, "gelu_tanh", True, "output"), (3000, 192, 5, 2, 1440, 800, CLAMP, True, "input"),
+    (5000, 128, 9, 2, 1312, 96, "silu", True, "output"), (2500, 320, 16, 3, 1056, 0, "relu2", False, "output"),
+    (6000, 64, 8, 2, 1408, 1408, "gelu_tanh", False, "output"), (40, 1024, 16, 2, 608, 0, "relu", True, "output"),
+    (9000, 640, 4, 2, 288, 288, "relu2", True, "output"), (1030, 2048, 4, 1, 1408, 0, CLAMP, True, "output"),
+    (1100, 704, 3, 2, 1888, 0, "silu", True, "input"), (700, 256, 4, 2, 1408, 1408, "relu", False, "output"),
+    (2500, 320, 6, 3, 1056, 96, "silu", False, "output")])
+def test_tiles_of_64_and_256_pairs(T, W, E, top, ff, ffs, act, gated, weigh, dtype):
+    """Whole rounds of 256 pairs by 256 rows and what is left over uncut, in halves and in quarters (some of them empty), for every
+    activation; 64 pairs; stages of 64 and a last one of 32."""
+    h, wts, gu, down = layer(T, W, E, top, ff, ffs, gated, dtype, T + W)
+    wts[T // 2] = 0.0
+    out = M.moe_chosen(h, wts, gu, down, E, top, ff, ffs, act, gated, weigh)
+    check(out, exact(h, wts, gu, down, E, ff, ffs, act, gated, weigh), dtype)
 
 
 def test_more_choices_than_top_stay_in_bounds():

@@ -25,7 +25,8 @@
 //   M = 64: 6.1 / 9.0, 15.3 / 17.6, 12.0 / 18.4, 29.4 / 27.9, 13.3 / 14.3, 52.0 / 45.1, 33.9 / 34.9
 //   M = 1:  3.8 / 8.3 (GEMV 4.4), 9.8 / 16.1 (10.5), 7.3 / 11.7 (6.6), 22.4 / 32.0 (22.9), 7.5 / 12.1
 //           (8.1), 30.7 / 51.6 (28.5), 17.2 / 20.6 (17.2)
-// The activation form (thin_act): a workgroup's tile is 16 activation columns -- their gate rows and
+// (16-column tiles throughout; matrices of up to 2048 rows now take tiles of eight, see pick)
+// The activation form (thin_act): a workgroup's tile is 16 (or 8) activation columns -- their gate rows and
 // their up rows -- so act(gate) * up, times the row's routing weight, is formed from the fp32 sums and
 // the [M, 2 ff] intermediate and its kernel are gone.  Routed experts: W holds every expert, and a
 // step of a few rows uses few of them.  `sparse` reads the routing weights first and streams the
@@ -46,6 +47,7 @@ using namespace lumen;
 namespace {
 
 constexpr int BK = 64, ROWB = 128;   // k per stage, bytes of an image row
+constexpr int kCUs = 256;
 
 // 16-byte chunk c of image row r lives at chunk c ^ swz(r): a fragment read (16 rows at one chunk)
 // touches 16 different bank slots
@@ -88,17 +90,19 @@ __device__ __forceinline__ int nth_bit(unsigned long long m, int i) {
   return __builtin_ctzll(m);
 }
 
-// XP: pieces of 8 x rows (1, 2, 4, 8: groups of up to 8, 16, 32, 64 rows, blockIdx.y names the group).  ACT: 0 plain, 1 activation of RT = 1 row
-// tile (no gate), 2 gated (RT = 2: the tile's gate rows, its up rows).
-template <typename T, int RT, int XP, int NW, int D, int ACT>
+// XP: pieces of 8 x rows (1, 2, 4, 8: groups of up to 8, 16, 32, 64 rows, blockIdx.y names the group).  ACT: 0 plain, 1 activation
+// (no gate), 2 gated.  RT: row tiles of W of a product; WP: pieces of 8 W rows, 2 RT or fewer: plain 1 of an RT of 1 (the product's upper
+// half repeats the lower one, never stored); gated half of them gate and half up rows (WP 2: the two halves of one row tile).
+template <typename T, int RT, int XP, int NW, int D, int ACT, int WP>
 __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
   constexpr int MT = XP < 2 ? 1 : XP / 2;
-  constexpr int WB = RT * 16 * ROWB, SB = WB + XP * 8 * ROWB;
-  constexpr int G = 2 * RT + XP;                   // DMA instructions of a stage
+  constexpr int WB = WP * 8 * ROWB, SB = WB + XP * 8 * ROWB;
+  constexpr int G = WP + XP;                       // DMA instructions of a stage
+  constexpr int TC = ACT == 2 ? 4 * WP : 8 * WP;   // result columns of a tile
   constexpr int PB = RT * MT * 1024;               // a wave's partial tile
   constexpr int WTS = XP <= 4 ? kMaxWts * 4 : 0;
   static_assert(G * (D - 1) < 64, "stages in flight");
-  static_assert(ACT == 0 || RT == ACT, "an activation tile is one row tile per operand");
+  static_assert(WP == 2 * RT || (RT == 1 && WP == 1 && ACT == 0) || (RT == 1 && WP == 2 && ACT == 2), "pieces of a tile");
   static_assert(NW * D * SB + 2 * NW * PB + WTS <= 163840, "LDS");
   __shared__ __attribute__((aligned(16))) char lds[NW * D * SB + 2 * NW * PB + WTS];
   const int lane = threadIdx.x & 63;
@@ -127,9 +131,9 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
     }
   }
   int tiles = p.tiles, kt = p.K / BK;
-  const int per = p.ff >> 4, ks = p.ff >> 6;       // tiles / k stages of an expert
+  const int per = p.ff / TC, ks = p.ff >> 6;       // tiles / k stages of an expert
   if (p.sparse) {
-    if (ACT) tiles = n_chosen * per + (p.ffs >> 4);
+    if (ACT) tiles = n_chosen * per + p.ffs / TC;
     else kt = n_chosen * ks + (p.ffs >> 6);
   }
   const int k0 = kt * wid / NW, nk = kt * (wid + 1) / NW - k0;
@@ -142,10 +146,10 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
     const int n = p.sparse ? n_chosen : p.E;
     if (p.E > 0 && i < n) {
       e = p.sparse ? nth_bit(chosen, i) : i;
-      col = (t - i * per) * 16;
+      col = (t - i * per) * TC;
     } else {
       e = p.E;
-      col = (t - n * per) * 16;
+      col = (t - n * per) * TC;
     }
   };
   int at_t = blockIdx.x, at_k = 0, issued = 0, put = 0;
@@ -161,14 +165,14 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
   int last = 0;
   const auto seat = [&]() {
     if constexpr (ACT == 0) {
-      Wa = W + (long long)at_t * (RT * 16) * p.K;
-      last = min(RT * 16, p.N - at_t * RT * 16) - 1;
+      Wa = W + (long long)at_t * TC * p.K;
+      last = min(TC, p.N - at_t * TC) - 1;
     } else {
       int e, col;
       block_of(at_t, e, col);
-      Wa = W + ((long long)e * RT * p.ff + col) * p.K;
+      Wa = W + ((long long)e * ACT * p.ff + col) * p.K;
       Wb = Wa + (long long)(e < p.E ? p.ff : p.ffs) * p.K;
-      last = RT * 16 - 1;
+      last = 8 * WP - 1;
     }
   };
   seek();
@@ -176,10 +180,10 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
   const auto issue = [&]() {
     char* img = ring + put * SB;
 #pragma unroll
-    for (int q = 0; q < 2 * RT; ++q) {
+    for (int q = 0; q < WP; ++q) {
       const int r = 8 * q + rr;
-      const T* base = ACT == 2 && q >= 2 ? Wb : Wa;
-      const int row = ACT == 2 && q >= 2 ? r - 16 : min(r, last);
+      const T* base = ACT == 2 && q >= WP / 2 ? Wb : Wa;
+      const int row = ACT == 2 && q >= WP / 2 ? r - 4 * WP : min(r, last);
       dma16(base, ((unsigned)row * (unsigned)p.K + kk + 8 * (c ^ swz(r))) * 2u, img + 8 * q * ROWB);
     }
 #pragma unroll
@@ -227,7 +231,7 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
         uint4 a[RT], b[MT];
 #pragma unroll
         for (int i = 0; i < RT; ++i) {
-          const int r = 16 * i + lr;
+          const int r = (16 * i + lr) & (8 * WP - 1);
           a[i] = *reinterpret_cast<const uint4*>(img + r * ROWB + (((4 * s + lg) ^ swz(r)) << 4));
         }
 #pragma unroll
@@ -266,8 +270,8 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
       for (int q = wid; q < RT * MT; q += NW) {
         const int i = q / MT, j = q - i * MT;
         f32x4 v = sum(q);
-        const int m = m0 + 16 * j + lr, n = t * RT * 16 + 16 * i + 4 * lg;
-        if (m >= p.M || 16 * j + lr >= M || n >= p.N) continue;
+        const int m = m0 + 16 * j + lr, n = t * TC + 16 * i + 4 * lg;
+        if (m >= p.M || 16 * j + lr >= M || n >= p.N || 4 * lg >= TC) continue;
         if (p.bias != nullptr) {
           const T* b = (const T*)p.bias + n;
 #pragma unroll
@@ -300,8 +304,14 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
       block_of(t, e, col);
       for (int j = wid; j < MT; j += NW) {
         const int m = 16 * j + lr;
-        f32x4 g = sum(j), u = ACT == 2 ? sum(MT + j) : f32x4{1.f, 1.f, 1.f, 1.f};
-        if (m >= M) continue;
+        f32x4 g = sum(j), u = f32x4{1.f, 1.f, 1.f, 1.f};
+        if constexpr (ACT == 2 && RT == 1) {       // up rows in the lanes of the tile's upper half
+#pragma unroll
+          for (int i = 0; i < 4; ++i) u[i] = __shfl(g[i], (lane + 32) & 63, 64);
+        } else if constexpr (ACT == 2) {
+          u = sum(MT + j);
+        }
+        if (m >= M || 4 * lg >= TC) continue;
         const float w = e < p.E ? wts[m * p.E + e] : 1.f;
         float o[4];
 #pragma unroll
@@ -317,11 +327,12 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
   }
 }
 
-template <typename T, int RT, int XP, int NW, int D, int ACT = 0>
+template <typename T, int RT, int XP, int NW, int D, int ACT = 0, int WP = 2 * RT>
 hipError_t run(ThinArgs p, int per_cu, hipStream_t st) {
-  p.tiles = ACT ? (p.E * p.ff + p.ffs) / 16 : (p.N + 16 * RT - 1) / (16 * RT);
+  constexpr int TC = ACT == 2 ? 4 * WP : 8 * WP;
+  p.tiles = ACT ? (p.E * p.ff + p.ffs) / TC : (p.N + TC - 1) / TC;
   const dim3 grid(p.tiles < 256 * per_cu ? p.tiles : 256 * per_cu, (p.M + 8 * XP - 1) / (8 * XP));
-  thin_kernel<T, RT, XP, NW, D, ACT><<<grid, 64 * NW, 0, st>>>(p);
+  thin_kernel<T, RT, XP, NW, D, ACT, WP><<<grid, 64 * NW, 0, st>>>(p);
   return hipGetLastError();
 }
 
@@ -334,9 +345,17 @@ hipError_t run(ThinArgs p, int per_cu, hipStream_t st) {
 // 4096 9.5 -> 4.9 (16 and eight waves; of 32 4.7, 6.9), 2048 x 2048 7.8 -> 6.1, 2048 x 5632 17.1 -> 12.0 (32), 3072 x 2048 8.1 -> 7.5
 // (32, 32-row tiles; 16-row ones 9.6), 4096 x 4096 14.2 -> 13.8, 6144 x 2048 13.3 -> 11.8; 32 rows: 128 x 2048 4.5 -> 3.6, 2048 x 2048
 // 6.2 -> 5.1, 2048 x 5632 12.4 -> 10.3 (16; 3072 x 2048 would go 6.5 -> 7.0).
+// Up to 16 rows of a matrix of up to 2048 rows take tiles of eight columns, eight waves and the stages that fit: as many CUs as
+// there are (16-column tiles of 2048 leave half of them idle).  us, 16-column tiles -> these, 1 / 8 / 16 rows: 2048 x 2048 4.7 / 5.0 /
+// 5.2 -> 4.3 / 4.4 / 4.8, 2048 x 5632 8.2 / 8.5 / 9.9 -> 6.9 / 7.2 / 8.5, 2048 x 12672 12.9 / 15.1 / 18.0 -> 11.0 / 12.2 / 14.8 (8 rows, 4.2 TB/s),
+// 1024 x 2816 5.2 / 5.4 / 6.0 -> 4.2 / 4.7 / 5.4, 256 x 4096 5.3 / 6.1 / 7.0 -> 4.5 / 5.0 / 6.0; the chosen of 16 experts of 1408, 2048 rows of W, 8
+// rows 25.5 -> 20.1, one row 6.9 -> 6.5.  Short rows have no use for eight waves (2048 x 512 3.1 -> 3.2), larger matrices none for
+// half tiles (2112 x 2048, 8 rows 4.9 -> 5.4).
 template <typename T>
 hipError_t pick(const ThinArgs& p, hipStream_t st) {
   const bool wide = p.N >= 8192, tiny = p.N <= 256;
+  if (p.N <= 8 * kCUs && p.K >= 1024 && p.M <= 16)
+    return p.M <= 8 ? run<T, 1, 1, 8, 5, 0, 1>(p, 1, st) : run<T, 1, 2, 8, 4, 0, 1>(p, 1, st);
   if (p.M <= 8) {
     if (wide && p.K >= 4096) return run<T, 2, 1, 4, 4>(p, 1, st);
     if (!wide && (p.K >= 4608 || tiny)) return run<T, 1, 1, 8, 4>(p, 2, st);
@@ -360,6 +379,12 @@ hipError_t pick(const ThinArgs& p, hipStream_t st) {
 
 template <typename T>
 hipError_t pick_act(const ThinArgs& p, int gated, hipStream_t st) {
+  // Tiles of eight columns, two workgroups a CU, where tiles of 16 are one or two rounds of the CUs and at most half of another
+  // (5632 columns of 2048, 1.4 rounds, 8 rows 12.7 -> 11.7 us, 5632 of 4096 21.4 -> 18.9, 10240 of 2048 18.6 -> 17.5; 1.6 rounds would go
+  // 13.3 -> 14.6, one whole one 14.4 -> 15.0, 2.75 33.0 -> 34.5, 1.4 of 512 6.5 -> 7.1).  Tiles of experts depend on the choice: 16.
+  const int t = p.N / 16, rest = t % kCUs;
+  if (gated && p.E == 0 && p.K >= 1024 && p.M <= 16 && t > kCUs && t < 3 * kCUs && rest > 0 && 2 * rest <= kCUs)
+    return p.M <= 8 ? run<T, 1, 1, 4, 5, 2, 2>(p, 2, st) : run<T, 1, 2, 4, 4, 2, 2>(p, 2, st);
   if (gated) {
     if (p.M <= 8) return run<T, 2, 1, 4, 4, 2>(p, 1, st);
     if (p.M <= 16) return run<T, 2, 2, 4, 4, 2>(p, 1, st);

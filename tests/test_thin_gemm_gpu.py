@@ -155,3 +155,46 @@ def test_rows_in_groups(M, N, K, dtype, bits):
     y, exact = thin_linear(x, w), x.double() @ w.double().t()
     acc, ulp = bound(x, w, bits)
     assert ((y.double() - exact).abs() <= acc + exact.abs() * ulp + 1e-30).all()
+
+
+@pytest.mark.parametrize("dtype,bits", [(torch.bfloat16, 8), (torch.float16, 11)])
+@pytest.mark.parametrize("M", [1, 7, 8, 9, 16])
+@pytest.mark.parametrize("N,K", [(4, 1024), (12, 1088), (2044, 1024), (2048, 1536), (2052, 1024), (40, 4096)])
+def test_tiles_of_eight_columns(M, N, K, dtype, bits):
+    """Up to 2048 columns of 1024 and more."""
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x = torch.randn(M, K + 8, device="cuda", generator=g).to(dtype)[:, :K]
+    w = (torch.randn(N, K, device="cuda", generator=g) / K ** 0.5).to(dtype)
+    b = torch.randn(N, device="cuda", generator=g).to(dtype)
+    want = x.double() @ w.double().t() + b.double()
+    acc, ulp = bound(x, w, bits)
+    y = thin_linear(x, w, b)
+    assert ((y.double() - want).abs() <= acc + want.abs() * (ulp + 2.0 ** -22) + 1e-30).all()
+    E, ff, ffs = 15, K // 16 // 64 * 64, K - 15 * (K // 16 // 64 * 64)
+    wts = torch.zeros(M, E, device="cuda")
+    wts[0, 3], wts[M - 1, E - 1] = 0.5, 0.5
+    on = torch.zeros(E, dtype=torch.bool, device="cuda")
+    on[3] = on[E - 1] = True
+    seen = torch.cat([on.repeat_interleave(ff), torch.ones(ffs, dtype=torch.bool, device="cuda")])
+    want = (x.double() * seen) @ w.double().t()
+    y = thin_linear(x, w.masked_fill(~seen, float("nan")), None, torch.float32, (wts, E, ff, ffs))
+    assert ((y.double() - want).abs() <= acc + want.abs() * 2.0 ** -23).all()
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 2.0 ** -8), (torch.float16, 2.0 ** -11)])
+@pytest.mark.parametrize("M,K,ff", [(1, 1024, 4112), (8, 1088, 6144), (9, 1024, 4112), (16, 1024, 6144), (16, 1024, 6160), (7, 1024, 8208)])
+def test_gated_tiles_of_eight_columns(M, K, ff, dtype, tol):
+    """One and two rounds of 16-column tiles and up to half of another."""
+    g = torch.Generator(device="cuda").manual_seed(M + ff)
+    h = torch.randn(M, K, device="cuda", generator=g).to(dtype)
+    w = (torch.randn(2 * ff, K, device="cuda", generator=g) / K ** 0.5).to(dtype)
+    z = h.double() @ w.double().t()
+    for act in ("silu", ClampedGate(1.0, 0.7, 1.702, 1.0)):
+        got = thin_act(h, w, None, 0, 0, ff, act, True, "output").double()
+        gate, up = z[:, :ff], z[:, ff:]
+        if act == "silu":
+            want = gate * torch.sigmoid(gate) * up
+        else:
+            gate, up = gate.clamp(max=act.limit_shared), up.clamp(-act.limit_shared, act.limit_shared)
+            want = gate * torch.sigmoid(act.slope * gate) * (up + act.shift)
+        assert ((got - want).abs() <= 1.05 * tol * want.abs() + 2e-5 * want.abs().max()).all()

@@ -320,29 +320,36 @@ __device__ __forceinline__ float sumsq8(uint4 v) {
   return s;
 }
 
+// KS 2 (few workgroups, see kSplit): 64 rows, a row's keys shared by two waves, each one half of every tile; the upper half's maximum, sum and
+// accumulators meet the lower one's in LDS at the end.
 // (register budget: left to itself the compiler takes > 300 registers and runs one wave per SIMD.  Two waves
 // for heads of 96 and 128, where three spill; of 256 two with spills are ahead of one without)
-template <typename T, int D, int NW, int KT>
+template <typename T, int D, int NW, int KT, int KS = 1>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 3 : 2)))
 tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ cache,
                  T* __restrict__ out, const int* __restrict__ tables, int maxb,
                  const int* __restrict__ tiles, const int* __restrict__ cu,
                  const int* __restrict__ start, int H, int G, int bs, float scale, float eps,
                  int chunk, int sink) {
-  constexpr int QT = 32 * NW, LK = D + 8, LT = KT + 8, NV = D / 8, SB = KT / 32;
+  constexpr int QT = 32 * NW / KS, LK = D + 8, LT = KT + 8, NV = D / 8, SB = KT / 32, WB = SB / KS;
+  static_assert(SB % KS == 0 && NW % KS == 0, "a wave's keys of a tile");
   // two buffers: a tile is stored while the one before it is read, one barrier per tile
   constexpr int NB = D <= 128 ? 2 : 1;
-  __shared__ __align__(16) T s_kb[NB][KT * LK];   // key tile, row-major
-  __shared__ __align__(16) T s_tb[NB][D * LT];    // key tile, transposed [d][key]
+  __shared__ __align__(16) T s_all[NB * (KT * LK + D * LT)];
+  T (*const s_kb)[KT * LK] = reinterpret_cast<T (*)[KT * LK]>(s_all);                    // key tile, row-major
+  T (*const s_tb)[D * LT] = reinterpret_cast<T (*)[D * LT]>(s_all + NB * KT * LK);       // key tile, transposed [d][key]
+  static_assert(KS == 1 || NW / 2 * (D / 2 + 2) * 64 * 4 <= (int)sizeof(s_all), "the other halves' results");
   __shared__ float s_nb[NB][KT];                  // 1 / rms of the tile's keys (power-of-two D / 8)
   constexpr int kTbl = 512;                   // block-table entries of the visible keys, in LDS
   __shared__ int s_tbl[kTbl];
   constexpr bool kStagedNorm = (NV & (NV - 1)) == 0 && NV <= 64;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 31, hi = lane >> 5;
+  const int tid = threadIdx.x, lane = tid & 63, w = (tid >> 6) % (NW / KS), c = lane & 31, hi = lane >> 5;
+  const int kb = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane((tid >> 6) / (NW / KS)) * WB;    // first block of 32 keys of a tile that the wave takes
   int tix, hd;
   heavy_first(blockIdx.x, gridDim.x, H, tix, hd);
   const int g = hd / (H / G);
-  const int sg = tiles[2 * tix], row0 = tiles[2 * tix + 1];
+  const int sg = tiles[2 * (tix / KS)], row0 = tiles[2 * (tix / KS) + 1] + tix % KS * QT;
+  if (KS > 1 && row0 >= cu[sg + 1]) return;              // (the whole workgroup: a tile of the list with few rows)
   const int seg_r0 = cu[sg], p0 = start[sg];
   const int nrows = min(QT, cu[sg + 1] - row0);
   const int* tbl = tables + (long long)sg * maxb;
@@ -377,7 +384,7 @@ tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ c
   const int bshift = (bs & (bs - 1)) == 0 ? __ffs(bs) - 1 : -1;
   __syncthreads();
 
-  float m = sink ? 0.f : -INFINITY, l = sink && hi == 0 ? 1.f : 0.f;   // (l: the lane's half)
+  float m = sink && kb == 0 ? 0.f : -INFINITY, l = sink && kb == 0 && hi == 0 ? 1.f : 0.f;   // (l: the lane's half)
   f32x16 O[D / 32];
 #pragma unroll
   for (int db = 0; db < D / 32; ++db)
@@ -463,15 +470,16 @@ tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ c
     }
   };
 
-  const int t0 = c * LT + 4 * (hi ^ (c >> 3)), t1 = c * LT + 4 * ((2 + hi) ^ (c >> 3));
+  const int t0 = c * LT + 4 * (hi ^ (c >> 3)) + 32 * kb, t1 = c * LT + 4 * ((2 + hi) ^ (c >> 3)) + 32 * kb;
   // the wave's share of tile k0
-  auto tile = [&](int k0, const T* s_k, const T* s_t, const float* s_kn) __attribute__((always_inline)) {
-    if (!wave_on || k0 > wpos_max || k0 + KT - 1 < wlo_min) return;   // nothing this wave may see
+  auto tile = [&](int kt, const T* s_k, const T* s_t, const float* s_kn) __attribute__((always_inline)) {
+    const int k0 = kt + 32 * kb;             // first of the wave's keys
+    if (!wave_on || k0 > wpos_max || k0 + 32 * WB - 1 < wlo_min) return;   // nothing this wave may see
 
-    f32x16 sc[SB];
-    float k2[SB], kn[SB];
+    f32x16 sc[WB];
+    float k2[WB], kn[WB];
 #pragma unroll
-    for (int b = 0; b < SB; ++b) {
+    for (int b = 0; b < WB; ++b) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) sc[b][r] = 0.f;
       k2[b] = kn[b] = 0.f;
@@ -479,14 +487,14 @@ tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ c
 #pragma unroll
     for (int kk = 0; kk < D / 16; ++kk)
 #pragma unroll
-      for (int b = 0; b < SB; ++b) {
-        const uint4 a = *reinterpret_cast<const uint4*>(&s_k[(32 * b + c) * LK + 16 * kk + 8 * hi]);
+      for (int b = 0; b < WB; ++b) {
+        const uint4 a = *reinterpret_cast<const uint4*>(&s_k[(32 * (kb + b) + c) * LK + 16 * kk + 8 * hi]);
         if (!kStagedNorm) k2[b] += sumsq8<T>(a);
         sc[b] = Mma32<T>::run(a, qreg[kk], sc[b]);
       }
     if (!kStagedNorm) {                                  // of key k0 + 32 b + c (other head sizes)
 #pragma unroll
-      for (int b = 0; b < SB; ++b) {
+      for (int b = 0; b < WB; ++b) {
         k2[b] += __shfl_xor(k2[b], 32, 64);
         kn[b] = 1.f / sqrtf(k2[b] / D + eps);
       }
@@ -494,18 +502,18 @@ tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ c
     // register r of sc[b] is key k0 + key_of(b, r)
     const auto key_of = [&](int b, int r) { return 32 * b + 8 * (r >> 2) + 4 * hi + (r & 3); };
     // a tile every query of the wave sees whole needs no mask
-    const bool whole = k0 >= (chunk > 0 ? (wpos_max / chunk) * chunk : 0) && k0 + KT - 1 <= wpos_min &&
+    const bool whole = k0 >= (chunk > 0 ? (wpos_max / chunk) * chunk : 0) && k0 + 32 * WB - 1 <= wpos_min &&
                        32 * w + 31 < nrows;
 #pragma unroll
-    for (int b = 0; b < SB; ++b)
+    for (int b = 0; b < WB; ++b)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float knr = kStagedNorm ? s_kn[key_of(b, r)] : __shfl(kn[b], key_of(0, r), 64);
+        const float knr = kStagedNorm ? s_kn[32 * kb + key_of(b, r)] : __shfl(kn[b], key_of(0, r), 64);
         sc[b][r] *= qn * knr;
       }
     if (!whole) {
 #pragma unroll
-      for (int b = 0; b < SB; ++b)
+      for (int b = 0; b < WB; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int j = k0 + key_of(b, r);
@@ -514,7 +522,7 @@ tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ c
     }
     float mloc = -INFINITY;
 #pragma unroll
-    for (int b = 0; b < SB; ++b)
+    for (int b = 0; b < WB; ++b)
 #pragma unroll
       for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, sc[b][r]);
     mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
@@ -534,12 +542,12 @@ tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ c
     // (v_exp_f32: this kernel serves 16-bit dtypes only, the weights are rounded to ~16 bits)
     float psum = 0.f;
 #pragma unroll
-    for (int b = 0; b < SB; ++b)
+    for (int b = 0; b < WB; ++b)
 #pragma unroll
       for (int r = 0; r < 16; ++r) { sc[b][r] = __expf(sc[b][r] - ms); psum += sc[b][r]; }
     l += psum;                                 // (the lane's half: the other lane's is added at the end)
 #pragma unroll
-    for (int s2 = 0; s2 < 2 * SB; ++s2) {
+    for (int s2 = 0; s2 < 2 * WB; ++s2) {
       unsigned ph[4], pl[4];
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
@@ -586,6 +594,27 @@ tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ c
       if (more) commit(k0 + KT, s_kb[cur ^ 1], s_tb[cur ^ 1], s_nb[cur ^ 1]);
       __syncthreads();
     }
+  }
+  if constexpr (KS == 2) {                   // the upper keys' waves hand their sums to the lower ones'
+    float* box = reinterpret_cast<float*>(s_all) + w * (D / 2 + 2) * 64 + lane;
+    if (kb > 0) {
+#pragma unroll
+      for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) box[(16 * db + r) * 64] = O[db][r];
+      box[D / 2 * 64] = m;
+      box[(D / 2 + 1) * 64] = l;
+    }
+    __syncthreads();
+    if (kb > 0) return;
+    const float m2 = box[D / 2 * 64], mn = fmaxf(m, m2);
+    const float c1 = m == mn ? 1.f : __expf(m - mn), c2 = m2 == mn ? 1.f : __expf(m2 - mn);
+    l = l * c1 + box[(D / 2 + 1) * 64] * c2;
+    m = mn;
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) O[db][r] = O[db][r] * c1 + box[(16 * db + r) * 64] * c2;
   }
   l += __shfl_xor(l, 32, 64);
   // A hidden key has weight 0, but 0 times an infinite or NaN value is NaN: channels that are not finite are formed
@@ -651,6 +680,12 @@ tile_attn_kernel(const T* __restrict__ q, long long ldq, const T* __restrict__ c
   }
 }
 
+// Tiles of 128 rows by heads up to which tiles of 64 rows with the keys in halves are faster: the exponentials and conversions of a wave's
+// scores bound the chain of key tiles, and few workgroups leave half of the vector units idle.  us, whole -> in halves, 16 heads of 128:
+// 1 x 512 tokens 33.8 -> 27.4 (chunks of 256 20.7 -> 17.1), 1 x 1024 59.8 -> 48.0, 4 x 512 34.3 -> 29.9; 5 x 512 37.0 -> 40.0; heads of 64, 1 x
+// 512 26.0 -> 21.9.
+constexpr int kSplit = 256;
+
 template <typename T>
 hipError_t launch_tiles(const void* q, long long ldq, const void* cache, void* out,
                         const int* tables, int maxb, const int* tiles, int ntiles, const int* cu,
@@ -660,6 +695,14 @@ hipError_t launch_tiles(const void* q, long long ldq, const void* cache, void* o
 #define GO(DD)                                                                                   \
   {                                                                                              \
     constexpr int KT = DD <= 128 ? 64 : 32;                                                      \
+    if constexpr (KT == 64) {                                                                    \
+      if (tile_rows == 128 && (long long)ntiles * H <= kSplit) {                                   \
+        tile_attn_kernel<T, DD, 4, KT, 2><<<2 * grid.x, 256, 0, st>>>((const T*)q, ldq, (const T*)cache, (T*)out, \
+                                                       tables, maxb, tiles, cu, start, H, G, bs, \
+                                                       scale, eps, chunk, sink);                 \
+        return hipGetLastError();                                                                \
+      }                                                                                          \
+    }                                                                                            \
     if (tile_rows == 128)                                                                        \
       tile_attn_kernel<T, DD, 4, KT><<<grid, 256, 0, st>>>((const T*)q, ldq, (const T*)cache, (T*)out, \
                                                        tables, maxb, tiles, cu, start, H, G, bs, \

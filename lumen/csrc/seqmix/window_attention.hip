@@ -28,6 +28,10 @@
 // results at the end, which later came to it, 0.1 - 1.3 us (8 x 512 x 16 39.0 -> 39.7, 1 x 64 9.2 -> 9.5; with a comparison
 // per result 0.3 - 1.9).  A portion of few keys pays for a whole tile of 64 (1 x 16 7.4 -> 9.0, 64 x 5 x 32 heads 22 -> 31).
 //
+// The exponentials and conversions of a wave's scores bound that chain, so few workgroups (kSplit below) leave half of the chip's vector
+// units idle: there a workgroup takes 64 rows and KS = 2 waves share a row's keys, each one half of every tile; the upper half's
+// maximum, sum and accumulators meet the lower one's in LDS at the end.
+//
 // Per wave (32 queries) and 32 keys, with v_mfma_f32_32x32x16:
 //   S^T = K Q^T      keys on the accumulator rows, queries on the columns (lane & 31): a lane
 //                    owns ONE query, so its running max / sum / correction are plain scalars;
@@ -88,23 +92,28 @@ constexpr int kDr = 64;
 // 58), 8 x 512 224 -> 65, 1 x 512 72 -> 42, 1 x 30 60 -> 29, 1 x 2048 x 32 714 -> 141: at every size.  Error against
 // float64, absorbed -> expanded: bf16 2.53e-3 -> 2.51e-3 and 2.57e-3 -> 2.53e-3, fp16 3.16e-4 -> 3.15e-4 (the weights through
 // __expf; with an exponential near to the last bit the same, and 34 -> 40 us for 1 x 512).
-template <typename T, int D, int DV, int NW, int KT, bool FRESH = false>
+template <typename T, int D, int DV, int NW, int KT, bool FRESH = false, int KS = 1>
 __global__ void __launch_bounds__(64 * NW)
     __attribute__((amdgpu_waves_per_eu((D <= 128 || FRESH) && DV <= 128 ? 2 : 1)))
 win_tile_attn_kernel(const WinTileArgs<T> a) {
-  constexpr int QT = 32 * NW, LK = D + 8, LT = KT + 8, NV = D / 8, NVV = DV / 8, SB = KT / 32;
+  constexpr int QT = 32 * NW / KS, LK = D + 8, LT = KT + 8, NV = D / 8, NVV = DV / 8, SB = KT / 32, WB = SB / KS;
+  static_assert(SB % KS == 0 && NW % KS == 0, "a wave's keys of a tile");
   // two buffers: a tile is stored while the one before it is read, one barrier per tile
-  __shared__ __align__(16) T s_kb[2][KT * LK];    // key tile, row-major
-  __shared__ __align__(16) T s_tb[2][DV * LT];    // value tile, transposed [d][key]
+  __shared__ __align__(16) T s_all[2 * KT * LK + 2 * DV * LT];
+  T (*const s_kb)[KT * LK] = reinterpret_cast<T (*)[KT * LK]>(s_all);                    // key tile, row-major
+  T (*const s_tb)[DV * LT] = reinterpret_cast<T (*)[DV * LT]>(s_all + 2 * KT * LK);      // value tile, transposed [d][key]
+  static_assert(KS == 1 || NW / 2 * (DV / 2 + 2) * 64 * 4 <= (int)sizeof(s_all), "the other halves' results");
   constexpr int kTbl = 512;                   // block-table entries of the window's keys, in LDS
   __shared__ int s_tbl[kTbl];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 31, hi = lane >> 5;
+  const int tid = threadIdx.x, lane = tid & 63, w = (tid >> 6) % (NW / KS), c = lane & 31, hi = lane >> 5;
+  const int kb = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane((tid >> 6) / (NW / KS)) * WB;    // first block of 32 keys of a tile that the wave takes
   int tix, hd;
   heavy_first(blockIdx.x, gridDim.x, a.H, tix, hd);
   const int g = hd / (a.H / a.G);
   const int Gv = a.G / a.vdiv, gv = g / a.vdiv;
   const float sbias = a.sigb != nullptr ? a.sigb[hd] : 0.f;
-  const int sg = a.tiles[2 * tix], row0 = a.tiles[2 * tix + 1];
+  const int sg = a.tiles[2 * (tix / KS)], row0 = a.tiles[2 * (tix / KS) + 1] + tix % KS * QT;
+  if (KS > 1 && row0 >= a.cu[sg + 1]) return;            // (the whole workgroup: a tile of the list with few rows)
   const int seg_r0 = a.cu[sg], p0 = a.start[sg];
   const int nrows = min(QT, a.cu[sg + 1] - row0);
   const int* tbl = a.tables + (long long)sg * a.maxb;
@@ -242,48 +251,49 @@ win_tile_attn_kernel(const WinTileArgs<T> a) {
     }
   };
 
-  const int t0 = c * LT + 4 * (hi ^ (c >> 3)), t1 = c * LT + 4 * ((2 + hi) ^ (c >> 3));
+  const int t0 = c * LT + 4 * (hi ^ (c >> 3)) + 32 * kb, t1 = c * LT + 4 * ((2 + hi) ^ (c >> 3)) + 32 * kb;
   // the wave's share of tile k0
-  auto tile = [&](int k0, const T* s_k, const T* s_t) __attribute__((always_inline)) {
+  auto tile = [&](int kt, const T* s_k, const T* s_t) __attribute__((always_inline)) {
+    const int k0 = kt + 32 * kb;             // first of the wave's keys
     // nothing this wave may see: past its last row, or before its first row's window and not kept
     if (!wave_on || k0 > wpos_max ||
-        (window > 0 && k0 + KT - 1 < wpos_min - window + 1 && k0 >= keep))
+        (window > 0 && k0 + 32 * WB - 1 < wpos_min - window + 1 && k0 >= keep))
       return;
 
-    f32x16 sc[SB];
+    f32x16 sc[WB];
 #pragma unroll
-    for (int b = 0; b < SB; ++b)
+    for (int b = 0; b < WB; ++b)
 #pragma unroll
       for (int r = 0; r < 16; ++r) sc[b][r] = 0.f;
 #pragma unroll
     for (int kk = 0; kk < D / 16; ++kk)
 #pragma unroll
-      for (int b = 0; b < SB; ++b)
-        sc[b] = Mma32<T>::run(*reinterpret_cast<const uint4*>(&s_k[(32 * b + c) * LK + 16 * kk + 8 * hi]),
+      for (int b = 0; b < WB; ++b)
+        sc[b] = Mma32<T>::run(*reinterpret_cast<const uint4*>(&s_k[(32 * (kb + b) + c) * LK + 16 * kk + 8 * hi]),
                               qreg[kk], sc[b]);
     // register r of sc[b] is key k0 + key_of(b, r)
     const auto key_of = [&](int b, int r) { return 32 * b + 8 * (r >> 2) + 4 * hi + (r & 3); };
     // a tile every query of the wave sees whole needs no mask
-    const bool whole = k0 + KT - 1 <= wpos_min && 32 * w + 31 < nrows &&
-                       (window <= 0 || k0 >= wpos_max - window + 1 || k0 + KT - 1 < keep);
+    const bool whole = k0 + 32 * WB - 1 <= wpos_min && 32 * w + 31 < nrows &&
+                       (window <= 0 || k0 >= wpos_max - window + 1 || k0 + 32 * WB - 1 < keep);
 #pragma unroll
-    for (int b = 0; b < SB; ++b) sc[b] *= a.scale;
+    for (int b = 0; b < WB; ++b) sc[b] *= a.scale;
     if (cap > 0.f) {
 #pragma unroll
-      for (int b = 0; b < SB; ++b)
+      for (int b = 0; b < WB; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r) sc[b][r] = cap * tanh_exp(sc[b][r] * rcap);
     }
     if (a.slopes != nullptr) {
       const float d0 = (float)(pos - k0);
 #pragma unroll
-      for (int b = 0; b < SB; ++b)
+      for (int b = 0; b < WB; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r) sc[b][r] -= slope * (d0 - (float)key_of(b, r));
     }
     if (!whole) {
 #pragma unroll
-      for (int b = 0; b < SB; ++b)
+      for (int b = 0; b < WB; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int j = k0 + key_of(b, r);
@@ -294,13 +304,13 @@ win_tile_attn_kernel(const WinTileArgs<T> a) {
     if (a.sigb != nullptr) {
       // weights as they are: a hidden key's -inf gives 1 / (1 + e^inf) = 0
 #pragma unroll
-      for (int b = 0; b < SB; ++b)
+      for (int b = 0; b < WB; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r) sc[b][r] = 1.f / (1.f + __expf(-(sc[b][r] + sbias)));
     } else {
       float mloc = -INFINITY;
 #pragma unroll
-      for (int b = 0; b < SB; ++b)
+      for (int b = 0; b < WB; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, sc[b][r]);
       mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
@@ -320,13 +330,13 @@ win_tile_attn_kernel(const WinTileArgs<T> a) {
       // (v_exp_f32: this kernel serves 16-bit dtypes only, the weights are rounded to ~16 bits)
       float psum = 0.f;
 #pragma unroll
-      for (int b = 0; b < SB; ++b)
+      for (int b = 0; b < WB; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r) { sc[b][r] = __expf(sc[b][r] - ms); psum += sc[b][r]; }
       l += psum;                               // (the lane's half: the other lane's is added at the end)
     }
 #pragma unroll
-    for (int s2 = 0; s2 < 2 * SB; ++s2) {
+    for (int s2 = 0; s2 < 2 * WB; ++s2) {
       unsigned ph[4], pl[4];
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
@@ -365,6 +375,27 @@ win_tile_attn_kernel(const WinTileArgs<T> a) {
     if (kn <= kend) commit(kn, s_kb[cur ^ 1], s_tb[cur ^ 1]);
     __syncthreads();
     k0 = kn;
+  }
+  if constexpr (KS == 2) {                   // the upper keys' waves hand their sums to the lower ones'
+    float* box = reinterpret_cast<float*>(s_all) + w * (DV / 2 + 2) * 64 + lane;
+    if (kb > 0) {
+#pragma unroll
+      for (int db = 0; db < DV / 32; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) box[(16 * db + r) * 64] = O[db][r];
+      box[DV / 2 * 64] = m;
+      box[(DV / 2 + 1) * 64] = l;
+    }
+    __syncthreads();
+    if (kb > 0) return;
+    const float m2 = box[DV / 2 * 64], mn = fmaxf(m, m2);
+    const float c1 = m == mn ? 1.f : __expf(m - mn), c2 = m2 == mn ? 1.f : __expf(m2 - mn);
+    l = l * c1 + box[(DV / 2 + 1) * 64] * c2;
+    m = mn;
+#pragma unroll
+    for (int db = 0; db < DV / 32; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) O[db][r] = O[db][r] * c1 + box[(16 * db + r) * 64] * c2;
   }
   l += __shfl_xor(l, 32, 64);
   // A hidden key has weight 0, but 0 times an infinite or NaN value is NaN: channels that are not finite are formed
@@ -432,6 +463,13 @@ win_tile_attn_kernel(const WinTileArgs<T> a) {
   }
 }
 
+// Tiles of 128 rows by heads up to which tiles of 64 rows with the keys in halves are faster.  us, whole -> in halves: heads of 128
+// 64 workgroups (1 x 512 x 16) 28.5 -> 21.4, 128 (x 32, soft cap) 33.0 -> 23.8, 256 (1 x 1024 x 32) 58.1 -> 44.9, (4 x 512 x 16) 30.2 -> 25.4, 100
+// rows behind 3000 keys 182 -> 126; 320 35.7 -> 34.8, 512 (8 x 512 x 16) 37.4 -> 47.1; heads of 64, 128 21.0 -> 15.7.  Two such workgroups share
+// a CU; of the fresh form one does: 64 workgroups (1 x 512 x 16) 33.3 -> 24.9, 128 (1 x 2048 x 8) 106.8 -> 76.6, 192 34.0 -> 40.1; its
+// key tiles are longer then, for nothing with portions of up to 64 rows (30 rows 6.8 -> 8.7).
+constexpr int kSplit = 256, kSplitFresh = 128;
+
 template <typename T>
 hipError_t launch_win_tiles(const WinTileArgs<T>& a, int ntiles, int D, int Dv, int tile_rows,
                             hipStream_t st) {
@@ -439,6 +477,12 @@ hipError_t launch_win_tiles(const WinTileArgs<T>& a, int ntiles, int D, int Dv, 
 #define GO(DD, DVV)                                                                          \
   {                                                                                          \
     constexpr int KT = DVV <= 128 ? 64 : 32;                                                 \
+    if constexpr (KT == 64) {                                                                \
+      if (tile_rows == 128 && (long long)ntiles * a.H <= kSplit) {                           \
+        win_tile_attn_kernel<T, DD, DVV, 4, KT, false, 2><<<2 * grid.x, 256, 0, st>>>(a);    \
+        return hipGetLastError();                                                            \
+      }                                                                                      \
+    }                                                                                        \
     if (tile_rows == 128) win_tile_attn_kernel<T, DD, DVV, 4, KT><<<grid, 256, 0, st>>>(a);  \
     else win_tile_attn_kernel<T, DD, DVV, 2, KT><<<grid, 128, 0, st>>>(a);                   \
   }
@@ -462,9 +506,11 @@ hipError_t launch_win_tiles(const WinTileArgs<T>& a, int ntiles, int D, int Dv, 
 }
 
 template <typename T>
-hipError_t launch_fresh_tiles(const WinTileArgs<T>& a, int ntiles, int tile_rows, hipStream_t st) {
+hipError_t launch_fresh_tiles(const WinTileArgs<T>& a, int rows, int ntiles, int tile_rows, hipStream_t st) {
   const dim3 grid((unsigned)((long long)ntiles * a.H));
-  if (tile_rows == 128) win_tile_attn_kernel<T, 192, 128, 4, 32, true><<<grid, 256, 0, st>>>(a);
+  if (tile_rows == 128 && (long long)ntiles * a.H <= kSplitFresh && rows > 64LL * ntiles)
+    win_tile_attn_kernel<T, 192, 128, 4, 64, true, 2><<<2 * grid.x, 256, 0, st>>>(a);
+  else if (tile_rows == 128) win_tile_attn_kernel<T, 192, 128, 4, 32, true><<<grid, 256, 0, st>>>(a);
   else win_tile_attn_kernel<T, 192, 128, 2, 32, true><<<grid, 128, 0, st>>>(a);
   return hipGetLastError();
 }
@@ -476,17 +522,17 @@ extern "C" {
 // Prompts from position 0 whose keys and values are rows of the step: q rows [T][>= H * (D1 + Dr)], k rows
 // [T][>= H * D1] and v rows [T][>= H * Dv] head after head, kr rows [T][>= Dr] the key part all heads share;
 // D1 = Dv = 128, Dr = 64; row strides % 8, 16-byte aligned bases; out [T][H][Dv] contiguous; tiles, cu and start
-// as below (every start is 0).
+// as below (every start is 0); rows: of all tiles.
 int sm_fresh_tiles_ok(int dt, int D1, int Dr, int Dv) {
   return (dt == kBF16 || dt == kF16) && D1 == 128 && Dr == kDr && Dv == 128;
 }
 
 hipError_t sm_fresh_tiles(int dt, const void* q, long long ldq, const void* k, long long ldk, const void* kr,
-                          long long ldr, const void* v, long long ldv, void* out, const int* tiles, int ntiles,
+                          long long ldr, const void* v, long long ldv, void* out, const int* tiles, int rows, int ntiles,
                           int tile_rows, const int* cu, const int* start, int H, int D1, int Dr, int Dv,
                           float scale, hipStream_t st) {
   if (ntiles == 0) return hipSuccess;
-  if (!sm_fresh_tiles_ok(dt, D1, Dr, Dv) || ntiles < 0 || H < 1 || (tile_rows != 64 && tile_rows != 128) ||
+  if (!sm_fresh_tiles_ok(dt, D1, Dr, Dv) || ntiles < 0 || rows < 0 || H < 1 || (tile_rows != 64 && tile_rows != 128) ||
       ldq % 8 || ldk % 8 || ldr % 8 || ldv % 8 || ldq < (long long)H * (D1 + Dr) || ldk < (long long)H * D1 ||
       ldr < Dr || ldv < (long long)H * Dv ||
       ((uintptr_t)q | (uintptr_t)k | (uintptr_t)kr | (uintptr_t)v) % 16 || (uintptr_t)out % 8)
@@ -495,7 +541,7 @@ hipError_t sm_fresh_tiles(int dt, const void* q, long long ldq, const void* k, l
   {                                                                                                       \
     WinTileArgs<TT> a{(const TT*)q, ldq, (const TT*)k, (const TT*)v, (const TT*)kr, ldk, ldv, ldr, (TT*)out, \
                       nullptr, 0, nullptr, 0, tiles, cu, start, H, H, 1, scale, 0.f, nullptr, 0, 0, nullptr, 1}; \
-    return launch_fresh_tiles<TT>(a, ntiles, tile_rows, st);                                              \
+    return launch_fresh_tiles<TT>(a, rows, ntiles, tile_rows, st);                                        \
   }
   if (dt == kBF16) CALL(bf16)
   CALL(fp16)

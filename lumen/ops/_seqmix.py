@@ -42,7 +42,7 @@ SIGNATURES = {
     "sm_row_attn": "i" "plli" "plli" "pl" "pli" "pll" "pi" "pp" "iiiii" "fffi" "pppp" "piipl"
                    "pi" "iipp",
     "sm_win_attn_tiles": "iplppppl" "pi" "pi" "pp" "iiii" "ff" "p" "iii" "ipi",
-    "sm_fresh_tiles": "i" "plplplpl" "p" "pii" "pp" "iiii" "f",
+    "sm_fresh_tiles": "i" "plplplpl" "p" "piii" "pp" "iiii" "f",
     "sm_talk_tiles": "i" "pll" "pp" "pll" "pi" "pii" "pp" "iiiii" "fffi" "pppp",
     "sm_expert_sort": "pppppiii",
     "sm_expert_act": "iplp" "ppppp" "iiiiii" "iii" "ffff",

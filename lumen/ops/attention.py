@@ -773,7 +773,7 @@ def fresh_latent_attention(q: torch.Tensor, k: torch.Tensor, kr: torch.Tensor, v
     if not use_seqmix(q):
         return fresh_latent_attention_ref(q, k, kr, v, out, seg, scale)
     call("sm_fresh_tiles", DT[q.dtype], q, q.stride(0), k, k.stride(0), kr, kr.stride(0), v, v.stride(0), out,
-         seg.q_tiles, seg.q_tiles.shape[0], seg.tile_size, seg.cu, seg.start, H, D, Dr, Dv, scale)
+         seg.q_tiles, seg.tile_rows, seg.q_tiles.shape[0], seg.tile_size, seg.cu, seg.start, H, D, Dr, Dv, scale)
     return out
 
 

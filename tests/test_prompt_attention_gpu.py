@@ -49,7 +49,7 @@ def close(out, ref, ulp):
     ([31, 32, 33, 63, 64, 65, 1], [0, 0, 1, 0, 70, 3, 5], 16, 0, 0),
     ([127, 128, 129], [0, 64, 1], 12, 70, 5), ([130, 66], [200, 61], 16, 64, 130), ([40, 5], [560, 0], 1, 0, 0),
     ([33], [700], 1, 620, 7)])
-@pytest.mark.parametrize("H,G,D,Dv", [(4, 2, 128, 128), (2, 2, 32, 64), (2, 1, 128, 256)])
+@pytest.mark.parametrize("H,G,D,Dv", [(4, 2, 128, 128), (2, 2, 32, 64), (2, 1, 128, 256), (258, 2, 32, 32), (258, 6, 64, 128)])
 def test_window_tiles(H, G, D, Dv, lens, starts, bs, window, keep, dtype, ulp):
     g = torch.Generator().manual_seed(D + bs + len(lens))
     T, seg, (k, v) = portions(lens, starts, bs, g, (G, D), (G, Dv))
@@ -67,7 +67,7 @@ def test_window_tiles(H, G, D, Dv, lens, starts, bs, window, keep, dtype, ulp):
 @pytest.mark.parametrize("lens,starts,bs,chunk", [
     ([31, 32, 33, 63, 64, 65, 1], [0, 0, 1, 0, 70, 3, 5], 16, 0), ([127, 128, 129], [0, 64, 1], 12, 75),
     ([40, 5], [560, 0], 1, 0)])
-@pytest.mark.parametrize("H,G,D", [(4, 2, 128), (2, 1, 96), (2, 2, 256)])
+@pytest.mark.parametrize("H,G,D", [(4, 2, 128), (2, 1, 96), (2, 2, 256), (258, 2, 32)])
 def test_chunk_tiles(H, G, D, lens, starts, bs, chunk, dtype, ulp):
     g = torch.Generator().manual_seed(D + bs + len(lens))
     T, seg, (k,) = portions(lens, starts, bs, g, (G, D))

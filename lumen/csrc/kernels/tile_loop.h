@@ -2,9 +2,8 @@
 // four waves per CU; the kernels around it choose the rows and write the results.
 //
 //  * A wave owns 16 MJ x 16 NI results.  Operands come by LDS-DMA in stages of 64 k under counted waits, as many steps
-//    ahead as fit into 160 KiB (six at most); one barrier per step.  256 x 192 and wider keep three slots of x and two of
-//    w: then w's DMA goes out in the second half of a step and x's in the first, where the CU's one address path would be
-//    busy all of the second half with both (256 x 192: 0.88 -> 0.80 us a step).
+//    ahead as fit into 160 KiB (six at most); one barrier per step.  256 x 160 and wider keep two slots of x, which comes from
+//    L2, and three or four of w: loads return in the order they were sent for, and w from HBM takes longer than a step.
 //  * With w from HBM few-row tiles wait for bytes: a CU takes 97 B/ns from L2 and 60 of lines from HBM, however many are in
 //    flight (48 KB do), so the tile is as narrow in x as the rows are.  Rows of w some KB apart, read a stage at
 //    a time by all workgroups in step, meet in the same memory channels: the caller may have a tile start its walk of k
@@ -47,9 +46,11 @@ constexpr int CUS = 256;
 template <int NI, int MJ>
 struct Shape {
   static constexpr int BM = 32 * MJ, BN = 32 * NI, XB = BM * ROWB, WB = BN * ROWB;
-  static constexpr int FIT = 160 * 1024 / (XB + WB);
-  static constexpr int NST = FIT < 6 ? FIT : 6, NSX = NST < 3 ? 3 : NST;         // slots of w and x
+  static constexpr bool DEEP = MJ == 8 && NI >= 5;       // two slots of x, more of w
+  static constexpr int FIT = DEEP ? (160 * 1024 - 2 * XB) / WB : 160 * 1024 / (XB + WB);
+  static constexpr int NST = FIT < 6 ? FIT : 6, NSX = DEEP ? 2 : NST;            // slots of w and x
   static constexpr int LDS = NSX * XB + NST * WB;
+  static_assert(NST >= 3, "slots");
   static constexpr int PIECES = MJ + NI;                 // 1-KiB LDS-DMA pieces of a wave and stage: MJ of x, NI of w
 };
 
@@ -111,18 +112,30 @@ __device__ __forceinline__ int colperm(int w) {
 // (lane & 7) ^ swz(row).  APART: the walk starts at stage `turn` < nk and comes round to it.  Lane (lr, lg) holds row 16 j + lr of its
 // wave's x, rows 16 i + 4 lg .. + 3 of its w.  HALF: with `odd` the last stage holds 32 k; its lanes of the upper half read the lower
 // one again, which is multiplied once.
+//
+// Step t multiplies stage t; at its start the first half's fragments are in registers.  Behind the first half's products it
+// reads the second half's; then stage t + 1 has to be there, and every wave done with stage t, whose slots the second half's
+// pieces may take.
+//  * NST slots of both: the second half sends for the last pieces of stage t + NST, the next step's first half for its others.
+//  * DEEP: the second half sends for all of x of stage t + 2 and then w of stage t + NST, which thus has a step and a half before x of
+//    stage t + 3 has to be there, sent for after it.  With three slots of x and two of w it had half a step to one, and the
+//    card's memory answered later: 512 rows x 2 x 11264 x 4096 with activation (256 x 192) 89.8 -> 81.6 us, x 18560 (256 x 160) 78 -> 72, x
+//    22016 (256 x 192) 83.6 -> 78.8; 4096 x 2 x 11008 x 4096 (256 x 256) 554 -> 535 and 521 -> 515 (two cards).  256 x 128 was no faster so
+//    (512 x 16384 61.7 -> 62.6).
 template <typename T, int NI, int MJ, bool APART = false, bool HALF = false>
 __device__ __forceinline__ void products(char* lds, const char* xb, const char* wb, int nk, int turn,
                                          const unsigned (&off)[Shape<NI, MJ>::PIECES], f32x4 (&acc)[NI][MJ], bool odd = false) {
   using S = Shape<NI, MJ>;
   constexpr int NSX = S::NSX, NST = S::NST, XB = S::XB, WB = S::WB, PIECES = S::PIECES;
-  // pieces [PB, PIECES) of a stage go out behind a second half's products, [0, PB) behind the first half's
-  constexpr int PB = NST == 2 ? MJ : PIECES - PIECES / 2, F = NSX - 1;
+  constexpr bool DEEP = S::DEEP;
+  static_assert(!DEEP || !APART, "no caller has wide tiles walk apart");
+  constexpr int PB = PIECES - PIECES / 2, F = NST - 1;   // !DEEP: pieces [PB, PIECES) go out in a second half, [0, PB) in a first
   struct Slot { int x, w; };
   const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const unsigned lds0 = (unsigned)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds);
   const unsigned upper = HALF && odd && (((lane >> 2) ^ wid) & 1) ? BK : 0;     // (bytes; chunk (lane & 7) ^ swz(row) >= 4)
+  // pieces q0 .. q1 - 1 of stage t, of x (q < MJ) to slot.x, of w to slot.w
   auto issue = [&](int t, Slot slot, int q0, int q1) __attribute__((always_inline)) {
     const unsigned back = HALF && t == nk - 1 ? upper : 0;
     const int u = APART ? (t + turn < nk ? t + turn : t + turn - nk) : t;
@@ -149,10 +162,9 @@ __device__ __forceinline__ void products(char* lds, const char* xb, const char* 
       else fb[h][u - NI] = *reinterpret_cast<const uint4*>(px + rb0 + (u - NI) * 16 * ROWB);
   };
   // the products of half h; between them the reads of the other half's fragments (from stage slot fs, in the first
-  // three quarters) and pieces q0 .. q1 - 1 of stage `t` into slot `ds` (t < 0: none)
-  auto half = [&](int h, Slot fs, int t, Slot ds, int q0, int q1) __attribute__((always_inline)) {
+  // three quarters) and `send(a, b)` for pieces a .. b - 1 of P
+  auto half = [&](int h, Slot fs, int P, auto&& send) __attribute__((always_inline)) {
     constexpr int U = NI * MJ, R = NI + MJ, UR = U * 3 / 4;
-    const int P = q1 - q0;
 #pragma unroll
     for (int j = 0; j < MJ; ++j)
 #pragma unroll
@@ -160,42 +172,74 @@ __device__ __forceinline__ void products(char* lds, const char* xb, const char* 
         const int n = j * NI + i;
         mfma<T>(acc[i][j], fa[h][i], fb[h][j]);
         frags(1 - h, fs, min(R, (n * R + UR - 1) / UR), min(R, ((n + 1) * R + UR - 1) / UR));
-        if (t >= 0) issue(t, ds, q0 + n * P / U, q0 + (n + 1) * P / U);
+        send(n * P / U, (n + 1) * P / U);
         __builtin_amdgcn_sched_barrier(0);
       }
   };
+  const auto none = [](int, int) __attribute__((always_inline)) {};
   auto after = [](Slot s) __attribute__((always_inline)) {
     return Slot{s.x == NSX - 1 ? 0 : s.x + 1, s.w == NST - 1 ? 0 : s.w + 1};
   };
-  // Step t multiplies stage t; at its start the first half's fragments are in registers.  Behind the first
-  // half's products it reads the second half's and sends for pieces [0, PB) of stage t + F; then stage t + 1 has to be
-  // there, and every wave done with stage t.  NST > 2: its slots take the other pieces of stage t + NST behind the second
-  // half's products.  NST 2: its w slot takes the w pieces of stage t + 2.
-  Slot s0{0, 0}, s1{1, 1}, sf{F, F % NST};               // slots of stages t, t + 1, t + F
+  Slot s0{0, 0}, s1{1, 1};                               // slots of stages t, t + 1
+  int t = 0;
+  if constexpr (DEEP) {
+    // sent for in this order: w and x of stage 0, w of the others, x of stage 1, the last slot's w
+    issue(0, s0, MJ, PIECES);
+    issue(0, s0, 0, MJ);
 #pragma unroll
-  for (int u = 0; u < F; ++u)
-    if (u < nk) issue(u, Slot{u, u % NST}, 0, PIECES);
-  constexpr int first = (F - 1) * PIECES;                // what may be missing behind stage 0
-  if (NST > 2 && nk > F) issue(F, sf, PB, PIECES), wait_vm<first + (NST > 2 ? PIECES - PB : 0)>();
-  else if (nk >= F) wait_vm<first>();
-  else wait_vm<0>();
+    for (int u = 1; u < NST - 1; ++u)
+      if (u < nk) issue(u, Slot{0, u}, MJ, PIECES);
+    if (nk > 1) issue(1, s1, 0, MJ);
+    if (nk >= NST) issue(NST - 1, Slot{0, NST - 1}, MJ, PIECES), wait_vm<(NST - 1) * NI + MJ>();
+    else wait_vm<0>();
+  } else {
+#pragma unroll
+    for (int u = 0; u < F; ++u)
+      if (u < nk) issue(u, Slot{u, u}, 0, PIECES);
+    if (nk > F) issue(F, Slot{F, F}, PB, PIECES), wait_vm<(F - 1) * PIECES + PIECES - PB>();
+    else if (nk == F) wait_vm<(F - 1) * PIECES>();
+    else wait_vm<0>();
+  }
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   frags(0, s0, 0, NI + MJ);
-  int t = 0;
-  for (; t + NST < nk; ++t) {
-    half(0, s0, t + F, sf, 0, PB);
-    wait_vm<(NST > 2 ? first : PB)>();
-    done_reading();
-    half(1, s1, t + NST, NST > 2 ? s0 : Slot{sf.x, s0.w}, PB, PIECES);
-    s0 = s1, s1 = after(s1), sf = after(sf);
-  }
-  for (; t < nk; ++t) {                                  // the last stages
-    half(0, s0, t + F < nk ? t + F : -1, sf, 0, PB);
-    wait_stages<NST == 2 ? 0 : F - 1, PIECES>(nk - 2 - t);
-    done_reading();
-    if (!HALF || !odd || t + 1 < nk) half(1, s1, -1, s1, 0, 0);      // (the last step reads a slot that holds an earlier stage: unused)
-    s0 = s1, s1 = after(s1), sf = after(sf);
+  if constexpr (DEEP) {
+    for (; t + NST < nk; ++t) {
+      half(0, s0, 0, none);
+      wait_vm<NI>();                                     // (all but w of stage t + NST - 1)
+      done_reading();
+      half(1, s1, PIECES, [&](int a, int b) __attribute__((always_inline)) {
+        issue(t + 2, s0, min(a, MJ), min(b, MJ));
+        issue(t + NST, s0, max(a, MJ), max(b, MJ));
+      });
+      s0 = s1, s1 = after(s1);
+    }
+    for (; t < nk; ++t) {                                // the last stages
+      half(0, s0, 0, none);
+      wait_vm<0>();
+      done_reading();
+      if (!HALF || !odd || t + 1 < nk)                   // (the last step reads a slot that holds an earlier stage: unused)
+        half(1, s1, MJ, [&](int a, int b) __attribute__((always_inline)) {
+          if (t + 2 < nk) issue(t + 2, s0, a, b);
+        });
+      s0 = s1, s1 = after(s1);
+    }
+  } else {
+    Slot sf{F, F};                                       // slot of stage t + F
+    for (; t + NST < nk; ++t) {
+      half(0, s0, PB, [&](int a, int b) __attribute__((always_inline)) { issue(t + F, sf, a, b); });
+      wait_vm<(F - 1) * PIECES>();
+      done_reading();
+      half(1, s1, PIECES - PB, [&](int a, int b) __attribute__((always_inline)) { issue(t + NST, s0, PB + a, PB + b); });
+      s0 = s1, s1 = after(s1), sf = after(sf);
+    }
+    for (; t < nk; ++t) {                                // the last stages
+      half(0, s0, PB, [&](int a, int b) __attribute__((always_inline)) { if (t + F < nk) issue(t + F, sf, a, b); });
+      wait_stages<F - 1, PIECES>(nk - 2 - t);
+      done_reading();
+      if (!HALF || !odd || t + 1 < nk) half(1, s1, 0, none);
+      s0 = s1, s1 = after(s1), sf = after(sf);
+    }
   }
   settle();
 }

@@ -151,7 +151,7 @@ __device__ __forceinline__ void dma4_o(const void* g, const char* lds_wave_base)
 template <typename T, int SW>
 __device__ __forceinline__ void stage64_async_o(char* img, const T* base, long long ld, int r0,
                                                 int rmax) {
-  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int row = (wid * 4 + i) * 4 + (lane >> 4);
@@ -159,21 +159,6 @@ __device__ __forceinline__ void stage64_async_o(char* img, const T* base, long l
     int gr = r0 + row;
     gr = gr < rmax ? gr : rmax - 1;
     dma16_o(base + (long long)gr * ld + ch * 8, img + (wid * 4 + i) * 1024);
-  }
-}
-
-// 8-wave (512-thread) variant: wave w fills image rows [8w, 8w + 8) in 2 DMA instructions
-template <typename T, int SW>
-__device__ __forceinline__ void stage64_async8_o(char* img, const T* base, long long ld, int r0,
-                                                 int rmax) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int row = (wid * 2 + i) * 4 + (lane >> 4);
-    const int ch = (lane & 15) ^ swz_t<SW>(row);
-    int gr = r0 + row;
-    gr = gr < rmax ? gr : rmax - 1;
-    dma16_o(base + (long long)gr * ld + ch * 8, img + (wid * 2 + i) * 1024);
   }
 }
 
@@ -414,8 +399,12 @@ __device__ __forceinline__ long long ds_tile(const Args& a, int head, int seq_ba
   return ((long long)head * a.ds_total + seq_base + (causal ? qt * (qt + 1) / 2 + kt : qt * ns + kt)) * 8192;
 }
 
-template <typename T, bool CAUSAL, bool WDS = false>
-__global__ void __launch_bounds__(256, 2) bwd_dkdv_kernel(Args a) {
+//
+// NG 2: two groups of four waves share an item, one takes its even steps and one its odd ones, with stages of their own; their
+// sums meet in LDS at the end, dK's in group 0 and dV's in group 1, which store them.  For steps of few items: every item is
+// then under way from the start and the launch takes as long as the longest chain of (head, query tile) steps, which this halves.
+template <typename T, bool CAUSAL, bool WDS = false, int NG = 1>
+__global__ void __launch_bounds__(256 * NG, 3 - NG) bwd_dkdv_kernel(Args a) {
   constexpr int STAGE = 2 * IMG + 512;  // Q image | dO image | lse[64] | delta[64]
   // two stages filled by LDS-DMA one (head, q-tile) step ahead.  S = Q K^T and dP = dO V^T are
   // computed with the queries as MFMA rows, so the accumulator lane (key L, queries 4g + r of each
@@ -424,10 +413,12 @@ __global__ void __launch_bounds__(256, 2) bwd_dkdv_kernel(Args a) {
   // two SEPARATE LDS objects, the loop unrolled by two (see fwd32_kernel): with one array indexed
   // by (j & 1) the compiler put s_waitcnt vmcnt(0) after the barrier of every step (it could not
   // tell the in-flight prefetch from the tile being read), serialising the DMA ring
-  __shared__ __attribute__((aligned(16))) char bufA[STAGE];
-  __shared__ __attribute__((aligned(16))) char bufB[STAGE];
-  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  __shared__ __attribute__((aligned(16))) char allA[NG][STAGE];
+  __shared__ __attribute__((aligned(16))) char allB[NG][STAGE];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wid = wave & 3, g = NG > 1 ? wave >> 2 : 0;     // wave of the group, the group
   const int lr = lane & 15, lg = lane >> 4;
+  char *bufA = allA[g], *bufB = allB[g];
   // persistent (a.nitems > 0): a grid of ~2 workgroups per CU walks the (key tile, kv head)
   // items in the host's heaviest-first order.  One workgroup's dK/dV stores (and dS flush) are
   // then still draining while its next item's K / V fragments and first Q / dO stage load,
@@ -476,7 +467,7 @@ __global__ void __launch_bounds__(256, 2) bwd_dkdv_kernel(Args a) {
   };
   // stage 0's DMA and this wave's K / V fragment loads are in flight together (one latency,
   // not two, before the first step); the full drain below retires both
-  if (nsteps > 0) stage(0, bufA);
+  if (g < nsteps) stage(g, bufA);
   uint4 kf[4], vf[4];
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) {
@@ -489,13 +480,18 @@ __global__ void __launch_bounds__(256, 2) bwd_dkdv_kernel(Args a) {
 #pragma unroll
   for (int n = 0; n < 8; ++n) { dk[n] = f32x4{0.f, 0.f, 0.f, 0.f}; dv[n] = dk[n]; }
   auto step = [&](int j, char* st, char* nx) {
+    if (NG > 1 && j >= nsteps) {  // (an odd number of steps: the others' last one)
+      lds_fence_barrier();
+      lds_fence_barrier();
+      return;
+    }
     char* qimg = st;
     char* oimg = st + IMG;
     const float* s_lse = reinterpret_cast<const float*>(st + 2 * IMG);
     const float* s_del = s_lse + 64;
     const int q0 = qstart + (j % nq) * 64;
-    if (j + 1 < nsteps) {
-      stage(j + 1, nx);
+    if (j + NG < nsteps) {
+      stage(j + NG, nx);
       if (wid < 2) asm volatile("s_waitcnt vmcnt(9)" ::: "memory");
       else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
     } else {
@@ -568,11 +564,24 @@ __global__ void __launch_bounds__(256, 2) bwd_dkdv_kernel(Args a) {
       pend_off = ds_tile(a, kvh * grp + j / nq, ds_base, q0 / 64, k0 / 64, (L + 63) / 64, CAUSAL);
     lds_fence_barrier();  // stage buffer free for the DMA two steps ahead
   };
-  for (int j = 0; j < nsteps; j += 2) {
-    step(j, bufA, bufB);
-    if (j + 1 < nsteps) step(j + 1, bufB, bufA);
+  for (int j = 0; j < nsteps; j += 2 * NG) {
+    step(j + g, bufA, bufB);
+    if (j + NG < nsteps) step(j + NG + g, bufB, bufA);
   }
   if constexpr (WDS) store_pend();
+  if constexpr (NG > 1) {
+    const auto meet = [&](const f32x4(&give)[8], f32x4(&keep)[8], char* mine, const char* theirs) {
+      const int at = (wid * 512 + lane) * 16;
+#pragma unroll
+      for (int n = 0; n < 8; ++n) *reinterpret_cast<f32x4*>(mine + at + 1024 * n) = give[n];
+      lds_fence_barrier();
+#pragma unroll
+      for (int n = 0; n < 8; ++n) keep[n] += *reinterpret_cast<const f32x4*>(theirs + at + 1024 * n);
+    };
+    if (g == 0) meet(dv, dk, allA[0], allA[NG - 1]);
+    else meet(dk, dv, allA[NG - 1], allA[0]);
+    lds_fence_barrier();  // (the next item's first stage lands there)
+  }
   // write dK (x softmax scale), dV : rows wk0 + 4lg + r, cols 16n + lr.  (Staging these tiles
   // through LDS for whole-row stores, as the forward's O, measured slower here and in the dQ
   // kernel: 88.9 -> 92.8 us and 32.6 -> 33.7 us, profiles/r3d/fa)
@@ -582,6 +591,11 @@ __global__ void __launch_bounds__(256, 2) bwd_dkdv_kernel(Args a) {
   for (int r = 0; r < 4; ++r) {
     const int kr = wk0 + 4 * lg + r;
     if (kr >= L) continue;
+    if (NG > 1 && g) {
+#pragma unroll
+      for (int n = 0; n < 8; ++n) dV[(long long)kr * a.lddv + n * 16 + lr] = from_f32<T>(dv[n][r]);
+      continue;
+    }
     float kv[8];
 #pragma unroll
     for (int n = 0; n < 8; ++n) kv[n] = dk[n][r] * a.scale;
@@ -594,7 +608,7 @@ __global__ void __launch_bounds__(256, 2) bwd_dkdv_kernel(Args a) {
 #pragma unroll
     for (int n = 0; n < 8; ++n) {
       dK[(long long)kr * a.lddk + n * 16 + lr] = from_f32<T>(kv[n]);
-      dV[(long long)kr * a.lddv + n * 16 + lr] = from_f32<T>(dv[n][r]);
+      if (NG == 1) dV[(long long)kr * a.lddv + n * 16 + lr] = from_f32<T>(dv[n][r]);
     }
   }
   };
@@ -1239,10 +1253,28 @@ static int cu_count() {
   return n;
 }
 
+// dK / dV of so few (key tile, kv head) items that two groups of waves an item pay: one a CU, or two where query heads share a kv
+// head and the chains are long.  Whole backward, us, one group -> two: 14 sequences of 63 - 509 tokens, 16 heads over 4 (276 items) 85
+// -> 75; 8 x 512 of them (256) 84 -> 75; 1 x 2048 (128) 244 -> 201; 1 x 4096 (256) 507 -> 431, 32 heads over 8 (512) 641 -> 594; 8 x
+// 512 of those (512) 115 -> 113; 1 x 512, 32 heads (256) 38.1 -> 37.4.  More: 2 x 512, 32 heads (512) 44 -> 47, 4 x 512 66 -> 82 (one
+// group's reads of Q and dO already keep LDS busy for a third of a step).
+static bool few_items(int items, int nh, int nkv) { return items <= (nh > nkv ? 2 : 1) * cu_count(); }
+
 template <typename T>
 static hipError_t launch(int which, int causal, int mt, int ntiles, const Args& a, hipStream_t st) {
   dim3 block(256);
-  if (which == 0) {  // forward: 32x32x16 kernel, 128-row tiles
+  if ((which == 2 || which == 7) && !a.tiles3 && few_items(ntiles * a.nkv, a.nh, a.nkv)) {
+    Args b = a;
+    b.nitems = ntiles * a.nkv;
+    const dim3 grid(std::min(b.nitems, cu_count())), both(512);
+    if (which == 7) {
+      if (causal) hipLaunchKernelGGL((bwd_dkdv_kernel<T, true, true, 2>), grid, both, 0, st, b);
+      else hipLaunchKernelGGL((bwd_dkdv_kernel<T, false, true, 2>), grid, both, 0, st, b);
+    } else {
+      if (causal) hipLaunchKernelGGL((bwd_dkdv_kernel<T, true, false, 2>), grid, both, 0, st, b);
+      else hipLaunchKernelGGL((bwd_dkdv_kernel<T, false, false, 2>), grid, both, 0, st, b);
+    }
+  } else if (which == 0) {  // forward: 32x32x16 kernel, 128-row tiles
     if (mt != 20) return hipErrorInvalidValue;
     dim3 grid(ntiles, a.tiles3 ? 1 : a.nh);
     if (a.nitems > 0) grid = dim3(std::min(a.nitems, (causal ? 2 : 1) * cu_count()), 1);

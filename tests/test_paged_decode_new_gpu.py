@@ -112,3 +112,20 @@ def test_refused():
     with pytest.raises(ValueError):
         native().paged_attention_decode(torch.empty_like(q), q, kc, vc, bt, cl, 4, 16, bt.shape[1], 0.1, one, one,
                                         one, 64, None, 3, pos, cos, sin, slots)
+
+
+@pytest.mark.parametrize("D,nh,nkv,dt", [(128, 5, 5, torch.bfloat16), (64, 6, 3, torch.float16), (32, 4, 1, torch.bfloat16), (256, 2, 2, torch.float16)])
+def test_merge_of_partitions(D, nh, nkv, dt):
+    """Up to 130 partitions, at the edges of the merge's 16 rows and 64 lanes, over scratch memory that holds NaN; against
+    the context in one partition, whose fp32 sums have another order, so a result may round the other way."""
+    from lumen.ops.attention import paged_decode
+
+    lens = [64, 65, 128, 129, 16 * 64, 16 * 64 + 1, 32 * 64 + 7, 64 * 64 - 1, 64 * 64 + 1, 80 * 64 + 1, 130 * 64 - 5]
+    qkv, kc, vc, bt, cl, *_ = _case(D, nh, nkv, lens, dt, False)
+    q = qkv[:, :nh * D].view(len(lens), nh, D)
+    scratch = torch.full((len(lens) * nh * 140 * (D + 2) + (1 << 20),), math.nan, device="cuda")
+    del scratch
+    got = paged_decode(q, kc, vc, bt, cl, 140 * 64, 1 / math.sqrt(D), 64).float()
+    one = paged_decode(q, kc, vc, bt, cl, 140 * 64, 1 / math.sqrt(D), 140 * 64).float()
+    ulp = 2.0 ** (-7 if dt == torch.bfloat16 else -10)
+    assert ((got - one).abs() <= ulp * one.abs() + 2.0 ** -16 * one.abs().max()).all()

@@ -12,7 +12,7 @@
 //  * talk_attn_kernel (mixed heads): a wave per key head, all of a tile's 64 keys; the shaped scores of all heads meet in
 //    LDS (a barrier a tile, two buffers), lane = key there, the mixing matrix is read from LDS.
 // The accumulators of the 16-lane rows are added by v_permlane32_swap / 16_swap, which halve the registers as they go.
-// Values of keys that a row does not see are not read: the row's own stand in, with weight 0.
+// Keys that a row does not see are not read: the row's own stands in.  Their values are zeros, as 0 times an infinity is NaN.
 // Measured in a graph, caches rotated through 700 MB, merge of the splits included, us, the general row kernel -> here (16 heads
 // over 4 key heads, bf16): 1 row of 331 tokens 12.0 -> 7.7, of 4000 22.1 -> 13.2; 16 rows of 62 - 500 19.3 -> 10.6; 64 rows of 125 -
 // 1000 56 -> 31.5 (its caches at 7 TB/s: 10.7), 200 of 62 - 500 94 -> 44; mixed heads with cap, distance bias and sink: 1 row of
@@ -103,6 +103,22 @@ template <typename T> __device__ __forceinline__ float query_scale(const RowAttn
   return a.tevery > 0 && a.tcoef != 0.f ? a.scale * (1.f + a.tcoef * logf((float)((pos + 1) / a.tevery) + 1.f)) : a.scale;
 }
 
+// does a row see all of the n keys from j0 on (one answer for the wave)
+template <typename T> __device__ __forceinline__ bool all_seen(const RowAttnArgs<T>& a, int j0, int n, int pos) {
+  return j0 + n - 1 <= pos && (a.window <= 0 || pos - j0 < a.window || j0 + n <= a.keep);
+}
+
+// the values of a cache row, or (row < 0) zeros for a key that is not seen.  Mixed heads choose the address: to blank 16 values
+// behind their loads is a longer program, and a step of one tile waits for its instructions too (30 rows 8.0 us, blanked 8.7,
+// here 8.2; of the four values of a wave of the other kernel, where a branch passes over whole tiles, 4.4 us, blanked 4.45, chosen
+// 4.5).  As a number, for the compiler took the choice of two pointers for a flat one, whose loads count as LDS reads too (8.6).
+__device__ const uint4 kNoValue = {0u, 0u, 0u, 0u};
+template <typename T> __device__ __forceinline__ uint4 values_of(const T* vb, int row, long long ld) {
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  const uintptr_t at = row < 0 ? reinterpret_cast<uintptr_t>(&kNoValue) : reinterpret_cast<uintptr_t>(vb + (long long)row * ld);
+  return __builtin_bit_cast(uint4, *reinterpret_cast<const __attribute__((address_space(1))) u32x4*>(at));
+}
+
 // acc += p v of one value chunk of 8 channels
 template <typename T, int HP>
 __device__ __forceinline__ void add_value(float (&acc)[HP][8], const uint4& v, const float (&p)[HP]) {
@@ -170,7 +186,7 @@ step_attn_kernel(const RowAttnArgs<T> a) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const uint4*>(vb + (long long)__shfl(rb, 4 * kg + i, 64) * a.vrow);
   };
-  const auto use = [&](int tv, const uint4 (&k)[4], const uint4 (&v)[4]) {
+  const auto use = [&](int tv, const uint4 (&k)[4], uint4 (&v)[4]) {
     const int j0 = first(tv);
     if (j0 > pos) return;
     f32x4 c = {0.f, 0.f, 0.f, 0.f};
@@ -208,6 +224,11 @@ step_attn_kernel(const RowAttnArgs<T> a) {
       const float ci = s_c[w][i];
 #pragma unroll
       for (int e = 0; e < 8; ++e) acc[i][e] *= ci;
+    }
+    if (!all_seen(a, j0, 16, pos)) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (!key_seen(j0 + 4 * kg + i, pos, a.window, a.keep)) v[i] = make_uint4(0u, 0u, 0u, 0u);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -330,16 +351,17 @@ talk_attn_kernel(const RowAttnArgs<T> a) {
     float* sc = s_sc + buf * TILE * ld;
     // the tile's keys and half of its values are asked for at once, the other half when the keys have been multiplied
     uint4 k[4][4], v[4][4];
-    int rb[4];
+    int rb[4], rv[4];
     const auto load_values = [&](int u) __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        v[u][i] = *reinterpret_cast<const uint4*>(vb + (long long)__shfl(rb[u], 4 * kg + i, 64) * a.vrow);
+      for (int i = 0; i < 4; ++i) v[u][i] = values_of(vb, __shfl(rv[u], 4 * kg + i, 64), a.vrow);
     };
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int j = j0 + 16 * u + lr;
-      rb[u] = cache_row(tbl, sh, key_seen(j, pos, a.window, a.keep) ? j : pos);
+      const bool seen = key_seen(j, pos, a.window, a.keep);
+      rb[u] = cache_row(tbl, sh, seen ? j : pos);
+      rv[u] = seen ? rb[u] : -1;
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {

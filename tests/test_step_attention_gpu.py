@@ -57,6 +57,33 @@ def test_shapings(T, H, G, bs, kind, dt):
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kind", ["plain", "window", "talk", "talk_window"])
+@pytest.mark.parametrize("H,G", [(4, 2), (16, 4), (8, 1)])
+def test_an_infinity_of_the_rows_own_value(H, G, kind, dt):
+    """It is the row's result in that channel, as the keys that the row does not see add nothing."""
+    if "talk" in kind and H // G > 4:
+        pytest.skip("mixed heads: up to four a key head")
+    g = torch.Generator().manual_seed(H)
+    seg, nb = step(CTX, 16, g)
+    k, v = (torch.randn(nb * 16, G, 128, generator=g).to(dt) for _ in range(2))
+    at = torch.tensor([c - 1 for c in CTX])
+    own = seg.tables[torch.arange(len(CTX)), at // 16].long() * 16 + at % 16
+    v[own, :, 5], v[own, :, 77] = float("inf"), -float("inf")
+    k, v = k.view(nb, 16, G, 128), v.view(nb, 16, G, 128)
+    q = torch.randn(len(CTX), H, 128, generator=g).to(dt)
+    kw = dict(window=21, keep_first=3) if "window" in kind else {}
+    if "talk" in kind:
+        kw["talk"] = torch.eye(H)
+    want = row_attention_ref(q, None, k, v, 128, torch.empty(len(CTX), H, 128), seg, H, G, 0.05, **kw)
+    assert (want[:, :, 5] == float("inf")).all() and (want[:, :, 77] == -float("inf")).all()
+    out = torch.empty(len(CTX), H, 128, dtype=dt, device="cuda")
+    kw = {n: x.cuda() if torch.is_tensor(x) else x for n, x in kw.items()}
+    row_attention(q.cuda(), None, k.cuda(), v.cuda(), 128, out, on_gpu(seg), H, G, 0.05, **kw)
+    assert torch.equal(out.cpu().isinf(), want.isinf()) and torch.equal(out.cpu().sign()[want.isinf()], want.sign()[want.isinf()])
+    assert out.cpu().nan_to_num(0, 0, 0).allclose(want.nan_to_num(0, 0, 0).to(dt), rtol=2 * torch.finfo(dt).eps, atol=1e-3)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("shaped,gated", [(False, False), (True, False), (True, True)])
 @pytest.mark.parametrize("T,H,R,D2,bs", [(3, 16, 512, 64, 16), (33, 16, 512, 64, 16), (17, 20, 512, 0, 8), (11, 5, 256, 32, 32),
                                          (40, 16, 256, 64, 16), (11, 16, 384, 32, 16), (40, 3, 384, 0, 16), (40, 16, 512, 40, 16)])

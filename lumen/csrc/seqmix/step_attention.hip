@@ -523,3 +523,21 @@ template hipError_t launch_step_attn<bf16>(const RowAttnArgs<bf16>&, int, hipStr
 template hipError_t launch_step_attn<fp16>(const RowAttnArgs<fp16>&, int, hipStream_t);
 
 }  // namespace lumen
+
+// 1 when sm_row_attn takes these kernels for the operands (arguments as there; mixed, sigmoid: are `talk`, `sigb` given), which
+// want other splits of the keys than the general one
+extern "C" int sm_step_attn_ok(int dt, const void* q1, long long q1r, long long q1h, int D1, int D2, const void* kc, long long krow,
+                               const void* vc, long long vrow, int Dv, const void* out, long long our, long long ouh, int H,
+                               int G, int bs, int mixed, int sigmoid, int vdiv) {
+  using namespace lumen;
+  if ((dt != kBF16 && dt != kF16) || G < 1 || H % G) return 0;
+  static const float given = 0.f;
+  RowAttnArgs<bf16> a{};
+  a.q1 = (const bf16*)q1; a.q1r = q1r; a.q1h = q1h; a.D1 = D1; a.D2 = D2;
+  a.kc = (const bf16*)kc; a.krow = krow; a.vc = (const bf16*)vc; a.vrow = vrow; a.Dv = Dv;
+  a.out = (bf16*)out; a.our = our; a.ouh = ouh;
+  a.H = H; a.G = G; a.bs = bs; a.vdiv = vdiv;
+  a.talk = mixed ? &given : nullptr;
+  a.sigb = sigmoid ? &given : nullptr;
+  return step_attn_ok(a);
+}

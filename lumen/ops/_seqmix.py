@@ -120,6 +120,8 @@ def _load():
         lib.sm_latent_attn_ok.restype = ctypes.c_int
         lib.sm_latent_tiles_ok.argtypes = [ctypes.c_int] * 6
         lib.sm_latent_tiles_ok.restype = ctypes.c_int
+        lib.sm_step_attn_ok.argtypes = [_T[k] for k in "ipllii" "plpli" "pll" "iiiiii"]
+        lib.sm_step_attn_ok.restype = ctypes.c_int
         lib.sm_head_scan_ahead_bytes.argtypes = [ctypes.c_int] * 5
         lib.sm_head_scan_ahead_bytes.restype = ctypes.c_longlong
         lib.sm_min_gru_sub.argtypes = []
@@ -188,6 +190,13 @@ def latent_attn_ok(dt: int, Dv: int, Dk: int, D1: int, bs: int) -> bool:
 def latent_tiles_ok(dt: int, Dv: int, Dk: int, D1: int, bs: int, max_blocks: int) -> bool:
     """Does the latent attention have a kernel that shares key tiles among rows for these sizes?"""
     return bool(_load().sm_latent_tiles_ok(dt, Dv, Dk, D1, bs, max_blocks))
+
+
+def step_attn_ok(dt: int, q1, D1: int, D2: int, kc, krow: int, vc, vrow: int, Dv: int, out, H: int, G: int, bs: int, mixed: bool,
+                 sigmoid: bool, vdiv: int) -> bool:
+    """Does the row attention take the kernels of decode steps (csrc/seqmix/step_attention.hip) for these operands?"""
+    return bool(_load().sm_step_attn_ok(dt, q1.data_ptr(), q1.stride(0), q1.stride(1), D1, D2, kc.data_ptr(), krow, vc.data_ptr(), vrow,
+                                        Dv, out.data_ptr(), out.stride(0), out.stride(1), H, G, bs, int(mixed), int(sigmoid), vdiv))
 
 
 def head_scan_ahead_bytes(delta: bool, Dk: int, H: int, rep: int, chunks: int) -> int:

@@ -1106,7 +1106,7 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
     of 128, no window, linear bias, gate or sigmoid weights) to ``talk_attention.hip``; the latent layout with ``vt`` goes to the
     latent kernels (``latent_tile.hip`` for large prompt portions); every other row (decoded rows, fp32, other shapes) to the row kernel.  A row's
     result does not depend on which of them computed it beyond rounding."""
-    from ._seqmix import (DT, call, latent_attn_ok, latent_tiles_ok, talk_tiles_ok, use_seqmix,
+    from ._seqmix import (DT, call, latent_attn_ok, latent_tiles_ok, step_attn_ok, talk_tiles_ok, use_seqmix,
                           win_tiles_ok)
 
     T, _, D1 = q1.shape
@@ -1241,10 +1241,12 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
     # 16 / 32 splits: 62 / 46; 8 heads over 2 46 / 34, where one block a row took 38; splits past a row's last tile cost 0 - 0.2).
     # Of 16 heads fewer workgroups fit a CU: 32 rows of 4000 77 / 81.
     nsplit = max(1, min(tiles, 32, (1024 if talk is None and HB <= 8 and blocks <= 32 else 512) // max(blocks, 1)))
-    # step_attention.hip (its conditions are the launcher's): a workgroup serves a row and key head, or all heads of a row when
+    # step_attention.hip, where the launcher takes it: a workgroup serves a row and key head, or all heads of a row when
     # they are mixed.  Workgroups of 3 and 2 a CU: half or twice as many splits are 2 - 20 % slower at 16 - 64 rows, and even below.
-    if (D1 == Dv == 128 and q2 is None and H // G in (2, 4, 8) and v_div == 1 and sigmoid_bias is None
-            and krow == vrow == G * 128 and q1.dtype != torch.float32):
+    # (The general kernel with these splits: 16 heads over 8, blocks of 12, 64 rows of 64 - 505 45 -> 112 us.)
+    if (D1 == Dv == 128 and q2 is None and q1.dtype != torch.float32
+            and step_attn_ok(DT[q1.dtype], q1, D1, D2, kcache, krow, vcache, vrow, Dv, out, H, G, bs, talk is not None,
+                             sigmoid_bias is not None, v_div)):
         nsplit = max(1, min(tiles, 64, 1024 // (T * G) if talk is None else 512 // T))
     ws_ml = ws_o = None
     if nsplit > 1:

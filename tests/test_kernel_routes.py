@@ -456,3 +456,28 @@ def test_halved_heads_of_few_rows_keep_as_many_splits(launched, T, H, heads, spl
     row_attention(q, None, kv, kv.clone(), 128, torch.zeros(T, H, 128, **BF), seg, H, H, 0.1)
     (name, a), = launched
     assert name == "sm_row_attn" and a[-3] == splits and a[24] == heads
+
+
+@pytest.mark.parametrize("T,H,G,bs,talk,offset,step", [
+    (64, 16, 4, 16, False, 0, True), (64, 16, 8, 16, False, 0, True), (64, 32, 8, 64, False, 0, True), (8, 16, 4, 16, True, 0, True),
+    (8, 32, 8, 8, True, 0, True), (64, 16, 4, 12, False, 0, False), (64, 16, 8, 24, False, 0, False), (8, 16, 4, 20, True, 0, False),
+    (64, 16, 8, 16, False, 4, False), (8, 16, 4, 16, True, 4, False), (64, 16, 16, 16, False, 0, False), (64, 32, 2, 16, False, 0, False),
+    (8, 32, 4, 16, True, 0, False), (8, 18, 9, 16, True, 0, False)])
+def test_splits_of_the_keys_are_those_of_the_kernel_that_runs(launched, T, H, G, bs, talk, offset, step):
+    """Behind tables of 4096 keys.  The kernels of decode steps deal keys out otherwise than the general one, which takes
+    blocks of no power of two, heads one or 16 a key head, mixed heads eight a key head, and rows off 16 bytes."""
+    from lumen.ops.attention import row_attention
+    from lumen.ops.segments import SegBatch
+
+    i32 = dict(dtype=torch.int32)
+    at = torch.arange(T, **i32)
+    seg = SegBatch(torch.arange(T + 1, **i32), at, at, at, at, torch.zeros(T, -(-4096 // bs), **i32), None)
+    q, kv = torch.zeros(T, H * 128 + 8, **BF)[:, offset:offset + H * 128], torch.zeros(1, bs, G, 128, **BF)
+    row_attention(q.view(T, H, 128), None, kv, kv.clone(), 128, torch.zeros(T, H, 128, **BF), seg, H, G, 0.1,
+                  talk=torch.eye(H) if talk else None)
+    (name, a), = launched
+    blocks = T * -(-H // a[24])
+    general = min(32, (1024 if not talk and a[24] <= 8 and blocks <= 32 else 512) // blocks)
+    deep = min(64, 512 // T if talk else 1024 // (T * G))
+    assert general != deep
+    assert name == "sm_row_attn" and a[-3] == (deep if step else general)

@@ -1138,7 +1138,7 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
     coef, every = (float(q_temp[0]), int(q_temp[1])) if q_temp is not None else (0.0, 0)
     bs = kcache.shape[1]
     al8 = lambda x: x.data_ptr() % 16 == 0 and x.stride(0) % 8 == 0 and x.stride(1) % 8 == 0  # noqa: E731
-    own = int(seg.cu.shape[0] - 1 == T)                  # decoded rows: every one a sequence of its own
+    own = int(seg.singles or seg.S == T)                 # decoded rows: every one a sequence of its own
     if (vt is not None and G == 1 and talk is None and vcache is kcache and D1 >= Dv
             and slopes is None and window == 0 and sigmoid_bias is None
             and (gate is None or gate.stride(1) == 1)
@@ -1162,7 +1162,7 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
                  gate.stride(0) if gate is not None else 0)
             if Tp >= T:
                 return out
-            full, T = out, T - Tp
+            full, T, own = out, T - Tp, 1                # (behind the portions: decoded rows)
             q1, out = q1[Tp:], out[Tp:]
             q2 = q2[Tp:] if q2 is not None else None
             gate = gate[Tp:] if gate is not None else None
@@ -1207,7 +1207,7 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
              v_div)
         if Tp >= T:
             return out
-        q1, out, T = q1[Tp:], out[Tp:], T - Tp
+        q1, out, T, own = q1[Tp:], out[Tp:], T - Tp, 1
         gate = gate[Tp:] if gate is not None else None
     # mixed heads: 16 rows and all heads of a tile on the matrix cores
     elif (talk is not None and seg.q_tiles is not None and seg.tile_rows > 0 and q2 is None and slopes is None
@@ -1222,7 +1222,7 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
              seg.cu, seg.start, H, G, D1, Dv, bs, scale, float(softcap or 0.0), coef, every, r1, r2, talk, sink)
         if Tp >= T:
             return out
-        q1, out, T = q1[Tp:], out[Tp:], T - Tp
+        q1, out, T, own = q1[Tp:], out[Tp:], T - Tp, 1
     row_seg, positions = seg.row_seg[Tp:], seg.positions[Tp:]
     HB = _heads_per_block(H, Dk, talk is not None)
     # few rows (decoding): deal a row's 64-key tiles out to several workgroups so that ~2 per CU

@@ -30,6 +30,7 @@ class SegBatch:
     fresh: bool = False       # every portion starts at position 0: its keys are rows of this step
     # the portions' (pairs of rows and keys, keys of the longest), where the host has counted them
     keys: Optional[tuple] = None
+    singles: bool = False     # the rows are decoded ones whatever the segments' count says (``decoded``)
 
     @property
     def S(self) -> int:
@@ -60,7 +61,7 @@ class SegBatch:
         attention reads (``row_seg``, ``positions``, ``tables``, ``cache_slots``)."""
         n = self.tile_rows
         return replace(self, row_seg=self.row_seg[n:], positions=self.positions[n:], q_tiles=None, tile_rows=0,
-                       fresh=False, keys=None, cache_slots=None if self.cache_slots is None else self.cache_slots[n:])
+                       fresh=False, keys=None, singles=True, cache_slots=None if self.cache_slots is None else self.cache_slots[n:])
 
 
 import os

@@ -481,3 +481,44 @@ def test_splits_of_the_keys_are_those_of_the_kernel_that_runs(launched, T, H, G,
     deep = min(64, 512 // T if talk else 1024 // (T * G))
     assert general != deep
     assert name == "sm_row_attn" and a[-3] == (deep if step else general)
+
+
+@pytest.mark.parametrize("form", ["window", "talk", "latent", "decoded"])
+@pytest.mark.parametrize("rows", [[1] * 5, [2100, 1, 1, 1], [2100, 1]])
+def test_decoded_rows_behind_portions_are_dealt_out_as_decoded_rows(launched, monkeypatch, form, rows):
+    """The portions' rows are another kernel's, so every row that is left is a sequence of its own."""
+    from lumen.ops.attention import row_attention
+    from lumen.ops.segments import SegBatch, tile_list
+
+    monkeypatch.setattr(_seqmix, "talk_tiles_ok", lambda *a: True)
+    i32, S, T = dict(dtype=torch.int32), len(rows), sum(rows)
+    cu = [sum(rows[:i]) for i in range(S + 1)]
+    P = rows.count(2100)
+    seg = SegBatch(torch.tensor(cu, **i32), torch.arange(S, **i32), torch.zeros(S, **i32),
+                   torch.repeat_interleave(torch.arange(S), torch.tensor(rows)).int(), torch.zeros(T, **i32), torch.zeros(S, 160, **i32),
+                   None, torch.tensor(tile_list(cu, P), **i32).view(-1, 2) if P else None, cu[P], 128)
+    H, n = 16, T
+    if form == "decoded":
+        seg, n = seg.decoded(), T - cu[P]
+    if form in ("latent", "decoded"):
+        q, c = torch.zeros(n, H, 576, **BF), torch.zeros(1, 16, 576, **BF)
+        row_attention(q[:, :, :512], q[:, :, 512:], c, c, 512, torch.zeros(n, H, 512, **BF), seg, H, 1, 0.1, vt=torch.zeros(1, 512, 16, **BF))
+        want = ["sm_latent_tiles"] * (P > 0 and form == "latent") + ["sm_latent_attn"]
+    else:
+        q, k = torch.zeros(n, H, 128, **BF), torch.zeros(1, 16, 4, 128, **BF)
+        row_attention(q, None, k, k.clone(), 128, torch.zeros(n, H, 128, **BF), seg, H, 4, 0.1, talk=torch.eye(H) if form == "talk" else None)
+        want = [{"window": "sm_win_attn_tiles", "talk": "sm_talk_tiles"}[form]] * (P > 0) + ["sm_row_attn"]
+    assert [n for n, _ in launched] == want
+    assert launched[-1][1][-4] == 1
+
+
+def test_rows_of_one_portion_are_not_dealt_out_as_decoded_rows(launched):
+    from lumen.ops.attention import row_attention
+    from lumen.ops.segments import SegBatch
+
+    i32 = dict(dtype=torch.int32)
+    seg = SegBatch(torch.tensor([0, 40], **i32), torch.zeros(1, **i32), torch.zeros(1, **i32), torch.zeros(40, **i32), torch.arange(40, **i32),
+                   torch.zeros(1, 160, **i32))
+    q, k = torch.zeros(40, 16, 128, **BF), torch.zeros(1, 16, 4, 128, **BF)
+    row_attention(q, None, k, k.clone(), 128, torch.zeros(40, 16, 128, **BF), seg, 16, 4, 0.1)
+    assert launched[0][0] == "sm_row_attn" and launched[0][1][-4] == 0

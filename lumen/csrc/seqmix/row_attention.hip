@@ -634,7 +634,7 @@ row_attn_kernel(const RowAttnArgs<T> a) {
 //      the weights of one head; the accumulator's column is the head, so the running correction is
 //      lane-local and nothing is merged across waves at the end.
 // Scores, maxima, sums and the accumulator are fp32.
-//
+
 // A workgroup whose split holds no key of its row: (max, sum) = (-inf, -1), and no values
 template <typename T>
 __device__ __forceinline__ bool latent_no_tile(const RowAttnArgs<T>& a, int t, int pos, int h0, int nh, int tile) {
@@ -655,8 +655,11 @@ __device__ __forceinline__ uint4 seen_mask(int n) {
   return make_uint4((unsigned)lo, (unsigned)(lo >> 32), (unsigned)hi, (unsigned)(hi >> 32));
 }
 
-template <typename T, int NT>   // NT: 16-channel tiles per wave, Dv = 64 NT
-__global__ void __launch_bounds__(64 * kWaves)
+// DEEP sends for four steps of keys while four are multiplied, and for the first values with the first keys: for key sizes that
+// latent_row_kernel is not built for.  It takes registers: many rows of small ranks, whose workgroups hide each other's loads, keep the
+// form without (1024 rows of 250 tokens over 256 + 32: 34 us, DEEP 50).
+template <typename T, int NT, bool DEEP>   // NT: 16-channel tiles per wave, Dv = 64 NT
+__global__ void __launch_bounds__(64 * kWaves, DEEP ? 2 : 1)
 latent_attn_kernel(const RowAttnArgs<T> a, const T* __restrict__ vt) {
   extern __shared__ float smem[];
   constexpr int kPRow = 128 + 8;                 // weights per head in LDS: 128 keys + padding
@@ -699,6 +702,40 @@ latent_attn_kernel(const RowAttnArgs<T> a, const T* __restrict__ vt) {
 #pragma unroll
   for (int n = 0; n < NT; ++n) O[n] = f32x4v{0.f, 0.f, 0.f, 0.f};
   const T* qp = s_qb + hd * (Dkp + kQPad);
+  // key fragments of kCh steps of 32 channels: one chunk is loaded while the one before it is multiplied
+  constexpr int kCh = DEEP ? 4 : 1;
+  uint4 ka[kCh], kb[kCh], kc[kCh], kd[kCh], vv[DEEP ? 2 : 1][NT];
+  const T *kp0 = a.kc, *kp1 = a.kc;
+  const auto keys = [&](int jw) {                          // the rows of the lane's keys (addressable ones)
+    const int k0 = min(jw + hd, pos), k1 = min(jw + 16 + hd, pos);
+    kp0 = a.kc + ((long long)tbl[k0 / a.bs] * a.bs + k0 % a.bs) * a.krow + 8 * kg;
+    kp1 = a.kc + ((long long)tbl[k1 / a.bs] * a.bs + k1 % a.bs) * a.krow + 8 * kg;
+  };
+  const auto load = [&](uint4 (&x)[kCh], uint4 (&y)[kCh], int d0) {
+#pragma unroll
+    for (int c = 0; c < kCh; ++c)
+      if (d0 + 32 * c < Dkp) {
+        const bool in = d0 + 32 * c + 8 * kg < Dk;         // (past the key: zeros)
+        x[c] = in ? *reinterpret_cast<const uint4*>(kp0 + d0 + 32 * c) : make_uint4(0u, 0u, 0u, 0u);
+        y[c] = in ? *reinterpret_cast<const uint4*>(kp1 + d0 + 32 * c) : make_uint4(0u, 0u, 0u, 0u);
+      }
+  };
+  const auto values = [&](uint4 (&v)[NT], int jb) {        // the lane's 8 keys from jb on, its channels
+    const int k = min(jb, pos);
+    const T* vp = vt + ((long long)tbl[k / a.bs] * a.Dv) * a.bs + jb % a.bs;
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+      v[n] = *reinterpret_cast<const uint4*>(vp + (long long)((w * NT + n) * 16 + hd) * a.bs);
+  };
+  if (128 * (int)blockIdx.z + 32 * w <= pos) {
+    keys(128 * blockIdx.z + 32 * w);
+    if (DEEP) load(ka, kb, 0);
+  }
+  const auto ahead = [&](int j0) {                         // the first two steps' values of a tile
+    if (DEEP && j0 <= pos) values(vv[0], j0 + 8 * kg);
+    if (DEEP && j0 + 32 <= pos) values(vv[DEEP], j0 + 32 + 8 * kg);
+  };
+  ahead(128 * blockIdx.z);
   __syncthreads();
 
   for (int j0 = 128 * blockIdx.z; j0 <= pos; j0 += 128 * a.nsplit) {
@@ -708,16 +745,25 @@ latent_attn_kernel(const RowAttnArgs<T> a, const T* __restrict__ vt) {
     float mx = -INFINITY;
     f32x4v c0 = {0.f, 0.f, 0.f, 0.f}, c1 = {0.f, 0.f, 0.f, 0.f};
     if (jw <= pos) {
-      const int k0 = min(jw + hd, pos), k1 = min(jw + 16 + hd, pos);       // the rows of the lane's keys (addressable ones)
-      const T* kp0 = a.kc + ((long long)tbl[k0 / a.bs] * a.bs + k0 % a.bs) * a.krow + 8 * kg;
-      const T* kp1 = a.kc + ((long long)tbl[k1 / a.bs] * a.bs + k1 % a.bs) * a.krow + 8 * kg;
-      for (int d0 = 0; d0 < Dkp; d0 += 32) {
-        const bool in = d0 + 8 * kg < Dk;                  // (past the key: zeros)
-        const uint4 x = in ? *reinterpret_cast<const uint4*>(kp0 + d0) : make_uint4(0u, 0u, 0u, 0u);
-        const uint4 y = in ? *reinterpret_cast<const uint4*>(kp1 + d0) : make_uint4(0u, 0u, 0u, 0u);
-        const uint4 bv = *reinterpret_cast<const uint4*>(qp + d0 + 8 * kg);
-        c0 = Mma16<T>::run(x, bv, c0);
-        c1 = Mma16<T>::run(y, bv, c1);
+      const auto mul = [&](const uint4 (&x)[kCh], const uint4 (&y)[kCh], int d0) {
+#pragma unroll
+        for (int c = 0; c < kCh; ++c)
+          if (d0 + 32 * c < Dkp) {
+            const uint4 bv = *reinterpret_cast<const uint4*>(qp + d0 + 32 * c + 8 * kg);
+            c0 = Mma16<T>::run(x[c], bv, c0);
+            c1 = Mma16<T>::run(y[c], bv, c1);
+          }
+      };
+      if (!DEEP)
+        for (int d0 = 0; d0 < Dkp; d0 += 32) {
+          load(ka, kb, d0);
+          mul(ka, kb, d0);
+        }
+      else for (int d0 = 0; d0 < Dkp; d0 += 64 * kCh) {
+        if (d0 + 32 * kCh < Dkp) load(kc, kd, d0 + 32 * kCh);
+        mul(ka, kb, d0);
+        if (d0 + 64 * kCh < Dkp) load(ka, kb, d0 + 64 * kCh);
+        if (d0 + 32 * kCh < Dkp) mul(kc, kd, d0 + 32 * kCh);
       }
     }
     if (jw <= pos) {
@@ -778,21 +824,23 @@ latent_attn_kernel(const RowAttnArgs<T> a, const T* __restrict__ vt) {
       if (j0 + 32 * ks > pos) continue;
       const uint4 bh = *reinterpret_cast<const uint4*>(s_ph + hd * kPRow + 32 * ks + 8 * kg);
       const uint4 bl = *reinterpret_cast<const uint4*>(s_pl + hd * kPRow + 32 * ks + 8 * kg);
-      const int k = min(jb, pos);
-      const T* vp = vt + ((long long)tbl[k / a.bs] * a.Dv) * a.bs + jb % a.bs;
-      uint4 vv[NT];
-#pragma unroll
-      for (int n = 0; n < NT; ++n)
-        vv[n] = *reinterpret_cast<const uint4*>(vp + (long long)((w * NT + n) * 16 + hd) * a.bs);
+      if (!DEEP) values(vv[0], jb);
       const uint4 mk = seen_mask(pos - jb + 1);
 #pragma unroll
       for (int n = 0; n < NT; ++n) {
-        uint4 av = vv[n];                                    // as A operand: the lane's channel
+        uint4 av = vv[DEEP ? ks & 1 : 0][n];                          // as A operand: the lane's channel
         av.x &= mk.x; av.y &= mk.y; av.z &= mk.z; av.w &= mk.w;
         O[n] = Mma16<T>::run(av, bh, O[n]);
         O[n] = Mma16<T>::run(av, bl, O[n]);
       }
+      if (DEEP && ks < 2 && j0 + 32 * (ks + 2) <= pos) values(vv[DEEP ? ks & 1 : 0], jb + 64);
     }
+    const int jn = j0 + 128 * a.nsplit + 32 * w;           // the next tile's first keys
+    if (jn <= pos) {
+      keys(jn);
+      if (DEEP) load(ka, kb, 0);
+    }
+    ahead(j0 + 128 * a.nsplit);
   }
   // O[n][i] = O^T[channel (w NT + n) 16 + 4 kg + i][head hd]
   if (head_on) {
@@ -989,29 +1037,38 @@ inline size_t latent_attn_lds(int Dk, int esz) {
 // few keys each, and many the fewer partial sums (64 / 128 keys, us: 1 row 14.0 / 17.1, 16 rows of 8 heads 18.8 / 21.4, 32 of 16
 // 18.3 / 20.3, 64 of 16 23.3 / 21.3, of 2000 keys 51 / 53)
 constexpr int kLatentNarrow = 32;
+// is latent_row_kernel built for the rank and the key size?  Others (512 + 96: 640 bytes a key and lane) keep latent_attn_kernel's DEEP
+// form.  Without load-ahead 64 rows of 64 - 505 tokens, 8 heads over 512 + 96, would take 26.5 us for 21.0, one row of 4000 23.6 for 19.6.
+inline bool latent_row_size(int Dv, int Dk) {
+  const int nt = Dv / 64, ks = (Dk + 31) / 32;
+  return (nt == 4 || nt == 6 || nt == 8) && ks >= 2 * nt && ks <= 2 * nt + 2;
+}
+inline bool latent_narrow(int Dv, int Dk, long long blocks) { return latent_row_size(Dv, Dk) && blocks <= kLatentNarrow; }
 
 template <typename T>
 hipError_t launch_latent_attn(const RowAttnArgs<T>& a, const T* vt, int Tn, hipStream_t st) {
   const size_t lds = latent_attn_lds(a.D1 + a.D2, sizeof(T));
   const dim3 grid(Tn, (a.H + 15) / 16, a.nsplit);
-  const int ks = (a.D1 + a.D2 + 31) / 32;
-  const bool few = (long long)grid.x * grid.y * grid.z <= 512, narrow = (long long)grid.x * grid.y <= kLatentNarrow;
-#define LATENT(N) latent_attn_kernel<T, N><<<grid, 64 * kWaves, lds, st>>>(a, vt)
+  const int nt = a.Dv / 64, ks = (a.D1 + a.D2 + 31) / 32;
+  // two workgroups of the deep form fit a CU, as of the other one at ranks of 384 and more
+  const bool few = nt > 4 || (long long)grid.x * grid.y * grid.z <= 512;
+  const bool narrow = latent_narrow(a.Dv, a.D1 + a.D2, (long long)grid.x * grid.y);
+#define LATENT(N, D) latent_attn_kernel<T, N, D><<<grid, 64 * kWaves, lds, st>>>(a, vt)
 #define ROW(N, KS)                                                                        \
   if (narrow) latent_row_kernel<T, N, KS, 4><<<grid, 256, 0, st>>>(a, vt);                \
   else latent_row_kernel<T, N, KS, 8><<<grid, 512, 0, st>>>(a, vt)
 #define ROWS(N)                                  \
-  if (ks == 2 * N) { ROW(N, 2 * N); }            \
+  if (!latent_row_size(a.Dv, a.D1 + a.D2)) LATENT(N, true); \
+  else if (ks == 2 * N) { ROW(N, 2 * N); }       \
   else if (ks == 2 * N + 1) { ROW(N, 2 * N + 1); } \
-  else if (ks == 2 * N + 2) { ROW(N, 2 * N + 2); } \
-  else LATENT(N)
-  switch (a.Dv / 64) {
-    case 1: LATENT(1); break;
-    case 2: LATENT(2); break;
-    case 3: LATENT(3); break;
-    case 4: if (few) { ROWS(4); } else { LATENT(4); } break;
-    case 6: ROWS(6); break;
-    case 8: ROWS(8); break;
+  else { ROW(N, 2 * N + 2); }
+  switch (nt) {
+    case 1: LATENT(1, false); break;
+    case 2: LATENT(2, false); break;
+    case 3: LATENT(3, false); break;
+    case 4: if (few || narrow) { ROWS(4) } else { LATENT(4, false); } break;
+    case 6: ROWS(6) break;
+    case 8: ROWS(8) break;
     default: return hipErrorInvalidValue;
   }
 #undef ROWS
@@ -1193,6 +1250,9 @@ int sm_latent_attn_ok(int dt, int Dv, int Dk, int D1, int bs) {
   return Dv % 64 == 0 && (nt == 1 || nt == 2 || nt == 3 || nt == 4 || nt == 6 || nt == 8) &&
          Dk % 8 == 0 && D1 % 8 == 0 && Dv <= Dk && bs % 8 == 0 && latent_attn_lds(Dk, 2) <= 65536;
 }
+
+// Keys that a workgroup of sm_latent_attn takes of T rows with H heads: what a split of the keys is a multiple of
+int sm_latent_tile(int Dv, int Dk, int T, int H) { return latent_narrow(Dv, Dk, (long long)T * ((H + 15) / 16)) ? 64 : 128; }
 
 // Latent attention (one key/value head, values = the first Dv columns of a key row) with the
 // value product on the matrix cores; `vt` is the per-block transposed copy of the values that

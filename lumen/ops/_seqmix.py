@@ -120,6 +120,8 @@ def _load():
         lib.sm_latent_attn_ok.restype = ctypes.c_int
         lib.sm_latent_tiles_ok.argtypes = [ctypes.c_int] * 6
         lib.sm_latent_tiles_ok.restype = ctypes.c_int
+        lib.sm_latent_tile.argtypes = [ctypes.c_int] * 4
+        lib.sm_latent_tile.restype = ctypes.c_int
         lib.sm_step_attn_ok.argtypes = [_T[k] for k in "ipllii" "plpli" "pll" "iiiiii"]
         lib.sm_step_attn_ok.restype = ctypes.c_int
         lib.sm_head_scan_ahead_bytes.argtypes = [ctypes.c_int] * 5
@@ -185,6 +187,11 @@ def row_attn_lds(HB: int, Dk: int) -> int:
 def latent_attn_ok(dt: int, Dv: int, Dk: int, D1: int, bs: int) -> bool:
     """Does the matrix-core latent attention have a kernel for these sizes?"""
     return bool(_load().sm_latent_attn_ok(dt, Dv, Dk, D1, bs))
+
+
+def latent_tile(Dv: int, Dk: int, T: int, H: int) -> int:
+    """Keys that a workgroup of the latent attention takes of T rows with H heads."""
+    return int(_load().sm_latent_tile(Dv, Dk, T, H))
 
 
 def latent_tiles_ok(dt: int, Dv: int, Dk: int, D1: int, bs: int, max_blocks: int) -> bool:

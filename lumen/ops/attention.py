@@ -1038,7 +1038,6 @@ def _heads_per_block(H: int, Dk: int, need_all: bool) -> int:
     return hb
 
 
-LATENT_NARROW = 32           # rows x 16-head blocks up to which row_attention.hip takes 64 keys a workgroup (kLatentNarrow there)
 LATENT_TILE_ROWS = 2048      # rows x 16-head blocks from which prompt portions take the tiled latent kernel
 
 
@@ -1106,7 +1105,7 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
     of 128, no window, linear bias, gate or sigmoid weights) to ``talk_attention.hip``; the latent layout with ``vt`` goes to the
     latent kernels (``latent_tile.hip`` for large prompt portions); every other row (decoded rows, fp32, other shapes) to the row kernel.  A row's
     result does not depend on which of them computed it beyond rounding."""
-    from ._seqmix import (DT, call, latent_attn_ok, latent_tiles_ok, step_attn_ok, talk_tiles_ok, use_seqmix,
+    from ._seqmix import (DT, call, latent_attn_ok, latent_tile, latent_tiles_ok, step_attn_ok, talk_tiles_ok, use_seqmix,
                           win_tiles_ok)
 
     T, _, D1 = q1.shape
@@ -1170,7 +1169,7 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
         else:
             full = out
         blocks = T * ((H + 15) // 16)
-        keys = 64 if blocks <= LATENT_NARROW else 128             # (a workgroup's tile: the launcher's rule)
+        keys = latent_tile(Dv, Dk, T, H)                          # (a workgroup's tile)
         tiles = (seg.tables.shape[1] * bs + keys - 1) // keys
         nsplit = max(1, min(tiles, 64 if keys == 64 else 32, 512 // max(blocks, 1)))
         ws_ml = ws_o = None

@@ -522,3 +522,20 @@ def test_rows_of_one_portion_are_not_dealt_out_as_decoded_rows(launched):
     q, k = torch.zeros(40, 16, 128, **BF), torch.zeros(1, 16, 4, 128, **BF)
     row_attention(q, None, k, k.clone(), 128, torch.zeros(40, 16, 128, **BF), seg, 16, 4, 0.1)
     assert launched[0][0] == "sm_row_attn" and launched[0][1][-4] == 0
+
+
+@pytest.mark.parametrize("T,R,D2,splits", [(1, 512, 64, 64), (32, 512, 64, 16), (33, 512, 64, 15), (1, 384, 0, 64), (1, 256, 64, 64), (1, 512, 96, 32),
+                                           (1, 384, 128, 32), (1, 256, 96, 32), (32, 512, 72, 16), (1, 192, 64, 32), (1, 64, 0, 32)])
+def test_splits_of_latent_keys_are_of_the_tile_that_the_kernel_takes(launched, T, R, D2, splits):
+    """Behind tables of 4096 keys: 64 splits of tiles of 128 keys would leave half of the workgroups without a key."""
+    from lumen.ops.attention import row_attention
+    from lumen.ops.segments import SegBatch
+
+    i32 = dict(dtype=torch.int32)
+    at = torch.arange(T, **i32)
+    seg = SegBatch(torch.arange(T + 1, **i32), at, at, at, at, torch.zeros(T, 256, **i32), None)
+    q, c = torch.zeros(T, 16, R + D2, **BF), torch.zeros(1, 16, R + D2, **BF)
+    row_attention(q[:, :, :R], q[:, :, R:] if D2 else None, c, c, R, torch.zeros(T, 16, R, **BF), seg, 16, 1, 0.1,
+                  vt=torch.zeros(1, R, 16, **BF))
+    (name, a), = launched
+    assert name == "sm_latent_attn" and a[-3] == splits

@@ -105,7 +105,7 @@ hipError_t lumen_flash_attn_ds(int, int, int, const void*, const void*, const vo
                                long long, long long, const float*, const int*, const int*, int, int,
                                int, int, float, const void*, long long, void*, void*, void*,
                                long long, long long, long long, const float*, const int*,
-                               const float*, const float*, void*, const int*, int, hipStream_t);
+                               const float*, const float*, void*, const int*, int, int, hipStream_t);
 long long lumen_car_signal_bytes();
 int lumen_car_max_blocks();
 int lumen_car_max_ranks();
@@ -916,7 +916,7 @@ void flash_attn_ds(int64_t which, bool causal, const at::Tensor& q, const at::Te
                    const at::Tensor& tiles, int64_t nh, int64_t nkv, double scale,
                    const at::Tensor& dout, const at::Tensor& dq, const at::Tensor& dk,
                    const at::Tensor& dv, const at::Tensor& delta, const at::Tensor& ds,
-                   const at::Tensor& ds_off, int64_t ds_total,
+                   const at::Tensor& ds_off, int64_t ds_total, int64_t longest,
                    const std::optional<at::Tensor>& rope_pos, const std::optional<at::Tensor>& rope_cos,
                    const std::optional<at::Tensor>& rope_sin) {
   if (!q.is_cuda() || !ds.is_cuda() || !ds_off.is_cuda())
@@ -940,7 +940,7 @@ void flash_attn_ds(int64_t which, bool causal, const at::Tensor& q, const at::Te
                             dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dq.stride(0), dk.stride(0),
                             dv.stride(0), delta.data_ptr<float>(), ptr<const int>(rope_pos),
                             ptr<const float>(rope_cos), ptr<const float>(rope_sin), ds.data_ptr(),
-                            ds_off.data_ptr<int>(), static_cast<int>(ds_total), cur_stream()),
+                            ds_off.data_ptr<int>(), static_cast<int>(ds_total), static_cast<int>(longest), cur_stream()),
         "flash_attn_ds");
 }
 

@@ -1253,17 +1253,21 @@ static int cu_count() {
   return n;
 }
 
-// dK / dV of so few (key tile, kv head) items that two groups of waves an item pay: one a CU, or two where query heads share a kv
-// head and the chains are long.  Whole backward, us, one group -> two: 14 sequences of 63 - 509 tokens, 16 heads over 4 (276 items) 85
-// -> 75; 8 x 512 of them (256) 84 -> 75; 1 x 2048 (128) 244 -> 201; 1 x 4096 (256) 507 -> 431, 32 heads over 8 (512) 641 -> 594; 8 x
-// 512 of those (512) 115 -> 113; 1 x 512, 32 heads (256) 38.1 -> 37.4.  More: 2 x 512, 32 heads (512) 44 -> 47, 4 x 512 66 -> 82 (one
-// group's reads of Q and dO already keep LDS busy for a third of a step).
-static bool few_items(int items, int nh, int nkv) { return items <= (nh > nkv ? 2 : 1) * cu_count(); }
+// Do two groups of waves an item pay for dK / dV?  `longest`: query tiles of the longest sequence, so its heaviest item is a chain of
+// nh / nkv as many steps.  Chains of eight and more where every item has a CU of its own, of 32 and more up to two items a CU: the sums
+// that meet cost 1 - 2 us and two items of a CU share it less well so.  Whole backward, us, one group -> two.  Up to an item a CU (256): chain 1
+// 13.9 -> 15.7 (4 sequences of 64 tokens, 16 heads), 2 18.3 -> 19.0, 4 25.8 -> 26.4 (4 x 256, 16) and 19.7 -> 18.8 (16 x 30, 16 heads over
+// 4), 8 30.1 -> 28.7 (2 x 512, 8) and 36.8 -> 35.4 (8 x 128, 32 over 8), 16 54.1 -> 49.9, 32 86 -> 77 (4 x 512, 32 over 8), 128 253 -> 208 (1 x
+// 2048 of those).  Up to two (512): 8 46.4 -> 51.1 (8 x 200, 32 over 16), 16 67.0 -> 68.8 (4 x 512), 32 95.8 -> 93.1 (2 x 1024), 64 158 -> 143;
+// 14 of 63 - 509, 16 over 4 (276 items, 32) 85 -> 75.
+static bool two_groups(int items, int chain) {
+  return chain >= (items <= cu_count() ? 8 : 32) && items <= 2 * cu_count();
+}
 
 template <typename T>
-static hipError_t launch(int which, int causal, int mt, int ntiles, const Args& a, hipStream_t st) {
+static hipError_t launch(int which, int causal, int mt, int ntiles, const Args& a, hipStream_t st) {   // mt of dK / dV: `longest`
   dim3 block(256);
-  if ((which == 2 || which == 7) && !a.tiles3 && few_items(ntiles * a.nkv, a.nh, a.nkv)) {
+  if ((which == 2 || which == 7) && !a.tiles3 && two_groups(ntiles * a.nkv, a.nh / a.nkv * mt)) {
     Args b = a;
     b.nitems = ntiles * a.nkv;
     const dim3 grid(std::min(b.nitems, cu_count())), both(512);
@@ -1331,7 +1335,7 @@ static int fa_persist() {
 }
 
 // which: 0 = forward (mt must be 20: the 32x32x16 kernel, 128-row tiles), 1 = delta,
-//        2 = dK/dV (64-key tiles), 5 = dQ (32x32x16, 128-query tiles).  (Measured-slower
+//        2 = dK/dV (64-key tiles; mt: 64-row tiles of the longest sequence, as far as the caller knows), 5 = dQ (32x32x16, 128-query tiles).  (Measured-slower
 //        variants -- a 16x16x32 forward, the transposed-formulation forward, 16x16x32 dQ and a
 //        32x32x16 dK/dV -- were removed, profiles/r02_fa and profiles/r2_fa.)
 extern "C" hipError_t lumen_flash_attn(int dtype, int which, int causal, int mt,
@@ -1397,7 +1401,8 @@ extern "C" hipError_t lumen_flash_attn_paged(int dtype, int causal, const void* 
 }
 
 // Backward with the dS hand-off: which 7 = dK/dV + dS store (64-key tiles), 8 = dQ from dS
-// (64-query tiles).  ds: [nh][ds_total][64 x 64] 16-bit, ds_off[seq] = the sequence's first tile.
+// (64-query tiles).  ds: [nh][ds_total][64 x 64] 16-bit, ds_off[seq] = the sequence's first tile; longest: 64-row tiles of the
+// longest sequence (which 7).
 extern "C" hipError_t lumen_flash_attn_ds(int dtype, int which, int causal, const void* q,
                                           const void* k, const void* v, long long ldq,
                                           long long ldk, long long ldv, const float* lse,
@@ -1407,7 +1412,7 @@ extern "C" hipError_t lumen_flash_attn_ds(int dtype, int which, int causal, cons
                                           long long lddq, long long lddk, long long lddv,
                                           const float* delta, const int* rope_pos,
                                           const float* rope_cos, const float* rope_sin, void* ds,
-                                          const int* ds_off, int ds_total, hipStream_t st) {
+                                          const int* ds_off, int ds_total, int longest, hipStream_t st) {
   const int tiles3 = (which >> 8) & 1;
   which &= 0xff;
   if (nkv <= 0 || nh % nkv != 0 || (which != 7 && which != 8) || ds == nullptr ||
@@ -1425,7 +1430,7 @@ extern "C" hipError_t lumen_flash_attn_ds(int dtype, int which, int causal, cons
   a.snake = (fa_persist() >> 3) & 1;
   a.nitems = tiles3 ? 0 : (which == 7 && (fa_persist() & 1)) ? ntiles * nkv
                         : (which == 8 && (fa_persist() & 4)) ? ntiles * nh : 0;
-  if (dtype == lumen::kBF16) return lumen::fa::launch<lumen::bf16>(which, causal, 1, ntiles, a, st);
-  if (dtype == lumen::kF16) return lumen::fa::launch<lumen::fp16>(which, causal, 1, ntiles, a, st);
+  if (dtype == lumen::kBF16) return lumen::fa::launch<lumen::bf16>(which, causal, longest, ntiles, a, st);
+  if (dtype == lumen::kF16) return lumen::fa::launch<lumen::fp16>(which, causal, longest, ntiles, a, st);
   return hipErrorInvalidValue;
 }

@@ -444,6 +444,7 @@ class _FlashAttn(torch.autograd.Function):
         qtiles = _tiles(cu, rq, qkv.device)
         ds_off, ds_total = (_ds_offsets(cu, causal, qkv.device) if FA_DS_MB > 0
                             else (None, 0))
+        longest = -(-max((b - a for a, b in zip(cu, cu[1:])), default=0) // rkv)      # (tiles of the longest sequence: how many waves an item takes)
         if ds_off is not None and nh * ds_total * 8192 <= FA_DS_MB * 2 ** 20:
             ds = torch.empty(nh, ds_total, 4096, device=qkv.device, dtype=qkv.dtype)
             if not handed:
@@ -453,14 +454,14 @@ class _FlashAttn(torch.autograd.Function):
             t7 = _tiles(cu, 64, qkv.device, heavy_low=causal)
             t8 = _tiles(cu, 64, qkv.device)
             C.flash_attn_ds(7, causal, q, k, v, lse, cut, t7, nh, nkv,
-                            scale, do, dq, dk, dv, delta, ds, ds_off, ds_total, pos, cos, sin)
+                            scale, do, dq, dk, dv, delta, ds, ds_off, ds_total, longest, pos, cos, sin)
             C.flash_attn_ds(8, causal, q, k, v, lse, cut, t8, nh, nkv,
-                            scale, do, dq, dk, dv, delta, ds, ds_off, ds_total, pos, cos, sin)
+                            scale, do, dq, dk, dv, delta, ds, ds_off, ds_total, longest, pos, cos, sin)
         else:
             if not handed:
                 C.flash_attn(1, causal, 1, q, k, v, o, lse, cut, _tiles(cu, 64, qkv.device), nh,
                              nkv, scale, do, None, None, None, delta, None, None, None)
-            C.flash_attn(wkv, causal, 1, q, k, v, o, lse, cut, _tiles(cu, rkv, qkv.device), nh,
+            C.flash_attn(wkv, causal, longest, q, k, v, o, lse, cut, _tiles(cu, rkv, qkv.device), nh,
                          nkv, scale, do, dq, dk, dv, delta, pos, cos, sin)
             C.flash_attn(wq, causal, 1, q, k, v, o, lse, cut, qtiles, nh, nkv,
                          scale, do, dq, dk, dv, delta, pos, cos, sin)

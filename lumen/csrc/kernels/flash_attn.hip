@@ -20,6 +20,8 @@
 //        in registers, loops over query tiles and the GQA group's heads), and dQ per 64-query
 //        tile (loops over key tiles); the softmax row statistics come from the forward's LSE
 //        and delta = rowsum(dO * O) (preprocess kernel).
+#include <algorithm>
+#include <cstdlib>
 #include "common.h"
 #include <cstdlib>
 
@@ -1253,6 +1255,19 @@ static int cu_count() {
   return n;
 }
 
+// persistent launches (bit 0 dK/dV, 1 forward, 2 dQ-from-dS; bit 3 snake item order);
+// LUMEN_FA_PERSIST overrides.
+// Default 15 = all three, snake order.  dK/dV: 109.6 -> 91.6 us persistent (gpurun r2_51),
+// snake 98.0 -> 96.3 (r2_55).  Forward: slower persistent with its round-2 prologue
+// (52.4 -> 55.6), faster since Q arrives by LDS-DMA with the first K/V tile: 45.1 -> 41.0 us at
+// B=8 S=512 and 128 -> 95 us at B=2 S=2048 causal.  dQ-from-dS: neutral at B=8 S=512, backward
+// 338 -> 320 us at B=2 S=2048 causal (profiles/r3d/fa; round 2 measured it slower, 35.2 -> 39.4,
+// before the dQ kernel's register fix).
+static int fa_persist() {
+  static int v = [] { const char* e = std::getenv("LUMEN_FA_PERSIST"); return e ? std::atoi(e) : 15; }();
+  return v;
+}
+
 // Do two groups of waves an item pay for dK / dV?  `longest`: query tiles of the longest sequence, so its heaviest item is a chain of
 // nh / nkv as many steps.  Chains of eight and more where every item has a CU of its own, of 32 and more up to two items a CU: the sums
 // that meet cost 1 - 2 us and two items of a CU share it less well so.  Whole backward, us, one group -> two.  Up to an item a CU (256): chain 1
@@ -1269,8 +1284,8 @@ static hipError_t launch(int which, int causal, int mt, int ntiles, const Args& 
   dim3 block(256);
   if ((which == 2 || which == 7) && !a.tiles3 && two_groups(ntiles * a.nkv, a.nh / a.nkv * mt)) {
     Args b = a;
-    b.nitems = ntiles * a.nkv;
-    const dim3 grid(std::min(b.nitems, cu_count())), both(512);
+    b.nitems = fa_persist() & 1 ? ntiles * a.nkv : 0;
+    const dim3 grid = b.nitems > 0 ? dim3(std::min(b.nitems, cu_count())) : dim3(ntiles, a.nkv), both(512);
     if (which == 7) {
       if (causal) hipLaunchKernelGGL((bwd_dkdv_kernel<T, true, true, 2>), grid, both, 0, st, b);
       else hipLaunchKernelGGL((bwd_dkdv_kernel<T, false, true, 2>), grid, both, 0, st, b);
@@ -1319,21 +1334,6 @@ static hipError_t launch(int which, int causal, int mt, int ntiles, const Args& 
 }  // namespace fa
 }  // namespace lumen
 
-#include <algorithm>
-#include <cstdlib>
-// persistent launches (bit 0 dK/dV, 1 forward, 2 dQ-from-dS; bit 3 snake item order);
-// LUMEN_FA_PERSIST overrides.
-// Default 15 = all three, snake order.  dK/dV: 109.6 -> 91.6 us persistent (gpurun r2_51),
-// snake 98.0 -> 96.3 (r2_55).  Forward: slower persistent with its round-2 prologue
-// (52.4 -> 55.6), faster since Q arrives by LDS-DMA with the first K/V tile: 45.1 -> 41.0 us at
-// B=8 S=512 and 128 -> 95 us at B=2 S=2048 causal.  dQ-from-dS: neutral at B=8 S=512, backward
-// 338 -> 320 us at B=2 S=2048 causal (profiles/r3d/fa; round 2 measured it slower, 35.2 -> 39.4,
-// before the dQ kernel's register fix).
-static int fa_persist() {
-  static int v = [] { const char* e = std::getenv("LUMEN_FA_PERSIST"); return e ? std::atoi(e) : 15; }();
-  return v;
-}
-
 // which: 0 = forward (mt must be 20: the 32x32x16 kernel, 128-row tiles), 1 = delta,
 //        2 = dK/dV (64-key tiles; mt: 64-row tiles of the longest sequence, as far as the caller knows), 5 = dQ (32x32x16, 128-query tiles).  (Measured-slower
 //        variants -- a 16x16x32 forward, the transposed-formulation forward, 16x16x32 dQ and a
@@ -1364,8 +1364,8 @@ extern "C" hipError_t lumen_flash_attn(int dtype, int which, int causal, int mt,
   a.rope_pos = rope_pos; a.rope_cos = rope_cos; a.rope_sin = rope_sin;
   a.kv_lens = nullptr; a.block_tables = nullptr; a.bt_stride = 0; a.block_size = 0;
   a.ds = nullptr; a.ds_off = nullptr; a.ds_total = 0; a.tiles3 = tiles3;
-  a.nitems = (which == 0 && mt == 20 && !tiles3 && (fa_persist() & 2)) ? ntiles * nh : 0;
-  a.snake = (fa_persist() >> 3) & 1;
+  a.nitems = (which == 0 && mt == 20 && !tiles3 && (lumen::fa::fa_persist() & 2)) ? ntiles * nh : 0;
+  a.snake = (lumen::fa::fa_persist() >> 3) & 1;
   if (which == 6 || which == 7 || which == 8) return hipErrorInvalidValue;  // other entries
   if (dtype == lumen::kBF16) return lumen::fa::launch<lumen::bf16>(which, causal, mt, ntiles, a, st);
   if (dtype == lumen::kF16) return lumen::fa::launch<lumen::fp16>(which, causal, mt, ntiles, a, st);
@@ -1427,9 +1427,9 @@ extern "C" hipError_t lumen_flash_attn_ds(int dtype, int which, int causal, cons
   a.lddv = lddv; a.delta = delta;
   a.rope_pos = rope_pos; a.rope_cos = rope_cos; a.rope_sin = rope_sin;
   a.ds = ds; a.ds_off = ds_off; a.ds_total = ds_total; a.tiles3 = tiles3;
-  a.snake = (fa_persist() >> 3) & 1;
-  a.nitems = tiles3 ? 0 : (which == 7 && (fa_persist() & 1)) ? ntiles * nkv
-                        : (which == 8 && (fa_persist() & 4)) ? ntiles * nh : 0;
+  a.snake = (lumen::fa::fa_persist() >> 3) & 1;
+  a.nitems = tiles3 ? 0 : (which == 7 && (lumen::fa::fa_persist() & 1)) ? ntiles * nkv
+                        : (which == 8 && (lumen::fa::fa_persist() & 4)) ? ntiles * nh : 0;
   if (dtype == lumen::kBF16) return lumen::fa::launch<lumen::bf16>(which, causal, longest, ntiles, a, st);
   if (dtype == lumen::kF16) return lumen::fa::launch<lumen::fp16>(which, causal, longest, ntiles, a, st);
   return hipErrorInvalidValue;

@@ -1,4 +1,8 @@
 """dK / dV of few (key tile, kv head) items: two groups of waves share an item's (head, query tile) steps."""
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -103,3 +107,19 @@ def test_short_chains_keep_one_group(nh, nkv, lens, two, hand_over, monkeypatch)
     do = torch.randn(sum(lens), nh * D, device="cuda", dtype=torch.bfloat16)
     names = [n for n, _, _ in launches(lambda: gradients(qkv, do, lens, nh, nkv, True)) if "dkdv" in n]
     assert [grouped(n) for n in names] == [two]
+
+
+@pytest.mark.parametrize("hand_over", [2048, 0])
+@pytest.mark.parametrize("switch,grid", [("15", (256, 1, 1)), ("14", (72, 4, 1))])
+def test_the_switch_of_persistent_launches(switch, grid, hand_over):
+    """288 items: persistent workgroups are one a CU, else there is one an item.  (The switch is read once a process.)"""
+    run = """
+import torch, test_flash_groups_gpu as t
+qkv, do = (torch.randn(9 * 512, n * 128, device="cuda", dtype=torch.bfloat16) for n in (24, 16))
+print(*[g for n, g, _ in t.launches(lambda: t.gradients(qkv, do, [512] * 9, 16, 4, True)) if "dkdv" in n])
+"""
+    tests = os.path.dirname(os.path.abspath(__file__))
+    env = dict(os.environ, LUMEN_FA_PERSIST=switch, LUMEN_FA_DS_MB=str(hand_over), PYTHONPATH=os.pathsep.join([os.path.dirname(tests), tests]))
+    out = subprocess.run([sys.executable, "-c", run], env=env, capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0, out.stderr
+    assert out.stdout.strip().splitlines()[-1] == str(grid)

@@ -344,7 +344,8 @@ hipError_t run(ThinArgs p, int per_cu, hipStream_t st) {
 // 16, each with workgroups of its own that hold more of W in flight.  All rows -> groups, us, 64 rows: 128 x 2048 6.1 -> 3.8, 256 x
 // 4096 9.5 -> 4.9 (16 and eight waves; of 32 4.7, 6.9), 2048 x 2048 7.8 -> 6.1, 2048 x 5632 17.1 -> 12.0 (32), 3072 x 2048 8.1 -> 7.5
 // (32, 32-row tiles; 16-row ones 9.6), 4096 x 4096 14.2 -> 13.8, 6144 x 2048 13.3 -> 11.8; 32 rows: 128 x 2048 4.5 -> 3.6, 2048 x 2048
-// 6.2 -> 5.1, 2048 x 5632 12.4 -> 10.3 (16; 3072 x 2048 would go 6.5 -> 7.0).
+// 6.2 -> 5.1, 2048 x 5632 12.4 -> 10.3 (16: two groups of 2048 columns' tiles are a workgroup a CU; 2112 would go x 512 3.0 -> 3.3, x 1024 4.1
+// -> 4.4, x 2048 6.0 -> 6.1, 3072 x 2048 6.5 -> 7.0).
 // Up to 16 rows of a matrix of up to 2048 rows take tiles of eight columns, eight waves and the stages that fit: as many CUs as
 // there are (16-column tiles of 2048 leave half of them idle).  us, 16-column tiles -> these, 1 / 8 / 16 rows: 2048 x 2048 4.7 / 5.0 /
 // 5.2 -> 4.3 / 4.4 / 4.8, 2048 x 5632 8.2 / 8.5 / 9.9 -> 6.9 / 7.2 / 8.5, 2048 x 12672 12.9 / 15.1 / 18.0 -> 11.0 / 12.2 / 14.8 (8 rows, 4.2 TB/s),
@@ -369,7 +370,7 @@ hipError_t pick(const ThinArgs& p, hipStream_t st) {
   if (p.M <= 32) {
     if (wide && p.K >= 4096) return run<T, 2, 4, 4, 3>(p, 1, st);
     if (wide) return run<T, 4, 4, 2, 3>(p, 1, st);
-    if (p.N <= 2112 && p.E == 0) return run<T, 1, 2, 4, 4>(p, 2, st);    // rows in groups of 16
+    if (p.N <= 8 * kCUs && p.E == 0) return run<T, 1, 2, 4, 4>(p, 2, st);   // rows in two groups of 16
     return run<T, 1, 4, 4, 3>(p, 2, st);
   }
   if (wide) return run<T, 4, 8, 2, 3>(p, 1, st);

@@ -4,6 +4,7 @@ rows, bias, fp32 results; and the rule that sends a projection to it."""
 import pytest
 import torch
 
+from launches import launches
 from lumen.ops.gemm import project, thin_linear, thin_ok
 from lumen.ops.moe import (ClampedGate, gated_act_ref, moe_dense, scaled_act_ref, thin_act,
                            thin_act_ok)
@@ -198,3 +199,15 @@ def test_gated_tiles_of_eight_columns(M, K, ff, dtype, tol):
             gate, up = gate.clamp(max=act.limit_shared), up.clamp(-act.limit_shared, act.limit_shared)
             want = gate * torch.sigmoid(act.slope * gate) * (up + act.shift)
         assert ((got - want).abs() <= 1.05 * tol * want.abs() + 2e-5 * want.abs().max()).all()
+
+
+@pytest.mark.parametrize("M,N,K,grid", [(17, 2048, 512, (128, 2)), (32, 2048, 2048, (128, 2)), (17, 2052, 512, (129, 1)), (32, 2112, 1024, (132, 1)),
+                                        (33, 2048, 512, (128, 2)), (64, 2052, 512, (65, 2))])
+def test_groups_of_rows_where_each_has_a_cu(M, N, K, grid):
+    """17 - 32 rows go in two groups of 16 while all of their workgroups have a CU each."""
+    x, w = torch.randn(M, K, device="cuda").bfloat16(), torch.randn(N, K, device="cuda").bfloat16()
+    (name, g, _), = launches(lambda: thin_linear(x, w))
+    assert "thin_kernel" in name and g[:2] == grid
+    want = x.double() @ w.double().t()
+    acc, ulp = bound(x, w, 8)
+    assert ((thin_linear(x, w).double() - want).abs() <= acc + want.abs() * ulp).all()

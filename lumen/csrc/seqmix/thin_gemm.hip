@@ -337,15 +337,16 @@ hipError_t run(ThinArgs p, int per_cu, hipStream_t st) {
 }
 
 // The tile.  One 16-row tile per step of four waves (two workgroups share a CU) is best or within 3 %
-// everywhere at M <= 16, except that long rows of a matrix with few tiles, and few tiles of any kind, want eight waves (2048 x
-// 5632: 8.3 vs 8.4 - 9 us, 256 x 4096: 4.6 vs 5.5) and the widest long-row matrices want 32-row tiles (22528 x 4096: 31.5 vs
+// everywhere at M <= 16, except that long rows want eight waves at M <= 8 (one row of 2112 x 5632 8.0 vs 9.6 us, of 4096 x 8192 13.4 vs
+// 16.1; 6144 x 5632 would be 14.3 for 15.4) and the widest long-row matrices want 32-row tiles (22528 x 4096: 31.5 vs
 // 32.8 us, x read half as often).  Above 16 rows x costs as much as W: many tiles take all rows of x, 64 to an x
 // fragment (11264 x 2048 at M = 64: 15.3 vs 18.7 us with 32); where that leaves CUs idle the rows are cut into groups of 32 or
 // 16, each with workgroups of its own that hold more of W in flight.  All rows -> groups, us, 64 rows: 128 x 2048 6.1 -> 3.8, 256 x
 // 4096 9.5 -> 4.9 (16 and eight waves; of 32 4.7, 6.9), 2048 x 2048 7.8 -> 6.1, 2048 x 5632 17.1 -> 12.0 (32), 3072 x 2048 8.1 -> 7.5
 // (32, 32-row tiles; 16-row ones 9.6), 4096 x 4096 14.2 -> 13.8, 6144 x 2048 13.3 -> 11.8; 32 rows: 128 x 2048 4.5 -> 3.6, 2048 x 2048
 // 6.2 -> 5.1, 2048 x 5632 12.4 -> 10.3 (16: two groups of 2048 columns' tiles are a workgroup a CU; 2112 would go x 512 3.0 -> 3.3, x 1024 4.1
-// -> 4.4, x 2048 6.0 -> 6.1, 3072 x 2048 6.5 -> 7.0).
+// -> 4.4, x 2048 6.0 -> 6.1, 3072 x 2048 6.5 -> 7.0).  The eight waves of up to 256 columns have use for more than three stages of k for every two
+// of them (64 rows of 256 columns, four waves over eight: k 64 - 256 0.88, 320 - 768 0.95, 832 1.02, 1536 1.05).
 // Up to 16 rows of a matrix of up to 2048 rows take tiles of eight columns, eight waves and the stages that fit: as many CUs as
 // there are (16-column tiles of 2048 leave half of them idle).  us, 16-column tiles -> these, 1 / 8 / 16 rows: 2048 x 2048 4.7 / 5.0 /
 // 5.2 -> 4.3 / 4.4 / 4.8, 2048 x 5632 8.2 / 8.5 / 9.9 -> 6.9 / 7.2 / 8.5, 2048 x 12672 12.9 / 15.1 / 18.0 -> 11.0 / 12.2 / 14.8 (8 rows, 4.2 TB/s),
@@ -354,19 +355,19 @@ hipError_t run(ThinArgs p, int per_cu, hipStream_t st) {
 // half tiles (2112 x 2048, 8 rows 4.9 -> 5.4).
 template <typename T>
 hipError_t pick(const ThinArgs& p, hipStream_t st) {
-  const bool wide = p.N >= 8192, tiny = p.N <= 256;
+  const bool wide = p.N >= 8192;
   if (p.N <= 8 * kCUs && p.K >= 1024 && p.M <= 16)
     return p.M <= 8 ? run<T, 1, 1, 8, 5, 0, 1>(p, 1, st) : run<T, 1, 2, 8, 4, 0, 1>(p, 1, st);
   if (p.M <= 8) {
     if (wide && p.K >= 4096) return run<T, 2, 1, 4, 4>(p, 1, st);
-    if (!wide && (p.K >= 4608 || tiny)) return run<T, 1, 1, 8, 4>(p, 2, st);
+    if (!wide && p.K >= 4608) return run<T, 1, 1, 8, 4>(p, 2, st);
     return run<T, 1, 1, 4, 4>(p, 2, st);
   }
-  if (tiny && p.E == 0) return run<T, 1, 2, 8, 4>(p, 1, st);
   if (p.M <= 16) {
     if (wide && p.K >= 4096) return run<T, 2, 2, 4, 4>(p, 1, st);
     return run<T, 1, 2, 4, 4>(p, 2, st);
   }
+  if (p.N <= 256 && p.E == 0) return p.K > 768 ? run<T, 1, 2, 8, 4>(p, 1, st) : run<T, 1, 2, 4, 4>(p, 2, st);
   if (p.M <= 32) {
     if (wide && p.K >= 4096) return run<T, 2, 4, 4, 3>(p, 1, st);
     if (wide) return run<T, 4, 4, 2, 3>(p, 1, st);

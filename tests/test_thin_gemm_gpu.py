@@ -211,3 +211,15 @@ def test_groups_of_rows_where_each_has_a_cu(M, N, K, grid):
     want = x.double() @ w.double().t()
     acc, ulp = bound(x, w, 8)
     assert ((thin_linear(x, w).double() - want).abs() <= acc + want.abs() * ulp).all()
+
+
+@pytest.mark.parametrize("M,N,K,waves", [(1, 256, 64, 4), (8, 64, 960, 4), (8, 256, 1024, 8), (9, 16, 512, 4), (16, 256, 960, 4), (17, 256, 768, 4),
+                                         (17, 128, 832, 8), (32, 16, 64, 4), (33, 64, 448, 4), (64, 256, 768, 4), (64, 256, 832, 8), (63, 256, 4096, 8)])
+def test_waves_of_small_matrices(M, N, K, waves):
+    """Eight waves of a workgroup want more than three stages of 64 for each pair of them."""
+    x, w = torch.randn(M, K, device="cuda").bfloat16(), torch.randn(N, K, device="cuda").bfloat16()
+    (name, _, block), = launches(lambda: thin_linear(x, w))
+    assert "thin_kernel" in name and block[0] == 64 * waves
+    want = x.double() @ w.double().t()
+    acc, ulp = bound(x, w, 8)
+    assert ((thin_linear(x, w).double() - want).abs() <= acc + want.abs() * ulp).all()

@@ -156,8 +156,7 @@ gated_rms_kernel(const float* __restrict__ x, const T* __restrict__ g, long long
 }
 
 // The same for aligned groups of at most N x 256 entries a wave, in registers: values, gates and weights are asked for together, as
-// a decoded row costs the chain of its loads (launch after launch, one group: one row of 2048 3.38 -> 2.82 us, of 4096 4.72 -> 3.60;
-// 4096 rows of 2048 15.7 -> 14.6).
+// a decoded row costs the chain of its loads (launch after launch, one group: one row of 2048 3.38 -> 2.82 us, of 4096 4.72 -> 3.60).
 template <typename T, int N>
 __global__ void __launch_bounds__(256)
 gated_rms_wide_kernel(const float* __restrict__ x, const T* __restrict__ g, long long ldg, const float* __restrict__ w,
@@ -383,8 +382,11 @@ hipError_t sm_gated_rms(int dt, const float* x, const void* g, long long ldg, co
   const int gs = W / groups;
   const bool small = vec && gs <= 256 && (uintptr_t)w % 16 == 0 && W % 4 == 0;
   const int wave_per = groups >= 4 ? 1 : groups == 1 ? 4 : groups == 2 ? 2 : 1, passes = (gs + 256 * wave_per - 1) / (256 * wave_per);
-  // (one pass leaves waves without an entry: many rows of 512, one group, 7.0 us through LDS, 7.6 in registers)
-  const bool wide = vec && (uintptr_t)w % 16 == 0 && (rows <= 1024 || passes > 1);
+  // In registers up to 768 rows; beyond, waves hide each other's chains, and lanes without an entry of the last part and the
+  // registers of four parts cost more than LDS does (LDS -> registers, us, 768 / 1024 / 4096 rows: 512, one group 3.2 -> 3.2 / 3.5 -> 3.6 / 7.0 ->
+  // 7.8; 2560 5.7 -> 5.6 / 6.3 -> 6.5 / 16.9 -> 17.9; 4096 7.2 -> 6.8 / 8.6 -> 8.4 / 24.1 -> 26.1; 3072 5.9 -> 5.5 / 7.0 -> 6.7 / 19.4 -> 19.5)
+  const bool full = wave_per == 1 || gs % (256 * wave_per) == 0 || (passes == 1 && gs >= 192 * wave_per);
+  const bool wide = vec && (uintptr_t)w % 16 == 0 && (rows <= 768 || (full && (passes <= 3 || rows <= 1024)));
   int SG = 1;
   while (4 * SG < gs) SG <<= 1;
   const long long items = (long long)rows * groups;
@@ -398,6 +400,9 @@ hipError_t sm_gated_rms(int dt, const float* x, const void* g, long long ldg, co
                                 groups, shared_w, gate_first, sigmoid, eps);                    \
   else if (wide && passes <= 2)                                                                 \
     gated_rms_wide_kernel<TT, 2><<<grid, 256, 0, st>>>(x, (const TT*)g, ldg, w, (TT*)out, W,    \
+                                groups, shared_w, gate_first, sigmoid, eps);                    \
+  else if (wide && passes <= 3)                                                                 \
+    gated_rms_wide_kernel<TT, 3><<<grid, 256, 0, st>>>(x, (const TT*)g, ldg, w, (TT*)out, W,    \
                                 groups, shared_w, gate_first, sigmoid, eps);                    \
   else if (wide && passes <= 4)                                                                 \
     gated_rms_wide_kernel<TT, 4><<<grid, 256, 0, st>>>(x, (const TT*)g, ldg, w, (TT*)out, W,    \

@@ -1,0 +1,30 @@
+"""Which row kernel a call takes: rows held in registers while a row's chain of loads is what it costs, in LDS or by passes where many
+rows hide that, at the edges of either; each against float64."""
+import pytest
+import torch
+
+from launches import launches
+from lumen.ops import norm
+from test_step_rows_gpu import gen, near
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+def kernel(run):
+    (name, _, _), = launches(run)
+    return name
+
+
+@pytest.mark.parametrize("T,W,groups,held", [
+    (1, 512, 1, 1), (768, 512, 1, 1), (769, 512, 1, 0), (2000, 1024, 1, 1), (769, 1536, 1, 0), (1025, 768, 2, 1), (1025, 768, 1, 1), (1025, 640, 1, 0), (1025, 2048, 2, 2), (1500, 1536, 4, 2),
+    (768, 2560, 1, 3), (769, 2560, 1, 0), (1500, 3072, 1, 3), (5, 3072, 2, 3), (1024, 4096, 1, 4), (1025, 4096, 1, 0), (1025, 4096, 4, 0), (769, 3584, 2, 0),
+    (3, 4100, 1, 0)])
+def test_gated_norms(T, W, groups, held):
+    r = gen(W + T)
+    o, z, w = r(T, W), r(T, W).to(BF16), r(W)
+    name = kernel(lambda: norm.gated_rms_norm(o, z, w, groups, 1e-6, "silu", True))
+    assert (f"gated_rms_wide_kernel<__hip_bfloat16, {held}>" in name) if held else "gated_rms_kernel<" in name
+    a = torch.sigmoid(z.double()) * z.double()
+    p = (o.double() * a).reshape(T, groups, -1)
+    near(norm.gated_rms_norm(o, z, w, groups, 1e-6, "silu", True), (p / torch.sqrt((p * p).mean(-1, keepdim=True) + 1e-6)).reshape(T, W) * w.double())

@@ -12,7 +12,8 @@
 //
 // One workgroup per row, four channels per lane.  Rows of up to 4096 aligned channels stay in registers, and everything that the row
 // takes, the norm's weight too, is asked for before the first sum: a decoded row costs its chain of loads (bf16,
-// launch after launch: one row of 2048 3.03 -> 2.72 us, of 4096 4.08 -> 3.29; 4096 rows of 2048 20.9 -> 20.4).  Other rows stay in LDS between the sum of squares and the output.
+// launch after launch: one row of 2048 3.03 -> 2.72 us, of 4096 4.08 -> 3.29).  Other rows, and many of them, stay in LDS between the sum
+// of squares and the output: see the launch.
 #include "seqmix.h"
 
 using namespace lumen;
@@ -209,13 +210,18 @@ hipError_t sm_stream_rms(int dt, float* x, int keep, const void* table, const lo
   const bool vec = W % 4 == 0 && al(x) && al(table) && al(table_rows) && al(y) && al(f0) &&
                    al(f1) && al(f2) && al(w) && al(h);
   const size_t lds = w != nullptr ? (size_t)W * sizeof(float) : 0;
+  // Many rows hide each other's chains, and the registers of a row then cost more than its LDS (LDS -> registers, us, 768 / 1024 / 2048 rows:
+  // 256 columns 2.9 -> 2.8 / 3.0 -> 3.1 / 3.4 -> 3.6, 1024 3.4 -> 3.3 / 3.8 -> 3.6 / 5.4 -> 5.2, 2048 4.6 -> 4.6 / 5.3 -> 5.2 / 7.1 -> 7.6, 3072 5.5 -> 5.4 /
+  // 6.2 -> 6.4 / 11.1 -> 12.5, 4096 6.4 -> 6.5 / 7.2 -> 7.7 / 16.0 -> 16.8; 1280 rows of 4096 8.5 -> 10.8)
+  const int most = W > 512 && W <= 1024 ? 4096 : W > 1024 && W <= 2048 ? 1024 : 768;
 #define CALL(T)                                                                                   \
   {                                                                                               \
     StreamArgs<T> a{x, keep, (const T*)table, tokens, vocab, scale, (T*)table_rows, (const T*)y,  \
                     f0, f1, f2, coef, w, (T*)h, split, (long long)rows * W, W, eps};              \
-    if (vec && W <= 1024) stream_row_kernel<T, 1><<<rows, kThreads, 0, st>>>(a);                  \
-    else if (vec && W <= 2048) stream_row_kernel<T, 2><<<rows, kThreads, 0, st>>>(a);             \
-    else if (vec && W <= 4096) stream_row_kernel<T, 4><<<rows, kThreads, 0, st>>>(a);             \
+    if (vec && rows <= most && W <= 1024) stream_row_kernel<T, 1><<<rows, kThreads, 0, st>>>(a);                  \
+    else if (vec && rows <= most && W <= 2048) stream_row_kernel<T, 2><<<rows, kThreads, 0, st>>>(a);             \
+    else if (vec && rows <= most && W <= 3072) stream_row_kernel<T, 3><<<rows, kThreads, 0, st>>>(a);             \
+    else if (vec && rows <= most && W <= 4096) stream_row_kernel<T, 4><<<rows, kThreads, 0, st>>>(a);             \
     else if (vec) stream_rms_kernel<T, 4><<<rows, kThreads, lds, st>>>(a);                        \
     else stream_rms_kernel<T, 1><<<rows, kThreads, lds, st>>>(a);                                 \
   }

@@ -28,3 +28,16 @@ def test_gated_norms(T, W, groups, held):
     a = torch.sigmoid(z.double()) * z.double()
     p = (o.double() * a).reshape(T, groups, -1)
     near(norm.gated_rms_norm(o, z, w, groups, 1e-6, "silu", True), (p / torch.sqrt((p * p).mean(-1, keepdim=True) + 1e-6)).reshape(T, W) * w.double())
+
+
+@pytest.mark.parametrize("T,W,held", [(1, 256, 1), (769, 256, 0), (769, 512, 0), (4096, 768, 1), (4097, 1024, 0), (1024, 2048, 2), (1025, 2048, 0),
+                                      (768, 2560, 3), (769, 2560, 0), (5, 3072, 3), (768, 4096, 4), (769, 4096, 0), (769, 3072, 0), (2, 4100, 0)])
+def test_stream_norms(T, W, held):
+    r = gen(W + T)
+    x, y, w = r(T, W), r(T, W).to(BF16), r(W)
+    want = x.double() + y.double()
+    h = norm.residual_rms(x, y, w, 1e-6)
+    near(x, want)
+    near(h, want / torch.sqrt((want * want).mean(-1, keepdim=True) + 1e-6) * w.double())
+    name = kernel(lambda: norm.residual_rms(x, y, w, 1e-6))
+    assert (f"stream_row_kernel<__hip_bfloat16, {held}>" in name) if held else "stream_rms_kernel<" in name

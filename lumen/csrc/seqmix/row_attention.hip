@@ -1204,7 +1204,9 @@ hipError_t sm_head_norm_write(int dt, void* qkv, long long ld, const float* wq, 
                    (uintptr_t)kcache % 16 == 0 && (uintptr_t)vcache % 16 == 0 &&
                    (uintptr_t)wq % 16 == 0 && (uintptr_t)wk % 16 == 0;
   const int SG = D / 8, rounds = SG > 0 && SG <= 64 ? ((H + 2 * G) * SG + 255) / 256 : 99;
-  if (vec && dt != kF32 && D == Dv && D % 8 == 0 && (SG & (SG - 1)) == 0 && ld % 8 == 0 && rounds <= 4) {
+  // (up to four heads to norm, a wave each is as short a chain, with a head over all lanes: 2 + 1 heads of 128 2.2 us, here 2.5, 4096 rows
+  // 5.5 and 6.6, 2 + 2 6.6 and 7.1; 4 + 1 2.8 and 2.4, 4 + 2 4096 rows 9.8 and 8.4)
+  if (vec && dt != kF32 && D == Dv && D % 8 == 0 && (SG & (SG - 1)) == 0 && ld % 8 == 0 && rounds <= 4 && H + G > 4) {
 #define LANES(TT, R) head_norm_write_lanes<TT, R><<<T, 256, 0, st>>>((TT*)qkv, ld, wq, wk, slots, (TT*)kcache, (TT*)vcache, H, G, D, SG, eps)
     if (dt == kBF16) { if (rounds <= 2) LANES(bf16, 2); else LANES(bf16, 4); }
     else { if (rounds <= 2) LANES(fp16, 2); else LANES(fp16, 4); }

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from launches import launches
+from lumen.ops import attention as A
 from lumen.ops import norm
 from test_step_rows_gpu import gen, near
 
@@ -41,3 +42,27 @@ def test_stream_norms(T, W, held):
     near(h, want / torch.sqrt((want * want).mean(-1, keepdim=True) + 1e-6) * w.double())
     name = kernel(lambda: norm.residual_rms(x, y, w, 1e-6))
     assert (f"stream_row_kernel<__hip_bfloat16, {held}>" in name) if held else "stream_rms_kernel<" in name
+
+
+def heads_of(T, H, G, D, dims):
+    r = gen(H * D + T)
+    slots = torch.randperm(T, generator=torch.Generator().manual_seed(T)).cuda()
+    caches = [torch.zeros(T, 1, G, D, device="cuda", dtype=BF16) for _ in range(2)]
+    return r(T, (H + 2 * G) * D).to(BF16), r, slots, caches
+
+
+@pytest.mark.parametrize("T,H,G,D,lanes", [(1, 2, 1, 128, 0), (70, 3, 1, 128, 0), (5, 1, 1, 512, 0), (3, 4, 1, 128, 1), (70, 2, 2, 128, 0),
+                                           (5, 4, 2, 64, 1), (2, 16, 4, 128, 1), (2, 32, 32, 128, 0)])
+def test_head_norms(T, H, G, D, lanes):
+    """Four heads and fewer to norm keep a wave each."""
+    z, r, slots, (kc, vc) = heads_of(T, H, G, D, 0)
+    wq, wk = r(D), r(D)
+    got = z.clone()
+    A.head_norm_write(got, wq, wk, slots, kc, vc, H, G, D, D, 1e-6)
+    x = z.double().view(T, H + 2 * G, D)
+    unit = x / torch.sqrt((x * x).mean(-1, keepdim=True) + 1e-6)
+    near(got[:, :H * D], (unit[:, :H] * wq.double()).reshape(T, -1), 1e-5)
+    near(kc[slots, 0].flatten(1), (unit[:, H:H + G] * wk.double()).reshape(T, -1), 1e-5)
+    assert torch.equal(vc[slots, 0].flatten(1), z[:, (H + G) * D:])
+    name = kernel(lambda: A.head_norm_write(got, wq, wk, slots, kc, vc, H, G, D, D, 1e-6))
+    assert ("head_norm_write_lanes<" if lanes else "head_norm_write_kernel<") in name

@@ -127,7 +127,10 @@ __global__ void __launch_bounds__(kThreads) row_norm_rotary_kernel(const RowRotA
 
 // The same with a thread's N items held in registers from the sums on: everything that a row takes is asked for at once (a
 // decoded row costs its chain of loads: 16 + 4 heads of 128, one row 3.24 -> 3.09 us, 64 rows 3.52 -> 3.34; 32 + 8 heads 3.97 -> 3.52,
-// 4.23 -> 3.88).  Many rows of few items leave threads without one (4096 rows of 8 + 2 heads of 64: 7.0 us above, 7.8 here).
+// 4.23 -> 3.88).  Many rows hide each other's chains, and threads without an item or its registers then cost more (us, 512 / 768 / 1024 /
+// 2048 rows, above -> here: 8 + 2 heads of 64 3.5 -> 3.5 / 3.6 -> 3.7 / 3.7 -> 3.9 / 4.9 -> 5.5, 16 + 4 of 128 3.9 -> 3.9 / 4.3 -> 4.3 / 4.7 -> 4.9 /
+// 6.8 -> 7.1, 32 + 8 of 128 5.1 -> 5.0 / 5.8 -> 5.7 / 6.5 -> 6.9 / 11.2 -> 12.4), unless every thread has its two items (32 + 32 of 128, 4096 rows
+// 38.5 -> 30.9) or there are rows enough to read them once (4096 rows of 32 + 8 19.6 -> 18.9, 8192 of 16 + 4 0.98; 3072 1.03).
 template <typename T, int N>
 __global__ void __launch_bounds__(kThreads) row_norm_rotary_held(const RowRotArgs<T> a) {
   __shared__ float s_cs[kMaxHead / 2], s_sn[kMaxHead / 2];
@@ -259,7 +262,8 @@ hipError_t sm_row_norm_rotary(int dt, void* z, long long ld, const float* wq, co
     RowRotArgs<TT> a{(TT*)z, ld, wq, wk, positions, slots, (TT*)kc, (TT*)vc, inv_freq, H, G, D,   \
                      vw, dims, amp, eps};                                                         \
     if constexpr (sizeof(TT) == 2) {                                                              \
-      if (fits(8) && items <= 2 * kThreads && (T <= 1024 || items > kThreads / 2)) {                                                     \
+      if (fits(8) && items <= 2 * kThreads && (T <= 512 || items == 2 * kThreads ||             \
+                                               (T > 3072 && items > kThreads / 2))) {             \
         if (items <= kThreads) row_norm_rotary_held<TT, 1><<<T, kThreads, 0, st>>>(a);            \
         else row_norm_rotary_held<TT, 2><<<T, kThreads, 0, st>>>(a);                              \
         return hipGetLastError();                                                                 \

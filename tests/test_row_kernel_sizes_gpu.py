@@ -66,3 +66,27 @@ def test_head_norms(T, H, G, D, lanes):
     assert torch.equal(vc[slots, 0].flatten(1), z[:, (H + G) * D:])
     name = kernel(lambda: A.head_norm_write(got, wq, wk, slots, kc, vc, H, G, D, D, 1e-6))
     assert ("head_norm_write_lanes<" if lanes else "head_norm_write_kernel<") in name
+
+
+@pytest.mark.parametrize("T,H,G,D,dims,held", [(512, 8, 2, 64, 64, 1), (513, 8, 2, 64, 64, 0), (513, 2, 1, 128, 0, 0), (512, 32, 8, 128, 128, 2),
+                                               (513, 32, 8, 128, 128, 0), (600, 16, 4, 128, 128, 0), (600, 32, 32, 128, 128, 2), (3073, 16, 4, 128, 128, 1), (3073, 8, 2, 64, 64, 0), (3, 33, 32, 128, 128, 0)])
+def test_row_norms_with_rotation(T, H, G, D, dims, held):
+    z, r, slots, (kc, vc) = heads_of(T, H, G, D, dims)
+    wq, wk, pos = r(H * D), r(G * D), torch.arange(T, device="cuda", dtype=torch.int32) % 90
+    f = 1.0 / 100 ** torch.linspace(0, 1, max(1, dims // 2), device="cuda")
+    got = z.clone()
+    run = lambda: A.row_norm_rotary_write(got, wq, wk, pos, slots, kc, vc, H, G, D, D, dims, f, 1.0, 1e-6)  # noqa: E731
+    run()
+    a = (pos.float().view(T, 1, 1) * f.view(1, 1, -1)).double()
+
+    def want(x, w, n):
+        x = (x / torch.sqrt((x * x).mean(-1, keepdim=True) + 1e-6) * w.double()).view(T, n, D)
+        u, v = x[..., :dims // 2], x[..., dims // 2:dims]
+        return torch.cat([u * a.cos() - v * a.sin(), v * a.cos() + u * a.sin(), x[..., dims:]], -1).flatten(1) if dims else x.flatten(1)
+
+    zd = z.double()
+    near(got[:, :H * D], want(zd[:, :H * D], wq, H), 1e-5)
+    near(kc[slots, 0].flatten(1), want(zd[:, H * D:(H + G) * D], wk, G), 1e-5)
+    assert torch.equal(vc[slots, 0].flatten(1), z[:, (H + G) * D:])
+    name = kernel(run)
+    assert (f"row_norm_rotary_held<__hip_bfloat16, {held}>" in name) if held else "row_norm_rotary_kernel<" in name

@@ -1,6 +1,6 @@
 // The chunked matrix-state recurrences of head_scan_chunk16.hip with every chunk's matrices built ahead, for steps whose
 // sequences and heads leave the chip idle: a prompt is a serial chain of chunks there, and a chunk costs as long as its producer
-// waves take to build it (delta rule 5.2 us, most of it the triangle's inverse in one wave; 3.3 without).
+// waves take to build it (32 heads of 128: delta rule 5.5 us, most of it the triangle's inverse in one wave; 3.3 without, 2.1 with constant decays).
 //
 // None of that depends on the state.  chunk_prep_kernel builds all chunks at once, a workgroup per chunk and key head: rows of q
 // and k (transposed once more) into LDS, then a wave forms G . Q K^T and the factors, and another the inverse, per head.  Its LDS
@@ -9,7 +9,7 @@
 // LDS.  One forms the read-outs a chunk later.  One fetches, LDS-DMA of whole images and rows of values.  They meet once a chunk
 // (twice with the delta rule).
 // Cycles a chunk at width 2048, busy: state waves 4030 (delta) and 2670, read-outs 2040 and 3010, fetching 1000 - 1400.  One state wave that
-// owned all rows was busy 5710 and 4000; one wave that formed the read-outs too took 2.9 and 2.05 us a chunk, now 1.7 and 1.3.
+// owned all rows was busy 5710 and 4000; one wave that formed the read-outs too took 2.9 and 2.05 us a chunk, now 1.85 and 1.25 (32 heads: 2.1 and 1.35).
 #include "head_chunk16.h"
 
 using namespace lumen;

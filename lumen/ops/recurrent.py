@@ -313,10 +313,21 @@ def head_scan_ref(q, k, v, state, seg: SegBatch, H, rep, Dk, Dv, decay, beta=Non
 
 
 # The scan whose chunks are built ahead (head_scan_ahead.hip): where sequences x heads x 32-column blocks leave CUs idle, a chunk of
-# the chain takes 1.7 us instead of 4.4 (delta rule), 1.3 instead of 2.8.  Chunk producers in each workgroup -> ahead, us, width 4096:
-# 1 x 512 rows delta 79 -> 46, constant decays 52 -> 34, state-space 47 -> 36; 1 x 2048 286 -> 135, 187 -> 101, 173 -> 104; 1 x 96 21 -> 18,
-# 15.5 -> 13.6, 15.8 -> 15.3.  Two rounds of workgroups (4 x 512) would go 81 -> 87, 55 -> 72, 67 -> 110, 64 rows a sequence 13.0 -> 13.7.
-AHEAD_MIN_ROWS, AHEAD_MAX_BLOCKS = 96, 256
+# the chain takes 2.1 us instead of 5.5 (delta rule), 1.35 instead of 3.3 (steps and decays per token) and 1.3 instead of 2.1 (constant
+# decays), 32 heads of 128.  Chunk producers in each workgroup -> ahead, us: 1 x 512 rows 91 -> 47, 58 -> 35, 41 -> 33; 1 x 2048 357 -> 146, 219 ->
+# 99, 143 -> 97.  Two rounds of workgroups (4 x 512) would go 81 -> 87, 67 -> 110, 55 -> 72.
+# What the second launch costs grows with the key heads and heads it builds for, and what it saves with a sequence's rows and with what a
+# chunk is to build: keys past 64, or keys that no 16-byte loads can read, and the triangle of the delta rule.  The rows of the longest
+# sequence from which it pays, for rows of its length x (heads + 3 key heads) / 4 of up to 32, up to 64 and more (ahead / producers, sequences
+# of one length, heads of their own keys):
+AHEAD_MAX_BLOCKS = 256
+AHEAD_MIN_ROWS = {
+    ("delta", False): (96, 96, 112),         # 8 heads of 64: 0.78 at 96 rows; x 8 0.91; 16 heads x 8 1.06, at 160 0.97
+    ("delta", True): (96, 96, 112),          # 16 of 128: 0.72; 16 of 96 x 8 1.05, at 128 0.98
+    ("token", False): (112, 160, 320),       # 16 of 64: 1.01 at 96, 0.94 at 128; x 4 1.13, at 160 1.03, 192 0.99; x 8 1.29, at 384 1.00
+    ("token", True): (96, 96, 224),          # 16 of 128: 0.79, x 4 0.90; 16 of 96 x 8 1.08, at 256 0.92
+    ("const", False): (192, 700, 1 << 30),   # 16 of 64: 1.11 at 96, 0.98 at 192; x 4 1.24, at 512 1.08, 1024 0.91; x 8 1.38, at 1024 1.06
+    ("const", True): (96, 96, 700)}          # 16 of 128: 0.87, x 4 0.99; 16 of 96 x 8 1.21, at 1024 1.00
 AHEAD_MAX_BYTES = 1 << 28        # of its workspace, 0.8 MB a chunk at width 4096
 
 
@@ -359,7 +370,11 @@ def head_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.Te
     if P:
         chunks = (rows + 31 * P) // 32
         size = 0
-        if (rows >= AHEAD_MIN_ROWS * P and P * H * ((Dv + 31) // 32) <= AHEAD_MAX_BLOCKS and q.dtype == torch.bfloat16
+        slow = Dk > 64 or (Dk | _ld(q) | _ld(k)) % 8 != 0 or (q.data_ptr() | k.data_ptr()) % 16 != 0
+        longest = seg.keys[1] if seg.fresh and seg.keys is not None else rows / P    # (as far as the host knows: its chain is what is saved)
+        load = rows / longest * (H + 3 * (H // rep))
+        least = AHEAD_MIN_ROWS["delta" if beta is not None else "const" if const else "token", slow][(load > 128) + (load > 256)]
+        if (longest >= least and P * H * ((Dv + 31) // 32) <= AHEAD_MAX_BLOCKS and q.dtype == torch.bfloat16
                 and Dv % 8 == 0 and v.data_ptr() % 16 == 0 and 0 < _ld(v) < 1 << 25 and _ld(v) % 8 == 0):
             size = head_scan_ahead_bytes(beta is not None, Dk, H, rep, chunks)
         if 0 < size <= AHEAD_MAX_BYTES:

@@ -371,7 +371,8 @@ def head_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.Te
         chunks = (rows + 31 * P) // 32
         size = 0
         slow = Dk > 64 or (Dk | _ld(q) | _ld(k)) % 8 != 0 or (q.data_ptr() | k.data_ptr()) % 16 != 0
-        longest = seg.keys[1] if seg.fresh and seg.keys is not None else rows / P    # (as far as the host knows: its chain is what is saved)
+        # (as far as the host knows: its chain is what is saved)
+        longest = max(1, seg.keys[1] if seg.fresh and seg.keys is not None else rows / P)
         load = rows / longest * (H + 3 * (H // rep))
         least = AHEAD_MIN_ROWS["delta" if beta is not None else "const" if const else "token", slow][(load > 128) + (load > 256)]
         if (longest >= least and P * H * ((Dv + 31) // 32) <= AHEAD_MAX_BLOCKS and q.dtype == torch.bfloat16

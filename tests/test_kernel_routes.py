@@ -539,3 +539,14 @@ def test_splits_of_latent_keys_are_of_the_tile_that_the_kernel_takes(launched, T
                   vt=torch.zeros(1, R, 16, **BF))
     (name, a), = launched
     assert name == "sm_latent_attn" and a[-3] == splits
+
+
+def test_scans_of_portions_without_rows(launched):
+    from lumen.ops.recurrent import head_scan
+    from lumen.ops.segments import SegBatch
+
+    i32 = dict(dtype=torch.int32)
+    seg = SegBatch(torch.zeros(3, **i32), torch.arange(2, **i32), torch.zeros(2, **i32), torch.zeros(0, **i32), torch.zeros(0, **i32))
+    x = torch.zeros(0, 4 * 32, **BF)
+    assert head_scan(x, x, x, torch.zeros(2, 4, 32, 32), seg, 4, 32, 32, torch.zeros(4)).shape == (0, 128)
+    assert [n for n, _ in launched] == ["sm_head_scan_chunk"]

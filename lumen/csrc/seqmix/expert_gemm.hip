@@ -324,27 +324,45 @@ long long tiles_of(int T, int E, int top, int bm, long long ce, long long cs) {
   return ((long long)T * top / bm + E) * ce + (long long)((T + bm - 1) / bm) * cs;
 }
 
-// Rows of a tile / 32: the least time of all rounds of the CUs, as far as the sizes tell.  Of T top / E rows each, more or less
-// by their root.  us a tile, by stages of 64 k, as measured (4096 rows, 8 experts of 1408 and a shared one, width 2048: act of 256
-// rows in rounds and a cut one 139 us, of 128 rows 165, of 64 240).
-int pick_rows(int T, int E, int top, int nk, int ce, int cs) {
-  const double r = (double)T * top / E, s = 1.5 * sqrt(r);
-  const auto tiles = [&](int bm) {
-    double n = 0.;
-    for (const double x : {r - s, r, r + s}) n += x <= bm ? 1. : ceil(x / bm);
-    return ceil(n * E / 3. * ce) + (double)((T + bm - 1) / bm) * cs;
+// Rows of a tile / 32: the least time expected of all rounds of the CUs; an expert's and the shared one's weights in bytes.  The host
+// knows T top / E rows an expert, more or less by their root and some for routers that prefer: the tiles are counted at eight places of that
+// spread, the rounds at that many and at their own spread above and below.  us a tile by stages of 64 k, and the memory's time for the
+// weights (behind which tiles of 256 rows leave the more to do), fitted to 616 sizes and routings by chance and by preference: over the best
+// of the three the choice takes 1.1 % more time on average, by the mean and one spread alone it took 1.8 %, tiles of 128 always 11 % (act, us,
+// rows 64 / 128 / 256: 256 rows, 4 experts of 5632, width 2048 67 / 45 / 55, 512 rows 61 / 75 / 55; 512 rows, 8 of 2816, width 4096 113 / 137 / 102;
+// 4096 rows, 8 of 1408 and a shared one 240 / 165 / 139).
+int pick_rows(int T, int E, int top, int nk, int ce, int cs, double expert, double shared) {
+  static const double kPlaces[8] = {-1.53, -0.89, -0.49, -0.16, 0.16, 0.49, 0.89, 1.53};
+  const double r = (double)T * top / E, s = 1.25 * sqrt(r);
+  const double t4 = 0.86 * nk + 10., t2 = 0.56 * nk + 8., cut = 0.33 * nk + 7., t8 = 1.2 * nk + 6.;
+  double chosen = 0.;                                     // the share of experts with rows
+  for (const double z : kPlaces) chosen += r + z * s > 0.5 ? 0.125 : 0.;
+  const double memory = (E * chosen * expert + shared) / 6.3e6;
+  const auto expected = [&](int bm, double least, const auto& cost) {
+    double sum = 0., sq = 0.;
+    for (const double z : kPlaces) {
+      const double x = r + z * s, n = x <= 0.5 ? 0. : ceil(x / bm);
+      sum += n;
+      sq += n * n;
+    }
+    const double mean = sum / 8., each = sqrt(fmax(0., sq / 8. - mean * mean) * E) * ce;
+    const double n = mean * E * ce + (double)((T + bm - 1) / bm) * cs;
+    return fmax(least, cost(ceil(n - each))) + fmax(least, cost(ceil(n))) + fmax(least, cost(ceil(n + each)));
   };
-  const auto rounds = [&](int bm) { return ceil(tiles(bm) / tile::CUS); };
-  const double full = floor(tiles(256) / tile::CUS), left = tiles(256) - full * tile::CUS;
-  const double t4 = 0.72 * nk + 10., t2 = 0.55 * nk + 9., cut = 0.42 * nk + 8., t8 = 1.25 * nk + 11.;
-  const double all8 = full * t8 + (left == 0. ? 0. : 4 * left <= tile::CUS ? cut : 2 * left <= tile::CUS ? t4 : t8);
-  const double all4 = rounds(128) * t4, all2 = rounds(64) * t2;
+  const double all8 = expected(256, memory + 16., [&](double n) {
+    const double full = floor(n / tile::CUS), left = n - full * tile::CUS;
+    return full * t8 + (left <= 0. ? 0. : 4 * left <= tile::CUS ? cut : 2 * left <= tile::CUS ? t4 : t8);
+  });
+  const double all4 = expected(128, memory, [&](double n) { return ceil(n / tile::CUS) * t4; });
+  const double all2 = expected(64, memory, [&](double n) { return ceil(n / tile::CUS) * t2; });
   return all8 < all4 && all8 < all2 ? 8 : all4 <= all2 ? 4 : 2;
 }
 
 template <typename T, int MODE, int ACT>
 hipError_t launch(const ExpertArgs& p, int top, int ce, int cs, hipStream_t st) {
-  const int nk = (MODE == 2 ? (p.ff > p.ffs ? p.ff : p.ffs) : p.W) / BK, mj = pick_rows(p.T, p.E, top, nk, ce, cs);
+  const int nk = (MODE == 2 ? (p.ff > p.ffs ? p.ff : p.ffs) : p.W) / BK;
+  const double row = (MODE == 0 ? 4. : 2.) * p.W;         // bytes of weights for an activation
+  const int mj = pick_rows(p.T, p.E, top, nk, ce, cs, row * p.ff, row * p.ffs);
   // (MJ 8: what is left over may take a round of its own)
   const unsigned grid = (unsigned)(tiles_of(p.T, p.E, top, 32 * mj, ce, cs) + (mj == 8 ? tile::CUS : 0));
   switch (mj) {

@@ -4,6 +4,7 @@ fewer choices than `top`, several thousand rows, row strides, every activation, 
 import pytest
 import torch
 
+from launches import launches
 from lumen.ops import moe as M
 
 pytestmark = pytest.mark.gpu
@@ -138,3 +139,14 @@ def test_replays():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, M.moe_chosen(h2, w2, gu, down, E, top, ff, ffs))
+
+
+@pytest.mark.parametrize("T,W,E,top,ff,ffs,act,down", [(256, 4096, 8, 2, 2816, 0, 4, 2), (256, 2048, 4, 1, 5632, 0, 4, 8), (4096, 2048, 8, 2, 1408, 1408, 8, 8),
+                                                       (64, 2048, 8, 2, 1408, 1408, 2, 2), (512, 4096, 8, 2, 2816, 0, 8, 4)])
+def test_tiles_by_the_rounds_to_be_expected(T, W, E, top, ff, ffs, act, down):
+    """64 rows an expert by the mean are more than one tile of 64 for half of them, and a round that was not counted."""
+    h, wts, gu, w2 = layer(T, W, E, top, ff, ffs, True, torch.bfloat16, 3)
+    args = (E, top, ff, ffs, "silu", True, "output")
+    names = [n for n, _, _ in launches(lambda: M.moe_chosen(h, wts, gu, w2, *args)) if "expert_kernel<" in n]
+    got = [n.split("expert_kernel<")[1].split(">")[0].split(", ")[1:3] for n in names]
+    assert got == [["0", str(act)], ["2", str(down)]]

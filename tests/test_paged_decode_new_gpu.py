@@ -116,16 +116,23 @@ def test_refused():
 
 @pytest.mark.parametrize("D,nh,nkv,dt", [(128, 5, 5, torch.bfloat16), (64, 6, 3, torch.float16), (32, 4, 1, torch.bfloat16), (256, 2, 2, torch.float16)])
 def test_merge_of_partitions(D, nh, nkv, dt):
-    """Up to 130 partitions, at the edges of the merge's 16 rows and 64 lanes, over scratch memory that holds NaN; against
-    the context in one partition, whose fp32 sums have another order, so a result may round the other way."""
-    from lumen.ops.attention import paged_decode
+    """Up to 130 partitions, at the edges of the merge's 4 and 16 rows and 64 lanes, over parts that hold NaN where no partition
+    lies; against the context in one partition, whose fp32 sums have another order, so a result may round the other way."""
+    from lumen.ops._native import native
+    from lumen.ops.attention import PA_ONE_PASS, paged_decode
 
-    lens = [64, 65, 128, 129, 16 * 64, 16 * 64 + 1, 32 * 64 + 7, 64 * 64 - 1, 64 * 64 + 1, 80 * 64 + 1, 130 * 64 - 5]
+    lens = [64, 65, 128, 129, 4 * 64, 4 * 64 + 1, 16 * 64, 16 * 64 + 1, 32 * 64 + 7, 64 * 64 - 1, 64 * 64 + 1, 80 * 64 + 1, 130 * 64 - 5]
     qkv, kc, vc, bt, cl, *_ = _case(D, nh, nkv, lens, dt, False)
     q = qkv[:, :nh * D].view(len(lens), nh, D)
-    scratch = torch.full((len(lens) * nh * 140 * (D + 2) + (1 << 20),), math.nan, device="cuda")
-    del scratch
-    got = paged_decode(q, kc, vc, bt, cl, 140 * 64, 1 / math.sqrt(D), 64).float()
+    m, l = (torch.full((len(lens), nh, 140), math.nan, device="cuda") for _ in range(2))
+    o = torch.full((len(lens), nh, 140, D), math.nan, device="cuda")
+    got = torch.full((len(lens), nh, D), math.nan, device="cuda", dtype=dt)
+    native().paged_attention_decode(got, q, kc, vc, bt, cl, nkv, kc.shape[2], bt.shape[1], 1 / math.sqrt(D), m, l, o, 64, None, PA_ONE_PASS)
+    for i, n in enumerate(lens):
+        parts = -(-n // 64) if n > 64 else 0                 # (one partition writes its result at once)
+        assert m[i, :, parts:].isnan().all() and l[i, :, parts:].isnan().all() and o[i, :, parts:].isnan().all()
+        assert parts == 0 or m[i, :, :parts].isfinite().all()
+    got = got.float()
     one = paged_decode(q, kc, vc, bt, cl, 140 * 64, 1 / math.sqrt(D), 140 * 64).float()
     ulp = 2.0 ** (-7 if dt == torch.bfloat16 else -10)
     assert ((got - one).abs() <= ulp * one.abs() + 2.0 ** -16 * one.abs().max()).all()

@@ -678,26 +678,19 @@ __global__ void __launch_bounds__(256) pa_decode1_kernel(
   }
 }
 
-// The partitions' parts of a sequence and head, a wave: 64 of their maxima and sums a lane each, 16 rows of values asked for
+// The partitions' parts of a sequence and head, a wave: 64 of their maxima and sums a lane each, B rows of values asked for
 // with them.  A chain of two trips to memory, the context's length and all of this; a loop over the maxima, one over the sums and
-// one over the values made four (a Llama decode step of 4 layers, one sequence of 387 tokens: 376.0 -> 372.6 us).
-template <typename T, int D>
-__global__ void __launch_bounds__(256) pa_reduce_kernel(T* __restrict__ out,
-                                                        const int* __restrict__ context_lens,
-                                                        const float* __restrict__ tmp_m,
-                                                        const float* __restrict__ tmp_l,
-                                                        const float* __restrict__ tmp_o, int nh, int max_parts, int PART) {
-  constexpr int W = D / 64 > 0 ? D / 64 : 1, B = 16;      // columns of a lane, rows at a time
-  const int seq = blockIdx.x, lane = threadIdx.x & 63;
-  const int head = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int nparts = (context_lens[seq] + PART - 1) / PART;
-  if (nparts <= 1 || head >= nh) return;                  // (one: written directly by the decode kernel)
-  const size_t row = static_cast<size_t>(seq) * nh + head, base = row * max_parts;
+// one over the values made four (a Llama decode step of 4 layers, one sequence of 387 tokens: 376.0 -> 372.6 us).  Up to four parts ask for
+// four rows: with 16 they waited for twelve copies of their last one (32 heads, two parts 8.4 us with the attention, now 7.5; loops 7.65).
+template <typename T, int D, int B>
+__device__ __forceinline__ void merge_parts(T* __restrict__ out, const float* __restrict__ tmp_m, const float* __restrict__ tmp_l,
+                                            const float* __restrict__ tmp_o, int lane, int nparts) {
+  constexpr int W = D / 64 > 0 ? D / 64 : 1;              // columns of a lane
   const int d = min(lane * W, D - W);
   float mp, lp, v[B][W];
   int n;
   const auto rows = [&](int p, int q0) __attribute__((always_inline)) {  // (past the end the last one again: not used)
-    const float* po = tmp_o + (base + p) * D + d;
+    const float* po = tmp_o + static_cast<size_t>(p) * D + d;
 #pragma unroll
     for (int q = 0; q < B; ++q)
 #pragma unroll
@@ -705,8 +698,8 @@ __global__ void __launch_bounds__(256) pa_reduce_kernel(T* __restrict__ out,
   };
   const auto ask = [&](int p) __attribute__((always_inline)) {
     n = min(64, nparts - p);
-    mp = tmp_m[base + p + min(lane, n - 1)];
-    lp = tmp_l[base + p + min(lane, n - 1)];
+    mp = tmp_m[p + min(lane, n - 1)];
+    lp = tmp_l[p + min(lane, n - 1)];
     rows(p, 0);
     // (all of it has arrived here: the compiler would move the rows' loads behind the maximum)
     asm volatile("" : "+v"(mp), "+v"(lp));
@@ -717,7 +710,7 @@ __global__ void __launch_bounds__(256) pa_reduce_kernel(T* __restrict__ out,
   };
   ask(0);
   float M = mp, L = 0.f, o[W];
-  for (int p = 64; p < nparts; p += 64) M = fmaxf(M, tmp_m[base + min(p + lane, nparts - 1)]);
+  for (int p = 64; p < nparts; p += 64) M = fmaxf(M, tmp_m[min(p + lane, nparts - 1)]);
   M = wave_max(M);
 #pragma unroll
   for (int j = 0; j < W; ++j) o[j] = 0.f;
@@ -741,7 +734,22 @@ __global__ void __launch_bounds__(256) pa_reduce_kernel(T* __restrict__ out,
   }
   if (lane * W < D)
 #pragma unroll
-    for (int j = 0; j < W; ++j) out[row * D + d + j] = from_f32<T>(o[j] / L);
+    for (int j = 0; j < W; ++j) out[d + j] = from_f32<T>(o[j] / L);
+}
+
+template <typename T, int D>
+__global__ void __launch_bounds__(256) pa_reduce_kernel(T* __restrict__ out,
+                                                        const int* __restrict__ context_lens,
+                                                        const float* __restrict__ tmp_m,
+                                                        const float* __restrict__ tmp_l,
+                                                        const float* __restrict__ tmp_o, int nh, int max_parts, int PART) {
+  const int seq = blockIdx.x, lane = threadIdx.x & 63;
+  const int head = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nparts = (context_lens[seq] + PART - 1) / PART;
+  if (nparts <= 1 || head >= nh) return;                  // (one: written directly by the decode kernel)
+  const size_t row = static_cast<size_t>(seq) * nh + head, base = row * max_parts;
+  if (nparts <= 4) merge_parts<T, D, 4>(out + row * D, tmp_m + base, tmp_l + base, tmp_o + base * D, lane, nparts);
+  else merge_parts<T, D, 16>(out + row * D, tmp_m + base, tmp_l + base, tmp_o + base * D, lane, nparts);
 }
 
 // k, v: [ntok, nkv, D] rows with row strides k_stride / v_stride (elements), scattered to

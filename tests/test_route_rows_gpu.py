@@ -46,7 +46,8 @@ def test_given_rows(T, W, E, top, dt, calls):
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("T,W,E,top", [(1, 8, 2, 1), (64, 2048, 8, 2), (3, 1032, 16, 3), (2, 8192, 5, 2), (9, 4096, 64, 4)])
+@pytest.mark.parametrize("T,W,E,top", [(1, 8, 2, 1), (64, 2048, 8, 2), (3, 1032, 16, 3), (2, 8192, 5, 2), (9, 4096, 64, 4),
+                                       (2, 2048, 16, 1), (2, 2048, 17, 1), (3, 1024, 32, 2), (3, 1024, 33, 2), (1, 2048, 60, 3)])
 def test_with_the_norm(T, W, E, top, dt, calls):
     r, y, R, b = _rows(T, W, E, dt)
     x0, w = r(T, W), 1 + 0.1 * r(W)

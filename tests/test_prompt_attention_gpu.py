@@ -5,6 +5,7 @@ that creep upwards, and unowned cache rows full of NaN."""
 import pytest
 import torch
 
+from launches import launches
 from lumen.ops.attention import chunk_sink_attention, chunk_sink_attention_ref, row_attention, row_attention_ref
 from lumen.ops.segments import SegBatch, tile_list
 
@@ -49,7 +50,8 @@ def close(out, ref, ulp):
     ([31, 32, 33, 63, 64, 65, 1], [0, 0, 1, 0, 70, 3, 5], 16, 0, 0),
     ([127, 128, 129], [0, 64, 1], 12, 70, 5), ([130, 66], [200, 61], 16, 64, 130), ([40, 5], [560, 0], 1, 0, 0),
     ([33], [700], 1, 620, 7)])
-@pytest.mark.parametrize("H,G,D,Dv", [(4, 2, 128, 128), (2, 2, 32, 64), (2, 1, 128, 256), (258, 2, 32, 32), (258, 6, 64, 128)])
+@pytest.mark.parametrize("H,G,D,Dv", [(4, 2, 128, 128), (2, 2, 32, 64), (2, 1, 128, 256), (258, 2, 32, 32), (258, 6, 64, 128),
+                                      (258, 2, 128, 128)])
 def test_window_tiles(H, G, D, Dv, lens, starts, bs, window, keep, dtype, ulp):
     g = torch.Generator().manual_seed(D + bs + len(lens))
     T, seg, (k, v) = portions(lens, starts, bs, g, (G, D), (G, Dv))
@@ -78,6 +80,21 @@ def test_chunk_tiles(H, G, D, lens, starts, bs, chunk, dtype, ulp):
 
 
 @pytest.mark.parametrize("dtype,ulp", DTYPES)
+@pytest.mark.parametrize("lens,starts,bs,chunk", [
+    ([31, 32, 33, 63, 64, 65, 1], [0, 0, 1, 0, 70, 3, 5], 16, 0), ([127, 128, 129], [0, 64, 1], 12, 75)])
+@pytest.mark.parametrize("H,G,D", [(258, 2, 128), (258, 3, 96)])
+def test_chunk_tiles_of_many_workgroups(H, G, D, lens, starts, bs, chunk, dtype, ulp):
+    """Whole tiles of keys a wave; the reference forms each key head's first and last query head."""
+    g = torch.Generator().manual_seed(D + bs + len(lens))
+    T, seg, (k,) = portions(lens, starts, bs, g, (G, D))
+    k = k.to(dtype).cuda()
+    q = torch.randn(T, H * D, generator=g).to(dtype).cuda()
+    out = chunk_sink_attention(q, k, seg, H, G, D, 0.3, chunk, 1e-6).view(T, G, H // G, D)[:, :, [0, -1]].reshape(T, -1)
+    some = q.view(T, G, H // G, D)[:, :, [0, -1]].reshape(T, -1)
+    close(out, chunk_sink_attention_ref(some.float(), k.float(), seg, 2 * G, G, D, 0.3, chunk, 1e-6), ulp)
+
+
+@pytest.mark.parametrize("dtype,ulp", DTYPES)
 @pytest.mark.parametrize("rise", [0.01, 0.07, 0.5, -0.5])
 def test_scores_that_creep(rise, dtype, ulp):
     """The score grows by ``rise`` per key: under and over what moves the reference within a tile."""
@@ -99,7 +116,7 @@ def test_scores_that_creep(rise, dtype, ulp):
 
 @pytest.mark.parametrize("dtype,ulp", DTYPES)
 @pytest.mark.parametrize("lens,extra", [([31, 32, 33, 1, 65], 0), ([127, 128, 129, 260], 3)])
-@pytest.mark.parametrize("H,tile", [(1, 128), (5, 128), (2, 64)])
+@pytest.mark.parametrize("H,tile", [(1, 128), (5, 128), (2, 64), (130, 128)])
 def test_fresh_latent_rows(H, tile, lens, extra, dtype, ulp):
     """Prompts over their own rows against the reference, rows of wider buffers, decoded rows behind them."""
     from lumen.ops.attention import fresh_latent_attention, fresh_latent_attention_ref, fresh_latent_ok
@@ -181,6 +198,30 @@ def test_mixed_head_tiles_hold_fp32_weights(H, G, dtype, share):
     assert (out != ref.to(dtype)).double().mean() < share
 
 
+@pytest.mark.parametrize("kind,rows,H,halves", [("window", 128, 256, True), ("window", 129, 128, True), ("window", 128, 258, False), ("window", 129, 130, False),
+                                                ("chunk", 128, 256, True), ("chunk", 129, 130, False), ("fresh", 128, 128, True), ("fresh", 65, 8, True),
+                                                ("fresh", 64, 8, False), ("fresh", 128, 129, False)])
+def test_few_workgroups_take_halves_of_the_keys(kind, rows, H, halves):
+    """Two workgroups a tile of 128 rows, each with 64 of them, up to 256 (fresh: 128) tiles x heads: the tests above hold both forms."""
+    from lumen.ops.attention import fresh_latent_attention
+
+    g = torch.Generator().manual_seed(1)
+    T, seg, (k, v) = portions([rows], [0], 16, g, (2, 128), (2, 128))
+    seg.fresh = True
+    k, v, out = k.bfloat16().cuda(), v.bfloat16().cuda(), torch.empty(T, H, 128, dtype=torch.bfloat16, device="cuda")
+    f = lambda *s: torch.randn(*s, generator=g).bfloat16().cuda()  # noqa: E731
+    if kind == "fresh":
+        args = (f(T, H, 192), f(T, H, 128), f(T, 64), f(T, H, 128), out, seg, 0.07)
+        (_, grid, _), = launches(lambda: fresh_latent_attention(*args))
+    elif kind == "chunk":
+        q = f(T, H * 128)
+        (_, grid, _), = launches(lambda: chunk_sink_attention(q, k, seg, H, 2, 128, 0.3, 0, 1e-6))
+    else:
+        q = f(T, H, 128)
+        (_, grid, _), = launches(lambda: row_attention(q, None, k, v, 128, out, seg, H, 2, 0.1))
+    assert grid[0] == (2 if halves else 1) * -(-rows // 128) * H
+
+
 ODD = {5: (0, float("inf")), 37: (9, float("-inf")), 100: (21, float("nan"))}     # position: channel, value
 
 
@@ -202,7 +243,8 @@ def odd_rows(run, v, seg, window=0):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("kind,H,G,D,Dv,window", [
     ("window", 4, 2, 128, 128, 0), ("window", 2, 2, 64, 128, 20), ("window", 2, 1, 128, 256, 0), ("talk", 8, 2, 128, 128, 0),
-    ("talk", 16, 4, 128, 128, 0), ("talk", 24, 6, 128, 128, 0), ("fresh", 3, 3, 128, 128, 0)])
+    ("talk", 16, 4, 128, 128, 0), ("talk", 24, 6, 128, 128, 0), ("fresh", 3, 3, 128, 128, 0), ("window", 130, 2, 128, 128, 0),
+    ("window", 130, 2, 64, 128, 20), ("fresh", 66, 66, 128, 128, 0)])
 def test_infinite_values_of_hidden_tokens(kind, H, G, D, Dv, window, dtype):
     g = torch.Generator().manual_seed(H)
     T, seg, (k, v) = portions([131], [0], 16, g, (G, D), (G, Dv))
@@ -220,7 +262,8 @@ def test_infinite_values_of_hidden_tokens(kind, H, G, D, Dv, window, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("H,G,D,chunk", [(4, 2, 128, 0), (2, 1, 96, 50), (2, 2, 256, 0), (2, 2, 64, 128)])
+@pytest.mark.parametrize("H,G,D,chunk", [(4, 2, 128, 0), (2, 1, 96, 50), (2, 2, 256, 0), (2, 2, 64, 128), (130, 2, 128, 0), (130, 1, 96, 50),
+                                           (130, 2, 64, 128)])
 def test_infinite_keys_of_hidden_tokens(H, G, D, chunk, dtype):
     """Keys that are their own values: whole rows that see such a token are lost, the others keep what they had."""
     g = torch.Generator().manual_seed(H)

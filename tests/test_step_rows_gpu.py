@@ -3,6 +3,7 @@ experts by counting -- at the edges of the widths and row counts that they take,
 import pytest
 import torch
 
+from launches import launches
 from lumen.ops import attention as A
 from lumen.ops import moe, norm
 
@@ -42,17 +43,24 @@ def test_stream(T, W, dt):
     near(h, rms(parts[:T].double() + parts[T:].double() + 0.25 * base.double()), 2e-5)      # (three terms may cancel)
 
 
-@pytest.mark.parametrize("dt", [BF16, torch.float32])
+@pytest.mark.parametrize("off", [4, 8])
+@pytest.mark.parametrize("dt", [BF16, torch.float16, torch.float32])
 @pytest.mark.parametrize("T,W,groups", [(1, 256, 1), (2, 2048, 1), (1, 2052, 1), (3, 4096, 1), (2, 4100, 1), (2, 1032, 2), (4, 1536, 3),
                                         (1, 4096, 4), (2, 4112, 4), (3, 640, 5), (2, 4096, 32), (2, 66, 3), (1030, 512, 1)])
-def test_groups(T, W, groups, dt):
+def test_groups(T, W, groups, dt, off):
+    """Columns of a wider projection: from the eighth on in registers (16 bytes), from the fourth by passes in 16 bits."""
     r = gen(W + groups)
-    z, w, x = r(T, W + 8).to(dt)[:, 4:4 + W], r(W), r(T, W)
+    z, w, x = r(T, W + 16).to(dt)[:, off:off + W], r(W), r(T, W)
     ref = norm.group_rms_norm_ref(z.double(), w, groups, 1e-6, torch.float64)
     ref64 = (z.double().reshape(T, groups, -1) / torch.sqrt((z.double().reshape(T, groups, -1) ** 2).mean(-1, keepdim=True) + 1e-6)
              ).reshape(T, W) * w.double()
     near(ref.float(), ref64, 1e-6)
     near(norm.group_rms_norm(z, w, groups, 1e-6), ref64)
+    (name, _, _), = launches(lambda: norm.group_rms_norm(z, w, groups, 1e-6))
+    waves = 1 if groups >= 3 else 4 // groups
+    parts = -(-W // groups // (256 * waves))
+    held = off * z.element_size() % 16 == 0 and W // groups % 4 == 0 and (W + 16) % 4 == 0 and parts <= 4
+    assert (f", {1 if parts <= 1 else 2 if parts <= 2 else 4}>" in name and "group_rms_held<" in name) if held else "group_rms_kernel<" in name
     want = x.double() + ref64
     x, xb = norm.group_rms_residual(x, z, w, groups, 1e-6, dt)
     near(x, want)

@@ -1242,7 +1242,7 @@ __global__ void __launch_bounds__(256) bwd_dq_ds_kernel(Args a) {
 }
 
 // (An 8-wave, 128-key dK/dV variant with a 3-deep DMA ring measured slower than the 4-wave
-// kernel above -- 117.6 vs 108.0 us at B=8 S=512, gpurun r2_36 -- and was removed.)
+// kernel above -- 117.6 vs 108.0 us at B=8 S=512 -- and was removed.)
 
 static int cu_count() {
   static int n = [] {
@@ -1257,12 +1257,11 @@ static int cu_count() {
 
 // persistent launches (bit 0 dK/dV, 1 forward, 2 dQ-from-dS; bit 3 snake item order);
 // LUMEN_FA_PERSIST overrides.
-// Default 15 = all three, snake order.  dK/dV: 109.6 -> 91.6 us persistent (gpurun r2_51),
-// snake 98.0 -> 96.3 (r2_55).  Forward: slower persistent with its round-2 prologue
-// (52.4 -> 55.6), faster since Q arrives by LDS-DMA with the first K/V tile: 45.1 -> 41.0 us at
-// B=8 S=512 and 128 -> 95 us at B=2 S=2048 causal.  dQ-from-dS: neutral at B=8 S=512, backward
-// 338 -> 320 us at B=2 S=2048 causal (profiles/r3d/fa; round 2 measured it slower, 35.2 -> 39.4,
-// before the dQ kernel's register fix).
+// Default 15 = all three, snake order.  dK/dV: 109.6 -> 91.6 us persistent, snake 98.0 -> 96.3.
+// Forward: slower persistent while Q came through registers (52.4 -> 55.6), faster since it
+// arrives by LDS-DMA with the first K/V tile: 45.1 -> 41.0 us at B=8 S=512 and 128 -> 95 us at
+// B=2 S=2048 causal.  dQ-from-dS: neutral at B=8 S=512, backward 338 -> 320 us at B=2 S=2048
+// causal (profiles/r3d/fa; slower, 35.2 -> 39.4, before the dQ kernel's register fix).
 static int fa_persist() {
   static int v = [] { const char* e = std::getenv("LUMEN_FA_PERSIST"); return e ? std::atoi(e) : 15; }();
   return v;

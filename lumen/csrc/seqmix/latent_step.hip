@@ -308,10 +308,11 @@ hipError_t sm_latent_out(int dt, const float* ml, const float* part, int nsplit,
       (uintptr_t)uv % 16 || (uintptr_t)o % 8 || orow % 4 || oh % 4 || (dt != kBF16 && dt != kF16) ||
       (nsplit > 1 ? !ml || !part || (uintptr_t)part % 16 : !x || (uintptr_t)x % 8 || xr % 4 || xh % 4))
     return hipErrorInvalidValue;
-  // rows of a workgroup: 16, fewer where that leaves CUs idle, as the sums of 16 rows and a head's weights are 300 KB to
-  // fetch for one (16 rows -> fewer, us with the attention: 8 rows of 16 heads 16.7 -> 14.1, 16 of 8 18.8 -> 13.8, 64 of 16 25.8 -> 21.3)
+  // rows of a workgroup: 16, fewer while all of them have a CU each, as the sums of 16 rows and a head's weights are 300 KB to
+  // fetch for one (16 rows -> fewer, us with the attention: 8 rows of 16 heads 16.7 -> 14.1, 16 of 8 18.8 -> 13.8, 48 of 16 23.2 -> 19.3; more than
+  // one a CU fetch a head's weights again: two of 4 rows 48 of 16 22.8, 48 rows of 32 heads over 128, 40 keys, 8.5 -> 10.6)
   int per = 16;
-  while (per > 1 && (long long)((rows + per - 1) / per) * H < 256) per /= 2;
+  while (per > 1 && (long long)((rows + per / 2 - 1) / (per / 2)) * H <= 256) per /= 2;
   const dim3 grid((rows + per - 1) / per, H);
 #define GO(T, KS)                                                                                                 \
   latent_out_kernel<T, KS><<<grid, 4 * Dv, 0, st>>>(OutArgs<T>{ml, part, nsplit, (const T*)x, xr, xh, (const T*)gate, \

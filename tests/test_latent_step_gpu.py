@@ -3,6 +3,7 @@ epilogue, against the separate forms in float64."""
 import pytest
 import torch
 
+from launches import launches
 from lumen.ops.attention import LATENT_STEP_MAX_T, latent_inputs, latent_query, latent_write_ref
 from lumen.ops.embedding import gated_token_project, gated_token_slice_ref
 from lumen.ops.norm import group_rms_norm_ref
@@ -115,3 +116,35 @@ def test_sums_and_expansion(T, H, R, Dr, Dv, ctx, gated, dt):
         near(o, want, dt, ULP[dt])
     else:
         assert torch.equal(got.transpose(0, 1), ol)
+
+
+def rows_behind(T, H, R, Dr, ctx, dt):
+    """Decoded rows of up to ``ctx`` keys, the first of all of them: (queries, cache, transposed values, segments)."""
+    from lumen.ops.segments import SegBatch
+
+    g = torch.Generator(device="cuda").manual_seed(T + ctx)
+    r = lambda *s: torch.randn(*s, device="cuda", generator=g).to(dt)  # noqa: E731
+    bs, per, i32 = 16, (ctx + 15) // 16, dict(dtype=torch.int32, device="cuda")
+    lens = torch.randint(1, ctx + 1, (T,), generator=torch.Generator().manual_seed(T))
+    lens[0] = ctx
+    tables = torch.randperm(64 * per, generator=torch.Generator().manual_seed(ctx))[torch.arange(T * per) % (64 * per)].view(T, per).to(**i32)
+    cache, pos, ar = r(64 * per, bs, R + Dr), (lens - 1).to(**i32), torch.arange(T + 1, **i32)
+    return r(T, H, R), r(T, H, Dr), cache, cache[:, :, :R].transpose(1, 2).contiguous(), SegBatch(ar, ar[:T], pos, ar[:T], pos, tables, None)
+
+
+@pytest.mark.parametrize("T,H,R,ctx,grid", [(1, 16, 512, 40, 1), (16, 16, 512, 300, 16), (17, 16, 512, 300, 9), (48, 16, 128, 300, 12), (49, 32, 128, 40, 7),
+                                            (65, 32, 256, 9, 5), (300, 32, 128, 20, 19)])
+def test_rows_of_an_expansion_have_a_cu(T, H, R, ctx, grid):
+    """Workgroups of the expansion take 16 rows, or fewer while each has a CU of its own."""
+    from lumen.ops.attention import row_attention
+
+    dt = torch.bfloat16
+    q, q2, cache, vt, seg = rows_behind(T, H, R, 64, ctx, dt)
+    uv, o = (torch.randn(H, 64, R, device="cuda") / R ** 0.5).to(dt), torch.empty(T, H, 64, dtype=dt, device="cuda")
+    ol, args = torch.empty_like(q), (seg, H, 1, 0.05)
+    row_attention(q, q2, cache, cache, R, ol, *args, vt=vt)
+    run = lambda: row_attention(q, q2, cache, cache, R, torch.empty_like(q), *args, vt=vt, expand=(uv, o))  # noqa: E731
+    (name, g, _) = launches(run)[-1]
+    assert "latent_out_kernel" in name and g == (grid, H, 1)
+    want = torch.matmul(ol.double().transpose(0, 1), uv.double().transpose(1, 2).contiguous()).transpose(0, 1)
+    near(o, want, dt, ULP[dt])

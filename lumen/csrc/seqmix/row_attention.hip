@@ -43,6 +43,7 @@
 // and angles are fp32; 16-bit types only appear at loads and stores.  (16-bit heads of 128, 2 - 8 of them a key head, go to
 // step_attention.hip.)
 #include "row_attn_args.h"
+#include <algorithm>
 
 using namespace lumen;
 
@@ -1035,30 +1036,39 @@ inline size_t latent_attn_lds(int Dk, int esz) {
 
 // Rows times blocks of 16 heads up to which a workgroup takes 64 keys instead of 128: a CU fetches 60 B/ns, so few workgroups want
 // few keys each, and many the fewer partial sums (64 / 128 keys, us: 1 row 14.0 / 17.1, 16 rows of 8 heads 18.8 / 21.4, 32 of 16
-// 18.3 / 20.3, 64 of 16 23.3 / 21.3, of 2000 keys 51 / 53)
+// 18.3 / 20.3, 64 of 16 23.3 / 21.3, of 2000 keys 51 / 53).  128 too where these are one round of the CUs and 64 more than one (16 heads over
+// 512 + 64, 8 rows of up to 4000 keys 26.9 / 18.9, 16 of 2000 21.6 / 17.6, 32 of 800 20.0 / 17.5), and of 65 - 128 keys whose splits a launch of
+// its own would add (one row over 256 + 32 7.7 / 5.7, over 384 + 64 9.9 / 7.3)
 constexpr int kLatentNarrow = 32;
+// Of 128 keys a workgroup fills a CU, so two or more blocks of heads a row leave much of the last round idle past 256 of them: four splits
+// of more than kLatentWhole tiles there (32 heads over 512 + 64, one split -> four, us: 140 rows of up to 1200 keys 132 -> 103, 193 of 1900 234
+// -> 184, 300 of 1900 324 -> 289; 193 of 600 would go 71 -> 81).  One block of heads a row takes one or few (500 rows of 1900 276 -> 298).
+constexpr int kLatentWhole = 7;
+// Two of latent_attn_kernel's DEEP form fit a CU, and a row's blocks of heads side by side read its keys from HBM once: up to 512
+// workgroups of it are one round (32 heads over 512 + 64, here -> DEEP: 256 rows of up to 1900 keys 285 -> 245, 240 of 1000 137 -> 122, of 500 72 ->
+// 68, 250 of 100 21.3 -> 22.0; 16 heads, 500 of 1900 276 -> 303)
+inline bool latent_two(int T, int heads) { return heads > 1 && (long long)T * heads > 448 && (long long)T * heads <= 512; }
 // is latent_row_kernel built for the rank and the key size?  Others (512 + 96: 640 bytes a key and lane) keep latent_attn_kernel's DEEP
 // form.  Without load-ahead 64 rows of 64 - 505 tokens, 8 heads over 512 + 96, would take 26.5 us for 21.0, one row of 4000 23.6 for 19.6.
 inline bool latent_row_size(int Dv, int Dk) {
   const int nt = Dv / 64, ks = (Dk + 31) / 32;
   return (nt == 4 || nt == 6 || nt == 8) && ks >= 2 * nt && ks <= 2 * nt + 2;
 }
-inline bool latent_narrow(int Dv, int Dk, long long blocks) { return latent_row_size(Dv, Dk) && blocks <= kLatentNarrow; }
 
 template <typename T>
-hipError_t launch_latent_attn(const RowAttnArgs<T>& a, const T* vt, int Tn, hipStream_t st) {
+hipError_t launch_latent_attn(const RowAttnArgs<T>& a, const T* vt, int Tn, int tile, hipStream_t st) {
   const size_t lds = latent_attn_lds(a.D1 + a.D2, sizeof(T));
   const dim3 grid(Tn, (a.H + 15) / 16, a.nsplit);
   const int nt = a.Dv / 64, ks = (a.D1 + a.D2 + 31) / 32;
   // two workgroups of the deep form fit a CU, as of the other one at ranks of 384 and more
   const bool few = nt > 4 || (long long)grid.x * grid.y * grid.z <= 512;
-  const bool narrow = latent_narrow(a.Dv, a.D1 + a.D2, (long long)grid.x * grid.y);
+  const bool narrow = tile == 64;
 #define LATENT(N, D) latent_attn_kernel<T, N, D><<<grid, 64 * kWaves, lds, st>>>(a, vt)
 #define ROW(N, KS)                                                                        \
   if (narrow) latent_row_kernel<T, N, KS, 4><<<grid, 256, 0, st>>>(a, vt);                \
   else latent_row_kernel<T, N, KS, 8><<<grid, 512, 0, st>>>(a, vt)
 #define ROWS(N)                                  \
-  if (!latent_row_size(a.Dv, a.D1 + a.D2)) LATENT(N, true); \
+  if (!latent_row_size(a.Dv, a.D1 + a.D2) || (N > 4 && a.nsplit == 1 && latent_two(Tn, grid.y))) LATENT(N, true); \
   else if (ks == 2 * N) { ROW(N, 2 * N); }       \
   else if (ks == 2 * N + 1) { ROW(N, 2 * N + 1); } \
   else { ROW(N, 2 * N + 2); }
@@ -1077,7 +1087,7 @@ hipError_t launch_latent_attn(const RowAttnArgs<T>& a, const T* vt, int Tn, hipS
   return hipGetLastError();
 }
 template <>
-hipError_t launch_latent_attn<float>(const RowAttnArgs<float>&, const float*, int, hipStream_t) {
+hipError_t launch_latent_attn<float>(const RowAttnArgs<float>&, const float*, int, int, hipStream_t) {
   return hipErrorInvalidValue;
 }
 
@@ -1253,8 +1263,20 @@ int sm_latent_attn_ok(int dt, int Dv, int Dk, int D1, int bs) {
          Dk % 8 == 0 && D1 % 8 == 0 && Dv <= Dk && bs % 8 == 0 && latent_attn_lds(Dk, 2) <= 65536;
 }
 
-// Keys that a workgroup of sm_latent_attn takes of T rows with H heads: what a split of the keys is a multiple of
-int sm_latent_tile(int Dv, int Dk, int T, int H) { return latent_narrow(Dv, Dk, (long long)T * ((H + 15) / 16)) ? 64 : 128; }
+// Keys that a workgroup of sm_latent_attn takes of T rows with H heads behind tables of `keys` keys, what a split of the keys is a
+// multiple of, and in *nsplit the splits.  joined: sm_latent_out adds the splits, else a launch of its own.
+int sm_latent_plan(int Dv, int Dk, int T, int H, int keys, int joined, int* nsplit) {
+  const long long blocks = (long long)T * ((H + 15) / 16), most = blocks > 0 && blocks < 512 ? 512 / blocks : 1;
+  const long long n64 = (keys + 63) / 64, n128 = (keys + 127) / 128;
+  int tile = latent_row_size(Dv, Dk) && blocks <= kLatentNarrow ? 64 : 128;
+  if (keys > 64 && keys <= 128 && !joined) tile = 128;
+  if (blocks * n64 > 256 && blocks * n128 <= 256) tile = 128;
+  *nsplit = (int)(tile == 64 ? std::min({n64, 64LL, most}) : std::min({n128, 32LL, most}));
+  const int heads = (H + 15) / 16;
+  if (latent_row_size(Dv, Dk) && Dv > 256 && heads > 1 && blocks > 256 && blocks <= 640 && n128 > kLatentWhole && !latent_two(T, heads)) *nsplit = 4;
+  *nsplit = std::max(*nsplit, 1);
+  return tile;
+}
 
 // Latent attention (one key/value head, values = the first Dv columns of a key row) with the
 // value product on the matrix cores; `vt` is the per-block transposed copy of the values that
@@ -1266,11 +1288,11 @@ hipError_t sm_latent_attn(int dt, const void* q1, long long q1r, long long q1h, 
                           long long ouh, const int* tables, int maxb, const int* row_seg,
                           const int* positions, int T, int H, int bs, float scale, float softcap,
                           float tcoef, int tevery, const float* r1, const float* r2,
-                          const float* sink, const void* gate, long long gater, int own,
+                          const float* sink, const void* gate, long long gater, int tile, int own,
                           int nsplit, float* ws_ml, float* ws_o, hipStream_t st) {
   if (T == 0) return hipSuccess;
   const auto al = [](const void* p) { return (uintptr_t)p % 16 == 0; };
-  if (!sm_latent_attn_ok(dt, Dv, D1 + D2, D1, bs) || nsplit < 1 || nsplit > 64 ||
+  if ((tile != 128 && !(tile == 64 && latent_row_size(Dv, D1 + D2))) || !sm_latent_attn_ok(dt, Dv, D1 + D2, D1, bs) || nsplit < 1 || nsplit > 64 ||
       (nsplit > 1 && (!ws_ml || !ws_o)) || krow % 8 || !al(kc) || !al(vt) || !al(q1) || q1r % 8 ||
       q1h % 8 || (D2 > 0 && (!q2 || !al(q2) || q2r % 8 || q2h % 8)) || our % 4 || ouh % 4 ||
       (uintptr_t)out % 8 || (!out && nsplit == 1))
@@ -1282,7 +1304,7 @@ hipError_t sm_latent_attn(int dt, const void* q1, long long q1r, long long q1h, 
                       tables, maxb, row_seg, positions, H, 1, 16, bs, scale, softcap, tcoef,  \
                       tevery, r1, r2, nullptr, sink, nullptr, 0, 0, (const TT*)gate, gater,   \
                       nullptr, 1, own, nsplit, ws_ml, ws_o};                                  \
-    hipError_t e = launch_latent_attn<TT>(a, (const TT*)vt, T, st);                           \
+    hipError_t e = launch_latent_attn<TT>(a, (const TT*)vt, T, tile, st);                        \
     if (e != hipSuccess) return e;                                                            \
     if (nsplit > 1 && out)      /* (without: the caller adds the splits, sm_latent_out) */     \
       row_attn_combine_kernel<TT><<<dim3(T, H), 256, 0, st>>>(                                \

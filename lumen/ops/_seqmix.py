@@ -38,7 +38,7 @@ SIGNATURES = {
     "sm_rotate_heads": "iplliiippi",
     "sm_latent_write": "iplpppppppiiiiif",
     "sm_head_norm_write": "iplpppppiiiiif",
-    "sm_latent_attn": "i" "plli" "plli" "pl" "pi" "pll" "pi" "pp" "iii" "fffi" "ppp" "pl" "iipp",
+    "sm_latent_attn": "i" "plli" "plli" "pl" "pi" "pll" "pi" "pp" "iii" "fffi" "ppp" "pl" "iiipp",
     "sm_row_attn": "i" "plli" "plli" "pl" "pli" "pll" "pi" "pp" "iiiii" "fffi" "pppp" "piipl"
                    "pi" "iipp",
     "sm_win_attn_tiles": "iplppppl" "pi" "pi" "pp" "iiii" "ff" "p" "iii" "ipi",
@@ -120,8 +120,8 @@ def _load():
         lib.sm_latent_attn_ok.restype = ctypes.c_int
         lib.sm_latent_tiles_ok.argtypes = [ctypes.c_int] * 6
         lib.sm_latent_tiles_ok.restype = ctypes.c_int
-        lib.sm_latent_tile.argtypes = [ctypes.c_int] * 4
-        lib.sm_latent_tile.restype = ctypes.c_int
+        lib.sm_latent_plan.argtypes = [ctypes.c_int] * 6 + [ctypes.POINTER(ctypes.c_int)]
+        lib.sm_latent_plan.restype = ctypes.c_int
         lib.sm_step_attn_ok.argtypes = [_T[k] for k in "ipllii" "plpli" "pll" "iiiiii"]
         lib.sm_step_attn_ok.restype = ctypes.c_int
         lib.sm_head_scan_ahead_bytes.argtypes = [ctypes.c_int] * 5
@@ -189,9 +189,11 @@ def latent_attn_ok(dt: int, Dv: int, Dk: int, D1: int, bs: int) -> bool:
     return bool(_load().sm_latent_attn_ok(dt, Dv, Dk, D1, bs))
 
 
-def latent_tile(Dv: int, Dk: int, T: int, H: int) -> int:
-    """Keys that a workgroup of the latent attention takes of T rows with H heads."""
-    return int(_load().sm_latent_tile(Dv, Dk, T, H))
+def latent_plan(Dv: int, Dk: int, T: int, H: int, keys: int, joined: bool) -> tuple:
+    """(keys that a workgroup of the latent attention takes, splits of the keys) for T rows with H heads behind tables of
+    ``keys`` keys.  ``joined``: the expansion adds the splits, else a launch of its own does."""
+    n = ctypes.c_int()
+    return int(_load().sm_latent_plan(Dv, Dk, T, H, keys, int(joined), ctypes.byref(n))), n.value
 
 
 def latent_tiles_ok(dt: int, Dv: int, Dk: int, D1: int, bs: int, max_blocks: int) -> bool:

@@ -1106,7 +1106,7 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
     of 128, no window, linear bias, gate or sigmoid weights) to ``talk_attention.hip``; the latent layout with ``vt`` goes to the
     latent kernels (``latent_tile.hip`` for large prompt portions); every other row (decoded rows, fp32, other shapes) to the row kernel.  A row's
     result does not depend on which of them computed it beyond rounding."""
-    from ._seqmix import (DT, call, latent_attn_ok, latent_tile, latent_tiles_ok, step_attn_ok, talk_tiles_ok, use_seqmix,
+    from ._seqmix import (DT, call, latent_attn_ok, latent_plan, latent_tiles_ok, step_attn_ok, talk_tiles_ok, use_seqmix,
                           win_tiles_ok)
 
     T, _, D1 = q1.shape
@@ -1169,21 +1169,18 @@ def row_attention(q1: torch.Tensor, q2: Optional[torch.Tensor], kcache: torch.Te
             row_seg, positions = row_seg[Tp:], positions[Tp:]
         else:
             full = out
-        blocks = T * ((H + 15) // 16)
-        keys = latent_tile(Dv, Dk, T, H)                          # (a workgroup's tile)
-        tiles = (seg.tables.shape[1] * bs + keys - 1) // keys
-        nsplit = max(1, min(tiles, 64 if keys == 64 else 32, 512 // max(blocks, 1)))
+        fused = expand is not None and full is out and _expand_ok(expand, q1, T, H, Dv)
+        tile, nsplit = latent_plan(Dv, Dk, T, H, seg.tables.shape[1] * bs, fused)
         ws_ml = ws_o = None
         if nsplit > 1:
             ws_ml = torch.empty(T * H * nsplit * 2, dtype=torch.float32, device=q1.device)
             ws_o = torch.empty(T * H * nsplit * Dv, dtype=torch.float32, device=q1.device)
-        fused = expand is not None and full is out and _expand_ok(expand, q1, T, H, Dv)
         call("sm_latent_attn", DT[q1.dtype], q1, q1.stride(0), q1.stride(1), D1,
              q2, q2.stride(0) if q2 is not None else 0, q2.stride(1) if q2 is not None else 0, D2,
              kcache, krow, vt, Dv, None if fused and nsplit > 1 else out, out.stride(0), out.stride(1),
              seg.tables, seg.tables.shape[1], row_seg, positions, T, H, bs,
              scale, float(softcap or 0.0), coef, every, r1, r2, sink,
-             gate, gate.stride(0) if gate is not None else 0, own, nsplit, ws_ml, ws_o)
+             gate, gate.stride(0) if gate is not None else 0, tile, own, nsplit, ws_ml, ws_o)
         if fused:
             uv, o = expand
             call("sm_latent_out", DT[q1.dtype], ws_ml, ws_o, nsplit, out, out.stride(0), out.stride(1), gate,

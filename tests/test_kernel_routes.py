@@ -550,3 +550,18 @@ def test_scans_of_portions_without_rows(launched):
     x = torch.zeros(0, 4 * 32, **BF)
     assert head_scan(x, x, x, torch.zeros(2, 4, 32, 32), seg, 4, 32, 32, torch.zeros(4)).shape == (0, 128)
     assert [n for n, _ in launched] == ["sm_head_scan_chunk"]
+
+
+@pytest.mark.parametrize("R,Dr,T,H,keys,joined,plan", [
+    (512, 64, 8, 16, 2048, False, (64, 32)), (512, 64, 8, 16, 2049, True, (128, 17)), (384, 64, 8, 16, 4096, False, (128, 32)),
+    (512, 64, 16, 16, 2048, True, (128, 16)), (512, 64, 16, 16, 2560, True, (64, 32)), (256, 32, 32, 16, 1025, False, (64, 16)),
+    (256, 32, 1, 16, 64, False, (64, 1)), (256, 32, 1, 16, 65, False, (128, 1)), (384, 64, 32, 4, 128, False, (128, 1)),
+    (512, 64, 1, 16, 128, True, (64, 2)), (512, 64, 1, 16, 129, False, (64, 3)),
+    (384, 64, 129, 32, 1024, True, (128, 4)), (384, 64, 129, 32, 896, True, (128, 1)), (512, 64, 258, 16, 1900, True, (128, 1)),
+    (512, 64, 224, 32, 1900, False, (128, 4)), (512, 64, 225, 32, 1900, False, (128, 1)), (512, 64, 256, 32, 1900, False, (128, 1)),
+    (512, 64, 257, 32, 1900, False, (128, 4)), (512, 64, 321, 32, 1900, False, (128, 1)), (256, 32, 140, 32, 1900, True, (128, 1)),
+    (512, 96, 140, 32, 1900, True, (128, 1)), (512, 64, 64, 16, 1, False, (128, 1)), (512, 64, 64, 16, 4096, False, (128, 8))])
+def test_tiles_and_splits_of_latent_keys(R, Dr, T, H, keys, joined, plan):
+    """Tiles of 64 keys for few rows, of 128 where those are one round of the CUs or one split; four splits where blocks of heads of
+    long contexts leave much of the last round idle."""
+    assert _seqmix.latent_plan(R, R + Dr, T, H, keys, joined) == plan

@@ -132,6 +132,26 @@ def rows_behind(T, H, R, Dr, ctx, dt):
     return r(T, H, R), r(T, H, Dr), cache, cache[:, :, :R].transpose(1, 2).contiguous(), SegBatch(ar, ar[:T], pos, ar[:T], pos, tables, None)
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,H,R,Dr,ctx,kernel,splits", [
+    (8, 16, 256, 32, 2100, ("latent_row_kernel<", ", 4, 9, 8>("), 17), (3, 16, 384, 64, 127, ("latent_row_kernel<", ", 6, 14, 8>("), 1),
+    (3, 16, 512, 64, 64, ("latent_row_kernel<", ", 8, 18, 4>("), 1), (130, 17, 384, 64, 1030, ("latent_row_kernel<", ", 6, 14, 8>("), 4),
+    (224, 17, 512, 32, 140, ("latent_row_kernel<", ", 8, 17, 8>("), 1), (225, 17, 512, 64, 140, ("latent_attn_kernel<", ", 8, true>("), 1),
+    (256, 32, 384, 0, 70, ("latent_attn_kernel<", ", 6, true>("), 1)])
+def test_rows_of_each_tile_and_split(T, H, R, Dr, ctx, kernel, splits, dt):
+    """The rounding of the result and ~16 bits of the weights: under two ulps of the largest entry."""
+    from lumen.ops.attention import row_attention, row_attention_ref
+
+    q, q2, cache, vt, seg = rows_behind(T, H, R, Dr, ctx, dt)
+    q2 = q2 if Dr else None
+    out, ref = torch.empty_like(q), torch.empty(T, H, R, device="cuda")
+    run = lambda: row_attention(q, q2, cache, cache, R, out, seg, H, 1, 0.05, vt=vt)  # noqa: E731
+    (name, grid, _), *_ = launches(run)
+    assert all(k in name for k in kernel) and grid == (T, (H + 15) // 16, splits), (name, grid)
+    row_attention_ref(q.float(), q2.float() if Dr else None, cache.float(), cache.float(), R, ref, seg, H, 1, 0.05)
+    assert (out.float() - ref).abs().max() < 2 * ULP[dt] * ref.abs().max()
+
+
 @pytest.mark.parametrize("T,H,R,ctx,grid", [(1, 16, 512, 40, 1), (16, 16, 512, 300, 16), (17, 16, 512, 300, 9), (48, 16, 128, 300, 12), (49, 32, 128, 40, 7),
                                             (65, 32, 256, 9, 5), (300, 32, 128, 20, 19)])
 def test_rows_of_an_expansion_have_a_cu(T, H, R, ctx, grid):

@@ -343,7 +343,8 @@ hipError_t run(ThinArgs p, int per_cu, hipStream_t st) {
 // fragment (11264 x 2048 at M = 64: 15.3 vs 18.7 us with 32); where that leaves CUs idle the rows are cut into groups of 32 or
 // 16, each with workgroups of its own that hold more of W in flight.  All rows -> groups, us, 64 rows: 128 x 2048 6.1 -> 3.8, 256 x
 // 4096 9.5 -> 4.9 (16 and eight waves; of 32 4.7, 6.9), 2048 x 2048 7.8 -> 6.1, 2048 x 5632 17.1 -> 12.0 (32), 3072 x 2048 8.1 -> 7.5
-// (32, 32-row tiles; 16-row ones 9.6), 4096 x 4096 14.2 -> 13.8, 6144 x 2048 13.3 -> 11.8; 32 rows: 128 x 2048 4.5 -> 3.6, 2048 x 2048
+// (32, 32-row tiles; 16-row ones 9.6), 4096 x 4096 14.2 -> 13.8, 6144 x 2048 13.3 -> 11.8 (past 4096 columns two groups are more than a
+// round: of k below 1024 all rows, 33 - 64 rows of 5504 x 256 4.2 us, 5.1 in groups, 7040 x 512 5.7 and 6.2, 4608 x 1024 1 : 0.91); 32 rows: 128 x 2048 4.5 -> 3.6, 2048 x 2048
 // 6.2 -> 5.1, 2048 x 5632 12.4 -> 10.3 (16: two groups of 2048 columns' tiles are a workgroup a CU; 2112 would go x 512 3.0 -> 3.3, x 1024 4.1
 // -> 4.4, x 2048 6.0 -> 6.1, 3072 x 2048 6.5 -> 7.0).  The eight waves of up to 256 columns have use for more than three stages of k for every two
 // of them (64 rows of 256 columns, four waves over eight: k 64 - 256 0.88, 320 - 768 0.95, 832 1.02, 1536 1.05).
@@ -376,7 +377,7 @@ hipError_t pick(const ThinArgs& p, hipStream_t st) {
   }
   if (wide) return run<T, 4, 8, 2, 3>(p, 1, st);
   if (p.N <= 2048) return run<T, 1, 4, 4, 3>(p, 2, st);                  // in groups of 32
-  return run<T, 2, 4, 4, 3>(p, 1, st);
+  return p.N <= 16 * kCUs || p.K >= 1024 ? run<T, 2, 4, 4, 3>(p, 1, st) : run<T, 1, 8, 4, 3>(p, 1, st);
 }
 
 template <typename T>

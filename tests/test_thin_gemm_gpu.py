@@ -223,3 +223,15 @@ def test_waves_of_small_matrices(M, N, K, waves):
     want = x.double() @ w.double().t()
     acc, ulp = bound(x, w, 8)
     assert ((thin_linear(x, w).double() - want).abs() <= acc + want.abs() * ulp).all()
+
+
+@pytest.mark.parametrize("M,N,K,grid", [(33, 4096, 128, (128, 2)), (33, 4112, 128, (256, 1)), (64, 4100, 960, (256, 1)), (64, 4112, 1024, (129, 2)),
+                                        (33, 8188, 64, (256, 1))])
+def test_groups_of_rows_past_a_round_of_columns(M, N, K, grid):
+    """33 - 64 rows of more than 4096 columns go in two groups from k of 1024 on."""
+    x, w = torch.randn(M, K, device="cuda").bfloat16(), torch.randn(N, K, device="cuda").bfloat16()
+    (name, g, _), = launches(lambda: thin_linear(x, w))
+    assert "thin_kernel" in name and g[:2] == grid
+    want = x.double() @ w.double().t()
+    acc, ulp = bound(x, w, 8)
+    assert ((thin_linear(x, w).double() - want).abs() <= acc + want.abs() * ulp).all()

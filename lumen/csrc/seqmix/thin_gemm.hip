@@ -137,7 +137,14 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
     else kt = n_chosen * ks + (p.ffs >> 6);
   }
   const int k0 = kt * wid / NW, nk = kt * (wid + 1) / NW - k0;
-  const int mine = max(0, (tiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x);
+  // The groups of a tile's rows on one XCD (workgroups are dealt out over eight, one after the other), so that its W comes from HBM once:
+  // where the tiles are no multiple of eight the later groups start some tiles on (64 rows in two groups: 7040 x 2048 12.2 -> 11.3 us, 3104 x 4096 10.2 -> 8.5)
+  int bx = blockIdx.x;
+  if (blockIdx.y > 0 && gridDim.x >= 8) {
+    bx += gridDim.x * blockIdx.y & 7;
+    if (bx >= (int)gridDim.x) bx -= gridDim.x;
+  }
+  const int mine = max(0, (tiles - bx + (int)gridDim.x - 1) / (int)gridDim.x);
   const int total = mine * nk;                     // stages this wave streams
   const int rr = lane >> 3, c = lane & 7;          // row within a piece, LDS chunk
   // expert (E: the last block) and column of activation tile t
@@ -152,7 +159,7 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
       col = (t - n * per) * TC;
     }
   };
-  int at_t = blockIdx.x, at_k = 0, issued = 0, put = 0;
+  int at_t = bx, at_k = 0, issued = 0, put = 0;
   int left = 0, seg = 0, kk = 0;                   // sparse second projection: place in the k walk
   const auto seek = [&]() {                        // to this wave's first stage
     if (ACT || !p.sparse) { kk = k0 * BK; return; }
@@ -213,7 +220,7 @@ __global__ void __launch_bounds__(64 * NW, 1) thin_kernel(const ThinArgs p) {
     if (issued < total) issue();
   const int lr = lane & 15, lg = lane >> 4;
   int get = 0, done = 0, buf = 0;
-  for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
+  for (int t = bx; t < tiles; t += gridDim.x) {
     f32x4 acc[RT][MT];
 #pragma unroll
     for (int i = 0; i < RT; ++i)
@@ -344,7 +351,7 @@ hipError_t run(ThinArgs p, int per_cu, hipStream_t st) {
 // 16, each with workgroups of its own that hold more of W in flight.  All rows -> groups, us, 64 rows: 128 x 2048 6.1 -> 3.8, 256 x
 // 4096 9.5 -> 4.9 (16 and eight waves; of 32 4.7, 6.9), 2048 x 2048 7.8 -> 6.1, 2048 x 5632 17.1 -> 12.0 (32), 3072 x 2048 8.1 -> 7.5
 // (32, 32-row tiles; 16-row ones 9.6), 4096 x 4096 14.2 -> 13.8, 6144 x 2048 13.3 -> 11.8 (past 4096 columns two groups are more than a
-// round: of k below 1024 all rows, 33 - 64 rows of 5504 x 256 4.2 us, 5.1 in groups, 7040 x 512 5.7 and 6.2, 4608 x 1024 1 : 0.91); 32 rows: 128 x 2048 4.5 -> 3.6, 2048 x 2048
+// round: of k below 1024 or past 7680 columns all rows, 33 - 64 rows of 5504 x 256 4.2 us, 5.1 in groups, 7040 x 512 5.7 and 6.2, 8176 x 1792 1 : 1.04 - 1.08; 5504 x 2048 11.2 and 10.2); 32 rows: 128 x 2048 4.5 -> 3.6, 2048 x 2048
 // 6.2 -> 5.1, 2048 x 5632 12.4 -> 10.3 (16: two groups of 2048 columns' tiles are a workgroup a CU; 2112 would go x 512 3.0 -> 3.3, x 1024 4.1
 // -> 4.4, x 2048 6.0 -> 6.1, 3072 x 2048 6.5 -> 7.0).  The eight waves of up to 256 columns have use for more than three stages of k for every two
 // of them (64 rows of 256 columns, four waves over eight: k 64 - 256 0.88, 320 - 768 0.95, 832 1.02, 1536 1.05).
@@ -377,7 +384,7 @@ hipError_t pick(const ThinArgs& p, hipStream_t st) {
   }
   if (wide) return run<T, 4, 8, 2, 3>(p, 1, st);
   if (p.N <= 2048) return run<T, 1, 4, 4, 3>(p, 2, st);                  // in groups of 32
-  return p.N <= 16 * kCUs || p.K >= 1024 ? run<T, 2, 4, 4, 3>(p, 1, st) : run<T, 1, 8, 4, 3>(p, 1, st);
+  return p.N <= 16 * kCUs || (p.K >= 1024 && p.N <= 30 * kCUs) ? run<T, 2, 4, 4, 3>(p, 1, st) : run<T, 1, 8, 4, 3>(p, 1, st);
 }
 
 template <typename T>

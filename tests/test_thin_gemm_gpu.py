@@ -226,9 +226,10 @@ def test_waves_of_small_matrices(M, N, K, waves):
 
 
 @pytest.mark.parametrize("M,N,K,grid", [(33, 4096, 128, (128, 2)), (33, 4112, 128, (256, 1)), (64, 4100, 960, (256, 1)), (64, 4112, 1024, (129, 2)),
-                                        (33, 8188, 64, (256, 1))])
+                                        (33, 8188, 64, (256, 1)), (64, 7680, 1024, (240, 2)), (33, 7684, 1024, (256, 1)), (64, 1996, 256, (125, 2)), (20, 112, 832, (7, 2)),
+                                        (64, 128, 832, (8, 4)), (50, 140, 832, (9, 4)), (64, 2404, 512, (76, 2))])
 def test_groups_of_rows_past_a_round_of_columns(M, N, K, grid):
-    """33 - 64 rows of more than 4096 columns go in two groups from k of 1024 on."""
+    """33 - 64 rows of more than 4096 columns go in two groups from k of 1024 on, up to 7680; later groups start some tiles on."""
     x, w = torch.randn(M, K, device="cuda").bfloat16(), torch.randn(N, K, device="cuda").bfloat16()
     (name, g, _), = launches(lambda: thin_linear(x, w))
     assert "thin_kernel" in name and g[:2] == grid

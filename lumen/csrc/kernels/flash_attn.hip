@@ -23,7 +23,6 @@
 #include <algorithm>
 #include <cstdlib>
 #include "common.h"
-#include <cstdlib>
 
 namespace lumen {
 namespace fa {
